@@ -145,13 +145,30 @@ __device__ __forceinline__ uint4 swizzle_fp8_pair(uint4 v, int lane) {
   return o ? make_uint4(g0, v.z, g1, v.w) : make_uint4(v.x, g0, v.y, g1);
 }
 
-// Row-major fast path: reduce dim contiguous, K % 8 == 0, 16-byte aligned rows.
+// Elements [k, k + 8) of a row of K >= 8 that starts at any element: one 16-byte load at 2-byte alignment (the target
+// allows it).  A row's last, partial vector is loaded eight elements before the row's end instead - nothing behind the
+// row is read - and row_tail_u4 moves its elements into place, zeros behind them.
+typedef u32x4 u32x4_elem __attribute__((aligned(2)));
+__device__ __forceinline__ uint4 ld_row_u4(const uint16_t *row, int64_t k, int64_t K) {
+  const u32x4 v = *reinterpret_cast<const u32x4_elem *>(row + (k + 8 <= K ? k : K - 8));
+  return make_uint4(v.x, v.y, v.z, v.w);
+}
+__device__ __forceinline__ uint4 row_tail_u4(uint4 v, int64_t k, int64_t K) {
+  if (k < K && k + 8 > K) {
+    const unsigned __int128 w = __builtin_bit_cast(unsigned __int128, v) >> (16 * (int)(k + 8 - K));
+    v = __builtin_bit_cast(uint4, w);
+  }
+  return v;
+}
+
+// Row-major fast path: reduce dim contiguous.  ALIGNED: K % 8 == 0, 16-byte aligned rows; otherwise element-aligned loads
+// (4001 x 5003 with its two-kernel global scale: 81 us with a lane per 64-chunk and two-byte loads, 33 us here).
 // A lane owns 8 consecutive elements (half a 16-block); lane pairs share the block amax
 // through one DPP quad_perm; the four scale bytes of a 64-chunk are gathered into the
 // chunk's first lane with three DPP row shifts and stored as one dword.
 //   CPR  = 64-element chunks per wave row (8*CPR lanes per row, 8/CPR rows per wave pass)
 //   ITER = wave passes per workgroup (independent loads in flight per lane)
-template <int CPR, int ITER, bool SWIZZLE>
+template <int CPR, int ITER, bool SWIZZLE, bool ALIGNED>
 __global__ __launch_bounds__(256) void quantize_nvfp4_rowmajor_kernel(
     uint8_t *__restrict__ out, uint8_t *__restrict__ sf, const uint16_t *__restrict__ in, const float *__restrict__ gs_ptr,
     QuantGeom g) {
@@ -166,7 +183,7 @@ __global__ __launch_bounds__(256) void quantize_nvfp4_rowmajor_kernel(
   const int64_t k = ((int64_t)(blockIdx.x % ngroups) * LPR + (lane % LPR)) * 8;
   const int64_t row0 = (int64_t)(blockIdx.x / ngroups) * (4 * RW * ITER) + lane / LPR;
   if (k >= g.Kp) return;
-  const uint16_t *src = in + (lead / g.d1) * g.s0 + (lead % g.d1) * g.s1 + k;
+  const uint16_t *src = in + (lead / g.d1) * g.s0 + (lead % g.d1) * g.s1;
   const bool kvalid = k < g.K;
 
   uint4 v[ITER];
@@ -174,8 +191,11 @@ __global__ __launch_bounds__(256) void quantize_nvfp4_rowmajor_kernel(
   for (int it = 0; it < ITER; ++it) {
     const int64_t r = row0 + (int64_t)(it * 4 + wave) * RW;
     v[it] = make_uint4(0, 0, 0, 0);
-    if (kvalid && r < g.R)
-      v[it] = ld_stream_u4(src + r * g.sR);
+    if (kvalid && r < g.R) {
+      if (ALIGNED) v[it] = ld_stream_u4(src + r * g.sR + k);
+      else v[it] = ld_row_u4(src + r * g.sR, k, g.K);
+    }
+    if (!ALIGNED) v[it] = row_tail_u4(v[it], k, g.K);
     if (SWIZZLE) v[it] = swizzle_nvfp4_quad(v[it], lane);
   }
 #pragma unroll
@@ -665,7 +685,11 @@ __device__ __forceinline__ uint2 rowfmt_pack8(uint4 v, float recp, bool nan_row)
 // Row-major fast path: the whole row lives in registers between the amax pass and the
 // convert pass, so the input is read from memory once.  LPR lanes share a row (DPP / swizzle
 // reduction), each lane holds NV 16-byte vectors at a stride of LPR*8 elements.
-template <RowFmt FMT, int LPR, int NV, bool SWIZZLE>
+// Bound by HBM.  ALIGNED: every vector lies on 16 bytes inside its row.  Otherwise (K % 8 != 0, odd row stride or
+// start) the same kernel runs on element-aligned 16-byte loads: a lane-per-row loop over single elements, which such
+// rows took before, needs 3000 - 3700 us for 4001 x 5003 int8 (4001 lanes on 256 CUs, 64 lines per wave load), this 15 us
+// = 4.1 TB/s (20 us fp8 with swizzle).
+template <RowFmt FMT, int LPR, int NV, bool SWIZZLE, bool ALIGNED>
 __global__ __launch_bounds__(256) void quantize_rowwise_rowmajor_kernel(
     uint8_t *__restrict__ out, float *__restrict__ sf, const uint16_t *__restrict__ in,
     const void *__restrict__ smax_p, QuantGeom g) {
@@ -681,7 +705,8 @@ __global__ __launch_bounds__(256) void quantize_rowwise_rowmajor_kernel(
   for (int j = 0; j < NV; ++j) {
     const int64_t k = ((int64_t)j * LPR + sub) * 8;
     v[j] = make_uint4(0, 0, 0, 0);
-    if (r < g.R && k < g.K) v[j] = ld_stream_u4(src + k);
+    if (r < g.R && k < g.K) v[j] = ALIGNED ? ld_stream_u4(src + k) : ld_row_u4(src, k, g.K);
+    if (!ALIGNED) v[j] = row_tail_u4(v[j], k, g.K);
     m = umax32(m, absmax_bf16x8(v[j]));
     if (SWIZZLE) v[j] = swizzle_fp8_pair(v[j], threadIdx.x);
   }
@@ -702,7 +727,7 @@ __global__ __launch_bounds__(256) void quantize_rowwise_rowmajor_kernel(
 
 // Rows longer than the register budget of the kernel above: one wave per row, two passes over the
 // row (the second one is served by the caches), 16-byte loads, 8-byte stores.
-template <RowFmt FMT>
+template <RowFmt FMT, bool SWIZZLE, bool ALIGNED>
 __global__ __launch_bounds__(256) void quantize_rowwise_longrow_kernel(
     uint8_t *__restrict__ out, float *__restrict__ sf, const uint16_t *__restrict__ in,
     const void *__restrict__ smax_p, QuantGeom g) {
@@ -717,7 +742,10 @@ __global__ __launch_bounds__(256) void quantize_rowwise_longrow_kernel(
   }
   const uint16_t *src = in + (lead / g.d1) * g.s0 + (lead % g.d1) * g.s1 + r * g.sR;
   uint32_t m = 0;
-  for (int64_t k = lane * 8; k < g.K; k += 512) m = umax32(m, absmax_bf16x8(*reinterpret_cast<const uint4 *>(src + k)));
+  auto load = [&](int64_t k) {
+    return ALIGNED ? *reinterpret_cast<const uint4 *>(src + k) : row_tail_u4(ld_row_u4(src, k, g.K), k, g.K);
+  };
+  for (int64_t k = lane * 8; k < g.K; k += 512) m = umax32(m, absmax_bf16x8(load(k)));
   m = group_umax<64>(m);
   const float amax = bf16_bits_to_f32(m);
   if (lane == 0) sf[lead * g.Rp + r] = amax / smax;
@@ -726,12 +754,14 @@ __global__ __launch_bounds__(256) void quantize_rowwise_longrow_kernel(
   uint8_t *op = out + (lead * g.R + r) * g.Kp;
   for (int64_t k = lane * 8; k < g.Kp; k += 512) {
     uint4 v = make_uint4(0, 0, 0, 0);
-    if (k < g.K) v = *reinterpret_cast<const uint4 *>(src + k);
+    if (k < g.K) v = load(k);
+    if (SWIZZLE) v = swizzle_fp8_pair(v, lane);  // (Kp % 16 == 0: both lanes of a pair are here)
     st_stream_u2(op + k, rowfmt_pack8<FMT>(v, recp, nan_row));
   }
 }
 
-// Generic path: any strides / swizzle / K.  One lane per row, two passes over the row.
+// Generic path: any strides / swizzle / K, for what neither the row-major nor the cross-major kernels take (both dims
+// strided, or fewer than eight elements in the contiguous one).  One lane per row, two passes over the row.
 template <RowFmt FMT, bool SWIZZLE>
 __global__ __launch_bounds__(256) void quantize_rowwise_generic_kernel(
     uint8_t *__restrict__ out, float *__restrict__ sf, const uint16_t *__restrict__ in,
@@ -783,7 +813,18 @@ __global__ __launch_bounds__(256) void quantize_rowwise_generic_kernel(
 // so block maxima, products and nibble/byte packing all stay inside the lane - no transposition -
 // and the swizzles are only a different choice of the 16 source positions.  Four adjacent lanes
 // hold the four blocks of a chunk: their stores of one row are contiguous.
+// Any start, any strides and any R >= 8: the loads need 2-byte alignment only, and the last group of a row count that is
+// not a multiple of eight is moved back to end at R (rows that two groups share are computed and stored twice, the same
+// bytes).  fp8 of (1, 4096, 8, 100), cross 3, reduce 1: 1588 us with a lane per row and
+// two-byte loads, 44 us here; int8 of a transposed 5003 x 4001: 3278 -> 81 us.
 // ===========================================================================
+
+// first row that the group of eight rows from row0 on reads and writes (row0 < R)
+__device__ __forceinline__ int64_t crossmajor_rows(int64_t row0, int64_t R) { return row0 + 8 <= R ? row0 : R - 8; }
+__device__ __forceinline__ uint4 ld_elem_u4(const uint16_t *p) {
+  const u32x4 v = *reinterpret_cast<const u32x4_elem *>(p);
+  return make_uint4(v.x, v.y, v.z, v.w);
+}
 
 // bf16 component j (0..7) of a 16-byte vector as float
 __device__ __forceinline__ float bf16_comp(const uint4 &v, int j) {
@@ -819,11 +860,12 @@ __global__ __launch_bounds__(256) void quantize_nvfp4_crossmajor_kernel(
   const int kb = lane & 3, rg = lane >> 2;
   const CrossMajorIdx gi = crossmajor_idx(g);
   const int64_t cc = gi.kblock * 4 + wave;                      // 64-chunk along the reduce dim
-  const int64_t row0 = (int64_t)blockIdx.y * 128 + rg * 8;      // first of the lane's eight rows
+  const int64_t group0 = (int64_t)blockIdx.y * 128 + rg * 8;
   const int64_t lead = gi.lead;
-  if (cc * 64 >= g.Kp || row0 >= g.Rp) return;
+  if (cc * 64 >= g.Kp || group0 >= g.Rp) return;
+  const bool rows_valid = group0 < g.R;
+  const int64_t row0 = rows_valid ? crossmajor_rows(group0, g.R) : group0;  // first of the lane's eight rows
   const uint16_t *src = in + (lead / g.d1) * g.s0 + (lead % g.d1) * g.s1 + row0;
-  const bool rows_valid = row0 < g.R;  // R % 8 == 0: all eight or none
 
   uint4 v[16];
   uint4 m8 = make_uint4(0, 0, 0, 0);
@@ -832,7 +874,7 @@ __global__ __launch_bounds__(256) void quantize_nvfp4_crossmajor_kernel(
     const int p = (kb & 1) * 16 + i;  // output position inside the 32-group
     const int64_t k = cc * 64 + (kb >> 1) * 32 + (SWIZZLE ? nvfp4_swizzle_src(p) : p);
     v[i] = make_uint4(0, 0, 0, 0);
-    if (rows_valid && k < g.K) v[i] = *reinterpret_cast<const uint4 *>(src + k * g.sK);
+    if (rows_valid && k < g.K) v[i] = ld_elem_u4(src + k * g.sK);
   }
 #pragma unroll
   for (int i = 0; i < 16; ++i) m8 = absmax_bf16x8_pairwise(m8, v[i]);
@@ -861,7 +903,15 @@ __global__ __launch_bounds__(256) void quantize_nvfp4_crossmajor_kernel(
   const uint2 mine = kb == 0 ? make_uint2(sfw[0], sfw[1])
                    : kb == 1 ? make_uint2(sfw[2], sfw[3])
                    : kb == 2 ? make_uint2(sfw[4], sfw[5]) : make_uint2(sfw[6], sfw[7]);
-  *reinterpret_cast<uint2 *>(reinterpret_cast<uint32_t *>(sf) + (lead * (g.Kp / 64) + cc) * g.Rp + row0 + 2 * kb) = mine;
+  uint32_t *sfcol = reinterpret_cast<uint32_t *>(sf) + (lead * (g.Kp / 64) + cc) * g.Rp;
+  if (row0 == group0) {
+    *reinterpret_cast<uint2 *>(sfcol + row0 + 2 * kb) = mine;
+  } else {  // group moved back to end at R: the pad rows of its place in the grid are zeros
+    sfcol[row0 + 2 * kb] = mine.x;
+    sfcol[row0 + 2 * kb + 1] = mine.y;
+    if (group0 + 2 * kb >= g.R) sfcol[group0 + 2 * kb] = 0u;
+    if (group0 + 2 * kb + 1 >= g.R) sfcol[group0 + 2 * kb + 1] = 0u;
+  }
 }
 
 // ---- per-row fp8 / int8 with the reduce dim strided: the row maximum is collected with atomic
@@ -879,18 +929,19 @@ __global__ __launch_bounds__(256) void rowwise_crossmajor_amax_kernel(uint32_t *
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int kq = lane & 3, rg = lane >> 2;
   const CrossMajorIdx gi = crossmajor_idx(g);
-  const int64_t row0 = (int64_t)blockIdx.y * 128 + rg * 8;
+  const int64_t group0 = (int64_t)blockIdx.y * 128 + rg * 8;
   const int64_t lead = gi.lead;
+  const int64_t row0 = crossmajor_rows(group0, g.R);
   const uint16_t *src = in + (lead / g.d1) * g.s0 + (lead % g.d1) * g.s1 + row0;
   uint4 m8 = make_uint4(0, 0, 0, 0);
-  if (row0 < g.R) {
+  if (group0 < g.R) {
     const int64_t kbeg = gi.kblock * CM_KSPAN, kend = kbeg + CM_KSPAN < g.K ? kbeg + CM_KSPAN : g.K;
     for (int64_t k = kbeg + wave * 4 + kq; k < kend; k += 64) {  // four loads in flight per lane
       uint4 a[4];
 #pragma unroll
       for (int u = 0; u < 4; ++u) {
         a[u] = make_uint4(0, 0, 0, 0);
-        if (k + u * 16 < kend) a[u] = *reinterpret_cast<const uint4 *>(src + (k + u * 16) * g.sK);
+        if (k + u * 16 < kend) a[u] = ld_elem_u4(src + (k + u * 16) * g.sK);
       }
 #pragma unroll
       for (int u = 0; u < 4; ++u) m8 = absmax_bf16x8_pairwise(m8, a[u]);
@@ -908,7 +959,7 @@ __global__ __launch_bounds__(256) void rowwise_crossmajor_amax_kernel(uint32_t *
   __shared__ uint4 red[4][16];
   if (kq == 0) red[wave][rg] = m8;
   __syncthreads();
-  if (wave == 0 && kq == 0 && row0 < g.R) {
+  if (wave == 0 && kq == 0 && group0 < g.R) {
     uint4 t = red[0][rg];
 #pragma unroll
     for (int w2 = 1; w2 < 4; ++w2) t = absmax_bf16x8_pairwise(t, red[w2][rg]);
@@ -929,16 +980,17 @@ __global__ __launch_bounds__(256) void quantize_rowwise_crossmajor_kernel(
   const int kb = lane & 3, rg = lane >> 2;
   const CrossMajorIdx gi = crossmajor_idx(g);
   const int64_t k0 = (gi.kblock * 4 + wave) * 64 + kb * 16;  // the lane's 16 output positions
-  const int64_t row0 = (int64_t)blockIdx.y * 128 + rg * 8;
+  const int64_t group0 = (int64_t)blockIdx.y * 128 + rg * 8;
   const int64_t lead = gi.lead;
-  if (k0 >= g.Kp || row0 >= g.R) return;
+  if (k0 >= g.Kp || group0 >= g.R) return;
+  const int64_t row0 = crossmajor_rows(group0, g.R);
   const uint16_t *src = in + (lead / g.d1) * g.s0 + (lead % g.d1) * g.s1 + row0;
   uint4 v[16];
 #pragma unroll
   for (int i = 0; i < 16; ++i) {
     const int64_t k = k0 + (SWIZZLE ? fp8_swizzle_src(i) : i);
     v[i] = make_uint4(0, 0, 0, 0);
-    if (k < g.K) v[i] = *reinterpret_cast<const uint4 *>(src + k * g.sK);
+    if (k < g.K) v[i] = ld_elem_u4(src + k * g.sK);
   }
 #pragma unroll
   for (int j = 0; j < 8; ++j) {
@@ -1005,27 +1057,36 @@ static bool dense_permutation(int64_t d0, int64_t d1, int64_t R, int64_t K, int6
   return true;
 }
 
+// reduce dim contiguous, every 8-element vector of every row on 16 bytes
 static bool rowmajor_ok(const void *in, int64_t K, int64_t s0, int64_t s1, int64_t sR, int64_t sK) {
   return sK == 1 && K % 8 == 0 && (reinterpret_cast<uintptr_t>(in) & 15) == 0 && sR % 8 == 0 &&
          s0 % 8 == 0 && s1 % 8 == 0;
 }
 
-// cross dim contiguous, every row group of eight 16-byte aligned
-static bool crossmajor_ok(const void *in, int64_t R, int64_t s0, int64_t s1, int64_t sR, int64_t sK) {
-  return sR == 1 && R % 8 == 0 && (reinterpret_cast<uintptr_t>(in) & 15) == 0 && sK % 8 == 0 && s0 % 8 == 0 &&
-         s1 % 8 == 0;
-}
+// cross dim contiguous, at least one whole group of eight rows
+static bool crossmajor_ok(int64_t R, int64_t sR) { return sR == 1 && R >= 8; }
 
-template <int CPR>
+template <int CPR, bool ALIGNED>
 static void launch_nvfp4_rowmajor(uint8_t *out, uint8_t *sf, const uint16_t *in, const float *gs,
                                   const QuantGeom &g, int64_t lead, hipStream_t st, bool swizzle) {
   constexpr int ITER = 4;
   constexpr int ROWS = 4 * (8 / CPR) * ITER;
   dim3 grid((unsigned)(ceil_div(g.Kp / 64, CPR) * ceil_div(g.Rp, ROWS)), (unsigned)lead);
   if (swizzle)
-    hipLaunchKernelGGL((quantize_nvfp4_rowmajor_kernel<CPR, ITER, true>), grid, dim3(256), 0, st, out, sf, in, gs, g);
+    hipLaunchKernelGGL((quantize_nvfp4_rowmajor_kernel<CPR, ITER, true, ALIGNED>), grid, dim3(256), 0, st, out, sf, in, gs, g);
   else
-    hipLaunchKernelGGL((quantize_nvfp4_rowmajor_kernel<CPR, ITER, false>), grid, dim3(256), 0, st, out, sf, in, gs, g);
+    hipLaunchKernelGGL((quantize_nvfp4_rowmajor_kernel<CPR, ITER, false, ALIGNED>), grid, dim3(256), 0, st, out, sf, in, gs, g);
+}
+
+// four chunks per wave row: a workgroup then covers 32 rows x 256 elements, and each scale
+// column gets a 128-byte run; eight chunks per row measured 4-12 % slower on every shape
+template <bool ALIGNED>
+static void launch_nvfp4_contiguous(uint8_t *out, uint8_t *sf, const uint16_t *in, const float *gs, const QuantGeom &g,
+                                    int64_t lead, hipStream_t st, bool swizzle) {
+  const int64_t chunks = g.Kp / 64;
+  if (chunks >= 3) launch_nvfp4_rowmajor<4, ALIGNED>(out, sf, in, gs, g, lead, st, swizzle);
+  else if (chunks == 2) launch_nvfp4_rowmajor<2, ALIGNED>(out, sf, in, gs, g, lead, st, swizzle);
+  else launch_nvfp4_rowmajor<1, ALIGNED>(out, sf, in, gs, g, lead, st, swizzle);
 }
 
 }  // namespace ac4k
@@ -1253,18 +1314,12 @@ static int launch_quantize_nvfp4(void *out, void *sf, const void *in, const floa
   const int64_t lead_all = d0 * d1;
   for (g.lead0 = 0; g.lead0 < lead_all; g.lead0 += 65535) {
     const int64_t lead = lead_all - g.lead0 < 65535 ? lead_all - g.lead0 : 65535;
-    if (rowmajor_ok(in, K, s0, s1, sR, sK) && ceil_div(g.Kp, 64) * ceil_div(g.Rp, 16) < (1ll << 31)) {
-      const int64_t chunks = g.Kp / 64;
-      const bool sw = swizzle != 0;
-      // four chunks per wave row: a workgroup then covers 32 rows x 256 elements, and each scale
-      // column gets a 128-byte run; eight chunks per row measured 4-12 % slower on every shape
-      if (chunks >= 3)
-        launch_nvfp4_rowmajor<4>(o, s, x, gsrc, g, lead, st, sw);
-      else if (chunks == 2)
-        launch_nvfp4_rowmajor<2>(o, s, x, gsrc, g, lead, st, sw);
+    if (sK == 1 && K >= 8 && ceil_div(g.Kp, 64) * ceil_div(g.Rp, 16) < (1ll << 31)) {
+      if (rowmajor_ok(in, K, s0, s1, sR, sK))
+        launch_nvfp4_contiguous<true>(o, s, x, gsrc, g, lead, st, swizzle != 0);
       else
-        launch_nvfp4_rowmajor<1>(o, s, x, gsrc, g, lead, st, sw);
-    } else if (crossmajor_ok(in, R, s0, s1, sR, sK) && ceil_div(g.Rp, 128) <= 65535) {
+        launch_nvfp4_contiguous<false>(o, s, x, gsrc, g, lead, st, swizzle != 0);
+    } else if (crossmajor_ok(R, sR) && ceil_div(g.Rp, 128) <= 65535) {
       // (position along the reduce dim as the fast grid index: the packed rows are written in runs along it)
       const dim3 grid = crossmajor_grid(g, ceil_div(g.Kp / 64, 4), ceil_div(g.Rp, 128), lead);
       if (swizzle)
@@ -1331,16 +1386,29 @@ extern "C" __attribute__((visibility("default"))) int64_t ac4k_debug_quantize_ti
 
 namespace ac4k {
 
-template <RowFmt FMT, int LPR, int NV>
+template <RowFmt FMT, int LPR, int NV, bool SWIZZLE, bool ALIGNED>
 static void launch_rowwise_rowmajor(uint8_t *out, float *sf, const uint16_t *in, const void *smax,
-                                    const QuantGeom &g, int64_t lead, hipStream_t st, bool swizzle) {
-  dim3 grid((unsigned)ceil_div(g.Rp, 256 / LPR), (unsigned)lead);
-  if (swizzle && FMT == RowFmt::FP8)
-    hipLaunchKernelGGL((quantize_rowwise_rowmajor_kernel<FMT, LPR, NV, FMT == RowFmt::FP8>), grid, dim3(256), 0, st, out,
-                       sf, in, smax, g);
+                                    const QuantGeom &g, int64_t lead, hipStream_t st) {
+  hipLaunchKernelGGL((quantize_rowwise_rowmajor_kernel<FMT, LPR, NV, SWIZZLE, ALIGNED>),
+                     dim3((unsigned)ceil_div(g.Rp, 256 / LPR), (unsigned)lead), dim3(256), 0, st, out, sf, in, smax, g);
+}
+
+// rows contiguous: in the registers of LPR lanes up to 16384 elements, longer ones one wave and two reads
+template <RowFmt FMT, bool SWIZZLE, bool ALIGNED>
+static void launch_rowwise_contiguous(uint8_t *out, float *sf, const uint16_t *in, const void *smax, const QuantGeom &g,
+                                      int64_t lead, hipStream_t st) {
+  if (g.K <= 64) launch_rowwise_rowmajor<FMT, 8, 1, SWIZZLE, ALIGNED>(out, sf, in, smax, g, lead, st);
+  else if (g.K <= 128) launch_rowwise_rowmajor<FMT, 16, 1, SWIZZLE, ALIGNED>(out, sf, in, smax, g, lead, st);
+  else if (g.K <= 256) launch_rowwise_rowmajor<FMT, 32, 1, SWIZZLE, ALIGNED>(out, sf, in, smax, g, lead, st);
+  else if (g.K <= 512) launch_rowwise_rowmajor<FMT, 64, 1, SWIZZLE, ALIGNED>(out, sf, in, smax, g, lead, st);
+  else if (g.K <= 1024) launch_rowwise_rowmajor<FMT, 64, 2, SWIZZLE, ALIGNED>(out, sf, in, smax, g, lead, st);
+  else if (g.K <= 2048) launch_rowwise_rowmajor<FMT, 64, 4, SWIZZLE, ALIGNED>(out, sf, in, smax, g, lead, st);
+  else if (g.K <= 4096) launch_rowwise_rowmajor<FMT, 64, 8, SWIZZLE, ALIGNED>(out, sf, in, smax, g, lead, st);
+  else if (g.K <= 8192) launch_rowwise_rowmajor<FMT, 64, 16, SWIZZLE, ALIGNED>(out, sf, in, smax, g, lead, st);
+  else if (g.K <= 16384) launch_rowwise_rowmajor<FMT, 64, 32, SWIZZLE, ALIGNED>(out, sf, in, smax, g, lead, st);
   else
-    hipLaunchKernelGGL((quantize_rowwise_rowmajor_kernel<FMT, LPR, NV, false>), grid, dim3(256), 0, st, out, sf, in,
-                       smax, g);
+    hipLaunchKernelGGL((quantize_rowwise_longrow_kernel<FMT, SWIZZLE, ALIGNED>),
+                       dim3((unsigned)ceil_div(g.Rp, 4), (unsigned)lead), dim3(256), 0, st, out, sf, in, smax, g);
 }
 
 template <RowFmt FMT>
@@ -1354,30 +1422,14 @@ static int quantize_rowwise(void *out, float *sf, const void *in, const void *sm
   const int64_t lead_all = d0 * d1;
   for (g.lead0 = 0; g.lead0 < lead_all; g.lead0 += 65535) {
     const int64_t lead = lead_all - g.lead0 < 65535 ? lead_all - g.lead0 : 65535;
-    if (rowmajor_ok(in, K, s0, s1, sR, sK) && K <= 16384) {
-      const bool sw = swizzle != 0;
-      if (K <= 64)
-        launch_rowwise_rowmajor<FMT, 8, 1>(o, sf, x, smax, g, lead, st, sw);
-      else if (K <= 128)
-        launch_rowwise_rowmajor<FMT, 16, 1>(o, sf, x, smax, g, lead, st, sw);
-      else if (K <= 256)
-        launch_rowwise_rowmajor<FMT, 32, 1>(o, sf, x, smax, g, lead, st, sw);
-      else if (K <= 512)
-        launch_rowwise_rowmajor<FMT, 64, 1>(o, sf, x, smax, g, lead, st, sw);
-      else if (K <= 1024)
-        launch_rowwise_rowmajor<FMT, 64, 2>(o, sf, x, smax, g, lead, st, sw);
-      else if (K <= 2048)
-        launch_rowwise_rowmajor<FMT, 64, 4>(o, sf, x, smax, g, lead, st, sw);
-      else if (K <= 4096)
-        launch_rowwise_rowmajor<FMT, 64, 8>(o, sf, x, smax, g, lead, st, sw);
-      else if (K <= 8192)
-        launch_rowwise_rowmajor<FMT, 64, 16>(o, sf, x, smax, g, lead, st, sw);
-      else
-        launch_rowwise_rowmajor<FMT, 64, 32>(o, sf, x, smax, g, lead, st, sw);
-    } else if (!swizzle && rowmajor_ok(in, K, s0, s1, sR, sK)) {  // rows too long for the register file
-      dim3 grid((unsigned)ceil_div(g.Rp, 4), (unsigned)lead);
-      hipLaunchKernelGGL((quantize_rowwise_longrow_kernel<FMT>), grid, dim3(256), 0, st, o, sf, x, smax, g);
-    } else if (crossmajor_ok(in, R, s0, s1, sR, sK) && ceil_div(g.Rp, 128) <= 65535 && ceil_div(K, CM_KSPAN) <= 65535) {
+    constexpr bool CAN_SWIZZLE = FMT == RowFmt::FP8;  // (the int8 entry point has no swizzle)
+    if (sK == 1 && K >= 8) {
+      const bool aligned = rowmajor_ok(in, K, s0, s1, sR, sK);
+      if (swizzle && aligned) launch_rowwise_contiguous<FMT, CAN_SWIZZLE, true>(o, sf, x, smax, g, lead, st);
+      else if (swizzle) launch_rowwise_contiguous<FMT, CAN_SWIZZLE, false>(o, sf, x, smax, g, lead, st);
+      else if (aligned) launch_rowwise_contiguous<FMT, false, true>(o, sf, x, smax, g, lead, st);
+      else launch_rowwise_contiguous<FMT, false, false>(o, sf, x, smax, g, lead, st);
+    } else if (crossmajor_ok(R, sR) && ceil_div(g.Rp, 128) <= 65535 && ceil_div(K, CM_KSPAN) <= 65535) {
       // row maxima as bf16 bit patterns in the scale array, quantize from them, then scale them in place
       uint32_t *bits = reinterpret_cast<uint32_t *>(sf) + g.lead0 * g.Rp;  // the kernels index by absolute lead
       const int64_t nsf = lead * g.Rp;

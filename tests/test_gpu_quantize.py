@@ -184,6 +184,34 @@ def test_crossmajor_layouts(shape, cross, red, swz):
         assert torch.equal(out.cpu(), eo) and torch.equal(sf.cpu(), es)
 
 
+# Rows and row groups that start at any element: K around one vector, one lane group and the register budget (64, 512,
+# 16384), R around a group of eight and a workgroup of 128 rows; the first element of the tensor off 16 bytes as well.
+RAGGED_SHAPES = [((5, 8), 0, 1), ((3, 9), 0, 1), ((17, 15), 0, 1), ((9, 63), 0, 1), ((33, 65), 0, 1), ((7, 513), 0, 1),
+                 ((3, 8191), 0, 1), ((2, 16383), 0, 1), ((2, 16387), 0, 1), ((3, 20008), 0, 1), ((4, 7), 0, 1), ((2, 3, 5, 100), 1, 3),
+                 ((70, 8), 1, 0), ((33, 9), 1, 0), ((100, 15), 1, 0), ((65, 127), 1, 0), ((130, 129), 1, 0), ((2060, 137), 1, 0),
+                 ((2, 90, 3, 100), 3, 1), ((40, 7), 1, 0)]
+
+
+@pytest.mark.parametrize("shape,cross,red", RAGGED_SHAPES)
+@pytest.mark.parametrize("off", [0, 1, 4])
+def test_ragged_contiguous_dims(shape, cross, red, off):
+    x = make_input(shape, seed=sum(shape) + off, outliers=True)
+    buf = torch.zeros(x.numel() + 16, dtype=torch.bfloat16, device="cuda")
+    y = buf[off:off + x.numel()].view(shape)
+    y.copy_(x)
+    for precision, oracle in (("fp8e4m3", T.quantize_fp8), ("int8", T.quantize_int8)):
+        for swz in ((False, True) if precision == "fp8e4m3" else (False,)):
+            args = (448.0, swz) if precision == "fp8e4m3" else (127,)
+            eo, es = oracle(x, cross, red, *args)
+            o, s = ops().quantize(y, cross, red, precision=precision, swizzle=swz)
+            assert torch.equal(o.cpu().view(torch.uint8), eo.view(torch.uint8)), (precision, swz)
+            assert torch.equal(s.cpu(), es), (precision, swz)
+    for swz in (False, True):
+        eo, es, eg = T.quantize_nvfp4(x, cross, red, swz)
+        o, s, gs = ops().quantize(y, cross, red, swizzle=swz)
+        assert torch.equal(gs.cpu(), eg) and torch.equal(o.cpu(), eo) and torch.equal(s.cpu().view(torch.uint8), es), swz
+
+
 def test_nvfp4_graph_replay():
     """A captured quantize call replays correctly: under capture the library takes the path whose whole
     state is in the caller's buffers, so nothing in it depends on host-side state that changes from
