@@ -34,6 +34,9 @@ typedef float f32x16 __attribute__((ext_vector_type(16)));
 
 typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+// the same at the alignment of a bf16 element / a byte: global memory takes vector accesses at any address
+typedef u32x4 u32x4_elem __attribute__((aligned(2)));
+typedef u32x2 u32x2_elem __attribute__((aligned(1)));
 
 // streaming (non-temporal) 16-byte load / 4- and 8-byte stores: data touched once
 __device__ __forceinline__ uint4 ld_stream_u4(const void *p) {
@@ -43,6 +46,10 @@ __device__ __forceinline__ uint4 ld_stream_u4(const void *p) {
 __device__ __forceinline__ void st_stream_u2(void *p, uint2 v) {
   u32x2 w = {v.x, v.y};
   __builtin_nontemporal_store(w, static_cast<u32x2 *>(p));
+}
+__device__ __forceinline__ void st_elem_u2(void *p, uint2 v) {
+  u32x2 w = {v.x, v.y};
+  *static_cast<u32x2_elem *>(p) = w;
 }
 __device__ __forceinline__ void st_stream_u1(void *p, uint32_t v) {
   __builtin_nontemporal_store(v, static_cast<uint32_t *>(p));
@@ -109,6 +116,17 @@ __device__ __forceinline__ uint32_t f32_to_ue4m3_satfinite(float x) {
 
 __device__ __forceinline__ float e4m3_to_f32(uint32_t code) {
   return __builtin_amdgcn_cvt_f32_fp8((int)code, 0);
+}
+
+// satfinite e4m3 of four floats -> four bytes, element 0 in the low byte.
+__device__ __forceinline__ uint32_t f32x4_to_e4m3x4(float a, float b, float c, float d) {
+  a = __builtin_amdgcn_fmed3f(a, -448.0f, 448.0f);
+  b = __builtin_amdgcn_fmed3f(b, -448.0f, 448.0f);
+  c = __builtin_amdgcn_fmed3f(c, -448.0f, 448.0f);
+  d = __builtin_amdgcn_fmed3f(d, -448.0f, 448.0f);
+  int w = __builtin_amdgcn_cvt_pk_fp8_f32(a, b, 0, false);
+  w = __builtin_amdgcn_cvt_pk_fp8_f32(c, d, w, true);
+  return (uint32_t)w;
 }
 
 // cvt.rn.satfinite.e2m1x2.f32 of eight floats -> eight nibbles, element 0 in bits 0..3.

@@ -21,7 +21,7 @@
 // nibbles are formed inside the lane, and the row maximum and row sum need one exchange between the two
 // halves of the wave.  The k slots of the second product are paired through the stored (swizzled) order
 // of V: slot s of step t holds kv position 8 (2t + (s>>1 & 1)) + 4h + 2 (s>>2) + (s & 1).
-#include "ac4k_common.h"
+#include "attention_quantize.h"
 
 #include <atomic>
 #include <type_traits>
@@ -660,21 +660,12 @@ __global__ __launch_bounds__(256) void quantize_int8_token_block_kernel(int8_t *
     if ((threadIdx.x & 63) == 0) wmax[threadIdx.x >> 6] = mx;
     __syncthreads();
     mx = umax32(umax32(wmax[0], wmax[1]), umax32(wmax[2], wmax[3]));
-    const float sc = bf16_bits_to_f32(mx) / 127.0f;
-    if (threadIdx.x == 0) scale[(b * H + head) * nb + blk] = sc;
+    const Int8BlockScale sc(mx);
+    if (threadIdx.x == 0) scale[(b * H + head) * nb + blk] = sc.scale;
 #pragma unroll
     for (int j = 0; j < 8; ++j) {
       const int i = threadIdx.x + j * 256;
-      if (i >= nvec) continue;
-      const uint32_t w[4] = {v[j].x, v[j].y, v[j].z, v[j].w};
-      uint32_t o2[2] = {0, 0};
-#pragma unroll
-      for (int e = 0; e < 8; ++e) {
-        const float xe = bf16_bits_to_f32((w[e >> 1] >> (16 * (e & 1))) & 0xffffu);
-        const int q = sc != 0.0f ? (int)(xe / sc) : 0;  // toward zero; |q| <= 127 up to rounding
-        o2[e >> 2] |= ((uint32_t)q & 0xffu) << (8 * (e & 3));
-      }
-      *reinterpret_cast<uint2 *>(dst + (int64_t)(i / vpr) * Dp + (i % vpr) * 8) = make_uint2(o2[0], o2[1]);
+      if (i < nvec) *reinterpret_cast<uint2 *>(dst + (int64_t)(i / vpr) * Dp + (i % vpr) * 8) = sc.quantize8(v[j]);
     }
     if (Dp != D) {  // D % 16 == 8: eight pad columns per row
       for (int rr = threadIdx.x; rr < rows; rr += 256) *reinterpret_cast<uint2 *>(dst + (int64_t)rr * Dp + D) = make_uint2(0, 0);
@@ -802,4 +793,50 @@ extern "C" __attribute__((visibility("default"))) int ac4k_quantize_int8_token_b
                      s_h, s_n, H, N, (int)D, (int)align_up(D, 16), block,
                      (D % 8 == 0 && ((uintptr_t)x & 15) == 0 && s_b % 8 == 0 && s_h % 8 == 0 && s_n % 8 == 0) ? 1 : 0);
   return check_launch("ac4k_quantize_int8_token_block_bf16");
+}
+
+// Replaces _int8_x_fp8_attention (python/ac4k_kernel/ops/attention.py:137-190): the quantizers of attention_quantize.hip,
+// then ac4k_mha_int8_x_fp8_fwd on their outputs.
+static int attention_int8_args(AttnQuantArgs &a, int64_t B, int64_t H, int64_t Nq, int64_t Nkv, int64_t Dqk, int64_t Dv) {
+  AC4K_REQUIRE(B >= 1 && H >= 1 && Nq >= 1 && Nkv >= 1, "B, H, Nq, Nkv must be positive (B=%lld H=%lld Nq=%lld Nkv=%lld)",
+               (long long)B, (long long)H, (long long)Nq, (long long)Nkv);
+  AC4K_REQUIRE(Dqk >= 8 && Dqk <= 128 && Dv >= 8 && Dv <= 128, "Dqk and Dv must be 8 to 128");
+  AC4K_REQUIRE(H <= 65535 && B <= 65535 && Nq < (1ll << 30) && Nkv < (1ll << 30) &&
+               B * H * (ceil_div(Nq, 64) + ceil_div(Nkv, 64)) < (1ll << 31), "problem too large");
+  a = AttnQuantArgs{};
+  a.B = (int)B, a.H = (int)H, a.Nq = (int)Nq, a.Nkv = (int)Nkv, a.D = (int)Dqk, a.Dv = (int)Dv;
+  return 0;
+}
+
+extern "C" __attribute__((visibility("default"))) int64_t ac4k_attention_int8_x_fp8_workspace_bytes(
+    int64_t B, int64_t H, int64_t Nq, int64_t Nkv, int64_t Dqk, int64_t Dv) {
+  AttnQuantArgs a;
+  if (attention_int8_args(a, B, H, Nq, Nkv, Dqk, Dv)) return -1;
+  return attn_quant_layout(a, nullptr);
+}
+
+extern "C" __attribute__((visibility("default"))) int ac4k_attention_int8_x_fp8_bf16(
+    void *O, int64_t o_b_stride, int64_t o_h_stride, int64_t o_n_stride, int64_t o_d_stride, const void *q, int64_t q_b_stride,
+    int64_t q_h_stride, int64_t q_n_stride, const void *k, int64_t k_b_stride, int64_t k_h_stride, int64_t k_n_stride,
+    const void *v, int64_t v_b_stride, int64_t v_h_stride, int64_t v_n_stride, int64_t B, int64_t H, int64_t Nq, int64_t Nkv,
+    int64_t Dqk, int64_t Dv, float v_scale_max, float sm_scale, void *workspace, int64_t workspace_bytes, ac4k_stream_t stream) {
+  AC4K_REQUIRE(O && q && k && v && workspace, "null pointer argument");
+  AttnQuantArgs a;
+  if (int rc = attention_int8_args(a, B, H, Nq, Nkv, Dqk, Dv)) return rc;
+  AC4K_REQUIRE((((uintptr_t)q | (uintptr_t)k | (uintptr_t)v) & 1) == 0 && ((uintptr_t)workspace & 15) == 0,
+               "q, k, v must be 2-byte aligned and the workspace 16-byte aligned");
+  AC4K_REQUIRE(q_b_stride >= 0 && q_h_stride >= 0 && q_n_stride >= 0 && k_b_stride >= 0 && k_h_stride >= 0 && k_n_stride >= 0 &&
+               v_b_stride >= 0 && v_h_stride >= 0 && v_n_stride >= 0, "strides of q, k and v must not be negative");
+  AC4K_REQUIRE(v_scale_max > 0.0f, "v_scale_max must be positive");
+  const int64_t need = attn_quant_layout(a, workspace);
+  AC4K_REQUIRE(workspace_bytes >= need, "workspace too small: %lld bytes, %lld needed", (long long)workspace_bytes, (long long)need);
+  a.q = {static_cast<const uint16_t *>(q), q_b_stride, q_h_stride, q_n_stride};
+  a.k = {static_cast<const uint16_t *>(k), k_b_stride, k_h_stride, k_n_stride};
+  a.v = {static_cast<const uint16_t *>(v), v_b_stride, v_h_stride, v_n_stride};
+  a.v_smax = v_scale_max;
+  attn_quant_plan(a);
+  launch_attn_quant(a, (hipStream_t)stream);
+  if (int rc = check_launch("ac4k_attention_int8_x_fp8_bf16")) return rc;
+  return ac4k_mha_int8_x_fp8_fwd(O, o_b_stride, o_h_stride, o_n_stride, o_d_stride, a.q8, a.q_sf, AQ_Q_BLOCK, a.k8, a.k_sf, AQ_K_BLOCK,
+                                 a.v8, a.v_sf, B, H, Nq, Nkv, a.Dp, Dv, sm_scale, stream);
 }

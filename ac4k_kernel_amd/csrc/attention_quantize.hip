@@ -1,0 +1,309 @@
+// The quantizers in front of the INT8 x FP8 attention forward as two launches, for the whole-attention entry point
+// (python/ac4k_kernel/ops/attention.py:137-190: K minus its token mean, per-token-block int8 of Q and K, per-channel
+// e4m3 of V with the 16-group swizzle).  Operator by operator the same work is nine launches - mean, subtraction, two
+// block quantizers, and fill / maxima / quantize / finalize for V - and K crosses memory four times:
+//   1. attn_column_stats_kernel     per (head, channel): sum of K and maximum of |V| over a span of tokens, one partial
+//                                   result per span (no atomics, so a call gives the same bits every time)
+//   2. attn_quantize_int8_fp8_kernel  every workgroup adds up the partials of its own channels (a few KB from L2) and
+//                                   quantizes one tile of V, K or Q
+// Both are bound by HBM: 2 (K + V) bytes read in the first, 2 (Q + K + V) read and half of that written in the second.
+// MI355X, quantizers alone: B 1, N 16384, H 40, D 128 (BNHD) 350 -> 250 us = 83 (4.0 TB/s) + 167 (4.5 TB/s), bit-identical
+// operands; a whole attention of 777 queries on 257 keys, B 2, H 12, D 64: 64 -> 26 us, three launches instead of nine.
+#include "attention_quantize.h"
+
+namespace ac4k {
+
+namespace {
+
+constexpr int AQ_COLS = 128;      // channels of a row of partial results (head dims up to 128)
+constexpr int AQ_MAX_SPLITS = 32; // token spans: every tile of the second kernel reads one partial row per span
+constexpr int AQ_MIN_SPAN = 32;
+constexpr int AQ_STAT_WAVES = 16;  // most waves of a workgroup of the first kernel
+
+// Lanes that share one row of a head: eight channels per lane.  The last lane of a head dim that is no multiple of
+// eight is moved back to end at it; channels that two lanes share are computed twice, with the same result.
+__device__ __forceinline__ int aq_lane_shift(int D) { return D > 64 ? 4 : 3; }
+__device__ __forceinline__ int aq_channel(int c, int D) { return c * 8 + 8 <= D ? c * 8 : D - 8; }
+
+__device__ __forceinline__ uint4 aq_load(const uint16_t *p) {
+  const u32x4 v = *reinterpret_cast<const u32x4_elem *>(p);
+  return make_uint4(v.x, v.y, v.z, v.w);
+}
+__device__ __forceinline__ uint4 aq_load_stream(const uint16_t *p) {
+  const u32x4 v = __builtin_nontemporal_load(reinterpret_cast<const u32x4_elem *>(p));
+  return make_uint4(v.x, v.y, v.z, v.w);
+}
+
+// ---- 1. sums of K, maxima of |V| -------------------------------------------------------------------------------
+// A wave instruction reads 1 KB: the rows of neighbouring heads of one token where these are neighbours in memory
+// (BNHD), rows of neighbouring tokens otherwise (BHND).
+template <bool ABSMAX>
+__device__ __forceinline__ void aq_column_stats(const AttnQuantArgs &a, const AttnOperand &t, int N, int D, void *part,
+                                                uint32_t (*red)[64][8]) {
+  const int W = blockDim.x >> 6;
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int ls = aq_lane_shift(D), lpr = 1 << ls, G = 64 >> ls;
+  const bool heads_adjacent = t.s_h < t.s_n && a.H > 1;
+  const int heads = heads_adjacent ? G : 1, HG = (a.H + heads - 1) / heads;
+  const int unit = blockIdx.x;
+  if (unit >= a.nsplit * a.B * HG) return;  // (whole workgroup)
+  const int hg = unit % HG, b = (unit / HG) % a.B, split = unit / (HG * a.B);
+  const int g = lane >> ls, c = lane & (lpr - 1);
+  const int head = heads_adjacent ? hg * G + g : hg;
+  const bool live = head < a.H && c * 8 < D;
+  const int c0 = aq_channel(live ? c : 0, D);
+  const uint16_t *src = t.p + b * t.s_b + (live ? head : 0) * t.s_h + c0;
+  const int beg = split * a.span, end = beg + a.span < N ? beg + a.span : N;
+  const int step = heads_adjacent ? W : W * G;
+  float s[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+  uint32_t m[4] = {0, 0, 0, 0};
+  constexpr int U = 8;  // loads in flight per lane
+  for (int n = beg + (heads_adjacent ? wave : wave * G + g); n < end; n += U * step) {
+    uint4 v[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      v[u] = make_uint4(0, 0, 0, 0);
+      if (live && n + u * step < end) v[u] = aq_load(src + (int64_t)(n + u * step) * t.s_n);
+    }
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const uint32_t w[4] = {v[u].x, v[u].y, v[u].z, v[u].w};
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        if (ABSMAX) {
+          m[i] = __builtin_bit_cast(uint32_t, __builtin_elementwise_max(__builtin_bit_cast(u16x2, m[i]), __builtin_bit_cast(u16x2, w[i] & 0x7fff7fffu)));
+        } else {
+          s[2 * i] += bf16_lo(w[i]);
+          s[2 * i + 1] += bf16_hi(w[i]);
+        }
+      }
+    }
+  }
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    red[wave][lane][2 * i] = ABSMAX ? m[i] & 0xffffu : __float_as_uint(s[2 * i]);
+    red[wave][lane][2 * i + 1] = ABSMAX ? m[i] >> 16 : __float_as_uint(s[2 * i + 1]);
+  }
+  __syncthreads();
+  const int groups = heads_adjacent ? 1 : G;  // lane groups of a wave that hold the same head
+  for (int i = tid; i < heads * lpr * 8; i += 64 * W) {
+    const int l = i >> 3, e = i & 7, oc = l & (lpr - 1), oh = heads_adjacent ? hg * G + (l >> ls) : hg;
+    float sum = 0.f;
+    uint32_t mx = 0;
+    for (int w = 0; w < W; ++w)
+      for (int k = 0; k < groups; ++k) {
+        const uint32_t x = red[w][l + k * lpr][e];
+        if (ABSMAX) mx = umax32(mx, x);
+        else sum += __uint_as_float(x);
+      }
+    if (oh < a.H && oc * 8 < D) {
+      const int64_t at = ((int64_t)split * a.B * a.H + b * a.H + oh) * AQ_COLS + aq_channel(oc, D) + e;
+      if (ABSMAX) static_cast<uint32_t *>(part)[at] = mx;
+      else static_cast<float *>(part)[at] = sum;
+    }
+  }
+}
+
+__global__ __launch_bounds__(64 * AQ_STAT_WAVES) void attn_column_stats_kernel(AttnQuantArgs a) {
+  __shared__ uint32_t red[AQ_STAT_WAVES][64][8];
+  if (blockIdx.y == 0) aq_column_stats<false>(a, a.k, a.Nkv, a.D, a.ksum, red);
+  else aq_column_stats<true>(a, a.v, a.Nkv, a.Dv, a.vmax, red);
+}
+
+// ---- 2. the tiles ----------------------------------------------------------------------------------------------
+// `BLOCK` tokens of one head to int8 with one scale; MEAN: minus the token mean of their channel, both rounded to
+// bf16 as the subtraction of two bf16 tensors rounds them.
+template <int BLOCK, bool MEAN>
+__device__ __forceinline__ void aq_int8_tile(const AttnQuantArgs &a, const AttnOperand &t, int N, int nb, int8_t *y,
+                                             float *scale, int b, int head, int blk, uint32_t *wmax) {
+  const int tid = threadIdx.x;
+  const int ls = aq_lane_shift(a.D), c = tid & ((1 << ls) - 1), r0 = tid >> ls, rstep = 256 >> ls;
+  constexpr int NV = BLOCK / 16;  // vectors per thread with 16 lanes per row (half of them with eight)
+  const bool live = c * 8 < a.D;
+  const int c0 = aq_channel(live ? c : 0, a.D);
+  const int n0 = blk * BLOCK, rows = N - n0 < BLOCK ? N - n0 : BLOCK;
+  const int64_t bh = (int64_t)b * a.H + head;
+  const uint16_t *src = t.p + b * t.s_b + head * t.s_h + (int64_t)n0 * t.s_n + c0;
+  uint4 v[NV];
+#pragma unroll
+  for (int j = 0; j < NV; ++j) {
+    const int r = r0 + j * rstep;
+    v[j] = make_uint4(0, 0, 0, 0);
+    if (live && r < rows) v[j] = aq_load_stream(src + r * t.s_n);
+  }
+  if (MEAN) {
+    float mean[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+    const float *p = a.ksum + bh * AQ_COLS + c0;
+    for (int s = 0; s < a.nsplit; ++s, p += (int64_t)a.B * a.H * AQ_COLS)
+#pragma unroll
+      for (int e = 0; e < 8; ++e) mean[e] += p[e];
+#pragma unroll
+    for (int e = 0; e < 8; ++e) mean[e] = (float)(__bf16)(mean[e] * a.inv_nkv);
+#pragma unroll
+    for (int j = 0; j < NV; ++j) {
+      if (!(live && r0 + j * rstep < rows)) continue;  // rows past the end stay zero
+      uint32_t w[4] = {v[j].x, v[j].y, v[j].z, v[j].w};
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const uint16_t lo = __builtin_bit_cast(uint16_t, (__bf16)(bf16_lo(w[i]) - mean[2 * i]));
+        const uint16_t hi = __builtin_bit_cast(uint16_t, (__bf16)(bf16_hi(w[i]) - mean[2 * i + 1]));
+        w[i] = lo | ((uint32_t)hi << 16);
+      }
+      v[j] = make_uint4(w[0], w[1], w[2], w[3]);
+    }
+  }
+  uint32_t mx = 0;
+#pragma unroll
+  for (int j = 0; j < NV; ++j) mx = umax32(mx, absmax_bf16x8(v[j]));
+  mx = group_umax<64>(mx);
+  if ((tid & 63) == 0) wmax[tid >> 6] = mx;
+  __syncthreads();
+  mx = umax32(umax32(wmax[0], wmax[1]), umax32(wmax[2], wmax[3]));
+  const Int8BlockScale sc(mx);
+  if (tid == 0) scale[bh * nb + blk] = sc.scale;
+  int8_t *dst = y + (bh * N + n0) * a.Dp;
+#pragma unroll
+  for (int j = 0; j < NV; ++j) {
+    const int r = r0 + j * rstep;
+    if (live && r < rows) st_elem_u2(dst + r * a.Dp + c0, sc.quantize8(v[j]));
+  }
+  if (a.Dp != a.D) {  // pad columns
+    const int pad = a.Dp - a.D;
+    for (int i = tid; i < rows * pad; i += 256) dst[(i / pad) * a.Dp + a.D + i % pad] = 0;
+  }
+}
+
+// 64 kv positions per wave, all channels of one head, to e4m3 along kv (the cross-major layout of the quantizers: a lane
+// holds eight channels of 16 stored positions)
+__device__ __forceinline__ void aq_fp8_tile(const AttnQuantArgs &a, int b, int head, int blk) {
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, kb = lane & 3, rg = lane >> 2;
+  const int64_t bh = (int64_t)b * a.H + head;
+  const int k0 = (blk * 4 + wave) * 64 + kb * 16;
+  const bool live = rg * 8 < a.Dv;
+  const int c0 = aq_channel(live ? rg : 0, a.Dv);
+  const uint16_t *src = a.v.p + b * a.v.s_b + head * a.v.s_h + c0;
+  uint4 v[16];
+#pragma unroll
+  for (int i = 0; i < 16; ++i) {
+    const int k = k0 + ((i & 3) >> 1) * 8 + (i >> 2) * 2 + (i & 1);  // the 16-group swizzle
+    v[i] = make_uint4(0, 0, 0, 0);
+    if (live && k < a.Nkv) v[i] = aq_load(src + (int64_t)k * a.v.s_n);
+  }
+  uint32_t mx[8] = {0, 0, 0, 0, 0, 0, 0, 0};
+  const uint32_t *p = a.vmax + bh * AQ_COLS + c0;
+  for (int s = 0; s < a.nsplit; ++s, p += (int64_t)a.B * a.H * AQ_COLS)
+#pragma unroll
+    for (int e = 0; e < 8; ++e) mx[e] = umax32(mx[e], p[e]);
+  if (blk == 0 && wave == 0 && kb == 0) {  // the scales of this head
+    float *sf = a.v_sf + bh * a.Dvp;
+    if (live)
+#pragma unroll
+      for (int e = 0; e < 8; ++e) sf[c0 + e] = bf16_bits_to_f32(mx[e]) / a.v_smax;
+    if (rg == 0)
+      for (int d = a.Dv; d < a.Dvp; ++d) sf[d] = 0.0f / a.v_smax;
+  }
+  if (!live || k0 >= a.Nkv16) return;
+  uint8_t *dst = a.v8 + (bh * a.Dv + c0) * a.Nkv16 + k0;
+#pragma unroll
+  for (int e = 0; e < 8; ++e) {
+    const float amax = bf16_bits_to_f32(mx[e]), recp = a.v_smax / amax;
+    float f[16];
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+      const uint32_t w = (e >> 1) == 0 ? v[i].x : (e >> 1) == 1 ? v[i].y : (e >> 1) == 2 ? v[i].z : v[i].w;
+      f[i] = ((e & 1) ? bf16_hi(w) : bf16_lo(w)) * recp;
+    }
+    uint4 o = make_uint4(f32x4_to_e4m3x4(f[0], f[1], f[2], f[3]), f32x4_to_e4m3x4(f[4], f[5], f[6], f[7]),
+                         f32x4_to_e4m3x4(f[8], f[9], f[10], f[11]), f32x4_to_e4m3x4(f[12], f[13], f[14], f[15]));
+    if (amax == 0.0f) o = make_uint4(0x7f7f7f7fu, 0x7f7f7f7fu, 0x7f7f7f7fu, 0x7f7f7f7fu);  // 0 * inf
+    *reinterpret_cast<uint4 *>(dst + (int64_t)e * a.Nkv16) = o;
+  }
+}
+
+__global__ __launch_bounds__(256) void attn_quantize_int8_fp8_kernel(AttnQuantArgs a) {
+  __shared__ uint32_t wmax[4];
+  uint32_t idx = blockIdx.x;
+  const uint32_t BH = a.B * a.H;
+  // (workgroup index -> tile: the dim that is nearer in memory runs fastest)
+  auto tile = [&](const AttnOperand &t, uint32_t nblk, int &b, int &head, int &blk) {
+    uint32_t bh;
+    if (t.s_h < t.s_n) {
+      head = idx % a.H;
+      blk = (idx / a.H) % nblk;
+      b = idx / (a.H * nblk);
+    } else {
+      blk = idx % nblk;
+      bh = idx / nblk;
+      head = bh % a.H;
+      b = bh / a.H;
+    }
+  };
+  int b, head, blk;
+  const uint32_t nv = BH * a.nvb, nk = BH * a.nkb;
+  if (idx < nv) {
+    tile(a.v, a.nvb, b, head, blk);
+    aq_fp8_tile(a, b, head, blk);
+  } else if (idx < nv + nk) {
+    idx -= nv;
+    tile(a.k, a.nkb, b, head, blk);
+    aq_int8_tile<AQ_K_BLOCK, true>(a, a.k, a.Nkv, a.nkb, a.k8, a.k_sf, b, head, blk, wmax);
+  } else {
+    idx -= nv + nk;
+    tile(a.q, a.nqb, b, head, blk);
+    aq_int8_tile<AQ_Q_BLOCK, false>(a, a.q, a.Nq, a.nqb, a.q8, a.q_sf, b, head, blk, wmax);
+  }
+}
+
+int64_t take(int64_t &at, int64_t bytes) {
+  const int64_t p = at;
+  at += align_up(bytes, 256);
+  return p;
+}
+
+}  // namespace
+
+// Token spans of the first kernel: enough workgroups to have the whole GPU loading (512 of 32 KB in flight each), at
+// least 32 tokens each, and at most 32 spans, because every tile of the second kernel reads one partial row per span.
+void attn_quant_plan(AttnQuantArgs &a) {
+  const int64_t groups = 2 * (int64_t)a.B * ceil_div(a.H, a.k.s_h < a.k.s_n && a.H > 1 ? (a.D > 64 ? 4 : 8) : 1);
+  int64_t nsplit = ceil_div(512, groups);
+  if (nsplit > AQ_MAX_SPLITS) nsplit = AQ_MAX_SPLITS;
+  if (nsplit > ceil_div(a.Nkv, AQ_MIN_SPAN)) nsplit = ceil_div(a.Nkv, AQ_MIN_SPAN);
+  a.span = (int)ceil_div(a.Nkv, nsplit);
+  a.nsplit = (int)ceil_div(a.Nkv, a.span);
+  a.inv_nkv = 1.0f / (float)a.Nkv;
+}
+
+int64_t attn_quant_layout(AttnQuantArgs &a, void *ws) {
+  const int64_t BH = (int64_t)a.B * a.H;
+  a.Dp = (int)align_up(a.D, 16), a.Dvp = (int)align_up(a.Dv, 16), a.Nkv16 = align_up(a.Nkv, 16);
+  a.nqb = (int)ceil_div(a.Nq, AQ_Q_BLOCK), a.nkb = (int)ceil_div(a.Nkv, AQ_K_BLOCK), a.nvb = (int)ceil_div(a.Nkv, 256);
+  uint8_t *w = static_cast<uint8_t *>(ws);
+  int64_t at = 0;
+  a.q8 = reinterpret_cast<int8_t *>(w + take(at, BH * a.Nq * a.Dp));
+  a.k8 = reinterpret_cast<int8_t *>(w + take(at, BH * a.Nkv * a.Dp));
+  a.v8 = w + take(at, BH * a.Dv * a.Nkv16);
+  a.q_sf = reinterpret_cast<float *>(w + take(at, BH * a.nqb * 4));
+  a.k_sf = reinterpret_cast<float *>(w + take(at, BH * a.nkb * 4));
+  a.v_sf = reinterpret_cast<float *>(w + take(at, BH * a.Dvp * 4));
+  // (bound of the plan's spans, so that the size does not depend on the strides)
+  a.ksum = reinterpret_cast<float *>(w + take(at, AQ_MAX_SPLITS * BH * AQ_COLS * 4));
+  a.vmax = reinterpret_cast<uint32_t *>(w + take(at, AQ_MAX_SPLITS * BH * AQ_COLS * 4));
+  return at;
+}
+
+void launch_attn_quant(const AttnQuantArgs &a, hipStream_t st) {
+  auto units = [&](const AttnOperand &t, int D) {
+    const int heads = t.s_h < t.s_n && a.H > 1 ? (D > 64 ? 4 : 8) : 1;
+    return (int64_t)a.nsplit * a.B * ceil_div(a.H, heads);
+  };
+  const int64_t uk = units(a.k, a.D), uv = units(a.v, a.Dv);
+  // Sixteen waves a workgroup where a span lasts them for several rounds of loads: with about two workgroups per CU (more
+  // would be more spans) the loads in flight are what the pass lives on, 116 us with 4 waves, 95 with 8, 83 with 16 for
+  // K and V of 16384 x 40 x 128.  Short spans: eight (one round, 4.9 against 5.6 us at 257 x 12 x 64).
+  const int waves = a.span > 256 ? AQ_STAT_WAVES : 8;
+  hipLaunchKernelGGL(attn_column_stats_kernel, dim3((unsigned)(uk > uv ? uk : uv), 2), dim3(64 * waves), 0, st, a);
+  hipLaunchKernelGGL(attn_quantize_int8_fp8_kernel, dim3((unsigned)((int64_t)a.B * a.H * (a.nvb + a.nkb + a.nqb))), dim3(256), 0, st, a);
+}
+
+}  // namespace ac4k

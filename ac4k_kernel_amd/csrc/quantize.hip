@@ -148,7 +148,6 @@ __device__ __forceinline__ uint4 swizzle_fp8_pair(uint4 v, int lane) {
 // Elements [k, k + 8) of a row of K >= 8 that starts at any element: one 16-byte load at 2-byte alignment (the target
 // allows it).  A row's last, partial vector is loaded eight elements before the row's end instead - nothing behind the
 // row is read - and row_tail_u4 moves its elements into place, zeros behind them.
-typedef u32x4 u32x4_elem __attribute__((aligned(2)));
 __device__ __forceinline__ uint4 ld_row_u4(const uint16_t *row, int64_t k, int64_t K) {
   const u32x4 v = *reinterpret_cast<const u32x4_elem *>(row + (k + 8 <= K ? k : K - 8));
   return make_uint4(v.x, v.y, v.z, v.w);
@@ -644,17 +643,6 @@ enum class RowFmt { FP8, INT8 };
 template <RowFmt FMT>
 __device__ __forceinline__ float load_scale_max(const void *p) {
   return FMT == RowFmt::FP8 ? *static_cast<const float *>(p) : (float)*static_cast<const int32_t *>(p);
-}
-
-// satfinite e4m3 of four floats -> four bytes, element 0 in the low byte.
-__device__ __forceinline__ uint32_t f32x4_to_e4m3x4(float a, float b, float c, float d) {
-  a = __builtin_amdgcn_fmed3f(a, -448.0f, 448.0f);
-  b = __builtin_amdgcn_fmed3f(b, -448.0f, 448.0f);
-  c = __builtin_amdgcn_fmed3f(c, -448.0f, 448.0f);
-  d = __builtin_amdgcn_fmed3f(d, -448.0f, 448.0f);
-  int w = __builtin_amdgcn_cvt_pk_fp8_f32(a, b, 0, false);
-  w = __builtin_amdgcn_cvt_pk_fp8_f32(c, d, w, true);
-  return (uint32_t)w;
 }
 
 __device__ __forceinline__ uint32_t f32_to_s8_sat(float x) {

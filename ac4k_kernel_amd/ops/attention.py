@@ -42,15 +42,20 @@ def _int8_x_fp8_attention(q, k, v, layout, Q_QUANTIZE_BLOCK_SIZE=64, K_QUANTIZE_
         Nq, H = q.shape[1], q.shape[2]
     else:
         H, Nq = q.shape[1], q.shape[2]
+    if out is None:
+        out_shape = (B, Nq, H, Dv) if layout == "BNHD" else (B, H, Nq, Dv)
+        out = torch.empty(out_shape, dtype=torch.bfloat16, device=q.device)
+    bhnd = (lambda t: t.permute(0, 2, 1, 3)) if layout == "BNHD" else (lambda t: t)
+    o_bhnd = bhnd(out)  # the kernel writes through the strides
+    # the operator takes dense V only; everything else goes operator by operator
+    if (Q_QUANTIZE_BLOCK_SIZE, K_QUANTIZE_BLOCK_SIZE) == (64, 128) and v.is_contiguous() and _rocm_ops.attention_int8_x_fp8(
+            o_bhnd, bhnd(q), bhnd(k), bhnd(v), 2.25, 1 / math.sqrt(Dqk)):
+        return out
     n_dim = 1 if layout == "BNHD" else 2
     k = k - k.mean(dim=n_dim, keepdim=True)
     q_int8, q_sf = _int8_quantize(q, layout, n_dim, BLOCK_SIZE=Q_QUANTIZE_BLOCK_SIZE)
     k_int8, k_sf = _int8_quantize(k, layout, n_dim, BLOCK_SIZE=K_QUANTIZE_BLOCK_SIZE)
     v_fp8, v_sf = quantize(v, 3, n_dim, swizzle=True, max_scale=2.25, precision="fp8e4m3")
-    if out is None:
-        out_shape = (B, Nq, H, Dv) if layout == "BNHD" else (B, H, Nq, Dv)
-        out = torch.empty(out_shape, dtype=torch.bfloat16, device=q.device)
-    o_bhnd = out.permute(0, 2, 1, 3) if layout == "BNHD" else out  # the kernel writes through the strides
     mha_int8_x_fp8_fwd(o_bhnd, q_int8, q_sf, Q_QUANTIZE_BLOCK_SIZE, k_int8, k_sf, K_QUANTIZE_BLOCK_SIZE, v_fp8, v_sf,
                        1 / math.sqrt(Dqk))
     return out

@@ -252,6 +252,20 @@ int ac4k_quantize_int8_token_block_bf16(void *y, float *scale, const void *x, in
                                         int64_t N, int64_t D, int64_t s_b, int64_t s_h, int64_t s_n,
                                         int block, ac4k_stream_t stream);
 
+/* Replaces _int8_x_fp8_attention (python/ac4k_kernel/ops/attention.py:137-190) as a whole: q, k, v bf16, addressed as
+ * [B,H,N,D] through their batch, head and token strides (elements; head dim contiguous).  K minus its token mean (bf16
+ * roundings as in the reference), int8 of Q per 64 and of K per 128 tokens, e4m3 of V along the tokens with scale maximum
+ * v_scale_max, then ac4k_mha_int8_x_fp8_fwd.  Dqk, Dv: 8 to 128.  The workspace (16-byte aligned) holds the quantized
+ * operands; its size function returns -1 for sizes the entry point does not take. */
+int64_t ac4k_attention_int8_x_fp8_workspace_bytes(int64_t B, int64_t H, int64_t Nq, int64_t Nkv, int64_t Dqk, int64_t Dv);
+int ac4k_attention_int8_x_fp8_bf16(void *O, int64_t o_b_stride, int64_t o_h_stride, int64_t o_n_stride, int64_t o_d_stride,
+                                   const void *q, int64_t q_b_stride, int64_t q_h_stride, int64_t q_n_stride,
+                                   const void *k, int64_t k_b_stride, int64_t k_h_stride, int64_t k_n_stride,
+                                   const void *v, int64_t v_b_stride, int64_t v_h_stride, int64_t v_n_stride,
+                                   int64_t B, int64_t H, int64_t Nq, int64_t Nkv, int64_t Dqk, int64_t Dv,
+                                   float v_scale_max, float sm_scale, void *workspace, int64_t workspace_bytes,
+                                   ac4k_stream_t stream);
+
 #ifdef __cplusplus
 }
 #endif

@@ -99,6 +99,23 @@ def test_entry_point_on_given_operands():
     assert (store[..., 0] == 0).all() and (store[..., 129] == 0).all()
 
 
+@pytest.mark.parametrize("B,Nq,Nkv,H,D,layout", [(1, 1, 1, 1, 8, "BNHD"), (3, 33, 31, 7, 71, "BNHD"), (2, 65, 257, 12, 64, "BNHD"),
+                                                 (2, 65, 257, 12, 64, "BHND"), (1, 64, 33, 5, 127, "BHND"), (1, 200, 2100, 9, 128, "BNHD"),
+                                                 (11, 100, 77, 12, 65, "BNHD"), (2, 64, 9000, 3, 100, "BHND"), (1, 40, 48, 2, 7, "BNHD")])
+def test_whole_call_equals_operator_by_operator(B, Nq, Nkv, H, D, layout, monkeypatch):
+    """The two-launch quantizers of attention() against the separate operators.  Everything is bit-identical except that
+    a channel mean summed in another order may round to the neighbouring bf16 (2^-9 of the mean, far below a step of
+    int8): at most a few int8 values of that channel move by one step, 1/127 of the block maximum of one score term."""
+    shape = lambda n: (B, n, H, D) if layout == "BNHD" else (B, H, n, D)  # noqa: E731
+    q, k, v = make_input(shape(Nq), seed=1), make_input(shape(Nkv), seed=2).float() + 1.5, make_input(shape(Nkv), seed=3)
+    q, k, v = q.cuda(), k.to(torch.bfloat16).cuda(), v.cuda()
+    got = ops().attention(q, k, v, layout=layout)
+    monkeypatch.setattr(binding(), "attention_int8_x_fp8", lambda *a: False)
+    want = ops().attention(q, k, v, layout=layout)
+    assert (got == want).float().mean().item() > 0.9
+    torch.testing.assert_close(got.float(), want.float(), atol=ATOL, rtol=RTOL)
+
+
 def test_error_behaviour():
     b = binding()
     q = torch.zeros((1, 1, 16, 128), dtype=torch.int8, device="cuda")
