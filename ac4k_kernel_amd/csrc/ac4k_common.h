@@ -13,6 +13,7 @@ namespace ac4k {
 // ---------------------------------------------------------------------------
 int set_error(const char *fmt, ...) __attribute__((format(printf, 1, 2)));
 int check_launch(const char *what);  // hipGetLastError() -> status
+int device_cu_count();               // of the current device; 0 if it cannot be asked
 
 #define AC4K_REQUIRE(cond, ...)                      \
   do {                                               \
@@ -53,6 +54,40 @@ __device__ __forceinline__ void st_elem_u2(void *p, uint2 v) {
 }
 __device__ __forceinline__ void st_stream_u1(void *p, uint32_t v) {
   __builtin_nontemporal_store(v, static_cast<uint32_t *>(p));
+}
+
+template <int N>
+__device__ __forceinline__ void wait_vmcnt() {
+  asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
+}
+
+// Pins a wave-uniform pointer to scalar registers (the halves are taken as unsigned: readfirstlane
+// returns a signed int, and a sign-extended low half would corrupt the high one).
+__device__ __forceinline__ const uint8_t *uniform_ptr(const void *p) {
+  const uint64_t v = (uint64_t)p;
+  const uint32_t lo = __builtin_amdgcn_readfirstlane((uint32_t)v), hi = __builtin_amdgcn_readfirstlane((uint32_t)(v >> 32));
+  return reinterpret_cast<const uint8_t *>(((uint64_t)hi << 32) | lo);
+}
+
+// LDS-DMA: global_load_lds with a scalar 64-bit base, a 32-bit lane offset and the LDS
+// destination of lane 0 in M0 (lane l lands at M0 + size * l).  Issued through inline asm so
+// that the compiler's wait-count insertion does not see these loads: with the builtin it puts
+// s_waitcnt vmcnt(0) in front of every later LDS read, which serialises the prefetch.  The
+// kernel waits with explicit s_waitcnt vmcnt(..) before the barrier that publishes a stage.
+__device__ __forceinline__ void dma16(const void *sbase, uint32_t voff, uint32_t lds_stage, uint32_t lds_piece) {
+  // (wave-uniform by construction; the read keeps them in scalar registers when the compiler cannot tell)
+  lds_stage = (uint32_t)__builtin_amdgcn_readfirstlane((int)lds_stage);
+  lds_piece = (uint32_t)__builtin_amdgcn_readfirstlane((int)lds_piece);
+  sbase = uniform_ptr(sbase);
+  asm volatile("s_add_u32 m0, %0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %2, %3"
+               :: "s"(lds_stage), "s"(lds_piece), "v"(voff), "s"(sbase) : "memory", "scc");
+}
+__device__ __forceinline__ void dma4(const void *sbase, uint32_t voff, uint32_t lds_stage, uint32_t lds_piece) {
+  lds_stage = (uint32_t)__builtin_amdgcn_readfirstlane((int)lds_stage);
+  lds_piece = (uint32_t)__builtin_amdgcn_readfirstlane((int)lds_piece);
+  sbase = uniform_ptr(sbase);
+  asm volatile("s_add_u32 m0, %0, %1\n\ts_nop 0\n\tglobal_load_lds_dword %2, %3"
+               :: "s"(lds_stage), "s"(lds_piece), "v"(voff), "s"(sbase) : "memory", "scc");
 }
 
 // DPP controls (lane i of a 16-lane row receives from ...)

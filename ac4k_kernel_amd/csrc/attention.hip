@@ -42,6 +42,45 @@ struct MhaArgs {
 constexpr float MHA_LOG2E = 1.4426950408889634f;
 constexpr float MHA_P_ALPHA = 2688.0f;  // 1 / (global scale of P)
 
+// Work of a launch: blocks of 256 query rows of all heads, one after the other.  The first `full` blocks are a workgroup
+// each; every block behind them is cut into `tail` workgroups of 256 / tail rows.
+struct MhaWork {
+  uint32_t full, blocks;  // full: a multiple of the number of XCDs; blocks per head
+};
+struct MhaTile {
+  int64_t block, head, b;  // block: in units of the rows of this workgroup
+};
+// Workgroups are dealt to the eight XCDs in turn: a run of consecutive blocks of one head is given to one XCD, whose L2 then
+// fetches the K and V of that head once for all of them, instead of all eight XCDs fetching those of every head
+// (4096 x 40 x 128 int8 x fp8: 262 -> 260 us, 4096 x 8: 59.3 -> 58.3).
+__device__ __forceinline__ MhaTile mha_tile(const MhaWork &w, int64_t H, uint32_t tail) {
+  const uint32_t first = blockIdx.x < w.full ? 0 : w.full, L = blockIdx.x - first;
+  const uint32_t T = blockIdx.x < w.full ? w.full : gridDim.x - w.full;
+  const uint32_t xcd = L & 7, q = T >> 3, rem = T & 7;
+  const uint32_t id = (xcd < rem ? xcd * (q + 1) : rem * (q + 1) + (xcd - rem) * q) + (L >> 3) + first * tail;
+  const uint32_t per_head = w.blocks * tail, bh = id / per_head;
+  return MhaTile{id - bh * per_head, bh % (uint32_t)H, bh / (uint32_t)H};
+}
+
+// Plan of a launch.  A workgroup that splits its tiles over 2 or 4 waves needs `tile_us` per kv tile and `fixed_us` for
+// everything else; what is left after the whole rounds of unsplit workgroups is cut so that the last round ends soonest.
+struct MhaCost {
+  float fixed_us[3], tile_us[3];  // split 1, 2, 4
+};
+static MhaWork mha_plan(const MhaCost &c, int64_t heads, int64_t Nq, int64_t ntiles, int *tail, unsigned *grid) {
+  const int64_t cus = device_cu_count() >= 8 ? device_cu_count() / 8 * 8 : 256;
+  const int64_t blocks = ceil_div(Nq, 256), T = heads * blocks, full = T / cus * cus, left = T - full;
+  float best = 0.0f;
+  *tail = 1;
+  for (int i = 0; i < 3 && left; ++i) {
+    const int64_t wgs = full ? left << i : heads * ceil_div(Nq << i, 256);  // (those without a row end at once)
+    const float us = (float)ceil_div(wgs, cus) * (c.fixed_us[i] + (float)ntiles * c.tile_us[i]);
+    if (i == 0 || us < best) best = us, *tail = 1 << i;
+  }
+  *grid = (unsigned)(full + left * *tail);
+  return MhaWork{(uint32_t)full, (uint32_t)blocks};
+}
+
 // eight nibbles times the block scale -> eight fp16 (exact)
 __device__ __forceinline__ f16x8 mha_decode8(uint32_t w, f16x2 sc) {
   const f16x2 d0 = __builtin_amdgcn_cvt_scalef32_pk_f16_fp4(w, 1.0f, 0) * sc;
@@ -80,45 +119,60 @@ __device__ __forceinline__ uint32_t mha_dword(const uint4 &a, const uint4 &b, in
 }
 
 // both halves of the wave (lanes 0-31 and 32-63) receive op(x of the lower half, x of the upper half)
-__device__ __forceinline__ float mha_halves_max(float x) { return __builtin_fmaxf(x, __shfl_xor(x, 32, 64)); }
-__device__ __forceinline__ float mha_halves_sum(float x) { return x + __shfl_xor(x, 32, 64); }
+// (v_permlane32_swap of x with itself: {lower, lower} and {upper, upper})
+__device__ __forceinline__ float mha_halves_max(float x) {
+  const u32x2 s = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+  return __builtin_fmaxf(__uint_as_float(s.x), __uint_as_float(s.y));
+}
+__device__ __forceinline__ int mha_halves_imax(int x) {
+  const u32x2 s = __builtin_amdgcn_permlane32_swap((uint32_t)x, (uint32_t)x, false, false);
+  return (int)s.x > (int)s.y ? (int)s.x : (int)s.y;
+}
+__device__ __forceinline__ int mha_halves_imin(int x) {
+  const u32x2 s = __builtin_amdgcn_permlane32_swap((uint32_t)x, (uint32_t)x, false, false);
+  return (int)s.x < (int)s.y ? (int)s.x : (int)s.y;
+}
+__device__ __forceinline__ float mha_halves_sum(float x) {
+  const u32x2 s = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+  return __uint_as_float(s.x) + __uint_as_float(s.y);
+}
 
-// Output of one wave: O^T in the MFMA accumulator layout (lane (r, h) owns query row r of the wave: OT[fd][e] is head
-// dim 32 fd + 8 (e >> 2) + 4 h + (e & 3)), already scaled, as bf16 bits in ob[fd][e].  Vector path (rows of O
-// contiguous along d, 16-byte aligned, Dv % 8 == 0): the wave's 32 x 128 tile goes through LDS (8448 bytes at
-// `stage`, free to use: every wave has passed the last barrier of the loop) and leaves as 16-byte pieces of
-// adjacent lanes, whole 256-byte rows; otherwise element by element.
-constexpr int MHA_OUT_PITCH = 264;  // bytes per row of the staged tile (256 + 8: bank spread)
-constexpr int MHA_OUT_LDS = 32 * MHA_OUT_PITCH;
+// Output of one wave: NFD fragments of O^T, head dims from d0 on, in the MFMA accumulator layout (lane (r, h) owns query
+// row r of the wave: OT[fd][e] is head dim d0 + 32 fd + 8 (e >> 2) + 4 h + (e & 3)), already scaled, as bf16 bits in
+// ob[fd][e].  Vector path (rows of O contiguous along d, 16-byte aligned, Dv % 8 == 0): the wave's 32 x (32 NFD) tile goes
+// through LDS (32 * mha_out_pitch(NFD) bytes at `stage`, the wave's own) and leaves as 16-byte pieces of adjacent lanes,
+// whole rows of the tile; otherwise element by element.
+constexpr int mha_out_pitch(int nfd) { return nfd * 64 + 8; }  // bytes per row of the staged tile (8: bank spread)
+constexpr int MHA_OUT_LDS = 32 * mha_out_pitch(4);
+template <int NFD>
 __device__ __forceinline__ void mha_store_rows(uint16_t *o_base, int64_t o_n, int64_t o_d, int o_vec, int64_t row0,
-                                               int64_t Nq, int Dv, int lane, uint8_t *stage,
-                                               const uint16_t (&ob)[4][16]) {
+                                               int64_t Nq, int Dv, int d0, int lane, uint8_t *stage,
+                                               const uint16_t (&ob)[NFD][16]) {
+  constexpr int PITCH = mha_out_pitch(NFD), LPR = NFD * 4;  // lanes per row of the staged tile
   const int r = lane & 31, h = lane >> 5;
   if (o_vec) {
 #pragma unroll
-    for (int fd = 0; fd < 4; ++fd)
+    for (int fd = 0; fd < NFD; ++fd)
 #pragma unroll
-      for (int q4 = 0; q4 < 4; ++q4) {
-        const int d = fd * 32 + q4 * 8 + h * 4;
-        *reinterpret_cast<uint2 *>(stage + r * MHA_OUT_PITCH + d * 2) =
+      for (int q4 = 0; q4 < 4; ++q4)
+        *reinterpret_cast<uint2 *>(stage + r * PITCH + (fd * 32 + q4 * 8 + h * 4) * 2) =
             make_uint2(ob[fd][4 * q4] | ((uint32_t)ob[fd][4 * q4 + 1] << 16), ob[fd][4 * q4 + 2] | ((uint32_t)ob[fd][4 * q4 + 3] << 16));
-      }
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
     __builtin_amdgcn_wave_barrier();
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 #pragma unroll
-    for (int p = 0; p < 8; ++p) {
-      const int row = p * 4 + (lane >> 4), d = (lane & 15) * 8;
-      const uint4 w = *reinterpret_cast<const uint4 *>(stage + row * MHA_OUT_PITCH + d * 2);
-      if (row0 + row < Nq && d < Dv) *reinterpret_cast<uint4 *>(o_base + (row0 + row) * o_n + d) = w;
+    for (int p = 0; p < 2 * NFD; ++p) {
+      const int row = p * (64 / LPR) + lane / LPR, d = (lane % LPR) * 8;
+      const uint4 w = *reinterpret_cast<const uint4 *>(stage + row * PITCH + d * 2);
+      if (row0 + row < Nq && d0 + d < Dv) *reinterpret_cast<uint4 *>(o_base + (row0 + row) * o_n + d0 + d) = w;
     }
   } else if (row0 + r < Nq) {
     uint16_t *orow = o_base + (row0 + r) * o_n;
 #pragma unroll
-    for (int fd = 0; fd < 4; ++fd)
+    for (int fd = 0; fd < NFD; ++fd)
 #pragma unroll
       for (int e = 0; e < 16; ++e) {
-        const int d = fd * 32 + (e >> 2) * 8 + h * 4 + (e & 3);
+        const int d = d0 + fd * 32 + (e >> 2) * 8 + h * 4 + (e & 3);
         if (d < Dv) orow[d * o_d] = ob[fd][e];
       }
   }
@@ -338,8 +392,8 @@ __global__ __launch_bounds__(64 * WAVES, 8 / WAVES) void mha_nvfp4_fwd_kernel(Mh
   for (int fd = 0; fd < 4; ++fd)
 #pragma unroll
     for (int e = 0; e < 16; ++e) ob[fd][e] = __builtin_bit_cast(uint16_t, (__bf16)(OT[fd][e] * scale));
-  mha_store_rows(a.O + b * a.o_b + head * a.o_h, a.o_n, a.o_d, a.o_vec, (int64_t)blockIdx.x * (32 * WAVES) + wave * 32, a.Nq,
-                 a.Dv, lane, mha_lds + wave * MHA_OUT_LDS, ob);
+  mha_store_rows<4>(a.O + b * a.o_b + head * a.o_h, a.o_n, a.o_d, a.o_vec, (int64_t)blockIdx.x * (32 * WAVES) + wave * 32, a.Nq,
+                    a.Dv, 0, lane, mha_lds + wave * MHA_OUT_LDS, ob);
 }
 
 // ---------------------------------------------------------------------------------------------------------------
@@ -375,94 +429,89 @@ typedef int i32x4 __attribute__((ext_vector_type(4)));
 typedef int i32x8 __attribute__((ext_vector_type(8)));
 typedef int i32x16 __attribute__((ext_vector_type(16)));
 
-constexpr int MHA8_PITCH = 144;                    // bytes per 128-byte row in LDS (bank spread)
-constexpr int MHA8_TILE_LDS = 128 * MHA8_PITCH;    // K tile: 128 kv rows; V tile: 128 d rows
-constexpr int MHA8_LDS_BYTES = 4 * MHA8_TILE_LDS;  // K tiles j & 1, then V tiles j & 1
+// LDS: K tiles j & 1 of 128 rows of 128 bytes, the 16-byte piece p of row n at p ^ (n & 7) (bank spread); behind them V
+// tiles j & 1 of 128 d rows at a pitch of 144 bytes
+constexpr int MHA8_K_LDS = 128 * 128;
+constexpr int MHA8_PITCH = 144;
+constexpr int MHA8_V_LDS = 128 * MHA8_PITCH;
+// split tiles: row maxima and sums behind the tile buffers and behind the parts of O of eight waves
+constexpr int mha8_stat_lds(int split) { return split == 1 ? 2 * MHA8_K_LDS + 2 * MHA8_V_LDS : 8 * 16384; }
+constexpr int mha8_lds_bytes(int split) { return mha8_stat_lds(split) + (split == 1 ? 0 : 2 * 512 * 4); }
+static_assert(2 * MHA8_K_LDS + 2 * MHA8_V_LDS <= mha8_stat_lds(2) && 8 * MHA_OUT_LDS <= mha8_lds_bytes(1));
 constexpr float MHA8_EXP_OFFSET = 7.5f;
 
-template <int WAVES>
-__global__ __launch_bounds__(64 * WAVES, 8 / WAVES) void mha_int8_x_fp8_fwd_kernel(Mha8Args a) {
-  constexpr int PARTS = 8 / WAVES, PROWS = 128 / PARTS;
+// Eight waves, two per SIMD; a wave owns 32 query rows and 1 / SPLIT of the kv positions of every tile: SPLIT waves
+// share a group of query rows, 256 / SPLIT rows per workgroup.  What a shared group needs per tile is the row maximum
+// over the whole tile, which goes through LDS with the barrier that ends the tile; the partial sums of O and of the row
+// meet at the end.  The maxima, and with them every rounding of P, are those of the unsplit tile.
+//
+// A tile step is a software pipeline over three tiles, written out in the order in which it issues (the compiler's
+// scheduler keeps an MFMA and the vector instructions that could run under it apart):
+//   O += Vhat . Phat of tile i - 1  |  maxima, exp2, e4m3 of tile i  |  S of tile i + 1, into the registers that the
+//   scores of tile i leave one 32-row fragment after the other
+// K arrives by LDS-DMA two tiles ahead, V through registers one tile ahead.
+// Bound by the issue of vector instructions (about 360 per tile and wave, 65 exp2 and 32 e4m3 conversions of them at half
+// rate: 73 % of the cycles) and, where the whole GPU is busy for long, by power: the clock falls to 2.0 - 2.15 GHz.
+// Kernel alone, before (128 or 256 rows, no split, no pipeline) and now: 16384 x 40 x 128 3447 -> 3314 us (1659 TFLOP/s),
+// 4096 x 40 264 -> 249, 8192 x 4 118 -> 103, 3000 x 24 143 -> 110, 512 x 2 on 8192 keys 114 -> 71, 75600 x 1 3007 -> 2071.
+template <int SPLIT>
+__device__ __forceinline__ void mha_int8_x_fp8_block(const Mha8Args &a, const MhaTile &wg) {
+  constexpr int NF = 4 / SPLIT;             // 32-row fragments of a tile per wave
+  constexpr int NPV = SPLIT == 1 ? 2 : 1;   // P.V operands of 64 kv positions per wave (SPLIT 4: half of one, zeros behind)
+  constexpr int ROWS = 256 / SPLIT;
   extern __shared__ __attribute__((aligned(16))) uint8_t mha_lds[];
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, r = lane & 31, h = lane >> 5;
-  const int srow = threadIdx.x >> 2, sq = threadIdx.x & 3;  // staging role: row of the tile, 32-byte quarter of it
-  const int64_t b = blockIdx.z, head = blockIdx.y, bh = b * a.H + head;
-  const int64_t m = (int64_t)blockIdx.x * (32 * WAVES) + wave * 32 + r;  // this lane's query row
-  const int64_t mq = m < a.Nq ? m : a.Nq - 1;                            // rows past Nq read the last row; never stored
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), r = lane & 31, h = lane >> 5;
+  const int group = wave / SPLIT, part = wave % SPLIT;
+  const int srow = threadIdx.x >> 2, sq = threadIdx.x & 3;  // staging role for V: row of the tile, 32-byte quarter of it
+  if (wg.block * ROWS >= a.Nq) return;
+  const int64_t bh = wg.b * a.H + wg.head;
+  const int64_t m = wg.block * ROWS + group * 32 + r;  // this lane's query row
+  const int64_t mq = m < a.Nq ? m : a.Nq - 1;          // rows past Nq read the last row; never stored
+  const int ntiles = (int)a.nkb;
+  // last kv row and last 16-group of V that exist in the last tile
+  const int k_last = (int)(a.Nkv - 1 - (int64_t)(ntiles - 1) * 128), v_last = (int)(a.Nkv16 - 16 - (int64_t)(ntiles - 1) * 128);
 
-  // head dims below 128: the missing columns of Q and K and the missing rows of V are zeros
-  const int8_t *k_src = a.k + bh * a.Nkv * a.Dp + sq * 32;
-  const uint8_t *v_src = a.v + (bh * a.Dv + srow) * a.Nkv16 + sq * 32;
-  const bool kc0 = sq * 32 < a.Dp, kc1 = sq * 32 + 16 < a.Dp;
-  struct Fetch {
-    uint4 k0, k1, v0, v1;
-  };
-  // rows of K past Nkv and 16-groups of V past its stored length are zeros
-  auto fetch = [&](int64_t n0, Fetch (&fs)[PARTS]) {
+  // What does not exist is read from a place that does, with no test in the loop: rows of K past Nkv repeat the last row
+  // (no other maximum, and P is set to zero), columns of K past the head dim (those of Q are zero), columns of V past its
+  // stored length (P is zero there) and rows of V past Dv (never stored).
+  const int8_t *k_head = a.k + bh * a.Nkv * a.Dp;
+  // K goes from global memory straight into LDS: transfer t of 16 lands in the eight rows from 8 t on, lane l in position
+  // l % 8 of row l / 8, so it fetches the 16-byte piece that belongs there
+  const int kpiece = (lane & 7) ^ (lane >> 4);  // even t; ^ 4 for odd t
+  const uint32_t kcol[2] = {(uint32_t)(kpiece * 16 < a.Dp ? kpiece * 16 : 0), (uint32_t)((kpiece ^ 4) * 16 < a.Dp ? (kpiece ^ 4) * 16 : 0)};
+  const uint32_t krow = (uint32_t)((wave * 16 + (lane >> 3)) * a.Dp);
+  const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint8_t *)mha_lds;
+  auto fetch_k = [&](int tile, int buf) {
+    if (tile >= ntiles) tile = ntiles - 1;
+    const int8_t *src = k_head + (int64_t)tile * 128 * a.Dp;
+    const uint32_t last_off = (uint32_t)((tile < ntiles - 1 ? 127 : k_last) * a.Dp);
 #pragma unroll
-    for (int p = 0; p < PARTS; ++p) {
-      Fetch &f = fs[p];
-      const int64_t n = n0 + srow + p * PROWS;
-      f.k0 = f.k1 = f.v0 = f.v1 = make_uint4(0, 0, 0, 0);
-      if (n < a.Nkv) {
-        const uint4 *src = reinterpret_cast<const uint4 *>(k_src + n * a.Dp);
-        if (kc0) f.k0 = src[0];
-        if (kc1) f.k1 = src[1];
-      }
-      const uint8_t *vs = v_src + p * PROWS * a.Nkv16 + n0;
-      const bool vrow = srow + p * PROWS < a.Dv;
-      if (vrow && n0 + sq * 32 < a.Nkv16) f.v0 = *reinterpret_cast<const uint4 *>(vs);
-      if (vrow && n0 + sq * 32 + 16 < a.Nkv16) f.v1 = *reinterpret_cast<const uint4 *>(vs + 16);
+    for (int j = 0; j < 2; ++j) {
+      const uint32_t off = krow + (uint32_t)(j * 8 * a.Dp);
+      dma16(src, (off < last_off ? off : last_off) + kcol[j], lds0 + buf * MHA8_K_LDS, (uint32_t)((wave * 2 + j) * 1024));
     }
   };
-  // the same for a tile that lies inside Nkv as a whole, head dims of 128: nothing to test, nothing to zero
-  auto fetch_whole = [&](int64_t n0, Fetch (&fs)[PARTS]) {
-#pragma unroll
-    for (int p = 0; p < PARTS; ++p) {
-      Fetch &f = fs[p];
-      const uint4 *src = reinterpret_cast<const uint4 *>(k_src + (n0 + srow + p * PROWS) * a.Dp);
-      f.k0 = src[0];
-      f.k1 = src[1];
-      const uint8_t *vs = v_src + p * PROWS * a.Nkv16 + n0;
-      f.v0 = *reinterpret_cast<const uint4 *>(vs);
-      f.v1 = *reinterpret_cast<const uint4 *>(vs + 16);
-    }
+  struct Piece {
+    uint4 lo, hi;
   };
-  // a whole tile with smaller head dims: columns of K and rows of V that do not exist are read from a place that does
-  // (column 0, row 0) and zeroed by a mask; places and masks do not change from tile to tile
-  const int8_t *k_src0 = kc0 ? k_src : k_src - sq * 32, *k_src1 = kc1 ? k_src + 16 : k_src - sq * 32;
-  const uint32_t km0 = kc0 ? ~0u : 0u, km1 = kc1 ? ~0u : 0u;
-  auto fetch_whole_masked = [&](int64_t n0, Fetch (&fs)[PARTS]) {
-#pragma unroll
-    for (int p = 0; p < PARTS; ++p) {
-      Fetch &f = fs[p];
-      const int64_t n = n0 + srow + p * PROWS;
-      const bool vrow = srow + p * PROWS < a.Dv;
-      const uint32_t vm = vrow ? ~0u : 0u;
-      const uint8_t *vs = (vrow ? v_src + p * PROWS * a.Nkv16 : a.v + bh * a.Dv * a.Nkv16 + sq * 32) + n0;
-      const uint4 k0 = *reinterpret_cast<const uint4 *>(k_src0 + n * a.Dp), k1 = *reinterpret_cast<const uint4 *>(k_src1 + n * a.Dp);
-      const uint4 v0 = *reinterpret_cast<const uint4 *>(vs), v1 = *reinterpret_cast<const uint4 *>(vs + 16);
-      f.k0 = make_uint4(k0.x & km0, k0.y & km0, k0.z & km0, k0.w & km0);
-      f.k1 = make_uint4(k1.x & km1, k1.y & km1, k1.z & km1, k1.w & km1);
-      f.v0 = make_uint4(v0.x & vm, v0.y & vm, v0.z & vm, v0.w & vm);
-      f.v1 = make_uint4(v1.x & vm, v1.y & vm, v1.z & vm, v1.w & vm);
-    }
+  const uint8_t *v_row = a.v + (bh * a.Dv + (srow < a.Dv ? srow : a.Dv - 1)) * a.Nkv16;
+  auto fetch_v = [&](int tile, Piece &v) {  // tiles in turn
+    const int last = tile < ntiles - 1 ? 127 : v_last, c0 = sq * 32 < last ? sq * 32 : last, c1 = sq * 32 + 16 < last ? sq * 32 + 16 : last;
+    v.lo = *reinterpret_cast<const uint4 *>(v_row + c0);
+    v.hi = *reinterpret_cast<const uint4 *>(v_row + c1);
+    v_row += 128;
   };
-  // K rows as they are; V: the thread's two 16-groups (2 sq, 2 sq + 1) regrouped so that the 8-byte pieces of lane
-  // half hh of both are one 16-byte run at 32 sq + 16 hh
-  auto stage = [&](int buf, const Fetch (&fs)[PARTS]) {
-#pragma unroll
-    for (int p = 0; p < PARTS; ++p) {
-      const Fetch &f = fs[p];
-      uint8_t *kd = mha_lds + buf * MHA8_TILE_LDS + (srow + p * PROWS) * MHA8_PITCH + sq * 32;
-      *reinterpret_cast<uint4 *>(kd) = f.k0;
-      *reinterpret_cast<uint4 *>(kd + 16) = f.k1;
-      uint8_t *vd = mha_lds + (2 + buf) * MHA8_TILE_LDS + (srow + p * PROWS) * MHA8_PITCH + sq * 32;
-      *reinterpret_cast<uint4 *>(vd) = make_uint4(f.v0.x, f.v0.y, f.v1.x, f.v1.y);
-      *reinterpret_cast<uint4 *>(vd + 16) = make_uint4(f.v0.z, f.v0.w, f.v1.z, f.v1.w);
-    }
+  // V: the thread's two 16-groups (2 sq, 2 sq + 1) regrouped so that the 8-byte pieces of lane half hh of both are one
+  // 16-byte run at 32 sq + 16 hh
+  auto stage_v = [&](int buf, const Piece &v) {
+    uint8_t *vd = mha_lds + 2 * MHA8_K_LDS + buf * MHA8_V_LDS + srow * MHA8_PITCH + sq * 32;
+    *reinterpret_cast<uint4 *>(vd) = make_uint4(v.lo.x, v.lo.y, v.hi.x, v.hi.y);
+    *reinterpret_cast<uint4 *>(vd + 16) = make_uint4(v.lo.z, v.lo.w, v.hi.z, v.hi.w);
   };
 
+  Piece vp;
+  fetch_k(0, 0);
+  fetch_k(1, 1);
   // Q of the lane's row: the 16 bytes [32 s + 16 h, +16) of k-step s, kept for the whole kernel
   i32x4 QF[4];
 #pragma unroll
@@ -471,163 +520,255 @@ __global__ __launch_bounds__(64 * WAVES, 8 / WAVES) void mha_int8_x_fp8_fwd_kern
     if (s4 * 32 + h * 16 < a.Dp) QF[s4] = *reinterpret_cast<const i32x4 *>(a.q + (bh * a.Nq + mq) * a.Dp + s4 * 32 + h * 16);
   }
   const float qs = (a.sm_scale * MHA_LOG2E) * a.q_sf[bh * a.nqb + mq / a.q_block];
+  const float *ksf_src = a.k_sf + bh * a.nkb;
+  // A negative product of scales turns the order of the scores of a tile around.  The quantizers write none; operands
+  // that hold one anywhere take a loop of their own.
+  bool negative = qs < 0.0f;
+  for (int t = lane; t < ntiles; t += 64) negative |= ksf_src[t] < 0.0f;
+  negative = __builtin_amdgcn_ballot_w64(negative) != 0;
+  float ksf_next = ksf_src[0];
 
   float m_run = -__builtin_inff(), l_run = 0.0f;  // running maximum (held 7.5 below the row maximum) and row sum
+  float alpha = 1.0f;                             // factor of O and l that the last tile's maximum asks for
   f32x16 OT[4];  // O^T: d = 32 fd + 8 (e >> 2) + 4 h + (e & 3), for the lane's query row
 #pragma unroll
-  for (int fd = 0; fd < 4; ++fd)
+  for (int fd = 0; fd < 4; ++fd) OT[fd] = (f32x16)(0.0f);
+  i32x8 P[NPV];  // P of a tile as e4m3, MFMA operands of 64 kv positions
 #pragma unroll
-    for (int e = 0; e < 16; ++e) OT[fd][e] = 0.0f;
-
-  Fetch nxt[PARTS];
-  fetch(0, nxt);
-  stage(0, nxt);
+  for (int j = 0; j < NPV; ++j) P[j] = (i32x8)(0);
+  {  // V of the tile in front of the first one: zeros, and so is its P
+    Piece z;
+    z.lo = z.hi = make_uint4(0, 0, 0, 0);
+    stage_v(1, z);
+  }
+  wait_vmcnt<0>();
   __syncthreads();
-  // one kv tile; TAIL: the last, partial one, whose positions past Nkv are masked (a copy of the code of its own:
-  // as a branch inside one body the masks were turned into selects that every tile paid for)
-  // The scale of a K tile is asked for in front of the loads of the next tile: behind them, its wait would be a wait
-  // for all of them in the middle of the tile.  With eight waves it is loaded a whole tile ahead (the four-wave
-  // kernel has no register left for that).
-  constexpr bool KSF_AHEAD = WAVES == 8;
-  const float *ksf_src = a.k_sf + bh * a.nkb;
-  float ksf_cur = KSF_AHEAD ? ksf_src[0] : 0.0f;
-  auto tile_step = [&](auto tail_tag, auto whole_next_tag, int64_t n0, int buf) {
-    constexpr bool tail = decltype(tail_tag)::value;
-    const int64_t t_next = n0 / 128 + 1 < a.nkb ? n0 / 128 + 1 : a.nkb - 1;
-    const float ksf_load = ksf_src[KSF_AHEAD ? t_next : n0 / 128];
-    asm volatile("" ::: "memory");  // keeps this load in front of the ones below
-    // the next tile travels while this one is multiplied (zeros past the end)
-    if constexpr (decltype(whole_next_tag)::value == 1) fetch_whole(n0 + 128, nxt);
-    else if constexpr (decltype(whole_next_tag)::value == 2) fetch_whole_masked(n0 + 128, nxt);
-    else fetch(n0 + 128, nxt);
-    const uint8_t *kb = mha_lds + buf * MHA8_TILE_LDS + r * MHA8_PITCH + h * 16;
-    const uint8_t *vb = mha_lds + (2 + buf) * MHA8_TILE_LDS + r * MHA8_PITCH + h * 16;
-    const float qk = qs * (KSF_AHEAD ? ksf_cur : ksf_load);
-    if (KSF_AHEAD) ksf_cur = ksf_load;
-    // ---- S^T = K . Q^T for the 128 kv positions of the tile (four 32-row fragments)
-    i32x16 SI[4];
-#pragma unroll
-    for (int s4 = 0; s4 < 4; ++s4)
-#pragma unroll
-      for (int f = 0; f < 4; ++f) {
-        const i32x4 KF = *reinterpret_cast<const i32x4 *>(kb + f * 32 * MHA8_PITCH + s4 * 32);
-        if (s4 == 0)
-          SI[f] = __builtin_amdgcn_mfma_i32_32x32x32_i8(KF, QF[s4], (i32x16)(0), 0, 0, 0);
-        else
-          SI[f] = __builtin_amdgcn_mfma_i32_32x32x32_i8(KF, QF[s4], SI[f], 0, 0, 0);
-      }
-    // ---- online softmax of the lane's row: its 64 values here, the other 64 in the lane 32 away
-    float ST[4][16];
-#pragma unroll
-    for (int f = 0; f < 4; ++f)
-#pragma unroll
-      for (int e = 0; e < 16; ++e) ST[f][e] = (float)SI[f][e];
-    const int left = (int)(a.Nkv - n0) - h * 4;  // kv positions of this tile that exist, seen from the lane's first one
-    if (tail) {  // positions past Nkv take no part in the maximum
-#pragma unroll
-      for (int f = 0; f < 4; ++f)
-#pragma unroll
-        for (int e = 0; e < 16; ++e)
-          if (f * 32 + (e >> 2) * 8 + (e & 3) >= left) ST[f][e] = -__builtin_inff();
-    }
-    // the maximum of s = float(S) * qk is taken over float(S): qk >= 0 keeps the order, qk < 0 reverses it
-    float hi = -__builtin_inff(), lo = __builtin_inff();
-#pragma unroll
-    for (int f = 0; f < 4; ++f)
-#pragma unroll
-      for (int e = 0; e < 16; ++e) hi = __builtin_fmaxf(hi, ST[f][e]);
-    if (qk < 0.0f) {
-      asm volatile("" ::: "memory");
-#pragma unroll
-      for (int f = 0; f < 4; ++f)
-#pragma unroll
-        for (int e = 0; e < 16; ++e)
-          lo = __builtin_fminf(lo, ST[f][e] == -__builtin_inff() ? __builtin_inff() : ST[f][e]);
-    }
-    const float smax = qk < 0.0f ? mha_halves_max(lo * qk) : mha_halves_max(hi * qk);
-    const float m_new = __builtin_fmaxf(smax - MHA8_EXP_OFFSET, m_run);
-    float lsum = 0.0f;
-#pragma unroll
-    for (int f = 0; f < 4; ++f)
-#pragma unroll
-      for (int e = 0; e < 16; ++e) {
-        ST[f][e] = __builtin_amdgcn_exp2f(__builtin_fmaf(ST[f][e], qk, -m_new));  // p <= 2^7.5
-        lsum += ST[f][e];
-      }
-    if (tail) {  // p of the masked positions is 0 whatever qk is (-inf * 0 would be NaN)
-      lsum = 0.0f;
-#pragma unroll
-      for (int f = 0; f < 4; ++f)
-#pragma unroll
-        for (int e = 0; e < 16; ++e) {
-          if (f * 32 + (e >> 2) * 8 + (e & 3) >= left) ST[f][e] = 0.0f;
-          lsum += ST[f][e];
-        }
-    }
-    const float l_new = mha_halves_sum(lsum);
-    const float alpha = __builtin_amdgcn_exp2f(m_run - m_new);
-    l_run = __builtin_fmaf(l_run, alpha, l_new);
-    m_run = m_new;
+
+  i32x16 SI[NF];  // S^T of the tile at hand
+  auto rescale = [&]() {
     if (__builtin_amdgcn_ballot_w64(alpha != 1.0f)) {  // else no row of this wave raised its maximum
 #pragma unroll
       for (int fd = 0; fd < 4; ++fd)
 #pragma unroll
         for (int e = 0; e < 16; ++e) OT[fd][e] *= alpha;
     }
-    // ---- P -> e4m3, O^T += Vhat . Phat^T: one MFMA (k = 64: v_mfma_scale_f32_32x32x64_f8f6f4 with unit scales; lane
-    // half h supplies 32 of the 64 k slots) per 64 kv positions and 32 rows of d
+  };
+  // O^T += Vhat . Phat^T: one MFMA (k = 64: v_mfma_scale_f32_32x32x64_f8f6f4 with unit scales; lane half h supplies 32
+  // of the 64 k slots) per 64 kv positions and 32 rows of d; step st = 4 (64 kv positions) + (32 rows of d)
+  const uint8_t *v_lane = mha_lds + 2 * MHA8_K_LDS + r * MHA8_PITCH + h * 16 + part * NF * 32;
+  auto v_operand = [&](int buf, int st) {
+    const uint8_t *p = v_lane + buf * MHA8_V_LDS + (st & 3) * 32 * MHA8_PITCH + (st >> 2) * 64;
+    const uint4 va = *reinterpret_cast<const uint4 *>(p);
+    const uint4 vc = SPLIT == 4 ? make_uint4(0, 0, 0, 0) : *reinterpret_cast<const uint4 *>(p + 32);
+    return (i32x8){(int)va.x, (int)va.y, (int)va.z, (int)va.w, (int)vc.x, (int)vc.y, (int)vc.z, (int)vc.w};
+  };
+  auto pv_mfma = [](i32x8 v, i32x8 p, f32x16 o) {
+    return __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(v, p, o, 0, 0, 0, 0x7f7f7f7f, 0, 0x7f7f7f7f);
+  };
+  // K for step t = 4 (fragment of 32 kv positions) + (32 columns) of S^T = K . Q^T
+  const int kswz = (part * NF * 32 + r) * 128 + ((h ^ ((r >> 1) & 7)) << 4);
+  auto k_rows = [&](int buf, const uint8_t *(&kb)[4]) {
 #pragma unroll
-    for (int j2 = 0; j2 < 2; ++j2) {
-      i32x8 PF;
+    for (int s4 = 0; s4 < 4; ++s4) kb[s4] = mha_lds + buf * MHA8_K_LDS + (kswz ^ (s4 * 32));
+  };
+  auto k_operand = [](const uint8_t *const (&kb)[4], int t) {
+    return *reinterpret_cast<const i32x4 *>(kb[t & 3] + (t >> 2) * 4096);
+  };
+  // maxima (minima) of a tile's parts, two tiles in turn: [tile & 1][max, min][group][part][row]
+  int *mx_lds = reinterpret_cast<int *>(mha_lds + mha8_stat_lds(SPLIT)) + group * (SPLIT * 32) + r;
+  auto part_extremum = [&](auto negative_tag, int parity) {
+    constexpr bool NEG = decltype(negative_tag)::value;
+    int hi = SI[0][0], lo = SI[0][0];
 #pragma unroll
-      for (int g4 = 0; g4 < 4; ++g4) {  // the lane's four 16-group halves of these 64 positions, in the stored order of V:
-        const float *pe = &ST[2 * j2 + (g4 >> 1)][8 * (g4 & 1)];  // e = 8 (g4 & 1) + {0, 1, 4, 5, 2, 3, 6, 7}
-        int w0 = __builtin_amdgcn_cvt_pk_fp8_f32(pe[0], pe[1], 0, false);
-        w0 = __builtin_amdgcn_cvt_pk_fp8_f32(pe[4], pe[5], w0, true);
-        int w1 = __builtin_amdgcn_cvt_pk_fp8_f32(pe[2], pe[3], 0, false);
-        w1 = __builtin_amdgcn_cvt_pk_fp8_f32(pe[6], pe[7], w1, true);
-        PF[2 * g4] = w0;
-        PF[2 * g4 + 1] = w1;
+    for (int f = 0; f < NF; ++f)
+#pragma unroll
+      for (int e = 0; e < 16; ++e) {
+        hi = SI[f][e] > hi ? SI[f][e] : hi;
+        if (NEG) lo = SI[f][e] < lo ? SI[f][e] : lo;
       }
+    mx_lds[parity * 512 + part * 32] = mha_halves_imax(hi);  // (both halves of the wave write the same value)
+    if (NEG) mx_lds[parity * 512 + 256 + part * 32] = mha_halves_imin(lo);
+  };
+  {
+    const uint8_t *kb[4];
+    k_rows(0, kb);
 #pragma unroll
-      for (int fd = 0; fd < 4; ++fd) {
-        const uint4 va = *reinterpret_cast<const uint4 *>(vb + fd * 32 * MHA8_PITCH + (2 * j2) * 32);
-        const uint4 vc = *reinterpret_cast<const uint4 *>(vb + fd * 32 * MHA8_PITCH + (2 * j2 + 1) * 32);
-        const i32x8 VF = {(int)va.x, (int)va.y, (int)va.z, (int)va.w, (int)vc.x, (int)vc.y, (int)vc.z, (int)vc.w};
-        OT[fd] = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(VF, PF, OT[fd], 0, 0, 0, 0x7f7f7f7f, 0, 0x7f7f7f7f);
+    for (int t = 0; t < 4 * NF; ++t)
+      SI[t >> 2] = __builtin_amdgcn_mfma_i32_32x32x32_i8(k_operand(kb, t), QF[t & 3], (t & 3) == 0 ? (i32x16)(0) : SI[t >> 2], 0, 0, 0);
+  }
+  if constexpr (SPLIT > 1) part_extremum(std::true_type{}, 0);
+  __syncthreads();
+
+  // One kv tile i.  TAIL: the last, partial one, where P of the positions past Nkv is zero.
+  auto tile_step = [&](auto negative_tag, auto tail_tag, int i) {
+    constexpr bool NEG = decltype(negative_tag)::value, TAIL = decltype(tail_tag)::value;
+    const int buf = i & 1;
+    float qk = qs * ksf_next;
+    // (here, not behind the loads below: the compiler does not count the transfers of K, and its wait for a load in front of
+    // them would be a wait for them too)
+    asm volatile("" : "+v"(qk));
+    ksf_next = ksf_src[i + 1 < ntiles ? i + 1 : i];
+    asm volatile("" ::: "memory");
+    fetch_k(i + 2, buf);
+    fetch_v(i, vp);
+    rescale();
+    // ---- maxima.  The maximum of s = float(S) * qk is taken over the integers S (the conversion keeps their order):
+    // qk >= 0 keeps it too, qk < 0 reverses it.  SPLIT 1: under them the first half of O of the tile before.
+    i32x8 VF[2];
+    VF[0] = v_operand(buf ^ 1, 0);
+    VF[1] = v_operand(buf ^ 1, 1);
+    int hi = SI[0][0], lo = SI[0][0];
+    if constexpr (SPLIT == 1) {
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int st = 0; st < 4; ++st) {
+        OT[st] = pv_mfma(VF[st & 1], P[0], OT[st]);
+        VF[st & 1] = v_operand(buf ^ 1, st + 2);
+#pragma unroll
+        for (int e = 0; e < 16; ++e) {
+          hi = SI[st][e] > hi ? SI[st][e] : hi;
+          if (NEG) lo = SI[st][e] < lo ? SI[st][e] : lo;
+        }
+        asm volatile("" : "+v"(hi));
+        __builtin_amdgcn_sched_barrier(0);
+      }
+      hi = mha_halves_imax(hi);
+      if (NEG) lo = mha_halves_imin(lo);
+    } else {
+      hi = mx_lds[buf * 512];
+      if (NEG) lo = mx_lds[buf * 512 + 256];
+#pragma unroll
+      for (int q = 1; q < SPLIT; ++q) {
+        const int up = mx_lds[buf * 512 + q * 32];
+        hi = up > hi ? up : hi;
+        if (NEG) {
+          const int down = mx_lds[buf * 512 + 256 + q * 32];
+          lo = down < lo ? down : lo;
+        }
       }
     }
-    stage(buf ^ 1, nxt);
+    const float smax = (float)(NEG && qk < 0.0f ? lo : hi) * qk;
+    const float m_new = __builtin_fmaxf(smax - MHA8_EXP_OFFSET, m_run);
+    alpha = __builtin_amdgcn_exp2f(m_run - m_new);
+    m_run = m_new;
+    // ---- P of this tile, under it (the rest of) O of the tile before and S of the next one
+    const int left = k_last + 1 - part * NF * 32 - h * 4;  // TAIL: kv positions that exist, from the lane's first one on
+    const uint8_t *kb[4];
+    k_rows(buf ^ 1, kb);
+    float lsum = 0.0f;
+    int w0, w1;
+    i32x8 PN[NPV];  // P of this tile (SPLIT 1 and 2 write all of it)
+#pragma unroll
+    for (int j = 0; j < NPV; ++j) PN[j] = P[j];
+    i32x4 KF[2];
+#pragma unroll
+    for (int st = 0; st < 4 * NF + 4; ++st) {  // step st: P of the st-th group of four scores; an O part or S part st - 4
+      if (st < 4) {
+        OT[st] = pv_mfma(VF[st & 1], P[NPV - 1], OT[st]);
+        if (st < 2) VF[st & 1] = v_operand(buf ^ 1, (NPV - 1) * 4 + st + 2);
+        else KF[st & 1] = k_operand(kb, st - 2);
+      } else {
+        const int t = st - 4, f = t >> 2, s4 = t & 3;
+        SI[f] = __builtin_amdgcn_mfma_i32_32x32x32_i8(KF[t & 1], QF[s4], s4 == 0 ? (i32x16)(0) : SI[f], 0, 0, 0);
+        if (t + 2 < 4 * NF) KF[t & 1] = k_operand(kb, t + 2);
+      }
+      if (st < 4 * NF) {
+        const int f = st >> 2, q = st & 3;
+        float p[4];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          p[e] = __builtin_amdgcn_exp2f(__builtin_fmaf((float)SI[f][4 * q + e], qk, -m_new));  // p <= 2^7.5
+          if (TAIL && f * 32 + q * 8 + e >= left) p[e] = 0.0f;
+          lsum += p[e];
+        }
+        // the lane's two 16-group halves of the fragment, in the stored order of V: e = {0, 1, 4, 5, 2, 3, 6, 7}
+        if (q & 1) {
+          w0 = __builtin_amdgcn_cvt_pk_fp8_f32(p[0], p[1], w0, true);
+          w1 = __builtin_amdgcn_cvt_pk_fp8_f32(p[2], p[3], w1, true);
+        } else {
+          asm volatile("" : "=v"(w0), "=v"(w1));  // (any value: both halves are written)
+          w0 = __builtin_amdgcn_cvt_pk_fp8_f32(p[0], p[1], w0, false);
+          w1 = __builtin_amdgcn_cvt_pk_fp8_f32(p[2], p[3], w1, false);
+        }
+        asm volatile("" : "+v"(lsum), "+v"(w0), "+v"(w1));
+        if (q & 1) {
+          PN[f >> 1][4 * (f & 1) + 2 * (q >> 1)] = w0;
+          PN[f >> 1][4 * (f & 1) + 2 * (q >> 1) + 1] = w1;
+        }
+      }
+      __builtin_amdgcn_sched_barrier(0);
+    }
+#pragma unroll
+    for (int j = 0; j < NPV; ++j) P[j] = PN[j];
+    l_run = __builtin_fmaf(l_run, alpha, mha_halves_sum(lsum));
+    if constexpr (SPLIT > 1) part_extremum(negative_tag, buf ^ 1);
+    stage_v(buf, vp);
+    wait_vmcnt<0>();  // the transfers of K
     __syncthreads();
   };
-  int buf = 0;
-  int64_t n0 = 0;
-  using FetchTested = std::integral_constant<int, 0>;
-  using FetchWhole = std::integral_constant<int, 1>;
-  using FetchWholeMasked = std::integral_constant<int, 2>;
-  if (a.Dp == 128 && a.Dv == 128)  // tiles followed by a whole tile: the fetch without tests
-    for (; n0 + 256 <= a.Nkv; n0 += 128, buf ^= 1) tile_step(std::false_type{}, FetchWhole{}, n0, buf);
-  else if constexpr (WAVES == 8)  // (the four-wave kernel has no registers to spare for a third copy of the loop)
-    for (; n0 + 256 <= a.Nkv; n0 += 128, buf ^= 1) tile_step(std::false_type{}, FetchWholeMasked{}, n0, buf);
-  for (; n0 + 128 <= a.Nkv; n0 += 128, buf ^= 1) tile_step(std::false_type{}, FetchTested{}, n0, buf);
-  if (n0 < a.Nkv) tile_step(std::true_type{}, FetchTested{}, n0, buf);
+  auto all_tiles = [&](auto negative_tag) {
+    int i = 0;
+    for (; i < (int)(a.Nkv / 128); ++i) tile_step(negative_tag, std::false_type{}, i);
+    if (i < ntiles) tile_step(negative_tag, std::true_type{}, i);
+  };
+  // (the probability keeps the registers of the loop that runs)
+  if (__builtin_expect_with_probability(negative, 0, 0.99999)) all_tiles(std::true_type{});
+  else all_tiles(std::false_type{});
+  rescale();
+#pragma unroll
+  for (int st = 0; st < 4 * NPV; ++st) OT[st & 3] = pv_mfma(v_operand((ntiles - 1) & 1, st), P[st >> 2], OT[st & 3]);
+  __syncthreads();  // what follows lies over the tile buffers
+
+  // The parts of O meet: every wave leaves its part in LDS and adds up, in order, those of 128 / SPLIT head dims.
+  constexpr int NFD = 4 / SPLIT;
+  const int d0 = part * NFD * 32;
+  if constexpr (SPLIT > 1) {
+    float *o_lds = reinterpret_cast<float *>(mha_lds) + lane;  // [wave][64 values][lane]
+    float *l_lds = reinterpret_cast<float *>(mha_lds + mha8_stat_lds(SPLIT)) + group * (SPLIT * 32) + r;
+#pragma unroll
+    for (int fd = 0; fd < 4; ++fd)
+#pragma unroll
+      for (int e = 0; e < 16; ++e) o_lds[wave * 4096 + (fd * 16 + e) * 64] = OT[fd][e];
+    l_lds[part * 32] = l_run;
+    __syncthreads();
+    l_run = 0.0f;
+#pragma unroll
+    for (int q = 0; q < SPLIT; ++q) {
+#pragma unroll
+      for (int fd = 0; fd < NFD; ++fd)
+#pragma unroll
+        for (int e = 0; e < 16; ++e) {
+          const float o = o_lds[(group * SPLIT + q) * 4096 + ((part * NFD + fd) * 16 + e) * 64];
+          OT[fd][e] = q == 0 ? o : OT[fd][e] + o;
+        }
+      l_run += l_lds[q * 32];
+    }
+    __syncthreads();  // the staged output lies over the parts
+  }
 
   // ---- O = O * ((1 / l) * v_sf[d]) -> bf16
   const float rl = 1.0f / l_run;
   const float *vsf = a.v_sf + bh * a.Dvp;
-  uint16_t ob[4][16];
+  uint16_t ob[NFD][16];
 #pragma unroll
-  for (int fd = 0; fd < 4; ++fd)
+  for (int fd = 0; fd < NFD; ++fd)
 #pragma unroll
     for (int q4 = 0; q4 < 4; ++q4) {
-      const int d = fd * 32 + q4 * 8 + h * 4;  // four consecutive head dims; the scale row is padded to 16
+      const int d = d0 + fd * 32 + q4 * 8 + h * 4;  // four consecutive head dims; the scale row is padded to 16
       const float4 sv = d < a.Dvp ? *reinterpret_cast<const float4 *>(vsf + d) : make_float4(0.f, 0.f, 0.f, 0.f);
       const float sc[4] = {rl * sv.x, rl * sv.y, rl * sv.z, rl * sv.w};
 #pragma unroll
       for (int e = 0; e < 4; ++e) ob[fd][4 * q4 + e] = __builtin_bit_cast(uint16_t, (__bf16)(OT[fd][4 * q4 + e] * sc[e]));
     }
-  mha_store_rows(a.O + b * a.o_b + head * a.o_h, a.o_n, a.o_d, a.o_vec, (int64_t)blockIdx.x * (32 * WAVES) + wave * 32, a.Nq,
-                 a.Dv, lane, mha_lds + wave * MHA_OUT_LDS, ob);
+  mha_store_rows<NFD>(a.O + wg.b * a.o_b + wg.head * a.o_h, a.o_n, a.o_d, a.o_vec, wg.block * ROWS + group * 32, a.Nq, a.Dv, d0,
+                      lane, mha_lds + wave * MHA_OUT_LDS, ob);
+}
+
+// (two bodies in one kernel, so that the workgroups of the last round start as the ones in front of them end)
+template <int TAIL>
+__global__ __launch_bounds__(512, 1) void mha_int8_x_fp8_fwd_kernel(Mha8Args a, MhaWork w) {
+  if (TAIL == 1 || blockIdx.x < w.full) mha_int8_x_fp8_block<1>(a, mha_tile(w, a.H, 1));
+  else mha_int8_x_fp8_block<TAIL>(a, mha_tile(w, a.H, TAIL));
 }
 
 // Per-token-block int8 quantizer in front of it (python/ac4k_kernel/ops/attention.py:18-99, a Triton kernel in the
@@ -751,30 +892,32 @@ extern "C" __attribute__((visibility("default"))) int ac4k_mha_int8_x_fp8_fwd(
   AC4K_REQUIRE(Dqk >= 16 && Dv >= 1, "Dqk and Dv must be positive");
   AC4K_REQUIRE((((uintptr_t)q | (uintptr_t)k | (uintptr_t)v | (uintptr_t)v_sf) & 15) == 0,
                "q, k, v and v_sf must be 16-byte aligned");
-  AC4K_REQUIRE(H <= 65535 && B <= 65535 && ceil_div(Nq, 128) < (1ll << 31), "problem too large");
+  AC4K_REQUIRE(H <= 65535 && B <= 65535 && ceil_div(Nq, 128) < (1ll << 31) && B * H * ceil_div(Nq, 256) < (1ll << 29), "problem too large");
   AC4K_REQUIRE(o_b_stride >= 0 && o_h_stride >= 0 && o_n_stride >= 1 && o_d_stride >= 1, "strides of O must be positive");
   Mha8Args a{static_cast<uint16_t *>(O), o_b_stride, o_h_stride, o_n_stride, o_d_stride,
              static_cast<const int8_t *>(q), static_cast<const int8_t *>(k), static_cast<const uint8_t *>(v),
              q_sf, k_sf, v_sf, H, Nq, Nkv, align_up(Nkv, 16), ceil_div(Nq, q_quantize_block_size), ceil_div(Nkv, 128),
              (int)Dqk, (int)Dv, (int)align_up(Dv, 16), q_quantize_block_size, sm_scale,
              (o_d_stride == 1 && Dv % 8 == 0 && ((uintptr_t)O & 15) == 0 && o_b_stride % 8 == 0 && o_h_stride % 8 == 0 && o_n_stride % 8 == 0) ? 1 : 0};
-  const bool wide = ceil_div(Nq, 256) * H * B >= 192 || ceil_div(Nq, 128) * H * B <= ceil_div(Nq, 256) * H * B;
-  auto kern = wide ? mha_int8_x_fp8_fwd_kernel<8> : mha_int8_x_fp8_fwd_kernel<4>;
+  // measured: 512 x 2 x 128 to 8192 x 4 x 128 on 4096 and 8192 keys, one round
+  static constexpr MhaCost cost{{4.5f, 6.0f, 5.0f}, {2.35f, 1.45f, 1.05f}};
+  int tail = 1;
+  unsigned grid = 0;
+  const MhaWork work = mha_plan(cost, B * H, Nq, ceil_div(Nkv, 128), &tail, &grid);
+  const int idx = tail >> 1, lds = mha8_lds_bytes(tail);
+  auto kern = tail == 1 ? mha_int8_x_fp8_fwd_kernel<1> : tail == 2 ? mha_int8_x_fp8_fwd_kernel<2> : mha_int8_x_fp8_fwd_kernel<4>;
   {  // more than 64 KB of dynamic LDS has to be allowed once per device and kernel
-    static std::atomic<uint32_t> lds_done[2] = {{0}, {0}};
+    static std::atomic<uint32_t> lds_done[3] = {{0}, {0}, {0}};
     int dev = 0;
     if (hipGetDevice(&dev) != hipSuccess) dev = 0;
     const uint32_t bit = 1u << (dev & 31);
-    if (!(lds_done[wide].load(std::memory_order_relaxed) & bit)) {
-      hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(kern), hipFuncAttributeMaxDynamicSharedMemorySize,
-                                         MHA8_LDS_BYTES);
-      if (e != hipSuccess) return set_error("hipFuncSetAttribute(LDS=%d): %s", MHA8_LDS_BYTES, hipGetErrorString(e));
-      lds_done[wide].fetch_or(bit, std::memory_order_relaxed);
+    if (!(lds_done[idx].load(std::memory_order_relaxed) & bit)) {
+      hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, lds);
+      if (e != hipSuccess) return set_error("hipFuncSetAttribute(LDS=%d): %s", lds, hipGetErrorString(e));
+      lds_done[idx].fetch_or(bit, std::memory_order_relaxed);
     }
   }
-  const int rows = wide ? 256 : 128;
-  hipLaunchKernelGGL(kern, dim3((unsigned)ceil_div(Nq, rows), (unsigned)H, (unsigned)B), dim3(rows * 2), MHA8_LDS_BYTES,
-                     (hipStream_t)stream, a);
+  hipLaunchKernelGGL(kern, dim3(grid), dim3(512), lds, (hipStream_t)stream, a, work);
   return check_launch("ac4k_mha_int8_x_fp8_fwd");
 }
 

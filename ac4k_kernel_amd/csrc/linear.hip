@@ -283,40 +283,6 @@ struct PLayout {               // byte offsets inside one LDS stage; PS stages
   static_assert(LDS_BYTES <= 160 * 1024, "stages must fit in the CU's LDS");
 };
 
-template <int N>
-__device__ __forceinline__ void wait_vmcnt() {
-  asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
-}
-
-// Pins a wave-uniform pointer to scalar registers (the halves are taken as unsigned: readfirstlane
-// returns a signed int, and a sign-extended low half would corrupt the high one).
-__device__ __forceinline__ const uint8_t *uniform_ptr(const void *p) {
-  const uint64_t v = (uint64_t)p;
-  const uint32_t lo = __builtin_amdgcn_readfirstlane((uint32_t)v), hi = __builtin_amdgcn_readfirstlane((uint32_t)(v >> 32));
-  return reinterpret_cast<const uint8_t *>(((uint64_t)hi << 32) | lo);
-}
-
-// LDS-DMA: global_load_lds with a scalar 64-bit base, a 32-bit lane offset and the LDS
-// destination of lane 0 in M0 (lane l lands at M0 + size * l).  Issued through inline asm so
-// that the compiler's wait-count insertion does not see these loads: with the builtin it puts
-// s_waitcnt vmcnt(0) in front of every later LDS read, which serialises the prefetch.  The
-// kernel waits with explicit s_waitcnt vmcnt(..) before the barrier that publishes a stage.
-__device__ __forceinline__ void dma16(const void *sbase, uint32_t voff, uint32_t lds_stage, uint32_t lds_piece) {
-  // (wave-uniform by construction; the read keeps them in scalar registers when the compiler cannot tell)
-  lds_stage = (uint32_t)__builtin_amdgcn_readfirstlane((int)lds_stage);
-  lds_piece = (uint32_t)__builtin_amdgcn_readfirstlane((int)lds_piece);
-  sbase = uniform_ptr(sbase);
-  asm volatile("s_add_u32 m0, %0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %2, %3"
-               :: "s"(lds_stage), "s"(lds_piece), "v"(voff), "s"(sbase) : "memory", "scc");
-}
-__device__ __forceinline__ void dma4(const void *sbase, uint32_t voff, uint32_t lds_stage, uint32_t lds_piece) {
-  lds_stage = (uint32_t)__builtin_amdgcn_readfirstlane((int)lds_stage);
-  lds_piece = (uint32_t)__builtin_amdgcn_readfirstlane((int)lds_piece);
-  sbase = uniform_ptr(sbase);
-  asm volatile("s_add_u32 m0, %0, %1\n\ts_nop 0\n\tglobal_load_lds_dword %2, %3"
-               :: "s"(lds_stage), "s"(lds_piece), "v"(voff), "s"(sbase) : "memory", "scc");
-}
-
 template <int MI, int NJ>
 struct DecFrags {
   f16x8 a[MI], b[NJ];

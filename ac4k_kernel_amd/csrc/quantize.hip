@@ -1212,18 +1212,6 @@ static std::atomic<int64_t> g_sync_timeout_ticks{20000};
 enum QuantPath { QPATH_NONE = 0, QPATH_SMALL = 1, QPATH_ONEPASS = 2, QPATH_TWO_KERNEL = 3 };
 static thread_local int g_last_quantize_path = QPATH_NONE;
 
-static int device_cu_count() {
-  static std::atomic<int> cached[64];
-  int dev = 0;
-  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return 0;
-  int n = cached[dev].load();
-  if (n == 0) {
-    if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess) return 0;
-    cached[dev].store(n);
-  }
-  return n;
-}
-
 struct OnePassLaunch {
   int slot;
   uint32_t tag, seq;

@@ -116,6 +116,28 @@ def test_whole_call_equals_operator_by_operator(B, Nq, Nkv, H, D, layout, monkey
     torch.testing.assert_close(got.float(), want.float(), atol=ATOL, rtol=RTOL)
 
 
+# Launches whose last round is cut: workgroups of 256, 128 and 64 query rows (one round; 256 of 256 rows and a rest of 4 and
+# 124 blocks), one kv tile and partial last tiles, groups without a row of their own; with scales of both signs, which
+# turn the order of the scores around.
+@pytest.mark.parametrize("H,Nq,Nkv", [(1, 50, 20), (2, 300, 129), (3, 129, 1030), (40, 513, 256), (130, 300, 200), (190, 260, 300)])
+@pytest.mark.parametrize("signs", [False, True])
+def test_split_plans_and_negative_scales(H, Nq, Nkv, signs):
+    g = torch.Generator().manual_seed(H + Nq)
+    q = torch.randint(-127, 128, (1, H, Nq, 64), generator=g, dtype=torch.int8)
+    k = torch.randint(-127, 128, (1, H, Nkv, 64), generator=g, dtype=torch.int8)
+    q_sf = (torch.rand((1, H, -(-Nq // 64)), generator=g) + 0.5) * 0.01
+    k_sf = (torch.rand((1, H, -(-Nkv // 128)), generator=g) + 0.5) * 0.01
+    if signs:
+        q_sf *= torch.where(torch.rand(q_sf.shape, generator=g) < 0.5, -1.0, 1.0)
+        k_sf *= torch.where(torch.rand(k_sf.shape, generator=g) < 0.5, -1.0, 1.0)
+    v8, v_sf = T.quantize_fp8(make_input((1, H, Nkv, 72), seed=6), 3, 2, 2.25, True)
+    ref = A.mha_int8_x_fp8_fwd(q, q_sf, 64, k, k_sf, 128, v8, v_sf, 0.125)
+    o = torch.zeros((1, H, Nq, 72), dtype=torch.bfloat16, device="cuda")
+    binding().mha_int8_x_fp8_fwd(o, q.cuda(), q_sf.cuda(), 64, k.cuda(), k_sf.cuda(), 128,
+                                 v8.cuda().view(torch.float8_e4m3fn), v_sf.cuda(), 0.125)
+    torch.testing.assert_close(o.cpu().float(), ref.float(), atol=ATOL, rtol=RTOL)
+
+
 def test_error_behaviour():
     b = binding()
     q = torch.zeros((1, 1, 16, 128), dtype=torch.int8, device="cuda")
