@@ -9,11 +9,10 @@
 //   positions {8g + 4h + j} (g, j = 0..3) of a 32-group, h = 0, 1 - the sets that the swizzle of
 //   quantize(v, 3, N_dim, swizzle=True) makes contiguous in V                                    :248-319
 //   O = (sum over tiles of Phat . Vhat^T, rescaled) * ((1/l) * (1/2688) * v_gs) -> bf16          :705-830
-// A workgroup (four waves) owns 128 query rows, a wave 32 of them.  Per kv tile of 128 the packed K rows and
-// the packed V rows (V is stored [d][kv]) are fetched once per workgroup - every thread two 16-byte pieces of
-// each plus one scale dword, issued a whole tile ahead -, decoded once to exact fp16 and written to LDS, from
-// where all four waves read their MFMA operands.  Two LDS buffers alternate, one barrier per tile.  Decoded rows
-// are 256 bytes at a pitch of 272, so that the 16-byte fragment reads of 16 lanes fall on 64 different banks.
+// A workgroup (eight waves) owns 256, 128 or 64 query rows.  Per kv tile of 128 the packed K rows and the packed V rows (V
+// is stored [d][kv]) are fetched once per workgroup, decoded once to exact fp16 and written to LDS, from where all waves
+// read their MFMA operands.  Two LDS buffers alternate, one barrier per tile.  Decoded rows are 256 bytes at a pitch of
+// 272, so that the 16-byte fragment reads of 16 lanes fall on 64 different banks.
 //
 // The MFMAs are issued so that a lane owns ONE query row: S^T = Khat . Qhat^T and O^T = Vhat . Phat^T
 // (v_mfma_f32_32x32x16_f16, exact fp16 decode as in the linear).  Lane (r, h) of a wave then holds, per
@@ -178,97 +177,123 @@ __device__ __forceinline__ void mha_store_rows(uint16_t *o_base, int64_t o_n, in
   }
 }
 
+// The parts of O and of the row sum of the SPLIT waves of a group meet: every wave leaves its part in LDS and adds up, in
+// order, those of its 128 / SPLIT head dims (OT[0 ..] afterwards).  o_lds: 8 * 16 KB, l_lds: 1 KB.
+template <int SPLIT>
+__device__ __forceinline__ void mha_meet(f32x16 (&OT)[4], float &l_run, float *o_lds, float *l_lds, int group, int part, int lane) {
+  constexpr int NFD = 4 / SPLIT;
+  o_lds += lane;  // [wave][64 values][lane]
+  l_lds += group * (SPLIT * 32) + (lane & 31);
+#pragma unroll
+  for (int fd = 0; fd < 4; ++fd)
+#pragma unroll
+    for (int e = 0; e < 16; ++e) o_lds[(group * SPLIT + part) * 4096 + (fd * 16 + e) * 64] = OT[fd][e];
+  l_lds[part * 32] = l_run;
+  __syncthreads();
+  l_run = 0.0f;
+#pragma unroll
+  for (int q = 0; q < SPLIT; ++q) {
+#pragma unroll
+    for (int fd = 0; fd < NFD; ++fd)
+#pragma unroll
+      for (int e = 0; e < 16; ++e) {
+        const float o = o_lds[(group * SPLIT + q) * 4096 + ((part * NFD + fd) * 16 + e) * 64];
+        OT[fd][e] = q == 0 ? o : OT[fd][e] + o;
+      }
+    l_run += l_lds[q * 32];
+  }
+  __syncthreads();  // what follows lies over the parts
+}
+
 constexpr int MHA_PITCH = 272;                   // bytes per decoded row in LDS: 128 fp16 + 16 (bank spread)
 constexpr int MHA_TILE_LDS = 128 * MHA_PITCH;    // one decoded operand tile: K 128 kv rows, V 128 d rows
-constexpr int MHA_LDS_BYTES = 4 * MHA_TILE_LDS;  // K tiles j & 1 at 0 and MHA_TILE_LDS, V tiles j & 1 behind them
+constexpr int MHA_STAT_LDS = 4 * MHA_TILE_LDS;   // K tiles j & 1, V tiles j & 1; behind them the row maxima and sums of split tiles
+constexpr int MHA_LUT_LDS = MHA_STAT_LDS + 2 * 256 * 4;  // exact reciprocals of the e4m3 values, as in the quantizer
+constexpr int mha_lds_bytes(int) { return MHA_LUT_LDS + 128 * 4; }
+static_assert(8 * 16384 <= MHA_STAT_LDS && 8 * MHA_OUT_LDS <= MHA_STAT_LDS, "the parts of O and the staged output fit below the maxima");
 
-// what one thread fetches per kv tile: a quarter of a packed K row (two 16-blocks), a quarter of a packed V row of
-// the tile (one 32-group of kv positions), and the two scale bytes of each
-struct MhaFetch {
-  uint4 k, v;
-  uint32_t ksc, vsc;
-};
-
-// WAVES = 8 (256 query rows per workgroup, two waves per SIMD: one wave's MFMAs run under the other's vector work)
-// or 4 (128 query rows, for problems with too few workgroups of 256 rows to fill the GPU).  Both are compiled for 256
-// registers per lane (the launch bounds ask for two 4-wave workgroups per CU, which the LDS tile buffers do not
-// allow anyway): with 512, the compiler keeps S^T and O^T in accumulation registers and copies all of them to
-// ordinary registers and back around the softmax of every tile.
-template <int WAVES>
-__global__ __launch_bounds__(64 * WAVES, 8 / WAVES) void mha_nvfp4_fwd_kernel(MhaArgs a) {
-  constexpr int PARTS = 8 / WAVES;  // staging shares per thread: a tile is 512 quarter rows of K and of V
+// Eight waves, two per SIMD; a wave owns 32 query rows and 1 / SPLIT of the kv positions of every tile (see the INT8 x FP8
+// kernel below, which has the same structure).  A tile step runs, in the order written out,
+//   O += Vhat . Phat of tile i - 1  |  maxima, exp2, NVFP4 of tile i  |  S of tile i + 1
+// and decodes K of tile i + 2 and V of tile i, which were fetched a step earlier, into LDS.
+// (The multiplier of a P block inside the exponent instead of 16 multiplications gains another 3 %, but moves values across
+// rounding boundaries of P.)
+// Bound by vector-instruction issue (70 % of the cycles, 550 instructions per tile and wave against 64 MFMAs, which hold the
+// matrix core for 50 %) and by power: 13 % fewer cycles than one tile after the other at a clock of 2.0 instead of 2.15
+// GHz.  Kernel alone, same box, before (128 or 256 rows, no pipeline, no split) and now: 16384 x 40 x 128 6042 -> 5410 us
+// (1016 TFLOP/s; 1085 on a cooler box), 4096 x 40 422 -> 370, 8192 x 4 194 -> 165, 3000 x 24 214 -> 162, 512 x 2 on 8192
+// keys 191 -> 107, 75600 x 1 5250 -> 3676.
+template <int SPLIT>
+__device__ __forceinline__ void mha_nvfp4_block(const MhaArgs &a, const MhaTile &wg) {
+  constexpr int NF = 4 / SPLIT;  // 32-row fragments of a tile per wave
+  constexpr int ROWS = 256 / SPLIT;
+  constexpr int RING = 4;        // MFMA operands in flight from LDS
   extern __shared__ __attribute__((aligned(16))) uint8_t mha_lds[];
-  __shared__ float lut[128];  // exact reciprocals of the e4m3 values, as in the quantizer
-  load_rcp_table(lut);
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, r = lane & 31, h = lane >> 5;
-  // staging role of share p: row srow + p * (128 / PARTS) of the tile, 64-chunk sc, half sh of the chunk (K:
-  // elements 32 sh.. of the chunk, V: 32-group 2 sc + sh)
+  if (wg.block * ROWS >= a.Nq) return;
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), r = lane & 31, h = lane >> 5;
+  const int group = wave / SPLIT, part = wave % SPLIT;
+  // staging role: row srow of the tile, 64-chunk sc, half sh of the chunk (K: elements 32 sh.. of the chunk, V: 32-group
+  // 2 sc + sh)
   const int srow = threadIdx.x >> 2, sc = (threadIdx.x >> 1) & 1, sh = threadIdx.x & 1;
-  constexpr int PROWS = 128 / PARTS;
-  const int64_t b = blockIdx.z, head = blockIdx.y, bh = b * a.H + head;
-  const int64_t m = (int64_t)blockIdx.x * (32 * WAVES) + wave * 32 + r;   // this lane's query row
-  const int64_t mq = m < a.Nq ? m : a.Nq - 1;                         // rows past Nq read the last row; never stored
-  const int64_t v_row_bytes = a.Nkv64 / 2, v_chunks = a.Nkv64 / 64;
+  const int64_t bh = wg.b * a.H + wg.head;
+  const int64_t m = wg.block * ROWS + group * 32 + r;  // this lane's query row
+  const int64_t mq = m < a.Nq ? m : a.Nq - 1;          // rows past Nq read the last row; never stored
+  const int ntiles = (int)((a.Nkv + 127) / 128);
+  const int k_last = (int)(a.Nkv - 1 - (int64_t)(ntiles - 1) * 128);             // last kv row of the last tile
+  const int v_chunks_last = (int)(a.Nkv64 / 64 - (int64_t)(ntiles - 1) * 2);     // 64-chunks of V in the last tile: 1 or 2
 
-  // head dims below 128: the missing chunk of Q and K and the missing rows of V are zeros
+  // What does not exist is read from a place that does and decoded with a scale of zero: kv rows past Nkv, the second
+  // chunk of head dims up to 64, columns of V past its stored length.  Rows of V past Dv are never stored.
   const int64_t qk_row = a.chunks * 32;  // packed bytes of a Q / K row
-  const uint8_t *k_src = a.k + bh * a.Nkv * qk_row + sc * 32 + sh * 16;
-  const uint8_t *ksf_src = a.k_sf + (bh * a.chunks + sc) * a.Nkvp * 4 + sh * 2;
-  const uint8_t *v_src = a.v + (bh * a.Dv + srow) * v_row_bytes + sc * 32 + sh * 16;
-  const uint8_t *vsf_src = a.v_sf + ((bh * v_chunks + sc) * a.Dvp + srow) * 4 + sh * 2;
-  // rows past Nkv and chunks past the stored length of V are zeros
-  auto fetch = [&](int64_t n0, MhaFetch (&fs)[PARTS]) {
-#pragma unroll
-    for (int p = 0; p < PARTS; ++p) {
-      MhaFetch &f = fs[p];
-      const int64_t n = n0 + srow + p * PROWS;
-      f.k = f.v = make_uint4(0, 0, 0, 0);
-      f.ksc = f.vsc = 0;
-      if (n < a.Nkv && sc < a.chunks) {
-        f.k = *reinterpret_cast<const uint4 *>(k_src + n * qk_row);
-        f.ksc = *reinterpret_cast<const uint16_t *>(ksf_src + n * 4);
-      }
-      if (n0 + 64 * sc < a.Nkv64 && srow + p * PROWS < a.Dv) {
-        f.v = *reinterpret_cast<const uint4 *>(v_src + p * PROWS * v_row_bytes + n0 / 2);
-        f.vsc = *reinterpret_cast<const uint16_t *>(vsf_src + p * PROWS * 4 + (n0 / 64) * (a.Dvp * 4));
-      }
-    }
+  const int ksc_mask = sc < a.chunks ? 0xffff : 0, kchunk = sc < a.chunks ? sc : 0;
+  const uint8_t *k_src = a.k + bh * a.Nkv * qk_row + kchunk * 32 + sh * 16;
+  const uint8_t *ksf_src = a.k_sf + (bh * a.chunks + kchunk) * a.Nkvp * 4 + sh * 2;
+  const int vrow = srow < a.Dv ? srow : a.Dv - 1;
+  const uint8_t *v_src = a.v + (bh * a.Dv + vrow) * (a.Nkv64 / 2) + sh * 16;
+  const uint8_t *vsf_src = a.v_sf + (bh * (a.Nkv64 / 64) * a.Dvp + vrow) * 4 + sh * 2;
+  uint4 fk, fv;         // fetched, packed
+  uint32_t fksc, fvsc;  // and the two scale bytes that go with them
+  auto fetch_k = [&](int tile) {
+    const bool last = tile >= ntiles - 1;
+    if (last) tile = ntiles - 1;
+    const int row = !last || srow < k_last ? srow : k_last;
+    const int64_t n = (int64_t)tile * 128 + row;
+    fk = *reinterpret_cast<const uint4 *>(k_src + n * qk_row);
+    fksc = *reinterpret_cast<const uint16_t *>(ksf_src + n * 4);
+    fksc &= last && srow > k_last ? 0 : ksc_mask;
   };
-  // the same for a tile that lies inside Nkv as a whole, head dims of 128: nothing to test, nothing to zero
-  auto fetch_whole = [&](int64_t n0, MhaFetch (&fs)[PARTS]) {
-#pragma unroll
-    for (int p = 0; p < PARTS; ++p) {
-      MhaFetch &f = fs[p];
-      const int64_t n = n0 + srow + p * PROWS;
-      f.k = *reinterpret_cast<const uint4 *>(k_src + n * qk_row);
-      f.ksc = *reinterpret_cast<const uint16_t *>(ksf_src + n * 4);
-      f.v = *reinterpret_cast<const uint4 *>(v_src + p * PROWS * v_row_bytes + n0 / 2);
-      f.vsc = *reinterpret_cast<const uint16_t *>(vsf_src + p * PROWS * 4 + (n0 / 64) * (a.Dvp * 4));
-    }
+  auto fetch_v = [&](int tile) {
+    const bool last = tile >= ntiles - 1;
+    if (last) tile = ntiles - 1;
+    const bool there = !last || sc < v_chunks_last;
+    const int64_t chunk = (int64_t)tile * 2 + (there ? sc : 0);
+    fv = *reinterpret_cast<const uint4 *>(v_src + chunk * 32);
+    fvsc = *reinterpret_cast<const uint16_t *>(vsf_src + chunk * a.Dvp * 4);
+    fvsc &= there ? 0xffff : 0;
   };
-  // decode once per workgroup, into LDS tile buffers `buf`.  V: the thread's 32-group holds 16 stored bytes; operand
-  // piece (t, hh) takes the t-th 16-bit halves of its dwords 2 hh and 2 hh + 1, and the scale of stored block hh.
-  auto stage = [&](int buf, const MhaFetch (&fs)[PARTS]) {
-#pragma unroll
-    for (int p = 0; p < PARTS; ++p) {
-    const MhaFetch &f = fs[p];
-    uint8_t *kd = mha_lds + buf * MHA_TILE_LDS + (srow + p * PROWS) * MHA_PITCH + sc * 128 + sh * 64;
-    const f16x2 ks = __builtin_amdgcn_cvt_scalef32_pk_f16_fp8(f.ksc, 1.0f, false);
-    const f16x2 kb0 = {ks.x, ks.x}, kb1 = {ks.y, ks.y};
-    *reinterpret_cast<f16x8 *>(kd + 0) = mha_decode8(f.k.x, kb0);
-    *reinterpret_cast<f16x8 *>(kd + 16) = mha_decode8(f.k.y, kb0);
-    *reinterpret_cast<f16x8 *>(kd + 32) = mha_decode8(f.k.z, kb1);
-    *reinterpret_cast<f16x8 *>(kd + 48) = mha_decode8(f.k.w, kb1);
-    uint8_t *vd = mha_lds + (2 + buf) * MHA_TILE_LDS + (srow + p * PROWS) * MHA_PITCH + sc * 128 + sh * 64;
-    const f16x2 vs = __builtin_amdgcn_cvt_scalef32_pk_f16_fp8(f.vsc, 1.0f, false);
-    const f16x2 vb0 = {vs.x, vs.x}, vb1 = {vs.y, vs.y};
-    *reinterpret_cast<f16x8 *>(vd + 0) = mha_decode8((f.v.x & 0xffffu) | (f.v.y << 16), vb0);           // t 0, hh 0
-    *reinterpret_cast<f16x8 *>(vd + 16) = mha_decode8((f.v.z & 0xffffu) | (f.v.w << 16), vb1);          // t 0, hh 1
-    *reinterpret_cast<f16x8 *>(vd + 32) = mha_decode8((f.v.x >> 16) | (f.v.y & 0xffff0000u), vb0);      // t 1, hh 0
-    *reinterpret_cast<f16x8 *>(vd + 48) = mha_decode8((f.v.z >> 16) | (f.v.w & 0xffff0000u), vb1);      // t 1, hh 1
+  // Decode, piece by piece (0..3 of K, 4..7 of V), into the tile buffers `buf`.  V: the thread's 32-group holds 16 stored
+  // bytes; operand piece (t, hh) takes the t-th 16-bit halves of its dwords 2 hh and 2 hh + 1, and the scale of stored
+  // block hh.
+  uint8_t *const kd = mha_lds + srow * MHA_PITCH + sc * 128 + sh * 64, *const vd = kd + 2 * MHA_TILE_LDS;
+  auto stage_piece = [&](int buf, int piece) {
+    const f16x2 s2 = __builtin_amdgcn_cvt_scalef32_pk_f16_fp8(piece < 4 ? fksc : fvsc, 1.0f, false);
+    const f16x2 b0 = {s2.x, s2.x}, b1 = {s2.y, s2.y};
+    const int j = piece & 3;
+    if (piece < 4) {
+      const uint32_t w = j == 0 ? fk.x : j == 1 ? fk.y : j == 2 ? fk.z : fk.w;
+      *reinterpret_cast<f16x8 *>(kd + buf * MHA_TILE_LDS + j * 16) = mha_decode8(w, j < 2 ? b0 : b1);
+    } else {
+      const uint32_t w = j == 0 ? (fv.x & 0xffffu) | (fv.y << 16) : j == 1 ? (fv.z & 0xffffu) | (fv.w << 16)
+                       : j == 2 ? (fv.x >> 16) | (fv.y & 0xffff0000u) : (fv.z >> 16) | (fv.w & 0xffff0000u);
+      *reinterpret_cast<f16x8 *>(vd + buf * MHA_TILE_LDS + j * 16) = mha_decode8(w, j & 1 ? b1 : b0);
     }
   };
 
+  float *const lut = reinterpret_cast<float *>(mha_lds + MHA_LUT_LDS);
+  if (threadIdx.x < 128) lut[threadIdx.x] = g_rcp_e4m3.v[threadIdx.x];
+  fetch_k(1);  // (both in flight together: the registers of V are free)
+  fv = fk, fvsc = fksc;
+  fetch_k(0);
   // Qhat of the lane's row: 8 operands of 16 k (chunk c, sub-step s), kept for the whole kernel
   f16x8 QF[2][4];
 #pragma unroll
@@ -278,7 +303,6 @@ __global__ __launch_bounds__(64 * WAVES, 8 / WAVES) void mha_nvfp4_fwd_kernel(Mh
     if (c < a.chunks)
       mha_load_row_chunk(a.q + (bh * a.Nq + mq) * qk_row, a.q_sf + ((bh * a.chunks + c) * a.Nqp + mq) * 4, c, h, QF[c]);
   }
-
   // exp2 argument = S * cs - (row maximum of S) * cs with cs = q_gs * k_gs * sm_scale * log2(e); a negative cs is
   // moved into Q so that the row maximum can be taken over the raw dot products
   float cs = (*a.q_gs) * (*a.k_gs) * a.sm_scale * MHA_LOG2E;
@@ -289,111 +313,196 @@ __global__ __launch_bounds__(64 * WAVES, 8 / WAVES) void mha_nvfp4_fwd_kernel(Mh
 #pragma unroll
       for (int s = 0; s < 4; ++s) QF[c][s] = -QF[c][s];
   }
+#pragma unroll
+  for (int p = 0; p < 4; ++p) stage_piece(0, p);
+  fk = fv, fksc = fvsc;
+  fetch_v(0);
   float ml_run = -__builtin_inff(), l_run = 0.0f;  // running row maximum (in log2 units) and row sum
+  float alpha = 1.0f;                              // factor of O and l that the last tile's maximum asks for
   f32x16 OT[4];  // O^T: d = 32 fd + 8 (e >> 2) + 4 h + (e & 3), for the lane's query row
 #pragma unroll
-  for (int fd = 0; fd < 4; ++fd)
+  for (int fd = 0; fd < 4; ++fd) OT[fd] = (f32x16)(0.0f);
+  uint32_t PW[2 * NF];  // P of a tile: eight nibbles per (fragment, step of 16 kv positions)
+  uint32_t pcode[NF];   // and its block scales
 #pragma unroll
-    for (int e = 0; e < 16; ++e) OT[fd][e] = 0.0f;
-
-  MhaFetch nxt[PARTS];
-  fetch(0, nxt);
-  stage(0, nxt);
+  for (int f = 0; f < NF; ++f) PW[2 * f] = PW[2 * f + 1] = pcode[f] = 0;
+  // V of the tile in front of the first one: zeros, and so is its P
+#pragma unroll
+  for (int j = 0; j < 4; ++j) *reinterpret_cast<uint4 *>(vd + MHA_TILE_LDS + j * 16) = make_uint4(0, 0, 0, 0);
+#pragma unroll
+  for (int p = 0; p < 4; ++p) stage_piece(1, p);
+  fetch_k(2);
   __syncthreads();
-  int buf = 0;
-  auto tile_step = [&](auto whole_next_tag, int64_t n0) {
-    // the next tile's packed bytes travel while this one is multiplied (zeros past the end)
-    if constexpr (decltype(whole_next_tag)::value) fetch_whole(n0 + 128, nxt);
-    else fetch(n0 + 128, nxt);
-    const uint8_t *kb = mha_lds + buf * MHA_TILE_LDS + r * MHA_PITCH + h * 64;
-    const uint8_t *vb = mha_lds + (2 + buf) * MHA_TILE_LDS + r * MHA_PITCH + h * 16;
-    // ---- S^T = Khat . Qhat^T for the 128 kv positions of the tile (four 32-row fragments)
-    f32x16 ST[4];
-#pragma unroll
-    for (int c = 0; c < 2; ++c)
-#pragma unroll
-      for (int s = 0; s < 4; ++s)
-#pragma unroll
-        for (int f = 0; f < 4; ++f) {  // consecutive MFMAs go to different accumulators
-          const f16x8 KF = *reinterpret_cast<const f16x8 *>(kb + f * 32 * MHA_PITCH + c * 128 + s * 16);
-          if (c == 0 && s == 0)
-            ST[f] = __builtin_amdgcn_mfma_f32_32x32x16_f16(KF, QF[c][s], (f32x16)(0.0f), 0, 0, 0);
-          else
-            ST[f] = __builtin_amdgcn_mfma_f32_32x32x16_f16(KF, QF[c][s], ST[f], 0, 0, 0);
-        }
-    // ---- online softmax of the lane's row: its 64 values here, the other 64 in the lane 32 away
-    // maxima of the raw values per fragment = per P block: exp2 and the scaling are monotonic, so the largest p of
-    // a block is the p of its largest raw value, bit for bit
-    float bmax[4];
-#pragma unroll
-    for (int f = 0; f < 4; ++f) {
-      bmax[f] = ST[f][0];
-#pragma unroll
-      for (int e = 1; e < 16; ++e) bmax[f] = __builtin_fmaxf(bmax[f], ST[f][e]);
-    }
-    const float mx = __builtin_fmaxf(__builtin_fmaxf(bmax[0], bmax[1]), __builtin_fmaxf(bmax[2], bmax[3]));
-    const float ml = __builtin_fmaxf(ml_run, mha_halves_max(mx) * cs);
-#pragma unroll
-    for (int f = 0; f < 4; ++f) bmax[f] = __builtin_amdgcn_exp2f(__builtin_fmaf(bmax[f], cs, -ml));
-    float lsum = 0.0f;
-#pragma unroll
-    for (int f = 0; f < 4; ++f)
-#pragma unroll
-      for (int e = 0; e < 16; ++e) {
-        ST[f][e] = __builtin_amdgcn_exp2f(__builtin_fmaf(ST[f][e], cs, -ml));  // p
-        lsum += ST[f][e];
-      }
-    const float l_new = mha_halves_sum(lsum);
-    const float alpha = __builtin_amdgcn_exp2f(ml_run - ml);
-    l_run = alpha * l_run + l_new;
-    ml_run = ml;
+
+  f32x16 ST[NF];  // S^T of the tile at hand
+  float bmax[NF];
+  auto rescale = [&]() {
     if (__builtin_amdgcn_ballot_w64(alpha != 1.0f)) {  // else no row of this wave raised its maximum
 #pragma unroll
       for (int fd = 0; fd < 4; ++fd)
 #pragma unroll
         for (int e = 0; e < 16; ++e) OT[fd][e] *= alpha;
     }
-
-    // ---- P -> NVFP4 (the lane's 16 values of a fragment are one block), then O^T += Vhat . Phat^T
+  };
+  // operands: K for step t = 8 (fragment) + (16 columns), V for step u = 8 (fragment) + 4 (16 kv positions) + (32 rows of d)
+  const uint8_t *const k_lane = mha_lds + (part * NF * 32 + r) * MHA_PITCH + h * 64;
+  const uint8_t *const v_lane = mha_lds + 2 * MHA_TILE_LDS + r * MHA_PITCH + h * 16 + part * NF * 64;
+  auto k_operand = [&](int buf, int t) {
+    return *reinterpret_cast<const f16x8 *>(k_lane + buf * MHA_TILE_LDS + (t >> 3) * 32 * MHA_PITCH + ((t >> 2) & 1) * 128 + (t & 3) * 16);
+  };
+  auto v_operand = [&](int buf, int u) {
+    return *reinterpret_cast<const f16x8 *>(v_lane + buf * MHA_TILE_LDS + (u & 3) * 32 * MHA_PITCH + (u >> 3) * 64 + ((u >> 2) & 1) * 32);
+  };
+  auto p_operand = [&](int g) {  // g = 2 (fragment) + (16 kv positions)
+    const f16x2 s2 = __builtin_amdgcn_cvt_scalef32_pk_f16_fp8(pcode[g >> 1], 1.0f, false);
+    return mha_decode8(PW[g], (f16x2){s2.x, s2.x});
+  };
+  // row maxima of a tile's parts, two tiles in turn: [tile & 1][group][part][row]
+  float *mx_lds = reinterpret_cast<float *>(mha_lds + MHA_STAT_LDS) + group * (SPLIT * 32) + r;
+  // maxima of the raw values per fragment = per P block: exp2 and the scaling are monotonic, so the largest p of a block
+  // is the p of its largest raw value, bit for bit
+  auto part_maximum = [&](int parity) {
+    float mx = -__builtin_inff();
 #pragma unroll
-    for (int f = 0; f < 4; ++f) {
-      uint32_t code;
-      const float o = nvfp4_block_scale(bmax[f], MHA_P_ALPHA, lut, code);  // 2688 / e4m3(2688 * (bm / 6)), 0 for code 0
-      const f16x2 s2 = __builtin_amdgcn_cvt_scalef32_pk_f16_fp8(code, 1.0f, false);
-      const f16x2 psc = {s2.x, s2.x};
+    for (int f = 0; f < NF; ++f) {
+      bmax[f] = ST[f][0];
 #pragma unroll
-      for (int t = 0; t < 2; ++t) {
-        // k slots of this step in the order the stored nibbles of V come in (see the header)
-        const float pv[8] = {ST[f][8 * t + 0] * o, ST[f][8 * t + 1] * o, ST[f][8 * t + 4] * o, ST[f][8 * t + 5] * o,
-                             ST[f][8 * t + 2] * o, ST[f][8 * t + 3] * o, ST[f][8 * t + 6] * o, ST[f][8 * t + 7] * o};
-        const f16x8 PF = mha_decode8(f32x8_to_e2m1x8(pv), psc);
-#pragma unroll
-        for (int fd = 0; fd < 4; ++fd) {
-          const f16x8 VF = *reinterpret_cast<const f16x8 *>(vb + fd * 32 * MHA_PITCH + f * 64 + t * 32);
-          OT[fd] = __builtin_amdgcn_mfma_f32_32x32x16_f16(VF, PF, OT[fd], 0, 0, 0);
-        }
-      }
+      for (int e = 1; e < 16; ++e) bmax[f] = __builtin_fmaxf(bmax[f], ST[f][e]);
+      mx = __builtin_fmaxf(mx, bmax[f]);
     }
-    stage(buf ^ 1, nxt);
+    mx_lds[parity * 256 + part * 32] = mha_halves_max(mx);  // (both halves of the wave write the same value)
+  };
+#pragma unroll
+  for (int t = 0; t < 8 * NF; ++t)
+    ST[t >> 3] = __builtin_amdgcn_mfma_f32_32x32x16_f16(k_operand(0, t), QF[(t >> 2) & 1][t & 3], (t & 7) == 0 ? (f32x16)(0.0f) : ST[t >> 3], 0, 0, 0);
+  if constexpr (SPLIT > 1) part_maximum(0);
+  __syncthreads();
+
+  auto tile_step = [&](int i) {
+    const int buf = i & 1;
+    f16x8 VF[RING];
+#pragma unroll
+    for (int u = 0; u < RING; ++u) VF[u] = v_operand(buf ^ 1, u);
+    rescale();
+    // ---- all but the last fragment of O of the tile before; under it the decoding of what was fetched and (SPLIT 1) the
+    // maxima of this tile
+    f16x8 PF = p_operand(0);
+    constexpr int PVA = 8 * (NF - 1);
+    if constexpr (NF == 1) {
+#pragma unroll
+      for (int p = 0; p < 8; ++p) stage_piece(buf, p);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int u = 0; u < PVA; ++u) {
+      OT[u & 3] = __builtin_amdgcn_mfma_f32_32x32x16_f16(VF[u % RING], PF, OT[u & 3], 0, 0, 0);
+      VF[u % RING] = v_operand(buf ^ 1, u + RING);
+      if ((u & 3) == 3) PF = p_operand((u >> 2) + 1);
+      if (SPLIT == 1 && u < 16) {
+        float &b = bmax[(u >> 2) % NF];
+#pragma unroll
+        for (int e = 4 * (u & 3); e < 4 * (u & 3) + 4; ++e) b = e == 0 ? ST[(u >> 2) % NF][0] : __builtin_fmaxf(b, ST[(u >> 2) % NF][e]);
+        asm volatile("" : "+v"(b));
+      }
+      if (NF == 4 && (u % 3) == 2) stage_piece(buf, u / 3);
+      if (NF == 2) stage_piece(buf, u);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    fetch_k(i + 3);
+    fetch_v(i + 1);
+    float mx;
+    if constexpr (SPLIT == 1) {
+      mx = mha_halves_max(__builtin_fmaxf(__builtin_fmaxf(bmax[0], bmax[1 % NF]), __builtin_fmaxf(bmax[2 % NF], bmax[3 % NF])));
+    } else {
+      mx = mx_lds[buf * 256];
+#pragma unroll
+      for (int q = 1; q < SPLIT; ++q) mx = __builtin_fmaxf(mx, mx_lds[buf * 256 + q * 32]);
+    }
+    const float ml = __builtin_fmaxf(ml_run, mx * cs);
+    alpha = __builtin_amdgcn_exp2f(ml_run - ml);
+    ml_run = ml;
+    // block scales: e4m3(2688 * (largest p / 6)), at most 448, and the multiplier 2688 / scale, 0 for code 0
+    float o[NF];
+    uint32_t code[NF];
+#pragma unroll
+    for (int f = 0; f < NF; ++f) {
+      const float bm = __builtin_amdgcn_exp2f(__builtin_fmaf(bmax[f], cs, -ml));
+      code[f] = (uint32_t)__builtin_amdgcn_cvt_pk_fp8_f32(MHA_P_ALPHA * (bm * 0.16666666666666666f), 0.0f, 0, false) & 0x7f;
+      o[f] = MHA_P_ALPHA * lut[code[f]];
+    }
+    // ---- P of this tile; under it the last fragment of O of the tile before and S of the next one
+    float lsum = 0.0f;
+    f16x8 KF[RING];
+    uint32_t w;
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int st = 0; st < 8 * NF + 8; ++st) {
+      if (st < 8) {
+        const int u = PVA + st;
+        OT[u & 3] = __builtin_amdgcn_mfma_f32_32x32x16_f16(VF[u % RING], PF, OT[u & 3], 0, 0, 0);
+        if (st + RING < 8) VF[u % RING] = v_operand(buf ^ 1, u + RING);
+        else KF[st % RING] = k_operand(buf ^ 1, st + RING - 8);
+        if (st == 3) PF = p_operand(2 * NF - 1);
+      } else {
+        const int t = st - 8;
+        ST[t >> 3] = __builtin_amdgcn_mfma_f32_32x32x16_f16(KF[t % RING], QF[(t >> 2) & 1][t & 3], (t & 7) == 0 ? (f32x16)(0.0f) : ST[t >> 3], 0, 0, 0);
+        if (t + RING < 8 * NF) KF[t % RING] = k_operand(buf ^ 1, t + RING);
+      }
+      if (st < 8 * NF) {
+        // two values of fragment f, in the order in which the stored nibbles of V come (see the header)
+        const int f = st >> 3, t = (st >> 2) & 1, j = st & 3, e = 8 * t + (j == 0 ? 0 : j == 1 ? 4 : j == 2 ? 2 : 6);
+        const float p0 = __builtin_amdgcn_exp2f(__builtin_fmaf(ST[f][e], cs, -ml));
+        const float p1 = __builtin_amdgcn_exp2f(__builtin_fmaf(ST[f][e + 1], cs, -ml));
+        lsum += p0;
+        lsum += p1;
+        if (j == 0) {
+          asm volatile("" : "=v"(w));  // (any value: all four bytes are written)
+          w = __builtin_amdgcn_cvt_scalef32_pk_fp4_f32(w, p0 * o[f], p1 * o[f], 1.0f, 0);
+        } else if (j == 1) w = __builtin_amdgcn_cvt_scalef32_pk_fp4_f32(w, p0 * o[f], p1 * o[f], 1.0f, 1);
+        else if (j == 2) w = __builtin_amdgcn_cvt_scalef32_pk_fp4_f32(w, p0 * o[f], p1 * o[f], 1.0f, 2);
+        else w = __builtin_amdgcn_cvt_scalef32_pk_fp4_f32(w, p0 * o[f], p1 * o[f], 1.0f, 3);
+        asm volatile("" : "+v"(w), "+v"(lsum));
+        if (j == 3) PW[2 * f + t] = w;
+      }
+      __builtin_amdgcn_sched_barrier(0);
+    }
+#pragma unroll
+    for (int f = 0; f < NF; ++f) pcode[f] = code[f];
+    l_run = __builtin_fmaf(l_run, alpha, mha_halves_sum(lsum));
+    if constexpr (SPLIT > 1) part_maximum(buf ^ 1);
     __syncthreads();
   };
-  int64_t n0 = 0;
-  // tiles followed by a whole tile: the fetch without tests (worth 2 % with eight waves; with four it loses 5 %)
-  if (WAVES == 8 && a.chunks == 2 && a.Dv == 128)
-    for (; n0 + 256 <= a.Nkv; n0 += 128, buf ^= 1) tile_step(std::true_type{}, n0);
-  for (; n0 < a.Nkv; n0 += 128, buf ^= 1) tile_step(std::false_type{}, n0);
+  for (int i = 0; i < ntiles; ++i) tile_step(i);
+  rescale();
+#pragma unroll
+  for (int u = 0; u < 8 * NF; ++u)
+    OT[u & 3] = __builtin_amdgcn_mfma_f32_32x32x16_f16(v_operand((ntiles - 1) & 1, u), p_operand(u >> 2), OT[u & 3], 0, 0, 0);
+  __syncthreads();  // what follows lies over the tile buffers
+
+  // The parts of O meet: every wave leaves its part in LDS and adds up, in order, those of 128 / SPLIT head dims.
+  constexpr int NFD = 4 / SPLIT;
+  const int d0 = part * NFD * 32;
+  if constexpr (SPLIT > 1)
+    mha_meet<SPLIT>(OT, l_run, reinterpret_cast<float *>(mha_lds), reinterpret_cast<float *>(mha_lds + MHA_STAT_LDS), group, part, lane);
 
   // the zero-filled kv positions of the last tile each added exp(0 - m) to the row sum
   if (a.Nkv % 128 != 0) l_run -= (float)(128 - a.Nkv % 128) / __builtin_amdgcn_exp2f(ml_run);
   // ---- O = O * ((1/l) * (1/2688) * v_gs) -> bf16
   const float scale = (1.0f / l_run) * (1.0f / MHA_P_ALPHA) * (*a.v_gs);
-  uint16_t ob[4][16];
+  uint16_t ob[NFD][16];
 #pragma unroll
-  for (int fd = 0; fd < 4; ++fd)
+  for (int fd = 0; fd < NFD; ++fd)
 #pragma unroll
     for (int e = 0; e < 16; ++e) ob[fd][e] = __builtin_bit_cast(uint16_t, (__bf16)(OT[fd][e] * scale));
-  mha_store_rows<4>(a.O + b * a.o_b + head * a.o_h, a.o_n, a.o_d, a.o_vec, (int64_t)blockIdx.x * (32 * WAVES) + wave * 32, a.Nq,
-                    a.Dv, 0, lane, mha_lds + wave * MHA_OUT_LDS, ob);
+  mha_store_rows<NFD>(a.O + wg.b * a.o_b + wg.head * a.o_h, a.o_n, a.o_d, a.o_vec, wg.block * ROWS + group * 32, a.Nq, a.Dv, d0,
+                      lane, mha_lds + wave * MHA_OUT_LDS, ob);
+}
+
+// (two bodies in one kernel, so that the workgroups of the last round start as the ones in front of them end)
+template <int TAIL>
+__global__ __launch_bounds__(512, 1) void mha_nvfp4_fwd_kernel(MhaArgs a, MhaWork w) {
+  if (TAIL == 1 || blockIdx.x < w.full) mha_nvfp4_block<1>(a, mha_tile(w, a.H, 1));
+  else mha_nvfp4_block<TAIL>(a, mha_tile(w, a.H, TAIL));
 }
 
 // ---------------------------------------------------------------------------------------------------------------
@@ -405,7 +514,7 @@ __global__ __launch_bounds__(64 * WAVES, 8 / WAVES) void mha_nvfp4_fwd_kernel(Mh
 //   P -> e4m3 per element (cvt.rn.satfinite, no scales); O = O * exp2(m_old - m) + Phat . Vhat^T        :323-345,828-880
 //   O * ((1 / l) * v_sf[d]) -> bf16                                                                   :886-905
 // The product Phat . Vhat^T is accumulated in fp32 here (the reference's MMA accumulates each tile in fp16).
-// Same structure as the NVFP4 kernel above: a lane owns one query row (S^T = K . Q^T with v_mfma_i32_32x32x32_i8,
+// Like in the NVFP4 kernel above a lane owns one query row (S^T = K . Q^T with v_mfma_i32_32x32x32_i8,
 // O^T = Vhat . Phat^T with v_mfma_scale_f32_32x32x64_f8f6f4 on e4m3 operands, scales 2^0), but nothing has to be decoded: the int8 rows of K and the
 // e4m3 rows of V go from global memory into LDS as they are, and from there into the MFMAs.  V is stored with the
 // 16-group swizzle of quantize(v, 3, N_dim, swizzle=True, precision="fp8e4m3"): stored byte 8 h + 4 (j >> 1) + 2 q
@@ -722,29 +831,8 @@ __device__ __forceinline__ void mha_int8_x_fp8_block(const Mha8Args &a, const Mh
   // The parts of O meet: every wave leaves its part in LDS and adds up, in order, those of 128 / SPLIT head dims.
   constexpr int NFD = 4 / SPLIT;
   const int d0 = part * NFD * 32;
-  if constexpr (SPLIT > 1) {
-    float *o_lds = reinterpret_cast<float *>(mha_lds) + lane;  // [wave][64 values][lane]
-    float *l_lds = reinterpret_cast<float *>(mha_lds + mha8_stat_lds(SPLIT)) + group * (SPLIT * 32) + r;
-#pragma unroll
-    for (int fd = 0; fd < 4; ++fd)
-#pragma unroll
-      for (int e = 0; e < 16; ++e) o_lds[wave * 4096 + (fd * 16 + e) * 64] = OT[fd][e];
-    l_lds[part * 32] = l_run;
-    __syncthreads();
-    l_run = 0.0f;
-#pragma unroll
-    for (int q = 0; q < SPLIT; ++q) {
-#pragma unroll
-      for (int fd = 0; fd < NFD; ++fd)
-#pragma unroll
-        for (int e = 0; e < 16; ++e) {
-          const float o = o_lds[(group * SPLIT + q) * 4096 + ((part * NFD + fd) * 16 + e) * 64];
-          OT[fd][e] = q == 0 ? o : OT[fd][e] + o;
-        }
-      l_run += l_lds[q * 32];
-    }
-    __syncthreads();  // the staged output lies over the parts
-  }
+  if constexpr (SPLIT > 1)
+    mha_meet<SPLIT>(OT, l_run, reinterpret_cast<float *>(mha_lds), reinterpret_cast<float *>(mha_lds + mha8_stat_lds(SPLIT)), group, part, lane);
 
   // ---- O = O * ((1 / l) * v_sf[d]) -> bf16
   const float rl = 1.0f / l_run;
@@ -828,6 +916,34 @@ __global__ __launch_bounds__(256) void quantize_int8_token_block_kernel(int8_t *
   }
 }
 
+// one kernel per cut of the last round (1, 2, 4)
+static void (*const mha_nvfp4_kernels[3])(MhaArgs, MhaWork) = {mha_nvfp4_fwd_kernel<1>, mha_nvfp4_fwd_kernel<2>, mha_nvfp4_fwd_kernel<4>};
+static void (*const mha_int8_x_fp8_kernels[3])(Mha8Args, MhaWork) = {mha_int8_x_fp8_fwd_kernel<1>, mha_int8_x_fp8_fwd_kernel<2>,
+                                                                     mha_int8_x_fp8_fwd_kernel<4>};
+
+template <typename Args>
+static int mha_launch(const Args &a, int64_t heads, int64_t Nq, int64_t ntiles, const MhaCost &cost, void (*const (&kernels)[3])(Args, MhaWork),
+                      int (*lds_bytes)(int), hipStream_t st, const char *what) {
+  int tail = 1;
+  unsigned grid = 0;
+  const MhaWork work = mha_plan(cost, heads, Nq, ntiles, &tail, &grid);
+  auto kern = kernels[tail >> 1];
+  const int lds = lds_bytes(tail);
+  {  // more than 64 KB of dynamic LDS has to be allowed once per device and kernel
+    static std::atomic<uint32_t> lds_done[3] = {{0}, {0}, {0}};
+    int dev = 0;
+    if (hipGetDevice(&dev) != hipSuccess) dev = 0;
+    const uint32_t bit = 1u << (dev & 31);
+    if (!(lds_done[tail >> 1].load(std::memory_order_relaxed) & bit)) {
+      hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, lds);
+      if (e != hipSuccess) return set_error("hipFuncSetAttribute(LDS=%d): %s", lds, hipGetErrorString(e));
+      lds_done[tail >> 1].fetch_or(bit, std::memory_order_relaxed);
+    }
+  }
+  hipLaunchKernelGGL(kern, dim3(grid), dim3(512), lds, st, a, work);
+  return check_launch(what);
+}
+
 }  // namespace ac4k
 
 using namespace ac4k;
@@ -846,7 +962,7 @@ extern "C" __attribute__((visibility("default"))) int ac4k_mha_nvfp4_fwd(
                (long long)Dqk, (long long)Dv);
   AC4K_REQUIRE((((uintptr_t)q | (uintptr_t)k | (uintptr_t)v) & 15) == 0 && (((uintptr_t)q_sf | (uintptr_t)k_sf | (uintptr_t)v_sf) & 3) == 0,
                "q, k, v must be 16-byte aligned and the scale tensors 4-byte aligned");
-  AC4K_REQUIRE(H <= 65535 && B <= 65535 && ceil_div(Nq, 128) < (1ll << 31), "problem too large");
+  AC4K_REQUIRE(H <= 65535 && B <= 65535 && ceil_div(Nq, 128) < (1ll << 31) && B * H * ceil_div(Nq, 256) < (1ll << 29), "problem too large");
   AC4K_REQUIRE(o_b_stride >= 0 && o_h_stride >= 0 && o_n_stride >= 1 && o_d_stride >= 1, "strides of O must be positive");
   MhaArgs a{static_cast<uint16_t *>(O), o_b_stride, o_h_stride, o_n_stride, o_d_stride,
             static_cast<const uint8_t *>(q), static_cast<const uint8_t *>(k), static_cast<const uint8_t *>(v),
@@ -854,25 +970,9 @@ extern "C" __attribute__((visibility("default"))) int ac4k_mha_nvfp4_fwd(
             q_gs, k_gs, v_gs, H, Nq, Nkv, align_up(Nq, 16), align_up(Nkv, 16), align_up(Nkv, 64), (int)(Dqk / 64), (int)Dv,
             (int)align_up(Dv, 16), sm_scale,
             (o_d_stride == 1 && Dv % 8 == 0 && ((uintptr_t)O & 15) == 0 && o_b_stride % 8 == 0 && o_h_stride % 8 == 0 && o_n_stride % 8 == 0) ? 1 : 0};
-  // 256 query rows per workgroup unless that leaves most of the GPU's 256 CUs without one
-  const bool wide = ceil_div(Nq, 256) * H * B >= 192 || ceil_div(Nq, 128) * H * B <= ceil_div(Nq, 256) * H * B;
-  auto kern = wide ? mha_nvfp4_fwd_kernel<8> : mha_nvfp4_fwd_kernel<4>;
-  {  // more than 64 KB of dynamic LDS has to be allowed once per device and kernel
-    static std::atomic<uint32_t> lds_done[2] = {{0}, {0}};
-    int dev = 0;
-    if (hipGetDevice(&dev) != hipSuccess) dev = 0;
-    const uint32_t bit = 1u << (dev & 31);
-    if (!(lds_done[wide].load(std::memory_order_relaxed) & bit)) {
-      hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(kern), hipFuncAttributeMaxDynamicSharedMemorySize,
-                                         MHA_LDS_BYTES);
-      if (e != hipSuccess) return set_error("hipFuncSetAttribute(LDS=%d): %s", MHA_LDS_BYTES, hipGetErrorString(e));
-      lds_done[wide].fetch_or(bit, std::memory_order_relaxed);
-    }
-  }
-  const int rows = wide ? 256 : 128;
-  hipLaunchKernelGGL(kern, dim3((unsigned)ceil_div(Nq, rows), (unsigned)H, (unsigned)B), dim3(rows * 2), MHA_LDS_BYTES,
-                     (hipStream_t)stream, a);
-  return check_launch("ac4k_mha_nvfp4_fwd");
+  // measured: 512 x 2 x 128 to 8192 x 4 x 128 and 16384 x 40 on 4096 to 16384 keys
+  static constexpr MhaCost cost{{5.0f, 6.0f, 5.5f}, {3.9f, 2.35f, 1.6f}};
+  return mha_launch(a, B * H, Nq, ceil_div(Nkv, 128), cost, mha_nvfp4_kernels, mha_lds_bytes, (hipStream_t)stream, "ac4k_mha_nvfp4_fwd");
 }
 
 // Replaces ac4k::mha_int8_x_fp8_fwd (lib/cuda/sm120/mha_int8_x_fp8.cu:979-1137).
@@ -901,24 +1001,7 @@ extern "C" __attribute__((visibility("default"))) int ac4k_mha_int8_x_fp8_fwd(
              (o_d_stride == 1 && Dv % 8 == 0 && ((uintptr_t)O & 15) == 0 && o_b_stride % 8 == 0 && o_h_stride % 8 == 0 && o_n_stride % 8 == 0) ? 1 : 0};
   // measured: 512 x 2 x 128 to 8192 x 4 x 128 on 4096 and 8192 keys, one round
   static constexpr MhaCost cost{{4.5f, 6.0f, 5.0f}, {2.35f, 1.45f, 1.05f}};
-  int tail = 1;
-  unsigned grid = 0;
-  const MhaWork work = mha_plan(cost, B * H, Nq, ceil_div(Nkv, 128), &tail, &grid);
-  const int idx = tail >> 1, lds = mha8_lds_bytes(tail);
-  auto kern = tail == 1 ? mha_int8_x_fp8_fwd_kernel<1> : tail == 2 ? mha_int8_x_fp8_fwd_kernel<2> : mha_int8_x_fp8_fwd_kernel<4>;
-  {  // more than 64 KB of dynamic LDS has to be allowed once per device and kernel
-    static std::atomic<uint32_t> lds_done[3] = {{0}, {0}, {0}};
-    int dev = 0;
-    if (hipGetDevice(&dev) != hipSuccess) dev = 0;
-    const uint32_t bit = 1u << (dev & 31);
-    if (!(lds_done[idx].load(std::memory_order_relaxed) & bit)) {
-      hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, lds);
-      if (e != hipSuccess) return set_error("hipFuncSetAttribute(LDS=%d): %s", lds, hipGetErrorString(e));
-      lds_done[idx].fetch_or(bit, std::memory_order_relaxed);
-    }
-  }
-  hipLaunchKernelGGL(kern, dim3(grid), dim3(512), lds, (hipStream_t)stream, a, work);
-  return check_launch("ac4k_mha_int8_x_fp8_fwd");
+  return mha_launch(a, B * H, Nq, ceil_div(Nkv, 128), cost, mha_int8_x_fp8_kernels, mha8_lds_bytes, (hipStream_t)stream, "ac4k_mha_int8_x_fp8_fwd");
 }
 
 // Replaces _int8_quantize / _triton_block_token_quantize (python/ac4k_kernel/ops/attention.py:18-99): x bf16 with element

@@ -81,6 +81,17 @@ def test_mha_entry_point_on_given_operands_and_out_argument():
     assert torch.equal(vq[0].cpu(), eq[0]) and torch.equal(vq[1].cpu().view(torch.uint8), eq[1])
 
 
+# Launches whose last round is cut into workgroups of 256, 128 and 64 query rows (one round; 256 blocks and a rest of 4 and
+# 124), one kv tile, partial last tiles and groups of waves without a row of their own.
+@pytest.mark.parametrize("H,Nq,Nkv,D", [(1, 50, 20, 64), (2, 300, 129, 128), (3, 129, 1030, 128), (40, 513, 256, 64),
+                                        (130, 300, 200, 64), (190, 260, 300, 64)])
+def test_split_plans(H, Nq, Nkv, D):
+    q, k, v = make_input((1, H, Nq, D), seed=41), make_input((1, H, Nkv, D), seed=42), make_input((1, H, Nkv, D), seed=43)
+    o = ops().attention(q.cuda(), k.cuda(), v.cuda(), layout="BHND", precision="nvfp4")
+    ref = A.attention_nvfp4(q, k, v, "BHND")
+    torch.testing.assert_close(o.cpu().float(), ref.float(), atol=ATOL, rtol=RTOL)
+
+
 def test_attention_argument_checks():
     o = ops()
     q = make_input((1, 16, 1, 128), seed=1).cuda()
