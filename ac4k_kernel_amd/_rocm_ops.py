@@ -347,10 +347,7 @@ def mha_int8_x_fp8_fwd(o, q, q_sf, q_quantize_block_size: int, k, k_sf, k_quanti
                                           v_sf.data_ptr(), B, H, Nq, Nkv, Dqk, Dv, float(sm_scale), _stream()))
 
 
-def attention_int8_x_fp8(o, q, k, v, v_scale_max: float, sm_scale: float) -> bool:
-    """The whole `_int8_x_fp8_attention` (python/ac4k_kernel/ops/attention.py:137-190) behind one C call on bf16 q, k, v
-    viewed as [B,H,N,D] (any batch, head and token strides).  False, with nothing done, for operands this call does not
-    take - odd shapes and the ones an operator-by-operator call rejects with its own message."""
+def _attention(entry, workspace_bytes, o, q, k, v, scale: float, sm_scale: float) -> bool:
     B, H, Nq, Dqk = q.shape
     Nkv, Dv = k.shape[2], v.shape[3]
     if not (k.shape == (B, H, Nkv, Dqk) and v.shape == (B, H, Nkv, Dv) and o.shape == (B, H, Nq, Dv)
@@ -359,14 +356,25 @@ def attention_int8_x_fp8(o, q, k, v, v_scale_max: float, sm_scale: float) -> boo
     (q_b, q_h, q_n, q_d), (k_b, k_h, k_n, k_d), (v_b, v_h, v_n, v_d) = q.stride(), k.stride(), v.stride()
     if q_d != 1 or k_d != 1 or v_d != 1:
         return False
-    nbytes = _L.ac4k_attention_int8_x_fp8_workspace_bytes(B, H, Nq, Nkv, Dqk, Dv)
+    nbytes = workspace_bytes(B, H, Nq, Nkv, Dqk, Dv)
     if nbytes < 0:
         return False
     ws = torch.empty((nbytes,), dtype=torch.uint8, device=q.device)
-    _lib.check(_L.ac4k_attention_int8_x_fp8_bf16(o.data_ptr(), *o.stride(), q.data_ptr(), q_b, q_h, q_n, k.data_ptr(), k_b, k_h,
-                                                 k_n, v.data_ptr(), v_b, v_h, v_n, B, H, Nq, Nkv, Dqk, Dv, v_scale_max, sm_scale,
-                                                 ws.data_ptr(), nbytes, _stream()))
+    _lib.check(entry(o.data_ptr(), *o.stride(), q.data_ptr(), q_b, q_h, q_n, k.data_ptr(), k_b, k_h, k_n, v.data_ptr(), v_b, v_h, v_n,
+                     B, H, Nq, Nkv, Dqk, Dv, scale, sm_scale, ws.data_ptr(), nbytes, _stream()))
     return True
+
+
+def attention_int8_x_fp8(o, q, k, v, v_scale_max: float, sm_scale: float) -> bool:
+    """The whole `_int8_x_fp8_attention` (python/ac4k_kernel/ops/attention.py:137-190) behind one C call on bf16 q, k, v
+    viewed as [B,H,N,D] (any batch, head and token strides).  False, with nothing done, for operands this call does not
+    take - odd shapes and the ones an operator-by-operator call rejects with its own message."""
+    return _attention(_L.ac4k_attention_int8_x_fp8_bf16, _L.ac4k_attention_int8_x_fp8_workspace_bytes, o, q, k, v, v_scale_max, sm_scale)
+
+
+def attention_nvfp4(o, q, k, v, sm_scale: float) -> bool:
+    """The same for `_nvfp4_attention` (python/ac4k_kernel/ops/attention.py:100-133) on dense q, k, v."""
+    return _attention(_L.ac4k_attention_nvfp4_bf16, _L.ac4k_attention_nvfp4_workspace_bytes, o, q, k, v, 2688.0, sm_scale)
 
 
 def quantize_int8_token_block(y, scale, x_bhnd, block: int) -> None:

@@ -1021,14 +1021,33 @@ extern "C" __attribute__((visibility("default"))) int ac4k_quantize_int8_token_b
   return check_launch("ac4k_quantize_int8_token_block_bf16");
 }
 
-// Replaces _int8_x_fp8_attention (python/ac4k_kernel/ops/attention.py:137-190): the quantizers of attention_quantize.hip,
-// then ac4k_mha_int8_x_fp8_fwd on their outputs.
-static int attention_int8_args(AttnQuantArgs &a, int64_t B, int64_t H, int64_t Nq, int64_t Nkv, int64_t Dqk, int64_t Dv) {
+// Whole attention calls on bf16 operands: the quantizers of attention_quantize.hip, then the forward on their outputs.
+static int attention_check_sizes(int64_t B, int64_t H, int64_t Nq, int64_t Nkv, int64_t Dqk, int64_t Dv) {
   AC4K_REQUIRE(B >= 1 && H >= 1 && Nq >= 1 && Nkv >= 1, "B, H, Nq, Nkv must be positive (B=%lld H=%lld Nq=%lld Nkv=%lld)",
                (long long)B, (long long)H, (long long)Nq, (long long)Nkv);
   AC4K_REQUIRE(Dqk >= 8 && Dqk <= 128 && Dv >= 8 && Dv <= 128, "Dqk and Dv must be 8 to 128");
   AC4K_REQUIRE(H <= 65535 && B <= 65535 && Nq < (1ll << 30) && Nkv < (1ll << 30) &&
                B * H * (ceil_div(Nq, 64) + ceil_div(Nkv, 64)) < (1ll << 31), "problem too large");
+  return 0;
+}
+template <typename Args>
+static int attention_operands(Args &a, const void *q, int64_t q_b, int64_t q_h, int64_t q_n, const void *k, int64_t k_b, int64_t k_h,
+                              int64_t k_n, const void *v, int64_t v_b, int64_t v_h, int64_t v_n, const void *workspace) {
+  AC4K_REQUIRE(q && k && v && workspace, "null pointer argument");
+  AC4K_REQUIRE((((uintptr_t)q | (uintptr_t)k | (uintptr_t)v) & 1) == 0 && ((uintptr_t)workspace & 15) == 0,
+               "q, k, v must be 2-byte aligned and the workspace 16-byte aligned");
+  AC4K_REQUIRE(q_b >= 0 && q_h >= 0 && q_n >= 0 && k_b >= 0 && k_h >= 0 && k_n >= 0 && v_b >= 0 && v_h >= 0 && v_n >= 0,
+               "strides of q, k and v must not be negative");
+  a.q = {static_cast<const uint16_t *>(q), q_b, q_h, q_n};
+  a.k = {static_cast<const uint16_t *>(k), k_b, k_h, k_n};
+  a.v = {static_cast<const uint16_t *>(v), v_b, v_h, v_n};
+  return 0;
+}
+
+// Replaces _int8_x_fp8_attention (python/ac4k_kernel/ops/attention.py:137-190): the quantizers of attention_quantize.hip,
+// then ac4k_mha_int8_x_fp8_fwd on their outputs.
+static int attention_int8_args(AttnQuantArgs &a, int64_t B, int64_t H, int64_t Nq, int64_t Nkv, int64_t Dqk, int64_t Dv) {
+  if (int rc = attention_check_sizes(B, H, Nq, Nkv, Dqk, Dv)) return rc;
   a = AttnQuantArgs{};
   a.B = (int)B, a.H = (int)H, a.Nq = (int)Nq, a.Nkv = (int)Nkv, a.D = (int)Dqk, a.Dv = (int)Dv;
   return 0;
@@ -1046,23 +1065,58 @@ extern "C" __attribute__((visibility("default"))) int ac4k_attention_int8_x_fp8_
     int64_t q_h_stride, int64_t q_n_stride, const void *k, int64_t k_b_stride, int64_t k_h_stride, int64_t k_n_stride,
     const void *v, int64_t v_b_stride, int64_t v_h_stride, int64_t v_n_stride, int64_t B, int64_t H, int64_t Nq, int64_t Nkv,
     int64_t Dqk, int64_t Dv, float v_scale_max, float sm_scale, void *workspace, int64_t workspace_bytes, ac4k_stream_t stream) {
-  AC4K_REQUIRE(O && q && k && v && workspace, "null pointer argument");
+  AC4K_REQUIRE(O, "null pointer argument");
   AttnQuantArgs a;
   if (int rc = attention_int8_args(a, B, H, Nq, Nkv, Dqk, Dv)) return rc;
-  AC4K_REQUIRE((((uintptr_t)q | (uintptr_t)k | (uintptr_t)v) & 1) == 0 && ((uintptr_t)workspace & 15) == 0,
-               "q, k, v must be 2-byte aligned and the workspace 16-byte aligned");
-  AC4K_REQUIRE(q_b_stride >= 0 && q_h_stride >= 0 && q_n_stride >= 0 && k_b_stride >= 0 && k_h_stride >= 0 && k_n_stride >= 0 &&
-               v_b_stride >= 0 && v_h_stride >= 0 && v_n_stride >= 0, "strides of q, k and v must not be negative");
+  if (int rc = attention_operands(a, q, q_b_stride, q_h_stride, q_n_stride, k, k_b_stride, k_h_stride, k_n_stride, v, v_b_stride,
+                                  v_h_stride, v_n_stride, workspace)) return rc;
   AC4K_REQUIRE(v_scale_max > 0.0f, "v_scale_max must be positive");
   const int64_t need = attn_quant_layout(a, workspace);
   AC4K_REQUIRE(workspace_bytes >= need, "workspace too small: %lld bytes, %lld needed", (long long)workspace_bytes, (long long)need);
-  a.q = {static_cast<const uint16_t *>(q), q_b_stride, q_h_stride, q_n_stride};
-  a.k = {static_cast<const uint16_t *>(k), k_b_stride, k_h_stride, k_n_stride};
-  a.v = {static_cast<const uint16_t *>(v), v_b_stride, v_h_stride, v_n_stride};
   a.v_smax = v_scale_max;
   attn_quant_plan(a);
   launch_attn_quant(a, (hipStream_t)stream);
   if (int rc = check_launch("ac4k_attention_int8_x_fp8_bf16")) return rc;
   return ac4k_mha_int8_x_fp8_fwd(O, o_b_stride, o_h_stride, o_n_stride, o_d_stride, a.q8, a.q_sf, AQ_Q_BLOCK, a.k8, a.k_sf, AQ_K_BLOCK,
                                  a.v8, a.v_sf, B, H, Nq, Nkv, a.Dp, Dv, sm_scale, stream);
+}
+
+// Replaces _nvfp4_attention (python/ac4k_kernel/ops/attention.py:100-133).
+static int attention_nvfp4_args(AttnNvfp4Args &a, int64_t B, int64_t H, int64_t Nq, int64_t Nkv, int64_t Dqk, int64_t Dv) {
+  if (int rc = attention_check_sizes(B, H, Nq, Nkv, Dqk, Dv)) return rc;
+  a = AttnNvfp4Args{};
+  a.B = (int)B, a.H = (int)H, a.Nq = (int)Nq, a.Nkv = (int)Nkv, a.D = (int)Dqk, a.Dv = (int)Dv;
+  return 0;
+}
+
+extern "C" __attribute__((visibility("default"))) int64_t ac4k_attention_nvfp4_workspace_bytes(int64_t B, int64_t H, int64_t Nq,
+                                                                                               int64_t Nkv, int64_t Dqk, int64_t Dv) {
+  AttnNvfp4Args a;
+  if (attention_nvfp4_args(a, B, H, Nq, Nkv, Dqk, Dv)) return -1;
+  return attn_nvfp4_layout(a, nullptr);
+}
+
+extern "C" __attribute__((visibility("default"))) int ac4k_attention_nvfp4_bf16(
+    void *O, int64_t o_b_stride, int64_t o_h_stride, int64_t o_n_stride, int64_t o_d_stride, const void *q, int64_t q_b_stride,
+    int64_t q_h_stride, int64_t q_n_stride, const void *k, int64_t k_b_stride, int64_t k_h_stride, int64_t k_n_stride,
+    const void *v, int64_t v_b_stride, int64_t v_h_stride, int64_t v_n_stride, int64_t B, int64_t H, int64_t Nq, int64_t Nkv,
+    int64_t Dqk, int64_t Dv, float max_scale, float sm_scale, void *workspace, int64_t workspace_bytes, ac4k_stream_t stream) {
+  AC4K_REQUIRE(O, "null pointer argument");
+  AttnNvfp4Args a;
+  if (int rc = attention_nvfp4_args(a, B, H, Nq, Nkv, Dqk, Dv)) return rc;
+  if (int rc = attention_operands(a, q, q_b_stride, q_h_stride, q_n_stride, k, k_b_stride, k_h_stride, k_n_stride, v, v_b_stride,
+                                  v_h_stride, v_n_stride, workspace)) return rc;
+  // the maxima are taken over the whole tensors: [B,N,H,D] or [B,H,N,D] without gaps (dims of one element carry any stride)
+  auto dense = [&](const AttnOperand &t, int64_t N, int64_t D) {
+    const bool bnhd = (t.s_h == D || H == 1) && (t.s_n == H * D || N == 1), bhnd = (t.s_n == D || N == 1) && (t.s_h == N * D || H == 1);
+    return (bnhd || bhnd) && (t.s_b == H * N * D || B == 1);
+  };
+  AC4K_REQUIRE(dense(a.q, Nq, Dqk) && dense(a.k, Nkv, Dqk) && dense(a.v, Nkv, Dv), "q, k and v must be dense");
+  a.max_scale = max_scale;
+  const int64_t need = attn_nvfp4_layout(a, workspace);
+  AC4K_REQUIRE(workspace_bytes >= need, "workspace too small: %lld bytes, %lld needed", (long long)workspace_bytes, (long long)need);
+  launch_attn_nvfp4(a, (hipStream_t)stream);
+  if (int rc = check_launch("ac4k_attention_nvfp4_bf16")) return rc;
+  return ac4k_mha_nvfp4_fwd(O, o_b_stride, o_h_stride, o_n_stride, o_d_stride, a.q4, a.q_sf, a.gs, a.k4, a.k_sf, a.gs + 1, a.v4, a.v_sf,
+                            a.gs + 2, B, H, Nq, Nkv, a.Dp, Dv, sm_scale, stream);
 }

@@ -1,4 +1,4 @@
-// Front end of the INT8 x FP8 attention forward: quantization of bf16 Q, K and V into a workspace.
+// Front ends of the two attention forwards: quantization of bf16 Q, K and V into a workspace.
 #pragma once
 
 #include "ac4k_common.h"
@@ -31,6 +31,23 @@ struct AttnQuantArgs {
 int64_t attn_quant_layout(AttnQuantArgs &a, void *ws);  // -> bytes of the workspace (ws may be null: size only)
 void attn_quant_plan(AttnQuantArgs &a);
 void launch_attn_quant(const AttnQuantArgs &a, hipStream_t st);
+
+constexpr int AQ_MAX_PARTS = 256;  // workgroups per tensor of the maximum kernel
+
+struct AttnNvfp4Args {
+  AttnOperand q, k, v;  // dense
+  int B, H, Nq, Nkv, D, Dv;
+  float max_scale;
+  // filled by attn_nvfp4_layout: the operands of ac4k_mha_nvfp4_fwd and the partial maxima, all in the workspace
+  int Dp, Dvp, Nqp, Nkvp, Nkv64, nqt, nkt, nvt;
+  uint8_t *q4, *k4, *v4, *q_sf, *k_sf, *v_sf;
+  float *gs;             // global scales of Q, K, V, four bytes apart
+  uint32_t *parts;       // [3][AQ_MAX_PARTS]
+  int nparts[3];
+};
+
+int64_t attn_nvfp4_layout(AttnNvfp4Args &a, void *ws);
+void launch_attn_nvfp4(const AttnNvfp4Args &a, hipStream_t st);
 
 // int8 block scale = max|x| / 127 of a block of bf16 values, q = int8(trunc(x / scale)).
 // One correction step on x * (1 / scale) gives the correctly rounded quotient: residual by fma, times the correctly rounded

@@ -10,6 +10,7 @@
 // MI355X, quantizers alone: B 1, N 16384, H 40, D 128 (BNHD) 350 -> 250 us = 83 (4.0 TB/s) + 167 (4.5 TB/s), bit-identical
 // operands; a whole attention of 777 queries on 257 keys, B 2, H 12, D 64: 64 -> 26 us, three launches instead of nine.
 #include "attention_quantize.h"
+#include "quantize_nvfp4.h"
 
 namespace ac4k {
 
@@ -108,6 +109,20 @@ __global__ __launch_bounds__(64 * AQ_STAT_WAVES) void attn_column_stats_kernel(A
   __shared__ uint32_t red[AQ_STAT_WAVES][64][8];
   if (blockIdx.y == 0) aq_column_stats<false>(a, a.k, a.Nkv, a.D, a.ksum, red);
   else aq_column_stats<true>(a, a.v, a.Nkv, a.Dv, a.vmax, red);
+}
+
+// workgroup index -> tile: the dim that is nearer in memory runs fastest
+__device__ __forceinline__ void aq_tile(const AttnOperand &t, uint32_t H, uint32_t nblk, uint32_t idx, int &b, int &head, int &blk) {
+  const uint32_t inner = t.s_h < t.s_n ? H : nblk, i = idx % inner, o = idx / inner;
+  if (t.s_h < t.s_n) {
+    head = i;
+    blk = o % nblk;
+    b = o / nblk;
+  } else {
+    blk = i;
+    head = o % H;
+    b = o / H;
+  }
 }
 
 // ---- 2. the tiles ----------------------------------------------------------------------------------------------
@@ -224,33 +239,119 @@ __global__ __launch_bounds__(256) void attn_quantize_int8_fp8_kernel(AttnQuantAr
   __shared__ uint32_t wmax[4];
   uint32_t idx = blockIdx.x;
   const uint32_t BH = a.B * a.H;
-  // (workgroup index -> tile: the dim that is nearer in memory runs fastest)
-  auto tile = [&](const AttnOperand &t, uint32_t nblk, int &b, int &head, int &blk) {
-    uint32_t bh;
-    if (t.s_h < t.s_n) {
-      head = idx % a.H;
-      blk = (idx / a.H) % nblk;
-      b = idx / (a.H * nblk);
-    } else {
-      blk = idx % nblk;
-      bh = idx / nblk;
-      head = bh % a.H;
-      b = bh / a.H;
-    }
-  };
   int b, head, blk;
   const uint32_t nv = BH * a.nvb, nk = BH * a.nkb;
   if (idx < nv) {
-    tile(a.v, a.nvb, b, head, blk);
+    aq_tile(a.v, a.H, a.nvb, idx, b, head, blk);
     aq_fp8_tile(a, b, head, blk);
   } else if (idx < nv + nk) {
     idx -= nv;
-    tile(a.k, a.nkb, b, head, blk);
+    aq_tile(a.k, a.H, a.nkb, idx, b, head, blk);
     aq_int8_tile<AQ_K_BLOCK, true>(a, a.k, a.Nkv, a.nkb, a.k8, a.k_sf, b, head, blk, wmax);
   } else {
     idx -= nv + nk;
-    tile(a.q, a.nqb, b, head, blk);
+    aq_tile(a.q, a.H, a.nqb, idx, b, head, blk);
     aq_int8_tile<AQ_Q_BLOCK, false>(a, a.q, a.Nq, a.nqb, a.q8, a.q_sf, b, head, blk, wmax);
+  }
+}
+
+// ---- NVFP4 ------------------------------------------------------------------------------------------------------
+// (python/ac4k_kernel/ops/attention.py:100-133: three quantize calls) as two launches instead of up to nine: maxima of Q, K
+// and V as one partial result per workgroup, then tiles of all three, every workgroup taking the global scale of its
+// tensor from the partial results.  MI355X, B 1, N 4096, H 40, D 128 (BHND):
+// 73 -> 57 us (25 + 31: 5.0 and 5.2 TB/s) with bit-identical operands, the whole attention 440 -> 431 us.
+__global__ __launch_bounds__(512) void attn_nvfp4_absmax_kernel(AttnNvfp4Args a) {
+  const int t = blockIdx.y;
+  if ((int)blockIdx.x >= a.nparts[t]) return;
+  const uint16_t *x = t == 0 ? a.q.p : t == 1 ? a.k.p : a.v.p;
+  const int64_t n = (int64_t)a.B * a.H * (t == 0 ? a.Nq : a.Nkv) * (t == 2 ? a.Dv : a.D), nvec = n / 8;
+  constexpr int U = 8;  // loads in flight per lane
+  const int64_t span = align_up(ceil_div(nvec, (int64_t)a.nparts[t]), 512);
+  const int64_t beg = blockIdx.x * span, end = beg + span < nvec ? beg + span : nvec;
+  uint32_t m = 0;
+  for (int64_t i = beg + threadIdx.x; i < end; i += U * 512) {
+    uint4 v[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      v[u] = make_uint4(0, 0, 0, 0);
+      if (i + u * 512 < end) v[u] = aq_load(x + (i + u * 512) * 8);
+    }
+#pragma unroll
+    for (int u = 0; u < U; ++u) m = umax32(m, absmax_bf16x8(v[u]));
+  }
+  if (blockIdx.x == 0 && (int64_t)threadIdx.x < n - nvec * 8) m = umax32(m, x[nvec * 8 + threadIdx.x] & 0x7fffu);
+  m = group_umax<64>(m);
+  __shared__ uint32_t red[8];
+  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = m;
+  __syncthreads();
+  if (threadIdx.x == 0) {
+#pragma unroll
+    for (int w = 1; w < 8; ++w) m = umax32(m, red[w]);
+    a.parts[t * AQ_MAX_PARTS + blockIdx.x] = m;
+  }
+}
+
+// 128 tokens of one head, head dim contiguous: the row-major layout of the quantizers (a lane owns eight elements, a lane
+// pair a block, eight lanes a 64-chunk)
+__device__ __forceinline__ void aq_nvfp4_tile(const AttnNvfp4Args &a, const AttnOperand &t, int N, int Np, uint8_t *out, uint8_t *sf,
+                                              int b, int head, int blk, float alpha, const float *lut) {
+  const int tid = threadIdx.x, ls = a.Dp > 64 ? 4 : 3, c = tid & ((1 << ls) - 1), r0 = tid >> ls, rstep = 256 >> ls;
+  const int64_t bh = (int64_t)b * a.H + head;
+  const uint16_t *src = t.p + b * t.s_b + head * t.s_h + (int64_t)blk * 128 * t.s_n;
+  const int rows = N - blk * 128 < 128 ? N - blk * 128 : 128, rows_sf = Np - blk * 128 < 128 ? Np - blk * 128 : 128;
+  uint4 v[8];
+#pragma unroll
+  for (int j = 0; j < 8; ++j) {
+    const int r = r0 + j * rstep;
+    v[j] = make_uint4(0, 0, 0, 0);
+    if (r < rows && c * 8 < a.D) v[j] = ld_row_u4(src + r * t.s_n, c * 8, a.D);
+  }
+#pragma unroll
+  for (int j = 0; j < 8; ++j) {
+    const int r = r0 + j * rstep;
+    if (r >= 128) break;
+    v[j] = row_tail_u4(v[j], c * 8, a.D);
+    uint32_t m = absmax_bf16x8(v[j]), code;
+    m = umax32(m, dpp_u32<DPP_QUAD_XOR1>(m));
+    const float o = nvfp4_block_scale(bf16_bits_to_f32(m), alpha, lut, code);
+    if (r >= rows) code = 0;  // pad rows carry zero scales
+    const uint32_t packed = nvfp4_pack8(v[j], o);
+    const uint32_t sfw = code | (dpp_u32<DPP_ROW_SHL(2)>(code) << 8) | (dpp_u32<DPP_ROW_SHL(4)>(code) << 16) |
+                         (dpp_u32<DPP_ROW_SHL(6)>(code) << 24);
+    if (r < rows) *reinterpret_cast<uint32_t *>(out + (bh * N + blk * 128 + r) * (a.Dp / 2) + c * 4) = packed;
+    if ((c & 7) == 0 && r < rows_sf)
+      reinterpret_cast<uint32_t *>(sf)[(bh * (a.Dp / 64) + (c >> 3)) * Np + blk * 128 + r] = sfw;
+  }
+}
+
+__global__ __launch_bounds__(256) void attn_nvfp4_quantize_kernel(AttnNvfp4Args a) {
+  __shared__ float lut[128];
+  __shared__ uint32_t red[4];
+  uint32_t idx = blockIdx.x;
+  const uint32_t BH = a.B * a.H, nv = BH * a.nvt, nk = BH * a.nkt;
+  const int t = idx < nv ? 2 : idx < nv + nk ? 1 : 0;
+  idx -= t == 2 ? 0 : t == 1 ? nv : nv + nk;
+  uint32_t m = (int)threadIdx.x < a.nparts[t] ? a.parts[t * AQ_MAX_PARTS + threadIdx.x] : 0u;
+  m = group_umax<64>(m);
+  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = m;
+  load_rcp_table(lut);  // (ends with a barrier)
+  m = umax32(umax32(red[0], red[1]), umax32(red[2], red[3]));
+  const float gs = bf16_bits_to_f32(m) / a.max_scale, alpha = 1.0f / gs;
+  if (idx == 0 && threadIdx.x == 0) a.gs[t] = gs;
+  const AttnOperand &op = t == 2 ? a.v : t == 1 ? a.k : a.q;
+  const uint32_t nblk = t == 2 ? a.nvt : t == 1 ? a.nkt : a.nqt;
+  int b, head, blk;
+  aq_tile(op, a.H, nblk, idx, b, head, blk);
+  if (t == 2) {
+    const int lane = threadIdx.x & 63, cc = blk * 4 + (threadIdx.x >> 6), group0 = (lane >> 2) * 8;
+    if (cc * 64 >= a.Nkv64 || group0 >= a.Dvp) return;
+    const int64_t bh = (int64_t)b * a.H + head;
+    nvfp4_crossmajor_lane<true>(a.v4 + bh * a.Dv * (a.Nkv64 / 2), reinterpret_cast<uint32_t *>(a.v_sf) + (bh * (a.Nkv64 / 64) + cc) * a.Dvp,
+                                op.p + b * op.s_b + head * op.s_h, op.s_n, a.Dv, a.Nkv, a.Nkv64, cc, group0, lane & 3, alpha, lut);
+  } else if (t == 1) {
+    aq_nvfp4_tile(a, op, a.Nkv, a.Nkvp, a.k4, a.k_sf, b, head, blk, alpha, lut);
+  } else {
+    aq_nvfp4_tile(a, op, a.Nq, a.Nqp, a.q4, a.q_sf, b, head, blk, alpha, lut);
   }
 }
 
@@ -304,6 +405,36 @@ void launch_attn_quant(const AttnQuantArgs &a, hipStream_t st) {
   const int waves = a.span > 256 ? AQ_STAT_WAVES : 8;
   hipLaunchKernelGGL(attn_column_stats_kernel, dim3((unsigned)(uk > uv ? uk : uv), 2), dim3(64 * waves), 0, st, a);
   hipLaunchKernelGGL(attn_quantize_int8_fp8_kernel, dim3((unsigned)((int64_t)a.B * a.H * (a.nvb + a.nkb + a.nqb))), dim3(256), 0, st, a);
+}
+
+int64_t attn_nvfp4_layout(AttnNvfp4Args &a, void *ws) {
+  const int64_t BH = (int64_t)a.B * a.H;
+  a.Dp = (int)align_up(a.D, 64), a.Dvp = (int)align_up(a.Dv, 16), a.Nqp = (int)align_up(a.Nq, 16), a.Nkvp = (int)align_up(a.Nkv, 16);
+  a.Nkv64 = (int)align_up(a.Nkv, 64);
+  a.nqt = (int)ceil_div(a.Nqp, 128), a.nkt = (int)ceil_div(a.Nkvp, 128), a.nvt = (int)ceil_div(a.Nkv64, 256);
+  const int64_t n[3] = {BH * a.Nq * a.D, BH * a.Nkv * a.D, BH * a.Nkv * a.Dv};
+  for (int t = 0; t < 3; ++t) {  // 32 KB per workgroup and round of loads
+    const int64_t parts = ceil_div(n[t], 512 * 8 * 4);
+    a.nparts[t] = (int)(parts < 1 ? 1 : parts < AQ_MAX_PARTS ? parts : AQ_MAX_PARTS);
+  }
+  uint8_t *w = static_cast<uint8_t *>(ws);
+  int64_t at = 0;
+  a.q4 = w + take(at, BH * a.Nq * a.Dp / 2);
+  a.k4 = w + take(at, BH * a.Nkv * a.Dp / 2);
+  a.v4 = w + take(at, BH * a.Dv * (int64_t)a.Nkv64 / 2);
+  a.q_sf = w + take(at, BH * a.Dp / 16 * a.Nqp);
+  a.k_sf = w + take(at, BH * a.Dp / 16 * a.Nkvp);
+  a.v_sf = w + take(at, BH * (a.Nkv64 / 16) * a.Dvp);
+  a.gs = reinterpret_cast<float *>(w + take(at, 16));
+  a.parts = reinterpret_cast<uint32_t *>(w + take(at, 3 * AQ_MAX_PARTS * 4));
+  return at;
+}
+
+void launch_attn_nvfp4(const AttnNvfp4Args &a, hipStream_t st) {
+  int most = a.nparts[0] > a.nparts[1] ? a.nparts[0] : a.nparts[1];
+  if (a.nparts[2] > most) most = a.nparts[2];
+  hipLaunchKernelGGL(attn_nvfp4_absmax_kernel, dim3(most, 3), dim3(512), 0, st, a);
+  hipLaunchKernelGGL(attn_nvfp4_quantize_kernel, dim3((unsigned)((int64_t)a.B * a.H * (a.nvt + a.nkt + a.nqt))), dim3(256), 0, st, a);
 }
 
 }  // namespace ac4k

@@ -69,14 +69,19 @@ def _nvfp4_attention(q, k, v, layout, out=None):
         Nq, H = q.shape[1], q.shape[2]
     else:
         H, Nq = q.shape[1], q.shape[2]
+    if out is None:
+        out_shape = (B, Nq, H, Dv) if layout == "BNHD" else (B, H, Nq, Dv)
+        out = torch.empty(out_shape, dtype=torch.bfloat16, device=q.device)
+    bhnd = (lambda t: t.permute(0, 2, 1, 3)) if layout == "BNHD" else (lambda t: t)
+    o_bhnd = bhnd(out)  # the kernel writes through the strides
+    # the quantizers take dense tensors only; everything else goes operator by operator
+    if q.is_contiguous() and k.is_contiguous() and v.is_contiguous() and _rocm_ops.attention_nvfp4(
+            o_bhnd, bhnd(q), bhnd(k), bhnd(v), 1 / math.sqrt(Dqk)):
+        return out
     n_dim = 1 if layout == "BNHD" else 2
     q_fp4, q_sf, q_alpha = quantize(q, n_dim, 3)
     k_fp4, k_sf, k_alpha = quantize(k, n_dim, 3)
     v_fp4, v_sf, v_alpha = quantize(v, 3, n_dim, swizzle=True)
-    if out is None:
-        out_shape = (B, Nq, H, Dv) if layout == "BNHD" else (B, H, Nq, Dv)
-        out = torch.empty(out_shape, dtype=torch.bfloat16, device=q.device)
-    o_bhnd = out.permute(0, 2, 1, 3) if layout == "BNHD" else out  # the kernel writes through the strides
     mha_nvfp4_fwd(o_bhnd, q_fp4, q_sf, q_alpha, k_fp4, k_sf, k_alpha, v_fp4, v_sf, v_alpha, 1 / math.sqrt(Dqk))
     return out
 

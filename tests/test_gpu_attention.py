@@ -92,6 +92,19 @@ def test_split_plans(H, Nq, Nkv, D):
     torch.testing.assert_close(o.cpu().float(), ref.float(), atol=ATOL, rtol=RTOL)
 
 
+@pytest.mark.parametrize("B,Nq,Nkv,H,D,layout", [(1, 1, 1, 1, 8, "BNHD"), (3, 33, 31, 7, 71, "BNHD"), (2, 65, 257, 12, 64, "BNHD"),
+                                                 (2, 65, 257, 12, 64, "BHND"), (1, 64, 33, 5, 127, "BHND"), (1, 200, 2100, 9, 128, "BNHD"),
+                                                 (11, 100, 77, 12, 65, "BNHD"), (2, 64, 9000, 3, 100, "BHND"), (1, 40, 48, 2, 7, "BNHD")])
+def test_whole_call_equals_operator_by_operator(B, Nq, Nkv, H, D, layout, monkeypatch):
+    """The two-launch quantizers of attention() give the operands of the separate ones, so the outputs are equal."""
+    from ac4k_kernel_amd import _rocm_ops
+    shape = lambda n: (B, n, H, D) if layout == "BNHD" else (B, H, n, D)  # noqa: E731
+    q, k, v = (make_input(shape(n), seed=s, outliers=True).cuda() for s, n in ((1, Nq), (2, Nkv), (3, Nkv)))
+    got = ops().attention(q, k, v, layout=layout, precision="nvfp4")
+    monkeypatch.setattr(_rocm_ops, "attention_nvfp4", lambda *a: False)
+    assert torch.equal(got, ops().attention(q, k, v, layout=layout, precision="nvfp4"))
+
+
 def test_attention_argument_checks():
     o = ops()
     q = make_input((1, 16, 1, 128), seed=1).cuda()
