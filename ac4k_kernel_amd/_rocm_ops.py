@@ -146,7 +146,7 @@ def _check_linear_operand(x, x_sf, x_gs, rows, name):
 
 def _skinny_scratch(device, M, N, K):
     """Workspace tensor for the shapes that split K, or None when the shape needs no scratch."""
-    nbytes = _L.ac4k_linear_nvfp4_skinny_workspace_bytes(M, N, K)
+    nbytes = _L.ac4k_linear_nvfp4_workspace_bytes(M, N, K)
     if nbytes <= 0:
         return None
     return torch.empty((nbytes,), dtype=torch.uint8, device=device)
@@ -183,10 +183,10 @@ def linear_nvfp4(D, A, A_sf, A_global_scale, B, B_sf, B_global_scale, bias=None)
     scratch = _skinny_scratch(D.device, M, N, K)
     if scratch is not None:
         ws = scratch
-        _lib.check(_L.ac4k_linear_nvfp4_skinny(D.data_ptr(), _DTYPE_TAG[D.dtype], A.data_ptr(), A_sf.data_ptr(),
-                                               A_global_scale.data_ptr(), B.data_ptr(), B_sf.data_ptr(),
-                                               B_global_scale.data_ptr(), bias_ptr, bias_tag, M, N, K,
-                                               ws.data_ptr(), ws.numel(), _stream()))
+        _lib.check(_L.ac4k_linear_nvfp4_workspace(D.data_ptr(), _DTYPE_TAG[D.dtype], A.data_ptr(), A_sf.data_ptr(),
+                                                  A_global_scale.data_ptr(), B.data_ptr(), B_sf.data_ptr(),
+                                                  B_global_scale.data_ptr(), bias_ptr, bias_tag, M, N, K,
+                                                  ws.data_ptr(), ws.numel(), _stream()))
         return
     _lib.check(_L.ac4k_linear_nvfp4(D.data_ptr(), _DTYPE_TAG[D.dtype], A.data_ptr(), A_sf.data_ptr(),
                                     A_global_scale.data_ptr(), B.data_ptr(), B_sf.data_ptr(),

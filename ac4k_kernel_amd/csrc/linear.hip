@@ -268,7 +268,10 @@ __global__ __launch_bounds__(256) void linear_nvfp4_tile128_kernel(LinearArgs a)
 // step so that the next stage is readable before the current one ends.
 // Split-K: blockIdx.y selects a contiguous range of stages; with more than one range the
 // accumulators go to an fp32 partial buffer and a second kernel adds the ranges.
-// Requires K % 128 == 0 and 16-byte aligned operands.
+// Requires K % 64 == 0, K >= 128 and 16-byte aligned operands.  K % 128 == 64: the stages start one
+// chunk early, at k = -64, so that only stage 0 is special and the loop is not: the prologue fetches k-chunk 0
+// into both halves of it and clears the scales of the first half.  (1001 x 5003 x 2880, fp32 out: 75 -> 45 us, the
+// 128x128 kernel against this one; 300 x 4096 x 4160: 93 -> 28.)
 // ===========================================================================
 constexpr int P_BK = 128;     // k per stage (two 64-chunks)
 constexpr int P_ROW = 64;     // packed bytes per row per stage: [chunk][half] x 16 B
@@ -472,8 +475,9 @@ __global__ __launch_bounds__(256, 1) void linear_nvfp4_tile256p_kernel(LinearArg
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int wm = wave >> 1, wn = wave & 1;
   const int half = lane >> 5;
-  // this workgroup's range of 128-k stages
-  const int nkt_all = (int)(a.K / P_BK);
+  // this workgroup's range of 128-k stages; `early`: bytes by which they start in front of the row (K % 128 == 64)
+  const int nkt_all = (int)ceil_div(a.K, P_BK);
+  const int early = (int)((a.K & 64) >> 1);
   const int kt0 = (int)((int64_t)nkt_all * blockIdx.y / sk.splits);
   const int nkt = (int)((int64_t)nkt_all * (blockIdx.y + 1) / sk.splits) - kt0;
 
@@ -514,8 +518,8 @@ __global__ __launch_bounds__(256, 1) void linear_nvfp4_tile256p_kernel(LinearArg
     }
   }
   const int64_t strideB = a.prepacked ? W_BLOCK_BYTES : P_ROW;  // bytes per stage along k
-  const uint8_t *baseA = uniform_ptr(a.A + tm * BM * kb + (int64_t)kt0 * P_ROW);
-  const uint8_t *baseB = uniform_ptr(a.prepacked ? a.B + (int64_t)kt0 * W_BLOCK_BYTES : a.B + tn * BN * kb + (int64_t)kt0 * P_ROW);
+  const uint8_t *baseA = uniform_ptr(a.A + tm * BM * kb + (int64_t)kt0 * P_ROW - early);
+  const uint8_t *baseB = uniform_ptr(a.prepacked ? a.B + (int64_t)kt0 * W_BLOCK_BYTES : a.B + tn * BN * kb + (int64_t)kt0 * P_ROW - early);
   // scale transfers: piece g = swave * NS + p (past the last piece: the last piece again, which
   // lands the same bytes in the same place).  g < NSA: operand A, chunk g / (BM/64), 64-row block
   // g % (BM/64); otherwise operand B, chunk (g-NSA) / (BN/64), block (g-NSA) % (BN/64).  Source
@@ -525,6 +529,7 @@ __global__ __launch_bounds__(256, 1) void linear_nvfp4_tile256p_kernel(LinearArg
   uint32_t offS[NS], ldsS[NS];
   const uint8_t *baseS[NS];
   int64_t strideS[NS];
+  uint32_t firstS = 0;  // bit p2: scale transfer p2 moves the first chunk of a stage
 #pragma unroll
   for (int p2 = 0; p2 < NS; ++p2) {
     const int gq = swave * NS + p2 < NSA + NSB ? swave * NS + p2 : NSA + NSB - 1;
@@ -543,8 +548,9 @@ __global__ __launch_bounds__(256, 1) void linear_nvfp4_tile256p_kernel(LinearArg
       sr = sr < rows ? sr : rows - 1;
       offS[p2] = (uint32_t)sr * 4u;  // byte offset inside a scale plane
       strideS[p2] = 2 * rows * 4;    // two planes (chunks) per stage
-      baseS[p2] = uniform_ptr((isB ? sfB8 : sfA8) + c * rows * 4 + kt0 * strideS[p2]);
+      baseS[p2] = uniform_ptr((isB ? sfB8 : sfA8) + (c - (early ? 1 : 0)) * rows * 4 + kt0 * strideS[p2]);
     }
+    if (c == 0) firstS |= 1u << p2;
     ldsS[p2] = (uint32_t)__builtin_amdgcn_readfirstlane((isB ? PL::OFF_SFB + c * BN * 4 : PL::OFF_SFA + c * BM * 4) + rb * 256);
   }
   const uint32_t lds_base = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) char *)plds;
@@ -673,18 +679,40 @@ __global__ __launch_bounds__(256, 1) void linear_nvfp4_tile256p_kernel(LinearArg
   // visible, chunk 0 fragments and first decode
   static_assert(PS >= 3 && (PS - 2) * NPIECES <= 63, "the wait counts below must fit the 6-bit counter");
   const int last = nkt - 1;
+  // the stage that fetches past the end repeat: never the short one, whose first half lies in front of the rows
+  // (a range of one stage then repeats the stage behind it, which exists: K >= 192)
+  const bool short0 = early && kt0 == 0;
+  const int again = short0 && last == 0 ? 1 : last;
+  if (short0) {  // k-chunk 0 into both halves
+    Src p = src_at(0);
+    const uint32_t shift = dma_piece < 2 ? 32u : 0u;
 #pragma unroll
-  for (int d = 0; d < PS - 1; ++d) issue_stage(lds_base + d * PL::STAGE_BYTES, src_at(d < last ? d : last));
+    for (int q = 0; q < NDA; ++q) dma16(p.a, offA[q] + shift, lds_base, ldsA[q]);
+#pragma unroll
+    for (int q = 0; q < NDB; ++q) dma16(p.b, offB[q] + shift, lds_base, ldsB[q]);
+#pragma unroll
+    for (int p2 = 0; p2 < NS; ++p2) dma4(p.s[p2] + ((firstS >> p2 & 1) ? strideS[p2] / 2 : 0), offS[p2], lds_base, ldsS[p2]);
+  } else {
+    issue_stage(lds_base, src_at(0));
+  }
+#pragma unroll
+  for (int d = 1; d < PS - 1; ++d) issue_stage(lds_base + d * PL::STAGE_BYTES, src_at(d < last ? d : again));
   wait_vmcnt<(PS - 2) * NPIECES>();  // everything of stage 0 has landed, later stages may be in flight
   __syncthreads();
   load_chunk(0, 0);
+  if (short0) {
+#pragma unroll
+    for (int i = 0; i < MI; ++i) SA[0][i] = (f16x2){(_Float16)0.0f, (_Float16)0.0f};
+#pragma unroll
+    for (int j = 0; j < NJ; ++j) SB[0][j] = (f16x2){(_Float16)0.0f, (_Float16)0.0f};
+  }
   decode(D[0], 0, I0{});
 
   // loop-carried, wave-uniform: LDS offsets of the stages holding k-steps kt, kt+1 and of the one
   // being filled with kt+PS-1 (a ring of PS), and the source pointers of k-step min(kt+PS-1, last)
   uint32_t st_cur = 0, st_nxt = PL::STAGE_BYTES, st_dma = (PS - 1) * PL::STAGE_BYTES;
   auto ring_next = [](uint32_t o) { return o + PL::STAGE_BYTES == (uint32_t)PL::LDS_BYTES ? 0u : o + PL::STAGE_BYTES; };
-  Src src = src_at(last < PS - 1 ? last : PS - 1);
+  Src src = src_at(last < PS - 1 ? again : PS - 1);
 #ifdef AC4K_LINEAR_TIMELINE
   const uint64_t tl_c0 = __builtin_readcyclecounter();
 #endif
@@ -818,9 +846,9 @@ static TilePlan tile_plan(int64_t M, int64_t N, int64_t K, bool allow_split) {
   TilePlan best{M <= 128 ? 2 : 4, 4, 1, 0};
   if (const uint32_t f = g_forced_tile_plan.load(std::memory_order_relaxed)) {
     const int mi = f & 0xff, nj = (f >> 8) & 0xff, sp = (int)(f >> 16);
-    if (sp <= K / P_BK && (sp == 1 || allow_split)) return TilePlan{mi, nj, sp, sp > 1 ? (int64_t)sp * M * N * 4 : 0};
+    if (sp <= ceil_div(K, P_BK) && (sp == 1 || allow_split)) return TilePlan{mi, nj, sp, sp > 1 ? (int64_t)sp * M * N * 4 : 0};
   }
-  const int64_t stages = K / P_BK;
+  const int64_t stages = ceil_div(K, P_BK);
   if (ceil_div(M, 64 * best.mi) * ceil_div(N, 256) >= 192) return best;
   double best_t = 0.0;
   bool first = true;
@@ -875,8 +903,33 @@ static int launch_tile256p(const LinearArgs &a, hipStream_t st) {
 // per stage.  The four k parts of the tile meet through LDS at the end: wave w receives the sums of a
 // quarter of the tile from the other three, adds them in wave order, and stores its quarter
 // (times gsA * gsB, plus bias), or the raw fp32 sums of this K range when K is split over workgroups.
-// Requires K % 256 == 0 and 16-byte aligned operands and scale tensors.
+// Requires K % 64 == 0, K >= 256 and 16-byte aligned operands and scale tensors.  The last stage of any other K
+// starts early enough to be whole, and the chunks of it that the stage before holds too count as zero.
+// (100 x 5003 x 2880: 66 -> 20 us, the 128x128 kernel against this one.)
 // ===========================================================================
+// Kernels with stages of four chunks.  TAIL: K is no multiple of 256 (a variant of its own: the few scalar instructions
+// a stage that it needs cost the other K 2 % in the K-split-waves kernel and 5 % in the LDS-ring kernels).  Of `nch` >= 4
+// chunks the last stage takes the last four; chunk c of it counts for nothing when the stage before holds it too:
+// `weight_factor` multiplies the weight scales, by 1 or by so little that the fp16 scale rounds to zero (the scale
+// conversion takes a power of two at no cost).  `offset` is where a stage starts, from the row's first chunk (TAIL) or
+// from the first one of the workgroup's range, given the bytes per chunk.
+template <bool TAIL>
+struct StageWalk {
+  int s0, nch;  // first stage of the range, chunks in the row
+  __device__ __forceinline__ int chunk(int st) const { return 4 * (s0 + st) < nch - 4 ? 4 * (s0 + st) : nch - 4; }
+  template <typename T>
+  __device__ __forceinline__ int64_t offset(int st, T per_chunk) const {
+    if constexpr (TAIL) return chunk(st) * (int64_t)per_chunk;
+    else return st * (int64_t)(4 * per_chunk);
+  }
+  template <typename T>
+  __device__ __forceinline__ int64_t start(T per_chunk) const { return TAIL ? 0 : s0 * (int64_t)(4 * per_chunk); }
+  __device__ __forceinline__ float weight_factor(int st, int c) const {
+    if constexpr (TAIL) return 4 * (s0 + st) - chunk(st) > c ? 0x1p-60f : 1.0f;
+    else return 1.0f;
+  }
+};
+
 constexpr int KW_BK = 256;          // k per stage
 constexpr int KW_ROW = KW_BK / 2;   // packed bytes per row per stage
 
@@ -900,7 +953,7 @@ struct KWLayout {
   static_assert(LDS_BYTES >= 16 * PPW * 4096, "the ring doubles as the exchange buffer of the four k parts");
 };
 
-template <int D_DT, int BIAS_DT, int MI, int NJ>
+template <int D_DT, int BIAS_DT, int MI, int NJ, bool TAIL>
 __global__ __launch_bounds__(256, 1) void linear_nvfp4_ksplit_kernel(LinearArgs a, SplitK sk) {
   using L = KWLayout<MI, NJ>;
   constexpr int BM = L::BM, BN = L::BN, PS = L::PS, NP = L::NPIECES;
@@ -911,9 +964,10 @@ __global__ __launch_bounds__(256, 1) void linear_nvfp4_ksplit_kernel(LinearArgs 
   const int64_t tiles_n = ceil_div(a.N, BN);
   const int64_t tm = blockIdx.x / tiles_n, tn = blockIdx.x % tiles_n;
   const int64_t m0 = tm * BM, n0 = tn * BN;
-  const int nst_all = (int)(a.K / KW_BK);
+  const int nst_all = (int)ceil_div(a.K, KW_BK);
   const int s0 = (int)((int64_t)nst_all * blockIdx.y / sk.splits);
   const int nst = (int)((int64_t)nst_all * (blockIdx.y + 1) / sk.splits) - s0;  // >= 1: splits <= stages
+  const StageWalk<TAIL> walk{s0, (int)(a.K >> 6)};
   const int64_t kb = a.K >> 1;
   // workgroup b starts at stage b % nst of its range and wraps around, so that the workgroups of a
   // launch do not all ask for the same column of their rows at the same time (memory channels)
@@ -933,7 +987,7 @@ __global__ __launch_bounds__(256, 1) void linear_nvfp4_ksplit_kernel(LinearArgs 
   const int64_t img_band_bytes = (a.K / W_BLOCK_K) * (int64_t)W_BLOCK_BYTES;
   uint32_t offR[L::NROW], ldsR[L::NROW];
   const uint8_t *srcR[L::NROW];
-  int strR[L::NROW];  // bytes per stage along k
+  int strR[L::NROW];  // bytes per chunk along k
 #pragma unroll
   for (int q = 0; q < L::NROW; ++q) {
     const int t = swave * L::NROW + q;
@@ -944,14 +998,14 @@ __global__ __launch_bounds__(256, 1) void linear_nvfp4_ksplit_kernel(LinearArgs 
       const int64_t wrow = n0 + loc;  // rows past N exist in the image (zeros)
       const int64_t band = wrow / W_BLOCK_ROWS, within = wrow % W_BLOCK_ROWS;
       offR[q] = (uint32_t)(band * img_band_bytes + (pp >> 2) * W_BLOCK_BYTES + within * 64 + (((pp & 3) ^ ((within >> 1) & 3)) * 16));
-      srcR[q] = uniform_ptr(a.B + (int64_t)s0 * (2 * W_BLOCK_BYTES));
-      strR[q] = 2 * W_BLOCK_BYTES;
+      strR[q] = W_BLOCK_BYTES / 2;
+      srcR[q] = uniform_ptr(a.B + walk.start(strR[q]));
     } else {
       const int64_t rows = isW ? a.N : a.M, first = isW ? n0 : m0;
       const int64_t row = first + loc < rows ? loc : rows - 1 - first;  // rows past the matrix read its last row
       offR[q] = (uint32_t)(row * kb + pp * 16);
-      srcR[q] = uniform_ptr((isW ? a.B + n0 * kb : a.A + m0 * kb) + (int64_t)s0 * KW_ROW);
-      strR[q] = KW_ROW;
+      strR[q] = KW_ROW / 4;
+      srcR[q] = uniform_ptr((isW ? a.B + n0 * kb : a.A + m0 * kb) + walk.start(strR[q]));
     }
     strR[q] = __builtin_amdgcn_readfirstlane(strR[q]);
     ldsR[q] = (uint32_t)__builtin_amdgcn_readfirstlane(t * 1024);
@@ -974,24 +1028,25 @@ __global__ __launch_bounds__(256, 1) void linear_nvfp4_ksplit_kernel(LinearArgs 
     if (isW && a.prepacked) {
       const int64_t band = row / W_BLOCK_ROWS, within = row % W_BLOCK_ROWS;
       offS = (uint32_t)(band * img_band_bytes + (chunk >> 1) * W_BLOCK_BYTES + W_BLOCK_DATA + (chunk & 1) * (W_BLOCK_ROWS * 4) + within * 4);
-      strideS = 2 * W_BLOCK_BYTES;
-      srcS = uniform_ptr(a.B + s0 * strideS);
+      strideS = W_BLOCK_BYTES / 2;
+      srcS = uniform_ptr(a.B + walk.start(strideS));
     } else {
       row = row + 4 <= rows_p ? row : rows_p - 4;         // groups past the padded rows read the last group
       offS = (uint32_t)((chunk * rows_p + row) * 4);
-      strideS = 4 * rows_p * 4;                           // bytes per stage: four chunk planes
-      srcS = uniform_ptr(reinterpret_cast<const uint8_t *>(isW ? a.B_sf : a.A_sf) + s0 * strideS);
+      strideS = rows_p * 4;                               // bytes per chunk plane
+      srcS = uniform_ptr(reinterpret_cast<const uint8_t *>(isW ? a.B_sf : a.A_sf) + walk.start(strideS));
     }
     ldsS = (uint32_t)__builtin_amdgcn_readfirstlane((isW ? L::OFF_SFW : L::OFF_SFA) + tt * 1024);
   }
   // Transfer q of this wave's NPIECES for stage `st` into the ring slot at `base`.  Past the end of the range
   // the loop keeps issuing, so that it stays free of branches and its wait counts stay fixed: those transfers
   // read the last stage again (cache hits) into slots nobody reads any more.
+  // (`st` counts from the start of the range; a weight image has K % 128 == 0, so its stages start at whole blocks)
   auto issue_piece = [&](uint32_t base, int st, int q) {
     if (q < L::NROW)
-      dma16(srcR[q] + (int64_t)st * strR[q], offR[q], base, ldsR[q]);
+      dma16(srcR[q] + walk.offset(st, strR[q]), offR[q], base, ldsR[q]);
     else
-      dma16(srcS + st * strideS, offS, base, ldsS);
+      dma16(srcS + walk.offset(st, strideS), offS, base, ldsS);
   };
   // the transfers of a stage are issued in four parts, one per 16-k sub-step
   auto issue_part = [&](uint32_t base, int st, int part) {
@@ -1005,14 +1060,16 @@ __global__ __launch_bounds__(256, 1) void linear_nvfp4_ksplit_kernel(LinearArgs 
   struct Frags {
     uint4 x[MI], w[NJ];
     uint32_t xs[MI], ws[NJ];
+    float wfac;
   };
   const int piece = swave * 2 + half;
   const int f_off = r32 * KW_ROW + ((piece ^ (r32 & 7)) * 16);  // rows 32 apart share the swizzle term
   const int ws_off = L::OFF_SFW + (swave * BN + r32) * 4 + half * 2;
   const int xs_off = L::OFF_SFA + (swave * BM + r32) * 4 + half * 2;
-  auto load_frags = [&](int slot) {
+  auto load_frags = [&](int slot, int step) {
     const char *st = kwlds + slot * L::STAGE_BYTES;
     Frags f;
+    f.wfac = walk.weight_factor(stage_of(step), swave);
 #pragma unroll
     for (int j = 0; j < NJ; ++j) {
       f.w[j] = *reinterpret_cast<const uint4 *>(st + L::OFF_W + f_off + j * 32 * KW_ROW);
@@ -1039,7 +1096,7 @@ __global__ __launch_bounds__(256, 1) void linear_nvfp4_ksplit_kernel(LinearArgs 
     constexpr int s = decltype(S)::value;
 #pragma unroll
     for (int j = 0; j < NJ; ++j)
-      d.b[j] = decode_dword<(s >= 2)>(dword_of<s>(f.w[j]), __builtin_amdgcn_cvt_scalef32_pk_f16_fp8(f.ws[j], 1.0f, false));
+      d.b[j] = decode_dword<(s >= 2)>(dword_of<s>(f.w[j]), __builtin_amdgcn_cvt_scalef32_pk_f16_fp8(f.ws[j], f.wfac, false));
 #pragma unroll
     for (int i = 0; i < MI; ++i)
       d.a[i] = decode_dword<(s >= 2)>(dword_of<s>(f.x[i]), __builtin_amdgcn_cvt_scalef32_pk_f16_fp8(f.xs[i], 1.0f, false));
@@ -1077,7 +1134,7 @@ __global__ __launch_bounds__(256, 1) void linear_nvfp4_ksplit_kernel(LinearArgs 
   }
   wait_vmcnt<(PS - 1) * NP>();
   __syncthreads();
-  Frags F0 = load_frags(0), F1;
+  Frags F0 = load_frags(0, 0), F1;
   decode(D[0], F0, I0{});
   wait_vmcnt<(PS - 2) * NP>();
   asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
@@ -1097,7 +1154,7 @@ __global__ __launch_bounds__(256, 1) void linear_nvfp4_ksplit_kernel(LinearArgs 
     const uint32_t base_new = lds_base + slot_cur * L::STAGE_BYTES;
     // fragments of the next stage (it landed before the previous barrier) travel from LDS while this
     // one is decoded and multiplied (past the range: a stage nobody uses)
-    nxt = load_frags(slot_next);
+    nxt = load_frags(slot_next, s + 1);
     decode(D[1], cur, I1{});
     issue_part(base_new, st_new, 0);
     mfma_all(D[0]);
@@ -1206,9 +1263,10 @@ __global__ __launch_bounds__(256, 1) void linear_nvfp4_ksplit_kernel(LinearArgs 
 template <int D_DT, int BIAS_DT, int MI, int NJ>
 static int launch_ksplit_t(const LinearArgs &a, const SplitK &sk, hipStream_t st) {
   using L = KWLayout<MI, NJ>;
-  auto *kern = linear_nvfp4_ksplit_kernel<D_DT, BIAS_DT, MI, NJ>;
-  static std::atomic<uint32_t> lds_ok{0};
-  if (int rc = allow_dynamic_lds(kern, lds_ok, L::LDS_BYTES)) return rc;
+  const bool tail = a.K % KW_BK != 0;
+  auto *kern = tail ? linear_nvfp4_ksplit_kernel<D_DT, BIAS_DT, MI, NJ, true> : linear_nvfp4_ksplit_kernel<D_DT, BIAS_DT, MI, NJ, false>;
+  static std::atomic<uint32_t> lds_ok[2];
+  if (int rc = allow_dynamic_lds(kern, lds_ok[tail], L::LDS_BYTES)) return rc;
   const int64_t ntiles = ceil_div(a.M, L::BM) * ceil_div(a.N, L::BN);
   hipLaunchKernelGGL(kern, dim3((unsigned)ntiles, (unsigned)sk.splits), dim3(256), L::LDS_BYTES, st, a, sk);
   return 0;
@@ -1223,7 +1281,7 @@ struct KsplitPlan {
 
 // shapes the K-split-waves kernel takes (its pointer conditions are in ksplit_aligned)
 static bool ksplit_shape(int64_t M, int64_t N, int64_t K) {
-  return M > 32 && M <= 128 && N >= 64 && K >= KW_BK && K % KW_BK == 0 && (K >> 1) * 128 < (1ll << 31) && N < (1ll << 27) &&
+  return M > 32 && M <= 128 && N >= 64 && K >= KW_BK && K % 64 == 0 && (K >> 1) * 128 < (1ll << 31) && N < (1ll << 27) &&
          g_forced_tile_plan.load(std::memory_order_relaxed) == 0;
 }
 static bool ksplit_aligned(const LinearArgs &a) {
@@ -1235,7 +1293,7 @@ static bool ksplit_aligned(const LinearArgs &a) {
 static KsplitPlan ksplit_plan(int64_t M, int64_t N, int64_t K, bool allow_split) {
   KsplitPlan p{M <= 64 ? 2 : 4, 2, 1, 0};
   if (M <= 64 && ceil_div(N, 128) >= 192) p.nj = 4;
-  const int64_t tiles = ceil_div(M, 32 * p.mi) * ceil_div(N, 32 * p.nj), stages = K / KW_BK;
+  const int64_t tiles = ceil_div(M, 32 * p.mi) * ceil_div(N, 32 * p.nj), stages = ceil_div(K, KW_BK);
   int64_t splits = 1;
   if (allow_split) {
     if (const int f = g_forced_skinny_ks.load(std::memory_order_relaxed)) {  // forced length of a K range
@@ -1502,7 +1560,9 @@ static void launch_reduce(const SkinnyArgs &a, hipStream_t st) {
 }
 
 // ===========================================================================
-// Decode-sized linear (1 <= M <= 32, K % 256 == 0): the weights are streamed once, through LDS.
+// Decode-sized linear (1 <= M <= 32, K % 64 == 0, K >= 256): the weights are streamed once, through LDS.
+// (The last stage of a K that is no multiple of 256 is treated as in the K-split-waves kernel: 1 x 28672 x 8320
+// 177 -> 36 us, 16 x 4096 x 14400 307 -> 18 us, the 128x128 kernel against these.)
 //
 // A workgroup (8 waves) owns 128 weight rows and a contiguous range of 256-k stages.  Weights, weight
 // scales, the packed activation rows and their scales go from global memory straight into an LDS ring
@@ -1552,13 +1612,14 @@ constexpr int ST_PRE_NPIECES = 3;
 struct StageFrags {
   uint4 w[2], x[2];
   uint32_t ws[2], xs[2];
+  float wfac[2];
 };
 
 // acc[c] += W . Xhat^T over the wave's two chunks of a stage (decode in registers)
 __device__ __forceinline__ void stream_multiply(const StageFrags &cur, f32x16 (&acc)[2]) {
 #pragma unroll
   for (int c = 0; c < 2; ++c) {
-    const f16x2 wsc = __builtin_amdgcn_cvt_scalef32_pk_f16_fp8(cur.ws[c], 1.0f, false);
+    const f16x2 wsc = __builtin_amdgcn_cvt_scalef32_pk_f16_fp8(cur.ws[c], cur.wfac[c], false);
     const f16x2 xsc = __builtin_amdgcn_cvt_scalef32_pk_f16_fp8(cur.xs[c], 1.0f, false);
     acc[c] = __builtin_amdgcn_mfma_f32_32x32x16_f16(decode_dword<false>(cur.w[c].x, wsc), decode_dword<false>(cur.x[c].x, xsc), acc[c], 0, 0, 0);
     acc[c] = __builtin_amdgcn_mfma_f32_32x32x16_f16(decode_dword<false>(cur.w[c].y, wsc), decode_dword<false>(cur.x[c].y, xsc), acc[c], 0, 0, 0);
@@ -1642,7 +1703,7 @@ __device__ __forceinline__ void stream_finish(f32x16 (&acc)[2], const SkinnyArgs
   }
 }
 
-template <int D_DT, int BIAS_DT, bool PRE, int MR>
+template <int D_DT, int BIAS_DT, bool PRE, int MR, bool TAIL>
 __global__ __launch_bounds__(ST_THREADS, 1) void linear_nvfp4_stream_kernel(SkinnyArgs a) {
   static_assert(MR == 32 || MR == 16, "activation rows per stage");
   constexpr int NPIECES = PRE ? ST_PRE_NPIECES : ST_NPIECES;
@@ -1653,9 +1714,10 @@ __global__ __launch_bounds__(ST_THREADS, 1) void linear_nvfp4_stream_kernel(Skin
   const int swave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int wn = swave & 3, kh = swave >> 2;
   const int64_t n0 = (int64_t)blockIdx.x * ST_BN;
-  const int nst_all = (int)(a.K / ST_BK);
+  const int nst_all = (int)ceil_div(a.K, ST_BK);
   const int s0 = (int)((int64_t)nst_all * blockIdx.y / a.split_k);
   const int nst = (int)((int64_t)nst_all * (blockIdx.y + 1) / a.split_k) - s0;  // >= 1: split_k <= stages
+  const StageWalk<TAIL> walk{s0, (int)(a.K >> 6)};
   const int64_t kb = a.K >> 1;
   // Workgroup b walks its stages starting at stage b % nst and wraps around.  In step, every workgroup
   // would ask for the same 128-byte column of its rows at the same time; with a row pitch that is a
@@ -1683,8 +1745,8 @@ __global__ __launch_bounds__(ST_THREADS, 1) void linear_nvfp4_stream_kernel(Skin
     offW[0] = (uint32_t)(swave * 2048 + lane * 16);
     offW[1] = offW[0] + 1024;
     offW[2] = (uint32_t)((16 + swave) * 1024 + lane * 16);
-    strideW = ST_PRE_W_BYTES;
-    srcW = uniform_ptr(a.B + ((int64_t)blockIdx.x * (a.K / W_BLOCK_K) + 2 * (int64_t)s0) * W_BLOCK_BYTES);
+    strideW = W_BLOCK_BYTES / 2;  // bytes per chunk (K % 128 == 0: a stage starts at a whole block)
+    srcW = uniform_ptr(a.B + (int64_t)blockIdx.x * (a.K / W_BLOCK_K) * W_BLOCK_BYTES + walk.start(strideW));
     ldsW = (uint32_t)__builtin_amdgcn_readfirstlane(swave * 2048);
   } else {
     // weight rows swave * 16 + {0..7}, {8..15}, 128 B each
@@ -1696,8 +1758,8 @@ __global__ __launch_bounds__(ST_THREADS, 1) void linear_nvfp4_stream_kernel(Skin
       offW[q] = (uint32_t)((row - n0) * kb + ((lane & 7) ^ (loc & 7)) * 16);
     }
     offW[2] = 0;
-    strideW = ST_ROW;
-    srcW = uniform_ptr(a.B + n0 * kb + (int64_t)s0 * ST_ROW);
+    strideW = ST_ROW / 4;
+    srcW = uniform_ptr(a.B + n0 * kb + walk.start(strideW));
     ldsW = (uint32_t)__builtin_amdgcn_readfirstlane(ST_OFF_B + swave * 2048);
   }
   // weight scales from the scale tensor: chunk swave / 2, rows (swave % 2) * 64 + lane of the tile
@@ -1708,8 +1770,8 @@ __global__ __launch_bounds__(ST_THREADS, 1) void linear_nvfp4_stream_kernel(Skin
     int64_t srow = n0 + (swave & 1) * 64 + lane;
     srow = srow < a.Np ? srow : a.Np - 1;
     offS = (uint32_t)(srow * 4);
-    strideS = 4 * a.Np * 4;  // bytes per stage (four chunk planes)
-    srcS = uniform_ptr(reinterpret_cast<const uint8_t *>(a.B_sf) + (int64_t)(swave >> 1) * a.Np * 4 + s0 * strideS);
+    strideS = a.Np * 4;  // bytes per chunk plane
+    srcS = uniform_ptr(reinterpret_cast<const uint8_t *>(a.B_sf) + (int64_t)(swave >> 1) * a.Np * 4 + walk.start(strideS));
     ldsS = (uint32_t)__builtin_amdgcn_readfirstlane(ST_OFF_SFB + (swave >> 1) * (ST_BN * 4) + (swave & 1) * 256);
   }
   // activation: MR / 8 waves take the packed rows w * 8 + {0..7}; the scale dwords are one transfer for
@@ -1726,12 +1788,12 @@ __global__ __launch_bounds__(ST_THREADS, 1) void linear_nvfp4_stream_kernel(Skin
     const int loc = (swave - A_FIRST) * 8 + (lane >> 3);
     const int64_t row = loc < a.M ? loc : a.M - 1;  // rows past M read row M - 1; their outputs are never stored
     off4 = (uint32_t)(row * kb + ((lane & 7) ^ (loc & 7)) * 16);
-    stride4 = ST_ROW;
-    src4 = uniform_ptr(a.Aq + (int64_t)s0 * ST_ROW);
+    stride4 = ST_ROW / 4;
+    src4 = uniform_ptr(a.Aq + walk.start(stride4));
     lds4 = (uint32_t)__builtin_amdgcn_readfirstlane(OFF_A + (swave - A_FIRST) * 1024);
   } else if (!PRE || swave >= 2) {
-    stride4 = 4 * a.Mp * 4;
-    src4 = uniform_ptr(a.A_sf + s0 * stride4);
+    stride4 = a.Mp * 4;
+    src4 = uniform_ptr(a.A_sf + walk.start(stride4));
     if constexpr (MR == 32) {
       const int pair = swave & 1;  // chunks 2 pair, 2 pair + 1
       const int64_t row = r32 < a.Mp ? r32 : a.Mp - 1;
@@ -1745,22 +1807,22 @@ __global__ __launch_bounds__(ST_THREADS, 1) void linear_nvfp4_stream_kernel(Skin
   auto issue_stage = [&](int slot, int step) {  // step: position in this workgroup's order of stages
     const int st = stage_of(step);
     const uint32_t base = lds_base + slot * ST_STAGE_BYTES;
-    const uint8_t *pw = srcW + (int64_t)st * strideW;
+    const uint8_t *pw = srcW + walk.offset(st, strideW);
     dma16(pw, offW[0], base, ldsW);
     dma16(pw, offW[1], base, ldsW + 1024);
     if constexpr (PRE) {
       if (swave < 2)
         dma16(pw, offW[2], base, (uint32_t)__builtin_amdgcn_readfirstlane((16 + swave) * 1024));
       else if (moves_rows)
-        dma16(src4 + st * stride4, off4, base, lds4);
+        dma16(src4 + walk.offset(st, stride4), off4, base, lds4);
       else
-        dma4(src4 + st * stride4, off4, base, lds4);
+        dma4(src4 + walk.offset(st, stride4), off4, base, lds4);
     } else {
-      dma4(srcS + st * strideS, offS, base, ldsS);
+      dma4(srcS + walk.offset(st, strideS), offS, base, ldsS);
       if (moves_rows)
-        dma16(src4 + st * stride4, off4, base, lds4);
+        dma16(src4 + walk.offset(st, stride4), off4, base, lds4);
       else
-        dma4(src4 + st * stride4, off4, base, lds4);
+        dma4(src4 + walk.offset(st, stride4), off4, base, lds4);
     }
   };
 
@@ -1780,7 +1842,7 @@ __global__ __launch_bounds__(ST_THREADS, 1) void linear_nvfp4_stream_kernel(Skin
   constexpr int ws_pitch = PRE ? W_BLOCK_ROWS * 4 : ST_BN * 4;
   const int ws_off = (PRE ? kh * W_BLOCK_BYTES + W_BLOCK_DATA : ST_OFF_SFB + (kh * 2) * (ST_BN * 4)) + wrow_l * 4 + half * 2;
   const int xs_off = OFF_SFA + (kh * 2) * (MR * 4) + xrow * 4 + half * 2;
-  auto load_frags = [&](int slot) {
+  auto load_frags = [&](int slot, int step) {
     const char *st = stlds + slot * ST_STAGE_BYTES;
     StageFrags f;
 #pragma unroll
@@ -1789,6 +1851,7 @@ __global__ __launch_bounds__(ST_THREADS, 1) void linear_nvfp4_stream_kernel(Skin
       f.x[c] = *reinterpret_cast<const uint4 *>(st + xf_off[c]);
       f.ws[c] = *reinterpret_cast<const uint16_t *>(st + ws_off + c * ws_pitch);
       f.xs[c] = *reinterpret_cast<const uint16_t *>(st + xs_off + c * (MR * 4));
+      f.wfac[c] = walk.weight_factor(stage_of(step), 2 * kh + c);
     }
     return f;
   };
@@ -1806,13 +1869,13 @@ __global__ __launch_bounds__(ST_THREADS, 1) void linear_nvfp4_stream_kernel(Skin
   for (int d = 0; d < ST_PS - 1; ++d) issue_stage(d, d < last ? d : last);
   wait_vmcnt<(ST_PS - 3) * NPIECES>();
   __syncthreads();
-  StageFrags cur = load_frags(0);
+  StageFrags cur = load_frags(0, 0);
 
   int slot_next = 1, slot_dma = ST_PS - 1;
   for (int s = 0; s < nst; ++s) {
     // fragments of the next stage (it landed before the previous barrier) travel from LDS while this
     // stage is decoded and multiplied (past the range: a stage nobody uses)
-    const StageFrags nxt = load_frags(slot_next);
+    const StageFrags nxt = load_frags(slot_next, s + 1 < nst ? s + 1 : s);
     stream_multiply(cur, acc);
     // refill the slot of the stage before this one (everybody read it before the previous barrier)
     const int sd = s + ST_PS - 1;
@@ -1850,16 +1913,17 @@ static_assert(S6_LDS_BYTES <= 160 * 1024, "the ring must fit in the CU's LDS");
 static_assert((S6_PS - 3) * S6_NPIECES <= 63, "the wait counts must fit the 6-bit counter");
 static_assert(S6_LDS_BYTES >= 3 * 2 * 64 * 16 * 4, "the ring doubles as the exchange buffer of the four k parts");
 
-template <int D_DT, int BIAS_DT>
+template <int D_DT, int BIAS_DT, bool TAIL>
 __global__ __launch_bounds__(ST_THREADS, 1) void linear_nvfp4_stream64_kernel(SkinnyArgs a) {
   extern __shared__ __attribute__((aligned(16))) char stlds[];
   const int tid = threadIdx.x, lane = tid & 63, half = lane >> 5, r32 = lane & 31;
   const int swave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int wn = swave & 1, kq = swave >> 1;
   const int64_t n0 = (int64_t)blockIdx.x * S6_BN;
-  const int nst_all = (int)(a.K / ST_BK);
+  const int nst_all = (int)ceil_div(a.K, ST_BK);
   const int s0 = (int)((int64_t)nst_all * blockIdx.y / a.split_k);
   const int nst = (int)((int64_t)nst_all * (blockIdx.y + 1) / a.split_k) - s0;  // >= 1: split_k <= stages
+  const StageWalk<TAIL> walk{s0, (int)(a.K >> 6)};
   const int64_t kb = a.K >> 1;
   const int rot = (int)(blockIdx.x % (unsigned)nst);  // stages are walked from stage b % nst on (see linear_nvfp4_stream_kernel)
   auto stage_of = [&](int step) {
@@ -1875,7 +1939,7 @@ __global__ __launch_bounds__(ST_THREADS, 1) void linear_nvfp4_stream64_kernel(Sk
     row = row < a.N ? row : a.N - 1;  // rows past N read the last row; their outputs are never stored
     offW = (uint32_t)((row - n0) * kb + ((lane & 7) ^ (loc & 7)) * 16);
   }
-  const uint8_t *srcW = uniform_ptr(a.B + n0 * kb + (int64_t)s0 * ST_ROW);
+  const uint8_t *srcW = uniform_ptr(a.B + n0 * kb + walk.start(ST_ROW / 4));
   const uint32_t ldsW = (uint32_t)__builtin_amdgcn_readfirstlane(S6_OFF_B + swave * 1024);
   // (2) waves 0..3: weight scale dwords of chunk swave, rows n0 + lane; waves 4..7: packed activation
   //     rows (swave - 4) * 8 + {0..7}
@@ -1886,15 +1950,15 @@ __global__ __launch_bounds__(ST_THREADS, 1) void linear_nvfp4_stream64_kernel(Sk
     int64_t srow = n0 + lane;
     srow = srow < a.Np ? srow : a.Np - 1;
     off2 = (uint32_t)(srow * 4);
-    stride2 = 4 * a.Np * 4;  // bytes per stage (four chunk planes)
-    src2 = uniform_ptr(reinterpret_cast<const uint8_t *>(a.B_sf) + (int64_t)swave * a.Np * 4 + s0 * stride2);
+    stride2 = a.Np * 4;  // bytes per chunk plane
+    src2 = uniform_ptr(reinterpret_cast<const uint8_t *>(a.B_sf) + (int64_t)swave * a.Np * 4 + walk.start(stride2));
     lds2 = (uint32_t)__builtin_amdgcn_readfirstlane(S6_OFF_SFB + swave * (S6_BN * 4));
   } else {
     const int loc = (swave - 4) * 8 + (lane >> 3);
     const int64_t row = loc < a.M ? loc : a.M - 1;  // rows past M read row M - 1; their outputs are never stored
     off2 = (uint32_t)(row * kb + ((lane & 7) ^ (loc & 7)) * 16);
-    stride2 = ST_ROW;
-    src2 = uniform_ptr(a.Aq + (int64_t)s0 * ST_ROW);
+    stride2 = ST_ROW / 4;
+    src2 = uniform_ptr(a.Aq + walk.start(stride2));
     lds2 = (uint32_t)__builtin_amdgcn_readfirstlane(S6_OFF_A + (swave - 4) * 1024);
   }
   // (3) activation scales of chunks 2 p + {0, 1}, p = swave % 2 (waves 2..7 repeat the transfers of waves
@@ -1902,18 +1966,18 @@ __global__ __launch_bounds__(ST_THREADS, 1) void linear_nvfp4_stream64_kernel(Sk
   const int pair = swave & 1;
   const int64_t arow = r32 < a.Mp ? r32 : a.Mp - 1;
   const uint32_t off3 = (uint32_t)(((2 * pair + half) * a.Mp + arow) * 4);
-  const int64_t stride3 = 4 * a.Mp * 4;
-  const uint8_t *src3 = uniform_ptr(a.A_sf + s0 * stride3);
+  const int64_t stride3 = a.Mp * 4;
+  const uint8_t *src3 = uniform_ptr(a.A_sf + walk.start(stride3));
   const uint32_t lds3 = (uint32_t)__builtin_amdgcn_readfirstlane(S6_OFF_SFA + pair * 256);
   auto issue_stage = [&](int slot, int step) {  // step: position in this workgroup's order of stages
     const int st = stage_of(step);
     const uint32_t base = lds_base + slot * S6_STAGE_BYTES;
-    dma16(srcW + (int64_t)st * ST_ROW, offW, base, ldsW);
+    dma16(srcW + walk.offset(st, ST_ROW / 4), offW, base, ldsW);
     if (swave < 4)
-      dma4(src2 + st * stride2, off2, base, lds2);
+      dma4(src2 + walk.offset(st, stride2), off2, base, lds2);
     else
-      dma16(src2 + st * stride2, off2, base, lds2);
-    dma4(src3 + st * stride3, off3, base, lds3);
+      dma16(src2 + walk.offset(st, stride2), off2, base, lds2);
+    dma4(src3 + walk.offset(st, stride3), off3, base, lds3);
   };
 
   // this wave's fragments of a stage: chunk kq, 32 packed elements of a weight row and of an activation
@@ -1921,6 +1985,7 @@ __global__ __launch_bounds__(ST_THREADS, 1) void linear_nvfp4_stream64_kernel(Sk
   struct Frags {
     uint4 w, x;
     uint32_t ws, xs;
+    float wfac;
   };
   const int wrow_l = wn * 32 + r32;
   const int piece = kq * 2 + half;
@@ -1928,9 +1993,10 @@ __global__ __launch_bounds__(ST_THREADS, 1) void linear_nvfp4_stream64_kernel(Sk
   const int xf_off = S6_OFF_A + r32 * ST_ROW + ((piece ^ (r32 & 7)) * 16);
   const int ws_off = S6_OFF_SFB + kq * (S6_BN * 4) + wrow_l * 4 + half * 2;
   const int xs_off = S6_OFF_SFA + kq * (32 * 4) + r32 * 4 + half * 2;
-  auto load_frags = [&](int slot) {
+  auto load_frags = [&](int slot, int step) {
     const char *st = stlds + slot * S6_STAGE_BYTES;
     Frags f;
+    f.wfac = walk.weight_factor(stage_of(step), kq);
     f.w = *reinterpret_cast<const uint4 *>(st + wf_off);
     f.x = *reinterpret_cast<const uint4 *>(st + xf_off);
     f.ws = *reinterpret_cast<const uint16_t *>(st + ws_off);
@@ -1949,12 +2015,12 @@ __global__ __launch_bounds__(ST_THREADS, 1) void linear_nvfp4_stream64_kernel(Sk
   for (int d = 0; d < S6_PS - 1; ++d) issue_stage(d, d < last ? d : last);
   wait_vmcnt<(S6_PS - 3) * S6_NPIECES>();
   __syncthreads();
-  Frags cur = load_frags(0);
+  Frags cur = load_frags(0, 0);
 
   int slot_next = 1, slot_dma = S6_PS - 1;
   for (int s = 0; s < nst; ++s) {
-    const Frags nxt = load_frags(slot_next);  // it landed before the previous barrier
-    const f16x2 wsc = __builtin_amdgcn_cvt_scalef32_pk_f16_fp8(cur.ws, 1.0f, false);
+    const Frags nxt = load_frags(slot_next, s + 1 < nst ? s + 1 : s);  // it landed before the previous barrier
+    const f16x2 wsc = __builtin_amdgcn_cvt_scalef32_pk_f16_fp8(cur.ws, cur.wfac, false);
     const f16x2 xsc = __builtin_amdgcn_cvt_scalef32_pk_f16_fp8(cur.xs, 1.0f, false);
     acc[0] = __builtin_amdgcn_mfma_f32_32x32x16_f16(decode_dword<false>(cur.w.x, wsc), decode_dword<false>(cur.x.x, xsc), acc[0], 0, 0, 0);
     acc[0] = __builtin_amdgcn_mfma_f32_32x32x16_f16(decode_dword<false>(cur.w.y, wsc), decode_dword<false>(cur.x.y, xsc), acc[0], 0, 0, 0);
@@ -2006,7 +2072,7 @@ static void plan_registers(int64_t M, int64_t N, int64_t K, SkinnyPlan &p) {
 static void plan_lds_ring(int64_t M, int64_t N, int64_t K, SkinnyPlan &p, int rows = ST_BN) {
   p.kind = rows == ST_BN ? DECODE_LDS_RING : DECODE_LDS_RING64;
   p.groups = ceil_div(N, rows);
-  const int64_t stages = K / ST_BK;
+  const int64_t stages = ceil_div(K, ST_BK);
   int64_t splits = 1;
   if (const int f = g_forced_skinny_ks.load(std::memory_order_relaxed)) {  // forced length of a K range
     splits = K / f;
@@ -2023,7 +2089,7 @@ static void plan_lds_ring(int64_t M, int64_t N, int64_t K, SkinnyPlan &p, int ro
   p.lds_bytes = rows == ST_BN ? st_lds_bytes(M <= 16 ? 16 : 32) : S6_LDS_BYTES;
 }
 
-// Shapes of the decode-sized kernels (all need K % 256 == 0) and the choice between them.  The
+// Shapes of the decode-sized kernels (K % 64 == 0, the register kernel K % 256 == 0) and the choice between them.  The
 // register kernel has all its loads in flight at once and four workgroups per CU, which wins while M
 // is small and the problem needs a K split anyway (few row tiles, long K); it pays for partial sums
 // and a second launch, and its registers run out as M grows.  The LDS-ring kernels take nearly the
@@ -2034,13 +2100,18 @@ static void plan_lds_ring(int64_t M, int64_t N, int64_t K, SkinnyPlan &p, int ro
 //   N = 14336, K = 4096 (112 / 224 tiles):  M = 1 14.0 / 15.5 / 13.8, M = 8 14.5 / 15.8 / 14.2, M = 16 17.6 / 16.4 / 13.9, M = 32 22.1 / 17.2 / 14.9
 //   N = 4096, K = 14336 (32 / 64 tiles):    M = 1 15.1 / 16.8 / 16.2, M = 8 16.3 / 17.3 / 16.3, M = 16 18.7 / 17.5 / 16.9, M = 32 22.9 / 17.8 / 17.1
 // Hence: with 192 tiles of 128 rows and more, 128-row tiles from M = 8 on; otherwise 64-row tiles when
-// there are 192 of those, or from M = 8 on; the register kernel in the remaining cases.
+// there are 192 of those, or from M = 8 on; the register kernel in the remaining cases.  A K that is no multiple of
+// 256 takes the ring kernels for every M.
 static bool skinny_plan(int64_t M, int64_t N, int64_t K, SkinnyPlan &p) {
-  if (M < 1 || M > 32 || K < SK_STEP || K % SK_STEP != 0 || N < 1) return false;
+  if (M < 1 || M > 32 || K < SK_STEP || K % 64 != 0 || N < 1) return false;
   const bool ring_ok = (K >> 1) * ST_BN < (1ll << 31) && N < (1ll << 27);  // 32-bit lane offsets
+  const bool whole = K % SK_STEP == 0;
+  if (!whole && !ring_ok) return false;
   int kind = g_forced_decode_kernel.load(std::memory_order_relaxed);
-  if (kind == 0) {
-    if (ceil_div(N, ST_BN) >= 192)
+  if (kind == 0 || (kind == DECODE_REGISTERS && !whole)) {
+    if (!whole)
+      kind = ceil_div(N, ST_BN) >= 192 ? DECODE_LDS_RING : DECODE_LDS_RING64;
+    else if (ceil_div(N, ST_BN) >= 192)
       kind = M >= 8 ? DECODE_LDS_RING : DECODE_REGISTERS;
     else
       kind = (M >= 8 || ceil_div(N, S6_BN) >= 192) ? DECODE_LDS_RING64 : DECODE_REGISTERS;
@@ -2065,9 +2136,10 @@ static int launch_skinny_it(const SkinnyArgs &a, const SkinnyPlan &p, hipStream_
 
 template <int D_DT, int BIAS_DT, bool PRE, int MR>
 static int launch_ring(const SkinnyArgs &a, const SkinnyPlan &p, hipStream_t st) {
-  auto *kern = linear_nvfp4_stream_kernel<D_DT, BIAS_DT, PRE, MR>;
-  static std::atomic<uint32_t> lds_ok{0};
-  if (int rc = allow_dynamic_lds(kern, lds_ok, st_lds_bytes(MR))) return rc;
+  const bool tail = a.K % ST_BK != 0;
+  auto *kern = tail ? linear_nvfp4_stream_kernel<D_DT, BIAS_DT, PRE, MR, true> : linear_nvfp4_stream_kernel<D_DT, BIAS_DT, PRE, MR, false>;
+  static std::atomic<uint32_t> lds_ok[2];
+  if (int rc = allow_dynamic_lds(kern, lds_ok[tail], st_lds_bytes(MR))) return rc;
   hipLaunchKernelGGL(kern, dim3((unsigned)p.groups, (unsigned)p.split_k), dim3(ST_THREADS), st_lds_bytes(MR), st, a);
   return 0;
 }
@@ -2082,9 +2154,10 @@ static int launch_skinny(const SkinnyArgs &a, const SkinnyPlan &p, hipStream_t s
       rc = a.prepacked ? launch_ring<D_DT, BIAS_DT, true, 32>(a, p, st) : launch_ring<D_DT, BIAS_DT, false, 32>(a, p, st);
     if (rc) return rc;
   } else if (p.kind == DECODE_LDS_RING64) {
-    auto *kern = linear_nvfp4_stream64_kernel<D_DT, BIAS_DT>;
-    static std::atomic<uint32_t> lds_ok{0};
-    if (int rc = allow_dynamic_lds(kern, lds_ok, S6_LDS_BYTES)) return rc;
+    const bool tail = a.K % ST_BK != 0;
+    auto *kern = tail ? linear_nvfp4_stream64_kernel<D_DT, BIAS_DT, true> : linear_nvfp4_stream64_kernel<D_DT, BIAS_DT, false>;
+    static std::atomic<uint32_t> lds_ok[2];
+    if (int rc = allow_dynamic_lds(kern, lds_ok[tail], S6_LDS_BYTES)) return rc;
     hipLaunchKernelGGL(kern, dim3((unsigned)p.groups, (unsigned)p.split_k), dim3(ST_THREADS), S6_LDS_BYTES, st, a);
   } else {
     int rc;
@@ -2117,10 +2190,10 @@ static int dispatch_skinny(const SkinnyArgs &a, const SkinnyPlan &p, int d_dtype
   return set_error("d must be bfloat16, half or float (dtype tag %d)", d_dtype);
 }
 
-// shapes the packed-LDS kernel takes: whole 128-k stages, 16-byte aligned rows, 32-bit lane offsets
+// shapes the packed-LDS kernel takes: whole 64-chunks, 16-byte aligned rows, 32-bit lane offsets
 // (256 operand rows in the loop, 4 output rows of up to 4-byte elements in the epilogue)
 static bool packed_kernel_ok(const LinearArgs &a) {
-  return a.K % P_BK == 0 && (((uintptr_t)a.A | (uintptr_t)a.B) & 15) == 0 && (a.K >> 1) * 256 < (1ll << 31) &&
+  return a.K % 64 == 0 && a.K >= P_BK && (((uintptr_t)a.A | (uintptr_t)a.B) & 15) == 0 && (a.K >> 1) * 256 < (1ll << 31) &&
          a.N < (1ll << 27);
 }
 
@@ -2142,7 +2215,7 @@ static bool noscratch_skinny_plan(const LinearArgs &a, SkinnyPlan &p) {
 
 // Decode-sized M goes to the weight-streaming kernels, 32 < M <= 128 to the K-split-waves kernel, larger
 // M to the packed-operand tile kernel, each whenever its layout conditions hold; the 128x128 kernel,
-// which has no condition beyond K % 64 == 0, takes everything else.
+// which has no condition beyond K % 16 == 0, takes everything else.
 template <int D_DT, int BIAS_DT>
 static int launch_linear(const LinearArgs &a, hipStream_t st) {
   SkinnyPlan sp;
@@ -2223,7 +2296,7 @@ struct MidPlan {
 };
 // shapes the workspace entry point takes with 32 < M
 static bool mid_plan(int64_t M, int64_t N, int64_t K, MidPlan &p) {
-  if (M <= 32 || N < 128 || K % P_BK != 0 || (K >> 1) * 256 >= (1ll << 31) || N >= (1ll << 27)) return false;
+  if (M <= 32 || N < 128 || K % 64 != 0 || K < P_BK || (K >> 1) * 256 >= (1ll << 31) || N >= (1ll << 27)) return false;
   p.tp = tile_plan(M, N, K, true);
   p.has_ksplit = ksplit_shape(M, N, K);
   p.kp = p.has_ksplit ? ksplit_plan(M, N, K, true) : KsplitPlan{0, 0, 1, 0};
@@ -2321,12 +2394,23 @@ static int check_skinny(const SkinnyPlan &p, bool ok, const void *B, void *works
 
 }  // namespace ac4k
 
-extern "C" __attribute__((visibility("default"))) int64_t ac4k_linear_nvfp4_skinny_workspace_bytes(int64_t M, int64_t N, int64_t K) {
+extern "C" __attribute__((visibility("default"))) int64_t ac4k_linear_nvfp4_workspace_bytes(int64_t M, int64_t N, int64_t K) {
   SkinnyPlan p;
   if (skinny_plan(M, N, K, p)) return p.partial_bytes;
   MidPlan mp;
   if (mid_plan(M, N, K, mp)) return mp.bytes;
   return 0;
+}
+
+namespace ac4k {
+
+// K that the `skinny` entry points take: whole stages of the kernels they began with
+static bool skinny_entry_k(int64_t M, int64_t K) { return K % (M > 32 ? P_BK : SK_STEP) == 0; }
+
+}  // namespace ac4k
+
+extern "C" __attribute__((visibility("default"))) int64_t ac4k_linear_nvfp4_skinny_workspace_bytes(int64_t M, int64_t N, int64_t K) {
+  return skinny_entry_k(M, K) ? ac4k_linear_nvfp4_workspace_bytes(M, N, K) : 0;
 }
 
 namespace ac4k {
@@ -2340,7 +2424,7 @@ static int linear_skinny_impl(void *D, int d_dtype, const void *A, const void *A
   AC4K_REQUIRE(M >= 1 && N >= 1 && K >= 1, "M, N, K must be positive (M=%lld N=%lld K=%lld)", (long long)M,
                (long long)N, (long long)K);
   MidPlan mp;
-  if (M > 32 && mid_plan(M, N, K, mp)) {  // few tiles, long K: split-K
+  if (M > 32 && skinny_entry_k(M, K) && mid_plan(M, N, K, mp)) {  // few tiles, long K: split-K
     AC4K_REQUIRE((((uintptr_t)A | (uintptr_t)B) & 15) == 0 && (((uintptr_t)A_sf | (uintptr_t)B_sf) & 3) == 0,
                  "A and B must be 16-byte aligned and the scale tensors 4-byte aligned");
     if (mp.bytes > 0) {  // one K range per tile needs no scratch
@@ -2355,7 +2439,7 @@ static int linear_skinny_impl(void *D, int d_dtype, const void *A, const void *A
     return check_launch(what);
   }
   SkinnyPlan p;
-  const bool ok = skinny_plan(M, N, K, p);
+  const bool ok = skinny_entry_k(M, K) && skinny_plan(M, N, K, p);
   if (int rc = check_skinny(p, ok, B, workspace, workspace_bytes)) return rc;
   AC4K_REQUIRE(((uintptr_t)A & 15) == 0, "A must be 16-byte aligned");
   if (int rc = run_skinny(D, d_dtype, A, A_sf, A_gs, B, B_sf, B_gs, bias, bias_dtype, M, N, K, p, workspace, st))
@@ -2398,6 +2482,36 @@ extern "C" __attribute__((visibility("default"))) int ac4k_linear_nvfp4_skinny(v
                                         int64_t workspace_bytes, ac4k_stream_t stream) {
   return linear_skinny_impl(D, d_dtype, A, A_sf, A_gs, B, B_sf, B_gs, bias, bias_dtype, M, N, K, workspace,
                             workspace_bytes, (hipStream_t)stream, "ac4k_linear_nvfp4_skinny");
+}
+
+extern "C" __attribute__((visibility("default"))) int ac4k_linear_nvfp4_workspace(void *D, int d_dtype, const void *A, const void *A_sf, const float *A_gs,
+                                        const void *B, const void *B_sf, const float *B_gs, const void *bias,
+                                        int bias_dtype, int64_t M, int64_t N, int64_t K, void *workspace,
+                                        int64_t workspace_bytes, ac4k_stream_t stream) {
+  const int64_t need = ac4k_linear_nvfp4_workspace_bytes(M, N, K);
+  if (need == 0 || skinny_entry_k(M, K))
+    return need == 0 ? ac4k_linear_nvfp4(D, d_dtype, A, A_sf, A_gs, B, B_sf, B_gs, bias, bias_dtype, M, N, K, stream)
+                     : linear_skinny_impl(D, d_dtype, A, A_sf, A_gs, B, B_sf, B_gs, bias, bias_dtype, M, N, K, workspace,
+                                          workspace_bytes, (hipStream_t)stream, "ac4k_linear_nvfp4_workspace");
+  // every other K: operands that are not aligned for the split kernels run without scratch
+  if (!(D && A && A_sf && A_gs && B && B_sf && B_gs) || (((uintptr_t)A | (uintptr_t)B) & 15) || (((uintptr_t)A_sf | (uintptr_t)B_sf) & 3))
+    return ac4k_linear_nvfp4(D, d_dtype, A, A_sf, A_gs, B, B_sf, B_gs, bias, bias_dtype, M, N, K, stream);
+  AC4K_REQUIRE(workspace && ((uintptr_t)workspace & 255) == 0, "workspace must be 256-byte aligned");
+  AC4K_REQUIRE(workspace_bytes >= need, "workspace too small: %lld bytes needed", (long long)need);
+  int rc;
+  SkinnyPlan p;
+  MidPlan mp;
+  if (skinny_plan(M, N, K, p)) {
+    rc = run_skinny(D, d_dtype, A, A_sf, A_gs, B, B_sf, B_gs, bias, bias_dtype, M, N, K, p, workspace, (hipStream_t)stream);
+  } else {
+    mid_plan(M, N, K, mp);
+    LinearArgs la{D, static_cast<const uint8_t *>(A), static_cast<const uint8_t *>(B),
+                  static_cast<const uint32_t *>(A_sf), static_cast<const uint32_t *>(B_sf), A_gs, B_gs, bias,
+                  M, N, K, align_up(M, 16), align_up(N, 16)};
+    rc = dispatch_mid(la, mp, static_cast<float *>(workspace), workspace_bytes, d_dtype, bias_dtype, (hipStream_t)stream);
+  }
+  if (rc) return rc;
+  return check_launch("ac4k_linear_nvfp4_workspace");
 }
 
 extern "C" __attribute__((visibility("default"))) int ac4k_linear_nvfp4_skinny_static(void *D, int d_dtype, const void *A, const void *A_sf,
@@ -2458,7 +2572,7 @@ struct PrepackedPlan {
 static bool prepacked_plan(int64_t M, int64_t N, int64_t K, PrepackedPlan &p) {
   const int64_t bytes = weight_image_bytes(N, K);
   if (M < 1 || bytes == 0 || bytes >= (1ll << 32) || (K >> 1) * 256 >= (1ll << 31) || N >= (1ll << 27)) return false;
-  p.ring = M <= 32 && K % ST_BK == 0;
+  p.ring = M <= 32 && K >= ST_BK;
   p.mid = !p.ring && ksplit_shape(M, N, K);
   if (p.ring) {
     plan_lds_ring(M, N, K, p.sp);
@@ -2551,7 +2665,7 @@ extern "C" __attribute__((visibility("default"))) int ac4k_linear_nvfp4_fused_bf
   AC4K_REQUIRE(M >= 1 && M <= 32, "the fused skinny linear takes 1 <= M <= 32 (got %lld)", (long long)M);
   AC4K_REQUIRE(N >= 1 && K >= 1, "N and K must be positive (N=%lld K=%lld)", (long long)N, (long long)K);
   SkinnyPlan p;
-  const bool ok = skinny_plan(M, N, K, p);
+  const bool ok = skinny_entry_k(M, K) && skinny_plan(M, N, K, p);
   if (int rc = check_skinny(p, ok, B, workspace, workspace_bytes)) return rc;
   hipStream_t st = (hipStream_t)stream;
   AC4K_REQUIRE(((uintptr_t)X & 15) == 0, "activation must be 16-byte aligned");

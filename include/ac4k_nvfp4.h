@@ -147,6 +147,15 @@ int ac4k_linear_nvfp4_skinny(void *D, int d_dtype, const void *A, const void *A_
                              int bias_dtype, int64_t M, int64_t N, int64_t K, void *workspace,
                              int64_t workspace_bytes, ac4k_stream_t stream);
 
+/* ac4k_linear_nvfp4 with scratch: every shape that ac4k_linear_nvfp4 takes, split along K where that fills the GPU,
+ * on the same kernels as ac4k_linear_nvfp4_skinny but for any K % 64 == 0.  `workspace` =
+ * ac4k_linear_nvfp4_workspace_bytes(M,N,K) bytes, 256-byte aligned, contents irrelevant (NULL when that is 0). */
+int64_t ac4k_linear_nvfp4_workspace_bytes(int64_t M, int64_t N, int64_t K);
+int ac4k_linear_nvfp4_workspace(void *D, int d_dtype, const void *A, const void *A_sf, const float *A_gs,
+                                const void *B, const void *B_sf, const float *B_gs, const void *bias,
+                                int bias_dtype, int64_t M, int64_t N, int64_t K, void *workspace,
+                                int64_t workspace_bytes, ac4k_stream_t stream);
+
 /* ac4k_linear_nvfp4_skinny without the workspace argument, for callers that cannot allocate
  * device memory (code under HIP graph capture, tight serving loops, harnesses that forbid
  * hipMalloc).  It has no counterpart in the reference.  The partial sums go to an array of
@@ -189,8 +198,8 @@ int ac4k_set_linear_tuning(int mi, int nj, int splits, int skinny_ks, int decode
  * image (16-byte aligned).
  * ac4k_linear_nvfp4_prepacked: contract of ac4k_linear_nvfp4 with W_image in place of B and B_sf;
  * `workspace` as for ac4k_linear_nvfp4_skinny, of ac4k_linear_nvfp4_prepacked_workspace_bytes(M,N,K)
- * bytes (may be NULL when that is 0).  M <= 32 with K % 256 == 0 streams the image through the LDS
- * ring; everything else runs the tile kernel, split along K when there are too few tiles. */
+ * bytes (may be NULL when that is 0).  M <= 32 with K >= 256 streams the image through the LDS
+ * ring, 32 < M <= 128 runs the K-split-waves kernel; everything else runs the tile kernel, split along K when there are too few tiles. */
 int64_t ac4k_prepack_weight_nvfp4_bytes(int64_t N, int64_t K);
 int ac4k_prepack_weight_nvfp4(void *image, const void *B, const void *B_sf, int64_t N, int64_t K,
                               ac4k_stream_t stream);

@@ -441,3 +441,37 @@ def test_k_not_a_multiple_of_64(m, n, k):
     ref_t = (dequant(a, m) @ dequant(b, n).t()).float()
     torch.testing.assert_close(ref_c, ref_t, atol=1e-4, rtol=1e-5)
     torch.testing.assert_close(d.cpu(), ref_c, atol=1e-4, rtol=1e-5)
+
+
+def check_tight(m, n, k, seed, image=False):
+    """fp32 output against the C oracle's double sum: a chunk of k lost or counted twice shows, which 1e-2 could hide."""
+    aq, bq = gpu_quant(make_input((m, k), seed=seed)), gpu_quant(make_input((n, k), seed=seed + 1, std=0.02))
+    out = torch.full((m, n), float("nan"), dtype=torch.float32, device="cuda")
+    if image:
+        ops().linear_prepacked(*aq, ops().prepack_weight(bq[0], bq[1]), bq[2], out=out)
+    else:
+        ops().linear(*aq, *bq, out=out)
+    # fp32 accumulation of k exact products: k * 2^-24 of the sum of their magnitudes at worst
+    torch.testing.assert_close(out.cpu(), C.linear_nvfp4(*cpu(aq), *cpu(bq)), atol=1e-5, rtol=1e-4, msg=lambda t: f"{(m, n, k)}: {t}")
+
+
+# K of every remainder the last 256-k (128-k) stage can have, from the shortest K a kernel takes, one K range and several
+@pytest.mark.parametrize("k", [320, 384, 448, 1152, 1216, 1344])
+@pytest.mark.parametrize("ks", [0, 256])
+def test_k_tails_of_four_chunk_stages(k, ks, linear_tuning):
+    for kind in (0, 2, 3):
+        linear_tuning(skinny_ks=ks, decode_kernel=kind)
+        for m in (1, 16, 27):
+            check_tight(m, 200, k, seed=k + m)
+    for m, n in ((40, 70), (128, 200), (50, 24580)):
+        check_tight(m, n, k, seed=k + m)
+    if k % 128 == 0:
+        for m in (5, 32, 100):
+            check_tight(m, 200, k, seed=k + m, image=True)
+
+
+@pytest.mark.parametrize("mi,nj,splits", TILE_PLANS)
+def test_k_tail_of_the_tile_kernel(mi, nj, splits, linear_tuning):
+    linear_tuning(mi, nj, splits)
+    for k in (192, 320, 1216):
+        check_tight(64 * mi + 5, 64 * nj + 130, k, seed=k + mi)
