@@ -912,18 +912,18 @@ static int launch_tile256p(const LinearArgs &a, hipStream_t st) {
 // chunks the last stage takes the last four; chunk c of it counts for nothing when the stage before holds it too:
 // `weight_factor` multiplies the weight scales, by 1 or by so little that the fp16 scale rounds to zero (the scale
 // conversion takes a power of two at no cost).  `offset` is where a stage starts, from the row's first chunk (TAIL) or
-// from the first one of the workgroup's range, given the bytes per chunk.
+// from the first one of the workgroup's range.
 template <bool TAIL>
 struct StageWalk {
   int s0, nch;  // first stage of the range, chunks in the row
+  // what a source advances by, given its bytes per chunk: a chunk (TAIL) or a whole stage
+  template <typename T>
+  static __device__ __forceinline__ constexpr T step(T per_chunk) { return TAIL ? per_chunk : 4 * per_chunk; }
   __device__ __forceinline__ int chunk(int st) const { return 4 * (s0 + st) < nch - 4 ? 4 * (s0 + st) : nch - 4; }
   template <typename T>
-  __device__ __forceinline__ int64_t offset(int st, T per_chunk) const {
-    if constexpr (TAIL) return chunk(st) * (int64_t)per_chunk;
-    else return st * (int64_t)(4 * per_chunk);
-  }
+  __device__ __forceinline__ int64_t offset(int st, T step) const { return (TAIL ? chunk(st) : st) * (int64_t)step; }
   template <typename T>
-  __device__ __forceinline__ int64_t start(T per_chunk) const { return TAIL ? 0 : s0 * (int64_t)(4 * per_chunk); }
+  __device__ __forceinline__ int64_t start(T step) const { return TAIL ? 0 : s0 * (int64_t)step; }
   __device__ __forceinline__ float weight_factor(int st, int c) const {
     if constexpr (TAIL) return 4 * (s0 + st) - chunk(st) > c ? 0x1p-60f : 1.0f;
     else return 1.0f;
@@ -987,7 +987,7 @@ __global__ __launch_bounds__(256, 1) void linear_nvfp4_ksplit_kernel(LinearArgs 
   const int64_t img_band_bytes = (a.K / W_BLOCK_K) * (int64_t)W_BLOCK_BYTES;
   uint32_t offR[L::NROW], ldsR[L::NROW];
   const uint8_t *srcR[L::NROW];
-  int strR[L::NROW];  // bytes per chunk along k
+  int strR[L::NROW];  // bytes per step of the walk along k
 #pragma unroll
   for (int q = 0; q < L::NROW; ++q) {
     const int t = swave * L::NROW + q;
@@ -998,13 +998,13 @@ __global__ __launch_bounds__(256, 1) void linear_nvfp4_ksplit_kernel(LinearArgs 
       const int64_t wrow = n0 + loc;  // rows past N exist in the image (zeros)
       const int64_t band = wrow / W_BLOCK_ROWS, within = wrow % W_BLOCK_ROWS;
       offR[q] = (uint32_t)(band * img_band_bytes + (pp >> 2) * W_BLOCK_BYTES + within * 64 + (((pp & 3) ^ ((within >> 1) & 3)) * 16));
-      strR[q] = W_BLOCK_BYTES / 2;
+      strR[q] = walk.step(W_BLOCK_BYTES / 2);
       srcR[q] = uniform_ptr(a.B + walk.start(strR[q]));
     } else {
       const int64_t rows = isW ? a.N : a.M, first = isW ? n0 : m0;
       const int64_t row = first + loc < rows ? loc : rows - 1 - first;  // rows past the matrix read its last row
       offR[q] = (uint32_t)(row * kb + pp * 16);
-      strR[q] = KW_ROW / 4;
+      strR[q] = walk.step(KW_ROW / 4);
       srcR[q] = uniform_ptr((isW ? a.B + n0 * kb : a.A + m0 * kb) + walk.start(strR[q]));
     }
     strR[q] = __builtin_amdgcn_readfirstlane(strR[q]);
@@ -1028,12 +1028,12 @@ __global__ __launch_bounds__(256, 1) void linear_nvfp4_ksplit_kernel(LinearArgs 
     if (isW && a.prepacked) {
       const int64_t band = row / W_BLOCK_ROWS, within = row % W_BLOCK_ROWS;
       offS = (uint32_t)(band * img_band_bytes + (chunk >> 1) * W_BLOCK_BYTES + W_BLOCK_DATA + (chunk & 1) * (W_BLOCK_ROWS * 4) + within * 4);
-      strideS = W_BLOCK_BYTES / 2;
+      strideS = walk.step(W_BLOCK_BYTES / 2);
       srcS = uniform_ptr(a.B + walk.start(strideS));
     } else {
       row = row + 4 <= rows_p ? row : rows_p - 4;         // groups past the padded rows read the last group
       offS = (uint32_t)((chunk * rows_p + row) * 4);
-      strideS = rows_p * 4;                               // bytes per chunk plane
+      strideS = walk.step(rows_p * 4);                    // chunk planes
       srcS = uniform_ptr(reinterpret_cast<const uint8_t *>(isW ? a.B_sf : a.A_sf) + walk.start(strideS));
     }
     ldsS = (uint32_t)__builtin_amdgcn_readfirstlane((isW ? L::OFF_SFW : L::OFF_SFA) + tt * 1024);
@@ -1745,7 +1745,7 @@ __global__ __launch_bounds__(ST_THREADS, 1) void linear_nvfp4_stream_kernel(Skin
     offW[0] = (uint32_t)(swave * 2048 + lane * 16);
     offW[1] = offW[0] + 1024;
     offW[2] = (uint32_t)((16 + swave) * 1024 + lane * 16);
-    strideW = W_BLOCK_BYTES / 2;  // bytes per chunk (K % 128 == 0: a stage starts at a whole block)
+    strideW = walk.step(W_BLOCK_BYTES / 2);  // (K % 128 == 0: a stage starts at a whole block)
     srcW = uniform_ptr(a.B + (int64_t)blockIdx.x * (a.K / W_BLOCK_K) * W_BLOCK_BYTES + walk.start(strideW));
     ldsW = (uint32_t)__builtin_amdgcn_readfirstlane(swave * 2048);
   } else {
@@ -1758,7 +1758,7 @@ __global__ __launch_bounds__(ST_THREADS, 1) void linear_nvfp4_stream_kernel(Skin
       offW[q] = (uint32_t)((row - n0) * kb + ((lane & 7) ^ (loc & 7)) * 16);
     }
     offW[2] = 0;
-    strideW = ST_ROW / 4;
+    strideW = walk.step(ST_ROW / 4);
     srcW = uniform_ptr(a.B + n0 * kb + walk.start(strideW));
     ldsW = (uint32_t)__builtin_amdgcn_readfirstlane(ST_OFF_B + swave * 2048);
   }
@@ -1770,7 +1770,7 @@ __global__ __launch_bounds__(ST_THREADS, 1) void linear_nvfp4_stream_kernel(Skin
     int64_t srow = n0 + (swave & 1) * 64 + lane;
     srow = srow < a.Np ? srow : a.Np - 1;
     offS = (uint32_t)(srow * 4);
-    strideS = a.Np * 4;  // bytes per chunk plane
+    strideS = walk.step(a.Np * 4);  // chunk planes
     srcS = uniform_ptr(reinterpret_cast<const uint8_t *>(a.B_sf) + (int64_t)(swave >> 1) * a.Np * 4 + walk.start(strideS));
     ldsS = (uint32_t)__builtin_amdgcn_readfirstlane(ST_OFF_SFB + (swave >> 1) * (ST_BN * 4) + (swave & 1) * 256);
   }
@@ -1788,11 +1788,11 @@ __global__ __launch_bounds__(ST_THREADS, 1) void linear_nvfp4_stream_kernel(Skin
     const int loc = (swave - A_FIRST) * 8 + (lane >> 3);
     const int64_t row = loc < a.M ? loc : a.M - 1;  // rows past M read row M - 1; their outputs are never stored
     off4 = (uint32_t)(row * kb + ((lane & 7) ^ (loc & 7)) * 16);
-    stride4 = ST_ROW / 4;
+    stride4 = walk.step(ST_ROW / 4);
     src4 = uniform_ptr(a.Aq + walk.start(stride4));
     lds4 = (uint32_t)__builtin_amdgcn_readfirstlane(OFF_A + (swave - A_FIRST) * 1024);
   } else if (!PRE || swave >= 2) {
-    stride4 = a.Mp * 4;
+    stride4 = walk.step(a.Mp * 4);
     src4 = uniform_ptr(a.A_sf + walk.start(stride4));
     if constexpr (MR == 32) {
       const int pair = swave & 1;  // chunks 2 pair, 2 pair + 1
@@ -1939,7 +1939,7 @@ __global__ __launch_bounds__(ST_THREADS, 1) void linear_nvfp4_stream64_kernel(Sk
     row = row < a.N ? row : a.N - 1;  // rows past N read the last row; their outputs are never stored
     offW = (uint32_t)((row - n0) * kb + ((lane & 7) ^ (loc & 7)) * 16);
   }
-  const uint8_t *srcW = uniform_ptr(a.B + n0 * kb + walk.start(ST_ROW / 4));
+  const uint8_t *srcW = uniform_ptr(a.B + n0 * kb + walk.start(walk.step(ST_ROW / 4)));
   const uint32_t ldsW = (uint32_t)__builtin_amdgcn_readfirstlane(S6_OFF_B + swave * 1024);
   // (2) waves 0..3: weight scale dwords of chunk swave, rows n0 + lane; waves 4..7: packed activation
   //     rows (swave - 4) * 8 + {0..7}
@@ -1950,14 +1950,14 @@ __global__ __launch_bounds__(ST_THREADS, 1) void linear_nvfp4_stream64_kernel(Sk
     int64_t srow = n0 + lane;
     srow = srow < a.Np ? srow : a.Np - 1;
     off2 = (uint32_t)(srow * 4);
-    stride2 = a.Np * 4;  // bytes per chunk plane
+    stride2 = walk.step(a.Np * 4);  // chunk planes
     src2 = uniform_ptr(reinterpret_cast<const uint8_t *>(a.B_sf) + (int64_t)swave * a.Np * 4 + walk.start(stride2));
     lds2 = (uint32_t)__builtin_amdgcn_readfirstlane(S6_OFF_SFB + swave * (S6_BN * 4));
   } else {
     const int loc = (swave - 4) * 8 + (lane >> 3);
     const int64_t row = loc < a.M ? loc : a.M - 1;  // rows past M read row M - 1; their outputs are never stored
     off2 = (uint32_t)(row * kb + ((lane & 7) ^ (loc & 7)) * 16);
-    stride2 = ST_ROW / 4;
+    stride2 = walk.step(ST_ROW / 4);
     src2 = uniform_ptr(a.Aq + walk.start(stride2));
     lds2 = (uint32_t)__builtin_amdgcn_readfirstlane(S6_OFF_A + (swave - 4) * 1024);
   }
@@ -1966,13 +1966,13 @@ __global__ __launch_bounds__(ST_THREADS, 1) void linear_nvfp4_stream64_kernel(Sk
   const int pair = swave & 1;
   const int64_t arow = r32 < a.Mp ? r32 : a.Mp - 1;
   const uint32_t off3 = (uint32_t)(((2 * pair + half) * a.Mp + arow) * 4);
-  const int64_t stride3 = a.Mp * 4;
+  const int64_t stride3 = walk.step(a.Mp * 4);
   const uint8_t *src3 = uniform_ptr(a.A_sf + walk.start(stride3));
   const uint32_t lds3 = (uint32_t)__builtin_amdgcn_readfirstlane(S6_OFF_SFA + pair * 256);
   auto issue_stage = [&](int slot, int step) {  // step: position in this workgroup's order of stages
     const int st = stage_of(step);
     const uint32_t base = lds_base + slot * S6_STAGE_BYTES;
-    dma16(srcW + walk.offset(st, ST_ROW / 4), offW, base, ldsW);
+    dma16(srcW + walk.offset(st, walk.step(ST_ROW / 4)), offW, base, ldsW);
     if (swave < 4)
       dma4(src2 + walk.offset(st, stride2), off2, base, lds2);
     else
