@@ -96,6 +96,7 @@ struct QuantGeom {
   // cross-major kernels: the leading index, not the position along the reduce dim, is the fast grid
   // index (its stride is the smaller one, so workgroups that run together read neighbouring memory)
   int lead_fast = 0;
+  int64_t kspan = 0;  // reduce positions per workgroup of the maximum kernel
 };
 
 // grid indices of the cross-major kernels: (position along the reduce dim, leading index)
@@ -818,32 +819,49 @@ __global__ void fill_u32_kernel(uint32_t *__restrict__ p, int64_t n, uint32_t v)
   if (i < n) p[i] = v;
 }
 
-constexpr int CM_KSPAN = 2048;  // reduce positions per workgroup of the maximum kernel
+// Bound by HBM, and by the atomics of a row where few rows are long: one lane per row for these, so that a wave's atomics
+// cover whole lines (with eight rows a lane, strided, the same split of (1, 30000, 1, 128) measured 30 us as a call, 15 so).
+// Eight waves a workgroup: four need twice as many atomics for the same loads in flight (17.3 us), sixteen measured the same.
+constexpr int CM_AMAX_WAVES = 8, CM_AMAX_LOADS = 4;
+constexpr int CM_AMAX_STEP = CM_AMAX_WAVES * 4 * CM_AMAX_LOADS;  // positions a workgroup reads at a time
 
-__global__ __launch_bounds__(256) void rowwise_crossmajor_amax_kernel(uint32_t *__restrict__ amax_bits,
-                                                                       const uint16_t *__restrict__ in, QuantGeom g) {
+// STREAM: loads that leave nothing in the caches, for an input that the memory-side cache does not hold from the maximum
+// kernel to the quantize kernel anyway
+template <bool STREAM>
+__device__ __forceinline__ uint4 ld_crossmajor_u4(const uint16_t *p) {
+  if constexpr (STREAM) {
+    const u32x4 v = __builtin_nontemporal_load(reinterpret_cast<const u32x4_elem *>(p));
+    return make_uint4(v.x, v.y, v.z, v.w);
+  } else {
+    return ld_elem_u4(p);
+  }
+}
+
+template <bool STREAM>
+__global__ __launch_bounds__(64 * CM_AMAX_WAVES) void rowwise_crossmajor_amax_kernel(uint32_t *__restrict__ amax_bits,
+                                                                                     const uint16_t *__restrict__ in, QuantGeom g) {
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int kq = lane & 3, rg = lane >> 2;
   const CrossMajorIdx gi = crossmajor_idx(g);
-  const int64_t group0 = (int64_t)blockIdx.y * 128 + rg * 8;
+  const int64_t block0 = (int64_t)blockIdx.y * 128, group0 = block0 + rg * 8;
   const int64_t lead = gi.lead;
-  const int64_t row0 = crossmajor_rows(group0, g.R);
-  const uint16_t *src = in + (lead / g.d1) * g.s0 + (lead % g.d1) * g.s1 + row0;
+  const uint16_t *src = in + (lead / g.d1) * g.s0 + (lead % g.d1) * g.s1 + crossmajor_rows(group0, g.R);
   uint4 m8 = make_uint4(0, 0, 0, 0);
   if (group0 < g.R) {
-    const int64_t kbeg = gi.kblock * CM_KSPAN, kend = kbeg + CM_KSPAN < g.K ? kbeg + CM_KSPAN : g.K;
-    for (int64_t k = kbeg + wave * 4 + kq; k < kend; k += 64) {  // four loads in flight per lane
-      uint4 a[4];
+    const int64_t kbeg = gi.kblock * g.kspan, kend = kbeg + g.kspan < g.K ? kbeg + g.kspan : g.K;
+    for (int64_t k = kbeg + wave * 4 + kq; k < kend; k += CM_AMAX_STEP) {
+      uint4 a[CM_AMAX_LOADS];
 #pragma unroll
-      for (int u = 0; u < 4; ++u) {
+      for (int u = 0; u < CM_AMAX_LOADS; ++u) {
+        const int64_t ku = k + u * (CM_AMAX_WAVES * 4);
         a[u] = make_uint4(0, 0, 0, 0);
-        if (k + u * 16 < kend) a[u] = ld_elem_u4(src + (k + u * 16) * g.sK);
+        if (ku < kend) a[u] = ld_crossmajor_u4<STREAM>(src + ku * g.sK);
       }
 #pragma unroll
-      for (int u = 0; u < 4; ++u) m8 = absmax_bf16x8_pairwise(m8, a[u]);
+      for (int u = 0; u < CM_AMAX_LOADS; ++u) m8 = absmax_bf16x8_pairwise(m8, a[u]);
     }
   }
-  // quad (same rows, different k) -> one value per row; then across the four waves through LDS
+  // quad (same rows, different k) -> one value per row; then across the waves through LDS
   auto quad_max = [](uint32_t w) {
     u16x2 x = __builtin_bit_cast(u16x2, w);
     x = __builtin_elementwise_max(x, __builtin_bit_cast(u16x2, dpp_u32<DPP_QUAD_XOR1>(w)));
@@ -852,22 +870,34 @@ __global__ __launch_bounds__(256) void rowwise_crossmajor_amax_kernel(uint32_t *
     return __builtin_bit_cast(uint32_t, x);
   };
   m8 = make_uint4(quad_max(m8.x), quad_max(m8.y), quad_max(m8.z), quad_max(m8.w));
-  __shared__ uint4 red[4][16];
-  if (kq == 0) red[wave][rg] = m8;
+  __shared__ __attribute__((aligned(16))) uint16_t red[CM_AMAX_WAVES][128];
+  if (kq == 0) *reinterpret_cast<uint4 *>(&red[wave][rg * 8]) = m8;
   __syncthreads();
-  if (wave == 0 && kq == 0 && group0 < g.R) {
-    uint4 t = red[0][rg];
+  // one row per lane, so that an atomic instruction covers whole lines of scales
+  const int i = threadIdx.x;
+  const int64_t row0 = block0 + (i & ~7);
+  if (i < 128 && row0 < g.R) {
+    uint32_t b = 0;
 #pragma unroll
-    for (int w2 = 1; w2 < 4; ++w2) t = absmax_bf16x8_pairwise(t, red[w2][rg]);
-#pragma unroll
-    for (int j = 0; j < 8; ++j) {
-      const uint32_t b = u16_comp(t, j);
-      if (b) atomicMax(amax_bits + lead * g.Rp + row0 + j, b);
-    }
+    for (int w = 0; w < CM_AMAX_WAVES; ++w) b = umax32(b, red[w][i]);
+    if (b) atomicMax(amax_bits + lead * g.Rp + crossmajor_rows(row0, g.R) + (i & 7), b);
   }
 }
 
-template <RowFmt FMT, bool SWIZZLE>
+// Positions per workgroup of the maximum kernel, `columns` workgroups side by side.  Two workgroups per CU where the tensor
+// gives them, at most 2048 positions each; 1024 or 256 workgroups measured the same within 2 - 6 %.  At most 128 workgroups
+// of one row as long as that keeps to 2048 positions: their atomics on the same scales follow one another.  A fixed span of 2048
+// left 15 workgroups to (1, 30000, 1, 128).  fp8 with swizzle, cross 3, reduce 1, before -> after (us): (1, 30000, 1, 128)
+// 31.4 -> 14.4, (1, 75600, 1, 128) 45.6 -> 21.0 (25.5 with at most 64 workgroups of a row), (1, 16384, 8, 96) 47.5 -> 17.8,
+// (1, 4097, 3, 100) 25.4 -> 12.4, (1, 4096, 40, 128) 52.5 -> 23.0, (1, 24000, 40, 128) 134.5 -> 114.3, (1, 64, 8, 128) 12.4.
+constexpr int CM_AMAX_WGS = 512, CM_AMAX_SPLITS = 128, CM_AMAX_SPAN = 2048;
+static int64_t crossmajor_amax_span(int64_t K, int64_t columns) {
+  const int64_t wanted = ceil_div(CM_AMAX_WGS, columns), splits = wanted < CM_AMAX_SPLITS ? wanted : CM_AMAX_SPLITS;
+  const int64_t span = align_up(ceil_div(K, splits), CM_AMAX_STEP);
+  return span < CM_AMAX_SPAN ? span : CM_AMAX_SPAN;
+}
+
+template <RowFmt FMT, bool SWIZZLE, bool STREAM>
 __global__ __launch_bounds__(256) void quantize_rowwise_crossmajor_kernel(
     uint8_t *__restrict__ out, const uint32_t *__restrict__ amax_bits, const uint16_t *__restrict__ in,
     const void *__restrict__ smax_p, QuantGeom g) {
@@ -886,7 +916,7 @@ __global__ __launch_bounds__(256) void quantize_rowwise_crossmajor_kernel(
   for (int i = 0; i < 16; ++i) {
     const int64_t k = k0 + (SWIZZLE ? fp8_swizzle_src(i) : i);
     v[i] = make_uint4(0, 0, 0, 0);
-    if (k < g.K) v[i] = ld_elem_u4(src + k * g.sK);
+    if (k < g.K) v[i] = ld_crossmajor_u4<STREAM>(src + k * g.sK);
   }
 #pragma unroll
   for (int j = 0; j < 8; ++j) {
@@ -1295,6 +1325,39 @@ static void launch_rowwise_contiguous(uint8_t *out, float *sf, const uint16_t *i
                        dim3((unsigned)ceil_div(g.Rp, 4), (unsigned)lead), dim3(256), 0, st, out, sf, in, smax, g);
 }
 
+// Inputs larger than the memory-side cache (256 MiB) are read past it by both kernels: the lines they would leave there are
+// gone before they are read again, and push out lines the output is collected in.  fp8, (1, 75600, 40, 128): 409 -> 390 us,
+// (1, 32768, 40, 128) (336 MB) 177 -> 162 with the span below; smaller inputs lose what the cache holds for the second
+// kernel: (1, 24000, 40, 128) (246 MB) the same, (1, 16384, 40, 128) 84 -> 104, (1, 4096, 40, 128) 53 -> 70.
+constexpr int64_t CM_STREAM_BYTES = 256 << 20;
+
+template <RowFmt FMT, bool STREAM>
+static void launch_rowwise_crossmajor(uint8_t *out, float *sf, const uint16_t *in, const void *smax, QuantGeom g, int64_t lead,
+                                      int swizzle, hipStream_t st) {
+  // row maxima as bf16 bit patterns in the scale array, quantize from them, then scale them in place
+  uint32_t *bits = reinterpret_cast<uint32_t *>(sf) + g.lead0 * g.Rp;  // the kernels index by absolute lead
+  const int64_t nsf = lead * g.Rp;
+  hipLaunchKernelGGL(fill_u32_kernel, dim3((unsigned)ceil_div(nsf, 256)), dim3(256), 0, st, bits, nsf, 0u);
+  // Both kernels walk the grid along the dim of smaller input stride first (measured on
+  // (1,75600,40,128), cross 3, reduce 1: 412 us against 440 us; the nvfp4 kernel, whose packed
+  // rows are a quarter as long, loses 6% by the same change and keeps the reduce dim first).
+  const int64_t kblocks = ceil_div(g.Kp / 16, 16);  // of the quantize kernel; the maxima kernel has fewer
+  g.lead_fast = crossmajor_lead_fast(g.d1, g.s1, g.sK, kblocks);
+  const int64_t rowblocks = ceil_div(g.Rp, 128);
+  g.kspan = crossmajor_amax_span(g.K, rowblocks * lead);
+  hipLaunchKernelGGL((rowwise_crossmajor_amax_kernel<STREAM>), crossmajor_grid(g, ceil_div(g.K, g.kspan), rowblocks, lead),
+                     dim3(64 * CM_AMAX_WAVES), 0, st, reinterpret_cast<uint32_t *>(sf), in, g);
+  const dim3 grid = crossmajor_grid(g, kblocks, rowblocks, lead);
+  if (swizzle)
+    hipLaunchKernelGGL((quantize_rowwise_crossmajor_kernel<FMT, true, STREAM>), grid, dim3(256), 0, st, out,
+                       reinterpret_cast<const uint32_t *>(sf), in, smax, g);
+  else
+    hipLaunchKernelGGL((quantize_rowwise_crossmajor_kernel<FMT, false, STREAM>), grid, dim3(256), 0, st, out,
+                       reinterpret_cast<const uint32_t *>(sf), in, smax, g);
+  hipLaunchKernelGGL(rowwise_crossmajor_finalize_kernel<FMT>, dim3((unsigned)ceil_div(nsf, 256)), dim3(256), 0, st,
+                     sf + g.lead0 * g.Rp, smax, nsf);
+}
+
 template <RowFmt FMT>
 static int quantize_rowwise(void *out, float *sf, const void *in, const void *smax, int64_t d0, int64_t d1,
                             int64_t R, int64_t K, int64_t s0, int64_t s1, int64_t sR, int64_t sK, int swizzle,
@@ -1313,27 +1376,9 @@ static int quantize_rowwise(void *out, float *sf, const void *in, const void *sm
       else if (swizzle) launch_rowwise_contiguous<FMT, CAN_SWIZZLE, false>(o, sf, x, smax, g, lead, st);
       else if (aligned) launch_rowwise_contiguous<FMT, false, true>(o, sf, x, smax, g, lead, st);
       else launch_rowwise_contiguous<FMT, false, false>(o, sf, x, smax, g, lead, st);
-    } else if (crossmajor_ok(R, sR) && ceil_div(g.Rp, 128) <= 65535 && ceil_div(K, CM_KSPAN) <= 65535) {
-      // row maxima as bf16 bit patterns in the scale array, quantize from them, then scale them in place
-      uint32_t *bits = reinterpret_cast<uint32_t *>(sf) + g.lead0 * g.Rp;  // the kernels index by absolute lead
-      const int64_t nsf = lead * g.Rp;
-      hipLaunchKernelGGL(fill_u32_kernel, dim3((unsigned)ceil_div(nsf, 256)), dim3(256), 0, st, bits, nsf, 0u);
-      // Both kernels walk the grid along the dim of smaller input stride first (measured on
-      // (1,75600,40,128), cross 3, reduce 1: 412 us against 440 us; the nvfp4 kernel, whose packed
-      // rows are a quarter as long, loses 6% by the same change and keeps the reduce dim first).
-      const int64_t kblocks = ceil_div(g.Kp / 16, 16);  // of the quantize kernel; the maxima kernel has fewer
-      g.lead_fast = crossmajor_lead_fast(d1, s1, sK, kblocks);
-      hipLaunchKernelGGL(rowwise_crossmajor_amax_kernel, crossmajor_grid(g, ceil_div(K, CM_KSPAN), ceil_div(g.Rp, 128), lead),
-                         dim3(256), 0, st, reinterpret_cast<uint32_t *>(sf), x, g);
-      const dim3 grid = crossmajor_grid(g, kblocks, ceil_div(g.Rp, 128), lead);
-      if (swizzle)
-        hipLaunchKernelGGL((quantize_rowwise_crossmajor_kernel<FMT, true>), grid, dim3(256), 0, st, o,
-                           reinterpret_cast<const uint32_t *>(sf), x, smax, g);
-      else
-        hipLaunchKernelGGL((quantize_rowwise_crossmajor_kernel<FMT, false>), grid, dim3(256), 0, st, o,
-                           reinterpret_cast<const uint32_t *>(sf), x, smax, g);
-      hipLaunchKernelGGL(rowwise_crossmajor_finalize_kernel<FMT>, dim3((unsigned)ceil_div(nsf, 256)), dim3(256), 0, st,
-                         sf + g.lead0 * g.Rp, smax, nsf);
+    } else if (crossmajor_ok(R, sR) && ceil_div(g.Rp, 128) <= 65535 && ceil_div(K, CM_AMAX_SPAN) <= 65535) {
+      if (lead * R * K * 2 > CM_STREAM_BYTES) launch_rowwise_crossmajor<FMT, true>(o, sf, x, smax, g, lead, swizzle, st);
+      else launch_rowwise_crossmajor<FMT, false>(o, sf, x, smax, g, lead, swizzle, st);
     } else {
       dim3 grid((unsigned)ceil_div(g.Rp, 256), (unsigned)lead);
       if (swizzle)

@@ -212,6 +212,33 @@ def test_ragged_contiguous_dims(shape, cross, red, off):
         assert torch.equal(gs.cpu(), eg) and torch.equal(o.cpu(), eo) and torch.equal(s.cpu().view(torch.uint8), es), swz
 
 
+# The reduce dim split over workgroups: lengths around the step of a workgroup (128 positions), around 128 of them, and so
+# long that a workgroup's span reaches its bound; row counts around a lane group and a row block.  The largest value of row r
+# lies at another position each, the ends of steps and of the dim among them.
+@pytest.mark.parametrize("K,R", [(1, 8), (127, 9), (128, 128), (129, 130), (16383, 8), (16385, 9), (300001, 17), (4099, 520)])
+@pytest.mark.parametrize("precision", ["fp8e4m3", "int8"])
+def test_crossmajor_maximum_of_split_rows(K, R, precision):
+    x = make_input((K, R), seed=K + R).clamp(-4, 4)
+    at = [0, K - 1, 127, 128, 255, 256, 2047, 2048, K // 2, K - 128]
+    for r in range(R):
+        x[min(max(at[r % len(at)], 0), K - 1), r] = 5 + r % 7
+    oracle, arg = (T.quantize_fp8, 448.0) if precision == "fp8e4m3" else (T.quantize_int8, 127)
+    eo, es = oracle(x, 1, 0, arg)
+    o, s = ops().quantize(x.cuda(), 1, 0, precision=precision)
+    assert torch.equal(s.cpu(), es) and torch.equal(o.cpu().view(torch.uint8), eo.view(torch.uint8))
+
+
+def test_crossmajor_larger_than_the_memory_side_cache():
+    """More than 256 MiB are read past the caches (ragged heads of 100 channels, so element-aligned): whole heads compared."""
+    g = torch.Generator(device="cuda").manual_seed(3)
+    x = torch.empty((1, 30011, 45, 100), dtype=torch.float32, device="cuda").normal_(generator=g).to(torch.bfloat16)
+    for precision, oracle, args in (("fp8e4m3", T.quantize_fp8, (448.0, True)), ("int8", T.quantize_int8, (127,))):
+        o, s = ops().quantize(x, 3, 1, precision=precision, swizzle=precision == "fp8e4m3")
+        for h in (0, 22, 44):
+            eo, es = oracle(x[:, :, h:h + 1].cpu(), 3, 1, *args)
+            assert torch.equal(o[:, h:h + 1].cpu().view(torch.uint8), eo.view(torch.uint8)) and torch.equal(s[:, h:h + 1].cpu(), es)
+
+
 def test_nvfp4_graph_replay():
     """A captured quantize call replays correctly: under capture the library takes the path whose whole
     state is in the caller's buffers, so nothing in it depends on host-side state that changes from
