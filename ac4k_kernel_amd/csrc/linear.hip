@@ -2559,7 +2559,7 @@ static int64_t weight_image_bytes(int64_t N, int64_t K) {
   return ceil_div(N, W_BLOCK_ROWS) * (K / W_BLOCK_K) * W_BLOCK_BYTES;
 }
 
-// How a linear on a weight image runs: the LDS-ring kernel for decode-sized M (K % 256 == 0), the K-split-waves
+// How a linear on a weight image runs: the LDS-ring kernel for decode-sized M (K >= 256), the K-split-waves
 // kernel for 32 < M <= 128, the tile kernel otherwise, split along K when the workspace entry point of the plain
 // layout would split too.
 struct PrepackedPlan {
