@@ -421,12 +421,15 @@ __device__ __forceinline__ void mha_nvfp4_block(const MhaArgs &a, const MhaTile 
     const float ml = __builtin_fmaxf(ml_run, mx * cs);
     alpha = __builtin_amdgcn_exp2f(ml_run - ml);
     ml_run = ml;
-    // block scales: e4m3(2688 * (largest p / 6)), at most 448, and the multiplier 2688 / scale, 0 for code 0
+    // block scales: e4m3(2688 * (largest p / 6)), saturated at 448, and the multiplier 2688 / scale, 0 for code 0.  ml is
+    // rounded and the argument below is not, so with maxima of 2^20 and more it exceeds zero by up to half an ulp of ml and
+    // the product reaches the 464 that the conversion turns into NaN.  A largest p held at 1 gives the code of 448, which is
+    // where the product saturates (the compiler makes it the output modifier of the exp2).
     float o[NF];
     uint32_t code[NF];
 #pragma unroll
     for (int f = 0; f < NF; ++f) {
-      const float bm = __builtin_amdgcn_exp2f(__builtin_fmaf(bmax[f], cs, -ml));
+      const float bm = __builtin_amdgcn_fmed3f(__builtin_amdgcn_exp2f(__builtin_fmaf(bmax[f], cs, -ml)), 0.0f, 1.0f);
       code[f] = (uint32_t)__builtin_amdgcn_cvt_pk_fp8_f32(MHA_P_ALPHA * (bm * 0.16666666666666666f), 0.0f, 0, false) & 0x7f;
       o[f] = MHA_P_ALPHA * lut[code[f]];
     }

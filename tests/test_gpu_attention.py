@@ -92,6 +92,34 @@ def test_split_plans(H, Nq, Nkv, D):
     torch.testing.assert_close(o.cpu().float(), ref.float(), atol=ATOL, rtol=RTOL)
 
 
+# Row maxima of 2^20 to 2^21 (in log2 units), where the exponent of the largest p of a row may exceed zero by half an ulp of
+# the maximum, 1/16: p up to 2^(1/16), a block scale beyond 448.  Workgroups of 256, 128 and 64 query rows.
+LARGE = [(256, 256), (128, 256), (3, 300)]
+
+
+@pytest.mark.parametrize("H,N", LARGE)
+def test_large_scores(H, N):
+    """Every query is its own nearest key by far, so a row of O is that row of V as the quantizers leave it, times
+    Phat / l: l = p is within 2^(+-1/16) of 1 (4.5 %), Phat the e4m3 value next to it, half a step of 32 off 416 (3.9 %)."""
+    q, v = make_input((1, H, N, 128), seed=51, std=280.0), make_input((1, H, N, 128), seed=52)
+    o = ops().attention(q.cuda(), q.cuda(), v.cuda(), layout="BHND", precision="nvfp4").cpu().float()
+    assert torch.isfinite(o).all()
+    torch.testing.assert_close(o, A.attention_nvfp4(q, q, v, "BHND").float(), atol=ATOL, rtol=0.045 + 0.039 + 2 ** -8)
+
+
+@pytest.mark.parametrize("H,N", LARGE[:2])  # whole kv tiles: a position without a key has score 0, which would be the maximum
+def test_large_negative_scores(H, N):
+    """All keys pushed down by one channel: maxima of -1.43 * 2^20, where an ulp is 1/8.  Eight accumulation steps of S and the
+    exponent round, half an ulp each at most, so a p is off by up to 2^(9/16) = 1.48, each p of a row by another factor; the
+    2-norm of what that leaves in a weighted mean is below 0.48 of it."""
+    q, k, v = (make_input((1, H, N, 128), seed=s) for s in (53, 54, 55))
+    q[..., 0], k[..., 0] = 3424.0, -3424.0
+    o = ops().attention(q.cuda(), k.cuda(), v.cuda(), layout="BHND", precision="nvfp4").cpu().float()
+    assert torch.isfinite(o).all()
+    ref = A.attention_nvfp4(q, k, v, "BHND").float()
+    assert ((o - ref).norm() / ref.norm()).item() < 0.48
+
+
 @pytest.mark.parametrize("B,Nq,Nkv,H,D,layout", [(1, 1, 1, 1, 8, "BNHD"), (3, 33, 31, 7, 71, "BNHD"), (2, 65, 257, 12, 64, "BNHD"),
                                                  (2, 65, 257, 12, 64, "BHND"), (1, 64, 33, 5, 127, "BHND"), (1, 200, 2100, 9, 128, "BNHD"),
                                                  (11, 100, 77, 12, 65, "BNHD"), (2, 64, 9000, 3, 100, "BHND"), (1, 40, 48, 2, 7, "BNHD")])
