@@ -16,7 +16,6 @@ namespace ac4k {
 
 namespace {
 
-constexpr int AQ_COLS = 128;      // channels of a row of partial results (head dims up to 128)
 constexpr int AQ_MAX_SPLITS = 32; // token spans: every tile of the second kernel reads one partial row per span
 constexpr int AQ_MIN_SPAN = 32;
 constexpr int AQ_STAT_WAVES = 16;  // most waves of a workgroup of the first kernel
@@ -39,7 +38,7 @@ __device__ __forceinline__ uint4 aq_load_stream(const uint16_t *p) {
 // A wave instruction reads 1 KB: the rows of neighbouring heads of one token where these are neighbours in memory
 // (BNHD), rows of neighbouring tokens otherwise (BHND).
 template <bool ABSMAX>
-__device__ __forceinline__ void aq_column_stats(const AttnQuantArgs &a, const AttnOperand &t, int N, int D, void *part,
+__device__ __forceinline__ void aq_column_stats(const AttnQuantArgs &a, const AttnOperand &t, int N, int D, int Dp, void *part,
                                                 uint32_t (*red)[64][8]) {
   const int W = blockDim.x >> 6;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
@@ -98,7 +97,7 @@ __device__ __forceinline__ void aq_column_stats(const AttnQuantArgs &a, const At
         else sum += __uint_as_float(x);
       }
     if (oh < a.H && oc * 8 < D) {
-      const int64_t at = ((int64_t)split * a.B * a.H + b * a.H + oh) * AQ_COLS + aq_channel(oc, D) + e;
+      const int64_t at = ((int64_t)split * a.B * a.H + b * a.H + oh) * Dp + aq_channel(oc, D) + e;
       if (ABSMAX) static_cast<uint32_t *>(part)[at] = mx;
       else static_cast<float *>(part)[at] = sum;
     }
@@ -107,8 +106,8 @@ __device__ __forceinline__ void aq_column_stats(const AttnQuantArgs &a, const At
 
 __global__ __launch_bounds__(64 * AQ_STAT_WAVES) void attn_column_stats_kernel(AttnQuantArgs a) {
   __shared__ uint32_t red[AQ_STAT_WAVES][64][8];
-  if (blockIdx.y == 0) aq_column_stats<false>(a, a.k, a.Nkv, a.D, a.ksum, red);
-  else aq_column_stats<true>(a, a.v, a.Nkv, a.Dv, a.vmax, red);
+  if (blockIdx.y == 0) aq_column_stats<false>(a, a.k, a.Nkv, a.D, a.Dp, a.ksum, red);
+  else aq_column_stats<true>(a, a.v, a.Nkv, a.Dv, a.Dvp, a.vmax, red);
 }
 
 // workgroup index -> tile: the dim that is nearer in memory runs fastest
@@ -148,8 +147,8 @@ __device__ __forceinline__ void aq_int8_tile(const AttnQuantArgs &a, const AttnO
   }
   if (MEAN) {
     float mean[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-    const float *p = a.ksum + bh * AQ_COLS + c0;
-    for (int s = 0; s < a.nsplit; ++s, p += (int64_t)a.B * a.H * AQ_COLS)
+    const float *p = a.ksum + bh * a.Dp + c0;
+    for (int s = 0; s < a.nsplit; ++s, p += (int64_t)a.B * a.H * a.Dp)
 #pragma unroll
       for (int e = 0; e < 8; ++e) mean[e] += p[e];
 #pragma unroll
@@ -205,8 +204,8 @@ __device__ __forceinline__ void aq_fp8_tile(const AttnQuantArgs &a, int b, int h
     if (live && k < a.Nkv) v[i] = aq_load(src + (int64_t)k * a.v.s_n);
   }
   uint32_t mx[8] = {0, 0, 0, 0, 0, 0, 0, 0};
-  const uint32_t *p = a.vmax + bh * AQ_COLS + c0;
-  for (int s = 0; s < a.nsplit; ++s, p += (int64_t)a.B * a.H * AQ_COLS)
+  const uint32_t *p = a.vmax + bh * a.Dvp + c0;
+  for (int s = 0; s < a.nsplit; ++s, p += (int64_t)a.B * a.H * a.Dvp)
 #pragma unroll
     for (int e = 0; e < 8; ++e) mx[e] = umax32(mx[e], p[e]);
   if (blk == 0 && wave == 0 && kb == 0) {  // the scales of this head
@@ -363,14 +362,19 @@ int64_t take(int64_t &at, int64_t bytes) {
 
 }  // namespace
 
-// Token spans of the first kernel: enough workgroups to have the whole GPU loading (512 of 32 KB in flight each), at
-// least 32 tokens each, and at most 32 spans, because every tile of the second kernel reads one partial row per span.
+// Token spans of the first kernel: enough workgroups to have the whole GPU loading, at least 32 tokens each, and at most
+// 32 spans, because every tile of the second kernel reads one partial row per span.  `groups`: groups of heads that a
+// workgroup takes, K and V together.
+static int64_t aq_spans(int64_t groups, int64_t Nkv) {
+  int64_t n = ceil_div(512, groups);
+  if (n > AQ_MAX_SPLITS) n = AQ_MAX_SPLITS;
+  return n < ceil_div(Nkv, AQ_MIN_SPAN) ? n : ceil_div(Nkv, AQ_MIN_SPAN);
+}
+static int aq_heads_per_wave(int D) { return D > 64 ? 4 : 8; }  // where the rows of neighbouring heads are adjacent
+
 void attn_quant_plan(AttnQuantArgs &a) {
-  const int64_t groups = 2 * (int64_t)a.B * ceil_div(a.H, a.k.s_h < a.k.s_n && a.H > 1 ? (a.D > 64 ? 4 : 8) : 1);
-  int64_t nsplit = ceil_div(512, groups);
-  if (nsplit > AQ_MAX_SPLITS) nsplit = AQ_MAX_SPLITS;
-  if (nsplit > ceil_div(a.Nkv, AQ_MIN_SPAN)) nsplit = ceil_div(a.Nkv, AQ_MIN_SPAN);
-  a.span = (int)ceil_div(a.Nkv, nsplit);
+  const int64_t groups = 2 * (int64_t)a.B * ceil_div(a.H, a.k.s_h < a.k.s_n && a.H > 1 ? aq_heads_per_wave(a.D) : 1);
+  a.span = (int)ceil_div(a.Nkv, aq_spans(groups, a.Nkv));
   a.nsplit = (int)ceil_div(a.Nkv, a.span);
   a.inv_nkv = 1.0f / (float)a.Nkv;
 }
@@ -387,15 +391,17 @@ int64_t attn_quant_layout(AttnQuantArgs &a, void *ws) {
   a.q_sf = reinterpret_cast<float *>(w + take(at, BH * a.nqb * 4));
   a.k_sf = reinterpret_cast<float *>(w + take(at, BH * a.nkb * 4));
   a.v_sf = reinterpret_cast<float *>(w + take(at, BH * a.Dvp * 4));
-  // (bound of the plan's spans, so that the size does not depend on the strides)
-  a.ksum = reinterpret_cast<float *>(w + take(at, AQ_MAX_SPLITS * BH * AQ_COLS * 4));
-  a.vmax = reinterpret_cast<uint32_t *>(w + take(at, AQ_MAX_SPLITS * BH * AQ_COLS * 4));
+  // the plan has at most the spans of the fewest groups, so that the size does not depend on the strides: one where there
+  // are many heads (4096 x 12 heads of 64 tokens, D = 64: 25 MB in all)
+  const int64_t most = aq_spans(2 * (int64_t)a.B * ceil_div(a.H, aq_heads_per_wave(a.D)), a.Nkv);
+  a.ksum = reinterpret_cast<float *>(w + take(at, most * BH * a.Dp * 4));
+  a.vmax = reinterpret_cast<uint32_t *>(w + take(at, most * BH * a.Dvp * 4));
   return at;
 }
 
 void launch_attn_quant(const AttnQuantArgs &a, hipStream_t st) {
   auto units = [&](const AttnOperand &t, int D) {
-    const int heads = t.s_h < t.s_n && a.H > 1 ? (D > 64 ? 4 : 8) : 1;
+    const int heads = t.s_h < t.s_n && a.H > 1 ? aq_heads_per_wave(D) : 1;
     return (int64_t)a.nsplit * a.B * ceil_div(a.H, heads);
   };
   const int64_t uk = units(a.k, a.D), uv = units(a.v, a.Dv);

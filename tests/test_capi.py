@@ -126,3 +126,16 @@ def test_reference_import_lines_resolve():
     # the alias must not pull in the checker either
     for f in ("__init__.py", os.path.join("ops", "__init__.py")):
         assert "oracle" not in open(os.path.join(ROOT, "ac4k_kernel", f)).read()
+
+
+@pytest.mark.parametrize("B,H,Nq,Nkv,D,Dv", [(4096, 12, 64, 64, 64, 64), (65535, 12, 49, 49, 32, 32), (1024, 3, 256, 256, 40, 128),
+                                             (2, 12, 777, 257, 64, 64), (1, 1, 40, 9000, 8, 128), (1, 40, 16384, 16384, 128, 128)])
+def test_attention_workspace_is_no_larger_than_the_separate_operators(B, H, Nq, Nkv, D, Dv):
+    """The whole INT8 x FP8 call keeps the quantized operands and partial results; operator by operator the same operands lie
+    beside a bf16 copy of K (less its mean), so whatever fits there fits here."""
+    from ac4k_kernel_amd import _lib
+    up = lambda a, b: -(-a // b) * b  # noqa: E731
+    operands = Nq * up(D, 16) + Nkv * up(D, 16) + Dv * up(Nkv, 16) + 4 * (-(-Nq // 64) - (-Nkv // 128) + up(Dv, 16))
+    k_copy = 2 * Nkv * D
+    got = _lib.load().ac4k_attention_int8_x_fp8_workspace_bytes(B, H, Nq, Nkv, D, Dv)
+    assert B * H * operands <= got <= B * H * (operands + k_copy) + 8 * 256  # eight buffers, 256-byte aligned
