@@ -45,6 +45,7 @@ constexpr float MHA_P_ALPHA = 2688.0f;  // 1 / (global scale of P)
 // each; every block behind them is cut into `tail` workgroups of 256 / tail rows.
 struct MhaWork {
   uint32_t full, blocks;  // full: a multiple of the number of XCDs; blocks per head
+  uint32_t head0;         // first head of the launch, of those of all batches
 };
 struct MhaTile {
   int64_t block, head, b;  // block: in units of the rows of this workgroup
@@ -57,8 +58,8 @@ __device__ __forceinline__ MhaTile mha_tile(const MhaWork &w, int64_t H, uint32_
   const uint32_t T = blockIdx.x < w.full ? w.full : gridDim.x - w.full;
   const uint32_t xcd = L & 7, q = T >> 3, rem = T & 7;
   const uint32_t id = (xcd < rem ? xcd * (q + 1) : rem * (q + 1) + (xcd - rem) * q) + (L >> 3) + first * tail;
-  const uint32_t per_head = w.blocks * tail, bh = id / per_head;
-  return MhaTile{id - bh * per_head, bh % (uint32_t)H, bh / (uint32_t)H};
+  const uint32_t per_head = w.blocks * tail, local = id / per_head, bh = local + w.head0;
+  return MhaTile{id - local * per_head, bh % (uint32_t)H, bh / (uint32_t)H};
 }
 
 // Plan of a launch.  A workgroup that splits its tiles over 2 or 4 waves needs `tile_us` per kv tile and `fixed_us` for
@@ -77,7 +78,7 @@ static MhaWork mha_plan(const MhaCost &c, int64_t heads, int64_t Nq, int64_t nti
     if (i == 0 || us < best) best = us, *tail = 1 << i;
   }
   *grid = (unsigned)(full + left * *tail);
-  return MhaWork{(uint32_t)full, (uint32_t)blocks};
+  return MhaWork{(uint32_t)full, (uint32_t)blocks, 0};
 }
 
 // eight nibbles times the block scale -> eight fp16 (exact)
@@ -924,15 +925,22 @@ static void (*const mha_nvfp4_kernels[3])(MhaArgs, MhaWork) = {mha_nvfp4_fwd_ker
 static void (*const mha_int8_x_fp8_kernels[3])(Mha8Args, MhaWork) = {mha_int8_x_fp8_fwd_kernel<1>, mha_int8_x_fp8_fwd_kernel<2>,
                                                                      mha_int8_x_fp8_fwd_kernel<4>};
 
+// A launch carries fewer than 2^32 threads along a grid dim: from 2^31 on the heads go out in several launches, each planned
+// by itself.
+constexpr int64_t MHA_MAX_BLOCKS = 1 << 22;
+
 template <typename Args>
 static int mha_launch(const Args &a, int64_t heads, int64_t Nq, int64_t ntiles, const MhaCost &cost, void (*const (&kernels)[3])(Args, MhaWork),
                       int (*lds_bytes)(int), hipStream_t st, const char *what) {
-  int tail = 1;
-  unsigned grid = 0;
-  const MhaWork work = mha_plan(cost, heads, Nq, ntiles, &tail, &grid);
-  auto kern = kernels[tail >> 1];
-  const int lds = lds_bytes(tail);
-  {  // more than 64 KB of dynamic LDS has to be allowed once per device and kernel
+  const int64_t blocks = ceil_div(Nq, 256), most = blocks < MHA_MAX_BLOCKS ? MHA_MAX_BLOCKS / blocks : 1;
+  for (int64_t head0 = 0; head0 < heads; head0 += most) {
+    int tail = 1;
+    unsigned grid = 0;
+    MhaWork work = mha_plan(cost, heads - head0 < most ? heads - head0 : most, Nq, ntiles, &tail, &grid);
+    work.head0 = (uint32_t)head0;
+    auto kern = kernels[tail >> 1];
+    const int lds = lds_bytes(tail);
+    // more than 64 KB of dynamic LDS has to be allowed once per device and kernel
     static std::atomic<uint32_t> lds_done[3] = {{0}, {0}, {0}};
     int dev = 0;
     if (hipGetDevice(&dev) != hipSuccess) dev = 0;
@@ -942,8 +950,8 @@ static int mha_launch(const Args &a, int64_t heads, int64_t Nq, int64_t ntiles, 
       if (e != hipSuccess) return set_error("hipFuncSetAttribute(LDS=%d): %s", lds, hipGetErrorString(e));
       lds_done[tail >> 1].fetch_or(bit, std::memory_order_relaxed);
     }
+    hipLaunchKernelGGL(kern, dim3(grid), dim3(512), lds, st, a, work);
   }
-  hipLaunchKernelGGL(kern, dim3(grid), dim3(512), lds, st, a, work);
   return check_launch(what);
 }
 
@@ -965,7 +973,7 @@ extern "C" __attribute__((visibility("default"))) int ac4k_mha_nvfp4_fwd(
                (long long)Dqk, (long long)Dv);
   AC4K_REQUIRE((((uintptr_t)q | (uintptr_t)k | (uintptr_t)v) & 15) == 0 && (((uintptr_t)q_sf | (uintptr_t)k_sf | (uintptr_t)v_sf) & 3) == 0,
                "q, k, v must be 16-byte aligned and the scale tensors 4-byte aligned");
-  AC4K_REQUIRE(H <= 65535 && B <= 65535 && ceil_div(Nq, 128) < (1ll << 31) && B * H * ceil_div(Nq, 256) < (1ll << 29), "problem too large");
+  AC4K_REQUIRE(H <= 65535 && B <= 65535 && ceil_div(Nq, 128) < (1ll << 31), "problem too large");
   AC4K_REQUIRE(o_b_stride >= 0 && o_h_stride >= 0 && o_n_stride >= 1 && o_d_stride >= 1, "strides of O must be positive");
   MhaArgs a{static_cast<uint16_t *>(O), o_b_stride, o_h_stride, o_n_stride, o_d_stride,
             static_cast<const uint8_t *>(q), static_cast<const uint8_t *>(k), static_cast<const uint8_t *>(v),
@@ -995,7 +1003,7 @@ extern "C" __attribute__((visibility("default"))) int ac4k_mha_int8_x_fp8_fwd(
   AC4K_REQUIRE(Dqk >= 16 && Dv >= 1, "Dqk and Dv must be positive");
   AC4K_REQUIRE((((uintptr_t)q | (uintptr_t)k | (uintptr_t)v | (uintptr_t)v_sf) & 15) == 0,
                "q, k, v and v_sf must be 16-byte aligned");
-  AC4K_REQUIRE(H <= 65535 && B <= 65535 && ceil_div(Nq, 128) < (1ll << 31) && B * H * ceil_div(Nq, 256) < (1ll << 29), "problem too large");
+  AC4K_REQUIRE(H <= 65535 && B <= 65535 && ceil_div(Nq, 128) < (1ll << 31), "problem too large");
   AC4K_REQUIRE(o_b_stride >= 0 && o_h_stride >= 0 && o_n_stride >= 1 && o_d_stride >= 1, "strides of O must be positive");
   Mha8Args a{static_cast<uint16_t *>(O), o_b_stride, o_h_stride, o_n_stride, o_d_stride,
              static_cast<const int8_t *>(q), static_cast<const int8_t *>(k), static_cast<const uint8_t *>(v),
@@ -1025,12 +1033,14 @@ extern "C" __attribute__((visibility("default"))) int ac4k_quantize_int8_token_b
 }
 
 // Whole attention calls on bf16 operands: the quantizers of attention_quantize.hip, then the forward on their outputs.
-static int attention_check_sizes(int64_t B, int64_t H, int64_t Nq, int64_t Nkv, int64_t Dqk, int64_t Dv) {
+// q_tile: query rows that a workgroup of the quantizers takes, beside 128 keys and 256 positions of V; 2^24 workgroups of
+// 256 threads would be 2^32 threads, more than a launch carries
+static int attention_check_sizes(int64_t B, int64_t H, int64_t Nq, int64_t Nkv, int64_t Dqk, int64_t Dv, int q_tile) {
   AC4K_REQUIRE(B >= 1 && H >= 1 && Nq >= 1 && Nkv >= 1, "B, H, Nq, Nkv must be positive (B=%lld H=%lld Nq=%lld Nkv=%lld)",
                (long long)B, (long long)H, (long long)Nq, (long long)Nkv);
   AC4K_REQUIRE(Dqk >= 8 && Dqk <= 128 && Dv >= 8 && Dv <= 128, "Dqk and Dv must be 8 to 128");
   AC4K_REQUIRE(H <= 65535 && B <= 65535 && Nq < (1ll << 30) && Nkv < (1ll << 30) &&
-               B * H * (ceil_div(Nq, 64) + ceil_div(Nkv, 64)) < (1ll << 31), "problem too large");
+               B * H * (ceil_div(Nq, (int64_t)q_tile) + ceil_div(Nkv, 128) + ceil_div(Nkv, 256)) < (1ll << 24), "problem too large");
   return 0;
 }
 template <typename Args>
@@ -1050,7 +1060,7 @@ static int attention_operands(Args &a, const void *q, int64_t q_b, int64_t q_h, 
 // Replaces _int8_x_fp8_attention (python/ac4k_kernel/ops/attention.py:137-190): the quantizers of attention_quantize.hip,
 // then ac4k_mha_int8_x_fp8_fwd on their outputs.
 static int attention_int8_args(AttnQuantArgs &a, int64_t B, int64_t H, int64_t Nq, int64_t Nkv, int64_t Dqk, int64_t Dv) {
-  if (int rc = attention_check_sizes(B, H, Nq, Nkv, Dqk, Dv)) return rc;
+  if (int rc = attention_check_sizes(B, H, Nq, Nkv, Dqk, Dv, AQ_Q_BLOCK)) return rc;
   a = AttnQuantArgs{};
   a.B = (int)B, a.H = (int)H, a.Nq = (int)Nq, a.Nkv = (int)Nkv, a.D = (int)Dqk, a.Dv = (int)Dv;
   return 0;
@@ -1086,7 +1096,7 @@ extern "C" __attribute__((visibility("default"))) int ac4k_attention_int8_x_fp8_
 
 // Replaces _nvfp4_attention (python/ac4k_kernel/ops/attention.py:100-133).
 static int attention_nvfp4_args(AttnNvfp4Args &a, int64_t B, int64_t H, int64_t Nq, int64_t Nkv, int64_t Dqk, int64_t Dv) {
-  if (int rc = attention_check_sizes(B, H, Nq, Nkv, Dqk, Dv)) return rc;
+  if (int rc = attention_check_sizes(B, H, Nq, Nkv, Dqk, Dv, 128)) return rc;
   a = AttnNvfp4Args{};
   a.B = (int)B, a.H = (int)H, a.Nq = (int)Nq, a.Nkv = (int)Nkv, a.D = (int)Dqk, a.Dv = (int)Dv;
   return 0;

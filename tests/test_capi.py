@@ -139,3 +139,12 @@ def test_attention_workspace_is_no_larger_than_the_separate_operators(B, H, Nq, 
     k_copy = 2 * Nkv * D
     got = _lib.load().ac4k_attention_int8_x_fp8_workspace_bytes(B, H, Nq, Nkv, D, Dv)
     assert B * H * operands <= got <= B * H * (operands + k_copy) + 8 * 256  # eight buffers, 256-byte aligned
+
+
+def test_whole_attention_leaves_head_counts_beyond_a_launch_to_the_separate_operators():
+    """2^24 workgroups of 256 threads are 2^32 threads: a launch does not carry them, so the whole calls do not take the sizes."""
+    from ac4k_kernel_amd import _lib
+    lib = _lib.load()
+    for f in (lib.ac4k_attention_int8_x_fp8_workspace_bytes, lib.ac4k_attention_nvfp4_workspace_bytes):
+        assert f(1024, 5461, 1, 1, 16, 16) > 0   # three workgroups a head: 2^24 - 1024
+        assert f(4096, 2049, 1, 1, 16, 16) == -1
