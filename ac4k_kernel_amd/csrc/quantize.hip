@@ -989,6 +989,10 @@ static bool rowmajor_ok(const void *in, int64_t K, int64_t s0, int64_t s1, int64
          s0 % 8 == 0 && s1 % 8 == 0;
 }
 
+// A launch carries fewer than 2^32 threads along a grid dim and drops the rest without an error.  The kernels that give a row
+// several lanes, and the fill of the scales, leave more rows than that to the generic kernels, which give it one.
+static bool launch_holds(int64_t threads) { return threads <= (1ll << 32) - 256; }
+
 // cross dim contiguous, at least one whole group of eight rows
 static bool crossmajor_ok(int64_t R, int64_t sR) { return sR == 1 && R >= 8; }
 
@@ -1006,12 +1010,17 @@ static void launch_nvfp4_rowmajor(uint8_t *out, uint8_t *sf, const uint16_t *in,
 
 // four chunks per wave row: a workgroup then covers 32 rows x 256 elements, and each scale
 // column gets a 128-byte run; eight chunks per row measured 4-12 % slower on every shape
+static int64_t nvfp4_chunks_per_row(const QuantGeom &g) { return g.Kp / 64 >= 3 ? 4 : g.Kp / 64; }
+static bool nvfp4_contiguous_ok(const QuantGeom &g, int64_t sK) {  // (a workgroup: 128 chunk rows)
+  const int64_t cpr = nvfp4_chunks_per_row(g);
+  return sK == 1 && g.K >= 8 && launch_holds(ceil_div(g.Kp / 64, cpr) * ceil_div(g.Rp, 128 / cpr) * 256);
+}
 template <bool ALIGNED>
 static void launch_nvfp4_contiguous(uint8_t *out, uint8_t *sf, const uint16_t *in, const float *gs, const QuantGeom &g,
                                     int64_t lead, hipStream_t st, bool swizzle) {
-  const int64_t chunks = g.Kp / 64;
-  if (chunks >= 3) launch_nvfp4_rowmajor<4, ALIGNED>(out, sf, in, gs, g, lead, st, swizzle);
-  else if (chunks == 2) launch_nvfp4_rowmajor<2, ALIGNED>(out, sf, in, gs, g, lead, st, swizzle);
+  const int64_t cpr = nvfp4_chunks_per_row(g);
+  if (cpr == 4) launch_nvfp4_rowmajor<4, ALIGNED>(out, sf, in, gs, g, lead, st, swizzle);
+  else if (cpr == 2) launch_nvfp4_rowmajor<2, ALIGNED>(out, sf, in, gs, g, lead, st, swizzle);
   else launch_nvfp4_rowmajor<1, ALIGNED>(out, sf, in, gs, g, lead, st, swizzle);
 }
 
@@ -1228,7 +1237,7 @@ static int launch_quantize_nvfp4(void *out, void *sf, const void *in, const floa
   const int64_t lead_all = d0 * d1;
   for (g.lead0 = 0; g.lead0 < lead_all; g.lead0 += 65535) {
     const int64_t lead = lead_all - g.lead0 < 65535 ? lead_all - g.lead0 : 65535;
-    if (sK == 1 && K >= 8 && ceil_div(g.Kp, 64) * ceil_div(g.Rp, 16) < (1ll << 31)) {
+    if (nvfp4_contiguous_ok(g, sK)) {
       if (rowmajor_ok(in, K, s0, s1, sR, sK))
         launch_nvfp4_contiguous<true>(o, s, x, gsrc, g, lead, st, swizzle != 0);
       else
@@ -1308,6 +1317,9 @@ static void launch_rowwise_rowmajor(uint8_t *out, float *sf, const uint16_t *in,
 }
 
 // rows contiguous: in the registers of LPR lanes up to 16384 elements, longer ones one wave and two reads
+static bool rowwise_contiguous_ok(const QuantGeom &g, int64_t sK) {
+  return sK == 1 && g.K >= 8 && launch_holds(align_up(g.Rp, 32) * (g.K <= 64 ? 8 : g.K <= 128 ? 16 : g.K <= 256 ? 32 : 64));
+}
 template <RowFmt FMT, bool SWIZZLE, bool ALIGNED>
 static void launch_rowwise_contiguous(uint8_t *out, float *sf, const uint16_t *in, const void *smax, const QuantGeom &g,
                                       int64_t lead, hipStream_t st) {
@@ -1370,13 +1382,14 @@ static int quantize_rowwise(void *out, float *sf, const void *in, const void *sm
   for (g.lead0 = 0; g.lead0 < lead_all; g.lead0 += 65535) {
     const int64_t lead = lead_all - g.lead0 < 65535 ? lead_all - g.lead0 : 65535;
     constexpr bool CAN_SWIZZLE = FMT == RowFmt::FP8;  // (the int8 entry point has no swizzle)
-    if (sK == 1 && K >= 8) {
+    if (rowwise_contiguous_ok(g, sK)) {
       const bool aligned = rowmajor_ok(in, K, s0, s1, sR, sK);
       if (swizzle && aligned) launch_rowwise_contiguous<FMT, CAN_SWIZZLE, true>(o, sf, x, smax, g, lead, st);
       else if (swizzle) launch_rowwise_contiguous<FMT, CAN_SWIZZLE, false>(o, sf, x, smax, g, lead, st);
       else if (aligned) launch_rowwise_contiguous<FMT, false, true>(o, sf, x, smax, g, lead, st);
       else launch_rowwise_contiguous<FMT, false, false>(o, sf, x, smax, g, lead, st);
-    } else if (crossmajor_ok(R, sR) && ceil_div(g.Rp, 128) <= 65535 && ceil_div(K, CM_AMAX_SPAN) <= 65535) {
+    } else if (crossmajor_ok(R, sR) && ceil_div(g.Rp, 128) <= 65535 && ceil_div(K, CM_AMAX_SPAN) <= 65535 &&
+               launch_holds(lead * g.Rp)) {
       if (lead * R * K * 2 > CM_STREAM_BYTES) launch_rowwise_crossmajor<FMT, true>(o, sf, x, smax, g, lead, swizzle, st);
       else launch_rowwise_crossmajor<FMT, false>(o, sf, x, smax, g, lead, swizzle, st);
     } else {

@@ -626,3 +626,20 @@ def test_quantize_next_to_a_long_gemm_on_another_stream():
         assert torch.equal(out.cpu(), exp[0]) and torch.equal(sf.cpu().view(torch.uint8), exp[1]) and gs.item() == exp[2].item()
     assert set(paths) <= {PATH_ONEPASS, PATH_TWO_KERNEL}
     L.ac4k_set_quantize_sync_timeout_us(200)
+
+
+@pytest.mark.parametrize("precision", ["fp8e4m3", "int8"])
+def test_more_rows_than_one_launch_of_the_contiguous_kernels_carries(precision):
+    """2^29 short rows, unaligned, at eight lanes a row: 2^32 threads and a few, which the launch would drop."""
+    block, times, rest = 1 << 20, 512, 33
+    base = make_input((block, 9), seed=61).cuda()
+    eo, es = ops().quantize(base, 0, 1, precision=precision)
+    x = torch.empty((times * block + rest, 9), dtype=torch.bfloat16, device="cuda")
+    x[:times * block].view(times, block, 9).copy_(base[None])
+    x[times * block:] = base[:rest]
+    out, sf = ops().quantize(x, 0, 1, precision=precision)
+    del x
+    raw, eo = out.view(torch.uint8), eo.view(torch.uint8)
+    for i in range(times + 1):
+        n = block if i < times else rest
+        assert torch.equal(raw[i * block:i * block + n], eo[:n]) and torch.equal(sf[i * block:i * block + n], es[:n]), i
