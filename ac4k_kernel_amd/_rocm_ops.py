@@ -350,8 +350,10 @@ def mha_int8_x_fp8_fwd(o, q, q_sf, q_quantize_block_size: int, k, k_sf, k_quanti
 def _attention(entry, workspace_bytes, o, q, k, v, scale: float, sm_scale: float) -> bool:
     B, H, Nq, Dqk = q.shape
     Nkv, Dv = k.shape[2], v.shape[3]
+    dev = q.get_device()  # -1 on the CPU
     if not (k.shape == (B, H, Nkv, Dqk) and v.shape == (B, H, Nkv, Dv) and o.shape == (B, H, Nq, Dv)
-            and q.is_cuda and k.is_cuda and v.is_cuda and o.is_cuda and o.dtype == torch.bfloat16):
+            and dev >= 0 and dev == k.get_device() == v.get_device() == o.get_device()
+            and q.dtype == k.dtype == v.dtype == o.dtype == torch.bfloat16):
         return False
     (q_b, q_h, q_n, q_d), (k_b, k_h, k_n, k_d), (v_b, v_h, v_n, v_d) = q.stride(), k.stride(), v.stride()
     if q_d != 1 or k_d != 1 or v_d != 1:
@@ -368,7 +370,7 @@ def _attention(entry, workspace_bytes, o, q, k, v, scale: float, sm_scale: float
 def attention_int8_x_fp8(o, q, k, v, v_scale_max: float, sm_scale: float) -> bool:
     """The whole `_int8_x_fp8_attention` (python/ac4k_kernel/ops/attention.py:137-190) behind one C call on bf16 q, k, v
     viewed as [B,H,N,D] (any batch, head and token strides).  False, with nothing done, for operands this call does not
-    take - odd shapes and the ones an operator-by-operator call rejects with its own message."""
+    take - odd shapes, other dtypes and the ones an operator-by-operator call rejects with its own message."""
     return _attention(_L.ac4k_attention_int8_x_fp8_bf16, _L.ac4k_attention_int8_x_fp8_workspace_bytes, o, q, k, v, v_scale_max, sm_scale)
 
 

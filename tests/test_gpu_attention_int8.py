@@ -155,6 +155,23 @@ def test_error_behaviour():
         b.mha_int8_x_fp8_fwd(o, q24, sf, 64, q24, sf, 128, v, v_sf, 1.0)
 
 
+@pytest.mark.parametrize("dtype", [torch.float16, torch.float32, torch.uint8])
+def test_whole_call_takes_bf16_on_one_device_only(dtype):
+    """The whole calls hand pointers to kernels that read bf16: everything else is left to the operators, whose checks name it."""
+    import importlib
+    front = importlib.import_module("ac4k_kernel_amd.ops.attention")
+    b, x = binding(), make_input((1, 2, 16, 64), seed=1).cuda()
+    for bad in (x.to(dtype), x.cpu()):
+        for args in ((bad, x, x), (x, bad, x), (x, x, bad)):
+            assert not b.attention_int8_x_fp8(torch.empty_like(x), *args, 2.25, 0.125)
+            assert not b.attention_nvfp4(torch.empty_like(x), *args, 0.125)
+        assert not b.attention_int8_x_fp8(torch.empty_like(bad), x, x, x, 2.25, 0.125)
+    y = x.to(dtype)
+    for call in (front._int8_x_fp8_attention, front._nvfp4_attention):
+        with pytest.raises(RuntimeError):
+            call(y, y, y, "BHND")
+
+
 @pytest.mark.parametrize("precision", ["int8+fp8e4m3", "nvfp4"])
 def test_reference_long_sequence_shape(precision):
     """The long shape of the reference's test list, (1, 75600, 1, 128) BNHD (test/test_attention_bench.py:69-77), for
