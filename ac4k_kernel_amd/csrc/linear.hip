@@ -2487,23 +2487,22 @@ extern "C" __attribute__((visibility("default"))) int ac4k_linear_nvfp4_workspac
                                         const void *B, const void *B_sf, const float *B_gs, const void *bias,
                                         int bias_dtype, int64_t M, int64_t N, int64_t K, void *workspace,
                                         int64_t workspace_bytes, ac4k_stream_t stream) {
-  const int64_t need = ac4k_linear_nvfp4_workspace_bytes(M, N, K);
-  if (need == 0 || skinny_entry_k(M, K))
-    return need == 0 ? ac4k_linear_nvfp4(D, d_dtype, A, A_sf, A_gs, B, B_sf, B_gs, bias, bias_dtype, M, N, K, stream)
-                     : linear_skinny_impl(D, d_dtype, A, A_sf, A_gs, B, B_sf, B_gs, bias, bias_dtype, M, N, K, workspace,
-                                          workspace_bytes, (hipStream_t)stream, "ac4k_linear_nvfp4_workspace");
-  // every other K: operands that are not aligned for the split kernels run without scratch
-  if (!(D && A && A_sf && A_gs && B && B_sf && B_gs) || (((uintptr_t)A | (uintptr_t)B) & 15) || (((uintptr_t)A_sf | (uintptr_t)B_sf) & 3))
-    return ac4k_linear_nvfp4(D, d_dtype, A, A_sf, A_gs, B, B_sf, B_gs, bias, bias_dtype, M, N, K, stream);
+  // what the kernels that split K do not take runs without scratch, for every K alike: shapes that need none, operands that
+  // are not aligned for them, and everything that ac4k_linear_nvfp4 refuses with its own message
+  SkinnyPlan p;
+  MidPlan mp;
+  const bool aligned = D && A && A_sf && A_gs && B && B_sf && B_gs && (((uintptr_t)A | (uintptr_t)B) & 15) == 0 &&
+                       (((uintptr_t)A_sf | (uintptr_t)B_sf) & 3) == 0;
+  const bool skinny = aligned && skinny_plan(M, N, K, p);
+  const bool mid = aligned && !skinny && mid_plan(M, N, K, mp);
+  const int64_t need = skinny ? p.partial_bytes : mid ? mp.bytes : 0;
+  if (need == 0) return ac4k_linear_nvfp4(D, d_dtype, A, A_sf, A_gs, B, B_sf, B_gs, bias, bias_dtype, M, N, K, stream);
   AC4K_REQUIRE(workspace && ((uintptr_t)workspace & 255) == 0, "workspace must be 256-byte aligned");
   AC4K_REQUIRE(workspace_bytes >= need, "workspace too small: %lld bytes needed", (long long)need);
   int rc;
-  SkinnyPlan p;
-  MidPlan mp;
-  if (skinny_plan(M, N, K, p)) {
+  if (skinny) {
     rc = run_skinny(D, d_dtype, A, A_sf, A_gs, B, B_sf, B_gs, bias, bias_dtype, M, N, K, p, workspace, (hipStream_t)stream);
   } else {
-    mid_plan(M, N, K, mp);
     LinearArgs la{D, static_cast<const uint8_t *>(A), static_cast<const uint8_t *>(B),
                   static_cast<const uint32_t *>(A_sf), static_cast<const uint32_t *>(B_sf), A_gs, B_gs, bias,
                   M, N, K, align_up(M, 16), align_up(N, 16)};

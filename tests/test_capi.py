@@ -148,3 +148,14 @@ def test_whole_attention_leaves_head_counts_beyond_a_launch_to_the_separate_oper
     for f in (lib.ac4k_attention_int8_x_fp8_workspace_bytes, lib.ac4k_attention_nvfp4_workspace_bytes):
         assert f(1024, 5461, 1, 1, 16, 16) > 0   # three workgroups a head: 2^24 - 1024
         assert f(4096, 2049, 1, 1, 16, 16) == -1
+
+
+@pytest.mark.parametrize("m,n,k", [(16, 4096, 14336), (16, 4096, 14400), (100, 5003, 2816), (100, 5003, 2880), (300, 256, 4160)])
+def test_linear_workspace_is_checked(m, n, k):
+    from ac4k_kernel_amd import _lib
+    lib, p = _lib.load(), ctypes.c_void_p(256)  # never dereferenced
+    need = lib.ac4k_linear_nvfp4_workspace_bytes(m, n, k)
+    assert need > 0
+    call = lambda ws, size: lib.ac4k_linear_nvfp4_workspace(p, 0, p, p, p, p, p, p, None, 0, m, n, k, ws, size, None)  # noqa: E731
+    for ws, size, text in ((p, need - 1, b"too small"), (None, need, b"256-byte aligned"), (ctypes.c_void_p(272), need, b"256-byte aligned")):
+        assert call(ws, size) != 0 and text in lib.ac4k_last_error()

@@ -475,3 +475,23 @@ def test_k_tail_of_the_tile_kernel(mi, nj, splits, linear_tuning):
     linear_tuning(mi, nj, splits)
     for k in (192, 320, 1216):
         check_tight(64 * mi + 5, 64 * nj + 130, k, seed=k + mi)
+
+
+@pytest.mark.parametrize("m,n,k", [(16, 200, 2048), (16, 200, 2112), (100, 200, 2048), (100, 200, 2112), (300, 256, 4096), (300, 256, 4160)])
+def test_operands_aligned_to_eight_bytes(m, n, k):
+    """Shapes that split K for operands on 16 bytes: the others run without scratch, whatever the remainder of K."""
+    from ac4k_kernel_amd import _lib
+    assert _lib.load().ac4k_linear_nvfp4_workspace_bytes(m, n, k) > 0
+
+    def shifted(q):
+        buf = torch.empty(q[0].numel() + 8, dtype=torch.uint8, device="cuda")
+        x = buf[8:].view(q[0].shape)
+        x.copy_(q[0])
+        assert x.data_ptr() % 16 == 8
+        return x, q[1], q[2]
+
+    aq, bq = gpu_quant(make_input((m, k), seed=m)), gpu_quant(make_input((n, k), seed=n, std=0.02))
+    ref = C.linear_nvfp4(*cpu(aq), *cpu(bq))
+    for a, b in ((shifted(aq), bq), (aq, shifted(bq))):
+        out = ops().linear(*a, *b, out=torch.empty((m, n), dtype=torch.float32, device="cuda"))
+        torch.testing.assert_close(out.cpu(), ref, atol=1e-5, rtol=1e-4)
