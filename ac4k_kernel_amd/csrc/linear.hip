@@ -268,10 +268,12 @@ __global__ __launch_bounds__(256) void linear_nvfp4_tile128_kernel(LinearArgs a)
 // step so that the next stage is readable before the current one ends.
 // Split-K: blockIdx.y selects a contiguous range of stages; with more than one range the
 // accumulators go to an fp32 partial buffer and a second kernel adds the ranges.
-// Requires K % 64 == 0, K >= 128 and 16-byte aligned operands.  K % 128 == 64: the stages start one
+// Requires K % 64 == 0, K >= 128 and 16-byte aligned operands.  EARLY: K % 128 == 64.  The stages start one
 // chunk early, at k = -64, so that only stage 0 is special and the loop is not: the prologue fetches k-chunk 0
 // into both halves of it and clears the scales of the first half.  (1001 x 5003 x 2880, fp32 out: 75 -> 45 us, the
-// 128x128 kernel against this one; 300 x 4096 x 4160: 93 -> 28.)
+// 128x128 kernel against this one; 300 x 4096 x 4160: 93 -> 28.)  A variant of its own: decided at run time, the longer
+// prologue cost the 128 x 128 tiles of every other K 0.2 to 0.4 us (kernel alone, 160 x 2000 x 8192 in eight K ranges:
+// 18.1 us, 17.3 without; 256 x 4096 x 4096 in four 20.7 and 19.8).
 // ===========================================================================
 constexpr int P_BK = 128;     // k per stage (two 64-chunks)
 constexpr int P_ROW = 64;     // packed bytes per row per stage: [chunk][half] x 16 B
@@ -456,7 +458,7 @@ __device__ __forceinline__ void store_tile(const f32x16 (&acc)[MI][NJ], char *ld
 // NJ = 32-column fragments per wave along N: 4 (BN = 256), 2 (BN = 128) or 1 (BN = 64);
 // PS = LDS stages: PS - 1 k-steps are in flight ahead of the one being multiplied, which a small
 // tile needs because its k-step is much shorter than the memory latency.
-template <int D_DT, int BIAS_DT, int MI, int NJ, int PS>
+template <int D_DT, int BIAS_DT, int MI, int NJ, int PS, bool EARLY>
 __global__ __launch_bounds__(256, 1) void linear_nvfp4_tile256p_kernel(LinearArgs a, SplitK sk) {
   extern __shared__ __attribute__((aligned(16))) char plds[];
   AC4K_LTL(0, wall_clock64());
@@ -475,9 +477,9 @@ __global__ __launch_bounds__(256, 1) void linear_nvfp4_tile256p_kernel(LinearArg
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int wm = wave >> 1, wn = wave & 1;
   const int half = lane >> 5;
-  // this workgroup's range of 128-k stages; `early`: bytes by which they start in front of the row (K % 128 == 64)
-  const int nkt_all = (int)ceil_div(a.K, P_BK);
-  const int early = (int)((a.K & 64) >> 1);
+  // this workgroup's range of 128-k stages; `early`: bytes by which they start in front of the row
+  const int nkt_all = (int)(EARLY ? ceil_div(a.K, P_BK) : a.K / P_BK);
+  constexpr int early = EARLY ? 32 : 0;
   const int kt0 = (int)((int64_t)nkt_all * blockIdx.y / sk.splits);
   const int nkt = (int)((int64_t)nkt_all * (blockIdx.y + 1) / sk.splits) - kt0;
 
@@ -548,7 +550,7 @@ __global__ __launch_bounds__(256, 1) void linear_nvfp4_tile256p_kernel(LinearArg
       sr = sr < rows ? sr : rows - 1;
       offS[p2] = (uint32_t)sr * 4u;  // byte offset inside a scale plane
       strideS[p2] = 2 * rows * 4;    // two planes (chunks) per stage
-      baseS[p2] = uniform_ptr((isB ? sfB8 : sfA8) + (c - (early ? 1 : 0)) * rows * 4 + kt0 * strideS[p2]);
+      baseS[p2] = uniform_ptr((isB ? sfB8 : sfA8) + (c - (EARLY ? 1 : 0)) * rows * 4 + kt0 * strideS[p2]);
     }
     if (c == 0) firstS |= 1u << p2;
     ldsS[p2] = (uint32_t)__builtin_amdgcn_readfirstlane((isB ? PL::OFF_SFB + c * BN * 4 : PL::OFF_SFA + c * BM * 4) + rb * 256);
@@ -681,10 +683,9 @@ __global__ __launch_bounds__(256, 1) void linear_nvfp4_tile256p_kernel(LinearArg
   const int last = nkt - 1;
   // the stage that fetches past the end repeat: never the short one, whose first half lies in front of the rows
   // (a range of one stage then repeats the stage behind it, which exists: K >= 192)
-  const bool short0 = early && kt0 == 0;
+  const bool short0 = EARLY && kt0 == 0;
   const int again = short0 && last == 0 ? 1 : last;
-  {  // stage 0; a short one takes k-chunk 0 into both halves (by its addresses: a second copy of the transfers behind a
-     // branch cost every launch 0.4 us, 1807 x 3320 x 1152 20.7 against 19.9 us)
+  {  // stage 0; a short one takes k-chunk 0 into both halves, by its addresses
     Src p = src_at(0);
     const uint32_t shift = short0 && dma_piece < 2 ? 32u : 0u;
 #pragma unroll
@@ -814,10 +815,11 @@ constexpr int tile_stages(int mi, int nj) { return mi * nj >= 16 ? 3 : mi * nj >
 template <int D_DT, int BIAS_DT, int MI, int NJ>
 static int launch_tile_p(const LinearArgs &a, const SplitK &sk, hipStream_t st) {
   constexpr int PS = tile_stages(MI, NJ);
-  auto *kern = linear_nvfp4_tile256p_kernel<D_DT, BIAS_DT, MI, NJ, PS>;
+  const bool early = a.K % P_BK != 0;
+  auto *kern = early ? linear_nvfp4_tile256p_kernel<D_DT, BIAS_DT, MI, NJ, PS, true> : linear_nvfp4_tile256p_kernel<D_DT, BIAS_DT, MI, NJ, PS, false>;
   using PL = PLayout<64 * MI, 64 * NJ, PS>;
-  static std::atomic<uint32_t> lds_ok{0};
-  if (int rc = allow_dynamic_lds(kern, lds_ok, PL::LDS_BYTES)) return rc;
+  static std::atomic<uint32_t> lds_ok[2];
+  if (int rc = allow_dynamic_lds(kern, lds_ok[early], PL::LDS_BYTES)) return rc;
   const int64_t ntiles = ceil_div(a.M, 64 * MI) * ceil_div(a.N, 64 * NJ);
   hipLaunchKernelGGL(kern, dim3((unsigned)ntiles, (unsigned)sk.splits), dim3(256), PL::LDS_BYTES, st, a, sk);
   return 0;
