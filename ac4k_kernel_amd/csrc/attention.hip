@@ -42,10 +42,10 @@ constexpr float MHA_LOG2E = 1.4426950408889634f;
 constexpr float MHA_P_ALPHA = 2688.0f;  // 1 / (global scale of P)
 
 // Work of a launch: blocks of 256 query rows of all heads, one after the other.  The first `full` blocks are a workgroup
-// each; every block behind them is cut into `tail` workgroups of 256 / tail rows.
+// each; what is behind them is cut into workgroups of 256 / tail rows.
 struct MhaWork {
-  uint32_t full, blocks;  // full: a multiple of the number of XCDs; blocks per head
-  uint32_t head0;         // first head of the launch, of those of all batches
+  uint32_t full, blocks, cut;  // full: a multiple of the number of XCDs; blocks and cut workgroups per head
+  uint32_t head0;              // first head of the launch, of those of all batches
 };
 struct MhaTile {
   int64_t block, head, b;  // block: in units of the rows of this workgroup
@@ -53,32 +53,40 @@ struct MhaTile {
 // Workgroups are dealt to the eight XCDs in turn: a run of consecutive blocks of one head is given to one XCD, whose L2 then
 // fetches the K and V of that head once for all of them, instead of all eight XCDs fetching those of every head
 // (4096 x 40 x 128 int8 x fp8: 262 -> 260 us, 4096 x 8: 59.3 -> 58.3).
-__device__ __forceinline__ MhaTile mha_tile(const MhaWork &w, int64_t H, uint32_t tail) {
+__device__ __forceinline__ MhaTile mha_tile(const MhaWork &w, int64_t H, uint32_t tail, uint32_t per_head) {
   const uint32_t first = blockIdx.x < w.full ? 0 : w.full, L = blockIdx.x - first;
   const uint32_t T = blockIdx.x < w.full ? w.full : gridDim.x - w.full;
   const uint32_t xcd = L & 7, q = T >> 3, rem = T & 7;
   const uint32_t id = (xcd < rem ? xcd * (q + 1) : rem * (q + 1) + (xcd - rem) * q) + (L >> 3) + first * tail;
-  const uint32_t per_head = w.blocks * tail, local = id / per_head, bh = local + w.head0;
+  const uint32_t local = id / per_head, bh = local + w.head0;
   return MhaTile{id - local * per_head, bh % (uint32_t)H, bh / (uint32_t)H};
 }
 
 // Plan of a launch.  A workgroup that splits its tiles over 2 or 4 waves needs `tile_us` per kv tile and `fixed_us` for
-// everything else; what is left after the whole rounds of unsplit workgroups is cut so that the last round ends soonest.
+// everything else.  Either whole rounds of unsplit workgroups and behind them the rest, cut so that the last round ends
+// soonest; or all of it cut alike, which leaves out the rows that the last block of a head does not have (windows of 49
+// tokens: 64 rows a workgroup instead of 256).
 struct MhaCost {
   float fixed_us[3], tile_us[3];  // split 1, 2, 4
 };
 static MhaWork mha_plan(const MhaCost &c, int64_t heads, int64_t Nq, int64_t ntiles, int *tail, unsigned *grid) {
   const int64_t cus = device_cu_count() >= 8 ? device_cu_count() / 8 * 8 : 256;
   const int64_t blocks = ceil_div(Nq, 256), T = heads * blocks, full = T / cus * cus, left = T - full;
+  auto rounds_us = [&](int64_t wgs, int i) { return (float)ceil_div(wgs, cus) * (c.fixed_us[i] + (float)ntiles * c.tile_us[i]); };
   float best = 0.0f;
-  *tail = 1;
-  for (int i = 0; i < 3 && left; ++i) {
-    const int64_t wgs = full ? left << i : heads * ceil_div(Nq << i, 256);  // (those without a row end at once)
-    const float us = (float)ceil_div(wgs, cus) * (c.fixed_us[i] + (float)ntiles * c.tile_us[i]);
-    if (i == 0 || us < best) best = us, *tail = 1 << i;
+  MhaWork work{0, (uint32_t)blocks, 0, 0};
+  *grid = 0;
+  auto offer = [&](float us, int64_t first, int64_t wgs, int64_t cut, int i) {
+    if ((*grid && us >= best) || first + wgs >= (1ll << 23)) return;  // (2^23 workgroups of 512 threads: more than a launch carries)
+    best = us, *tail = 1 << i, *grid = (unsigned)(first + wgs);
+    work.full = (uint32_t)first, work.cut = (uint32_t)cut;
+  };
+  for (int i = 0; i < (left ? 3 : 1) && full; ++i) offer(rounds_us(full, 0) + rounds_us(left << i, i), full, left << i, blocks << i, i);
+  for (int i = 0; i < 3; ++i) {  // (beside whole rounds only where it gains more than the costs are good for)
+    const int64_t cut = ceil_div(Nq << i, 256);
+    offer(rounds_us(heads * cut, i) * (full ? 1.05f : 1.0f), 0, heads * cut, cut, i);
   }
-  *grid = (unsigned)(full + left * *tail);
-  return MhaWork{(uint32_t)full, (uint32_t)blocks, 0};
+  return work;
 }
 
 // eight nibbles times the block scale -> eight fp16 (exact)
@@ -505,8 +513,8 @@ __device__ __forceinline__ void mha_nvfp4_block(const MhaArgs &a, const MhaTile 
 // (two bodies in one kernel, so that the workgroups of the last round start as the ones in front of them end)
 template <int TAIL>
 __global__ __launch_bounds__(512, 1) void mha_nvfp4_fwd_kernel(MhaArgs a, MhaWork w) {
-  if (TAIL == 1 || blockIdx.x < w.full) mha_nvfp4_block<1>(a, mha_tile(w, a.H, 1));
-  else mha_nvfp4_block<TAIL>(a, mha_tile(w, a.H, TAIL));
+  if (TAIL == 1 || blockIdx.x < w.full) mha_nvfp4_block<1>(a, mha_tile(w, a.H, 1, w.blocks));
+  else mha_nvfp4_block<TAIL>(a, mha_tile(w, a.H, TAIL, w.cut));
 }
 
 // ---------------------------------------------------------------------------------------------------------------
@@ -859,8 +867,8 @@ __device__ __forceinline__ void mha_int8_x_fp8_block(const Mha8Args &a, const Mh
 // (two bodies in one kernel, so that the workgroups of the last round start as the ones in front of them end)
 template <int TAIL>
 __global__ __launch_bounds__(512, 1) void mha_int8_x_fp8_fwd_kernel(Mha8Args a, MhaWork w) {
-  if (TAIL == 1 || blockIdx.x < w.full) mha_int8_x_fp8_block<1>(a, mha_tile(w, a.H, 1));
-  else mha_int8_x_fp8_block<TAIL>(a, mha_tile(w, a.H, TAIL));
+  if (TAIL == 1 || blockIdx.x < w.full) mha_int8_x_fp8_block<1>(a, mha_tile(w, a.H, 1, w.blocks));
+  else mha_int8_x_fp8_block<TAIL>(a, mha_tile(w, a.H, TAIL, w.cut));
 }
 
 // Per-token-block int8 quantizer in front of it (python/ac4k_kernel/ops/attention.py:18-99, a Triton kernel in the

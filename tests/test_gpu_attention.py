@@ -84,7 +84,9 @@ def test_mha_entry_point_on_given_operands_and_out_argument():
 # Launches whose last round is cut into workgroups of 256, 128 and 64 query rows (one round; 256 blocks and a rest of 4 and
 # 124), one kv tile, partial last tiles and groups of waves without a row of their own.
 @pytest.mark.parametrize("H,Nq,Nkv,D", [(1, 50, 20, 64), (2, 300, 129, 128), (3, 129, 1030, 128), (40, 513, 256, 64),
-                                        (130, 300, 200, 64), (190, 260, 300, 64)])
+                                        (130, 300, 200, 64), (190, 260, 300, 64),
+                                        # more than a round of blocks, most of whose rows do not exist: all of them cut in four or in two
+                                        (300, 49, 49, 64), (300, 40, 600, 40), (512, 100, 300, 64), (24, 2637, 1100, 64)])
 def test_split_plans(H, Nq, Nkv, D):
     q, k, v = make_input((1, H, Nq, D), seed=41), make_input((1, H, Nkv, D), seed=42), make_input((1, H, Nkv, D), seed=43)
     o = ops().attention(q.cuda(), k.cuda(), v.cuda(), layout="BHND", precision="nvfp4")

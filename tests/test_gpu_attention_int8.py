@@ -119,7 +119,9 @@ def test_whole_call_equals_operator_by_operator(B, Nq, Nkv, H, D, layout, monkey
 # Launches whose last round is cut: workgroups of 256, 128 and 64 query rows (one round; 256 of 256 rows and a rest of 4 and
 # 124 blocks), one kv tile and partial last tiles, groups without a row of their own; with scales of both signs, which
 # turn the order of the scores around.
-@pytest.mark.parametrize("H,Nq,Nkv", [(1, 50, 20), (2, 300, 129), (3, 129, 1030), (40, 513, 256), (130, 300, 200), (190, 260, 300)])
+@pytest.mark.parametrize("H,Nq,Nkv", [(1, 50, 20), (2, 300, 129), (3, 129, 1030), (40, 513, 256), (130, 300, 200), (190, 260, 300),
+                                      # more than a round of blocks, most of whose rows do not exist: all of them cut in four or in two
+                                      (300, 49, 49), (300, 40, 600), (512, 100, 300), (24, 2637, 1100)])
 @pytest.mark.parametrize("signs", [False, True])
 def test_split_plans_and_negative_scales(H, Nq, Nkv, signs):
     g = torch.Generator().manual_seed(H + Nq)
