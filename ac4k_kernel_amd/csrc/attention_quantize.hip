@@ -19,6 +19,7 @@ namespace {
 constexpr int AQ_MAX_SPLITS = 32; // token spans: every tile of the second kernel reads one partial row per span
 constexpr int AQ_MIN_SPAN = 32;
 constexpr int AQ_STAT_WAVES = 16;  // most waves of a workgroup of the first kernel
+constexpr int AQ_STAT_LOADS = 8;   // loads in flight per lane there
 
 // Lanes that share one row of a head: eight channels per lane.  The last lane of a head dim that is no multiple of
 // eight is moved back to end at it; channels that two lanes share are computed twice, with the same result.
@@ -57,7 +58,7 @@ __device__ __forceinline__ void aq_column_stats(const AttnQuantArgs &a, const At
   const int step = heads_adjacent ? W : W * G;
   float s[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
   uint32_t m[4] = {0, 0, 0, 0};
-  constexpr int U = 8;  // loads in flight per lane
+  constexpr int U = AQ_STAT_LOADS;
   for (int n = beg + (heads_adjacent ? wave : wave * G + g); n < end; n += U * step) {
     uint4 v[U];
 #pragma unroll
@@ -105,7 +106,7 @@ __device__ __forceinline__ void aq_column_stats(const AttnQuantArgs &a, const At
 }
 
 __global__ __launch_bounds__(64 * AQ_STAT_WAVES) void attn_column_stats_kernel(AttnQuantArgs a) {
-  __shared__ uint32_t red[AQ_STAT_WAVES][64][8];
+  extern __shared__ uint32_t red[][64][8];  // one per wave
   if (blockIdx.y == 0) aq_column_stats<false>(a, a.k, a.Nkv, a.D, a.Dp, a.ksum, red);
   else aq_column_stats<true>(a, a.v, a.Nkv, a.Dv, a.Dvp, a.vmax, red);
 }
@@ -400,16 +401,23 @@ int64_t attn_quant_layout(AttnQuantArgs &a, void *ws) {
 }
 
 void launch_attn_quant(const AttnQuantArgs &a, hipStream_t st) {
+  auto adjacent = [&](const AttnOperand &t) { return t.s_h < t.s_n && a.H > 1; };
   auto units = [&](const AttnOperand &t, int D) {
-    const int heads = t.s_h < t.s_n && a.H > 1 ? aq_heads_per_wave(D) : 1;
-    return (int64_t)a.nsplit * a.B * ceil_div(a.H, heads);
+    return (int64_t)a.nsplit * a.B * ceil_div(a.H, adjacent(t) ? aq_heads_per_wave(D) : 1);
   };
   const int64_t uk = units(a.k, a.D), uv = units(a.v, a.Dv);
   // Sixteen waves a workgroup where a span lasts them for several rounds of loads: with about two workgroups per CU (more
   // would be more spans) the loads in flight are what the pass lives on, 116 us with 4 waves, 95 with 8, 83 with 16 for
   // K and V of 16384 x 40 x 128.  Short spans: eight (one round, 4.9 against 5.6 us at 257 x 12 x 64).
-  const int waves = a.span > 256 ? AQ_STAT_WAVES : 8;
-  hipLaunchKernelGGL(attn_column_stats_kernel, dim3((unsigned)(uk > uv ? uk : uv), 2), dim3(64 * waves), 0, st, a);
+  // More workgroups than the GPU holds at once, neighbouring tokens in a wave: no more waves than one round of loads needs, so
+  // that the sums of a wave meet fewer others and more workgroups are there (BHND, us with eight waves and now: 1024 x 8 windows
+  // of 49 tokens, D = 32, 80 and 13; 256 x 12 of 64, D = 64, 32 and 10; 128 x 16 of 100, D = 128, 23 and 18).
+  int waves = a.span > 256 ? AQ_STAT_WAVES : 8;
+  if (a.span <= 256 && uk + uv > 1024 && !adjacent(a.k) && !adjacent(a.v)) {
+    const int rows = AQ_STAT_LOADS * aq_heads_per_wave(a.D > a.Dv ? a.D : a.Dv);
+    for (waves = 1; waves * rows < a.span; waves *= 2) {}
+  }
+  hipLaunchKernelGGL(attn_column_stats_kernel, dim3((unsigned)(uk > uv ? uk : uv), 2), dim3(64 * waves), waves * sizeof(uint32_t[64][8]), st, a);
   hipLaunchKernelGGL(attn_quantize_int8_fp8_kernel, dim3((unsigned)((int64_t)a.B * a.H * (a.nvb + a.nkb + a.nqb))), dim3(256), 0, st, a);
 }
 

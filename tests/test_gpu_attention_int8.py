@@ -101,7 +101,10 @@ def test_entry_point_on_given_operands():
 
 @pytest.mark.parametrize("B,Nq,Nkv,H,D,layout", [(1, 1, 1, 1, 8, "BNHD"), (3, 33, 31, 7, 71, "BNHD"), (2, 65, 257, 12, 64, "BNHD"),
                                                  (2, 65, 257, 12, 64, "BHND"), (1, 64, 33, 5, 127, "BHND"), (1, 200, 2100, 9, 128, "BNHD"),
-                                                 (11, 100, 77, 12, 65, "BNHD"), (2, 64, 9000, 3, 100, "BHND"), (1, 40, 48, 2, 7, "BNHD")])
+                                                 (11, 100, 77, 12, 65, "BNHD"), (2, 64, 9000, 3, 100, "BHND"), (1, 40, 48, 2, 7, "BNHD"),
+                                                 # statistics with one, two, four and eight waves a workgroup (BHND, many heads)
+                                                 (80, 20, 49, 8, 40, "BHND"), (80, 20, 100, 8, 64, "BHND"), (100, 9, 127, 6, 128, "BHND"),
+                                                 (100, 9, 200, 6, 100, "BHND")])
 def test_whole_call_equals_operator_by_operator(B, Nq, Nkv, H, D, layout, monkeypatch):
     """The two-launch quantizers of attention() against the separate operators.  Everything is bit-identical except that
     a channel mean summed in another order may round to the neighbouring bf16 (2^-9 of the mean, far below a step of
