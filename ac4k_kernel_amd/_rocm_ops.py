@@ -348,12 +348,14 @@ def mha_int8_x_fp8_fwd(o, q, q_sf, q_quantize_block_size: int, k, k_sf, k_quanti
 
 
 def _attention(entry, workspace_bytes, o, q, k, v, scale: float, sm_scale: float) -> bool:
-    B, H, Nq, Dqk = q.shape
-    Nkv, Dv = k.shape[2], v.shape[3]
-    dev = q.get_device()  # -1 on the CPU
-    if not (k.shape == (B, H, Nkv, Dqk) and v.shape == (B, H, Nkv, Dv) and o.shape == (B, H, Nq, Dv)
+    try:
+        (B, H, Nq, Dqk), (k_B, k_H, Nkv, k_D), (v_B, v_H, v_N, Dv), (o_B, o_H, o_N, o_D) = q.shape, k.shape, v.shape, o.shape
+    except ValueError:  # not 4D
+        return False
+    dev, bf16 = q.get_device(), torch.bfloat16  # -1 on the CPU
+    if not (B == k_B == v_B == o_B and H == k_H == v_H == o_H and Nkv == v_N and Nq == o_N and Dqk == k_D and Dv == o_D
             and dev >= 0 and dev == k.get_device() == v.get_device() == o.get_device()
-            and q.dtype == k.dtype == v.dtype == o.dtype == torch.bfloat16):
+            and q.dtype is bf16 and k.dtype is bf16 and v.dtype is bf16 and o.dtype is bf16):
         return False
     (q_b, q_h, q_n, q_d), (k_b, k_h, k_n, k_d), (v_b, v_h, v_n, v_d) = q.stride(), k.stride(), v.stride()
     if q_d != 1 or k_d != 1 or v_d != 1:

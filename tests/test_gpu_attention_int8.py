@@ -171,6 +171,9 @@ def test_whole_call_takes_bf16_on_one_device_only(dtype):
             assert not b.attention_int8_x_fp8(torch.empty_like(x), *args, 2.25, 0.125)
             assert not b.attention_nvfp4(torch.empty_like(x), *args, 0.125)
         assert not b.attention_int8_x_fp8(torch.empty_like(bad), x, x, x, 2.25, 0.125)
+    for bad in (x[0], x[:, :1], x[:, :, :8], x[..., :32]):  # other dims, heads, lengths, head dims than the rest
+        for o, k, v in ((bad, x, x), (x, bad, x), (x, x, bad)):
+            assert not b.attention_int8_x_fp8(o.contiguous(), x, k.contiguous(), v.contiguous(), 2.25, 0.125), (o.shape, k.shape, v.shape)
     y = x.to(dtype)
     for call in (front._int8_x_fp8_attention, front._nvfp4_attention):
         with pytest.raises(RuntimeError):
