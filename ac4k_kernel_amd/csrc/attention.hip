@@ -232,7 +232,12 @@ static_assert(8 * 16384 <= MHA_STAT_LDS && 8 * MHA_OUT_LDS <= MHA_STAT_LDS, "the
 // GHz.  Kernel alone, same box, before (128 or 256 rows, no pipeline, no split) and now: 16384 x 40 x 128 6042 -> 5410 us
 // (1016 TFLOP/s; 1085 on a cooler box), 4096 x 40 422 -> 370, 8192 x 4 194 -> 165, 3000 x 24 214 -> 162, 512 x 2 on 8192
 // keys 191 -> 107, 75600 x 1 5250 -> 3676.
-template <int SPLIT>
+// TILES: 1 and 2 for calls of so many kv tiles, 0 for any number.  The step in front of the first tile and the one behind the
+// last are then not there - multiplying by zeros and fetching a tile again - which made the pipeline slower than one tile after
+// the other at those lengths.  Kernels of their own: written out for every length, or behind a branch in this one, they cost
+// the loop registers (2 %, and spills).  Kernel alone, us, before the pipeline / with its loop / now: 8192 heads of 49 x 49, D = 32,
+// 240 / 209 / 168 (workgroups of 64 rows); 1024 heads of 256 x 256, D = 64, 55.5 / 58.5 / 49.5; 40 heads of 16384 x 200 148 / 152 / 130.
+template <int SPLIT, int TILES>
 __device__ __forceinline__ void mha_nvfp4_block(const MhaArgs &a, const MhaTile &wg) {
   constexpr int NF = 4 / SPLIT;  // 32-row fragments of a tile per wave
   constexpr int ROWS = 256 / SPLIT;
@@ -300,9 +305,12 @@ __device__ __forceinline__ void mha_nvfp4_block(const MhaArgs &a, const MhaTile 
 
   float *const lut = reinterpret_cast<float *>(mha_lds + MHA_LUT_LDS);
   if (threadIdx.x < 128) lut[threadIdx.x] = g_rcp_e4m3.v[threadIdx.x];
-  fetch_k(1);  // (both in flight together: the registers of V are free)
-  fv = fk, fvsc = fksc;
+  if constexpr (TILES != 1) {
+    fetch_k(1);  // (both in flight together: the registers of V are free)
+    fv = fk, fvsc = fksc;
+  }
   fetch_k(0);
+  if constexpr (TILES == 1) fetch_v(0);
   // Qhat of the lane's row: 8 operands of 16 k (chunk c, sub-step s), kept for the whole kernel
   f16x8 QF[2][4];
 #pragma unroll
@@ -324,8 +332,10 @@ __device__ __forceinline__ void mha_nvfp4_block(const MhaArgs &a, const MhaTile 
   }
 #pragma unroll
   for (int p = 0; p < 4; ++p) stage_piece(0, p);
-  fk = fv, fksc = fvsc;
-  fetch_v(0);
+  if constexpr (TILES != 1) {
+    fk = fv, fksc = fvsc;
+    fetch_v(0);
+  }
   float ml_run = -__builtin_inff(), l_run = 0.0f;  // running row maximum (in log2 units) and row sum
   float alpha = 1.0f;                              // factor of O and l that the last tile's maximum asks for
   f32x16 OT[4];  // O^T: d = 32 fd + 8 (e >> 2) + 4 h + (e & 3), for the lane's query row
@@ -333,14 +343,18 @@ __device__ __forceinline__ void mha_nvfp4_block(const MhaArgs &a, const MhaTile 
   for (int fd = 0; fd < 4; ++fd) OT[fd] = (f32x16)(0.0f);
   uint32_t PW[2 * NF];  // P of a tile: eight nibbles per (fragment, step of 16 kv positions)
   uint32_t pcode[NF];   // and its block scales
+  if constexpr (TILES == 0) {
 #pragma unroll
-  for (int f = 0; f < NF; ++f) PW[2 * f] = PW[2 * f + 1] = pcode[f] = 0;
-  // V of the tile in front of the first one: zeros, and so is its P
+    for (int f = 0; f < NF; ++f) PW[2 * f] = PW[2 * f + 1] = pcode[f] = 0;
+    // V of the tile in front of the first one: zeros, and so is its P
 #pragma unroll
-  for (int j = 0; j < 4; ++j) *reinterpret_cast<uint4 *>(vd + MHA_TILE_LDS + j * 16) = make_uint4(0, 0, 0, 0);
+    for (int j = 0; j < 4; ++j) *reinterpret_cast<uint4 *>(vd + MHA_TILE_LDS + j * 16) = make_uint4(0, 0, 0, 0);
+  }
+  if constexpr (TILES != 1) {
 #pragma unroll
-  for (int p = 0; p < 4; ++p) stage_piece(1, p);
-  fetch_k(2);
+    for (int p = 0; p < 4; ++p) stage_piece(1, p);
+  }
+  if constexpr (TILES == 0) fetch_k(2);
   __syncthreads();
 
   f32x16 ST[NF];  // S^T of the tile at hand
@@ -387,38 +401,43 @@ __device__ __forceinline__ void mha_nvfp4_block(const MhaArgs &a, const MhaTile 
   if constexpr (SPLIT > 1) part_maximum(0);
   __syncthreads();
 
-  auto tile_step = [&](int i) {
+  auto tile_step = [&](auto first_tag, auto last_tag, int i) {
+    constexpr bool FIRST = decltype(first_tag)::value, LAST = decltype(last_tag)::value;  // no tile in front of / behind this one
     const int buf = i & 1;
-    f16x8 VF[RING];
+    f16x8 VF[RING], PF;
+    if constexpr (!FIRST) {
 #pragma unroll
-    for (int u = 0; u < RING; ++u) VF[u] = v_operand(buf ^ 1, u);
-    rescale();
+      for (int u = 0; u < RING; ++u) VF[u] = v_operand(buf ^ 1, u);
+      rescale();
+      PF = p_operand(0);
+    }
     // ---- all but the last fragment of O of the tile before; under it the decoding of what was fetched and (SPLIT 1) the
     // maxima of this tile
-    f16x8 PF = p_operand(0);
-    constexpr int PVA = 8 * (NF - 1);
+    constexpr int PVA = 8 * (NF - 1), PIECE0 = TILES != 0 ? 4 : 0;
     if constexpr (NF == 1) {
 #pragma unroll
-      for (int p = 0; p < 8; ++p) stage_piece(buf, p);
+      for (int p = PIECE0; p < 8; ++p) stage_piece(buf, p);
     }
     __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
     for (int u = 0; u < PVA; ++u) {
-      OT[u & 3] = __builtin_amdgcn_mfma_f32_32x32x16_f16(VF[u % RING], PF, OT[u & 3], 0, 0, 0);
-      VF[u % RING] = v_operand(buf ^ 1, u + RING);
-      if ((u & 3) == 3) PF = p_operand((u >> 2) + 1);
+      if constexpr (!FIRST) {
+        OT[u & 3] = __builtin_amdgcn_mfma_f32_32x32x16_f16(VF[u % RING], PF, OT[u & 3], 0, 0, 0);
+        VF[u % RING] = v_operand(buf ^ 1, u + RING);
+        if ((u & 3) == 3) PF = p_operand((u >> 2) + 1);
+      }
       if (SPLIT == 1 && u < 16) {
         float &b = bmax[(u >> 2) % NF];
 #pragma unroll
         for (int e = 4 * (u & 3); e < 4 * (u & 3) + 4; ++e) b = e == 0 ? ST[(u >> 2) % NF][0] : __builtin_fmaxf(b, ST[(u >> 2) % NF][e]);
         asm volatile("" : "+v"(b));
       }
-      if (NF == 4 && (u % 3) == 2) stage_piece(buf, u / 3);
-      if (NF == 2) stage_piece(buf, u);
+      if (NF == 4 && (u % 3) == 2 && u / 3 >= PIECE0) stage_piece(buf, u / 3);
+      if (NF == 2 && u >= PIECE0) stage_piece(buf, u);
       __builtin_amdgcn_sched_barrier(0);
     }
-    fetch_k(i + 3);
-    fetch_v(i + 1);
+    if constexpr (TILES == 0) fetch_k(i + 3);
+    if constexpr (!LAST) fetch_v(i + 1);
     float mx;
     if constexpr (SPLIT == 1) {
       mx = mha_halves_max(__builtin_fmaxf(__builtin_fmaxf(bmax[0], bmax[1 % NF]), __builtin_fmaxf(bmax[2 % NF], bmax[3 % NF])));
@@ -451,11 +470,13 @@ __device__ __forceinline__ void mha_nvfp4_block(const MhaArgs &a, const MhaTile 
     for (int st = 0; st < 8 * NF + 8; ++st) {
       if (st < 8) {
         const int u = PVA + st;
-        OT[u & 3] = __builtin_amdgcn_mfma_f32_32x32x16_f16(VF[u % RING], PF, OT[u & 3], 0, 0, 0);
-        if (st + RING < 8) VF[u % RING] = v_operand(buf ^ 1, u + RING);
-        else KF[st % RING] = k_operand(buf ^ 1, st + RING - 8);
-        if (st == 3) PF = p_operand(2 * NF - 1);
-      } else {
+        if constexpr (!FIRST) {
+          OT[u & 3] = __builtin_amdgcn_mfma_f32_32x32x16_f16(VF[u % RING], PF, OT[u & 3], 0, 0, 0);
+          if (st + RING < 8) VF[u % RING] = v_operand(buf ^ 1, u + RING);
+          if (st == 3) PF = p_operand(2 * NF - 1);
+        }
+        if (!LAST && st + RING >= 8) KF[st % RING] = k_operand(buf ^ 1, st + RING - 8);
+      } else if constexpr (!LAST) {
         const int t = st - 8;
         ST[t >> 3] = __builtin_amdgcn_mfma_f32_32x32x16_f16(KF[t % RING], QF[(t >> 2) & 1][t & 3], (t & 7) == 0 ? (f32x16)(0.0f) : ST[t >> 3], 0, 0, 0);
         if (t + RING < 8 * NF) KF[t % RING] = k_operand(buf ^ 1, t + RING);
@@ -481,10 +502,17 @@ __device__ __forceinline__ void mha_nvfp4_block(const MhaArgs &a, const MhaTile 
 #pragma unroll
     for (int f = 0; f < NF; ++f) pcode[f] = code[f];
     l_run = __builtin_fmaf(l_run, alpha, mha_halves_sum(lsum));
-    if constexpr (SPLIT > 1) part_maximum(buf ^ 1);
+    if constexpr (SPLIT > 1 && !LAST) part_maximum(buf ^ 1);
     __syncthreads();
   };
-  for (int i = 0; i < ntiles; ++i) tile_step(i);
+  if constexpr (TILES == 0) {
+    for (int i = 0; i < ntiles; ++i) tile_step(std::false_type{}, std::false_type{}, i);
+  } else if constexpr (TILES == 1) {
+    tile_step(std::true_type{}, std::true_type{}, 0);
+  } else {
+    tile_step(std::true_type{}, std::false_type{}, 0);
+    tile_step(std::false_type{}, std::true_type{}, 1);
+  }
   rescale();
 #pragma unroll
   for (int u = 0; u < 8 * NF; ++u)
@@ -511,10 +539,10 @@ __device__ __forceinline__ void mha_nvfp4_block(const MhaArgs &a, const MhaTile 
 }
 
 // (two bodies in one kernel, so that the workgroups of the last round start as the ones in front of them end)
-template <int TAIL>
+template <int TAIL, int TILES>
 __global__ __launch_bounds__(512, 1) void mha_nvfp4_fwd_kernel(MhaArgs a, MhaWork w) {
-  if (TAIL == 1 || blockIdx.x < w.full) mha_nvfp4_block<1>(a, mha_tile(w, a.H, 1, w.blocks));
-  else mha_nvfp4_block<TAIL>(a, mha_tile(w, a.H, TAIL, w.cut));
+  if (TAIL == 1 || blockIdx.x < w.full) mha_nvfp4_block<1, TILES>(a, mha_tile(w, a.H, 1, w.blocks));
+  else mha_nvfp4_block<TAIL, TILES>(a, mha_tile(w, a.H, TAIL, w.cut));
 }
 
 // ---------------------------------------------------------------------------------------------------------------
@@ -575,7 +603,9 @@ constexpr float MHA8_EXP_OFFSET = 7.5f;
 // rate: 73 % of the cycles) and, where the whole GPU is busy for long, by power: the clock falls to 2.0 - 2.15 GHz.
 // Kernel alone, before (128 or 256 rows, no split, no pipeline) and now: 16384 x 40 x 128 3447 -> 3314 us (1659 TFLOP/s),
 // 4096 x 40 264 -> 249, 8192 x 4 118 -> 103, 3000 x 24 143 -> 110, 512 x 2 on 8192 keys 114 -> 71, 75600 x 1 3007 -> 2071.
-template <int SPLIT>
+// TILES as above: 8192 heads of 49 x 49, D = 32, 209 / 179 / 144 us; 1024 heads of 256 x 256, D = 64, 42 / 44 / 41.5; 40 heads
+// of 16384 x 200 133 / 122 / 114.
+template <int SPLIT, int TILES>
 __device__ __forceinline__ void mha_int8_x_fp8_block(const Mha8Args &a, const MhaTile &wg) {
   constexpr int NF = 4 / SPLIT;             // 32-row fragments of a tile per wave
   constexpr int NPV = SPLIT == 1 ? 2 : 1;   // P.V operands of 64 kv positions per wave (SPLIT 4: half of one, zeros behind)
@@ -632,7 +662,8 @@ __device__ __forceinline__ void mha_int8_x_fp8_block(const Mha8Args &a, const Mh
 
   Piece vp;
   fetch_k(0, 0);
-  fetch_k(1, 1);
+  if constexpr (TILES == 1) fetch_v(0, vp);
+  else fetch_k(1, 1);
   // Q of the lane's row: the 16 bytes [32 s + 16 h, +16) of k-step s, kept for the whole kernel
   i32x4 QF[4];
 #pragma unroll
@@ -654,10 +685,10 @@ __device__ __forceinline__ void mha_int8_x_fp8_block(const Mha8Args &a, const Mh
   f32x16 OT[4];  // O^T: d = 32 fd + 8 (e >> 2) + 4 h + (e & 3), for the lane's query row
 #pragma unroll
   for (int fd = 0; fd < 4; ++fd) OT[fd] = (f32x16)(0.0f);
-  i32x8 P[NPV];  // P of a tile as e4m3, MFMA operands of 64 kv positions
+  i32x8 P[NPV];  // P of a tile as e4m3, MFMA operands of 64 kv positions (SPLIT 4: 32, and zeros)
 #pragma unroll
   for (int j = 0; j < NPV; ++j) P[j] = (i32x8)(0);
-  {  // V of the tile in front of the first one: zeros, and so is its P
+  if constexpr (TILES == 0) {  // V of the tile in front of the first one: zeros, and so is its P
     Piece z;
     z.lo = z.hi = make_uint4(0, 0, 0, 0);
     stage_v(1, z);
@@ -721,30 +752,35 @@ __device__ __forceinline__ void mha_int8_x_fp8_block(const Mha8Args &a, const Mh
   __syncthreads();
 
   // One kv tile i.  TAIL: the last, partial one, where P of the positions past Nkv is zero.
-  auto tile_step = [&](auto negative_tag, auto tail_tag, int i) {
+  auto tile_step = [&](auto negative_tag, auto tail_tag, auto first_tag, auto last_tag, int i) {
+    constexpr bool FIRST = decltype(first_tag)::value, LAST = decltype(last_tag)::value;  // no tile in front of / behind this one
     constexpr bool NEG = decltype(negative_tag)::value, TAIL = decltype(tail_tag)::value;
     const int buf = i & 1;
     float qk = qs * ksf_next;
     // (here, not behind the loads below: the compiler does not count the transfers of K, and its wait for a load in front of
     // them would be a wait for them too)
     asm volatile("" : "+v"(qk));
-    ksf_next = ksf_src[i + 1 < ntiles ? i + 1 : i];
+    if constexpr (!LAST) ksf_next = ksf_src[i + 1 < ntiles ? i + 1 : i];
     asm volatile("" ::: "memory");
-    fetch_k(i + 2, buf);
-    fetch_v(i, vp);
-    rescale();
+    if constexpr (TILES == 0) fetch_k(i + 2, buf);
+    if constexpr (TILES != 1) fetch_v(i, vp);
+    if constexpr (!FIRST) rescale();
     // ---- maxima.  The maximum of s = float(S) * qk is taken over the integers S (the conversion keeps their order):
     // qk >= 0 keeps it too, qk < 0 reverses it.  SPLIT 1: under them the first half of O of the tile before.
     i32x8 VF[2];
-    VF[0] = v_operand(buf ^ 1, 0);
-    VF[1] = v_operand(buf ^ 1, 1);
+    if constexpr (!FIRST) {
+      VF[0] = v_operand(buf ^ 1, 0);
+      VF[1] = v_operand(buf ^ 1, 1);
+    }
     int hi = SI[0][0], lo = SI[0][0];
     if constexpr (SPLIT == 1) {
       __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
       for (int st = 0; st < 4; ++st) {
-        OT[st] = pv_mfma(VF[st & 1], P[0], OT[st]);
-        VF[st & 1] = v_operand(buf ^ 1, st + 2);
+        if constexpr (!FIRST) {
+          OT[st] = pv_mfma(VF[st & 1], P[0], OT[st]);
+          VF[st & 1] = v_operand(buf ^ 1, st + 2);
+        }
 #pragma unroll
         for (int e = 0; e < 16; ++e) {
           hi = SI[st][e] > hi ? SI[st][e] : hi;
@@ -785,10 +821,12 @@ __device__ __forceinline__ void mha_int8_x_fp8_block(const Mha8Args &a, const Mh
 #pragma unroll
     for (int st = 0; st < 4 * NF + 4; ++st) {  // step st: P of the st-th group of four scores; an O part or S part st - 4
       if (st < 4) {
-        OT[st] = pv_mfma(VF[st & 1], P[NPV - 1], OT[st]);
-        if (st < 2) VF[st & 1] = v_operand(buf ^ 1, (NPV - 1) * 4 + st + 2);
-        else KF[st & 1] = k_operand(kb, st - 2);
-      } else {
+        if constexpr (!FIRST) {
+          OT[st] = pv_mfma(VF[st & 1], P[NPV - 1], OT[st]);
+          if (st < 2) VF[st & 1] = v_operand(buf ^ 1, (NPV - 1) * 4 + st + 2);
+        }
+        if (!LAST && st >= 2) KF[st & 1] = k_operand(kb, st - 2);
+      } else if constexpr (!LAST) {
         const int t = st - 4, f = t >> 2, s4 = t & 3;
         SI[f] = __builtin_amdgcn_mfma_i32_32x32x32_i8(KF[t & 1], QF[s4], s4 == 0 ? (i32x16)(0) : SI[f], 0, 0, 0);
         if (t + 2 < 4 * NF) KF[t & 1] = k_operand(kb, t + 2);
@@ -822,19 +860,29 @@ __device__ __forceinline__ void mha_int8_x_fp8_block(const Mha8Args &a, const Mh
 #pragma unroll
     for (int j = 0; j < NPV; ++j) P[j] = PN[j];
     l_run = __builtin_fmaf(l_run, alpha, mha_halves_sum(lsum));
-    if constexpr (SPLIT > 1) part_extremum(negative_tag, buf ^ 1);
+    if constexpr (SPLIT > 1 && !LAST) part_extremum(negative_tag, buf ^ 1);
     stage_v(buf, vp);
     wait_vmcnt<0>();  // the transfers of K
     __syncthreads();
   };
+  using No = std::false_type;
+  using Yes = std::true_type;
   auto all_tiles = [&](auto negative_tag) {
     int i = 0;
-    for (; i < (int)(a.Nkv / 128); ++i) tile_step(negative_tag, std::false_type{}, i);
-    if (i < ntiles) tile_step(negative_tag, std::true_type{}, i);
+    for (; i < (int)(a.Nkv / 128); ++i) tile_step(negative_tag, No{}, No{}, No{}, i);
+    if (i < ntiles) tile_step(negative_tag, Yes{}, No{}, No{}, i);
   };
   // (the probability keeps the registers of the loop that runs)
-  if (__builtin_expect_with_probability(negative, 0, 0.99999)) all_tiles(std::true_type{});
-  else all_tiles(std::false_type{});
+  if constexpr (TILES == 1) {  // (a code for both signs and both ends)
+    tile_step(Yes{}, Yes{}, Yes{}, Yes{}, 0);
+  } else if constexpr (TILES == 2) {
+    tile_step(Yes{}, No{}, Yes{}, No{}, 0);
+    tile_step(Yes{}, Yes{}, No{}, Yes{}, 1);
+  } else if (__builtin_expect_with_probability(negative, 0, 0.99999)) {
+    all_tiles(Yes{});
+  } else {
+    all_tiles(No{});
+  }
   rescale();
 #pragma unroll
   for (int st = 0; st < 4 * NPV; ++st) OT[st & 3] = pv_mfma(v_operand((ntiles - 1) & 1, st), P[st >> 2], OT[st & 3]);
@@ -865,10 +913,10 @@ __device__ __forceinline__ void mha_int8_x_fp8_block(const Mha8Args &a, const Mh
 }
 
 // (two bodies in one kernel, so that the workgroups of the last round start as the ones in front of them end)
-template <int TAIL>
+template <int TAIL, int TILES>
 __global__ __launch_bounds__(512, 1) void mha_int8_x_fp8_fwd_kernel(Mha8Args a, MhaWork w) {
-  if (TAIL == 1 || blockIdx.x < w.full) mha_int8_x_fp8_block<1>(a, mha_tile(w, a.H, 1, w.blocks));
-  else mha_int8_x_fp8_block<TAIL>(a, mha_tile(w, a.H, TAIL, w.cut));
+  if (TAIL == 1 || blockIdx.x < w.full) mha_int8_x_fp8_block<1, TILES>(a, mha_tile(w, a.H, 1, w.blocks));
+  else mha_int8_x_fp8_block<TAIL, TILES>(a, mha_tile(w, a.H, TAIL, w.cut));
 }
 
 // Per-token-block int8 quantizer in front of it (python/ac4k_kernel/ops/attention.py:18-99, a Triton kernel in the
@@ -928,17 +976,22 @@ __global__ __launch_bounds__(256) void quantize_int8_token_block_kernel(int8_t *
   }
 }
 
-// one kernel per cut of the last round (1, 2, 4)
-static void (*const mha_nvfp4_kernels[3])(MhaArgs, MhaWork) = {mha_nvfp4_fwd_kernel<1>, mha_nvfp4_fwd_kernel<2>, mha_nvfp4_fwd_kernel<4>};
-static void (*const mha_int8_x_fp8_kernels[3])(Mha8Args, MhaWork) = {mha_int8_x_fp8_fwd_kernel<1>, mha_int8_x_fp8_fwd_kernel<2>,
-                                                                     mha_int8_x_fp8_fwd_kernel<4>};
+// one kernel per number of tiles (any, 1, 2) and cut (1, 2, 4)
+static void (*const mha_nvfp4_kernels[3][3])(MhaArgs, MhaWork) = {
+    {mha_nvfp4_fwd_kernel<1, 0>, mha_nvfp4_fwd_kernel<2, 0>, mha_nvfp4_fwd_kernel<4, 0>},
+    {mha_nvfp4_fwd_kernel<1, 1>, mha_nvfp4_fwd_kernel<2, 1>, mha_nvfp4_fwd_kernel<4, 1>},
+    {mha_nvfp4_fwd_kernel<1, 2>, mha_nvfp4_fwd_kernel<2, 2>, mha_nvfp4_fwd_kernel<4, 2>}};
+static void (*const mha_int8_x_fp8_kernels[3][3])(Mha8Args, MhaWork) = {
+    {mha_int8_x_fp8_fwd_kernel<1, 0>, mha_int8_x_fp8_fwd_kernel<2, 0>, mha_int8_x_fp8_fwd_kernel<4, 0>},
+    {mha_int8_x_fp8_fwd_kernel<1, 1>, mha_int8_x_fp8_fwd_kernel<2, 1>, mha_int8_x_fp8_fwd_kernel<4, 1>},
+    {mha_int8_x_fp8_fwd_kernel<1, 2>, mha_int8_x_fp8_fwd_kernel<2, 2>, mha_int8_x_fp8_fwd_kernel<4, 2>}};
 
 // A launch carries fewer than 2^32 threads along a grid dim: from 2^31 on the heads go out in several launches, each planned
 // by itself.
 constexpr int64_t MHA_MAX_BLOCKS = 1 << 22;
 
 template <typename Args>
-static int mha_launch(const Args &a, int64_t heads, int64_t Nq, int64_t ntiles, const MhaCost &cost, void (*const (&kernels)[3])(Args, MhaWork),
+static int mha_launch(const Args &a, int64_t heads, int64_t Nq, int64_t ntiles, const MhaCost &cost, void (*const (&kernels)[3][3])(Args, MhaWork),
                       int (*lds_bytes)(int), hipStream_t st, const char *what) {
   const int64_t blocks = ceil_div(Nq, 256), most = blocks < MHA_MAX_BLOCKS ? MHA_MAX_BLOCKS / blocks : 1;
   for (int64_t head0 = 0; head0 < heads; head0 += most) {
@@ -946,17 +999,18 @@ static int mha_launch(const Args &a, int64_t heads, int64_t Nq, int64_t ntiles, 
     unsigned grid = 0;
     MhaWork work = mha_plan(cost, heads - head0 < most ? heads - head0 : most, Nq, ntiles, &tail, &grid);
     work.head0 = (uint32_t)head0;
-    auto kern = kernels[tail >> 1];
+    const int tiles = ntiles <= 2 ? (int)ntiles : 0;
+    auto kern = kernels[tiles][tail >> 1];
     const int lds = lds_bytes(tail);
     // more than 64 KB of dynamic LDS has to be allowed once per device and kernel
-    static std::atomic<uint32_t> lds_done[3] = {{0}, {0}, {0}};
+    static std::atomic<uint32_t> lds_done[3][3];
     int dev = 0;
     if (hipGetDevice(&dev) != hipSuccess) dev = 0;
     const uint32_t bit = 1u << (dev & 31);
-    if (!(lds_done[tail >> 1].load(std::memory_order_relaxed) & bit)) {
+    if (!(lds_done[tiles][tail >> 1].load(std::memory_order_relaxed) & bit)) {
       hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, lds);
       if (e != hipSuccess) return set_error("hipFuncSetAttribute(LDS=%d): %s", lds, hipGetErrorString(e));
-      lds_done[tail >> 1].fetch_or(bit, std::memory_order_relaxed);
+      lds_done[tiles][tail >> 1].fetch_or(bit, std::memory_order_relaxed);
     }
     hipLaunchKernelGGL(kern, dim3(grid), dim3(512), lds, st, a, work);
   }
@@ -1018,9 +1072,9 @@ extern "C" __attribute__((visibility("default"))) int ac4k_mha_int8_x_fp8_fwd(
              q_sf, k_sf, v_sf, H, Nq, Nkv, align_up(Nkv, 16), ceil_div(Nq, q_quantize_block_size), ceil_div(Nkv, 128),
              (int)Dqk, (int)Dv, (int)align_up(Dv, 16), q_quantize_block_size, sm_scale,
              (o_d_stride == 1 && Dv % 8 == 0 && ((uintptr_t)O & 15) == 0 && o_b_stride % 8 == 0 && o_h_stride % 8 == 0 && o_n_stride % 8 == 0) ? 1 : 0};
-  // measured: 512 x 2 x 128 to 8192 x 4 x 128 on 4096 and 8192 keys, one round
-  static constexpr MhaCost cost{{4.5f, 6.0f, 5.0f}, {2.35f, 1.45f, 1.05f}};
-  return mha_launch(a, B * H, Nq, ceil_div(Nkv, 128), cost, mha_int8_x_fp8_kernels, mha8_lds_bytes, (hipStream_t)stream, "ac4k_mha_int8_x_fp8_fwd");
+  // measured: 512 x 2 x 128 to 8192 x 4 x 128 on 4096 and 8192 keys, one round; one tile: 8192 heads of 49 to 128 rows
+  static constexpr MhaCost cost{{4.5f, 6.0f, 5.0f}, {2.35f, 1.45f, 1.05f}}, one{{6.9f, 6.5f, 4.6f}, {0.0f, 0.0f, 0.0f}};
+  return mha_launch(a, B * H, Nq, ceil_div(Nkv, 128), Nkv <= 128 ? one : cost, mha_int8_x_fp8_kernels, mha8_lds_bytes, (hipStream_t)stream, "ac4k_mha_int8_x_fp8_fwd");
 }
 
 // Replaces _int8_quantize / _triton_block_token_quantize (python/ac4k_kernel/ops/attention.py:18-99): x bf16 with element

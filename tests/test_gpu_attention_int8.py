@@ -124,7 +124,9 @@ def test_whole_call_equals_operator_by_operator(B, Nq, Nkv, H, D, layout, monkey
 # turn the order of the scores around.
 @pytest.mark.parametrize("H,Nq,Nkv", [(1, 50, 20), (2, 300, 129), (3, 129, 1030), (40, 513, 256), (130, 300, 200), (190, 260, 300),
                                       # more than a round of blocks, most of whose rows do not exist: all of them cut in four or in two
-                                      (300, 49, 49), (300, 40, 600), (512, 100, 300), (24, 2637, 1100)])
+                                      (300, 49, 49), (300, 40, 600), (512, 100, 300), (24, 2637, 1100),
+                                      # one and two kv tiles in workgroups of 256 and 128 rows and with a cut rest
+                                      (256, 200, 128), (512, 100, 77), (260, 256, 100), (256, 256, 256), (512, 100, 190), (300, 256, 129)])
 @pytest.mark.parametrize("signs", [False, True])
 def test_split_plans_and_negative_scales(H, Nq, Nkv, signs):
     g = torch.Generator().manual_seed(H + Nq)
