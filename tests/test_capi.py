@@ -159,3 +159,24 @@ def test_linear_workspace_is_checked(m, n, k):
     call = lambda ws, size: lib.ac4k_linear_nvfp4_workspace(p, 0, p, p, p, p, p, p, None, 0, m, n, k, ws, size, None)  # noqa: E731
     for ws, size, text in ((p, need - 1, b"too small"), (None, need, b"256-byte aligned"), (ctypes.c_void_p(272), need, b"256-byte aligned")):
         assert call(ws, size) != 0 and text in lib.ac4k_last_error()
+
+
+def test_attention_operands_and_workspace_are_checked():
+    """Dense [1, 2, 64, 64] operands, in either layout, and what the whole calls refuse about them."""
+    from ac4k_kernel_amd import _lib
+    lib, p = _lib.load(), ctypes.c_void_p(256)  # never dereferenced
+    size = (1, 2, 64, 64, 64, 64)
+    for entry, bytes_, scale in ((lib.ac4k_attention_int8_x_fp8_bf16, lib.ac4k_attention_int8_x_fp8_workspace_bytes, 2.25),
+                                 (lib.ac4k_attention_nvfp4_bf16, lib.ac4k_attention_nvfp4_workspace_bytes, 2688.0)):
+        need, dense = bytes_(*size), (8192, 4096, 64)
+
+        def call(q=dense, k=dense, v=dense, ptr=p, size=size, ws=p, ws_bytes=need):
+            return entry(p, 8192, 4096, 64, 1, ptr, *q, p, *k, p, *v, *size, scale, 0.125, ws, ws_bytes, None)
+
+        for kw, text in (({"ws_bytes": need - 1}, b"too small"), ({"ws": ctypes.c_void_p(264)}, b"16-byte aligned"), ({"ptr": None}, b"null"),
+                         ({"ptr": ctypes.c_void_p(257)}, b"2-byte aligned"), ({"k": (8192, -64, 64)}, b"negative"),
+                         ({"size": (1, 2, 64, 64, 64, 136)}, b"8 to 128"), ({"size": (1, 2, 0, 64, 64, 64)}, b"positive")):
+            assert call(**kw) != 0 and text in lib.ac4k_last_error(), (kw, lib.ac4k_last_error())
+        assert bytes_(1, 2, 64, 64, 7, 64) == -1 and bytes_(1, 2, 64, 64, 64, 129) == -1 and bytes_(0, 2, 64, 64, 64, 64) == -1
+    for gap in ((8192, 4096, 65), (8192, 4097, 64)):  # the NVFP4 maxima are taken over whole tensors
+        assert call(k=gap) != 0 and b"dense" in lib.ac4k_last_error()

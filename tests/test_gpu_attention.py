@@ -141,6 +141,61 @@ def test_whole_call_equals_operator_by_operator(B, Nq, Nkv, H, D, layout, monkey
     assert torch.equal(got, ops().attention(q, k, v, layout=layout, precision="nvfp4"))
 
 
+@pytest.mark.parametrize("H,N", LARGE)
+def test_negative_scale(H, N):
+    """A negative product of the scales goes into Q; workgroups of 256, 128 and 64 query rows."""
+    q, k, v = (make_input((1, H, N, 128), seed=s).cuda() for s in (56, 57, 58))
+    o = ops()
+    qq, kq, vq = o.quantize(q, 2, 3), o.quantize(k, 2, 3), o.quantize(v, 3, 2, swizzle=True)
+    out = torch.empty((1, H, N, 128), dtype=torch.bfloat16, device="cuda")
+    o.mha_nvfp4_fwd(out, *qq, *kq, *vq, -0.088)
+    cpu = lambda t3: (t3[0].cpu(), t3[1].cpu().view(torch.uint8), t3[2].cpu())  # noqa: E731
+    ref = A.mha_nvfp4_fwd(*cpu(qq), *cpu(kq), *cpu(vq), -0.088)
+    torch.testing.assert_close(out.cpu().float(), ref.float(), atol=ATOL, rtol=RTOL)
+
+
+def test_whole_call_on_infinite_and_nan_operands(monkeypatch):
+    """Through one C call the same as operator by operator: NaN where that gives NaN, the same values elsewhere."""
+    from ac4k_kernel_amd import _rocm_ops
+    base = [make_input((1, 3, 150, 64), seed=s).cuda() for s in (1, 2, 3)]
+    cases = [(t, x) for t in range(3) for x in (float("inf"), -float("inf"), float("nan"))]
+    got = []
+    for whole in (True, False):
+        if not whole:
+            monkeypatch.setattr(_rocm_ops, "attention_nvfp4", lambda *a: False)
+        for n, (t, x) in enumerate(cases):
+            qkv = [b.clone() for b in base]
+            qkv[t][0, 1, 77, 5] = x
+            o = ops().attention(*qkv, layout="BHND", precision="nvfp4")
+            if whole:
+                got.append(o)
+            else:
+                assert torch.allclose(o, got[n], rtol=0, atol=0, equal_nan=True), (t, x)
+
+
+@pytest.mark.parametrize("precision", ["nvfp4", "int8+fp8e4m3"])
+def test_head_dims_below_eight_go_operator_by_operator(precision):
+    from ac4k_kernel_amd import _lib
+    q, k, v = (make_input((1, 40, 2, 7), seed=s) for s in (1, 2, 3))
+    lib = _lib.load()
+    f = lib.ac4k_attention_nvfp4_workspace_bytes if precision == "nvfp4" else lib.ac4k_attention_int8_x_fp8_workspace_bytes
+    assert f(1, 2, 40, 40, 7, 7) == -1
+    o = ops().attention(q.cuda(), k.cuda(), v.cuda(), layout="BNHD", precision=precision)
+    ref = A.attention_nvfp4(q, k, v) if precision == "nvfp4" else A.attention_int8_x_fp8(q, k, v)
+    torch.testing.assert_close(o.cpu().float(), ref.float(), atol=ATOL, rtol=RTOL)
+
+
+@pytest.mark.parametrize("layout", ["BNHD", "BHND"])
+@pytest.mark.parametrize("Dqk,Dv", [(128, 64), (64, 128), (40, 100), (100, 8)])
+def test_whole_call_with_another_head_dim_of_v(Dqk, Dv, layout, monkeypatch):
+    from ac4k_kernel_amd import _rocm_ops
+    shape = lambda n, d: (2, n, 5, d) if layout == "BNHD" else (2, 5, n, d)  # noqa: E731
+    q, k, v = make_input(shape(70, Dqk), seed=1).cuda(), make_input(shape(200, Dqk), seed=2).cuda(), make_input(shape(200, Dv), seed=3).cuda()
+    got = ops().attention(q, k, v, layout=layout, precision="nvfp4")
+    monkeypatch.setattr(_rocm_ops, "attention_nvfp4", lambda *a: False)
+    assert got.shape == shape(70, Dv) and torch.equal(got, ops().attention(q, k, v, layout=layout, precision="nvfp4"))
+
+
 def test_more_heads_than_one_launch_carries():
     """2^23 workgroups of 512 threads are 2^32 threads: with so many heads (one query, one key each) both forwards and both
     whole calls still give what they give for a part of the batches."""

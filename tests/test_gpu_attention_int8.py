@@ -117,6 +117,79 @@ def test_whole_call_equals_operator_by_operator(B, Nq, Nkv, H, D, layout, monkey
     want = ops().attention(q, k, v, layout=layout)
     assert (got == want).float().mean().item() > 0.9
     torch.testing.assert_close(got.float(), want.float(), atol=ATOL, rtol=RTOL)
+    # one step of int8 in a channel moves a score by |q| max|k| / 127 / sqrt(D), at most 2 % of a p, whatever the size of the outputs
+    dims = (1, 3) if layout == "BNHD" else (2, 3)
+    assert ((got.float() - want.float()).norm(dim=dims) / want.float().norm(dim=dims)).max().item() < 0.02
+
+
+def exact_mean_keys(shape, n_dim, seed):
+    """Keys whose token mean is 1.5 in every channel and every order of summation: multiples of 1/16, in pairs around it."""
+    n = shape[n_dim]
+    k = torch.full(shape, 1.5)
+    r = (make_input(shape, seed=seed).float().clamp(-4, 4) * 16).round() / 16
+    half = r.narrow(n_dim, 0, n // 2)
+    k.narrow(n_dim, 0, n // 2).add_(half)
+    k.narrow(n_dim, n // 2, n // 2).sub_(half)
+    return k.to(torch.bfloat16).cuda()
+
+
+@pytest.mark.parametrize("B,Nq,Nkv,H,Dqk,Dv,layout", [(1, 1, 1, 1, 8, 8, "BNHD"), (3, 33, 31, 7, 71, 71, "BNHD"), (2, 65, 257, 12, 64, 64, "BHND"),
+                                                      (1, 200, 2100, 9, 128, 128, "BNHD"), (2, 64, 9000, 3, 100, 100, "BHND"),
+                                                      (80, 20, 49, 8, 40, 40, "BHND"), (2, 70, 200, 5, 128, 64, "BNHD"),
+                                                      (2, 70, 200, 5, 64, 128, "BHND"), (2, 70, 200, 5, 40, 100, "BNHD"), (1, 70, 300, 9, 100, 8, "BHND")])
+def test_whole_call_with_exact_means_is_bit_identical(B, Nq, Nkv, H, Dqk, Dv, layout, monkeypatch):
+    shape = lambda n, d: (B, n, H, d) if layout == "BNHD" else (B, H, n, d)  # noqa: E731
+    q, v = make_input(shape(Nq, Dqk), seed=1).cuda(), make_input(shape(Nkv, Dv), seed=3).cuda()
+    k = exact_mean_keys(shape(Nkv, Dqk), 1 if layout == "BNHD" else 2, 2)
+    got = ops().attention(q, k, v, layout=layout)
+    monkeypatch.setattr(binding(), "attention_int8_x_fp8", lambda *a: False)
+    want = ops().attention(q, k, v, layout=layout)
+    assert torch.equal(got, want) and torch.isfinite(got).all()
+
+
+@pytest.mark.parametrize("D", [64, 65, 128])
+def test_whole_call_takes_views(D):
+    """q and k as views of one buffer of q, k and v, k as a view of the other layout, tokens and heads shared by stride 0."""
+    B, N, H = 2, 150, 5
+    q, v = make_input((B, N, H, D), seed=1).cuda(), make_input((B, N, H, D), seed=3).cuda()
+    k = exact_mean_keys((B, N, H, D), 1, 2)
+    want = ops().attention(q, k, v)
+    calls = []
+    whole = binding().attention_int8_x_fp8
+    try:
+        binding().attention_int8_x_fp8 = lambda *a: calls.append(whole(*a)) or calls[-1]
+        fused = torch.stack((q, k, v), dim=2)  # [B, N, 3, H, D]
+        assert torch.equal(ops().attention(fused[:, :, 0], fused[:, :, 1], v), want)
+        other = k.transpose(1, 2).contiguous().transpose(1, 2)  # the tokens of a head adjacent
+        assert torch.equal(ops().attention(q, other, v), want)
+        assert torch.equal(ops().attention(q.transpose(1, 2), k.transpose(1, 2), v.transpose(1, 2).contiguous(), layout="BHND"), want.transpose(1, 2))
+        one_q, one_k = q[:, :, :1].expand(B, N, H, D), k[:, :, :1].expand(B, N, H, D)
+        assert torch.equal(ops().attention(one_q, one_k, v), ops().attention(one_q.contiguous(), one_k.contiguous(), v))
+        assert calls == [True] * 5
+    finally:
+        binding().attention_int8_x_fp8 = whole
+
+
+def test_whole_call_on_infinite_and_nan_operands(monkeypatch):
+    """Through one C call the same as operator by operator: NaN where that gives NaN, the same values elsewhere."""
+    B, N, H, D = 1, 150, 3, 64
+    base = [make_input((B, N, H, D), seed=1).cuda(), exact_mean_keys((B, N, H, D), 1, 2), make_input((B, N, H, D), seed=3).cuda()]
+    cases = [(t, x) for t in range(3) for x in (float("inf"), -float("inf"), float("nan"), 0.0)]
+    got = []
+    for whole in (True, False):
+        if not whole:
+            monkeypatch.setattr(binding(), "attention_int8_x_fp8", lambda *a: False)
+        for n, (t, x) in enumerate(cases):
+            qkv = [b.clone() for b in base]
+            if x == 0.0:
+                qkv[t][0, :, 1, 5] = x  # a channel without a value
+            else:
+                qkv[t][0, 77, 1, 5] = x
+            o = ops().attention(*qkv)
+            if whole:
+                got.append(o)
+            else:
+                assert torch.allclose(o, got[n], rtol=0, atol=0, equal_nan=True), (t, x)
 
 
 # Launches whose last round is cut: workgroups of 256, 128 and 64 query rows (one round; 256 of 256 rows and a rest of 4 and

@@ -93,7 +93,7 @@ def test_global_scale_writes_four_bytes():
     assert w.t.item() == (x.abs().max().float().cpu() / 2688.0).item()  # IEEE division, as on the CPU
 
 
-# (M, N, K, tile plan or None): generic kernel (K % 64 != 0), fp16-tile kernel (K % 128 == 64), packed-LDS kernel
+# (M, N, K, tile plan or None): generic kernel (K % 64 != 0), packed-LDS kernel (K % 128 == 64 among them)
 # with interior and edge tiles of every shape, row lengths that rule the 16-byte stores out, K ranges
 LINEAR_CASES = [
     (5, 33, 48, None), (130, 140, 48, None), (200, 300, 192, None), (300, 330, 256, None), (300, 333, 256, None),
@@ -219,3 +219,44 @@ def test_attention_stays_inside_its_output():
         torch.cuda.synchronize()
         assert w.intact() and same_bytes(w.t, ref)
         assert wy.intact() and ws.intact() and same_bytes(wy.t, q8) and same_bytes(ws.t, q_sf)
+
+
+@pytest.mark.parametrize("kind", [0, 2, 3])
+@pytest.mark.parametrize("m,n,k", [(5, 136, 320), (16, 130, 1216), (32, 520, 1344), (16, 4096, 14400), (100, 300, 1216), (128, 1024, 4160),
+                                   (300, 256, 4160), (64, 1000, 4096)])
+def test_linear_with_any_k_stays_inside_workspace_and_output(m, n, k, kind, linear_tuning):
+    from ac4k_kernel_amd import _lib
+    L = _lib.load()
+    if kind and m > 32:
+        pytest.skip("the kernel choice only exists for decode-sized shapes")
+    linear_tuning(decode_kernel=kind)
+    aq = ops().quantize(make_input((m, k), seed=m).cuda(), 0, 1)
+    bq = ops().quantize(make_input((n, k), seed=n, std=0.02).cuda(), 0, 1)
+    nbytes = L.ac4k_linear_nvfp4_workspace_bytes(m, n, k)
+    ref = ops().linear(*aq, *bq)
+    d, ws = Window((m, n), torch.bfloat16), Window((max(nbytes, 256),), torch.uint8)
+    _lib.check(L.ac4k_linear_nvfp4_workspace(d.t.data_ptr(), 0, aq[0].data_ptr(), aq[1].data_ptr(), aq[2].data_ptr(),
+                                             bq[0].data_ptr(), bq[1].data_ptr(), bq[2].data_ptr(), None, 0, m, n, k,
+                                             ws.t.data_ptr(), nbytes, torch.cuda.current_stream().cuda_stream))
+    torch.cuda.synchronize()
+    assert d.intact() and ws.intact()
+    assert same_bytes(d.t, ref)
+
+
+@pytest.mark.parametrize("precision", ["int8+fp8e4m3", "nvfp4"])
+@pytest.mark.parametrize("B,H,Nq,Nkv,D,Dv", [(1, 2, 33, 70, 128, 128), (2, 3, 130, 130, 65, 65), (1, 5, 260, 200, 100, 40), (2, 2, 5, 1030, 127, 8),
+                                             (80, 8, 20, 49, 40, 64), (1, 1, 1, 1, 8, 9)])
+def test_whole_attention_stays_inside_workspace_and_output(B, H, Nq, Nkv, D, Dv, precision):
+    import math
+    from ac4k_kernel_amd import _lib
+    L = _lib.load()
+    q, k, v = make_input((B, H, Nq, D), seed=3).cuda(), make_input((B, H, Nkv, D), seed=4).cuda(), make_input((B, H, Nkv, Dv), seed=5).cuda()
+    ref = ops().attention(q, k, v, layout="BHND", precision=precision)
+    entry, size, scale = ((L.ac4k_attention_nvfp4_bf16, L.ac4k_attention_nvfp4_workspace_bytes, 2688.0) if precision == "nvfp4" else
+                          (L.ac4k_attention_int8_x_fp8_bf16, L.ac4k_attention_int8_x_fp8_workspace_bytes, 2.25))
+    nbytes = size(B, H, Nq, Nkv, D, Dv)
+    o, ws = Window((B, H, Nq, Dv), torch.bfloat16), Window((nbytes,), torch.uint8)
+    _lib.check(entry(o.t.data_ptr(), *o.t.stride(), q.data_ptr(), *q.stride()[:3], k.data_ptr(), *k.stride()[:3], v.data_ptr(), *v.stride()[:3],
+                     B, H, Nq, Nkv, D, Dv, scale, 1 / math.sqrt(D), ws.t.data_ptr(), nbytes, torch.cuda.current_stream().cuda_stream))
+    torch.cuda.synchronize()
+    assert o.intact() and ws.intact() and same_bytes(o.t, ref)
