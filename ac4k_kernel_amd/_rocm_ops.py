@@ -251,7 +251,7 @@ def linear_nvfp4_fused(D, X, X_q, X_sf, X_global_scale, B, B_sf, B_global_scale,
     _check(B.dim() == 2 and B.size(0) == N and B.size(1) == K // 2, "weight must be [N, K/2]")
     _check_linear_operand(B, B_sf, B_global_scale, N, "b")
     bias_ptr, bias_tag = _bias_args(bias, N)
-    if K % 256 != 0:  # no weight-streaming kernel: the composition itself
+    if K % 256 != 0:  # the C entry point takes whole stages of the kernels it began with: the composition itself, same kernels
         quantize_nvfp4_with_global_scale(X_q, X_sf, X_global_scale, X, 0, 1, False, 2688.0)
         linear_nvfp4(D, X_q, X_sf, X_global_scale, B, B_sf, B_global_scale, bias)
         return

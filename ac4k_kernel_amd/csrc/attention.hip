@@ -227,9 +227,8 @@ static_assert(8 * 16384 <= MHA_STAT_LDS && 8 * MHA_OUT_LDS <= MHA_STAT_LDS, "the
 // and decodes K of tile i + 2 and V of tile i, which were fetched a step earlier, into LDS.
 // (The multiplier of a P block inside the exponent instead of 16 multiplications gains another 3 %, but moves values across
 // rounding boundaries of P.)
-// Bound by vector-instruction issue (70 % of the cycles, 550 instructions per tile and wave against 64 MFMAs, which hold the
-// matrix core for 50 %) and by power: 13 % fewer cycles than one tile after the other at a clock of 2.0 instead of 2.15
-// GHz.  Kernel alone, same box, before (128 or 256 rows, no pipeline, no split) and now: 16384 x 40 x 128 6042 -> 5410 us
+// Bound by vector-instruction issue - 551 instructions per tile and wave beside 64 MFMAs; at 8192 x 40 x 128 the counters show the
+// vector port busy for 73 % of a SIMD's time and the matrix core for 49 % - and by power: the clock is 1.9 GHz there.  Kernel alone, same box, before (128 or 256 rows, no pipeline, no split) and now: 16384 x 40 x 128 6042 -> 5410 us
 // (1016 TFLOP/s; 1085 on a cooler box), 4096 x 40 422 -> 370, 8192 x 4 194 -> 165, 3000 x 24 214 -> 162, 512 x 2 on 8192
 // keys 191 -> 107, 75600 x 1 5250 -> 3676.
 // TILES: 1 and 2 for calls of so many kv tiles, 0 for any number.  The step in front of the first tile and the one behind the
@@ -578,7 +577,7 @@ typedef int i32x4 __attribute__((ext_vector_type(4)));
 typedef int i32x8 __attribute__((ext_vector_type(8)));
 typedef int i32x16 __attribute__((ext_vector_type(16)));
 
-// LDS: K tiles j & 1 of 128 rows of 128 bytes, the 16-byte piece p of row n at p ^ (n & 7) (bank spread); behind them V
+// LDS: K tiles j & 1 of 128 rows of 128 bytes, the 16-byte piece p of row n at p ^ ((n >> 1) & 7) (bank spread); behind them V
 // tiles j & 1 of 128 d rows at a pitch of 144 bytes
 constexpr int MHA8_K_LDS = 128 * 128;
 constexpr int MHA8_PITCH = 144;
@@ -592,15 +591,18 @@ constexpr float MHA8_EXP_OFFSET = 7.5f;
 // Eight waves, two per SIMD; a wave owns 32 query rows and 1 / SPLIT of the kv positions of every tile: SPLIT waves
 // share a group of query rows, 256 / SPLIT rows per workgroup.  What a shared group needs per tile is the row maximum
 // over the whole tile, which goes through LDS with the barrier that ends the tile; the partial sums of O and of the row
-// meet at the end.  The maxima, and with them every rounding of P, are those of the unsplit tile.
+// meet at the end.  The maxima, and with them every rounding of P, are those of the unsplit tile; the sums of O and of the row
+// are added in another order, so equal rows of two launches, or of the cut and the uncut part of one, may differ by an fp32
+// rounding (outputs 2e-5 apart, relative).
 //
 // A tile step is a software pipeline over three tiles, written out in the order in which it issues (the compiler's
 // scheduler keeps an MFMA and the vector instructions that could run under it apart):
 //   O += Vhat . Phat of tile i - 1  |  maxima, exp2, e4m3 of tile i  |  S of tile i + 1, into the registers that the
 //   scores of tile i leave one 32-row fragment after the other
 // K arrives by LDS-DMA two tiles ahead, V through registers one tile ahead.
-// Bound by the issue of vector instructions (about 360 per tile and wave, 65 exp2 and 32 e4m3 conversions of them at half
-// rate: 73 % of the cycles) and, where the whole GPU is busy for long, by power: the clock falls to 2.0 - 2.15 GHz.
+// Bound by the issue of vector instructions (349 per tile and wave beside 24 MFMAs, 65 exp2 of them at a quarter of the rate; at
+// 8192 x 40 x 128 the vector port is busy for 78 % of a SIMD's time and the matrix core for 37 %) and, where the whole GPU is busy
+// for long, by power (2.05 GHz there).
 // Kernel alone, before (128 or 256 rows, no split, no pipeline) and now: 16384 x 40 x 128 3447 -> 3314 us (1659 TFLOP/s),
 // 4096 x 40 264 -> 249, 8192 x 4 118 -> 103, 3000 x 24 143 -> 110, 512 x 2 on 8192 keys 114 -> 71, 75600 x 1 3007 -> 2071.
 // TILES as above: 8192 heads of 49 x 49, D = 32, 209 / 179 / 144 us; 1024 heads of 256 x 256, D = 64, 42 / 44 / 41.5; 40 heads

@@ -7,8 +7,9 @@
 //   2. attn_quantize_int8_fp8_kernel  every workgroup adds up the partials of its own channels (a few KB from L2) and
 //                                   quantizes one tile of V, K or Q
 // Both are bound by HBM: 2 (K + V) bytes read in the first, 2 (Q + K + V) read and half of that written in the second.
-// MI355X, quantizers alone: B 1, N 16384, H 40, D 128 (BNHD) 350 -> 250 us = 83 (4.0 TB/s) + 167 (4.5 TB/s), bit-identical
-// operands; a whole attention of 777 queries on 257 keys, B 2, H 12, D 64: 64 -> 26 us, three launches instead of nine.
+// MI355X, quantizers alone: B 1, N 16384, H 40, D 128 (BNHD) 350 -> 250 us = 83 (4.0 TB/s) + 167 (4.5 TB/s); a whole
+// attention of 777 queries on 257 keys, B 2, H 12, D 64: 64 -> 22 us, three launches instead of nine.  The operands are those
+// of the separate calls bit for bit, except that a channel mean of K summed in another order may round to the other bf16.
 #include "attention_quantize.h"
 #include "quantize_nvfp4.h"
 
@@ -427,7 +428,8 @@ int64_t attn_nvfp4_layout(AttnNvfp4Args &a, void *ws) {
   a.Nkv64 = (int)align_up(a.Nkv, 64);
   a.nqt = (int)ceil_div(a.Nqp, 128), a.nkt = (int)ceil_div(a.Nkvp, 128), a.nvt = (int)ceil_div(a.Nkv64, 256);
   const int64_t n[3] = {BH * a.Nq * a.D, BH * a.Nkv * a.D, BH * a.Nkv * a.Dv};
-  for (int t = 0; t < 3; ++t) {  // 32 KB per workgroup and round of loads
+  // a part of 32 KB and more: half of what a workgroup has in flight (512 lanes, eight loads), so that smaller tensors spread wider
+  for (int t = 0; t < 3; ++t) {
     const int64_t parts = ceil_div(n[t], 512 * 8 * 4);
     a.nparts[t] = (int)(parts < 1 ? 1 : parts < AQ_MAX_PARTS ? parts : AQ_MAX_PARTS);
   }

@@ -149,7 +149,8 @@ int ac4k_linear_nvfp4_skinny(void *D, int d_dtype, const void *A, const void *A_
 
 /* ac4k_linear_nvfp4 with scratch: every shape that ac4k_linear_nvfp4 takes, split along K where that fills the GPU,
  * on the same kernels as ac4k_linear_nvfp4_skinny but for any K % 64 == 0.  `workspace` =
- * ac4k_linear_nvfp4_workspace_bytes(M,N,K) bytes, 256-byte aligned, contents irrelevant (NULL when that is 0). */
+ * ac4k_linear_nvfp4_workspace_bytes(M,N,K) bytes, 256-byte aligned, contents irrelevant (NULL when that is 0).  Operands
+ * that are not aligned to 16 bytes (scale tensors: 4) run without scratch, like shapes that need none. */
 int64_t ac4k_linear_nvfp4_workspace_bytes(int64_t M, int64_t N, int64_t K);
 int ac4k_linear_nvfp4_workspace(void *D, int d_dtype, const void *A, const void *A_sf, const float *A_gs,
                                 const void *B, const void *B_sf, const float *B_gs, const void *bias,
@@ -228,7 +229,9 @@ int ac4k_linear_nvfp4_fused_bf16(void *D, int d_dtype, const void *X, void *X_q,
  * O bf16 [B,H,Nq,Dv] addressed through its four element strides (the reference passes a permuted view).
  * The attention probabilities are re-quantized to NVFP4 per 16-block with the global scale 1/2688, as in
  * mha_nvfp4.cu:248-319.  Dqk = 2 * (packed row bytes) must be 64 or 128 (the quantizer pads packed rows to whole 64-chunks), Dv any
- * number up to 128. */
+ * number up to 128.  Every call gives the same bits again.  How a launch cuts its query rows follows from B * H, Nq and Nkv, and the
+ * cut decides the order of fp32 sums: equal rows of two launches, or of two heads of one, may differ by an fp32 rounding
+ * (2e-5 of the output, 2-norm).  The same holds for ac4k_mha_int8_x_fp8_fwd. */
 int ac4k_mha_nvfp4_fwd(void *O, int64_t o_b_stride, int64_t o_h_stride, int64_t o_n_stride,
                        int64_t o_d_stride, const void *q, const void *q_sf, const float *q_gs,
                        const void *k, const void *k_sf, const float *k_gs, const void *v,
