@@ -106,8 +106,10 @@ __device__ __forceinline__ void aq_column_stats(const AttnQuantArgs &a, const At
   }
 }
 
-__global__ __launch_bounds__(64 * AQ_STAT_WAVES) void attn_column_stats_kernel(AttnQuantArgs a) {
-  extern __shared__ uint32_t red[][64][8];  // one per wave
+// MOST: waves that the LDS of a workgroup holds
+template <int MOST>
+__global__ __launch_bounds__(64 * MOST) void attn_column_stats_kernel(AttnQuantArgs a) {
+  __shared__ uint32_t red[MOST][64][8];
   if (blockIdx.y == 0) aq_column_stats<false>(a, a.k, a.Nkv, a.D, a.Dp, a.ksum, red);
   else aq_column_stats<true>(a, a.v, a.Nkv, a.Dv, a.Dvp, a.vmax, red);
 }
@@ -418,7 +420,9 @@ void launch_attn_quant(const AttnQuantArgs &a, hipStream_t st) {
     const int rows = AQ_STAT_LOADS * aq_heads_per_wave(a.D > a.Dv ? a.D : a.Dv);
     for (waves = 1; waves * rows < a.span; waves *= 2) {}
   }
-  hipLaunchKernelGGL(attn_column_stats_kernel, dim3((unsigned)(uk > uv ? uk : uv), 2), dim3(64 * waves), waves * sizeof(uint32_t[64][8]), st, a);
+  // (less LDS, more workgroups; the LDS sized by the launch instead cost the kernel of long spans 0.1 us)
+  hipLaunchKernelGGL(waves <= 4 ? attn_column_stats_kernel<4> : attn_column_stats_kernel<AQ_STAT_WAVES>,
+                     dim3((unsigned)(uk > uv ? uk : uv), 2), dim3(64 * waves), 0, st, a);
   hipLaunchKernelGGL(attn_quantize_int8_fp8_kernel, dim3((unsigned)((int64_t)a.B * a.H * (a.nvb + a.nkb + a.nqb))), dim3(256), 0, st, a);
 }
 
