@@ -32,7 +32,8 @@ struct MhaArgs {
   int64_t o_b, o_h, o_n, o_d;  // element strides of O [B, H, Nq, 128]
   const uint8_t *q, *k, *v, *q_sf, *k_sf, *v_sf;
   const float *q_gs, *k_gs, *v_gs;
-  int64_t H, Nq, Nkv, Nqp, Nkvp, Nkv64;  // padded: rows of the Q / K scale planes (16), stored kv length of V (64)
+  uint32_t H, head0;                  // heads; first head of the launch, of those of all batches
+  int64_t Nq, Nkv, Nqp, Nkvp, Nkv64;  // padded: rows of the Q / K scale planes (16), stored kv length of V (64)
   int chunks, Dv, Dvp;                   // 64-chunks of a Q / K row (1 or 2), rows of V, rows of a V scale plane (16)
   float sm_scale;
   int o_vec;  // O rows are contiguous along d, 16-byte aligned, Dv % 8 == 0: rows leave as 16-byte pieces
@@ -45,7 +46,6 @@ constexpr float MHA_P_ALPHA = 2688.0f;  // 1 / (global scale of P)
 // each; what is behind them is cut into workgroups of 256 / tail rows.
 struct MhaWork {
   uint32_t full, blocks, cut;  // full: a multiple of the number of XCDs; blocks and cut workgroups per head
-  uint32_t head0;              // first head of the launch, of those of all batches
 };
 struct MhaTile {
   int64_t block, head, b;  // block: in units of the rows of this workgroup
@@ -53,13 +53,13 @@ struct MhaTile {
 // Workgroups are dealt to the eight XCDs in turn: a run of consecutive blocks of one head is given to one XCD, whose L2 then
 // fetches the K and V of that head once for all of them, instead of all eight XCDs fetching those of every head
 // (4096 x 40 x 128 int8 x fp8: 262 -> 260 us, 4096 x 8: 59.3 -> 58.3).
-__device__ __forceinline__ MhaTile mha_tile(const MhaWork &w, int64_t H, uint32_t tail, uint32_t per_head) {
+__device__ __forceinline__ MhaTile mha_tile(const MhaWork &w, uint32_t H, uint32_t head0, uint32_t tail, uint32_t per_head) {
   const uint32_t first = blockIdx.x < w.full ? 0 : w.full, L = blockIdx.x - first;
   const uint32_t T = blockIdx.x < w.full ? w.full : gridDim.x - w.full;
   const uint32_t xcd = L & 7, q = T >> 3, rem = T & 7;
   const uint32_t id = (xcd < rem ? xcd * (q + 1) : rem * (q + 1) + (xcd - rem) * q) + (L >> 3) + first * tail;
-  const uint32_t local = id / per_head, bh = local + w.head0;
-  return MhaTile{id - local * per_head, bh % (uint32_t)H, bh / (uint32_t)H};
+  const uint32_t local = id / per_head, bh = local + head0;
+  return MhaTile{id - local * per_head, bh % H, bh / H};
 }
 
 // Plan of a launch.  A workgroup that splits its tiles over 2 or 4 waves needs `tile_us` per kv tile and `fixed_us` for
@@ -74,7 +74,7 @@ static MhaWork mha_plan(const MhaCost &c, int64_t heads, int64_t Nq, int64_t nti
   const int64_t blocks = ceil_div(Nq, 256), T = heads * blocks, full = T / cus * cus, left = T - full;
   auto rounds_us = [&](int64_t wgs, int i) { return (float)ceil_div(wgs, cus) * (c.fixed_us[i] + (float)ntiles * c.tile_us[i]); };
   float best = 0.0f;
-  MhaWork work{0, (uint32_t)blocks, 0, 0};
+  MhaWork work{0, (uint32_t)blocks, 0};
   *grid = 0;
   auto offer = [&](float us, int64_t first, int64_t wgs, int64_t cut, int i) {
     if ((*grid && us >= best) || first + wgs >= (1ll << 23)) return;  // (2^23 workgroups of 512 threads: more than a launch carries)
@@ -540,8 +540,8 @@ __device__ __forceinline__ void mha_nvfp4_block(const MhaArgs &a, const MhaTile 
 // (two bodies in one kernel, so that the workgroups of the last round start as the ones in front of them end)
 template <int TAIL, int TILES>
 __global__ __launch_bounds__(512, 1) void mha_nvfp4_fwd_kernel(MhaArgs a, MhaWork w) {
-  if (TAIL == 1 || blockIdx.x < w.full) mha_nvfp4_block<1, TILES>(a, mha_tile(w, a.H, 1, w.blocks));
-  else mha_nvfp4_block<TAIL, TILES>(a, mha_tile(w, a.H, TAIL, w.cut));
+  if (TAIL == 1 || blockIdx.x < w.full) mha_nvfp4_block<1, TILES>(a, mha_tile(w, a.H, a.head0, 1, w.blocks));
+  else mha_nvfp4_block<TAIL, TILES>(a, mha_tile(w, a.H, a.head0, TAIL, w.cut));
 }
 
 // ---------------------------------------------------------------------------------------------------------------
@@ -566,7 +566,8 @@ struct Mha8Args {
   const int8_t *q, *k;
   const uint8_t *v;
   const float *q_sf, *k_sf, *v_sf;
-  int64_t H, Nq, Nkv, Nkv16, nqb, nkb;  // stored kv length of V (16), scales per head of Q and K
+  uint32_t H, head0;                 // heads; first head of the launch, of those of all batches
+  int64_t Nq, Nkv, Nkv16, nqb, nkb;  // stored kv length of V (16), scales per head of Q and K
   int Dp, Dv, Dvp;                      // bytes of a Q / K row (head dim padded to 16), rows of V, scales of V per head (16)
   int q_block;
   float sm_scale;
@@ -917,8 +918,8 @@ __device__ __forceinline__ void mha_int8_x_fp8_block(const Mha8Args &a, const Mh
 // (two bodies in one kernel, so that the workgroups of the last round start as the ones in front of them end)
 template <int TAIL, int TILES>
 __global__ __launch_bounds__(512, 1) void mha_int8_x_fp8_fwd_kernel(Mha8Args a, MhaWork w) {
-  if (TAIL == 1 || blockIdx.x < w.full) mha_int8_x_fp8_block<1, TILES>(a, mha_tile(w, a.H, 1, w.blocks));
-  else mha_int8_x_fp8_block<TAIL, TILES>(a, mha_tile(w, a.H, TAIL, w.cut));
+  if (TAIL == 1 || blockIdx.x < w.full) mha_int8_x_fp8_block<1, TILES>(a, mha_tile(w, a.H, a.head0, 1, w.blocks));
+  else mha_int8_x_fp8_block<TAIL, TILES>(a, mha_tile(w, a.H, a.head0, TAIL, w.cut));
 }
 
 // Per-token-block int8 quantizer in front of it (python/ac4k_kernel/ops/attention.py:18-99, a Triton kernel in the
@@ -993,14 +994,14 @@ static void (*const mha_int8_x_fp8_kernels[3][3])(Mha8Args, MhaWork) = {
 constexpr int64_t MHA_MAX_BLOCKS = 1 << 22;
 
 template <typename Args>
-static int mha_launch(const Args &a, int64_t heads, int64_t Nq, int64_t ntiles, const MhaCost &cost, void (*const (&kernels)[3][3])(Args, MhaWork),
+static int mha_launch(Args a, int64_t heads, int64_t Nq, int64_t ntiles, const MhaCost &cost, void (*const (&kernels)[3][3])(Args, MhaWork),
                       int (*lds_bytes)(int), hipStream_t st, const char *what) {
   const int64_t blocks = ceil_div(Nq, 256), most = blocks < MHA_MAX_BLOCKS ? MHA_MAX_BLOCKS / blocks : 1;
   for (int64_t head0 = 0; head0 < heads; head0 += most) {
     int tail = 1;
     unsigned grid = 0;
-    MhaWork work = mha_plan(cost, heads - head0 < most ? heads - head0 : most, Nq, ntiles, &tail, &grid);
-    work.head0 = (uint32_t)head0;
+    const MhaWork work = mha_plan(cost, heads - head0 < most ? heads - head0 : most, Nq, ntiles, &tail, &grid);
+    a.head0 = (uint32_t)head0;
     const int tiles = ntiles <= 2 ? (int)ntiles : 0;
     auto kern = kernels[tiles][tail >> 1];
     const int lds = lds_bytes(tail);
@@ -1042,7 +1043,7 @@ extern "C" __attribute__((visibility("default"))) int ac4k_mha_nvfp4_fwd(
   MhaArgs a{static_cast<uint16_t *>(O), o_b_stride, o_h_stride, o_n_stride, o_d_stride,
             static_cast<const uint8_t *>(q), static_cast<const uint8_t *>(k), static_cast<const uint8_t *>(v),
             static_cast<const uint8_t *>(q_sf), static_cast<const uint8_t *>(k_sf), static_cast<const uint8_t *>(v_sf),
-            q_gs, k_gs, v_gs, H, Nq, Nkv, align_up(Nq, 16), align_up(Nkv, 16), align_up(Nkv, 64), (int)(Dqk / 64), (int)Dv,
+            q_gs, k_gs, v_gs, (uint32_t)H, 0, Nq, Nkv, align_up(Nq, 16), align_up(Nkv, 16), align_up(Nkv, 64), (int)(Dqk / 64), (int)Dv,
             (int)align_up(Dv, 16), sm_scale,
             (o_d_stride == 1 && Dv % 8 == 0 && ((uintptr_t)O & 15) == 0 && o_b_stride % 8 == 0 && o_h_stride % 8 == 0 && o_n_stride % 8 == 0) ? 1 : 0};
   // measured: 512 x 2 x 128 to 8192 x 4 x 128 and 16384 x 40 on 4096 to 16384 keys
@@ -1071,7 +1072,7 @@ extern "C" __attribute__((visibility("default"))) int ac4k_mha_int8_x_fp8_fwd(
   AC4K_REQUIRE(o_b_stride >= 0 && o_h_stride >= 0 && o_n_stride >= 1 && o_d_stride >= 1, "strides of O must be positive");
   Mha8Args a{static_cast<uint16_t *>(O), o_b_stride, o_h_stride, o_n_stride, o_d_stride,
              static_cast<const int8_t *>(q), static_cast<const int8_t *>(k), static_cast<const uint8_t *>(v),
-             q_sf, k_sf, v_sf, H, Nq, Nkv, align_up(Nkv, 16), ceil_div(Nq, q_quantize_block_size), ceil_div(Nkv, 128),
+             q_sf, k_sf, v_sf, (uint32_t)H, 0, Nq, Nkv, align_up(Nkv, 16), ceil_div(Nq, q_quantize_block_size), ceil_div(Nkv, 128),
              (int)Dqk, (int)Dv, (int)align_up(Dv, 16), q_quantize_block_size, sm_scale,
              (o_d_stride == 1 && Dv % 8 == 0 && ((uintptr_t)O & 15) == 0 && o_b_stride % 8 == 0 && o_h_stride % 8 == 0 && o_n_stride % 8 == 0) ? 1 : 0};
   // measured: 512 x 2 x 128 to 8192 x 4 x 128 on 4096 and 8192 keys, one round; one tile: 8192 heads of 49 to 128 rows

@@ -414,7 +414,7 @@ void launch_attn_quant(const AttnQuantArgs &a, hipStream_t st) {
   // K and V of 16384 x 40 x 128.  Short spans: eight (one round, 4.9 against 5.6 us at 257 x 12 x 64).
   // More workgroups than the GPU holds at once, neighbouring tokens in a wave: no more waves than one round of loads needs, so
   // that the sums of a wave meet fewer others and more workgroups are there (BHND, us with eight waves and now: 1024 x 8 windows
-  // of 49 tokens, D = 32, 80 and 13; 256 x 12 of 64, D = 64, 32 and 10; 128 x 16 of 100, D = 128, 23 and 18).
+  // of 49 tokens, D = 32, 80 and 17; 256 x 12 of 64, D = 64, 32 and 11; 128 x 16 of 100, D = 128, 23 and 18).
   int waves = a.span > 256 ? AQ_STAT_WAVES : 8;
   if (a.span <= 256 && uk + uv > 1024 && !adjacent(a.k) && !adjacent(a.v)) {
     const int rows = AQ_STAT_LOADS * aq_heads_per_wave(a.D > a.Dv ? a.D : a.Dv);
