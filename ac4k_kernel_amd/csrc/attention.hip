@@ -588,6 +588,11 @@ constexpr int mha8_stat_lds(int split) { return split == 1 ? 2 * MHA8_K_LDS + 2 
 constexpr int mha8_lds_bytes(int split) { return mha8_stat_lds(split) + (split == 1 ? 0 : 2 * 512 * 4); }
 static_assert(2 * MHA8_K_LDS + 2 * MHA8_V_LDS <= mha8_stat_lds(2) && 8 * MHA_OUT_LDS <= mha8_lds_bytes(1));
 constexpr float MHA8_EXP_OFFSET = 7.5f;
+// start of S: the bits of 1 / (2 pi), the inline constant whose mantissa (2292099 of 2^23) leaves room for every S on both sides;
+// 1 / the unit of its last place
+constexpr int MHA8_S_BIAS = 0x3e22f983;
+constexpr float MHA8_S_UNIT = 67108864.0f;  // 2^26
+static_assert((MHA8_S_BIAS & 0x7fffff) > 128 * 128 * 128 && (MHA8_S_BIAS & 0x7fffff) + 128 * 128 * 128 < 0x800000);
 
 // Eight waves, two per SIMD; a wave owns 32 query rows and 1 / SPLIT of the kv positions of every tile: SPLIT waves
 // share a group of query rows, 256 / SPLIT rows per workgroup.  What a shared group needs per tile is the row maximum
@@ -598,14 +603,17 @@ constexpr float MHA8_EXP_OFFSET = 7.5f;
 //
 // A tile step is a software pipeline over three tiles, written out in the order in which it issues (the compiler's
 // scheduler keeps an MFMA and the vector instructions that could run under it apart):
-//   O += Vhat . Phat of tile i - 1  |  maxima, exp2, e4m3 of tile i  |  S of tile i + 1, into the registers that the
-//   scores of tile i leave one 32-row fragment after the other
+//   O += Vhat . Phat of tile i - 1  |  exp2, e4m3 of tile i  |  S of tile i + 1, into the registers that the scores of
+//   tile i leave one 32-row fragment after the other; under its last fragment the maxima of the others
 // K arrives by LDS-DMA two tiles ahead, V through registers one tile ahead.
-// Bound by the issue of vector instructions (349 per tile and wave beside 24 MFMAs, 65 exp2 of them at a quarter of the rate; at
-// 8192 x 40 x 128 the vector port is busy for 78 % of a SIMD's time and the matrix core for 37 %) and, where the whole GPU is busy
-// for long, by power (2.05 GHz there).
-// Kernel alone, before (128 or 256 rows, no split, no pipeline) and now: 16384 x 40 x 128 3447 -> 3314 us (1659 TFLOP/s),
-// 4096 x 40 264 -> 249, 8192 x 4 118 -> 103, 3000 x 24 143 -> 110, 512 x 2 on 8192 keys 114 -> 71, 75600 x 1 3007 -> 2071.
+// Bound by the issue of vector instructions (about 350 per tile and wave beside 24 MFMAs; two waves share a SIMD and take 8.3 cycles for
+// an exp2, 9.6 for a pair of e4m3, 4.3 for a maximum or an integer conversion, 2.4 to 2.9 for an addition or fma, which they issue
+// together) and, where the whole GPU is busy for long, by power (2.0 GHz there).
+// Of the two waves of a SIMD the older one is served first: it ran a whole step alone, at the rate of one wave, and then waited at
+// the barrier for half of the next.  A wave therefore lowers its priority as it gets on with a step, which keeps the two side by side:
+// 16384 x 40 x 128 5270 -> 4955 cycles per tile of both (priorities that alternate step by step 5160 to 5220).
+// The whole call on 16384 x 40 x 128 3474 -> 3301 us with all of it (moving the maxima and the conversion alone 3446), 4096 x 40 284 -> 277,
+// 3000 x 2 x 24 x 64 194 -> 188.  The conversion and the maxima cost less than they save in the clock: power takes back about a third.
 // TILES as above: 8192 heads of 49 x 49, D = 32, 209 / 179 / 144 us; 1024 heads of 256 x 256, D = 64, 42 / 44 / 41.5; 40 heads
 // of 16384 x 200 133 / 122 / 114.
 template <int SPLIT, int TILES>
@@ -676,10 +684,10 @@ __device__ __forceinline__ void mha_int8_x_fp8_block(const Mha8Args &a, const Mh
   }
   const float qs = (a.sm_scale * MHA_LOG2E) * a.q_sf[bh * a.nqb + mq / a.q_block];
   const float *ksf_src = a.k_sf + bh * a.nkb;
-  // A negative product of scales turns the order of the scores of a tile around.  The quantizers write none; operands
-  // that hold one anywhere take a loop of their own.
-  bool negative = qs < 0.0f;
-  for (int t = lane; t < ntiles; t += 64) negative |= ksf_src[t] < 0.0f;
+  // A negative product of scales turns the order of the scores of a tile around, and one near the end of the range (2^100) does not take
+  // the unit of S.  The quantizers write none; operands that hold one anywhere take a loop of their own.
+  bool negative = !(qs >= 0.0f);
+  for (int t = lane; t < ntiles; t += 64) negative |= !(ksf_src[t] >= 0.0f && qs * ksf_src[t] < 0x1p100f);
   negative = __builtin_amdgcn_ballot_w64(negative) != 0;
   float ksf_next = ksf_src[0];
 
@@ -729,69 +737,78 @@ __device__ __forceinline__ void mha_int8_x_fp8_block(const Mha8Args &a, const Mh
   auto k_operand = [](const uint8_t *const (&kb)[4], int t) {
     return *reinterpret_cast<const i32x4 *>(kb[t & 3] + (t >> 2) * 4096);
   };
+  // A score as a float.  Scales of one sign and of ordinary size: S starts at the bits of a float, MHA8_S_BIAS, so that its bits, read as a
+  // float, are that number + S units of its last place (no sum leaves the binade).  Taking the number off again is exact, as is the unit, a
+  // power of two, in the scale: the scores are those of a conversion, bit for bit, by an addition that two waves of a SIMD issue
+  // together (2.4 cycles a wave) where the conversion of an integer takes 4.3.
+  auto score = [&](auto negative_tag, int s) {
+    return decltype(negative_tag)::value ? (float)s : __int_as_float(s) - __int_as_float(MHA8_S_BIAS);
+  };
+  // extrema over the scores of fragments
+  int hi, lo;
+  auto extremum = [&](auto negative_tag, int f) {
+#pragma unroll
+    for (int e = 0; e < 16; ++e) {
+      hi = SI[f][e] > hi ? SI[f][e] : hi;
+      if (decltype(negative_tag)::value) lo = SI[f][e] < lo ? SI[f][e] : lo;
+    }
+    asm volatile("" : "+v"(hi));
+  };
   // maxima (minima) of a tile's parts, two tiles in turn: [tile & 1][max, min][group][part][row]
   int *mx_lds = reinterpret_cast<int *>(mha_lds + mha8_stat_lds(SPLIT)) + group * (SPLIT * 32) + r;
-  auto part_extremum = [&](auto negative_tag, int parity) {
+  auto part_extremum = [&](auto negative_tag, int parity) {  // (the last fragment's; the others are in hi and lo)
     constexpr bool NEG = decltype(negative_tag)::value;
-    int hi = SI[0][0], lo = SI[0][0];
-#pragma unroll
-    for (int f = 0; f < NF; ++f)
-#pragma unroll
-      for (int e = 0; e < 16; ++e) {
-        hi = SI[f][e] > hi ? SI[f][e] : hi;
-        if (NEG) lo = SI[f][e] < lo ? SI[f][e] : lo;
-      }
+    if (NF == 1) hi = lo = SI[0][0];
+    extremum(negative_tag, NF - 1);
     mx_lds[parity * 512 + part * 32] = mha_halves_imax(hi);  // (both halves of the wave write the same value)
     if (NEG) mx_lds[parity * 512 + 256 + part * 32] = mha_halves_imin(lo);
   };
-  {
+  // (in registers of its own: folded into the first MFMA of one fragment, but copied from scalars for four of them in a loop)
+  i32x16 start = (i32x16)(MHA8_S_BIAS);
+  auto first_scores = [&](auto negative_tag) {
+    if (!decltype(negative_tag)::value) asm volatile("" : "+v"(start));
+    constexpr bool NEG = decltype(negative_tag)::value;
     const uint8_t *kb[4];
     k_rows(0, kb);
 #pragma unroll
     for (int t = 0; t < 4 * NF; ++t)
-      SI[t >> 2] = __builtin_amdgcn_mfma_i32_32x32x32_i8(k_operand(kb, t), QF[t & 3], (t & 3) == 0 ? (i32x16)(0) : SI[t >> 2], 0, 0, 0);
-  }
-  if constexpr (SPLIT > 1) part_extremum(std::true_type{}, 0);
-  __syncthreads();
+      SI[t >> 2] = __builtin_amdgcn_mfma_i32_32x32x32_i8(k_operand(kb, t), QF[t & 3], (t & 3) == 0 ? (i32x16)(NEG ? 0 : MHA8_S_BIAS) : SI[t >> 2], 0, 0, 0);
+    hi = lo = SI[0][0];
+#pragma unroll
+    for (int f = 0; f < NF - 1; ++f) extremum(negative_tag, f);
+    if constexpr (SPLIT > 1) part_extremum(negative_tag, 0);
+    __syncthreads();
+  };
 
   // One kv tile i.  TAIL: the last, partial one, where P of the positions past Nkv is zero.
   auto tile_step = [&](auto negative_tag, auto tail_tag, auto first_tag, auto last_tag, int i) {
     constexpr bool FIRST = decltype(first_tag)::value, LAST = decltype(last_tag)::value;  // no tile in front of / behind this one
     constexpr bool NEG = decltype(negative_tag)::value, TAIL = decltype(tail_tag)::value;
+    constexpr int PV0 = SPLIT == 1 ? 1 : 0;  // steps of O in front of P
     const int buf = i & 1;
+    __builtin_amdgcn_s_setprio(3);
     float qk = qs * ksf_next;
     // (here, not behind the loads below: the compiler does not count the transfers of K, and its wait for a load in front of
     // them would be a wait for them too)
     asm volatile("" : "+v"(qk));
     if constexpr (!LAST) ksf_next = ksf_src[i + 1 < ntiles ? i + 1 : i];
     asm volatile("" ::: "memory");
-    if constexpr (TILES == 0) fetch_k(i + 2, buf);
-    if constexpr (TILES != 1) fetch_v(i, vp);
-    if constexpr (!FIRST) rescale();
-    // ---- maxima.  The maximum of s = float(S) * qk is taken over the integers S (the conversion keeps their order):
-    // qk >= 0 keeps it too, qk < 0 reverses it.  SPLIT 1: under them the first half of O of the tile before.
     i32x8 VF[2];
     if constexpr (!FIRST) {
       VF[0] = v_operand(buf ^ 1, 0);
       VF[1] = v_operand(buf ^ 1, 1);
     }
-    int hi = SI[0][0], lo = SI[0][0];
+    if constexpr (TILES == 0) fetch_k(i + 2, buf);
+    if constexpr (TILES != 1) fetch_v(i, vp);
+    if constexpr (!FIRST) rescale();
+    __builtin_amdgcn_sched_barrier(0);
+    // ---- maxima.  The maximum of s = float(S) * qk is taken over the integers S (the conversion keeps their order):
+    // qk >= 0 keeps it too, qk < 0 reverses it.  SPLIT 1: those of the last fragment; the step before took the others.
     if constexpr (SPLIT == 1) {
-      __builtin_amdgcn_sched_barrier(0);
+      if constexpr (FIRST || NF == 1) hi = lo = SI[0][0];
+      if constexpr (!FIRST) OT[0] = pv_mfma(VF[0], P[0], OT[0]), VF[0] = v_operand(buf ^ 1, 2);
 #pragma unroll
-      for (int st = 0; st < 4; ++st) {
-        if constexpr (!FIRST) {
-          OT[st] = pv_mfma(VF[st & 1], P[0], OT[st]);
-          VF[st & 1] = v_operand(buf ^ 1, st + 2);
-        }
-#pragma unroll
-        for (int e = 0; e < 16; ++e) {
-          hi = SI[st][e] > hi ? SI[st][e] : hi;
-          if (NEG) lo = SI[st][e] < lo ? SI[st][e] : lo;
-        }
-        asm volatile("" : "+v"(hi));
-        __builtin_amdgcn_sched_barrier(0);
-      }
+      for (int f = FIRST ? 0 : NF - 1; f < NF; ++f) extremum(negative_tag, f);
       hi = mha_halves_imax(hi);
       if (NEG) lo = mha_halves_imin(lo);
     } else {
@@ -807,7 +824,8 @@ __device__ __forceinline__ void mha_int8_x_fp8_block(const Mha8Args &a, const Mh
         }
       }
     }
-    const float smax = (float)(NEG && qk < 0.0f ? lo : hi) * qk;
+    const float qk1 = NEG ? qk : qk * MHA8_S_UNIT;
+    const float smax = score(negative_tag, NEG && qk < 0.0f ? lo : hi) * qk1;
     const float m_new = __builtin_fmaxf(smax - MHA8_EXP_OFFSET, m_run);
     alpha = __builtin_amdgcn_exp2f(m_run - m_new);
     m_run = m_new;
@@ -822,24 +840,31 @@ __device__ __forceinline__ void mha_int8_x_fp8_block(const Mha8Args &a, const Mh
     for (int j = 0; j < NPV; ++j) PN[j] = P[j];
     i32x4 KF[2];
 #pragma unroll
-    for (int st = 0; st < 4 * NF + 4; ++st) {  // step st: P of the st-th group of four scores; an O part or S part st - 4
-      if (st < 4) {
-        if constexpr (!FIRST) {
-          OT[st] = pv_mfma(VF[st & 1], P[NPV - 1], OT[st]);
-          if (st < 2) VF[st & 1] = v_operand(buf ^ 1, (NPV - 1) * 4 + st + 2);
+    for (int st = 0; st < 4 * NF + 4; ++st) {  // step st: P of the st-th group of four scores; a part of O; a part of S, st - 4
+      if (st == NF) __builtin_amdgcn_s_setprio(2);
+      if (st == NF * 9 / 4) __builtin_amdgcn_s_setprio(1);
+      if (st == NF * 7 / 2) __builtin_amdgcn_s_setprio(0);
+      if constexpr (!FIRST) {
+        const int u = st + PV0;
+        if (u < 4 * NPV) {
+          OT[u & 3] = pv_mfma(VF[u & 1], P[u >> 2], OT[u & 3]);
+          if (u + 2 < 4 * NPV) VF[u & 1] = v_operand(buf ^ 1, u + 2);
         }
-        if (!LAST && st >= 2) KF[st & 1] = k_operand(kb, st - 2);
-      } else if constexpr (!LAST) {
-        const int t = st - 4, f = t >> 2, s4 = t & 3;
-        SI[f] = __builtin_amdgcn_mfma_i32_32x32x32_i8(KF[t & 1], QF[s4], s4 == 0 ? (i32x16)(0) : SI[f], 0, 0, 0);
-        if (t + 2 < 4 * NF) KF[t & 1] = k_operand(kb, t + 2);
+      }
+      if constexpr (!LAST) {
+        if (st == 2 || st == 3) KF[st & 1] = k_operand(kb, st - 2);
+        if (st >= 4) {
+          const int t = st - 4, f = t >> 2, s4 = t & 3;
+          SI[f] = __builtin_amdgcn_mfma_i32_32x32x32_i8(KF[t & 1], QF[s4], s4 == 0 ? (NEG ? (i32x16)(0) : start) : SI[f], 0, 0, 0);
+          if (t + 2 < 4 * NF) KF[t & 1] = k_operand(kb, t + 2);
+        }
       }
       if (st < 4 * NF) {
         const int f = st >> 2, q = st & 3;
         float p[4];
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
-          p[e] = __builtin_amdgcn_exp2f(__builtin_fmaf((float)SI[f][4 * q + e], qk, -m_new));  // p <= 2^7.5
+          p[e] = __builtin_amdgcn_exp2f(__builtin_fmaf(score(negative_tag, SI[f][4 * q + e]), qk1, -m_new));  // p <= 2^7.5
           if (TAIL && f * 32 + q * 8 + e >= left) p[e] = 0.0f;
           lsum += p[e];
         }
@@ -857,28 +882,36 @@ __device__ __forceinline__ void mha_int8_x_fp8_block(const Mha8Args &a, const Mh
           PN[f >> 1][4 * (f & 1) + 2 * (q >> 1)] = w0;
           PN[f >> 1][4 * (f & 1) + 2 * (q >> 1) + 1] = w1;
         }
+      } else if constexpr (!LAST) {  // under S of the last fragment, the extrema of the others
+        const int f = st - 4 * NF;
+        if (f == 0) hi = lo = SI[0][0];
+        if (f < NF - 1) extremum(negative_tag, f);
+        if (f == 3) stage_v(buf, vp);
       }
       __builtin_amdgcn_sched_barrier(0);
     }
+    if constexpr (LAST) stage_v(buf, vp);
 #pragma unroll
     for (int j = 0; j < NPV; ++j) P[j] = PN[j];
     l_run = __builtin_fmaf(l_run, alpha, mha_halves_sum(lsum));
     if constexpr (SPLIT > 1 && !LAST) part_extremum(negative_tag, buf ^ 1);
-    stage_v(buf, vp);
     wait_vmcnt<0>();  // the transfers of K
     __syncthreads();
   };
   using No = std::false_type;
   using Yes = std::true_type;
   auto all_tiles = [&](auto negative_tag) {
+    first_scores(negative_tag);
     int i = 0;
     for (; i < (int)(a.Nkv / 128); ++i) tile_step(negative_tag, No{}, No{}, No{}, i);
     if (i < ntiles) tile_step(negative_tag, Yes{}, No{}, No{}, i);
   };
   // (the probability keeps the registers of the loop that runs)
   if constexpr (TILES == 1) {  // (a code for both signs and both ends)
+    first_scores(Yes{});
     tile_step(Yes{}, Yes{}, Yes{}, Yes{}, 0);
   } else if constexpr (TILES == 2) {
+    first_scores(Yes{});
     tile_step(Yes{}, No{}, Yes{}, No{}, 0);
     tile_step(Yes{}, Yes{}, No{}, Yes{}, 1);
   } else if (__builtin_expect_with_probability(negative, 0, 0.99999)) {

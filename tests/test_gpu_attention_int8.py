@@ -218,6 +218,26 @@ def test_split_plans_and_negative_scales(H, Nq, Nkv, signs):
     torch.testing.assert_close(o.cpu().float(), ref.float(), atol=ATOL, rtol=RTOL)
 
 
+# |S| up to 128 * 128 * 128, the largest that the biased sums of the fast loop hold, at ordinary and at denormal products of scales; from
+# 2^100 on the loop of the general case takes them (a score apart is then all of the softmax)
+@pytest.mark.parametrize("q_log2,k_log2", [(-9, -9), (-70, -70), (55, 44), (60, 44)])
+@pytest.mark.parametrize("H,Nq,Nkv", [(1, 40, 500), (256, 256, 300)])
+def test_extreme_scores(H, Nq, Nkv, q_log2, k_log2):
+    sm_scale = 0.08664339780807495  # times log2(e) 0.125 exactly: every score is a float, and so is its distance from the maximum
+    g = torch.Generator().manual_seed(Nq)
+    q = torch.randint(0, 2, (1, H, Nq, 1), generator=g).mul(255).sub(128).to(torch.int8).expand(-1, -1, -1, 128).contiguous()
+    k = torch.randint(0, 2, (1, H, Nkv, 1), generator=g).mul(255).sub(128).to(torch.int8).expand(-1, -1, -1, 128).contiguous()
+    k[:, :, ::3] = torch.randint(-128, 128, k[:, :, ::3].shape, generator=g, dtype=torch.int8)
+    q_sf = torch.full((1, H, -(-Nq // 64)), 2.0 ** q_log2)
+    k_sf = torch.full((1, H, -(-Nkv // 128)), 2.0 ** k_log2)
+    v8, v_sf = T.quantize_fp8(make_input((1, H, Nkv, 64), seed=6), 3, 2, 2.25, True)
+    ref = A.mha_int8_x_fp8_fwd(q, q_sf, 64, k, k_sf, 128, v8, v_sf, sm_scale)
+    o = torch.zeros((1, H, Nq, 64), dtype=torch.bfloat16, device="cuda")
+    binding().mha_int8_x_fp8_fwd(o, q.cuda(), q_sf.cuda(), 64, k.cuda(), k_sf.cuda(), 128,
+                                 v8.cuda().view(torch.float8_e4m3fn), v_sf.cuda(), sm_scale)
+    torch.testing.assert_close(o.cpu().float(), ref.float(), atol=ATOL, rtol=RTOL)
+
+
 def test_error_behaviour():
     b = binding()
     q = torch.zeros((1, 1, 16, 128), dtype=torch.int8, device="cuda")
