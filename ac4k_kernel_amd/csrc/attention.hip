@@ -69,24 +69,45 @@ __device__ __forceinline__ MhaTile mha_tile(const MhaWork &w, uint32_t H, uint32
 struct MhaCost {
   float fixed_us[3], tile_us[3];  // split 1, 2, 4
 };
-static MhaWork mha_plan(const MhaCost &c, int64_t heads, int64_t Nq, int64_t ntiles, int *tail, unsigned *grid) {
-  const int64_t cus = device_cu_count() >= 8 ? device_cu_count() / 8 * 8 : 256;
+struct MhaPlan {
+  MhaWork work;
+  unsigned grid;
+  int tail;  // 1, 2, 4
+  float us;
+};
+static int64_t mha_cus() { return device_cu_count() >= 8 ? device_cu_count() / 8 * 8 : 256; }
+static MhaPlan mha_plan(const MhaCost &c, int64_t heads, int64_t Nq, int64_t ntiles) {
+  const int64_t cus = mha_cus();
   const int64_t blocks = ceil_div(Nq, 256), T = heads * blocks, full = T / cus * cus, left = T - full;
   auto rounds_us = [&](int64_t wgs, int i) { return (float)ceil_div(wgs, cus) * (c.fixed_us[i] + (float)ntiles * c.tile_us[i]); };
-  float best = 0.0f;
-  MhaWork work{0, (uint32_t)blocks, 0};
-  *grid = 0;
+  MhaPlan p{{0, (uint32_t)blocks, 0}, 0, 1, 0.0f};
   auto offer = [&](float us, int64_t first, int64_t wgs, int64_t cut, int i) {
-    if ((*grid && us >= best) || first + wgs >= (1ll << 23)) return;  // (2^23 workgroups of 512 threads: more than a launch carries)
-    best = us, *tail = 1 << i, *grid = (unsigned)(first + wgs);
-    work.full = (uint32_t)first, work.cut = (uint32_t)cut;
+    if ((p.grid && us >= p.us) || first + wgs >= (1ll << 23)) return;  // (2^23 workgroups of 512 threads: more than a launch carries)
+    p.us = us, p.tail = 1 << i, p.grid = (unsigned)(first + wgs);
+    p.work.full = (uint32_t)first, p.work.cut = (uint32_t)cut;
   };
   for (int i = 0; i < (left ? 3 : 1) && full; ++i) offer(rounds_us(full, 0) + rounds_us(left << i, i), full, left << i, blocks << i, i);
   for (int i = 0; i < 3; ++i) {  // (beside whole rounds only where it gains more than the costs are good for)
     const int64_t cut = ceil_div(Nq << i, 256);
     offer(rounds_us(heads * cut, i) * (full ? 1.05f : 1.0f), 0, heads * cut, cut, i);
   }
-  return work;
+  return p;
+}
+// Workgroups of four waves, 128 rows or 128 / split, all alike: a CU holds two of them, and one that has it to itself is faster.
+struct Mha4Cost {
+  MhaCost alone, shared;
+};
+static MhaPlan mha4_plan(const Mha4Cost &c, int64_t heads, int64_t Nq, int64_t ntiles) {
+  const int64_t cus = mha_cus();
+  MhaPlan p{{0, 0, 0}, 0, 1, 0.0f};
+  for (int i = 0; i < 3; ++i) {
+    const int64_t cut = ceil_div(Nq << i, 128), wgs = heads * cut, rounds = ceil_div(wgs, 2 * cus);
+    const MhaCost &m = wgs <= cus ? c.alone : c.shared;
+    const float us = (float)rounds * (m.fixed_us[i] + (float)ntiles * m.tile_us[i]);
+    if ((p.grid && us >= p.us) || wgs >= (1ll << 24)) continue;  // (2^24 workgroups of 256 threads: more than a launch carries)
+    p = MhaPlan{{0, 0, (uint32_t)cut}, (unsigned)wgs, 1 << i, us};
+  }
+  return p;
 }
 
 // eight nibbles times the block scale -> eight fp16 (exact)
@@ -218,7 +239,7 @@ constexpr int MHA_PITCH = 272;                   // bytes per decoded row in LDS
 constexpr int MHA_TILE_LDS = 128 * MHA_PITCH;    // one decoded operand tile: K 128 kv rows, V 128 d rows
 constexpr int MHA_STAT_LDS = 4 * MHA_TILE_LDS;   // K tiles j & 1, V tiles j & 1; behind them the row maxima and sums of split tiles
 constexpr int MHA_LUT_LDS = MHA_STAT_LDS + 2 * 256 * 4;  // exact reciprocals of the e4m3 values, as in the quantizer
-constexpr int mha_lds_bytes(int) { return MHA_LUT_LDS + 128 * 4; }
+constexpr int MHA_LDS = MHA_LUT_LDS + 128 * 4;
 static_assert(8 * 16384 <= MHA_STAT_LDS && 8 * MHA_OUT_LDS <= MHA_STAT_LDS, "the parts of O and the staged output fit below the maxima");
 
 // Eight waves, two per SIMD; a wave owns 32 query rows and 1 / SPLIT of the kv positions of every tile (see the INT8 x FP8
@@ -589,10 +610,12 @@ typedef int i32x16 __attribute__((ext_vector_type(16)));
 constexpr int MHA8_K_LDS = 128 * 128;
 constexpr int MHA8_PITCH = 144;
 constexpr int MHA8_V_LDS = 128 * MHA8_PITCH;
-// split tiles: row maxima and sums behind the tile buffers and behind the parts of O of eight waves
-constexpr int mha8_stat_lds(int split) { return split == 1 ? 2 * MHA8_K_LDS + 2 * MHA8_V_LDS : 8 * 16384; }
-constexpr int mha8_lds_bytes(int split) { return mha8_stat_lds(split) + (split == 1 ? 0 : 2 * 512 * 4); }
-static_assert(2 * MHA8_K_LDS + 2 * MHA8_V_LDS <= mha8_stat_lds(2) && 8 * MHA_OUT_LDS <= mha8_lds_bytes(1));
+// split tiles: row maxima and sums behind the tile buffers and behind the parts of O of all waves
+constexpr int mha8_stat_lds(int waves, int split) {
+  return split == 1 || waves * 16384 < 2 * MHA8_K_LDS + 2 * MHA8_V_LDS ? 2 * MHA8_K_LDS + 2 * MHA8_V_LDS : waves * 16384;
+}
+constexpr int mha8_lds_bytes(int waves, int split) { return mha8_stat_lds(waves, split) + (split == 1 ? 0 : 2 * 512 * 4); }
+static_assert(8 * MHA_OUT_LDS <= mha8_lds_bytes(8, 1) && 2 * mha8_lds_bytes(4, 4) <= 160 * 1024);
 constexpr float MHA8_EXP_OFFSET = 7.5f;
 // start of S: the bits of 1 / (2 pi), the inline constant whose mantissa (2292099 of 2^23) leaves room for every S on both sides;
 // 1 / the unit of its last place
@@ -600,8 +623,8 @@ constexpr int MHA8_S_BIAS = 0x3e22f983;
 constexpr float MHA8_S_UNIT = 67108864.0f;  // 2^26
 static_assert((MHA8_S_BIAS & 0x7fffff) > 128 * 128 * 128 && (MHA8_S_BIAS & 0x7fffff) + 128 * 128 * 128 < 0x800000);
 
-// Eight waves, two per SIMD; a wave owns 32 query rows and 1 / SPLIT of the kv positions of every tile: SPLIT waves
-// share a group of query rows, 256 / SPLIT rows per workgroup.  What a shared group needs per tile is the row maximum
+// Two waves per SIMD; a wave owns 32 query rows and 1 / SPLIT of the kv positions of every tile: SPLIT waves
+// share a group of query rows, 32 * WAVES / SPLIT rows per workgroup.  What a shared group needs per tile is the row maximum
 // over the whole tile, which goes through LDS with the barrier that ends the tile; the partial sums of O and of the row
 // meet at the end.  The maxima, and with them every rounding of P, are those of the unsplit tile; the sums of O and of the row
 // are added in another order, so equal rows of two launches, or of the cut and the uncut part of one, may differ by an fp32
@@ -620,17 +643,22 @@ static_assert((MHA8_S_BIAS & 0x7fffff) > 128 * 128 * 128 && (MHA8_S_BIAS & 0x7ff
 // 16384 x 40 x 128 5270 -> 4955 cycles per tile of both (priorities that alternate step by step 5160 to 5220).
 // The whole call on 16384 x 40 x 128 3474 -> 3301 us with all of it (moving the maxima and the conversion alone 3446), 4096 x 40 284 -> 277,
 // 3000 x 2 x 24 x 64 194 -> 188.  The conversion and the maxima cost less than they save in the clock: power takes back about a third.
-// TILES as above: 8192 heads of 49 x 49, D = 32, 209 / 179 / 144 us; 1024 heads of 256 x 256, D = 64, 42 / 44 / 41.5; 40 heads
-// of 16384 x 200 133 / 122 / 114.
-template <int SPLIT, int TILES>
+// TILES as above: 8192 heads of 49 x 49, D = 32, 209 / 179 / 144 us with eight waves; 1024 heads of 256 x 256, D = 64, 42 / 44 / 41.5;
+// 40 heads of 16384 x 200 133 / 122 / 114.
+// WAVES: eight, or four and two workgroups on a CU, which wait for their barriers and their ends one under the other's work, but
+// fetch every tile of K and V twice per CU.  Whole rounds of many tiles go to eight (kernel alone, us, eight / four: 40 heads of 4096 x
+// 4096 224 / 250, 24 of 4096 x 8192 260 / 277); short loops and grids that leave CUs idle, which finer cuts fill, to four (2 heads of 4096 x 8192 70 / 63,
+// 3 of 2111 x 7000 61 / 56, 24 of 2637 x 2637 75 / 65; whole calls on 40 heads of 16384 x 77 134 -> 120).
+template <int WAVES, int SPLIT, int TILES>
 __device__ __forceinline__ void mha_int8_x_fp8_block(const Mha8Args &a, const MhaTile &wg) {
   constexpr int NF = 4 / SPLIT;             // 32-row fragments of a tile per wave
   constexpr int NPV = SPLIT == 1 ? 2 : 1;   // P.V operands of 64 kv positions per wave (SPLIT 4: half of one, zeros behind)
-  constexpr int ROWS = 256 / SPLIT;
+  constexpr int ROWS = WAVES * 32 / SPLIT;
+  constexpr int KT = 16 / WAVES, VT = WAVES / 2, VP = 8 / VT;  // transfers of K per wave; threads on a row of V, their 16-groups
   extern __shared__ __attribute__((aligned(16))) uint8_t mha_lds[];
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), r = lane & 31, h = lane >> 5;
   const int group = wave / SPLIT, part = wave % SPLIT;
-  const int srow = threadIdx.x >> 2, sq = threadIdx.x & 3;  // staging role for V: row of the tile, 32-byte quarter of it
+  const int srow = threadIdx.x / VT, sv = threadIdx.x % VT;  // staging role for V: row of the tile, part of it
   if (wg.block * ROWS >= a.Nq) return;
   const int64_t bh = wg.b * a.H + wg.head;
   const int64_t m = wg.block * ROWS + group * 32 + r;  // this lane's query row
@@ -647,34 +675,40 @@ __device__ __forceinline__ void mha_int8_x_fp8_block(const Mha8Args &a, const Mh
   // l % 8 of row l / 8, so it fetches the 16-byte piece that belongs there
   const int kpiece = (lane & 7) ^ (lane >> 4);  // even t; ^ 4 for odd t
   const uint32_t kcol[2] = {(uint32_t)(kpiece * 16 < a.Dp ? kpiece * 16 : 0), (uint32_t)((kpiece ^ 4) * 16 < a.Dp ? (kpiece ^ 4) * 16 : 0)};
-  const uint32_t krow = (uint32_t)((wave * 16 + (lane >> 3)) * a.Dp);
+  const uint32_t krow = (uint32_t)((wave * 8 * KT + (lane >> 3)) * a.Dp);
   const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint8_t *)mha_lds;
   auto fetch_k = [&](int tile, int buf) {
     if (tile >= ntiles) tile = ntiles - 1;
     const int8_t *src = k_head + (int64_t)tile * 128 * a.Dp;
     const uint32_t last_off = (uint32_t)((tile < ntiles - 1 ? 127 : k_last) * a.Dp);
 #pragma unroll
-    for (int j = 0; j < 2; ++j) {
+    for (int j = 0; j < KT; ++j) {
       const uint32_t off = krow + (uint32_t)(j * 8 * a.Dp);
-      dma16(src, (off < last_off ? off : last_off) + kcol[j], lds0 + buf * MHA8_K_LDS, (uint32_t)((wave * 2 + j) * 1024));
+      dma16(src, (off < last_off ? off : last_off) + kcol[j & 1], lds0 + buf * MHA8_K_LDS, (uint32_t)((wave * KT + j) * 1024));
     }
   };
   struct Piece {
-    uint4 lo, hi;
+    uint4 g[VP];
   };
   const uint8_t *v_row = a.v + (bh * a.Dv + (srow < a.Dv ? srow : a.Dv - 1)) * a.Nkv16;
   auto fetch_v = [&](int tile, Piece &v) {  // tiles in turn
-    const int last = tile < ntiles - 1 ? 127 : v_last, c0 = sq * 32 < last ? sq * 32 : last, c1 = sq * 32 + 16 < last ? sq * 32 + 16 : last;
-    v.lo = *reinterpret_cast<const uint4 *>(v_row + c0);
-    v.hi = *reinterpret_cast<const uint4 *>(v_row + c1);
+    const int last = tile < ntiles - 1 ? 112 : v_last;
+#pragma unroll
+    for (int j = 0; j < VP; ++j) {
+      const int c = (sv * VP + j) * 16;
+      v.g[j] = *reinterpret_cast<const uint4 *>(v_row + (c < last ? c : last));
+    }
     v_row += 128;
   };
-  // V: the thread's two 16-groups (2 sq, 2 sq + 1) regrouped so that the 8-byte pieces of lane half hh of both are one
-  // 16-byte run at 32 sq + 16 hh
+  // V: the thread's 16-groups regrouped in pairs so that the 8-byte pieces of lane half hh of both are one 16-byte run at
+  // 32 (pair) + 16 hh
   auto stage_v = [&](int buf, const Piece &v) {
-    uint8_t *vd = mha_lds + 2 * MHA8_K_LDS + buf * MHA8_V_LDS + srow * MHA8_PITCH + sq * 32;
-    *reinterpret_cast<uint4 *>(vd) = make_uint4(v.lo.x, v.lo.y, v.hi.x, v.hi.y);
-    *reinterpret_cast<uint4 *>(vd + 16) = make_uint4(v.lo.z, v.lo.w, v.hi.z, v.hi.w);
+    uint8_t *vd = mha_lds + 2 * MHA8_K_LDS + buf * MHA8_V_LDS + srow * MHA8_PITCH + sv * VP * 16;
+#pragma unroll
+    for (int j = 0; j < VP; j += 2) {
+      *reinterpret_cast<uint4 *>(vd + j * 16) = make_uint4(v.g[j].x, v.g[j].y, v.g[j + 1].x, v.g[j + 1].y);
+      *reinterpret_cast<uint4 *>(vd + j * 16 + 16) = make_uint4(v.g[j].z, v.g[j].w, v.g[j + 1].z, v.g[j + 1].w);
+    }
   };
 
   Piece vp;
@@ -707,7 +741,8 @@ __device__ __forceinline__ void mha_int8_x_fp8_block(const Mha8Args &a, const Mh
   for (int j = 0; j < NPV; ++j) P[j] = (i32x8)(0);
   if constexpr (TILES == 0) {  // V of the tile in front of the first one: zeros, and so is its P
     Piece z;
-    z.lo = z.hi = make_uint4(0, 0, 0, 0);
+#pragma unroll
+    for (int j = 0; j < VP; ++j) z.g[j] = make_uint4(0, 0, 0, 0);
     stage_v(1, z);
   }
   wait_vmcnt<0>();
@@ -761,7 +796,7 @@ __device__ __forceinline__ void mha_int8_x_fp8_block(const Mha8Args &a, const Mh
     asm volatile("" : "+v"(hi));
   };
   // maxima (minima) of a tile's parts, two tiles in turn: [tile & 1][max, min][group][part][row]
-  int *mx_lds = reinterpret_cast<int *>(mha_lds + mha8_stat_lds(SPLIT)) + group * (SPLIT * 32) + r;
+  int *mx_lds = reinterpret_cast<int *>(mha_lds + mha8_stat_lds(WAVES, SPLIT)) + group * (SPLIT * 32) + r;
   auto part_extremum = [&](auto negative_tag, int parity) {  // (the last fragment's; the others are in hi and lo)
     constexpr bool NEG = decltype(negative_tag)::value;
     if (NF == 1) hi = lo = SI[0][0];
@@ -934,7 +969,7 @@ __device__ __forceinline__ void mha_int8_x_fp8_block(const Mha8Args &a, const Mh
   constexpr int NFD = 4 / SPLIT;
   const int d0 = part * NFD * 32;
   if constexpr (SPLIT > 1)
-    mha_meet<SPLIT>(OT, l_run, reinterpret_cast<float *>(mha_lds), reinterpret_cast<float *>(mha_lds + mha8_stat_lds(SPLIT)), group, part, lane);
+    mha_meet<SPLIT>(OT, l_run, reinterpret_cast<float *>(mha_lds), reinterpret_cast<float *>(mha_lds + mha8_stat_lds(WAVES, SPLIT)), group, part, lane);
 
   // ---- O = O * ((1 / l) * v_sf[d]) -> bf16
   const float rl = 1.0f / l_run;
@@ -955,10 +990,14 @@ __device__ __forceinline__ void mha_int8_x_fp8_block(const Mha8Args &a, const Mh
 }
 
 // (two bodies in one kernel, so that the workgroups of the last round start as the ones in front of them end)
-template <int TAIL, int TILES>
+template <int TAIL>
 __global__ __launch_bounds__(512, 1) void mha_int8_x_fp8_fwd_kernel(Mha8Args a, MhaWork w) {
-  if (TAIL == 1 || blockIdx.x < w.full) mha_int8_x_fp8_block<1, TILES>(a, mha_tile(w, a.H, a.head0, 1, w.blocks));
-  else mha_int8_x_fp8_block<TAIL, TILES>(a, mha_tile(w, a.H, a.head0, TAIL, w.cut));
+  if (TAIL == 1 || blockIdx.x < w.full) mha_int8_x_fp8_block<8, 1, 0>(a, mha_tile(w, a.H, a.head0, 1, w.blocks));
+  else mha_int8_x_fp8_block<8, TAIL, 0>(a, mha_tile(w, a.H, a.head0, TAIL, w.cut));
+}
+template <int SPLIT, int TILES>
+__global__ __launch_bounds__(256, 2) void mha_int8_x_fp8_fwd4_kernel(Mha8Args a, MhaWork w) {
+  mha_int8_x_fp8_block<4, SPLIT, TILES>(a, mha_tile(w, a.H, a.head0, SPLIT, w.cut));
 }
 
 // Per-token-block int8 quantizer in front of it (python/ac4k_kernel/ops/attention.py:18-99, a Triton kernel in the
@@ -1023,40 +1062,35 @@ static void (*const mha_nvfp4_kernels[3][3])(MhaArgs, MhaWork) = {
     {mha_nvfp4_fwd_kernel<1, 0>, mha_nvfp4_fwd_kernel<2, 0>, mha_nvfp4_fwd_kernel<4, 0>},
     {mha_nvfp4_fwd_kernel<1, 1>, mha_nvfp4_fwd_kernel<2, 1>, mha_nvfp4_fwd_kernel<4, 1>},
     {mha_nvfp4_fwd_kernel<1, 2>, mha_nvfp4_fwd_kernel<2, 2>, mha_nvfp4_fwd_kernel<4, 2>}};
-static void (*const mha_int8_x_fp8_kernels[3][3])(Mha8Args, MhaWork) = {
-    {mha_int8_x_fp8_fwd_kernel<1, 0>, mha_int8_x_fp8_fwd_kernel<2, 0>, mha_int8_x_fp8_fwd_kernel<4, 0>},
-    {mha_int8_x_fp8_fwd_kernel<1, 1>, mha_int8_x_fp8_fwd_kernel<2, 1>, mha_int8_x_fp8_fwd_kernel<4, 1>},
-    {mha_int8_x_fp8_fwd_kernel<1, 2>, mha_int8_x_fp8_fwd_kernel<2, 2>, mha_int8_x_fp8_fwd_kernel<4, 2>}};
+// (row 0: eight waves; they gain nothing on one and two tiles)
+static void (*const mha_int8_x_fp8_kernels[4][3])(Mha8Args, MhaWork) = {
+    {mha_int8_x_fp8_fwd_kernel<1>, mha_int8_x_fp8_fwd_kernel<2>, mha_int8_x_fp8_fwd_kernel<4>},
+    {mha_int8_x_fp8_fwd4_kernel<1, 1>, mha_int8_x_fp8_fwd4_kernel<2, 1>, mha_int8_x_fp8_fwd4_kernel<4, 1>},
+    {mha_int8_x_fp8_fwd4_kernel<1, 2>, mha_int8_x_fp8_fwd4_kernel<2, 2>, mha_int8_x_fp8_fwd4_kernel<4, 2>},
+    {mha_int8_x_fp8_fwd4_kernel<1, 0>, mha_int8_x_fp8_fwd4_kernel<2, 0>, mha_int8_x_fp8_fwd4_kernel<4, 0>}};
 
 // A launch carries fewer than 2^32 threads along a grid dim: from 2^31 on the heads go out in several launches, each planned
 // by itself.
 constexpr int64_t MHA_MAX_BLOCKS = 1 << 22;
+static int64_t mha_heads_per_launch(int64_t Nq) {
+  const int64_t blocks = ceil_div(Nq, 256);
+  return blocks < MHA_MAX_BLOCKS ? MHA_MAX_BLOCKS / blocks : 1;
+}
 
 template <typename Args>
-static int mha_launch(Args a, int64_t heads, int64_t Nq, int64_t ntiles, const MhaCost &cost, void (*const (&kernels)[3][3])(Args, MhaWork),
-                      int (*lds_bytes)(int), hipStream_t st, const char *what) {
-  const int64_t blocks = ceil_div(Nq, 256), most = blocks < MHA_MAX_BLOCKS ? MHA_MAX_BLOCKS / blocks : 1;
-  for (int64_t head0 = 0; head0 < heads; head0 += most) {
-    int tail = 1;
-    unsigned grid = 0;
-    const MhaWork work = mha_plan(cost, heads - head0 < most ? heads - head0 : most, Nq, ntiles, &tail, &grid);
-    a.head0 = (uint32_t)head0;
-    const int tiles = ntiles <= 2 ? (int)ntiles : 0;
-    auto kern = kernels[tiles][tail >> 1];
-    const int lds = lds_bytes(tail);
-    // more than 64 KB of dynamic LDS has to be allowed once per device and kernel
-    static std::atomic<uint32_t> lds_done[3][3];
-    int dev = 0;
-    if (hipGetDevice(&dev) != hipSuccess) dev = 0;
-    const uint32_t bit = 1u << (dev & 31);
-    if (!(lds_done[tiles][tail >> 1].load(std::memory_order_relaxed) & bit)) {
-      hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, lds);
-      if (e != hipSuccess) return set_error("hipFuncSetAttribute(LDS=%d): %s", lds, hipGetErrorString(e));
-      lds_done[tiles][tail >> 1].fetch_or(bit, std::memory_order_relaxed);
-    }
-    hipLaunchKernelGGL(kern, dim3(grid), dim3(512), lds, st, a, work);
+static int mha_launch(const Args &a, const MhaPlan &p, void (*kern)(Args, MhaWork), std::atomic<uint32_t> &lds_done, int lds, int threads,
+                      hipStream_t st) {
+  // more than 64 KB of dynamic LDS has to be allowed once per device and kernel
+  int dev = 0;
+  if (hipGetDevice(&dev) != hipSuccess) dev = 0;
+  const uint32_t bit = 1u << (dev & 31);
+  if (!(lds_done.load(std::memory_order_relaxed) & bit)) {
+    hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, lds);
+    if (e != hipSuccess) return set_error("hipFuncSetAttribute(LDS=%d): %s", lds, hipGetErrorString(e));
+    lds_done.fetch_or(bit, std::memory_order_relaxed);
   }
-  return check_launch(what);
+  hipLaunchKernelGGL(kern, dim3(p.grid), dim3(threads), lds, st, a, p.work);
+  return 0;
 }
 
 }  // namespace ac4k
@@ -1087,7 +1121,15 @@ extern "C" __attribute__((visibility("default"))) int ac4k_mha_nvfp4_fwd(
             (o_d_stride == 1 && Dv % 8 == 0 && ((uintptr_t)O & 15) == 0 && o_b_stride % 8 == 0 && o_h_stride % 8 == 0 && o_n_stride % 8 == 0) ? 1 : 0};
   // measured: 512 x 2 x 128 to 8192 x 4 x 128 and 16384 x 40 on 4096 to 16384 keys
   static constexpr MhaCost cost{{5.0f, 6.0f, 5.5f}, {3.9f, 2.35f, 1.6f}};
-  return mha_launch(a, B * H, Nq, ceil_div(Nkv, 128), cost, mha_nvfp4_kernels, mha_lds_bytes, (hipStream_t)stream, "ac4k_mha_nvfp4_fwd");
+  static std::atomic<uint32_t> lds_done[3][3];
+  const int64_t ntiles = ceil_div(Nkv, 128), heads = B * H, most = mha_heads_per_launch(Nq);
+  for (int64_t head0 = 0; head0 < heads; head0 += most) {
+    const MhaPlan p = mha_plan(cost, heads - head0 < most ? heads - head0 : most, Nq, ntiles);
+    const int tiles = ntiles <= 2 ? (int)ntiles : 0;
+    a.head0 = (uint32_t)head0;
+    if (int rc = mha_launch(a, p, mha_nvfp4_kernels[tiles][p.tail >> 1], lds_done[tiles][p.tail >> 1], MHA_LDS, 512, (hipStream_t)stream)) return rc;
+  }
+  return check_launch("ac4k_mha_nvfp4_fwd");
 }
 
 // Replaces ac4k::mha_int8_x_fp8_fwd (lib/cuda/sm120/mha_int8_x_fp8.cu:979-1137).
@@ -1114,9 +1156,25 @@ extern "C" __attribute__((visibility("default"))) int ac4k_mha_int8_x_fp8_fwd(
              q_sf, k_sf, v_sf, (uint32_t)H, 0, Nq, Nkv, align_up(Nkv, 16), ceil_div(Nq, q_quantize_block_size), ceil_div(Nkv, 128),
              (int)Dqk, (int)Dv, (int)align_up(Dv, 16), q_quantize_block_size, sm_scale,
              (o_d_stride == 1 && Dv % 8 == 0 && ((uintptr_t)O & 15) == 0 && o_b_stride % 8 == 0 && o_h_stride % 8 == 0 && o_n_stride % 8 == 0) ? 1 : 0};
-  // measured: 512 x 2 x 128 to 8192 x 4 x 128 on 4096 and 8192 keys, one round; one tile: 8192 heads of 49 to 128 rows
-  static constexpr MhaCost cost{{4.5f, 6.0f, 5.0f}, {2.35f, 1.45f, 1.05f}}, one{{6.9f, 6.5f, 4.6f}, {0.0f, 0.0f, 0.0f}};
-  return mha_launch(a, B * H, Nq, ceil_div(Nkv, 128), Nkv <= 128 ? one : cost, mha_int8_x_fp8_kernels, mha8_lds_bytes, (hipStream_t)stream, "ac4k_mha_int8_x_fp8_fwd");
+  // measured: 4096 rows of 1 to 40 heads on 1024 and 8192 keys, D = 128, every split of both kernels
+  static constexpr MhaCost cost{{6.7f, 5.0f, 4.1f}, {2.36f, 1.43f, 1.06f}};
+  static constexpr Mha4Cost cost4{{{2.9f, 2.7f, 2.1f}, {1.50f, 1.10f, 0.905f}}, {{6.7f, 4.7f, 4.3f}, {2.50f, 1.55f, 1.21f}}};
+  static std::atomic<uint32_t> lds_done[4][3];
+  const int64_t ntiles = ceil_div(Nkv, 128), heads = B * H, most = mha_heads_per_launch(Nq);
+  for (int64_t head0 = 0; head0 < heads; head0 += most) {
+    const int64_t n = heads - head0 < most ? heads - head0 : most;
+    MhaPlan p = mha4_plan(cost4, n, Nq, ntiles);
+    int kind = ntiles <= 2 ? (int)ntiles : 3;
+    if (ntiles > 2) {
+      const MhaPlan p8 = mha_plan(cost, n, Nq, ntiles);
+      if (p8.us <= p.us) p = p8, kind = 0;
+    }
+    a.head0 = (uint32_t)head0;
+    const int waves = kind == 0 ? 8 : 4;
+    if (int rc = mha_launch(a, p, mha_int8_x_fp8_kernels[kind][p.tail >> 1], lds_done[kind][p.tail >> 1],
+                            mha8_lds_bytes(waves, kind == 0 && p.tail == 1 ? 1 : p.tail), waves * 64, (hipStream_t)stream)) return rc;
+  }
+  return check_launch("ac4k_mha_int8_x_fp8_fwd");
 }
 
 // Replaces _int8_quantize / _triton_block_token_quantize (python/ac4k_kernel/ops/attention.py:18-99): x bf16 with element

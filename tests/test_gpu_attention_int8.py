@@ -218,6 +218,14 @@ def test_split_plans_and_negative_scales(H, Nq, Nkv, signs):
     torch.testing.assert_close(o.cpu().float(), ref.float(), atol=ATOL, rtol=RTOL)
 
 
+# Workgroups of eight waves in whole rounds (no rest, a rest cut in two and in four), cut alike, and of four waves on one, two and more tiles
+@pytest.mark.parametrize("H,Nq,Nkv", [(256, 256, 300), (384, 250, 300), (260, 256, 300), (130, 250, 300), (128, 250, 3900), (8, 1100, 700),
+                                      (150, 100, 300), (300, 60, 200), (300, 60, 600), (1, 300, 4000)])
+@pytest.mark.parametrize("signs", [False, True])
+def test_four_and_eight_waves(H, Nq, Nkv, signs):
+    test_split_plans_and_negative_scales(H, Nq, Nkv, signs)
+
+
 # |S| up to 128 * 128 * 128, the largest that the biased sums of the fast loop hold, at ordinary and at denormal products of scales; from
 # 2^100 on the loop of the general case takes them (a score apart is then all of the softmax)
 @pytest.mark.parametrize("q_log2,k_log2", [(-9, -9), (-70, -70), (55, 44), (60, 44)])
