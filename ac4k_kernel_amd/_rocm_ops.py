@@ -180,9 +180,8 @@ def linear_nvfp4(D, A, A_sf, A_global_scale, B, B_sf, B_global_scale, bias=None)
     bias_ptr, bias_tag = _bias_args(bias, N)
     if M == 0 or N == 0:
         return
-    scratch = _skinny_scratch(D.device, M, N, K)
-    if scratch is not None:
-        ws = scratch
+    if _L.ac4k_linear_nvfp4_scratch_bytes(M, N, K) > 0:
+        ws = _skinny_scratch(D.device, M, N, K)
         _lib.check(_L.ac4k_linear_nvfp4_workspace(D.data_ptr(), _DTYPE_TAG[D.dtype], A.data_ptr(), A_sf.data_ptr(),
                                                   A_global_scale.data_ptr(), B.data_ptr(), B_sf.data_ptr(),
                                                   B_global_scale.data_ptr(), bias_ptr, bias_tag, M, N, K,

@@ -2040,7 +2040,127 @@ __global__ __launch_bounds__(ST_THREADS, 1) void linear_nvfp4_stream64_kernel(Sk
   stream_finish<D_DT, BIAS_DT, 4, 2>(acc, a, stlds, *a.A_gs, wn, kq, lane, n0);
 }
 
-// Plan of a decode-sized linear: which of the two kernels, its K split and the fp32 scratch it needs.
+// ===========================================================================
+// Decode-sized linear (1 <= M <= 32, K % 64 == 0, K >= 256) with 16 weight rows per workgroup and all of K in it: weights with too
+// few rows for the LDS-ring kernels, which split their K over workgroups and add the parts in a second launch.
+//
+// Eight waves take the 128-k steps of a row in turn.  Nothing is shared between them, so nothing goes through LDS: lane (row r,
+// quarter g) loads the 16 bytes [32 g, 32 g + 32) of the step of its weight row - four lanes a 64-byte run - with the two block
+// scales, and the same of activation row r, three steps ahead, and has with each dword the operand of one v_mfma_f32_16x16x32_f16 (the
+// order of k is free as long as both sides share it).  The eight sums meet through LDS in the order of the waves.
+// A step's second half that K does not have is read from its first one, with weight scales so small that they round to zero.
+// Bound by the weights from memory and, from about M = 8 on, by the decoding of the activation, which every workgroup does again for
+// as many bytes as its weights (M <= 16; twice as many above): 16 x 4096 x 14336, weights from HBM, 17.8 -> 11.4 us (64 rows, K split in
+// four, and the second launch before), M = 1 15.8 -> 10.4; 16 x 4096 x 4096 10.2 -> 5.1; 1 x 20000 x 2880 23.4 -> 11.2; 32 x 1024 x 1024
+// 7.6 -> 3.2.  Three steps ahead and two workgroups on a CU: two more cost 0.7 us at 16 x 4096 x 14336 in registers, sixteen waves 2.5 us at
+// 1 x 14336 x 4096, four waves 3 us at 16 x 4096 x 14336; loads past the caches lose where the activation is read again.
+// ===========================================================================
+constexpr int R16_ROWS = 16, R16_WAVES = 8, R16_STEP = 128, R16_DEPTH = 3;
+
+// MT: tiles of 16 activation rows.  TAIL: K is no multiple of 128.
+template <int D_DT, int BIAS_DT, int MT, bool TAIL>
+__global__ __launch_bounds__(64 * R16_WAVES, 2) void linear_nvfp4_rows16_kernel(SkinnyArgs a) {
+  __shared__ float4 part[R16_WAVES][MT][64];
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), r = lane & 15, g = lane >> 4;
+  const int64_t n0 = (int64_t)blockIdx.x * R16_ROWS, kb = a.K >> 1;
+  const int nst = (int)ceil_div(a.K, R16_STEP);
+  const int cnt = (nst - wave + R16_WAVES - 1) / R16_WAVES;  // steps of this wave; none where K is short
+  const int wr = n0 + r < a.N ? r : (int)(a.N - 1 - n0);  // rows past N read the last row; their outputs are never stored
+  const uint8_t *const w_src = uniform_ptr(a.B + n0 * kb), *const ws_src = uniform_ptr(reinterpret_cast<const uint8_t *>(a.B_sf) + n0 * 4);
+  const uint32_t w_row = (uint32_t)(wr * kb), ws_row = (uint32_t)(wr * 4);
+  uint32_t x_row[MT], xs_row[MT];
+#pragma unroll
+  for (int i = 0; i < MT; ++i) {
+    const int m = i * 16 + r < a.M ? i * 16 + r : (int)a.M - 1;  // rows past M likewise
+    x_row[i] = (uint32_t)(m * kb), xs_row[i] = (uint32_t)(m * 4);
+  }
+  struct Step {
+    uint4 w, x[MT];
+    uint32_t ws, xs[MT];
+  };
+  auto load = [&](Step &st, int t) {
+    const int s = wave + t * R16_WAVES;
+    const uint32_t gg = TAIL && s == nst - 1 ? g & 1 : g;
+    const int64_t at = (int64_t)s * (R16_STEP / 2);
+    st.w = *reinterpret_cast<const uint4 *>(w_src + at + (w_row + gg * 16));
+    st.ws = *reinterpret_cast<const uint16_t *>(ws_src + (int64_t)(2 * s) * a.Np * 4 + ((gg >> 1) * (uint32_t)a.Np * 4 + ws_row + (gg & 1) * 2));
+#pragma unroll
+    for (int i = 0; i < MT; ++i) {
+      st.x[i] = *reinterpret_cast<const uint4 *>(a.Aq + at + (x_row[i] + gg * 16));
+      st.xs[i] = *reinterpret_cast<const uint16_t *>(a.A_sf + (int64_t)(2 * s) * a.Mp * 4 + ((gg >> 1) * (uint32_t)a.Mp * 4 + xs_row[i] + (gg & 1) * 2));
+    }
+  };
+  f32x4 acc[MT][2];  // two independent accumulation chains
+#pragma unroll
+  for (int i = 0; i < MT; ++i) acc[i][0] = acc[i][1] = (f32x4)(0.0f);
+  auto multiply = [&](const Step &st, int t) {
+    const float fac = TAIL && wave + t * R16_WAVES == nst - 1 && g >= 2 ? 0x1p-60f : 1.0f;
+    const f16x2 wsc = __builtin_amdgcn_cvt_scalef32_pk_f16_fp8(st.ws, fac, false);
+    const f16x8 w0 = decode_dword<false>(st.w.x, wsc), w1 = decode_dword<false>(st.w.y, wsc);
+    const f16x8 w2 = decode_dword<true>(st.w.z, wsc), w3 = decode_dword<true>(st.w.w, wsc);
+#pragma unroll
+    for (int i = 0; i < MT; ++i) {
+      const f16x2 xsc = __builtin_amdgcn_cvt_scalef32_pk_f16_fp8(st.xs[i], 1.0f, false);
+      acc[i][0] = __builtin_amdgcn_mfma_f32_16x16x32_f16(w0, decode_dword<false>(st.x[i].x, xsc), acc[i][0], 0, 0, 0);
+      acc[i][1] = __builtin_amdgcn_mfma_f32_16x16x32_f16(w1, decode_dword<false>(st.x[i].y, xsc), acc[i][1], 0, 0, 0);
+      acc[i][0] = __builtin_amdgcn_mfma_f32_16x16x32_f16(w2, decode_dword<true>(st.x[i].z, xsc), acc[i][0], 0, 0, 0);
+      acc[i][1] = __builtin_amdgcn_mfma_f32_16x16x32_f16(w3, decode_dword<true>(st.x[i].w, xsc), acc[i][1], 0, 0, 0);
+    }
+  };
+  Step ring[R16_DEPTH];
+#pragma unroll
+  for (int d = 0; d < R16_DEPTH; ++d)
+    if (d < cnt) load(ring[d], d);
+  int t = 0;
+  for (; t + R16_DEPTH < cnt; t += R16_DEPTH) {
+#pragma unroll
+    for (int d = 0; d < R16_DEPTH; ++d) {
+      multiply(ring[d], t + d);
+      if (t + d + R16_DEPTH < cnt) load(ring[d], t + d + R16_DEPTH);
+    }
+  }
+#pragma unroll
+  for (int d = 0; d < R16_DEPTH; ++d)
+    if (t + d < cnt) multiply(ring[d], t + d);
+
+  // lane (r, g): activation row r of tile i, weight rows 4 g .. 4 g + 3
+#pragma unroll
+  for (int i = 0; i < MT; ++i) {
+    const f32x4 v = acc[i][0] + acc[i][1];
+    part[wave][i][lane] = make_float4(v[0], v[1], v[2], v[3]);
+  }
+  __syncthreads();
+  if (wave >= MT) return;
+  float4 v = part[0][wave][lane];
+#pragma unroll
+  for (int q = 1; q < R16_WAVES; ++q) {
+    const float4 o = part[q][wave][lane];
+    v.x += o.x, v.y += o.y, v.z += o.z, v.w += o.w;
+  }
+  const int m = wave * 16 + r;
+  const int64_t n = n0 + g * 4;
+  if (m >= (int)a.M || n >= a.N) return;
+  using DE = Elem<D_DT>;
+  const float scale = (*a.A_gs) * (*a.B_gs);
+  float o[4] = {v.x * scale, v.y * scale, v.z * scale, v.w * scale};
+  if constexpr (BIAS_DT != BIAS_NONE) {
+#pragma unroll
+    for (int q = 0; q < 4; ++q) o[q] += n + q < a.N ? Elem<BIAS_DT>::load(a.bias, n + q) : 0.0f;
+  }
+  typename DE::T *dst = static_cast<typename DE::T *>(a.D) + (int64_t)m * a.N + n;
+  if ((a.N & 3) == 0 && ((uintptr_t)a.D & 15) == 0) {
+    if constexpr (sizeof(typename DE::T) == 2)
+      *reinterpret_cast<uint2 *>(dst) = make_uint2(DE::cvt2(o[0], o[1]), DE::cvt2(o[2], o[3]));
+    else
+      *reinterpret_cast<float4 *>(dst) = make_float4(o[0], o[1], o[2], o[3]);
+  } else {
+#pragma unroll
+    for (int q = 0; q < 4; ++q)
+      if (n + q < a.N) dst[q] = DE::cvt(o[q]);
+  }
+}
+
+// Plan of a decode-sized linear: which kernel, its K split and the fp32 scratch it needs.
 enum { DECODE_REGISTERS = 1, DECODE_LDS_RING = 2, DECODE_LDS_RING64 = 3 };
 struct SkinnyPlan {
   int kind;                // DECODE_REGISTERS: linear_nvfp4_skinny_kernel; DECODE_LDS_RING: linear_nvfp4_stream_kernel;
@@ -2049,6 +2169,9 @@ struct SkinnyPlan {
   int split_k;             // K ranges; > 1 needs `partial_bytes` of fp32 scratch
   int64_t partial_bytes, groups;
   int lds_bytes;
+  // linear_nvfp4_rows16_kernel runs instead, and needs no scratch.  The rest of the plan is what the entry points go on asking of
+  // their callers for these shapes.
+  bool rows16;
 };
 static std::atomic<int> g_forced_decode_kernel{0};  // ac4k_set_linear_tuning: 0 = by shape
 
@@ -2103,6 +2226,24 @@ static void plan_lds_ring(int64_t M, int64_t N, int64_t K, SkinnyPlan &p, int ro
 // Hence: with 192 tiles of 128 rows and more, 128-row tiles from M = 8 on; otherwise 64-row tiles when
 // there are 192 of those, or from M = 8 on; the register kernel in the remaining cases.  A K that is no multiple of
 // 256 takes the ring kernels for every M.
+//
+// 16-row workgroups take what they are faster at by these estimates (us, weights from HBM, fitted to 27 shapes of N = 128 to 57344,
+// K = 512 to 16384 and M = 1 to 32; 2^-20 weights = "million").  They grow with M, which the ring kernels hardly notice, and a wave
+// has its steps of K one after the other; the ring kernels run in whole rounds of workgroups and, like the register kernel, pay for
+// a K split.  Both sides as measured (other kernel / 16 rows): M = 16, 4096 x 14336 17.8 / 11.4, 8192 x 8192 18.7 / 13.2, 10240 x 10240
+// 33.5 / 23.5, 14336 x 4096 14.2 / 12.5, 28672 x 8192 33.5 / 41.0, 16384 x 16384 42.7 / 47.0; M = 32, 4096 x 14336 18.2 / 16.6, 14336 x 4096
+// 14.5 / 17.7, 128 x 8192 7.8 / 9.8, 1000 x 1024 7.6 / 3.3; M = 1, 20480 x 8192 41.5 / 23.2, 28672 x 8192 29.2 / 30.0, 300 x 14336 7.8 / 8.8.
+static bool rows16_faster(int64_t M, int64_t N, int64_t K, const SkinnyPlan &p) {
+  const double million = 1e-6 * (double)N * (double)K, steps = (double)ceil_div(ceil_div(K, R16_STEP), R16_WAVES);
+  const double stream = M <= 16 ? 0.114 + 0.0031 * (double)M : 0.150 + 0.0023 * (double)M, chain = M <= 16 ? 0.45 + 0.007 * (double)M : 0.87;
+  const double rows16 = 2.5 + fmax(stream * million, chain * steps);
+  if (p.kind == DECODE_REGISTERS)
+    return rows16 < (N >= 24576 ? 7.5 + (0.0925 + 0.0018 * (double)M) * million : 5.3 + 0.15 * million);
+  if (p.split_k > 1) return rows16 < 7.6 + 0.16 * million;
+  const double rounds = (double)ceil_div(p.groups, (int64_t)device_cu_count());
+  return rows16 < rounds * (5.0 + (p.kind == DECODE_LDS_RING ? 0.88 : 0.54) * (double)ceil_div(K, ST_BK));
+}
+
 static bool skinny_plan(int64_t M, int64_t N, int64_t K, SkinnyPlan &p) {
   if (M < 1 || M > 32 || K < SK_STEP || K % 64 != 0 || N < 1) return false;
   const bool ring_ok = (K >> 1) * ST_BN < (1ll << 31) && N < (1ll << 27);  // 32-bit lane offsets
@@ -2123,6 +2264,8 @@ static bool skinny_plan(int64_t M, int64_t N, int64_t K, SkinnyPlan &p) {
     plan_lds_ring(M, N, K, p);
   else
     plan_registers(M, N, K, p);
+  const bool forced = g_forced_decode_kernel.load(std::memory_order_relaxed) != 0 || g_forced_skinny_ks.load(std::memory_order_relaxed) != 0;
+  p.rows16 = !forced && ring_ok && rows16_faster(M, N, K, p);  // (32-bit lane offsets, as in the ring kernels)
   return true;
 }
 
@@ -2147,6 +2290,13 @@ static int launch_ring(const SkinnyArgs &a, const SkinnyPlan &p, hipStream_t st)
 
 template <int D_DT, int BIAS_DT>
 static int launch_skinny(const SkinnyArgs &a, const SkinnyPlan &p, hipStream_t st) {
+  if (p.rows16) {
+    const bool tail = a.K % R16_STEP != 0;
+    auto *kern = a.M <= 16 ? tail ? linear_nvfp4_rows16_kernel<D_DT, BIAS_DT, 1, true> : linear_nvfp4_rows16_kernel<D_DT, BIAS_DT, 1, false>
+                           : tail ? linear_nvfp4_rows16_kernel<D_DT, BIAS_DT, 2, true> : linear_nvfp4_rows16_kernel<D_DT, BIAS_DT, 2, false>;
+    hipLaunchKernelGGL(kern, dim3((unsigned)ceil_div(a.N, R16_ROWS)), dim3(64 * R16_WAVES), 0, st, a);
+    return 0;
+  }
   if (p.kind == DECODE_LDS_RING) {
     int rc;
     if (a.M <= 16)
@@ -2203,7 +2353,7 @@ static bool packed_kernel_ok(const LinearArgs &a) {
 // workgroups than the split plan, still the weights streamed once instead of the 128x128 tile kernel.
 static bool noscratch_skinny_plan(const LinearArgs &a, SkinnyPlan &p) {
   if (!skinny_plan(a.M, a.N, a.K, p) || (((uintptr_t)a.A | (uintptr_t)a.B) & 15) != 0) return false;
-  if (p.partial_bytes == 0) return true;
+  if (p.rows16 || p.partial_bytes == 0) return true;
   if (!((a.K >> 1) * ST_BN < (1ll << 31) && a.N < (1ll << 27))) return false;  // the ring kernels' 32-bit lane offsets
   p.kind = ceil_div(a.N, ST_BN) >= 192 ? DECODE_LDS_RING : DECODE_LDS_RING64;
   p.groups = ceil_div(a.N, p.kind == DECODE_LDS_RING ? ST_BN : S6_BN);
@@ -2403,6 +2553,12 @@ extern "C" __attribute__((visibility("default"))) int64_t ac4k_linear_nvfp4_work
   return 0;
 }
 
+extern "C" __attribute__((visibility("default"))) int64_t ac4k_linear_nvfp4_scratch_bytes(int64_t M, int64_t N, int64_t K) {
+  SkinnyPlan p;
+  if (skinny_plan(M, N, K, p) && p.rows16) return 0;
+  return ac4k_linear_nvfp4_workspace_bytes(M, N, K);
+}
+
 namespace ac4k {
 
 // K that the `skinny` entry points take: whole stages of the kernels they began with
@@ -2576,6 +2732,7 @@ static bool prepacked_plan(int64_t M, int64_t N, int64_t K, PrepackedPlan &p) {
   p.mid = !p.ring && ksplit_shape(M, N, K);
   if (p.ring) {
     plan_lds_ring(M, N, K, p.sp);
+    p.sp.rows16 = false;
     p.partial_bytes = p.sp.partial_bytes;
   } else {
     p.tp = tile_plan(M, N, K, true);

@@ -470,6 +470,25 @@ def test_k_tails_of_four_chunk_stages(k, ks, linear_tuning):
             check_tight(m, 200, k, seed=k + m, image=True)
 
 
+# 16 weight rows per workgroup: one and two tiles of activation rows, rows that do not exist, waves with no step, fewer steps than
+# are loaded ahead, more, and every remainder of the steps and of K; outputs that start at any element
+@pytest.mark.parametrize("m", [1, 15, 16, 17, 32])
+@pytest.mark.parametrize("n,k", [(1, 256), (16, 320), (130, 1024), (129, 1088), (4, 2944), (1000, 3072), (36, 4160), (2500, 5120)])
+def test_sixteen_row_workgroups(m, n, k):
+    from ac4k_kernel_amd import _lib
+    assert _lib.load().ac4k_linear_nvfp4_scratch_bytes(m, n, k) == 0  # (other kernels would split K here, or be slower)
+    check_tight(m, n, k, seed=m + k)
+    aq, bq = gpu_quant(make_input((m, k), seed=m)), gpu_quant(make_input((n, k), seed=n, std=0.02))
+    bias = make_input((1, n), seed=3)
+    for dt in (torch.bfloat16, torch.float16, torch.float32):
+        ref = T.linear_nvfp4(*cpu(aq), *cpu(bq), bias=bias.to(dt), out_dtype=dt)
+        buf = torch.full((m * n + 3,), 7.0, dtype=dt, device="cuda")
+        out = ops().linear(*aq, *bq, bias=bias.to(dt).cuda(), out=buf[1:1 + m * n].view(m, n))
+        torch.testing.assert_close(out.cpu(), ref, atol=ATOL, rtol=RTOL)
+        assert buf[0] == 7.0 and (buf[1 + m * n:] == 7.0).all()
+        assert torch.equal(ops().linear(*aq, *bq, bias=bias.to(dt).cuda(), out=torch.empty((m, n), dtype=dt, device="cuda")), out)
+
+
 @pytest.mark.parametrize("mi,nj,splits", TILE_PLANS)
 def test_k_tail_of_the_tile_kernel(mi, nj, splits, linear_tuning):
     linear_tuning(mi, nj, splits)
