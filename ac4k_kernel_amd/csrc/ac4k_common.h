@@ -37,6 +37,8 @@ typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 // the same at the alignment of a bf16 element / a byte: global memory takes vector accesses at any address
 typedef u32x4 u32x4_elem __attribute__((aligned(2)));
+typedef f32x4 f32x4_elem __attribute__((aligned(2)));
+typedef uint32_t u32_elem __attribute__((aligned(2)));
 typedef u32x2 u32x2_elem __attribute__((aligned(1)));
 
 // streaming (non-temporal) 16-byte load / 4- and 8-byte stores: data touched once

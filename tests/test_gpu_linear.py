@@ -489,6 +489,25 @@ def test_sixteen_row_workgroups(m, n, k):
         assert torch.equal(ops().linear(*aq, *bq, bias=bias.to(dt).cuda(), out=torch.empty((m, n), dtype=dt, device="cuda")), out)
 
 
+# outputs whose rows start on any element: every remainder of a 16-byte piece, a tile with less than one piece inside the matrix, and
+# nothing written beside the matrix; the tile kernel, its K split and the K-split-waves kernel (which takes M <= 128 by itself)
+@pytest.mark.parametrize("mi,nj,splits", [(2, 1, 1), (2, 2, 1), (2, 4, 2), (4, 2, 1), (4, 4, 1), (0, 0, 0)])
+def test_rows_that_start_on_any_element(mi, nj, splits, linear_tuning):
+    if mi:
+        linear_tuning(mi, nj, splits)
+    for m in ([64 * mi + 37] if mi else [50, 100]):
+        aq = gpu_quant(make_input((m, 256 * max(splits, 1)), seed=m))
+        for n in [64 * max(nj, 2) + r for r in (1, 2, 3, 4, 5, 6, 7, 24 + 8 * mi)]:
+            bq = gpu_quant(make_input((n, 256 * max(splits, 1)), seed=n, std=0.02))
+            bias = make_input((1, n), seed=3)
+            for dt in (torch.bfloat16, torch.float16, torch.float32):
+                ref = T.linear_nvfp4(*cpu(aq), *cpu(bq), bias=bias.to(dt), out_dtype=dt)
+                buf = torch.full((m * n + 4,), 7.0, dtype=dt, device="cuda")
+                out = ops().linear(*aq, *bq, bias=bias.to(dt).cuda(), out=buf[3:3 + m * n].view(m, n))
+                torch.testing.assert_close(out.cpu(), ref, atol=ATOL, rtol=RTOL)
+                assert (buf[:3] == 7.0).all() and (buf[3 + m * n:] == 7.0).all(), (m, n, dt)
+
+
 @pytest.mark.parametrize("mi,nj,splits", TILE_PLANS)
 def test_k_tail_of_the_tile_kernel(mi, nj, splits, linear_tuning):
     linear_tuning(mi, nj, splits)
