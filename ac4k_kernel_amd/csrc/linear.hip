@@ -360,7 +360,7 @@ __device__ __forceinline__ void store_tile(const f32x16 (&acc)[MI][NJ], char *ld
   DT *Dp = static_cast<DT *>(out);
   constexpr int S = sizeof(DT);
   constexpr int WN = 32 * NJ;               // columns per wave
-  constexpr int RP = S == 2 ? 64 : 32;      // rows per staging pass
+  constexpr int RP = S == 2 && MI % 2 == 0 ? 64 : 32;  // rows per staging pass
   constexpr int PITCH = WN * S + 16;        // bytes per staged row, 16 bytes of padding
   constexpr int STG_BYTES = 4 * RP * PITCH;
   static_assert(STG_BYTES + 2 * WN * 4 <= LDS_BYTES, "epilogue staging and bias must fit in LDS");
@@ -458,7 +458,7 @@ __device__ __forceinline__ void store_tile(const f32x16 (&acc)[MI][NJ], char *ld
   }
 }
 
-// MI = 32-row fragments per wave along M: 4 (BM = 256) or 2 (BM = 128);
+// MI = 32-row fragments per wave along M: 4 (BM = 256), 3 (BM = 192) or 2 (BM = 128);
 // NJ = 32-column fragments per wave along N: 4 (BN = 256), 2 (BN = 128) or 1 (BN = 64);
 // PS = LDS stages: PS - 1 k-steps are in flight ahead of the one being multiplied, which a small
 // tile needs because its k-step is much shorter than the memory latency.
@@ -836,45 +836,82 @@ struct TilePlan {
   int64_t partial_bytes;
 };
 
-// Picks the tile and the split by a rough cost model in microseconds on 256 CUs: rounds of
-// workgroups x stages per range x time per 128-k stage of that tile, a fixed prologue/epilogue,
-// and for more than one range the partial sums written and read back at about 4.5 TB/s plus the
-// second launch.  Big problems (192 or more of the largest tiles) take the largest tile as is.
-// The time per stage is a fit to measured loops of the five tile shapes: per 16-k sub-step about
-// 14 cycles per MFMA plus 5 per decode instruction, 400 cycles per stage on top, at 2.1 GHz.
 // Tuning overrides (ac4k_set_linear_tuning): a forced tile plan packed as mi | nj << 8 | splits << 16
 // (0 = the cost model decides) and a forced K slice of the decode-sized kernel (0 = automatic).
 static std::atomic<uint32_t> g_forced_tile_plan{0};
 static std::atomic<int> g_forced_skinny_ks{0};
+static bool forced_tile_plan(int64_t M, int64_t N, int64_t K, TilePlan &p) {
+  const uint32_t f = g_forced_tile_plan.load(std::memory_order_relaxed);
+  const int64_t sp = f >> 16;
+  p = TilePlan{(int)(f & 0xff), (int)((f >> 8) & 0xff), (int)sp, sp > 1 ? sp * M * N * 4 : 0};
+  return f != 0 && sp <= ceil_div(K, P_BK);
+}
 
-static TilePlan tile_plan(int64_t M, int64_t N, int64_t K, bool allow_split) {
-  TilePlan best{M <= 128 ? 2 : 4, 4, 1, 0};
-  if (const uint32_t f = g_forced_tile_plan.load(std::memory_order_relaxed)) {
-    const int mi = f & 0xff, nj = (f >> 8) & 0xff, sp = (int)(f >> 16);
-    if (sp <= ceil_div(K, P_BK) && (sp == 1 || allow_split)) return TilePlan{mi, nj, sp, sp > 1 ? (int64_t)sp * M * N * 4 : 0};
-  }
+// Scratch that the entry points ask for, for the tile kernel's partial sums; 0: they take none (and ac4k_linear_nvfp4_skinny not
+// the shape).  Callers keep these sizes, so they stay what this estimate has always given, although the plan comes from the
+// measured costs below and fits into them: on 50 shapes of M = 129 to 9000 a plan with room for any split would be faster on two,
+// 150 x 4096 x 4096 21.3 -> 20.8 us and 129 x 14336 x 4096 34.5 -> 32.1.
+static int64_t tile_scratch_bytes(int64_t M, int64_t N, int64_t K) {
+  TilePlan forced;
+  if (forced_tile_plan(M, N, K, forced)) return forced.partial_bytes;
   const int64_t stages = ceil_div(K, P_BK);
-  if (ceil_div(M, 64 * best.mi) * ceil_div(N, 256) >= 192) return best;
+  if (ceil_div(M, M <= 128 ? 128 : 256) * ceil_div(N, 256) >= 192) return 0;
   double best_t = 0.0;
-  bool first = true;
+  int64_t best = 0;
   for (int mi = 2; mi <= 4; mi += 2) {
     if (mi == 4 && M <= 128) continue;
     for (int nj = 4; nj >= 1; nj >>= 1) {
-      if (mi == 4 && nj == 1) continue;  // not instantiated
+      if (mi == 4 && nj == 1) continue;
       if (nj < 4 && N < 64 * nj * 2) continue;
       const int nm = mi * nj, nv = 8 * (mi + nj);
       const double stage_us = (8.0 * (14.0 * nm + 5.0 * nv) + 400.0) / 2100.0;
       const double fixed_us = 5.0 + 0.1 * nm;
       const int64_t tiles = ceil_div(M, 64 * mi) * ceil_div(N, 64 * nj);
-      for (int64_t sp = 1; sp <= 32 && (sp == 1 || (allow_split && sp * 2 <= stages)); ++sp) {
+      for (int64_t sp = 1; sp <= 32 && (sp == 1 || sp * 2 <= stages); ++sp) {
         const double rounds = (double)ceil_div(tiles * sp, 256);
         double t = rounds * (double)ceil_div(stages, sp) * stage_us + fixed_us;
         if (sp > 1) t += (double)sp * (double)(M * N) * 8.0 / 4.5e6 + 2.5;
-        if (first || t < best_t) {
-          first = false;
-          best_t = t;
-          best = TilePlan{mi, nj, (int)sp, sp > 1 ? sp * M * N * 4 : 0};
-        }
+        if (best == 0 || t < best_t) best_t = t, best = sp;
+      }
+    }
+  }
+  return best > 1 ? best * M * N * 4 : 0;
+}
+
+// Picks the tile and the K split by measured costs in microseconds on 256 CUs, with at most `scratch` bytes of partial sums:
+// rounds of 256 workgroups, stages per range times the time of a 128-k stage of that tile, a prologue and epilogue per round
+// and for more than one range the partial sums and the second launch.  A stage takes `stage` as long as up to three fifths of the
+// CUs have work and grows with their share from there to stage + 0.4 power, as the clock comes down.  Fitted to 50 shapes of
+// M = 129 to 9000, N = 256 to 28672, K = 512 to 14336 with every tile and up to twelve ranges; of the plans that fit the scratch it
+// takes the fastest everywhere to 0.5 %.  The tiles of 192 rows are what fills a round where 128 or 256 rows leave CUs idle (us, best
+// of the other tiles / with them): 4096 x 5120 x 5120 197.5 / 180.9, 7000 x 5120 x 5120 328.4 / 284.6, 6000 x 4096 x 4096 171.5 / 157.6,
+// 300 x 14336 x 4096 50.9 / 45.3, 1001 x 5003 x 2880 40.1 / 38.4, 180 x 20000 x 1024 17.7 / 16.9.
+struct TileCost {
+  int mi, nj;
+  double stage, power, fixed;
+};
+constexpr TileCost TILE_COSTS[] = {{4, 4, 2.05, 2.1, 9.2},   {3, 4, 1.65, 1.5, 8.9}, {4, 2, 1.295, 0.83, 7.2}, {2, 4, 1.3, 0.9, 8.2},
+                                   {3, 2, 1.08, 0.57, 7.8}, {2, 2, 0.865, 0.28, 6.7}, {2, 1, 0.6, 0.15, 5.2}};
+static TilePlan tile_plan(int64_t M, int64_t N, int64_t K, int64_t scratch) {
+  TilePlan best{};
+  if (forced_tile_plan(M, N, K, best) && best.partial_bytes <= scratch) return best;
+  constexpr double ROUND_US = 3.5, SPLIT_US = 4.5, PARTIAL_BYTES_PER_US = 9.4e6;  // (8 bytes of a sum: written and read)
+  const int64_t stages = ceil_div(K, P_BK);
+  double best_t = 0.0;
+  best.splits = 0;
+  for (const TileCost &c : TILE_COSTS) {
+    if (c.mi > 2 && M <= 128) continue;
+    if (c.nj < 4 && N < 64 * c.nj * 2) continue;
+    const int64_t tiles = ceil_div(M, 64 * c.mi) * ceil_div(N, 64 * c.nj);
+    for (int64_t sp = 1; sp == 1 || (sp <= 32 && sp * 2 <= stages && tiles * sp <= 1024 && sp * M * N * 4 <= scratch); ++sp) {
+      const double len = (double)ceil_div(stages, sp);
+      const int64_t full = tiles * sp / 256, tail = tiles * sp % 256;
+      double t = c.fixed - ROUND_US + (double)full * (len * (c.stage + 0.4 * c.power) + ROUND_US);
+      if (tail) t += len * (c.stage + (tail > 153 ? ((double)tail / 256.0 - 0.6) * c.power : 0.0)) + ROUND_US;
+      if (sp > 1) t += SPLIT_US + (double)(sp * M * N) * 8.0 / PARTIAL_BYTES_PER_US;
+      if (best.splits == 0 || t < best_t) {
+        best_t = t;
+        best = TilePlan{c.mi, c.nj, (int)sp, sp > 1 ? sp * M * N * 4 : 0};
       }
     }
   }
@@ -884,6 +921,7 @@ static TilePlan tile_plan(int64_t M, int64_t N, int64_t K, bool allow_split) {
 template <int D_DT, int BIAS_DT>
 static int launch_tile_plan(const LinearArgs &a, const TilePlan &p, const SplitK &sk, hipStream_t st) {
   if (p.mi == 4) return p.nj == 4 ? launch_tile_p<D_DT, BIAS_DT, 4, 4>(a, sk, st) : launch_tile_p<D_DT, BIAS_DT, 4, 2>(a, sk, st);
+  if (p.mi == 3) return p.nj == 4 ? launch_tile_p<D_DT, BIAS_DT, 3, 4>(a, sk, st) : launch_tile_p<D_DT, BIAS_DT, 3, 2>(a, sk, st);
   if (p.nj == 4) return launch_tile_p<D_DT, BIAS_DT, 2, 4>(a, sk, st);
   return p.nj == 2 ? launch_tile_p<D_DT, BIAS_DT, 2, 2>(a, sk, st) : launch_tile_p<D_DT, BIAS_DT, 2, 1>(a, sk, st);
 }
@@ -892,7 +930,7 @@ static int launch_tile_plan(const LinearArgs &a, const TilePlan &p, const SplitK
 template <int D_DT, int BIAS_DT>
 static int launch_tile256p(const LinearArgs &a, hipStream_t st) {
   const SplitK one{nullptr, 1};
-  return launch_tile_plan<D_DT, BIAS_DT>(a, tile_plan(a.M, a.N, a.K, false), one, st);
+  return launch_tile_plan<D_DT, BIAS_DT>(a, tile_plan(a.M, a.N, a.K, 0), one, st);
 }
 
 // ===========================================================================
@@ -2446,16 +2484,17 @@ struct MidPlan {
   bool has_ksplit;   // the shape suits the K-split-waves kernel (taken when the pointers are aligned for it)
   KsplitPlan kp;
   TilePlan tp;       // what the tile kernel does with the shape otherwise (given enough scratch)
-  int64_t bytes;     // scratch of the preferred choice
+  int64_t bytes;     // scratch that the entry points ask for
 };
 // shapes the workspace entry point takes with 32 < M
 static bool mid_plan(int64_t M, int64_t N, int64_t K, MidPlan &p) {
   if (M <= 32 || N < 128 || K % 64 != 0 || K < P_BK || (K >> 1) * 256 >= (1ll << 31) || N >= (1ll << 27)) return false;
-  p.tp = tile_plan(M, N, K, true);
+  const int64_t tile_bytes = tile_scratch_bytes(M, N, K);
+  p.tp = tile_plan(M, N, K, tile_bytes);
   p.has_ksplit = ksplit_shape(M, N, K);
   p.kp = p.has_ksplit ? ksplit_plan(M, N, K, true) : KsplitPlan{0, 0, 1, 0};
-  p.bytes = p.has_ksplit ? p.kp.partial_bytes : p.tp.partial_bytes;
-  return p.has_ksplit || p.tp.splits > 1;
+  p.bytes = p.has_ksplit ? p.kp.partial_bytes : tile_bytes;
+  return p.has_ksplit || tile_bytes > 0;
 }
 
 // `partial_bytes` of scratch at `partial` (possibly none): the K-split-waves kernel when the shape and the
@@ -2467,7 +2506,7 @@ static int launch_mid(const LinearArgs &a, const MidPlan &p, float *partial, int
     splits = p.kp.splits;
     if (int rc = launch_ksplit<D_DT, BIAS_DT>(a, p.kp, SplitK{splits > 1 ? partial : nullptr, splits}, st)) return rc;
   } else {
-    const TilePlan tp = p.tp.partial_bytes <= partial_bytes ? p.tp : tile_plan(a.M, a.N, a.K, false);
+    const TilePlan tp = p.tp.partial_bytes <= partial_bytes ? p.tp : tile_plan(a.M, a.N, a.K, 0);
     splits = tp.splits;
     if (int rc = launch_tile_plan<D_DT, BIAS_DT>(a, tp, SplitK{splits > 1 ? partial : nullptr, splits}, st)) return rc;
   }
@@ -2558,8 +2597,10 @@ extern "C" __attribute__((visibility("default"))) int64_t ac4k_linear_nvfp4_work
 
 extern "C" __attribute__((visibility("default"))) int64_t ac4k_linear_nvfp4_scratch_bytes(int64_t M, int64_t N, int64_t K) {
   SkinnyPlan p;
-  if (skinny_plan(M, N, K, p) && p.rows16) return 0;
-  return ac4k_linear_nvfp4_workspace_bytes(M, N, K);
+  if (skinny_plan(M, N, K, p)) return p.rows16 ? 0 : p.partial_bytes;
+  MidPlan mp;
+  if (mid_plan(M, N, K, mp)) return mp.has_ksplit || mp.tp.splits > 1 ? mp.bytes : 0;
+  return 0;
 }
 
 namespace ac4k {
@@ -2738,8 +2779,8 @@ static bool prepacked_plan(int64_t M, int64_t N, int64_t K, PrepackedPlan &p) {
     p.sp.rows16 = false;
     p.partial_bytes = p.sp.partial_bytes;
   } else {
-    p.tp = tile_plan(M, N, K, true);
-    p.partial_bytes = p.tp.partial_bytes;
+    p.partial_bytes = tile_scratch_bytes(M, N, K);
+    p.tp = tile_plan(M, N, K, p.partial_bytes);
     if (p.mid) {
       p.kp = ksplit_plan(M, N, K, true);
       p.partial_bytes = p.kp.partial_bytes;
@@ -2843,9 +2884,9 @@ extern "C" __attribute__((visibility("default"))) int ac4k_set_linear_tuning(int
                "decode_kernel must be 0 (by shape), 1 (register kernel), 2 (LDS-ring kernel) or 3 (LDS-ring kernel with "
                "64-row tiles) (got %d)", decode_kernel);
   const bool no_plan = mi == 0 && nj == 0 && splits == 0;
-  AC4K_REQUIRE(no_plan || ((mi == 2 || mi == 4) && (nj == 1 || nj == 2 || nj == 4) && !(mi == 4 && nj == 1) && splits >= 1 &&
+  AC4K_REQUIRE(no_plan || (mi >= 2 && mi <= 4 && (nj == 1 || nj == 2 || nj == 4) && !(mi != 2 && nj == 1) && splits >= 1 &&
                            splits <= 0xffff),
-               "tile plan must be mi in {2,4}, nj in {1,2,4} (not 4,1), 1 <= splits (got %d,%d,%d)", mi, nj, splits);
+               "tile plan must be mi in {2,3,4}, nj in {1,2,4} (1 with mi = 2), 1 <= splits (got %d,%d,%d)", mi, nj, splits);
   AC4K_REQUIRE(skinny_ks >= 0 && skinny_ks % 256 == 0, "skinny_ks must be 0 (automatic) or a multiple of 256 (got %d)",
                skinny_ks);
   ac4k::g_forced_decode_kernel.store(decode_kernel);

@@ -153,7 +153,7 @@ int ac4k_linear_nvfp4_skinny(void *D, int d_dtype, const void *A, const void *A_
  * that are not aligned to 16 bytes (scale tensors: 4) run without scratch, like shapes that need none. */
 int64_t ac4k_linear_nvfp4_workspace_bytes(int64_t M, int64_t N, int64_t K);
 /* How many of these bytes the kernels for operands on 16 bytes write: 0 where ac4k_linear_nvfp4 runs the same kernel without a
- * workspace (decode-sized shapes on 16 weight rows per workgroup ask for one and leave it alone), otherwise all of them. */
+ * workspace (some shapes ask for one and their kernels leave it alone), otherwise all of them. */
 int64_t ac4k_linear_nvfp4_scratch_bytes(int64_t M, int64_t N, int64_t K);
 int ac4k_linear_nvfp4_workspace(void *D, int d_dtype, const void *A, const void *A_sf, const float *A_gs,
                                 const void *B, const void *B_sf, const float *B_gs, const void *bias,
@@ -178,7 +178,7 @@ int ac4k_linear_nvfp4_skinny_static(void *D, int d_dtype, const void *A, const v
 
 /* Tuning aid of the linear entry points (no counterpart in the reference; results stay within the
  * same tolerance): forces the tile of the packed-operand kernel to (64 mi) x (64 nj) with `splits` K
- * ranges (mi in {2,4}, nj in {1,2,4}, not (4,1); splits > 1 only takes effect in the workspace entry
+ * ranges (mi in {2,3,4}, nj in {1,2,4}, 1 only with mi = 2; splits > 1 only takes effect in the workspace entry
  * points), the length of a K range of the decode-sized kernels (a multiple of 256; the register
  * kernel takes 256, 512 or 1024) and which decode-sized kernel runs (1 = weights streamed into
  * registers, 2 = weights streamed through an LDS ring in 128-row tiles, 3 = in 64-row tiles).  Zeros give each choice back to the library.

@@ -283,7 +283,8 @@ def test_ksplit_kernel_against_c_oracle():
 
 # every tile shape of the packed-LDS kernel (64*mi rows x 64*nj columns, its own LDS stage depth),
 # alone and split along K, forced through ac4k_set_linear_tuning; ragged M and N included
-TILE_PLANS = [(2, 1, 1), (2, 2, 1), (2, 4, 1), (4, 2, 1), (4, 4, 1), (2, 1, 3), (2, 2, 2), (2, 4, 5), (4, 2, 2), (4, 4, 4)]
+TILE_PLANS = [(2, 1, 1), (2, 2, 1), (2, 4, 1), (4, 2, 1), (4, 4, 1), (2, 1, 3), (2, 2, 2), (2, 4, 5), (4, 2, 2), (4, 4, 4),
+              (3, 2, 1), (3, 4, 1), (3, 2, 4), (3, 4, 2)]
 
 
 @pytest.mark.parametrize("mi,nj,splits", TILE_PLANS)
@@ -491,7 +492,7 @@ def test_sixteen_row_workgroups(m, n, k):
 
 # outputs whose rows start on any element: every remainder of a 16-byte piece, a tile with less than one piece inside the matrix, and
 # nothing written beside the matrix; the tile kernel, its K split and the K-split-waves kernel (which takes M <= 128 by itself)
-@pytest.mark.parametrize("mi,nj,splits", [(2, 1, 1), (2, 2, 1), (2, 4, 2), (4, 2, 1), (4, 4, 1), (0, 0, 0)])
+@pytest.mark.parametrize("mi,nj,splits", [(2, 1, 1), (2, 2, 1), (2, 4, 2), (3, 2, 1), (3, 4, 1), (4, 2, 1), (4, 4, 1), (0, 0, 0)])
 def test_rows_that_start_on_any_element(mi, nj, splits, linear_tuning):
     if mi:
         linear_tuning(mi, nj, splits)
