@@ -129,11 +129,35 @@ __device__ __forceinline__ void aq_tile(const AttnOperand &t, uint32_t H, uint32
 }
 
 // ---- 2. the tiles ----------------------------------------------------------------------------------------------
+// The partial results of a head's channels put together in the order of the spans, a channel per thread: channel[i] = the result of
+// add(a, b) over all spans.  Every lane of a tile needs eight of them and used to fetch these from all spans by itself, one span after
+// the other, up to 32 waits for the L2.  Whole calls, us, before -> after: 600 queries on 16000 keys of 12 heads 190 -> 174, 2048 x 8 x 100 52.5 -> 46.7,
+// 1024 x 40 x 128 56.4 -> 52.0, 16384 x 40 x 128 3336 -> 3300, 2 x 2048 on 512 keys, 12 x 64, 34.7 -> 32.0; sixteen spans in flight the same; eight
+// in every lane's registers cost a wave per SIMD (16384 queries on 77 keys 137 -> 145).
+constexpr int AQ_PART_LOADS = 8;  // spans in flight
+template <typename Add>
+__device__ __forceinline__ void aq_join_spans(const uint32_t *part, int D, int nsplit, int64_t pitch, uint32_t *channel, Add add) {
+  const int tid = threadIdx.x;
+  if (tid < D) {
+    uint32_t sum = 0;
+    for (int s = 0; s < nsplit; s += AQ_PART_LOADS) {
+      uint32_t x[AQ_PART_LOADS];
+#pragma unroll
+      for (int u = 0; u < AQ_PART_LOADS; ++u) x[u] = s + u < nsplit ? part[(s + u) * pitch + tid] : 0u;
+#pragma unroll
+      for (int u = 0; u < AQ_PART_LOADS; ++u)
+        if (s + u < nsplit) sum = add(sum, x[u]);
+    }
+    channel[tid] = sum;
+  }
+  __syncthreads();
+}
+
 // `BLOCK` tokens of one head to int8 with one scale; MEAN: minus the token mean of their channel, both rounded to
 // bf16 as the subtraction of two bf16 tensors rounds them.
 template <int BLOCK, bool MEAN>
 __device__ __forceinline__ void aq_int8_tile(const AttnQuantArgs &a, const AttnOperand &t, int N, int nb, int8_t *y,
-                                             float *scale, int b, int head, int blk, uint32_t *wmax) {
+                                             float *scale, int b, int head, int blk, uint32_t *wmax, uint32_t *channel) {
   const int tid = threadIdx.x;
   const int ls = aq_lane_shift(a.D), c = tid & ((1 << ls) - 1), r0 = tid >> ls, rstep = 256 >> ls;
   constexpr int NV = BLOCK / 16;  // vectors per thread with 16 lanes per row (half of them with eight)
@@ -150,13 +174,11 @@ __device__ __forceinline__ void aq_int8_tile(const AttnQuantArgs &a, const AttnO
     if (live && r < rows) v[j] = aq_load_stream(src + r * t.s_n);
   }
   if (MEAN) {
-    float mean[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-    const float *p = a.ksum + bh * a.Dp + c0;
-    for (int s = 0; s < a.nsplit; ++s, p += (int64_t)a.B * a.H * a.Dp)
+    aq_join_spans(reinterpret_cast<const uint32_t *>(a.ksum + bh * a.Dp), a.D, a.nsplit, (int64_t)a.B * a.H * a.Dp, channel,
+                  [](uint32_t sum, uint32_t x) { return __float_as_uint(__uint_as_float(sum) + __uint_as_float(x)); });
+    float mean[8];
 #pragma unroll
-      for (int e = 0; e < 8; ++e) mean[e] += p[e];
-#pragma unroll
-    for (int e = 0; e < 8; ++e) mean[e] = (float)(__bf16)(mean[e] * a.inv_nkv);
+    for (int e = 0; e < 8; ++e) mean[e] = (float)(__bf16)(__uint_as_float(channel[c0 + e]) * a.inv_nkv);
 #pragma unroll
     for (int j = 0; j < NV; ++j) {
       if (!(live && r0 + j * rstep < rows)) continue;  // rows past the end stay zero
@@ -193,7 +215,7 @@ __device__ __forceinline__ void aq_int8_tile(const AttnQuantArgs &a, const AttnO
 
 // 64 kv positions per wave, all channels of one head, to e4m3 along kv (the cross-major layout of the quantizers: a lane
 // holds eight channels of 16 stored positions)
-__device__ __forceinline__ void aq_fp8_tile(const AttnQuantArgs &a, int b, int head, int blk) {
+__device__ __forceinline__ void aq_fp8_tile(const AttnQuantArgs &a, int b, int head, int blk, uint32_t *channel) {
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, kb = lane & 3, rg = lane >> 2;
   const int64_t bh = (int64_t)b * a.H + head;
   const int k0 = (blk * 4 + wave) * 64 + kb * 16;
@@ -207,11 +229,10 @@ __device__ __forceinline__ void aq_fp8_tile(const AttnQuantArgs &a, int b, int h
     v[i] = make_uint4(0, 0, 0, 0);
     if (live && k < a.Nkv) v[i] = aq_load(src + (int64_t)k * a.v.s_n);
   }
-  uint32_t mx[8] = {0, 0, 0, 0, 0, 0, 0, 0};
-  const uint32_t *p = a.vmax + bh * a.Dvp + c0;
-  for (int s = 0; s < a.nsplit; ++s, p += (int64_t)a.B * a.H * a.Dvp)
+  aq_join_spans(a.vmax + bh * a.Dvp, a.Dv, a.nsplit, (int64_t)a.B * a.H * a.Dvp, channel, [](uint32_t m, uint32_t x) { return umax32(m, x); });
+  uint32_t mx[8];
 #pragma unroll
-    for (int e = 0; e < 8; ++e) mx[e] = umax32(mx[e], p[e]);
+  for (int e = 0; e < 8; ++e) mx[e] = channel[c0 + e];
   if (blk == 0 && wave == 0 && kb == 0) {  // the scales of this head
     float *sf = a.v_sf + bh * a.Dvp;
     if (live)
@@ -239,22 +260,22 @@ __device__ __forceinline__ void aq_fp8_tile(const AttnQuantArgs &a, int b, int h
 }
 
 __global__ __launch_bounds__(256) void attn_quantize_int8_fp8_kernel(AttnQuantArgs a) {
-  __shared__ uint32_t wmax[4];
+  __shared__ uint32_t wmax[4], channel[128];
   uint32_t idx = blockIdx.x;
   const uint32_t BH = a.B * a.H;
   int b, head, blk;
   const uint32_t nv = BH * a.nvb, nk = BH * a.nkb;
   if (idx < nv) {
     aq_tile(a.v, a.H, a.nvb, idx, b, head, blk);
-    aq_fp8_tile(a, b, head, blk);
+    aq_fp8_tile(a, b, head, blk, channel);
   } else if (idx < nv + nk) {
     idx -= nv;
     aq_tile(a.k, a.H, a.nkb, idx, b, head, blk);
-    aq_int8_tile<AQ_K_BLOCK, true>(a, a.k, a.Nkv, a.nkb, a.k8, a.k_sf, b, head, blk, wmax);
+    aq_int8_tile<AQ_K_BLOCK, true>(a, a.k, a.Nkv, a.nkb, a.k8, a.k_sf, b, head, blk, wmax, channel);
   } else {
     idx -= nv + nk;
     aq_tile(a.q, a.H, a.nqb, idx, b, head, blk);
-    aq_int8_tile<AQ_Q_BLOCK, false>(a, a.q, a.Nq, a.nqb, a.q8, a.q_sf, b, head, blk, wmax);
+    aq_int8_tile<AQ_Q_BLOCK, false>(a, a.q, a.Nq, a.nqb, a.q8, a.q_sf, b, head, blk, wmax, channel);
   }
 }
 

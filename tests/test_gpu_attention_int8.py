@@ -147,6 +147,19 @@ def test_whole_call_with_exact_means_is_bit_identical(B, Nq, Nkv, H, Dqk, Dv, la
     assert torch.equal(got, want) and torch.isfinite(got).all()
 
 
+# numbers of token spans around those that are in flight together, and the most; more channels than lanes of a wave, and few
+@pytest.mark.parametrize("spans", [2, 7, 8, 9, 16, 17, 31, 32])
+@pytest.mark.parametrize("Dqk,Dv", [(128, 100), (8, 128)])
+def test_whole_call_joins_every_span(spans, Dqk, Dv, monkeypatch):
+    n = spans * 32 - 5
+    q, v = make_input((1, 40, 1, Dqk), seed=1).cuda(), make_input((1, n, 1, Dv), seed=3).cuda()
+    k = exact_mean_keys((1, n, 1, Dqk), 1, 2)
+    v[0, n - 1] *= 50.0  # the maxima are in the last span
+    got = ops().attention(q, k, v)
+    monkeypatch.setattr(binding(), "attention_int8_x_fp8", lambda *a: False)
+    assert torch.equal(got, ops().attention(q, k, v)) and torch.isfinite(got).all()
+
+
 @pytest.mark.parametrize("D", [64, 65, 128])
 def test_whole_call_takes_views(D):
     """q and k as views of one buffer of q, k and v, k as a view of the other layout, tokens and heads shared by stride 0."""
