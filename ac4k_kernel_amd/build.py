@@ -16,8 +16,8 @@ PKG_DIR = os.path.dirname(os.path.abspath(__file__))
 ROOT = os.path.dirname(PKG_DIR)
 CSRC = os.path.join(PKG_DIR, "csrc")
 LIB_PATH = os.path.join(PKG_DIR, "libac4k_nvfp4.so")
-SOURCES = ["capi.hip", "quantize.hip", "linear.hip", "attention.hip", "attention_quantize.hip"]
-HEADERS = [os.path.join(CSRC, "ac4k_common.h"), os.path.join(CSRC, "attention_quantize.h"), os.path.join(CSRC, "quantize_nvfp4.h"),
+SOURCES = ["capi.hip", "quantize.hip", "linear.hip", "linear_fused.hip", "attention.hip", "attention_quantize.hip"]
+HEADERS = [os.path.join(CSRC, "ac4k_common.h"), os.path.join(CSRC, "attention_quantize.h"), os.path.join(CSRC, "quantize_nvfp4.h"), os.path.join(CSRC, "linear_common.h"),
            os.path.join(ROOT, "include", "ac4k_nvfp4.h")]
 
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")

@@ -17,7 +17,7 @@
 #include <mutex>
 #include <type_traits>
 
-#include "ac4k_common.h"
+#include "linear_common.h"
 
 namespace ac4k {
 
@@ -41,46 +41,6 @@ struct LinearArgs {
 constexpr int W_BLOCK_ROWS = 128, W_BLOCK_K = 128;
 constexpr int W_BLOCK_DATA = W_BLOCK_ROWS * W_BLOCK_K / 2;            // 8192
 constexpr int W_BLOCK_BYTES = W_BLOCK_DATA + 2 * W_BLOCK_ROWS * 4;    // 9216
-
-// --- output / bias element types -------------------------------------------
-template <int DT>
-struct Elem;
-template <>
-struct Elem<AC4K_DTYPE_BF16> {
-  using T = uint16_t;
-  static __device__ __forceinline__ float load(const void *p, int64_t i) {
-    return bf16_bits_to_f32(static_cast<const uint16_t *>(p)[i]);
-  }
-  // round to nearest even, NaN stays NaN: v_cvt_pk_bf16_f32
-  static __device__ __forceinline__ T cvt(float f) { return __builtin_bit_cast(uint16_t, (__bf16)f); }
-  static __device__ __forceinline__ uint32_t cvt2(float lo, float hi) {
-    typedef __bf16 bf16x2_t __attribute__((ext_vector_type(2)));
-    const f32x2 v = {lo, hi};
-    return __builtin_bit_cast(uint32_t, __builtin_convertvector(v, bf16x2_t));
-  }
-};
-template <>
-struct Elem<AC4K_DTYPE_FP16> {
-  using T = _Float16;
-  static __device__ __forceinline__ float load(const void *p, int64_t i) {
-    return (float)static_cast<const _Float16 *>(p)[i];
-  }
-  static __device__ __forceinline__ T cvt(float f) { return (_Float16)f; }
-  static __device__ __forceinline__ uint32_t cvt2(float lo, float hi) {
-    const f16x2 v = {(_Float16)lo, (_Float16)hi};
-    return __builtin_bit_cast(uint32_t, v);
-  }
-};
-template <>
-struct Elem<AC4K_DTYPE_FP32> {
-  using T = float;
-  static __device__ __forceinline__ float load(const void *p, int64_t i) {
-    return static_cast<const float *>(p)[i];
-  }
-  static __device__ __forceinline__ T cvt(float f) { return f; }
-  static __device__ __forceinline__ uint32_t cvt2(float lo, float) { return __float_as_uint(lo); }  // unused: 4-byte outputs are not packed
-};
-constexpr int BIAS_NONE = 3;
 
 // --- decode -------------------------------------------------------------------
 // E4M3 scale byte -> fp16x2 pattern worth scale * 2^-8 in both halves (exponent bias 7 vs 15;
@@ -292,17 +252,6 @@ template <int MI, int NJ>
 struct DecFrags {
   f16x8 a[MI], b[NJ];
 };
-
-// dword `w` (8 nibbles) times block scale `sc` (both halves of `sc2` hold candidates, HI picks)
-template <bool HI>
-__device__ __forceinline__ f16x8 decode_dword(uint32_t w, f16x2 sc2) {
-  const f16x2 sc = HI ? (f16x2){sc2.y, sc2.y} : (f16x2){sc2.x, sc2.x};
-  f16x2 d0 = __builtin_amdgcn_cvt_scalef32_pk_f16_fp4(w, 1.0f, 0) * sc;
-  f16x2 d1 = __builtin_amdgcn_cvt_scalef32_pk_f16_fp4(w, 1.0f, 1) * sc;
-  f16x2 d2 = __builtin_amdgcn_cvt_scalef32_pk_f16_fp4(w, 1.0f, 2) * sc;
-  f16x2 d3 = __builtin_amdgcn_cvt_scalef32_pk_f16_fp4(w, 1.0f, 3) * sc;
-  return (f16x8){d0.x, d0.y, d1.x, d1.y, d2.x, d2.y, d3.x, d3.y};
-}
 
 template <int S>
 __device__ __forceinline__ uint32_t dword_of(const uint4 &v) {
@@ -2096,7 +2045,7 @@ __global__ __launch_bounds__(ST_THREADS, 1) void linear_nvfp4_stream64_kernel(Sk
 // 7.6 -> 3.2.  Three steps ahead and two workgroups on a CU: two more cost 0.7 us at 16 x 4096 x 14336 in registers, sixteen waves 2.5 us at
 // 1 x 14336 x 4096, four waves 3 us at 16 x 4096 x 14336; loads past the caches lose where the activation is read again.
 // ===========================================================================
-constexpr int R16_ROWS = 16, R16_WAVES = 8, R16_STEP = 128, R16_DEPTH = 3;
+constexpr int R16_DEPTH = 3;
 
 // MT: tiles of 16 activation rows.  TAIL: K is no multiple of 128.
 template <int D_DT, int BIAS_DT, int MT, bool TAIL>
@@ -2164,41 +2113,7 @@ __global__ __launch_bounds__(64 * R16_WAVES, 2) void linear_nvfp4_rows16_kernel(
   for (int d = 0; d < R16_DEPTH; ++d)
     if (t + d < cnt) multiply(ring[d], t + d);
 
-  // lane (r, g): activation row r of tile i, weight rows 4 g .. 4 g + 3
-#pragma unroll
-  for (int i = 0; i < MT; ++i) {
-    const f32x4 v = acc[i][0] + acc[i][1];
-    part[wave][i][lane] = make_float4(v[0], v[1], v[2], v[3]);
-  }
-  __syncthreads();
-  if (wave >= MT) return;
-  float4 v = part[0][wave][lane];
-#pragma unroll
-  for (int q = 1; q < R16_WAVES; ++q) {
-    const float4 o = part[q][wave][lane];
-    v.x += o.x, v.y += o.y, v.z += o.z, v.w += o.w;
-  }
-  const int m = wave * 16 + r;
-  const int64_t n = n0 + g * 4;
-  if (m >= (int)a.M || n >= a.N) return;
-  using DE = Elem<D_DT>;
-  const float scale = (*a.A_gs) * (*a.B_gs);
-  float o[4] = {v.x * scale, v.y * scale, v.z * scale, v.w * scale};
-  if constexpr (BIAS_DT != BIAS_NONE) {
-#pragma unroll
-    for (int q = 0; q < 4; ++q) o[q] += n + q < a.N ? Elem<BIAS_DT>::load(a.bias, n + q) : 0.0f;
-  }
-  typename DE::T *dst = static_cast<typename DE::T *>(a.D) + (int64_t)m * a.N + n;
-  if ((a.N & 3) == 0 && ((uintptr_t)a.D & 15) == 0) {
-    if constexpr (sizeof(typename DE::T) == 2)
-      *reinterpret_cast<uint2 *>(dst) = make_uint2(DE::cvt2(o[0], o[1]), DE::cvt2(o[2], o[3]));
-    else
-      *reinterpret_cast<float4 *>(dst) = make_float4(o[0], o[1], o[2], o[3]);
-  } else {
-#pragma unroll
-    for (int q = 0; q < 4; ++q)
-      if (n + q < a.N) dst[q] = DE::cvt(o[q]);
-  }
+  rows16_finish<D_DT, BIAS_DT, MT>(acc, part, a.D, a.bias, (*a.A_gs) * (*a.B_gs), a.M, a.N, n0);
 }
 
 // Plan of a decode-sized linear: which kernel, its K split and the fp32 scratch it needs.
@@ -2274,15 +2189,31 @@ static void plan_lds_ring(int64_t M, int64_t N, int64_t K, SkinnyPlan &p, int ro
 // a K split.  Both sides as measured (other kernel / 16 rows): M = 16, 4096 x 14336 17.8 / 11.4, 8192 x 8192 18.7 / 13.2, 10240 x 10240
 // 33.5 / 23.5, 14336 x 4096 14.2 / 12.5, 28672 x 8192 33.5 / 41.0, 16384 x 16384 42.7 / 47.0; M = 32, 4096 x 14336 18.2 / 16.6, 14336 x 4096
 // 14.5 / 17.7, 128 x 8192 7.8 / 9.8, 1000 x 1024 7.6 / 3.3; M = 1, 20480 x 8192 41.5 / 23.2, 28672 x 8192 29.2 / 30.0, 300 x 14336 7.8 / 8.8.
-static bool rows16_faster(int64_t M, int64_t N, int64_t K, const SkinnyPlan &p) {
+//
+// `start`: what they save on top of that by quantizing the activation themselves (ac4k_linear_nvfp4_fused_bf16).
+static bool rows16_faster(int64_t M, int64_t N, int64_t K, const SkinnyPlan &p, double start = 0.0) {
   const double million = 1e-6 * (double)N * (double)K, steps = (double)ceil_div(ceil_div(K, R16_STEP), R16_WAVES);
   const double stream = M <= 16 ? 0.114 + 0.0031 * (double)M : 0.150 + 0.0023 * (double)M, chain = M <= 16 ? 0.45 + 0.007 * (double)M : 0.87;
-  const double rows16 = 2.5 + fmax(stream * million, chain * steps);
+  const double rows16 = 2.5 - start + fmax(stream * million, chain * steps);
   if (p.kind == DECODE_REGISTERS)
     return rows16 < (N >= 24576 ? 7.5 + (0.0925 + 0.0018 * (double)M) * million : 5.3 + 0.15 * million);
   if (p.split_k > 1) return rows16 < 7.6 + 0.16 * million;
   const double rounds = (double)ceil_div(p.groups, (int64_t)device_cu_count());
   return rows16 < rounds * (5.0 + (p.kind == DECODE_LDS_RING ? 0.88 : 0.54) * (double)ceil_div(K, ST_BK));
+}
+
+static bool forced_decode_kernel() {
+  return g_forced_decode_kernel.load(std::memory_order_relaxed) != 0 || g_forced_skinny_ks.load(std::memory_order_relaxed) != 0;
+}
+
+// Shapes whose fused call runs one launch: the activation fits into the registers and the LDS of a workgroup, and 16-row workgroups are
+// faster than the other kernels with the quantizer's launch in front of these.  Every workgroup quantizes all of it, which costs the
+// more beside its 16 weight rows the more rows the activation has; in a grid of two rounds and less that is hidden (us in a graph,
+// two launches / one: 8 x 28672 x 2048 15.6 / 17.7, 16 x 28672 x 1024 11.5 / 14.6; 4 x 28672 x 4096 22.2 / 21.5, 8 x 6144 x 2048 8.0 / 7.3,
+// 32 x 8192 x 512 6.7 / 6.1).
+static bool fused_rows16(int64_t M, int64_t N, int64_t K, const SkinnyPlan &p) {
+  if (M * K > FUSED_ELEMS || K % R16_STEP != 0 || N >= (1ll << 27) || forced_decode_kernel()) return false;
+  return (M <= 4 || ceil_div(N, R16_ROWS) <= 2 * (int64_t)device_cu_count()) && rows16_faster(M, N, K, p, 2.5);
 }
 
 static bool skinny_plan(int64_t M, int64_t N, int64_t K, SkinnyPlan &p) {
@@ -2305,8 +2236,7 @@ static bool skinny_plan(int64_t M, int64_t N, int64_t K, SkinnyPlan &p) {
     plan_lds_ring(M, N, K, p);
   else
     plan_registers(M, N, K, p);
-  const bool forced = g_forced_decode_kernel.load(std::memory_order_relaxed) != 0 || g_forced_skinny_ks.load(std::memory_order_relaxed) != 0;
-  p.rows16 = !forced && ring_ok && rows16_faster(M, N, K, p);  // (32-bit lane offsets, as in the ring kernels)
+  p.rows16 = !forced_decode_kernel() && ring_ok && rows16_faster(M, N, K, p);  // (32-bit lane offsets, as in the ring kernels)
   return true;
 }
 
@@ -2870,6 +2800,12 @@ extern "C" __attribute__((visibility("default"))) int ac4k_linear_nvfp4_fused_bf
   if (int rc = check_skinny(p, ok, B, workspace, workspace_bytes)) return rc;
   hipStream_t st = (hipStream_t)stream;
   AC4K_REQUIRE(((uintptr_t)X & 15) == 0, "activation must be 16-byte aligned");
+  if (fused_rows16(M, N, K, p) && (((uintptr_t)X_q | (uintptr_t)B) & 15) == 0 && (((uintptr_t)X_sf | (uintptr_t)B_sf) & 3) == 0) {
+    const FusedArgs a{D, static_cast<const uint16_t *>(X), static_cast<uint8_t *>(X_q), static_cast<uint8_t *>(X_sf), X_gs,
+                      static_cast<const uint8_t *>(B), static_cast<const uint32_t *>(B_sf), B_gs, bias, M, N, K, align_up(M, 16), align_up(N, 16)};
+    if (int rc = launch_fused_rows16(a, d_dtype, bias_dtype, st)) return rc;
+    return check_launch("ac4k_linear_nvfp4_fused_bf16");
+  }
   if (int rc = ac4k_quantize_nvfp4_bf16(X_q, X_sf, X_gs, X, 1, 1, M, K, 0, 0, K, 1, 0, 2688.0f, stream)) return rc;
   if (int rc = run_skinny(D, d_dtype, X_q, X_sf, X_gs, B, B_sf, B_gs, bias, bias_dtype, M, N, K, p, workspace,
                           st))

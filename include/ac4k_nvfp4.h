@@ -216,7 +216,7 @@ int ac4k_linear_nvfp4_prepacked(void *D, int d_dtype, const void *A, const void 
 /* Fused decode-sized linear: quantize(X,0,1) followed by linear(...) in one call.  No single
  * reference function: it equals the composition the reference's tests make
  * (test/test_linear_bench.py:128-137) — the activation bytes, scales and global scale it
- * produces are those of ac4k_quantize_nvfp4_bf16 (it is that call), and they are returned:
+ * produces are those of ac4k_quantize_nvfp4_bf16, bit for bit, and they are returned:
  * X bf16 [M,K] contiguous -> X_q [M,K/2], X_sf [K/64,align_up(M,16),4], X_gs (1 float).
  * workspace as for ac4k_linear_nvfp4_skinny. */
 int ac4k_linear_nvfp4_fused_bf16(void *D, int d_dtype, const void *X, void *X_q, void *X_sf,

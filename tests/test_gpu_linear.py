@@ -157,6 +157,28 @@ def test_fused_skinny_equals_composition(m, n, k):
     assert torch.equal(d, comp)  # same packed activation, same kernel arithmetic, same slice order
 
 
+# one launch: activations of 16384 elements and just above, one and two tiles of rows, threads with two blocks, one and none, waves
+# without a step; weights that the other decode kernels would take from an activation quantized beforehand
+@pytest.mark.parametrize("m,k", [(1, 256), (1, 8192), (1, 16384), (2, 8192), (3, 5376), (15, 1024), (16, 1024), (17, 768), (31, 512), (32, 512),
+                                 (2, 8448), (32, 768)])
+@pytest.mark.parametrize("n", [1, 130, 4099])
+def test_fused_in_one_launch(m, k, n):
+    x = make_input((m, k), seed=m + k, outliers=True)
+    wq = gpu_quant(make_input((n, k), seed=n, std=0.02))
+    eq, esf, egs = T.quantize_nvfp4(x, 0, 1)
+    for dt, bdt in ((torch.bfloat16, None), (torch.float16, torch.float32), (torch.float32, torch.bfloat16)):
+        bias = None if bdt is None else make_input((1, n), seed=7).to(bdt)
+        buf = torch.full((m * n + 2,), 7.0, dtype=dt, device="cuda")
+        d, (xq, xsf, xgs) = ops().fused_linear(x.cuda(), *wq, bias=None if bias is None else bias.cuda(), out=buf[1:1 + m * n].view(m, n),
+                                               return_quantized=True)
+        assert torch.equal(xq.cpu(), eq) and torch.equal(xsf.cpu().view(torch.uint8), esf) and xgs.item() == egs.item()
+        ref = T.linear_nvfp4(eq, esf, egs, *cpu(wq), bias=bias, out_dtype=dt)
+        torch.testing.assert_close(d.cpu(), ref, atol=ATOL, rtol=RTOL)
+        assert buf[0] == 7.0 and buf[-1] == 7.0
+    comp = ops().linear(xq, xsf, xgs, *wq, bias=bias.cuda(), out=torch.empty((m, n), device="cuda"))
+    torch.testing.assert_close(d, comp, atol=1e-5, rtol=1e-4)
+
+
 def test_more_than_2_to_31_outputs():
     """An output of 2.15e9 elements: element offsets past 32 bits in the epilogue.  Sampled rows and a
     band of the last columns against the fp32 dequantize-matmul (on the GPU: the oracle would take
