@@ -2116,6 +2116,12 @@ __global__ __launch_bounds__(64 * R16_WAVES, 2) void linear_nvfp4_rows16_kernel(
   rows16_finish<D_DT, BIAS_DT, MT>(acc, part, a.D, a.bias, (*a.A_gs) * (*a.B_gs), a.M, a.N, n0);
 }
 
+// CUs that the decode plans count on; a process without a GPU may ask for scratch sizes, too
+static int64_t decode_cu_count() {
+  const int n = device_cu_count();
+  return n > 0 ? n : 256;
+}
+
 // Plan of a decode-sized linear: which kernel, its K split and the fp32 scratch it needs.
 enum { DECODE_REGISTERS = 1, DECODE_LDS_RING = 2, DECODE_LDS_RING64 = 3 };
 struct SkinnyPlan {
@@ -2198,7 +2204,7 @@ static bool rows16_faster(int64_t M, int64_t N, int64_t K, const SkinnyPlan &p, 
   if (p.kind == DECODE_REGISTERS)
     return rows16 < (N >= 24576 ? 7.5 + (0.0925 + 0.0018 * (double)M) * million : 5.3 + 0.15 * million);
   if (p.split_k > 1) return rows16 < 7.6 + 0.16 * million;
-  const double rounds = (double)ceil_div(p.groups, (int64_t)device_cu_count());
+  const double rounds = (double)ceil_div(p.groups, decode_cu_count());
   return rows16 < rounds * (5.0 + (p.kind == DECODE_LDS_RING ? 0.88 : 0.54) * (double)ceil_div(K, ST_BK));
 }
 
@@ -2213,7 +2219,7 @@ static bool forced_decode_kernel() {
 // 32 x 8192 x 512 6.7 / 6.1).
 static bool fused_rows16(int64_t M, int64_t N, int64_t K, const SkinnyPlan &p) {
   if (M * K > FUSED_ELEMS || K % R16_STEP != 0 || N >= (1ll << 27) || forced_decode_kernel()) return false;
-  return (M <= 4 || ceil_div(N, R16_ROWS) <= 2 * (int64_t)device_cu_count()) && rows16_faster(M, N, K, p, 2.5);
+  return (M <= 4 || ceil_div(N, R16_ROWS) <= 2 * decode_cu_count()) && rows16_faster(M, N, K, p, 2.5);
 }
 
 static bool skinny_plan(int64_t M, int64_t N, int64_t K, SkinnyPlan &p) {

@@ -180,3 +180,18 @@ def test_attention_operands_and_workspace_are_checked():
         assert bytes_(1, 2, 64, 64, 7, 64) == -1 and bytes_(1, 2, 64, 64, 64, 129) == -1 and bytes_(0, 2, 64, 64, 64, 64) == -1
     for gap in ((8192, 4096, 65), (8192, 4097, 64)):  # the NVFP4 maxima are taken over whole tensors
         assert call(k=gap) != 0 and b"dense" in lib.ac4k_last_error()
+
+
+def test_scratch_sizes_of_every_plan_without_gpu():
+    """The sizes are pure functions of the shape: decode-sized, K-split and tile plans answer without a GPU, and what a linear
+    writes is nothing or all of what it asks for.  Three sizes that callers may have kept."""
+    from ac4k_kernel_amd import _lib
+    lib = _lib.load()
+    for m in (1, 2, 8, 16, 17, 32, 33, 64, 100, 128, 129, 200, 300, 1001, 4096):
+        for n in (1, 128, 1000, 4096, 14336, 28672, 65536):
+            for k in (64, 256, 320, 1024, 2880, 4096, 14336):
+                asked = lib.ac4k_linear_nvfp4_workspace_bytes(m, n, k)
+                assert lib.ac4k_linear_nvfp4_scratch_bytes(m, n, k) in (0, asked)
+                assert lib.ac4k_linear_nvfp4_prepacked_workspace_bytes(m, n, k) >= 0
+    sizes = [lib.ac4k_linear_nvfp4_workspace_bytes(*s) for s in ((512, 4096, 14336), (150, 4096, 4096), (16, 4096, 14336))]
+    assert sizes == [33554432, 9830400, 1048576]
