@@ -29,6 +29,7 @@ SIGNATURES = {
     "ac4k_quantize_int8": (_int, [_vp, _vp, _vp, _vp] + [_i64] * 8 + [_vp]),
     "ac4k_linear_nvfp4": (_int, [_vp, _int, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _int, _i64, _i64, _i64, _vp]),
     "ac4k_linear_nvfp4_workspace_bytes": (_i64, [_i64, _i64, _i64]),
+    "ac4k_debug_linear_decode_kernel": (_int, [_i64, _i64, _i64, _vp]),
     "ac4k_linear_nvfp4_scratch_bytes": (_i64, [_i64, _i64, _i64]),
     "ac4k_linear_nvfp4_workspace": (_int, [_vp, _int, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _int, _i64, _i64, _i64,
                                            _vp, _i64, _vp]),

@@ -2123,7 +2123,7 @@ static int64_t decode_cu_count() {
 }
 
 // Plan of a decode-sized linear: which kernel, its K split and the fp32 scratch it needs.
-enum { DECODE_REGISTERS = 1, DECODE_LDS_RING = 2, DECODE_LDS_RING64 = 3 };
+enum { DECODE_REGISTERS = 1, DECODE_LDS_RING = 2, DECODE_LDS_RING64 = 3, DECODE_ROWS16 = 4 };
 struct SkinnyPlan {
   int kind;                // DECODE_REGISTERS: linear_nvfp4_skinny_kernel; DECODE_LDS_RING: linear_nvfp4_stream_kernel;
                            // DECODE_LDS_RING64: linear_nvfp4_stream64_kernel
@@ -2218,7 +2218,7 @@ static bool forced_decode_kernel() {
 // two launches / one: 8 x 28672 x 2048 15.6 / 17.7, 16 x 28672 x 1024 11.5 / 14.6; 4 x 28672 x 4096 22.2 / 21.5, 8 x 6144 x 2048 8.0 / 7.3,
 // 32 x 8192 x 512 6.7 / 6.1).
 static bool fused_rows16(int64_t M, int64_t N, int64_t K, const SkinnyPlan &p) {
-  if (M * K > FUSED_ELEMS || K % R16_STEP != 0 || N >= (1ll << 27) || forced_decode_kernel()) return false;
+  if (M * K > FUSED_ELEMS || K % R16_STEP != 0 || !rows16_grid_ok(N) || forced_decode_kernel()) return false;
   return (M <= 4 || ceil_div(N, R16_ROWS) <= 2 * decode_cu_count()) && rows16_faster(M, N, K, p, 2.5);
 }
 
@@ -2242,7 +2242,8 @@ static bool skinny_plan(int64_t M, int64_t N, int64_t K, SkinnyPlan &p) {
     plan_lds_ring(M, N, K, p);
   else
     plan_registers(M, N, K, p);
-  p.rows16 = !forced_decode_kernel() && ring_ok && rows16_faster(M, N, K, p);  // (32-bit lane offsets, as in the ring kernels)
+  // (ring_ok: 32-bit lane offsets, as in the ring kernels)
+  p.rows16 = !forced_decode_kernel() && ring_ok && rows16_grid_ok(N) && rows16_faster(M, N, K, p);
   return true;
 }
 
@@ -2545,6 +2546,13 @@ namespace ac4k {
 static bool skinny_entry_k(int64_t M, int64_t K) { return K % (M > 32 ? P_BK : SK_STEP) == 0; }
 
 }  // namespace ac4k
+
+extern "C" __attribute__((visibility("default"))) int ac4k_debug_linear_decode_kernel(int64_t M, int64_t N, int64_t K, int *fused_launches) {
+  SkinnyPlan p;
+  const bool ok = skinny_plan(M, N, K, p);
+  if (fused_launches) *fused_launches = !ok || !skinny_entry_k(M, K) ? 0 : fused_rows16(M, N, K, p) ? 1 : p.rows16 || p.split_k == 1 ? 2 : 3;
+  return !ok ? 0 : p.rows16 ? DECODE_ROWS16 : p.kind;
+}
 
 extern "C" __attribute__((visibility("default"))) int64_t ac4k_linear_nvfp4_skinny_workspace_bytes(int64_t M, int64_t N, int64_t K) {
   return skinny_entry_k(M, K) ? ac4k_linear_nvfp4_workspace_bytes(M, N, K) : 0;

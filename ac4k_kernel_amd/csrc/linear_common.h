@@ -58,6 +58,8 @@ __device__ __forceinline__ f16x8 decode_dword(uint32_t w, f16x2 sc2) {
 
 // --- 16 weight rows per workgroup ------------------------------------------------
 constexpr int R16_ROWS = 16, R16_WAVES = 8, R16_STEP = 128;
+// A launch carries fewer than 2^32 threads along a grid dim and drops the rest without an error: weights of up to 2^27 - 16 rows.
+static inline bool rows16_grid_ok(int64_t N) { return ceil_div(N, R16_ROWS) * (64 * R16_WAVES) < (1ll << 32); }
 
 // End of these kernels: the sums of the eight waves in the order of the waves, scale, bias, store.
 template <int D_DT, int BIAS_DT, int MT>

@@ -195,3 +195,19 @@ def test_scratch_sizes_of_every_plan_without_gpu():
                 assert lib.ac4k_linear_nvfp4_prepacked_workspace_bytes(m, n, k) >= 0
     sizes = [lib.ac4k_linear_nvfp4_workspace_bytes(*s) for s in ((512, 4096, 14336), (150, 4096, 4096), (16, 4096, 14336))]
     assert sizes == [33554432, 9830400, 1048576]
+
+
+def decode_kernel(m, n, k):
+    from ac4k_kernel_amd import _lib
+    launches = ctypes.c_int(-1)
+    return _lib.load().ac4k_debug_linear_decode_kernel(m, n, k, ctypes.byref(launches)), launches.value
+
+
+@pytest.mark.parametrize("m,k", [(1, 256), (1, 512), (1, 2048), (4, 256), (16, 256), (16, 320), (32, 256), (16, 2880)])
+def test_sixteen_row_workgroups_stay_within_a_launch(m, k):
+    """512 threads for 16 weight rows: 2^23 workgroups are 2^32 threads, more than a launch carries, and no error when it drops them."""
+    assert decode_kernel(16, 4096, 256) == (4, 1) and decode_kernel(16, 4096, 14336) == (4, 2) and decode_kernel(64, 4096, 4096) == (0, 0)
+    for n in (2 ** 27 - 15, 2 ** 27 - 8, 2 ** 27 - 1, 2 ** 27):
+        kernel, launches = decode_kernel(m, n, k)
+        assert kernel != 4 and launches != 1, n
+    assert decode_kernel(16, 2 ** 27 - 16, 256)[0] == 4  # the last that a launch carries
