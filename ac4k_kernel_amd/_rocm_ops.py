@@ -144,14 +144,6 @@ def _check_linear_operand(x, x_sf, x_gs, rows, name):
     return K
 
 
-def _skinny_scratch(device, M, N, K):
-    """Workspace tensor for the shapes that split K, or None when the shape needs no scratch."""
-    nbytes = _L.ac4k_linear_nvfp4_workspace_bytes(M, N, K)
-    if nbytes <= 0:
-        return None
-    return torch.empty((nbytes,), dtype=torch.uint8, device=device)
-
-
 def _bias_args(bias, N):
     if bias is None:
         return None, 0
@@ -180,12 +172,13 @@ def linear_nvfp4(D, A, A_sf, A_global_scale, B, B_sf, B_global_scale, bias=None)
     bias_ptr, bias_tag = _bias_args(bias, N)
     if M == 0 or N == 0:
         return
-    if _L.ac4k_linear_nvfp4_scratch_bytes(M, N, K) > 0:
-        ws = _skinny_scratch(D.device, M, N, K)
+    nbytes = _L.ac4k_linear_nvfp4_scratch_bytes(M, N, K)
+    if nbytes > 0:
+        ws = torch.empty((nbytes,), dtype=torch.uint8, device=D.device)
         _lib.check(_L.ac4k_linear_nvfp4_workspace(D.data_ptr(), _DTYPE_TAG[D.dtype], A.data_ptr(), A_sf.data_ptr(),
                                                   A_global_scale.data_ptr(), B.data_ptr(), B_sf.data_ptr(),
                                                   B_global_scale.data_ptr(), bias_ptr, bias_tag, M, N, K,
-                                                  ws.data_ptr(), ws.numel(), _stream()))
+                                                  ws.data_ptr(), nbytes, _stream()))
         return
     _lib.check(_L.ac4k_linear_nvfp4(D.data_ptr(), _DTYPE_TAG[D.dtype], A.data_ptr(), A_sf.data_ptr(),
                                     A_global_scale.data_ptr(), B.data_ptr(), B_sf.data_ptr(),
@@ -254,12 +247,12 @@ def linear_nvfp4_fused(D, X, X_q, X_sf, X_global_scale, B, B_sf, B_global_scale,
         quantize_nvfp4_with_global_scale(X_q, X_sf, X_global_scale, X, 0, 1, False, 2688.0)
         linear_nvfp4(D, X_q, X_sf, X_global_scale, B, B_sf, B_global_scale, bias)
         return
-    ws = _skinny_scratch(D.device, M, N, K)  # None: one K range per tile, no scratch
+    nbytes = _L.ac4k_linear_nvfp4_workspace_bytes(M, N, K)  # 0: one K range per tile, no scratch
+    ws = torch.empty((nbytes,), dtype=torch.uint8, device=D.device) if nbytes > 0 else None
     _lib.check(_L.ac4k_linear_nvfp4_fused_bf16(D.data_ptr(), _DTYPE_TAG[D.dtype], X.data_ptr(), X_q.data_ptr(),
                                                X_sf.data_ptr(), X_global_scale.data_ptr(), B.data_ptr(),
                                                B_sf.data_ptr(), B_global_scale.data_ptr(), bias_ptr, bias_tag,
-                                               M, N, K, None if ws is None else ws.data_ptr(),
-                                               0 if ws is None else ws.numel(), _stream()))
+                                               M, N, K, None if ws is None else ws.data_ptr(), nbytes, _stream()))
 
 
 def _check_attention_operand(x, x_sf, x_gs, B, H, rows, width, name):

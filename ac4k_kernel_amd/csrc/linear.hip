@@ -796,6 +796,22 @@ static bool forced_tile_plan(int64_t M, int64_t N, int64_t K, TilePlan &p) {
   return f != 0 && sp <= ceil_div(K, P_BK);
 }
 
+// What both estimates below use for every number of K ranges that they weigh: `most` of them, each two stages long at least (beyond
+// 32 the sums cost more than any of the measured shapes gained).
+struct SplitCosts {
+  double len[33], sums_us[33];  // stages of a range; the partial sums written and read and the second launch
+  int most;
+};
+static SplitCosts split_costs(int64_t M, int64_t N, int stages, double bytes_per_us, double launch_us, int most) {
+  SplitCosts c;
+  c.most = stages / 2 < most ? stages / 2 : most;
+  if (c.most < 1) c.most = 1;
+  c.len[1] = stages, c.sums_us[1] = 0.0;
+  const double sum_us = (double)M * (double)N * 8.0 / bytes_per_us;
+  for (int sp = 2; sp <= c.most; ++sp) c.len[sp] = (double)((stages + sp - 1) / sp), c.sums_us[sp] = sp * sum_us + launch_us;
+  return c;
+}
+
 // Scratch that the entry points ask for, for the tile kernel's partial sums; 0: they take none (and ac4k_linear_nvfp4_skinny not
 // the shape).  Callers keep these sizes, so they stay what this estimate has always given, although the plan comes from the
 // measured costs below and fits into them: on 50 shapes of M = 129 to 9000 a plan with room for any split would be faster on two,
@@ -803,8 +819,9 @@ static bool forced_tile_plan(int64_t M, int64_t N, int64_t K, TilePlan &p) {
 static int64_t tile_scratch_bytes(int64_t M, int64_t N, int64_t K) {
   TilePlan forced;
   if (forced_tile_plan(M, N, K, forced)) return forced.partial_bytes;
-  const int64_t stages = ceil_div(K, P_BK);
+  const int stages = (int)ceil_div(K, P_BK);
   if (ceil_div(M, M <= 128 ? 128 : 256) * ceil_div(N, 256) >= 192) return 0;
+  const SplitCosts c = split_costs(M, N, stages, 4.5e6, 2.5, 32);
   double best_t = 0.0;
   int64_t best = 0;
   for (int mi = 2; mi <= 4; mi += 2) {
@@ -815,11 +832,11 @@ static int64_t tile_scratch_bytes(int64_t M, int64_t N, int64_t K) {
       const int nm = mi * nj, nv = 8 * (mi + nj);
       const double stage_us = (8.0 * (14.0 * nm + 5.0 * nv) + 400.0) / 2100.0;
       const double fixed_us = 5.0 + 0.1 * nm;
-      const int64_t tiles = ceil_div(M, 64 * mi) * ceil_div(N, 64 * nj);
-      for (int64_t sp = 1; sp <= 32 && (sp == 1 || sp * 2 <= stages); ++sp) {
-        const double rounds = (double)ceil_div(tiles * sp, 256);
-        double t = rounds * (double)ceil_div(stages, sp) * stage_us + fixed_us;
-        if (sp > 1) t += (double)sp * (double)(M * N) * 8.0 / 4.5e6 + 2.5;
+      const int tiles = (int)(ceil_div(M, 64 * mi) * ceil_div(N, 64 * nj));
+      const double least = fixed_us + 0.999 * tiles * stages / 256.0 * stage_us;  // without the partial sums
+      for (int sp = 1; sp <= c.most; ++sp) {
+        if (best && least + c.sums_us[sp] >= best_t) break;  // nor will more ranges be faster
+        const double t = (double)((tiles * sp + 255) / 256) * c.len[sp] * stage_us + fixed_us + c.sums_us[sp];
         if (best == 0 || t < best_t) best_t = t, best = sp;
       }
     }
@@ -845,22 +862,25 @@ static TilePlan tile_plan(int64_t M, int64_t N, int64_t K, int64_t scratch) {
   TilePlan best{};
   if (forced_tile_plan(M, N, K, best) && best.partial_bytes <= scratch) return best;
   constexpr double ROUND_US = 3.5, SPLIT_US = 4.5, PARTIAL_BYTES_PER_US = 9.4e6;  // (8 bytes of a sum: written and read)
-  const int64_t stages = ceil_div(K, P_BK);
+  const int stages = (int)ceil_div(K, P_BK);
+  const int64_t sums_bytes = M * N * 4;
+  const SplitCosts s = split_costs(M, N, stages, PARTIAL_BYTES_PER_US, SPLIT_US, scratch / sums_bytes < 32 ? (int)(scratch / sums_bytes) : 32);
   double best_t = 0.0;
   best.splits = 0;
   for (const TileCost &c : TILE_COSTS) {
     if (c.mi > 2 && M <= 128) continue;
     if (c.nj < 4 && N < 64 * c.nj * 2) continue;
     const int64_t tiles = ceil_div(M, 64 * c.mi) * ceil_div(N, 64 * c.nj);
-    for (int64_t sp = 1; sp == 1 || (sp <= 32 && sp * 2 <= stages && tiles * sp <= 1024 && sp * M * N * 4 <= scratch); ++sp) {
-      const double len = (double)ceil_div(stages, sp);
+    const double least = c.fixed + 0.999 * (double)tiles * stages / 256.0 * c.stage;  // without the partial sums
+    for (int sp = 1; sp <= s.most && (sp == 1 || tiles * sp <= 1024); ++sp) {
+      if (best.splits && least + s.sums_us[sp] >= best_t) break;  // nor will more ranges be faster
+      const double len = s.len[sp];
       const int64_t full = tiles * sp / 256, tail = tiles * sp % 256;
-      double t = c.fixed - ROUND_US + (double)full * (len * (c.stage + 0.4 * c.power) + ROUND_US);
+      double t = c.fixed - ROUND_US + (double)full * (len * (c.stage + 0.4 * c.power) + ROUND_US) + s.sums_us[sp];
       if (tail) t += len * (c.stage + (tail > 153 ? ((double)tail / 256.0 - 0.6) * c.power : 0.0)) + ROUND_US;
-      if (sp > 1) t += SPLIT_US + (double)(sp * M * N) * 8.0 / PARTIAL_BYTES_PER_US;
       if (best.splits == 0 || t < best_t) {
         best_t = t;
-        best = TilePlan{c.mi, c.nj, (int)sp, sp > 1 ? sp * M * N * 4 : 0};
+        best = TilePlan{c.mi, c.nj, sp, sp > 1 ? sp * sums_bytes : 0};
       }
     }
   }
@@ -2420,18 +2440,21 @@ namespace ac4k {
 struct MidPlan {
   bool has_ksplit;   // the shape suits the K-split-waves kernel (taken when the pointers are aligned for it)
   KsplitPlan kp;
-  TilePlan tp;       // what the tile kernel does with the shape otherwise (given enough scratch)
+  TilePlan tp;       // the plan of the tile kernel where the shape does not
   int64_t bytes;     // scratch that the entry points ask for
 };
 // shapes the workspace entry point takes with 32 < M
 static bool mid_plan(int64_t M, int64_t N, int64_t K, MidPlan &p) {
   if (M <= 32 || N < 128 || K % 64 != 0 || K < P_BK || (K >> 1) * 256 >= (1ll << 31) || N >= (1ll << 27)) return false;
-  const int64_t tile_bytes = tile_scratch_bytes(M, N, K);
-  p.tp = tile_plan(M, N, K, tile_bytes);
   p.has_ksplit = ksplit_shape(M, N, K);
-  p.kp = p.has_ksplit ? ksplit_plan(M, N, K, true) : KsplitPlan{0, 0, 1, 0};
-  p.bytes = p.has_ksplit ? p.kp.partial_bytes : tile_bytes;
-  return p.has_ksplit || tile_bytes > 0;
+  if (p.has_ksplit) {
+    p.kp = ksplit_plan(M, N, K, true);
+    p.bytes = p.kp.partial_bytes;
+    return true;
+  }
+  p.bytes = tile_scratch_bytes(M, N, K);
+  if (p.bytes > 0) p.tp = tile_plan(M, N, K, p.bytes);
+  return p.bytes > 0;
 }
 
 // `partial_bytes` of scratch at `partial` (possibly none): the K-split-waves kernel when the shape and the
@@ -2443,7 +2466,8 @@ static int launch_mid(const LinearArgs &a, const MidPlan &p, float *partial, int
     splits = p.kp.splits;
     if (int rc = launch_ksplit<D_DT, BIAS_DT>(a, p.kp, SplitK{splits > 1 ? partial : nullptr, splits}, st)) return rc;
   } else {
-    const TilePlan tp = p.tp.partial_bytes <= partial_bytes ? p.tp : tile_plan(a.M, a.N, a.K, 0);
+    TilePlan tp = p.has_ksplit ? tile_plan(a.M, a.N, a.K, tile_scratch_bytes(a.M, a.N, a.K)) : p.tp;
+    if (tp.partial_bytes > partial_bytes) tp = tile_plan(a.M, a.N, a.K, 0);
     splits = tp.splits;
     if (int rc = launch_tile_plan<D_DT, BIAS_DT>(a, tp, SplitK{splits > 1 ? partial : nullptr, splits}, st)) return rc;
   }
@@ -2722,13 +2746,12 @@ static bool prepacked_plan(int64_t M, int64_t N, int64_t K, PrepackedPlan &p) {
     plan_lds_ring(M, N, K, p.sp);
     p.sp.rows16 = false;
     p.partial_bytes = p.sp.partial_bytes;
+  } else if (p.mid) {
+    p.kp = ksplit_plan(M, N, K, true);
+    p.partial_bytes = p.kp.partial_bytes;
   } else {
     p.partial_bytes = tile_scratch_bytes(M, N, K);
     p.tp = tile_plan(M, N, K, p.partial_bytes);
-    if (p.mid) {
-      p.kp = ksplit_plan(M, N, K, true);
-      p.partial_bytes = p.kp.partial_bytes;
-    }
   }
   return true;
 }

@@ -152,8 +152,9 @@ int ac4k_linear_nvfp4_skinny(void *D, int d_dtype, const void *A, const void *A_
  * ac4k_linear_nvfp4_workspace_bytes(M,N,K) bytes, 256-byte aligned, contents irrelevant (NULL when that is 0).  Operands
  * that are not aligned to 16 bytes (scale tensors: 4) run without scratch, like shapes that need none. */
 int64_t ac4k_linear_nvfp4_workspace_bytes(int64_t M, int64_t N, int64_t K);
-/* How many of these bytes the kernels for operands on 16 bytes write: 0 where ac4k_linear_nvfp4 runs the same kernel without a
- * workspace (some shapes ask for one and their kernels leave it alone), otherwise all of them. */
+/* What to allocate for a call: 0 where ac4k_linear_nvfp4 runs the same kernel without a workspace on operands on 16 bytes (some shapes
+ * ask for one and their kernels leave it alone), otherwise ac4k_linear_nvfp4_workspace_bytes, which ac4k_linear_nvfp4_workspace insists
+ * on (a tile plan may write fewer: 200 x 4096 x 4096 asks for 13107200 and writes 6553600). */
 int64_t ac4k_linear_nvfp4_scratch_bytes(int64_t M, int64_t N, int64_t K);
 int ac4k_linear_nvfp4_workspace(void *D, int d_dtype, const void *A, const void *A_sf, const float *A_gs,
                                 const void *B, const void *B_sf, const float *B_gs, const void *bias,

@@ -184,7 +184,8 @@ def test_attention_operands_and_workspace_are_checked():
 
 def test_scratch_sizes_of_every_plan_without_gpu():
     """The sizes are pure functions of the shape: decode-sized, K-split and tile plans answer without a GPU, and what a linear
-    writes is nothing or all of what it asks for.  Three sizes that callers may have kept."""
+    allocates is nothing or all of what the workspace entry point insists on.  Sizes that callers may have kept, and which of
+    them are not allocated: a plan of one K range, a 16-row kernel, and (all of it) a plan that writes half of what it asks for."""
     from ac4k_kernel_amd import _lib
     lib = _lib.load()
     for m in (1, 2, 8, 16, 17, 32, 33, 64, 100, 128, 129, 200, 300, 1001, 4096):
@@ -195,6 +196,39 @@ def test_scratch_sizes_of_every_plan_without_gpu():
                 assert lib.ac4k_linear_nvfp4_prepacked_workspace_bytes(m, n, k) >= 0
     sizes = [lib.ac4k_linear_nvfp4_workspace_bytes(*s) for s in ((512, 4096, 14336), (150, 4096, 4096), (16, 4096, 14336))]
     assert sizes == [33554432, 9830400, 1048576]
+    for shape, asked, taken in (((512, 4096, 14336), 33554432, 33554432), ((200, 4096, 4096), 13107200, 13107200), ((300, 4096, 4096), 9830400, 0),
+                                ((16, 4096, 14336), 1048576, 0), ((3, 337, 14336), 226464, 226464), ((64, 1024, 4096), 2097152, 2097152),
+                                ((2048, 14336, 4096), 0, 0), ((300, 4096, 4112), 0, 0)):
+        assert (lib.ac4k_linear_nvfp4_workspace_bytes(*shape), lib.ac4k_linear_nvfp4_scratch_bytes(*shape)) == (asked, taken), shape
+
+
+def test_a_linear_asks_for_its_scratch_once(monkeypatch):
+    """One size query per linear, whose answer is the size of the scratch."""
+    import torch
+    from ac4k_kernel_amd import _lib, _rocm_ops
+    lib, asked, launched = _lib.load(), [], []
+
+    class Counting:
+        def __getattr__(self, name):
+            f = getattr(lib, name)
+            if name.endswith("_bytes"):
+                return lambda *a: asked.append((name, f(*a))) or asked[-1][1]
+            return lambda *a: launched.append((name, a)) or 0
+
+    class OnGpu(torch.Tensor):  # passes the device checks; nothing is launched on it
+        is_cuda = True
+
+    monkeypatch.setattr(_rocm_ops, "_L", Counting())
+    monkeypatch.setattr(_rocm_ops, "_stream", lambda: 0)
+    t = lambda shape, dtype: torch.zeros(shape, dtype=dtype).as_subclass(OnGpu)  # noqa: E731
+    for m, n, k, size in ((64, 1024, 4096, 2097152), (200, 4096, 4096, 13107200), (16, 1024, 2048, 0)):
+        asked.clear(), launched.clear()
+        gs = t((), torch.float32)
+        operand = lambda rows: (t((rows, k // 2), torch.uint8), t((k // 64, -(-rows // 16) * 16, 4), torch.float8_e4m3fn), gs)  # noqa: E731
+        _rocm_ops.linear_nvfp4(t((m, n), torch.bfloat16), *operand(m), *operand(n))
+        assert [size] == [b for _, b in asked] and len(launched) == 1
+        name, args = launched[0]
+        assert (name, args[-2]) == (("ac4k_linear_nvfp4_workspace", size) if size else ("ac4k_linear_nvfp4", k))
 
 
 def decode_kernel(m, n, k):
