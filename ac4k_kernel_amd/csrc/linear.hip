@@ -2825,6 +2825,14 @@ extern "C" __attribute__((visibility("default"))) int ac4k_linear_nvfp4_prepacke
   return check_launch("ac4k_linear_nvfp4_prepacked");
 }
 
+namespace ac4k {
+
+static bool overlap(const void *a, int64_t a_bytes, const void *b, int64_t b_bytes) {
+  return (uintptr_t)a < (uintptr_t)b + (uintptr_t)b_bytes && (uintptr_t)b < (uintptr_t)a + (uintptr_t)a_bytes;
+}
+
+}  // namespace ac4k
+
 extern "C" __attribute__((visibility("default"))) int ac4k_linear_nvfp4_fused_bf16(void *D, int d_dtype, const void *X, void *X_q, void *X_sf,
                                             float *X_gs, const void *B, const void *B_sf, const float *B_gs,
                                             const void *bias, int bias_dtype, int64_t M, int64_t N, int64_t K,
@@ -2837,7 +2845,10 @@ extern "C" __attribute__((visibility("default"))) int ac4k_linear_nvfp4_fused_bf
   if (int rc = check_skinny(p, ok, B, workspace, workspace_bytes)) return rc;
   hipStream_t st = (hipStream_t)stream;
   AC4K_REQUIRE(((uintptr_t)X & 15) == 0, "activation must be 16-byte aligned");
-  if (fused_rows16(M, N, K, p) && (((uintptr_t)X_q | (uintptr_t)B) & 15) == 0 && (((uintptr_t)X_sf | (uintptr_t)B_sf) & 3) == 0) {
+  // (one launch reads X to its end while it stores: outputs over X, as in a linear in place, need the order of two)
+  if (fused_rows16(M, N, K, p) && (((uintptr_t)X_q | (uintptr_t)B) & 15) == 0 && (((uintptr_t)X_sf | (uintptr_t)B_sf) & 3) == 0 &&
+      !overlap(X, M * K * 2, D, M * N * (d_dtype == AC4K_DTYPE_FP32 ? 4 : 2)) && !overlap(X, M * K * 2, X_q, M * K / 2) &&
+      !overlap(X, M * K * 2, X_sf, K / 64 * align_up(M, 16) * 4) && !overlap(X, M * K * 2, X_gs, 4)) {
     const FusedArgs a{D, static_cast<const uint16_t *>(X), static_cast<uint8_t *>(X_q), static_cast<uint8_t *>(X_sf), X_gs,
                       static_cast<const uint8_t *>(B), static_cast<const uint32_t *>(B_sf), B_gs, bias, M, N, K, align_up(M, 16), align_up(N, 16)};
     if (int rc = launch_fused_rows16(a, d_dtype, bias_dtype, st)) return rc;

@@ -179,6 +179,19 @@ def test_fused_in_one_launch(m, k, n):
     torch.testing.assert_close(d, comp, atol=1e-5, rtol=1e-4)
 
 
+# the output over the activation, as in a linear in place, or over a part of it: the activation is quantized before anything is stored
+@pytest.mark.parametrize("m,n,k,at", [(1, 4096, 4096, 0), (4, 1024, 1024, 0), (16, 1024, 1024, 0), (1, 2048, 4096, 2048), (1, 8192, 4096, 0),
+                                      (2, 4096, 4096, 4096)])
+def test_fused_output_over_the_activation(m, n, k, at):
+    wq = gpu_quant(make_input((n, k), seed=n, std=0.02))
+    for seed in range(3):
+        buf = torch.zeros(m * max(k, n) + at, dtype=torch.bfloat16, device="cuda")
+        x, out = buf[:m * k].view(m, k), buf[at:at + m * n].view(m, n)
+        x.copy_(make_input((m, k), seed=seed, outliers=True))
+        want = ops().linear(*ops().quantize(x, 0, 1), *wq)
+        assert torch.equal(ops().fused_linear(x, *wq, out=out), want), seed
+
+
 def test_more_than_2_to_31_outputs():
     """An output of 2.15e9 elements: element offsets past 32 bits in the epilogue.  Sampled rows and a
     band of the last columns against the fp32 dequantize-matmul (on the GPU: the oracle would take
