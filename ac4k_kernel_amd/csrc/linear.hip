@@ -364,6 +364,7 @@ __device__ __forceinline__ void store_tile(const f32x16 (&acc)[MI][NJ], char *ld
   const uint32_t lane_off = (uint32_t)(lrow * row_bytes) + lq * 16;
   char *out0 = reinterpret_cast<char *>(Dp) + (m0 * N + n0) * S;  // wave-uniform
   const bool interior = m0 + 32 * MI <= M && n0 + WN <= N;
+  const bool whole = N % (16 / S) == 0 || n0 + WN <= N;  // no piece is cut: rows past M and pieces past N are left out
   const int64_t cl = N - n0 - lq * (16 / S);
   const int cols_left = cl > 16 / S ? 16 / S : (int)cl;  // columns of this lane's piece inside the matrix
   const int64_t rl = M - m0 - lrow;
@@ -396,8 +397,16 @@ __device__ __forceinline__ void store_tile(const f32x16 (&acc)[MI][NJ], char *ld
 #pragma unroll
       for (int it = 0; it < RP / RS; ++it)
         *reinterpret_cast<u32x4_elem *>(rowp + it * RS * row_bytes + lane_off) = *reinterpret_cast<const u32x4 *>(src + it * RS * PITCH);
-    } else {
+    } else if (whole) {
 #pragma unroll
+      for (int it = 0; it < RP / RS; ++it) {
+        const u32x4 v = *reinterpret_cast<const u32x4 *>(src + it * RS * PITCH);
+        if (cols_left > 0 && p * RP + it * RS < rows_left) *reinterpret_cast<u32x4_elem *>(rowp + it * RS * row_bytes + lane_off) = v;
+      }
+    } else {
+      // (unrolled by four for the small tiles: with all of it 128 x 128 tiles ran 2 % longer, also where no piece is cut - 256 x 4096 x 4096
+      // 34.7 -> 33.7 us, 34.3 before there were pieces -; the larger ones lose 0.5 % by it)
+#pragma unroll(MI * NJ <= 4 ? 4 : RP / RS)
       for (int it = 0; it < RP / RS; ++it) {
         const u32x4 v = *reinterpret_cast<const u32x4 *>(src + it * RS * PITCH);
         if (cols_left > 0 && p * RP + it * RS < rows_left) store_piece<S>(rowp + it * RS * row_bytes + lane_off, v, cols_left);
