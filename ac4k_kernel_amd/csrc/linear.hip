@@ -823,8 +823,7 @@ static SplitCosts split_costs(int64_t M, int64_t N, int stages, double bytes_per
 
 // Scratch that the entry points ask for, for the tile kernel's partial sums; 0: they take none (and ac4k_linear_nvfp4_skinny not
 // the shape).  Callers keep these sizes, so they stay what this estimate has always given, although the plan comes from the
-// measured costs below and fits into them: on 50 shapes of M = 129 to 9000 a plan with room for any split would be faster on two,
-// 150 x 4096 x 4096 21.3 -> 20.8 us and 129 x 14336 x 4096 34.5 -> 32.1.
+// measured costs below and fits into them.
 static int64_t tile_scratch_bytes(int64_t M, int64_t N, int64_t K) {
   TilePlan forced;
   if (forced_tile_plan(M, N, K, forced)) return forced.partial_bytes;
@@ -856,21 +855,25 @@ static int64_t tile_scratch_bytes(int64_t M, int64_t N, int64_t K) {
 // Picks the tile and the K split by measured costs in microseconds on 256 CUs, with at most `scratch` bytes of partial sums:
 // rounds of 256 workgroups, stages per range times the time of a 128-k stage of that tile, a prologue and epilogue per round
 // and for more than one range the partial sums and the second launch.  A stage takes `stage` as long as up to three fifths of the
-// CUs have work and grows with their share from there to stage + 0.4 power, as the clock comes down.  Fitted to 50 shapes of
-// M = 129 to 9000, N = 256 to 28672, K = 512 to 14336 with every tile and up to twelve ranges; of the plans that fit the scratch it
-// takes the fastest everywhere to 0.5 %.  The tiles of 192 rows are what fills a round where 128 or 256 rows leave CUs idle (us, best
-// of the other tiles / with them): 4096 x 5120 x 5120 197.5 / 180.9, 7000 x 5120 x 5120 328.4 / 284.6, 6000 x 4096 x 4096 171.5 / 157.6,
-// 300 x 14336 x 4096 50.9 / 45.3, 1001 x 5003 x 2880 40.1 / 38.4, 180 x 20000 x 1024 17.7 / 16.9.
+// CUs have work and grows with their share from there to stage + 0.4 power, as the clock comes down.  Fitted to 1000 random shapes of
+// M = 129 to 12000, N = 256 to 28672, K = 256 to 14336 with every tile and up to 32 ranges that fit the scratch (750 of them; the others
+// alike), and checked on 431 more: on average 0.3 % slower than the fastest of these plans, and on six of the 431 by 2 to 5 % slower than
+// the plan of tile_scratch_bytes, which on average is 3 % slower than the fastest and at most 36 %.  (Fitted to 50 shapes before: 0.5 %,
+// and 19 slower by 2 to 11 %, short K and few tiles above all: 285 x 504 x 1280 12.3 us, 11.0 with five ranges; 437 x 3968 x 6720 42.0
+// and 38.6.)  The sweeps held up to four rounds of
+// workgroups and 32 ranges, and so does the plan.
+// The tiles of 192 rows are what fills a round where 128 or 256 rows leave CUs idle (us, best of the other tiles / with
+// them): 4096 x 5120 x 5120 197.5 / 180.9, 7000 x 5120 x 5120 328.4 / 284.6, 6000 x 4096 x 4096 171.5 / 157.6, 300 x 14336 x 4096 50.9 / 45.3.
 struct TileCost {
   int mi, nj;
   double stage, power, fixed;
 };
-constexpr TileCost TILE_COSTS[] = {{4, 4, 2.05, 2.1, 9.2},   {3, 4, 1.65, 1.5, 8.9}, {4, 2, 1.295, 0.83, 7.2}, {2, 4, 1.3, 0.9, 8.2},
-                                   {3, 2, 1.08, 0.57, 7.8}, {2, 2, 0.865, 0.28, 6.7}, {2, 1, 0.6, 0.15, 5.2}};
+constexpr TileCost TILE_COSTS[] = {{4, 4, 2.05, 2.015, 9.02},    {3, 4, 1.674, 1.595, 8.74}, {4, 2, 1.319, 0.798, 7.434}, {2, 4, 1.294, 0.908, 7.6},
+                                   {3, 2, 1.104, 0.584, 7.455}, {2, 2, 0.88, 0.257, 7.583}, {2, 1, 0.593, 0.139, 6.231}};
 static TilePlan tile_plan(int64_t M, int64_t N, int64_t K, int64_t scratch) {
   TilePlan best{};
   if (forced_tile_plan(M, N, K, best) && best.partial_bytes <= scratch) return best;
-  constexpr double ROUND_US = 3.5, SPLIT_US = 4.5, PARTIAL_BYTES_PER_US = 9.4e6;  // (8 bytes of a sum: written and read)
+  constexpr double ROUND_US = 3.29, SPLIT_US = 2.98, PARTIAL_BYTES_PER_US = 10.3e6;  // (8 bytes of a sum: written and read)
   const int stages = (int)ceil_div(K, P_BK);
   const int64_t sums_bytes = M * N * 4;
   const SplitCosts s = split_costs(M, N, stages, PARTIAL_BYTES_PER_US, SPLIT_US, scratch / sums_bytes < 32 ? (int)(scratch / sums_bytes) : 32);
