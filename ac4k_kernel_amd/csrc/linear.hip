@@ -2166,6 +2166,7 @@ struct SkinnyPlan {
   // linear_nvfp4_rows16_kernel runs instead, and needs no scratch.  The rest of the plan is what the entry points go on asking of
   // their callers for these shapes.
   bool rows16;
+  bool fused;  // and so it does, with the quantizer in it, in a fused call
 };
 static std::atomic<int> g_forced_decode_kernel{0};  // ac4k_set_linear_tuning: 0 = by shape
 
@@ -2222,14 +2223,14 @@ static void plan_lds_ring(int64_t M, int64_t N, int64_t K, SkinnyPlan &p, int ro
 // 256 takes the ring kernels for every M.
 //
 // 16-row workgroups take what they are faster at by these estimates (us, weights from HBM, fitted to 27 shapes of N = 128 to 57344,
-// K = 512 to 16384 and M = 1 to 32; 2^-20 weights = "million").  They grow with M, which the ring kernels hardly notice, and a wave
+// K = 512 to 16384 and M = 1 to 32; `million`: of weights).  They grow with M, which the ring kernels hardly notice, and a wave
 // has its steps of K one after the other; the ring kernels run in whole rounds of workgroups and, like the register kernel, pay for
 // a K split.  Both sides as measured (other kernel / 16 rows): M = 16, 4096 x 14336 17.8 / 11.4, 8192 x 8192 18.7 / 13.2, 10240 x 10240
 // 33.5 / 23.5, 14336 x 4096 14.2 / 12.5, 28672 x 8192 33.5 / 41.0, 16384 x 16384 42.7 / 47.0; M = 32, 4096 x 14336 18.2 / 16.6, 14336 x 4096
 // 14.5 / 17.7, 128 x 8192 7.8 / 9.8, 1000 x 1024 7.6 / 3.3; M = 1, 20480 x 8192 41.5 / 23.2, 28672 x 8192 29.2 / 30.0, 300 x 14336 7.8 / 8.8.
 //
-// `start`: what they save on top of that by quantizing the activation themselves (ac4k_linear_nvfp4_fused_bf16).
-static bool rows16_faster(int64_t M, int64_t N, int64_t K, const SkinnyPlan &p, double start = 0.0) {
+// `start`: what a fused call saves by quantizing the activation in these workgroups.
+static bool rows16_faster(int64_t M, int64_t N, int64_t K, const SkinnyPlan &p, double start) {
   const double million = 1e-6 * (double)N * (double)K, steps = (double)ceil_div(ceil_div(K, R16_STEP), R16_WAVES);
   const double stream = M <= 16 ? 0.114 + 0.0031 * (double)M : 0.150 + 0.0023 * (double)M, chain = M <= 16 ? 0.45 + 0.007 * (double)M : 0.87;
   const double rows16 = 2.5 - start + fmax(stream * million, chain * steps);
@@ -2249,9 +2250,13 @@ static bool forced_decode_kernel() {
 // more beside its 16 weight rows the more rows the activation has; in a grid of two rounds and less that is hidden (us in a graph,
 // two launches / one: 8 x 28672 x 2048 15.6 / 17.7, 16 x 28672 x 1024 11.5 / 14.6; 4 x 28672 x 4096 22.2 / 21.5, 8 x 6144 x 2048 8.0 / 7.3,
 // 32 x 8192 x 512 6.7 / 6.1).
+//
+// A fused call is quantize and linear bit for bit, so a linear of these shapes takes the 16-row kernel, too, also where that is up to 2.5 us
+// slower by the estimate: M = 1 or 2 on few rows of long K and on N >= 24576, K >= 8192.  Linear alone in a graph, weights from HBM, register
+// kernel / 16 rows: 1 x 256 x 8192 7.1 / 6.3, 1 x 512 x 12288 8.0 / 8.3, 1 x 1024 x 12288 9.3 / 8.5, 1 x 1024 x 16384 10.3 / 10.6, 1 x 1536 x 16384
+// 11.3 / 10.8, 2 x 512 x 8192 7.3 / 6.4; 1 x 28672 x 8192 31.1 / 31.5, 1 x 24576 x 10240 35.2 / 35.8, 1 x 28672 x 10240 38.7 / 40.3.
 static bool fused_rows16(int64_t M, int64_t N, int64_t K, const SkinnyPlan &p) {
-  if (M * K > FUSED_ELEMS || K % R16_STEP != 0 || !rows16_grid_ok(N) || forced_decode_kernel()) return false;
-  return (M <= 4 || ceil_div(N, R16_ROWS) <= 2 * decode_cu_count()) && rows16_faster(M, N, K, p, 2.5);
+  return M * K <= FUSED_ELEMS && K % SK_STEP == 0 && (M <= 4 || ceil_div(N, R16_ROWS) <= 2 * decode_cu_count()) && rows16_faster(M, N, K, p, 2.5);
 }
 
 static bool skinny_plan(int64_t M, int64_t N, int64_t K, SkinnyPlan &p) {
@@ -2275,7 +2280,9 @@ static bool skinny_plan(int64_t M, int64_t N, int64_t K, SkinnyPlan &p) {
   else
     plan_registers(M, N, K, p);
   // (ring_ok: 32-bit lane offsets, as in the ring kernels)
-  p.rows16 = !forced_decode_kernel() && ring_ok && rows16_grid_ok(N) && rows16_faster(M, N, K, p);
+  const bool rows16_ok = !forced_decode_kernel() && ring_ok && rows16_grid_ok(N);
+  p.fused = rows16_ok && fused_rows16(M, N, K, p);
+  p.rows16 = p.fused || (rows16_ok && rows16_faster(M, N, K, p, 0.0));
   return true;
 }
 
@@ -2586,7 +2593,7 @@ static bool skinny_entry_k(int64_t M, int64_t K) { return K % (M > 32 ? P_BK : S
 extern "C" __attribute__((visibility("default"))) int ac4k_debug_linear_decode_kernel(int64_t M, int64_t N, int64_t K, int *fused_launches) {
   SkinnyPlan p;
   const bool ok = skinny_plan(M, N, K, p);
-  if (fused_launches) *fused_launches = !ok || !skinny_entry_k(M, K) ? 0 : fused_rows16(M, N, K, p) ? 1 : p.rows16 || p.split_k == 1 ? 2 : 3;
+  if (fused_launches) *fused_launches = !ok || !skinny_entry_k(M, K) ? 0 : p.fused ? 1 : p.rows16 || p.split_k == 1 ? 2 : 3;
   return !ok ? 0 : p.rows16 ? DECODE_ROWS16 : p.kind;
 }
 
@@ -2756,7 +2763,7 @@ static bool prepacked_plan(int64_t M, int64_t N, int64_t K, PrepackedPlan &p) {
   p.mid = !p.ring && ksplit_shape(M, N, K);
   if (p.ring) {
     plan_lds_ring(M, N, K, p.sp);
-    p.sp.rows16 = false;
+    p.sp.rows16 = p.sp.fused = false;
     p.partial_bytes = p.sp.partial_bytes;
   } else if (p.mid) {
     p.kp = ksplit_plan(M, N, K, true);
@@ -2858,7 +2865,7 @@ extern "C" __attribute__((visibility("default"))) int ac4k_linear_nvfp4_fused_bf
   hipStream_t st = (hipStream_t)stream;
   AC4K_REQUIRE(((uintptr_t)X & 15) == 0, "activation must be 16-byte aligned");
   // (one launch reads X to its end while it stores: outputs over X, as in a linear in place, need the order of two)
-  if (fused_rows16(M, N, K, p) && (((uintptr_t)X_q | (uintptr_t)B) & 15) == 0 && (((uintptr_t)X_sf | (uintptr_t)B_sf) & 3) == 0 &&
+  if (p.fused && (((uintptr_t)X_q | (uintptr_t)B) & 15) == 0 && (((uintptr_t)X_sf | (uintptr_t)B_sf) & 3) == 0 &&
       !overlap(X, M * K * 2, D, M * N * (d_dtype == AC4K_DTYPE_FP32 ? 4 : 2)) && !overlap(X, M * K * 2, X_q, M * K / 2) &&
       !overlap(X, M * K * 2, X_sf, K / 64 * align_up(M, 16) * 4) && !overlap(X, M * K * 2, X_gs, 4)) {
     const FusedArgs a{D, static_cast<const uint16_t *>(X), static_cast<uint8_t *>(X_q), static_cast<uint8_t *>(X_sf), X_gs,

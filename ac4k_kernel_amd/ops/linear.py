@@ -39,7 +39,7 @@ _LINEAR_OP = Ac4kLinearOp()
 
 def fused_linear(x, weight, weight_scale, weight_global_scale, bias=None, out=None, return_quantized=False):
     """Decode-sized linear on a bf16 activation x [M, K], 1 <= M <= 32, K % 64 == 0:
-    equals linear(*quantize(x, 0, 1), weight, weight_scale, weight_global_scale, bias, out)."""
+    equals linear(*quantize(x, 0, 1), weight, weight_scale, weight_global_scale, bias, out) bit for bit."""
     m, k = x.shape
     n = weight.shape[0]
     dev = x.device
@@ -57,9 +57,9 @@ def fused_linear(x, weight, weight_scale, weight_global_scale, bias=None, out=No
 
 
 def linear_prepacked(x, x_scale, x_global_scale, weight_image, weight_global_scale, bias=None, out=None, n=None):
-    """`linear` on a weight image from `prepack_weight(weight, weight_scale)`: same result as
-    linear(x, x_scale, x_global_scale, weight, weight_scale, weight_global_scale, bias, out).  The image
-    does not carry N: pass `out` or `n`."""
+    """`linear` on a weight image from `prepack_weight(weight, weight_scale)`: the result of
+    linear(x, x_scale, x_global_scale, weight, weight_scale, weight_global_scale, bias, out), for M <= 32 up to
+    the order of its fp32 sums.  The image does not carry N: pass `out` or `n`."""
     if (bias is not None) and (bias.ndim == 1):
         bias = bias.reshape(1, -1)
     if out is None:

@@ -196,10 +196,10 @@ int ac4k_debug_linear_decode_kernel(int64_t M, int64_t N, int64_t K, int *fused_
  * tensor layout on every call (lib/cuda/sm120/linear_nvfp4.cu:586-633); it would sit beside
  * ac4k::linear_nvfp4 (lib/cuda/sm120/linear_nvfp4.cu:753-901).  Static weights are re-laid ONCE into
  * the order the kernels fetch them, and the linear then reads the image instead of B and B_sf.
- * The arithmetic is untouched: same nibbles, same scale bytes, same order of accumulation, so the
+ * The arithmetic is untouched: same nibbles, same scale bytes, and for M > 32 the same order of accumulation, so the
  * output is bit-identical to the entry point of the plain layout that runs the same kernel
- * (ac4k_linear_nvfp4, or ac4k_linear_nvfp4_skinny for the shapes it splits along K or streams
- * through the LDS ring).
+ * (ac4k_linear_nvfp4, or ac4k_linear_nvfp4_skinny for the shapes it splits along K).  For M <= 32 it is where the plain
+ * layout streams through the 128-row LDS ring, too, and otherwise equal up to the order of the fp32 sums.
  * Image: one block of 9216 bytes per (128 rows, 128 k), blocks of a 128-row band consecutive along
  * k, bands consecutive along n, N padded with zero rows to a whole band.  A block holds 128 rows x
  * 64 packed bytes, the 16-byte piece p of row r at position p ^ ((r >> 1) & 3) of its row, then the
@@ -224,8 +224,8 @@ int ac4k_linear_nvfp4_prepacked(void *D, int d_dtype, const void *A, const void 
  * reference function: it equals the composition the reference's tests make
  * (test/test_linear_bench.py:128-137) — the activation bytes, scales and global scale it
  * produces are those of ac4k_quantize_nvfp4_bf16, bit for bit, and they are returned:
- * X bf16 [M,K] contiguous -> X_q [M,K/2], X_sf [K/64,align_up(M,16),4], X_gs (1 float).
- * workspace as for ac4k_linear_nvfp4_skinny. */
+ * X bf16 [M,K] contiguous -> X_q [M,K/2], X_sf [K/64,align_up(M,16),4], X_gs (1 float), and D is that of
+ * ac4k_linear_nvfp4_workspace on them, bit for bit.  workspace as for ac4k_linear_nvfp4_skinny. */
 int ac4k_linear_nvfp4_fused_bf16(void *D, int d_dtype, const void *X, void *X_q, void *X_sf,
                                  float *X_gs, const void *B, const void *B_sf, const float *B_gs,
                                  const void *bias, int bias_dtype, int64_t M, int64_t N, int64_t K,

@@ -176,7 +176,47 @@ def test_fused_in_one_launch(m, k, n):
         torch.testing.assert_close(d.cpu(), ref, atol=ATOL, rtol=RTOL)
         assert buf[0] == 7.0 and buf[-1] == 7.0
     comp = ops().linear(xq, xsf, xgs, *wq, bias=bias.cuda(), out=torch.empty((m, n), device="cuda"))
-    torch.testing.assert_close(d, comp, atol=1e-5, rtol=1e-4)
+    assert torch.equal(d, comp)
+
+
+# weights that a linear alone would give another kernel, were it not for the fused call (few rows of long K, many rows), and ordinary ones
+@pytest.mark.parametrize("m,n,k", [(1, 512, 8192), (1, 384, 12288), (1, 1024, 16384), (2, 300, 8192), (1, 24700, 10240), (1, 28672, 8192),
+                                   (2, 28672, 8192), (4, 28672, 4096), (1, 1000, 1024), (16, 28672, 1024)])
+def test_fused_call_is_the_composition_in_fp32(m, n, k):
+    g = torch.Generator(device="cuda").manual_seed(n + k)
+    w = ops().quantize(torch.empty((n, k), device="cuda").normal_(0.0, 0.02, generator=g).to(torch.bfloat16), 0, 1)
+    x = make_input((m, k), seed=m, outliers=True).cuda()
+    out = lambda: torch.empty((m, n), dtype=torch.float32, device="cuda")  # noqa: E731
+    assert torch.equal(ops().fused_linear(x, *w, out=out()), ops().linear(*ops().quantize(x, 0, 1), *w, out=out()))
+
+
+# an activation of zeros alone (a global scale of zero), subnormals, infinities, NaN, the largest values: what quantize and linear give
+@pytest.mark.parametrize("m,k", [(1, 4096), (4, 1024), (3, 5376)])
+@pytest.mark.parametrize("kind", ["zeros", "negative zeros", "subnormal", "infinity", "nan", "largest", "one"])
+def test_fused_in_one_launch_on_special_values(m, k, kind):
+    wq = gpu_quant(make_input((200, k), seed=k, std=0.02))
+    x = make_input((m, k), seed=m, outliers=True)
+    if kind in ("zeros", "negative zeros", "one", "subnormal"):
+        x.zero_()
+    if kind == "negative zeros":
+        x = -x
+    elif kind == "subnormal":
+        x.view(torch.int16).copy_(torch.arange(m * k).remainder(128).view(m, k))
+    elif kind == "one":
+        x[m - 1, k - 1] = -3.0
+    elif kind == "infinity":
+        x[0, 17], x[m - 1, k - 1] = float("inf"), float("-inf")
+    elif kind == "nan":
+        x[m - 1, 5] = float("nan")
+    elif kind == "largest":
+        x[0, 3], x[m - 1, 7] = torch.finfo(torch.bfloat16).max, torch.finfo(torch.bfloat16).min
+    x = x.cuda()
+    out = lambda: torch.empty((m, 200), dtype=torch.float32, device="cuda")  # noqa: E731
+    d, (xq, xsf, xgs) = ops().fused_linear(x, *wq, out=out(), return_quantized=True)
+    q = ops().quantize(x, 0, 1)
+    assert torch.equal(xq, q[0]) and torch.equal(xsf.view(torch.uint8), q[1].view(torch.uint8))
+    assert torch.equal(xgs.view(torch.int32), q[2].view(torch.int32))
+    torch.testing.assert_close(d, ops().linear(*q, *wq, out=out()), rtol=0, atol=0, equal_nan=True)
 
 
 # the output over the activation, as in a linear in place, or over a part of it: the activation is quantized before anything is stored
