@@ -637,14 +637,15 @@ static_assert((MHA8_S_BIAS & 0x7fffff) > 128 * 128 * 128 && (MHA8_S_BIAS & 0x7ff
 // K arrives by LDS-DMA two tiles ahead, V through registers one tile ahead.
 // Bound by the issue of vector instructions (about 350 per tile and wave beside 24 MFMAs; two waves share a SIMD and take 8.3 cycles for
 // an exp2, 9.6 for a pair of e4m3, 4.3 for a maximum or an integer conversion, 2.4 to 2.9 for an addition or fma, which they issue
-// together) and, where the whole GPU is busy for long, by power (2.0 GHz there).
+// together; at 8192 x 40 x 128 the vector port is busy for 86 % of a SIMD's time, the matrix core for 41 %) and, where the whole GPU is
+// busy for long, by power (2.0 GHz there).
 // Of the two waves of a SIMD the older one is served first: it ran a whole step alone, at the rate of one wave, and then waited at
 // the barrier for half of the next.  A wave therefore lowers its priority as it gets on with a step, which keeps the two side by side:
 // 16384 x 40 x 128 5270 -> 4955 cycles per tile of both (priorities that alternate step by step 5160 to 5220).
 // The whole call on 16384 x 40 x 128 3474 -> 3301 us with all of it (moving the maxima and the conversion alone 3446), 4096 x 40 284 -> 277,
 // 3000 x 2 x 24 x 64 194 -> 188.  The conversion and the maxima cost less than they save in the clock: power takes back about a third.
-// TILES as above: 8192 heads of 49 x 49, D = 32, 209 / 179 / 144 us with eight waves; 1024 heads of 256 x 256, D = 64, 42 / 44 / 41.5;
-// 40 heads of 16384 x 200 133 / 122 / 114.
+// TILES as above, with eight waves, where they gained the same: 8192 heads of 49 x 49, D = 32, 209 / 179 / 144 us; 1024 heads of 256 x 256,
+// D = 64, 42 / 44 / 41.5; 40 heads of 16384 x 200 133 / 122 / 114.
 // WAVES: eight, or four and two workgroups on a CU, which wait for their barriers and their ends one under the other's work, but
 // fetch every tile of K and V twice per CU.  Whole rounds of many tiles go to eight (kernel alone, us, eight / four: 40 heads of 4096 x
 // 4096 224 / 250, 24 of 4096 x 8192 260 / 277); short loops and grids that leave CUs idle, which finer cuts fill, to four (2 heads of 4096 x 8192 70 / 63,
@@ -1062,7 +1063,9 @@ static void (*const mha_nvfp4_kernels[3][3])(MhaArgs, MhaWork) = {
     {mha_nvfp4_fwd_kernel<1, 0>, mha_nvfp4_fwd_kernel<2, 0>, mha_nvfp4_fwd_kernel<4, 0>},
     {mha_nvfp4_fwd_kernel<1, 1>, mha_nvfp4_fwd_kernel<2, 1>, mha_nvfp4_fwd_kernel<4, 1>},
     {mha_nvfp4_fwd_kernel<1, 2>, mha_nvfp4_fwd_kernel<2, 2>, mha_nvfp4_fwd_kernel<4, 2>}};
-// (row 0: eight waves; they gain nothing on one and two tiles)
+// (row 0: eight waves.  One and two tiles always run four: kernel alone, us, eight / four: 8192 heads of 49 x 49, D = 32, 143 / 75; of
+// 64 x 64 151 / 81, of 128 x 128 211 / 124, D = 64; 1024 of 256 x 256, D = 64, 40.5 / 36.9; 40 of 4096 x 77 27.4 / 22.8, of 16384 x 200
+// 114 / 98; 300 of 200 x 200, D = 64, 16.7 / 16.6)
 static void (*const mha_int8_x_fp8_kernels[4][3])(Mha8Args, MhaWork) = {
     {mha_int8_x_fp8_fwd_kernel<1>, mha_int8_x_fp8_fwd_kernel<2>, mha_int8_x_fp8_fwd_kernel<4>},
     {mha_int8_x_fp8_fwd4_kernel<1, 1>, mha_int8_x_fp8_fwd4_kernel<2, 1>, mha_int8_x_fp8_fwd4_kernel<4, 1>},
@@ -1172,7 +1175,7 @@ extern "C" __attribute__((visibility("default"))) int ac4k_mha_int8_x_fp8_fwd(
     a.head0 = (uint32_t)head0;
     const int waves = kind == 0 ? 8 : 4;
     if (int rc = mha_launch(a, p, mha_int8_x_fp8_kernels[kind][p.tail >> 1], lds_done[kind][p.tail >> 1],
-                            mha8_lds_bytes(waves, kind == 0 && p.tail == 1 ? 1 : p.tail), waves * 64, (hipStream_t)stream)) return rc;
+                            mha8_lds_bytes(waves, p.tail), waves * 64, (hipStream_t)stream)) return rc;
   }
   return check_launch("ac4k_mha_int8_x_fp8_fwd");
 }

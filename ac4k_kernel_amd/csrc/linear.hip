@@ -2071,9 +2071,10 @@ __global__ __launch_bounds__(ST_THREADS, 1) void linear_nvfp4_stream64_kernel(Sk
 // scales, and the same of activation row r, three steps ahead, and has with each dword the operand of one v_mfma_f32_16x16x32_f16 (the
 // order of k is free as long as both sides share it).  The eight sums meet through LDS in the order of the waves.
 // A step's second half that K does not have is read from its first one, with weight scales so small that they round to zero.
-// Bound by the weights from memory and, from about M = 8 on, by the decoding of the activation, which every workgroup does again for
-// as many bytes as its weights (M <= 16; twice as many above): 16 x 4096 x 14336, weights from HBM, 17.8 -> 11.4 us (64 rows, K split in
-// four, and the second launch before), M = 1 15.8 -> 10.4; 16 x 4096 x 4096 10.2 -> 5.1; 1 x 20000 x 2880 23.4 -> 11.2; 32 x 1024 x 1024
+// Bound by the latency of what is in flight: at 16 x 4096 x 14336, one workgroup a CU, 36.1 MiB are read for 31.6 of operands, at 3.6 TB/s,
+// and the counters show a SIMD's vector port busy for 40 % of the time and its matrix core for 8 %.  The activation, read and decoded again by
+// every workgroup, as many bytes as its weights (M <= 16; twice as many above), adds a tenth from M = 1 to 16.
+// 16 x 4096 x 14336, weights from HBM, 17.8 -> 11.4 us (64 rows, K split in four, and the second launch before), M = 1 15.8 -> 10.4; 16 x 4096 x 4096 10.2 -> 5.1; 1 x 20000 x 2880 23.4 -> 11.2; 32 x 1024 x 1024
 // 7.6 -> 3.2.  Three steps ahead and two workgroups on a CU: two more cost 0.7 us at 16 x 4096 x 14336 in registers, sixteen waves 2.5 us at
 // 1 x 14336 x 4096, four waves 3 us at 16 x 4096 x 14336; loads past the caches lose where the activation is read again.
 // ===========================================================================
@@ -2229,6 +2230,8 @@ static void plan_lds_ring(int64_t M, int64_t N, int64_t K, SkinnyPlan &p, int ro
 // 33.5 / 23.5, 14336 x 4096 14.2 / 12.5, 28672 x 8192 33.5 / 41.0, 16384 x 16384 42.7 / 47.0; M = 32, 4096 x 14336 18.2 / 16.6, 14336 x 4096
 // 14.5 / 17.7, 128 x 8192 7.8 / 9.8, 1000 x 1024 7.6 / 3.3; M = 1, 20480 x 8192 41.5 / 23.2, 28672 x 8192 29.2 / 30.0, 300 x 14336 7.8 / 8.8.
 //
+// The register kernel has two costs because it is planned in two ranges: below 12288 rows, K in short slices, and from 24576 rows (192
+// groups of 128) on.
 // `start`: what a fused call saves by quantizing the activation in these workgroups.
 static bool rows16_faster(int64_t M, int64_t N, int64_t K, const SkinnyPlan &p, double start) {
   const double million = 1e-6 * (double)N * (double)K, steps = (double)ceil_div(ceil_div(K, R16_STEP), R16_WAVES);

@@ -8,11 +8,14 @@ namespace ac4k {
 // reads the whole activation (from the L2, all but the first time), takes its maximum and quantizes it - a thread one or two 16-blocks,
 // by the quantizers' own steps, so the operands are theirs bit for bit.  The activation stays in LDS as the fp16 operands of
 // the MFMAs and is not decoded again for every workgroup's weights.  Workgroup 0 stores the packed activation for the caller.
-// Bound by the weights from memory; before that, by the launch.  Two launches -> one, us in a graph, weights from HBM: 1 x 4096 x 4096
+// Bound by the weights from memory (1 x 28672 x 8192: 140.4 MiB read for 126.0 in 31 us, 4.7 TB/s); small ones by the launch.  Two launches -> one, us in a graph, weights from HBM: 1 x 4096 x 4096
 // 8.1 -> 5.9, 1 x 14336 x 4096 13.9 -> 11.5, 1 x 4096 x 14336 14.2 -> 11.3, 4 x 4096 x 4096 8.5 -> 6.7, 16 x 4096 x 1024 6.2 -> 4.6,
 // 1 x 1024 x 2048 5.9 -> 4.0; called one after the other 1 x 4096 x 4096 22.2 -> 19.4 (host time), 1 x 28672 x 8192 33.0 -> 31.4.
-// DEPTH steps of weights in flight per wave: four, and six for long rows in several rounds of workgroups (1 x 28672 x 8192 35.1 with
-// four, 31.4 with six; 1 x 14336 x 4096 11.5 and 11.9, 1 x 4096 x 14336 11.3 and 11.7; eight: 13.1 for 1 x 14336 x 4096).
+// DEPTH steps of weights in flight per wave: four, and six for K above 4096 on 16384 rows and more, several rounds of workgroups.  It is
+// K = 8192 and 16384 that need them (rows a power of two apart meet on few memory channels, and a step takes longer to come; us in a graph,
+// four / six): 1 x 28672 x 8192 33.1 / 31.0, 1 x 20480 x 8192 25.5 / 24.0, 2 x 16384 x 8192 23.5 / 22.0, 1 x 16384 x 16384 35.3 / 34.6.  Other K do
+// not mind (1 x 28672 x 5120 22.8 / 22.7, 1 x 20480 x 12288 32.3 / 32.9, 3 x 28672 x 5120 25.1 / 24.6), short ones neither (1 x 28672 x 4096 19.3 /
+// 19.4), and fewer rows lose as often as they gain (1 x 8192 x 12288 15.1 / 16.2, 1 x 8192 x 5120 9.1 / 9.4, 1 x 14336 x 8192 20.5 / 19.1).
 constexpr int FU_THREADS = 64 * R16_WAVES;
 constexpr int FU_BLOCKS = (int)(FUSED_ELEMS / 16 / FU_THREADS);  // 16-blocks of a thread
 constexpr int FU_PAD = 8;  // elements between the rows in LDS: rows start on different banks
