@@ -406,7 +406,8 @@ __device__ __forceinline__ void store_tile(const f32x16 (&acc)[MI][NJ], char *ld
     } else {
       // (unrolled by four for the small tiles: with all of it 128 x 128 tiles ran 2 % longer, also where no piece is cut - 256 x 4096 x 4096
       // 34.7 -> 33.7 us, 34.3 before there were pieces -; the larger ones lose 0.5 % by it)
-#pragma unroll(MI * NJ <= 4 ? 4 : RP / RS)
+      constexpr int CUT = MI * NJ <= 4 ? 4 : RP / RS;
+#pragma unroll CUT
       for (int it = 0; it < RP / RS; ++it) {
         const u32x4 v = *reinterpret_cast<const u32x4 *>(src + it * RS * PITCH);
         if (cols_left > 0 && p * RP + it * RS < rows_left) store_piece<S>(rowp + it * RS * row_bytes + lane_off, v, cols_left);
@@ -2156,7 +2157,7 @@ static int64_t decode_cu_count() {
 }
 
 // Plan of a decode-sized linear: which kernel, its K split and the fp32 scratch it needs.
-enum { DECODE_REGISTERS = 1, DECODE_LDS_RING = 2, DECODE_LDS_RING64 = 3, DECODE_ROWS16 = 4 };
+enum { DECODE_REGISTERS = 1, DECODE_LDS_RING = 2, DECODE_LDS_RING64 = 3, DECODE_ROWS16 = 4, DECODE_ROWS16_LDS = 5 };
 struct SkinnyPlan {
   int kind;                // DECODE_REGISTERS: linear_nvfp4_skinny_kernel; DECODE_LDS_RING: linear_nvfp4_stream_kernel;
                            // DECODE_LDS_RING64: linear_nvfp4_stream64_kernel
@@ -2168,6 +2169,7 @@ struct SkinnyPlan {
   // their callers for these shapes.
   bool rows16;
   bool fused;  // and so it does, with the quantizer in it, in a fused call
+  bool lds_x;  // and the kernel of the fused call runs a linear alone, too
 };
 static std::atomic<int> g_forced_decode_kernel{0};  // ac4k_set_linear_tuning: 0 = by shape
 
@@ -2254,10 +2256,13 @@ static bool forced_decode_kernel() {
 // two launches / one: 8 x 28672 x 2048 15.6 / 17.7, 16 x 28672 x 1024 11.5 / 14.6; 4 x 28672 x 4096 22.2 / 21.5, 8 x 6144 x 2048 8.0 / 7.3,
 // 32 x 8192 x 512 6.7 / 6.1).
 //
-// A fused call is quantize and linear bit for bit, so a linear of these shapes takes the 16-row kernel, too, also where that is up to 2.5 us
-// slower by the estimate: M = 1 or 2 on few rows of long K and on N >= 24576, K >= 8192.  Linear alone in a graph, weights from HBM, register
-// kernel / 16 rows: 1 x 256 x 8192 7.1 / 6.3, 1 x 512 x 12288 8.0 / 8.3, 1 x 1024 x 12288 9.3 / 8.5, 1 x 1024 x 16384 10.3 / 10.6, 1 x 1536 x 16384
-// 11.3 / 10.8, 2 x 512 x 8192 7.3 / 6.4; 1 x 28672 x 8192 31.1 / 31.5, 1 x 24576 x 10240 35.2 / 35.8, 1 x 28672 x 10240 38.7 / 40.3.
+// A fused call is quantize and linear bit for bit, so a linear of these shapes sums like it.  Where linear_nvfp4_rows16_kernel is not the
+// fastest for it - M = 1 or 2 on few rows of long K and on N >= 24576, K >= 8192 - the kernel of the fused call takes the quantized
+// activation (`lds_x`), decodes it once a workgroup and has more weights in flight.  Linear alone, weights from HBM, one call after the other,
+// register kernel / linear_nvfp4_rows16_kernel / this: 1 x 28672 x 8192 29.5 / 30.2 / 27.9 us, 2 x 28672 x 8192 30.5 / 30.8 / 28.9, 1 x 28672 x 10240
+// 37.3 / 38.1 / 34.1, 1 x 24576 x 12288 37.6 / 37.9 / 33.9, 1 x 256 x 8192 6.6 / 5.8 / 5.5, 1 x 512 x 12288 7.5 / 7.6 / 6.7, 1 x 1536 x 16384 10.9 /
+// 10.6 / 9.1; where linear_nvfp4_rows16_kernel is faster than the others, M above 4 or shorter K, the two are mostly alike (1 x 14336 x 4096
+// 10.3 / 10.6, 16 x 4096 x 1024 3.9 / 4.0, 1 x 4096 x 14336 10.3 / 10.0).
 static bool fused_rows16(int64_t M, int64_t N, int64_t K, const SkinnyPlan &p) {
   return M * K <= FUSED_ELEMS && K % SK_STEP == 0 && (M <= 4 || ceil_div(N, R16_ROWS) <= 2 * decode_cu_count()) && rows16_faster(M, N, K, p, 2.5);
 }
@@ -2285,7 +2290,9 @@ static bool skinny_plan(int64_t M, int64_t N, int64_t K, SkinnyPlan &p) {
   // (ring_ok: 32-bit lane offsets, as in the ring kernels)
   const bool rows16_ok = !forced_decode_kernel() && ring_ok && rows16_grid_ok(N);
   p.fused = rows16_ok && fused_rows16(M, N, K, p);
-  p.rows16 = p.fused || (rows16_ok && rows16_faster(M, N, K, p, 0.0));
+  p.rows16 = rows16_ok && rows16_faster(M, N, K, p, 0.0);
+  p.lds_x = p.fused && !p.rows16 && M <= 16;
+  p.rows16 |= p.fused;
   return true;
 }
 
@@ -2310,6 +2317,9 @@ static int launch_ring(const SkinnyArgs &a, const SkinnyPlan &p, hipStream_t st)
 
 template <int D_DT, int BIAS_DT>
 static int launch_skinny(const SkinnyArgs &a, const SkinnyPlan &p, hipStream_t st) {
+  if (p.lds_x)
+    return launch_fused_rows16({a.D, nullptr, const_cast<uint8_t *>(a.Aq), const_cast<uint8_t *>(a.A_sf), const_cast<float *>(a.A_gs), a.B, a.B_sf, a.B_gs,
+                                a.bias, a.M, a.N, a.K, a.Mp, a.Np}, D_DT, BIAS_DT, st);
   if (p.rows16) {
     const bool tail = a.K % R16_STEP != 0;
     auto *kern = a.M <= 16 ? tail ? linear_nvfp4_rows16_kernel<D_DT, BIAS_DT, 1, true> : linear_nvfp4_rows16_kernel<D_DT, BIAS_DT, 1, false>
@@ -2597,7 +2607,7 @@ extern "C" __attribute__((visibility("default"))) int ac4k_debug_linear_decode_k
   SkinnyPlan p;
   const bool ok = skinny_plan(M, N, K, p);
   if (fused_launches) *fused_launches = !ok || !skinny_entry_k(M, K) ? 0 : p.fused ? 1 : p.rows16 || p.split_k == 1 ? 2 : 3;
-  return !ok ? 0 : p.rows16 ? DECODE_ROWS16 : p.kind;
+  return !ok ? 0 : p.lds_x ? DECODE_ROWS16_LDS : p.rows16 ? DECODE_ROWS16 : p.kind;
 }
 
 extern "C" __attribute__((visibility("default"))) int64_t ac4k_linear_nvfp4_skinny_workspace_bytes(int64_t M, int64_t N, int64_t K) {
@@ -2766,7 +2776,7 @@ static bool prepacked_plan(int64_t M, int64_t N, int64_t K, PrepackedPlan &p) {
   p.mid = !p.ring && ksplit_shape(M, N, K);
   if (p.ring) {
     plan_lds_ring(M, N, K, p.sp);
-    p.sp.rows16 = p.sp.fused = false;
+    p.sp.rows16 = p.sp.fused = p.sp.lds_x = false;
     p.partial_bytes = p.sp.partial_bytes;
   } else if (p.mid) {
     p.kp = ksplit_plan(M, N, K, true);

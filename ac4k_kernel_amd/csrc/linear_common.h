@@ -105,7 +105,7 @@ __device__ __forceinline__ void rows16_finish(const f32x4 (&acc)[MT][2], float4 
 // quantize and linear in one launch (linear_fused.hip); rows16 kernels fit the shape and the operands are on 16 bytes
 struct FusedArgs {
   void *D;
-  const uint16_t *X;       // [M, K] bf16
+  const uint16_t *X;       // [M, K] bf16; null: the activation is in X_q, X_sf and X_gs (M <= 16)
   uint8_t *X_q, *X_sf;     // the quantized activation, for the caller
   float *X_gs;
   const uint8_t *B;

@@ -187,7 +187,7 @@ int ac4k_linear_nvfp4_skinny_static(void *D, int d_dtype, const void *A, const v
 int ac4k_set_linear_tuning(int mi, int nj, int splits, int skinny_ks, int decode_kernel);
 
 /* Testing aid: which decode-sized kernel a linear of this shape runs on operands on 16 bytes, with the workspace it asks for, by the numbers
- * of ac4k_set_linear_tuning; 4 = 16 weight rows per workgroup, 0 = none of them.  *fused_launches (may be NULL): launches of
+ * of ac4k_set_linear_tuning; 4 = 16 weight rows per workgroup, 5 = the same with the activation in LDS, 0 = none of them.  *fused_launches (may be NULL): launches of
  * ac4k_linear_nvfp4_fused_bf16 behind the fills and maxima of the quantizer: 1 = quantizer and linear in one, 2 = quantizer and linear,
  * 3 = and the sums of the K ranges; 0 = not its shape.  Runs nothing. */
 int ac4k_debug_linear_decode_kernel(int64_t M, int64_t N, int64_t K, int *fused_launches);

@@ -190,6 +190,25 @@ def test_fused_call_is_the_composition_in_fp32(m, n, k):
     assert torch.equal(ops().fused_linear(x, *w, out=out()), ops().linear(*ops().quantize(x, 0, 1), *w, out=out()))
 
 
+# 16-row workgroups with the quantized activation in LDS (what a linear runs beside the fused call on few rows of long K and on many): one and
+# two rows, weight rows that do not exist, threads with two blocks, one and none, four and six steps ahead; and a scale byte with its sign
+@pytest.mark.parametrize("m,n,k", [(1, 300, 8192), (1, 513, 12288), (2, 331, 8192), (1, 1024, 16384), (1, 24577, 10240), (2, 28672, 8192)])
+def test_sixteen_row_workgroups_with_the_activation_in_lds(m, n, k):
+    from ac4k_kernel_amd import _lib
+    assert _lib.load().ac4k_debug_linear_decode_kernel(m, n, k, None) == 5
+    g = torch.Generator(device="cuda").manual_seed(n)
+    bq = ops().quantize(torch.empty((n, k), device="cuda").normal_(0.0, 0.02, generator=g).to(torch.bfloat16), 0, 1)
+    aq = gpu_quant(make_input((m, k), seed=m, outliers=True))
+    aq[1].view(torch.uint8)[3, 0, 1] ^= 0x80
+    ref = gpu_dequant(aq, m) @ gpu_dequant(bq, n).t()
+    for dt in (torch.bfloat16, torch.float16, torch.float32):
+        bias = make_input((1, n), seed=3).to(dt).cuda()
+        buf = torch.full((m * n + 3,), 7.0, dtype=dt, device="cuda")
+        out = ops().linear(*aq, *bq, bias=bias, out=buf[1:1 + m * n].view(m, n))
+        torch.testing.assert_close(out, (ref + bias.float()).to(dt), atol=ATOL, rtol=RTOL)
+        assert buf[0] == 7.0 and (buf[1 + m * n:] == 7.0).all()
+
+
 # an activation of zeros alone (a global scale of zero), subnormals, infinities, NaN, the largest values: what quantize and linear give
 @pytest.mark.parametrize("m,k", [(1, 4096), (4, 1024), (3, 5376)])
 @pytest.mark.parametrize("kind", ["zeros", "negative zeros", "subnormal", "infinity", "nan", "largest", "one"])
