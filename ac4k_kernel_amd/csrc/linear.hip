@@ -66,19 +66,32 @@ __device__ __forceinline__ void decode8(uint32_t w, f16x2 sp, f16x2 (&h)[4]) {
 // the tiles in bands of GROUP_M tile-rows, column by column inside a band: the workgroups resident
 // on one XCD at a time then cover a compact GROUP_M x (CUs / GROUP_M) patch and share its operand
 // panels through that L2.
+// (32 bits: a grid has fewer than 2^32 workgroups.  The quotients of 64 bits that were here, and of the K ranges below, took every workgroup
+// a third of a microsecond: 300 x 1024 x 256 5.23 -> 4.83 us, 2898 x 600 x 256 5.83 -> 5.46.)
 struct TileCoord {
-  int64_t m, n;
+  uint32_t m, n;
 };
 template <int GROUP_M>
-__device__ __forceinline__ TileCoord tile_of_workgroup(int64_t pid, int64_t tiles_m, int64_t tiles_n) {
-  const int64_t ntiles = tiles_m * tiles_n;
-  const int64_t per = ntiles / 8, rem = ntiles % 8;
-  const int64_t xcd = pid % 8, idx = pid / 8;
+__device__ __forceinline__ TileCoord tile_of_workgroup(uint32_t pid, uint32_t tiles_m, uint32_t tiles_n) {
+  const uint32_t ntiles = tiles_m * tiles_n;
+  const uint32_t per = ntiles / 8, rem = ntiles % 8;
+  const uint32_t xcd = pid % 8, idx = pid / 8;
   pid = xcd * per + (xcd < rem ? xcd : rem) + idx;
-  const int64_t band = pid / (GROUP_M * tiles_n), in_band = pid % (GROUP_M * tiles_n);
-  const int64_t first_m = band * GROUP_M;
-  const int64_t rows = (tiles_m - first_m) < GROUP_M ? (tiles_m - first_m) : GROUP_M;
-  return {first_m + in_band % rows, in_band / rows};
+  const uint32_t band = pid / (GROUP_M * tiles_n), in_band = pid - band * (GROUP_M * tiles_n);
+  const uint32_t first_m = band * GROUP_M;
+  const uint32_t rows = (tiles_m - first_m) < GROUP_M ? (tiles_m - first_m) : GROUP_M;
+  const uint32_t col = in_band / rows;
+  return {first_m + in_band - col * rows, col};
+}
+// stages [first, first + count) of K range `range` of `ranges`; in scalar registers, said plainly: the compiler otherwise takes the
+// quotients, and with them the loop and the addresses, to the lanes
+struct StageRange {
+  int first, count;
+};
+__device__ __forceinline__ StageRange stage_range(int stages, uint32_t range, int ranges) {
+  if (ranges == 1) return {0, stages};
+  const int first = __builtin_amdgcn_readfirstlane((int)((int64_t)stages * range / ranges));
+  return {first, __builtin_amdgcn_readfirstlane((int)((int64_t)stages * (range + 1) / ranges)) - first};
 }
 
 // ===========================================================================
@@ -221,11 +234,16 @@ __global__ __launch_bounds__(256) void linear_nvfp4_tile128_kernel(LinearArgs a)
 // and B, so the permutation of k inside a chunk cancels in the dot product.  Decode per dword:
 // 4 x v_cvt_scalef32_pk_f16_fp4 + 4 x v_pk_mul_f16 by the block scale (E4M3 -> fp16 with
 // v_cvt_scalef32_pk_f16_fp8, splat through op_sel); the decode of a sub-step is interleaved with
-// the MFMAs of the previous one.  A single wave per SIMD is bound by instruction issue: the
-// 4 decode instructions per MFMA of the 256x256 tile stretch a 32-cycle MFMA slot to about 38
-// cycles, the smaller tiles (more decode per MFMA) are decode-bound outright; that, not LDS or
-// HBM, bounds the loop.  There is one workgroup barrier per 128 k, placed in the middle of the
-// step so that the next stage is readable before the current one ends.
+// the MFMAs of the previous one (TileWave below).
+// KW == 1: the waves multiply a quarter of the tile each, over all of a stage, with one workgroup barrier per 128 k, placed in the
+// middle of the step so that the next stage is readable before the current one ends.  KW == 2, for the tiles of up to 256 x 128: two waves
+// multiply one half of the tile each over one 64-chunk of a stage and two over the other, and meet at the end through LDS: 4 decode
+// instructions per MFMA instead of 6 for 256 x 128 and 128 x 256, 4.7 instead of 6.7 for 192 x 128, 6 instead of 8 for 128 x 128.
+// Bound by instruction issue of a single wave per SIMD and, where the whole GPU is busy for long, by power.  Cycles per MFMA and wave, with
+// KW == 1, the decoding pinned between the MFMAs and the scales fetched a dword per lane / now: 256 x 256 41.2 / 35.2, 256 x 128 51 / 39,
+// 192 x 128 58 / 44, 128 x 128 70 / 51.  Back to back, us: 1024 x 4096 x 4096 38.3 / 32.8, 1001 x 5003 x 2880 35.7 / 33.6, 2048 x 4096 x 4096
+// 58.2 / 53.8, 2048 x 14336 x 4096 183.8 / 175.5, 75600 x 5120 x 5120 2776 / 2673 (the clock comes down by half of what the loop gains).  The
+// exchange costs half a microsecond a round: two stages of K lose by it what they gain (381 x 21120 x 256 11.6 / 12.0).
 // Split-K: blockIdx.y selects a contiguous range of stages; with more than one range the
 // accumulators go to an fp32 partial buffer and a second kernel adds the ranges.
 // Requires K % 64 == 0, K >= 128 and 16-byte aligned operands.  EARLY: K % 128 == 64.  The stages start one
@@ -242,21 +260,83 @@ template <int BM, int BN, int PS>
 struct PLayout {               // byte offsets inside one LDS stage; PS stages
   static constexpr int OFF_B = BM * P_ROW;                 // B rows follow the A rows
   static constexpr int OFF_SFA = OFF_B + BN * P_ROW;       // scale dwords: [chunk][BM rows]
-  static constexpr int OFF_SFB = OFF_SFA + 2 * BM * 4;     // [chunk][BN rows]
-  static constexpr int STAGE_BYTES = OFF_SFB + 2 * BN * 4;
+  static constexpr int NSA = (BM + 127) / 128, NSB = (BN + 127) / 128;  // kilobytes, and transfers, of scales
+  static constexpr int OFF_SFB = OFF_SFA + NSA * 1024;     // [chunk][BN rows]
+  static constexpr int STAGE_BYTES = OFF_SFB + NSB * 1024;
+  static_assert(NSA + NSB <= 4, "a scale transfer per wave");
   static constexpr int LDS_BYTES = PS * STAGE_BYTES;
   static_assert(LDS_BYTES <= 160 * 1024, "stages must fit in the CU's LDS");
 };
 
-template <int MI, int NJ>
-struct DecFrags {
-  f16x8 a[MI], b[NJ];
-};
-
-template <int S>
-__device__ __forceinline__ uint32_t dword_of(const uint4 &v) {
-  return S == 0 ? v.x : S == 1 ? v.y : S == 2 ? v.z : v.w;
+// two of the eight values of a dword of nibbles, without their scale; q (0..3) is a constant after unrolling
+__device__ __forceinline__ f16x2 decode_pair(uint32_t w, int q) {
+  if (q == 0) return __builtin_amdgcn_cvt_scalef32_pk_f16_fp4(w, 1.0f, 0);
+  if (q == 1) return __builtin_amdgcn_cvt_scalef32_pk_f16_fp4(w, 1.0f, 1);
+  if (q == 2) return __builtin_amdgcn_cvt_scalef32_pk_f16_fp4(w, 1.0f, 2);
+  return __builtin_amdgcn_cvt_scalef32_pk_f16_fp4(w, 1.0f, 3);
 }
+
+// f(i) for the share of COUNT things that belongs behind the m-th of OF instructions (a loop of a known length, so that it unrolls
+// before the one over m does)
+template <int COUNT, int OF, typename F>
+__device__ __forceinline__ void deal(int m, F &&f) {
+#pragma unroll
+  for (int x = 0; x < (COUNT + OF - 1) / OF; ++x) {
+    const int i = COUNT * m / OF + x;
+    if (i < COUNT * (m + 1) / OF) f(i);
+  }
+}
+
+// What a wave of the tile kernels holds: packed fragments of a 64-chunk, 32 rows each, WI of A first, then WJ of B, in two sets (one
+// multiplied while the other arrives), and the sums of WI x WJ blocks.  Lane (row r, half h) of a fragment has elements
+// [32 h, 32 h + 32) of the chunk; dword s of them belongs to sub-step s, 16 k.
+//
+// The loop bodies are written out in the order in which they issue.  A wave is alone on its SIMD and issues an instruction of any kind
+// every 5 cycles; an MFMA takes 8.6 of these and keeps the matrix core busy for 32.  Up to four or five instructions behind every
+// MFMA are free, and what stands in a clump leaves the matrix core idle, so everything is dealt out evenly: the decoding,
+// the LDS reads and the transfers.  (Left to the compiler, with only the decoding pinned between the MFMAs: 41.2 cycles an MFMA in
+// 256 x 256 tiles, 36.4 so, 35.2 with the scales in 16-byte transfers.)
+template <int WI, int WJ>
+struct TileWave {
+  static constexpr int NF = WI + WJ, NM = WI * WJ;
+  uint4 packed[2][NF];
+  uint32_t sf[2][NF];    // the scale bytes of the lane's two blocks
+  f16x2 scale[2][NF];    // the same as fp16
+  u32x4 decoded[2][NF];  // operands of a sub-step, double buffered
+  f32x16 acc[WI][WJ];
+
+  // item i of decoding sub-step s of set `set` into buffer d: two values of fragment i / 4.  wfac: power of two on the scales of B
+  __device__ __forceinline__ void decode_item(int d, int set, int s, int i, float wfac = 1.0f) {
+    const int f = i >> 2, q = i & 3;
+    if (s == 0 && q == 0) scale[set][f] = __builtin_amdgcn_cvt_scalef32_pk_f16_fp8(sf[set][f], f < WI ? 1.0f : wfac, false);
+    const f16x2 sc = s < 2 ? (f16x2){scale[set][f].x, scale[set][f].x} : (f16x2){scale[set][f].y, scale[set][f].y};
+    const uint4 &v = packed[set][f];
+    decoded[d][f][q] = __builtin_bit_cast(uint32_t, decode_pair(s == 0 ? v.x : s == 1 ? v.y : s == 2 ? v.z : v.w, q) * sc);
+  }
+  // One sub-step: the MFMAs on buffer d, under them the decoding of sub-step s of set `set` into the other buffer, and extra(m) behind MFMA m
+  template <typename F>
+  __device__ __forceinline__ void substep(int d, int set, int s, F &&extra, float wfac = 1.0f) {
+#pragma unroll
+    for (int m = 0; m < NM; ++m) {
+      // boustrophedon order: every MFMA shares one operand with the one before it (measured 0.6 %
+      // faster than row by row on the power-limited 8192^3 problem: less operand switching)
+      const int i = m / WJ, j = (i & 1) ? WJ - 1 - m % WJ : m % WJ;
+      acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(f16x8, decoded[d][WI + j]), __builtin_bit_cast(f16x8, decoded[d][i]),
+                                                         acc[i][j], 0, 0, 0);  // D^T block
+      deal<4 * NF, NM>(m, [&](int e) { decode_item(1 - d, set, s, e, wfac); });
+      extra(m);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+  }
+  __device__ __forceinline__ void clear() {
+#pragma unroll
+    for (int i = 0; i < WI; ++i)
+#pragma unroll
+      for (int j = 0; j < WJ; ++j)
+#pragma unroll
+        for (int e = 0; e < 16; ++e) acc[i][j][e] = 0.0f;
+  }
+};
 
 // Build with -DAC4K_LINEAR_TIMELINE (`build.py --timeline`) to record per workgroup the 100 MHz clock at
 // kernel entry, loop entry, loop exit and kernel exit plus the shader cycles spent in the loop of the
@@ -421,7 +501,7 @@ __device__ __forceinline__ void store_tile(const f32x16 (&acc)[MI][NJ], char *ld
 // NJ = 32-column fragments per wave along N: 4 (BN = 256), 2 (BN = 128) or 1 (BN = 64);
 // PS = LDS stages: PS - 1 k-steps are in flight ahead of the one being multiplied, which a small
 // tile needs because its k-step is much shorter than the memory latency.
-template <int D_DT, int BIAS_DT, int MI, int NJ, int PS, bool EARLY>
+template <int D_DT, int BIAS_DT, int MI, int NJ, int PS, int KW, bool EARLY>
 __global__ __launch_bounds__(256, 1) void linear_nvfp4_tile256p_kernel(LinearArgs a, SplitK sk) {
   extern __shared__ __attribute__((aligned(16))) char plds[];
   AC4K_LTL(0, wall_clock64());
@@ -429,22 +509,22 @@ __global__ __launch_bounds__(256, 1) void linear_nvfp4_tile256p_kernel(LinearArg
   using PL = PLayout<BM, BN, PS>;
   constexpr int NDA = BM / 4 / 16;         // 16-row A transfers per wave per stage
   constexpr int NDB = BN / 4 / 16;         // 16-row B transfers per wave per stage
-  constexpr int NSA = 2 * (BM / 64);       // scale transfers of A per stage: chunks x 64-row blocks
-  constexpr int NSB = 2 * (BN / 64);
-  constexpr int NS = (NSA + NSB + 3) / 4;  // scale transfers per wave (a remainder repeats the last one)
-  constexpr int NPIECES = NDA + NDB + NS;
+  constexpr int NPIECES = NDA + NDB + 1;   // and one of scales
 
-  const TileCoord tc = tile_of_workgroup<4>(blockIdx.x, ceil_div(a.M, BM), ceil_div(a.N, BN));
-  const int64_t tm = tc.m, tn = tc.n;
+  const TileCoord tc = tile_of_workgroup<4>(blockIdx.x, (uint32_t)ceil_div(a.M, BM), (uint32_t)ceil_div(a.N, BN));
+  const int64_t tm = (uint32_t)__builtin_amdgcn_readfirstlane((int)tc.m), tn = (uint32_t)__builtin_amdgcn_readfirstlane((int)tc.n);
 
+  // KW == 2: the pair of waves (WI > MI: 0 and 2, 1 and 3; WJ > NJ: 0 and 1, 2 and 3) multiplies the blocks of both
+  constexpr bool PAIR_M = KW == 2 && MI < NJ, PAIR_N = KW == 2 && !PAIR_M;
+  constexpr int WI = PAIR_M ? 2 * MI : MI, WJ = PAIR_N ? 2 * NJ : NJ;  // fragments that a wave multiplies
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int wm = wave >> 1, wn = wave & 1;
+  const int wm = PAIR_M ? 0 : wave >> 1, wn = PAIR_N ? 0 : wave & 1;
   const int half = lane >> 5;
   // this workgroup's range of 128-k stages; `early`: bytes by which they start in front of the row
   const int nkt_all = (int)(EARLY ? ceil_div(a.K, P_BK) : a.K / P_BK);
   constexpr int early = EARLY ? 32 : 0;
-  const int kt0 = (int)((int64_t)nkt_all * blockIdx.y / sk.splits);
-  const int nkt = (int)((int64_t)nkt_all * (blockIdx.y + 1) / sk.splits) - kt0;
+  const StageRange range = stage_range(nkt_all, blockIdx.y, sk.splits);
+  const int kt0 = range.first, nkt = range.count;
 
   // LDS-DMA.  One transfer moves 16 rows x 64 B: the four lanes 4r .. 4r+3 read the four 16-byte
   // pieces of row r (one 64-byte sector) and land at LDS base + 16*l, i.e. row-major 64-byte rows.
@@ -485,38 +565,36 @@ __global__ __launch_bounds__(256, 1) void linear_nvfp4_tile256p_kernel(LinearArg
   const int64_t strideB = a.prepacked ? W_BLOCK_BYTES : P_ROW;  // bytes per stage along k
   const uint8_t *baseA = uniform_ptr(a.A + tm * BM * kb + (int64_t)kt0 * P_ROW - early);
   const uint8_t *baseB = uniform_ptr(a.prepacked ? a.B + (int64_t)kt0 * W_BLOCK_BYTES : a.B + tn * BN * kb + (int64_t)kt0 * P_ROW - early);
-  // scale transfers: piece g = swave * NS + p (past the last piece: the last piece again, which
-  // lands the same bytes in the same place).  g < NSA: operand A, chunk g / (BM/64), 64-row block
-  // g % (BM/64); otherwise operand B, chunk (g-NSA) / (BN/64), block (g-NSA) % (BN/64).  Source
-  // base, bytes per stage and LDS offset are wave-uniform and fixed, computed here so that the
-  // loop body stays free of branches.
-  const uint8_t *sfA8 = uniform_ptr(a.A_sf), *sfB8 = uniform_ptr(a.B_sf);
-  uint32_t offS[NS], ldsS[NS];
-  const uint8_t *baseS[NS];
-  int64_t strideS[NS];
-  uint32_t firstS = 0;  // bit p2: scale transfer p2 moves the first chunk of a stage
-#pragma unroll
-  for (int p2 = 0; p2 < NS; ++p2) {
-    const int gq = swave * NS + p2 < NSA + NSB ? swave * NS + p2 : NSA + NSB - 1;
-    const bool isB = gq >= NSA;
-    const int gl = isB ? gq - NSA : gq, nb = isB ? BN / 64 : BM / 64;
-    const int c = gl / nb, rb = gl % nb;
-    const int64_t rows = isB ? a.Np : a.Mp;
+  // scales: a transfer is 256 dwords of the [chunk][row] picture of an operand, a lane four rows of a chunk (16 bytes; the address is on
+  // four).  Waves 0 .. NSA - 1 move those of A, the others those of B; a wave past the last transfer repeats the last one, and so do
+  // lanes past the picture's end with rows of its last chunk, into the rest of the kilobyte.  (A dword per lane, up to four transfers a wave, cost
+  // the loop of 192 x 128 tiles 377 of its 2420 cycles a stage.)
+  uint32_t offS, ldsS;
+  const uint8_t *baseS;
+  int64_t strideS;
+  bool firstS;  // this lane's rows belong to the first chunk of a stage
+  {
+    const int t = swave < PL::NSA + PL::NSB ? swave : PL::NSA + PL::NSB - 1;
+    const bool isB = t >= PL::NSA;
+    const int tt = isB ? t - PL::NSA : t, rows_t = isB ? BN : BM;
+    const int at = tt * 256 + lane * 4, c = at >= rows_t ? 1 : 0;
+    const int loc = at < 2 * rows_t ? at - c * rows_t : 0;
+    const int64_t rows = isB ? a.Np : a.Mp, first = isB ? tn * BN : tm * BM;
+    firstS = c == 0;
     if (isB && a.prepacked) {  // the scale dwords follow the packed rows of the block
       int64_t within;
-      const int64_t band = w_band_of(tn * BN + rb * 64, within);
-      offS[p2] = (uint32_t)(band * w_band_bytes + W_BLOCK_DATA + c * (W_BLOCK_ROWS * 4) + (within + lane) * 4);
-      strideS[p2] = W_BLOCK_BYTES;
-      baseS[p2] = uniform_ptr(a.B + (int64_t)kt0 * W_BLOCK_BYTES);
+      const int64_t band = w_band_of(first + loc, within);
+      offS = (uint32_t)(band * w_band_bytes + W_BLOCK_DATA + c * (W_BLOCK_ROWS * 4) + within * 4);
+      strideS = W_BLOCK_BYTES;
+      baseS = uniform_ptr(a.B + (int64_t)kt0 * W_BLOCK_BYTES);
     } else {
-      int64_t sr = (isB ? tn * BN : tm * BM) + rb * 64 + lane;
-      sr = sr < rows ? sr : rows - 1;
-      offS[p2] = (uint32_t)sr * 4u;  // byte offset inside a scale plane
-      strideS[p2] = 2 * rows * 4;    // two planes (chunks) per stage
-      baseS[p2] = uniform_ptr((isB ? sfB8 : sfA8) + (c - (EARLY ? 1 : 0)) * rows * 4 + kt0 * strideS[p2]);
+      const int64_t row = first + loc + 4 <= rows ? loc : rows - 4 - first;  // (rows are padded to 16)
+      offS = (uint32_t)((c * rows + row) * 4);
+      strideS = 2 * rows * 4;  // two planes (chunks) per stage
+      baseS = uniform_ptr(reinterpret_cast<const uint8_t *>(isB ? a.B_sf : a.A_sf) + (first - (EARLY ? rows : 0)) * 4 + kt0 * strideS);
     }
-    if (c == 0) firstS |= 1u << p2;
-    ldsS[p2] = (uint32_t)__builtin_amdgcn_readfirstlane((isB ? PL::OFF_SFB + c * BN * 4 : PL::OFF_SFA + c * BM * 4) + rb * 256);
+    strideS = (int64_t)uniform_ptr((const void *)strideS);
+    ldsS = (uint32_t)__builtin_amdgcn_readfirstlane((isB ? PL::OFF_SFB : PL::OFF_SFA) + tt * 1024);
   }
   const uint32_t lds_base = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) char *)plds;
   // LDS destinations of this wave's transfers inside a stage (wave-uniform, loop invariant)
@@ -529,14 +607,13 @@ __global__ __launch_bounds__(256, 1) void linear_nvfp4_tile256p_kernel(LinearArg
   // at the last step of the range: fetches past the end re-read the last slice into a stage buffer
   // nobody reads again, which keeps the main loop free of branches.
   struct Src {
-    const uint8_t *a, *b, *s[NS];
+    const uint8_t *a, *b, *s;
   };
   auto src_at = [&](int kt) {
     Src p;
     p.a = baseA + (int64_t)kt * P_ROW;
     p.b = baseB + (int64_t)kt * strideB;
-#pragma unroll
-    for (int p2 = 0; p2 < NS; ++p2) p.s[p2] = baseS[p2] + kt * strideS[p2];
+    p.s = baseS + kt * strideS;
     return p;
   };
   auto issue_piece = [&](uint32_t stage_lds, const Src &p, int q) {
@@ -545,104 +622,47 @@ __global__ __launch_bounds__(256, 1) void linear_nvfp4_tile256p_kernel(LinearArg
     } else if (q < NDA + NDB) {
       dma16(p.b, offB[q - NDA], stage_lds, ldsB[q - NDA]);
     } else {
-      const int p2 = q - NDA - NDB;
-      dma4(p.s[p2], offS[p2], stage_lds, ldsS[p2]);
+      dma16(p.s, offS, stage_lds, ldsS);
     }
   };
   auto issue_stage = [&](uint32_t stage_lds, const Src &p) {
 #pragma unroll
     for (int q = 0; q < NPIECES; ++q) issue_piece(stage_lds, p, q);
   };
-  // pieces issued in quarter `qr` (0..3) of the second half of a step
-  auto issue_quarter = [&](uint32_t stage_lds, const Src &p, int qr) {
-#pragma unroll
-    for (int q = 0; q < NDA; ++q)
-      if (q * 4 / NDA == qr) issue_piece(stage_lds, p, q);
-#pragma unroll
-    for (int q = 0; q < NDB; ++q)
-      if (q * 4 / NDB == qr) issue_piece(stage_lds, p, NDA + q);
-#pragma unroll
-    for (int q = 0; q < NS; ++q)
-      if (q * 4 / NS == qr) issue_piece(stage_lds, p, NDA + NDB + q);
-  };
-
-  f32x16 acc[MI][NJ];
-#pragma unroll
-  for (int i = 0; i < MI; ++i)
-#pragma unroll
-    for (int j = 0; j < NJ; ++j)
-#pragma unroll
-      for (int e = 0; e < 16; ++e) acc[i][j][e] = 0.0f;
+  TileWave<WI, WJ> w;
+  w.clear();
 
   // fragment addresses inside a stage (bytes)
   // (a lane's rows differ by multiples of 32, so the swizzle term of its row is (lane >> 1) & 3 for all of them)
   const int fa_off = (wm * (32 * MI) + (lane & 31)) * P_ROW;
   const int fb_off = PL::OFF_B + (wn * (32 * NJ) + (lane & 31)) * P_ROW;
   const int piece_off[2] = {((0 + half) ^ ((lane >> 1) & 3)) * 16, ((2 + half) ^ ((lane >> 1) & 3)) * 16};  // chunk 0, chunk 1
+  // KW == 2: the chunk of every stage that this wave multiplies; its first MI x NJ fragments are the ones that it will keep, behind
+  // them those of the other wave of the pair, so that no register is chosen at run time
+  const int kw = PAIR_M ? swave >> 1 : swave & 1;
+  auto row_a = [&](int i) { return 32 * (PAIR_M ? (i < MI ? kw * MI : (1 - kw) * MI) + i % MI : i); };
+  auto row_b = [&](int j) { return 32 * (PAIR_N ? (j < NJ ? kw * NJ : (1 - kw) * NJ) + j % NJ : j); };
   // a lane needs the two scale bytes of its half of the chunk: blocks 2*half, 2*half+1
   const int sa_off = PL::OFF_SFA + (wm * (32 * MI) + (lane & 31)) * 4 + half * 2;
   const int sb_off = PL::OFF_SFB + (wn * (32 * NJ) + (lane & 31)) * 4 + half * 2;
 
-  uint4 PA[2][MI], PB[2][NJ];  // packed fragments of a 64-chunk, double buffered by chunk parity
-  f16x2 SA[2][MI], SB[2][NJ];  // their two block scales (blocks 2*half, 2*half+1) as fp16
-  auto load_chunk = [&](uint32_t stage_off, int c) {
+  // read r of a chunk into set `set` (by chunk parity, KW == 2 by stage parity): the packed fragments, then the scale bytes
+  constexpr int NF = WI + WJ, NM = WI * WJ;
+  auto load_item = [&](uint32_t stage_off, int c, int set, int r) {
     const char *st = plds + stage_off;
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      if (i < MI) PA[c][i] = *reinterpret_cast<const uint4 *>(st + fa_off + piece_off[c] + i * 32 * P_ROW);
-      if (i < NJ) PB[c][i] = *reinterpret_cast<const uint4 *>(st + fb_off + piece_off[c] + i * 32 * P_ROW);
-    }
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      if (i < MI) {
-        const uint32_t wa = *reinterpret_cast<const uint16_t *>(st + sa_off + c * (BM * 4) + i * 128);
-        SA[c][i] = __builtin_amdgcn_cvt_scalef32_pk_f16_fp8(wa, 1.0f, false);
-      }
-      if (i < NJ) {
-        const uint32_t wb = *reinterpret_cast<const uint16_t *>(st + sb_off + c * (BN * 4) + i * 128);
-        SB[c][i] = __builtin_amdgcn_cvt_scalef32_pk_f16_fp8(wb, 1.0f, false);
-      }
+    const int f = r % NF;
+    if (r < NF) {
+      const int piece = KW == 2 ? (kw ? piece_off[1] : piece_off[0]) : piece_off[c];
+      w.packed[set][f] = *reinterpret_cast<const uint4 *>(st + piece + (f < WI ? fa_off + row_a(f) * P_ROW : fb_off + row_b(f - WI) * P_ROW));
+    } else {
+      w.sf[set][f] = *reinterpret_cast<const uint16_t *>(st + (f < WI ? sa_off + c * (BM * 4) + row_a(f) * 4 : sb_off + c * (BN * 4) + row_b(f - WI) * 4));
     }
   };
 
-  DecFrags<MI, NJ> D[2];
-  auto decode = [&](DecFrags<MI, NJ> &d, int c, auto S) {
-    constexpr int s = decltype(S)::value;
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      if (i < MI) d.a[i] = decode_dword<(s >= 2)>(dword_of<s>(PA[c][i]), SA[c][i]);
-      if (i < NJ) d.b[i] = decode_dword<(s >= 2)>(dword_of<s>(PB[c][i]), SB[c][i]);
-    }
-  };
-  auto mfma16 = [&](const DecFrags<MI, NJ> &d) {
-#pragma unroll
-    for (int i = 0; i < MI; ++i)
-#pragma unroll
-      for (int jj = 0; jj < NJ; ++jj) {
-        // boustrophedon order: every MFMA shares one operand with the one before it (measured 0.6 %
-        // faster than row by row on the power-limited 8192^3 problem: less operand switching)
-        const int j = (i & 1) ? NJ - 1 - jj : jj;
-        acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(d.b[j], d.a[i], acc[i][j], 0, 0, 0);  // D^T block
-      }
-  };
-  auto interleave = [&]() {  // the decode of the next sub-step rides in the shadow of the MFMAs
-    constexpr int NMFMA = MI * NJ, NVALU = 8 * (MI + NJ);
-    constexpr int PER = (NVALU + NMFMA - 1) / NMFMA;  // 4 for 4x4, 6 for 2x4 and 4x2, 8 for 2x2, ...
-#pragma unroll
-    for (int g = 0; g < NMFMA; ++g) {
-      __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-      __builtin_amdgcn_sched_group_barrier(0x002, PER, 0);
-    }
-    __builtin_amdgcn_sched_barrier(0);
-  };
-  using I0 = std::integral_constant<int, 0>;
-  using I1 = std::integral_constant<int, 1>;
-  using I2 = std::integral_constant<int, 2>;
-  using I3 = std::integral_constant<int, 3>;
-
-  // prologue: stages 0 .. PS-2 in flight (past the last k-step: the last one again), stage 0
-  // visible, chunk 0 fragments and first decode
-  static_assert(PS >= 3 && (PS - 2) * NPIECES <= 63, "the wait counts below must fit the 6-bit counter");
+  // prologue: stages 0 .. PS-2 (KW == 2: PS-1) in flight (past the last k-step: the last one again), stage 0
+  // visible, the wave's first fragments and first decode
+  constexpr int AHEAD = KW == 2 ? PS : PS - 1;
+  static_assert(PS >= 3 && (AHEAD - 1) * NPIECES <= 63, "the wait counts below must fit the 6-bit counter");
   const int last = nkt - 1;
   // the stage that fetches past the end repeat: never the short one, whose first half lies in front of the rows
   // (a range of one stage then repeats the stage behind it, which exists: K >= 192)
@@ -655,46 +675,78 @@ __global__ __launch_bounds__(256, 1) void linear_nvfp4_tile256p_kernel(LinearArg
     for (int q = 0; q < NDA; ++q) dma16(p.a, offA[q] + shift, lds_base, ldsA[q]);
 #pragma unroll
     for (int q = 0; q < NDB; ++q) dma16(p.b, offB[q] + shift, lds_base, ldsB[q]);
-#pragma unroll
-    for (int p2 = 0; p2 < NS; ++p2) dma4(p.s[p2] + (short0 && (firstS >> p2 & 1) ? strideS[p2] / 2 : 0), offS[p2], lds_base, ldsS[p2]);
+    dma16(p.s, offS + (short0 && firstS ? (uint32_t)(strideS / 2) : 0), lds_base, ldsS);
   }
+  // A range shorter than the ring is fetched as it is and waited for as a whole: its repeats would be most of a short prologue
+  // (10650 x 512 x 384 11.4 -> 10.9 us).
+  const bool brief = nkt < AHEAD;
 #pragma unroll
-  for (int d = 1; d < PS - 1; ++d) issue_stage(lds_base + d * PL::STAGE_BYTES, src_at(d < last ? d : again));
-  wait_vmcnt<(PS - 2) * NPIECES>();  // everything of stage 0 has landed, later stages may be in flight
+  for (int d = 1; d < AHEAD; ++d)
+    if (!brief || d < nkt) issue_stage(lds_base + d * PL::STAGE_BYTES, src_at(d < last ? d : again));
+  if (brief) wait_vmcnt<0>();
+  else wait_vmcnt<(AHEAD - 1) * NPIECES>();  // everything of stage 0 has landed, later stages may be in flight
   __syncthreads();
-  load_chunk(0, 0);
-  if (short0) {
 #pragma unroll
-    for (int i = 0; i < MI; ++i) SA[0][i] = (f16x2){(_Float16)0.0f, (_Float16)0.0f};
+  for (int r = 0; r < 2 * NF; ++r) load_item(0, KW == 2 ? kw : 0, 0, r);
+  if (short0 && (KW == 1 || kw == 0)) {
 #pragma unroll
-    for (int j = 0; j < NJ; ++j) SB[0][j] = (f16x2){(_Float16)0.0f, (_Float16)0.0f};
+    for (int f = 0; f < NF; ++f) w.sf[0][f] = 0;
   }
-  decode(D[0], 0, I0{});
+#pragma unroll
+  for (int e = 0; e < 4 * NF; ++e) w.decode_item(0, 0, 0, e);
+  if constexpr (KW == 2) {  // stage 1 landed, and everybody's fragments of stage 0 in registers
+    wait_vmcnt<(AHEAD - 2) * NPIECES>();
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    __syncthreads();
+  }
 
   // loop-carried, wave-uniform: LDS offsets of the stages holding k-steps kt, kt+1 and of the one
-  // being filled with kt+PS-1 (a ring of PS), and the source pointers of k-step min(kt+PS-1, last)
+  // being filled with kt+AHEAD (a ring of PS), and the source pointers of k-step min(kt+AHEAD, last)
   uint32_t st_cur = 0, st_nxt = PL::STAGE_BYTES, st_dma = (PS - 1) * PL::STAGE_BYTES;
   auto ring_next = [](uint32_t o) { return o + PL::STAGE_BYTES == (uint32_t)PL::LDS_BYTES ? 0u : o + PL::STAGE_BYTES; };
-  Src src = src_at(last < PS - 1 ? again : PS - 1);
+  Src src = src_at(last < AHEAD ? again : AHEAD);
+  auto advance = [&](int kt) {  // the sources, unless they already sit on the last k-step
+    const bool adv = kt + AHEAD < last;
+    src.a += adv ? P_ROW : 0;
+    src.b += adv ? strideB : 0;
+    src.s += adv ? strideS : 0;
+  };
 #ifdef AC4K_LINEAR_TIMELINE
   const uint64_t tl_c0 = __builtin_readcyclecounter();
 #endif
   AC4K_LTL(1, wall_clock64());
-  for (int kt = 0; kt < nkt; ++kt) {
+  // KW == 2: a step multiplies chunk kw of stage kt out of registers (set kt & 1) while that of stage kt+1, which landed before
+  // the last barrier, travels to the other set, and stage kt+PS to the ring slot of stage kt
+  auto pair_step = [&](int kt, int cur) {
+    const uint32_t dma_lds = lds_base + st_cur;
+#pragma unroll
+    for (int s = 0; s < 4; ++s)
+      w.substep(s & 1, s < 3 ? cur : 1 - cur, (s + 1) & 3, [&](int m) {
+        if (s < 3) deal<2 * NF, 3 * NM>(s * NM + m, [&](int r) { load_item(st_nxt, kw, 1 - cur, r); });  // past the end this reads a stale stage; the result is never used
+        deal<NPIECES, 4 * NM>(s * NM + m, [&](int q) { issue_piece(dma_lds, src, q); });
+      });
+    wait_vmcnt<(PS - 2) * NPIECES>();                   // own transfers of stage kt+2 have landed
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // and the fragments of stage kt+1 are in registers
+    __syncthreads();
+    st_cur = st_nxt;
+    st_nxt = ring_next(st_nxt);
+    advance(kt);
+  };
+  if constexpr (KW == 2) {  // (nkt >= 1: splits <= stages)
+    int kt = 0;
+    do {
+      pair_step(kt, 0);
+      if (kt + 1 < nkt) pair_step(kt + 1, 1);
+      kt += 2;
+    } while (kt < nkt);
+  }
+  for (int kt = 0; KW == 1 && kt < nkt; ++kt) {
     // chunk 0: sub-steps 0..3 (fragments of chunk 1 are fetched meanwhile)
-    load_chunk(st_cur, 1);
-    decode(D[1], 0, I1{});
-    mfma16(D[0]);
-    interleave();
-    decode(D[0], 0, I2{});
-    mfma16(D[1]);
-    interleave();
-    decode(D[1], 0, I3{});
-    mfma16(D[0]);
-    interleave();
-    decode(D[0], 1, I0{});
-    mfma16(D[1]);
-    interleave();
+#pragma unroll
+    for (int s = 0; s < 4; ++s)
+      w.substep(s & 1, s < 3 ? 0 : 1, (s + 1) & 3, [&](int m) {
+        if (s < 3) deal<2 * NF, 3 * NM>(s * NM + m, [&](int r) { load_item(st_cur, 1, 1, r); });
+      });
     // stage kt+1 must be complete (own DMA done, then everybody's; stages kt+2 .. kt+PS-2 may still
     // be in flight); stage kt-1 is free after this
     wait_vmcnt<(PS - 3) * NPIECES>();
@@ -702,32 +754,16 @@ __global__ __launch_bounds__(256, 1) void linear_nvfp4_tile256p_kernel(LinearArg
     // chunk 1: sub-steps 4..7 (chunk 0 of the next stage is fetched meanwhile); the DMA of stage
     // kt+PS-1 is spread over these sub-steps
     const uint32_t dma_lds = lds_base + st_dma;
-    decode(D[1], 1, I1{});
-    issue_quarter(dma_lds, src, 0);
-    mfma16(D[0]);
-    interleave();
-    load_chunk(st_nxt, 0);  // past the end this reads a stale stage; the result is never used
-    decode(D[0], 1, I2{});
-    issue_quarter(dma_lds, src, 1);
-    mfma16(D[1]);
-    interleave();
-    decode(D[1], 1, I3{});
-    issue_quarter(dma_lds, src, 2);
-    mfma16(D[0]);
-    interleave();
-    decode(D[0], 0, I0{});  // first sub-step of the next stage (unused after the last step)
-    issue_quarter(dma_lds, src, 3);
-    mfma16(D[1]);
-    interleave();
-    // rotate the stages; advance the sources unless they already sit on the last k-step
+#pragma unroll
+    for (int s = 0; s < 4; ++s)
+      w.substep(s & 1, s < 3 ? 1 : 0, (s + 1) & 3, [&](int m) {
+        if (s < 3) deal<2 * NF, 3 * NM>(s * NM + m, [&](int r) { load_item(st_nxt, 0, 0, r); });  // past the end this reads a stale stage; the result is never used
+        deal<NPIECES, 4 * NM>(s * NM + m, [&](int q) { issue_piece(dma_lds, src, q); });
+      });
     st_cur = st_nxt;
     st_nxt = ring_next(st_nxt);
     st_dma = ring_next(st_dma);
-    const bool adv = kt + PS <= last;
-    src.a += adv ? P_ROW : 0;
-    src.b += adv ? strideB : 0;
-#pragma unroll
-    for (int p2 = 0; p2 < NS; ++p2) src.s[p2] += adv ? strideS[p2] : 0;
+    advance(kt);
   }
   AC4K_LTL(2, wall_clock64());
 #ifdef AC4K_LINEAR_TIMELINE
@@ -748,12 +784,48 @@ __global__ __launch_bounds__(256, 1) void linear_nvfp4_tile256p_kernel(LinearArg
   // stages are reused, and every wave must be done reading them
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
   __syncthreads();
-  if (sk.partial) {  // split-K: raw fp32 sums of this K range; the reduce kernel scales and converts
-    store_tile<AC4K_DTYPE_FP32, BIAS_NONE, true, MI, NJ, PL::LDS_BYTES>(
-        acc, plds, sk.partial + (int64_t)blockIdx.y * a.M * a.N, nullptr, 1.0f, a.M, a.N, m0, n0, tn * BN);
+  auto store = [&](const f32x16 (&sums)[MI][NJ]) {
+    if (sk.partial) {  // split-K: raw fp32 sums of this K range; the reduce kernel scales and converts
+      store_tile<AC4K_DTYPE_FP32, BIAS_NONE, true, MI, NJ, PL::LDS_BYTES>(
+          sums, plds, sk.partial + (int64_t)blockIdx.y * a.M * a.N, nullptr, 1.0f, a.M, a.N, m0, n0, tn * BN);
+    } else {
+      store_tile<D_DT, BIAS_DT, false, MI, NJ, PL::LDS_BYTES>(sums, plds, a.D, a.bias, (*a.A_gs) * (*a.B_gs), a.M, a.N,
+                                                             m0, n0, tn * BN);
+    }
+  };
+  const auto &acc = w.acc;
+  if constexpr (KW == 1) {
+    store(acc);
   } else {
-    store_tile<D_DT, BIAS_DT, false, MI, NJ, PL::LDS_BYTES>(acc, plds, a.D, a.bias, (*a.A_gs) * (*a.B_gs), a.M, a.N,
-                                                           m0, n0, tn * BN);
+    // the waves of a pair exchange halves of their blocks and add them: wave (wm, wn) of the 2 x 2 grid keeps its own
+    static_assert(4 * MI * NJ * 4096 <= PL::LDS_BYTES, "the exchanged halves must fit in LDS");
+    float4 *xch = reinterpret_cast<float4 *>(plds) + lane;
+    auto xch_at = [&](int w, int i, int j, int g) { return xch + ((w * MI * NJ + i * NJ + j) * 4 + g) * 64; };
+#pragma unroll
+    for (int i = 0; i < MI; ++i)
+#pragma unroll
+      for (int j = 0; j < NJ; ++j)
+#pragma unroll
+        for (int g = 0; g < 4; ++g) {
+          const f32x16 &o = acc[PAIR_M ? MI + i : i][PAIR_N ? NJ + j : j];
+          *xch_at(swave ^ (PAIR_M ? 2 : 1), i, j, g) = make_float4(o[4 * g], o[4 * g + 1], o[4 * g + 2], o[4 * g + 3]);
+        }
+    __syncthreads();
+    f32x16 sums[MI][NJ];
+#pragma unroll
+    for (int i = 0; i < MI; ++i)
+#pragma unroll
+      for (int j = 0; j < NJ; ++j)
+#pragma unroll
+        for (int g = 0; g < 4; ++g) {
+          const float4 t = *xch_at(swave, i, j, g);
+          sums[i][j][4 * g] = acc[i][j][4 * g] + t.x;
+          sums[i][j][4 * g + 1] = acc[i][j][4 * g + 1] + t.y;
+          sums[i][j][4 * g + 2] = acc[i][j][4 * g + 2] + t.z;
+          sums[i][j][4 * g + 3] = acc[i][j][4 * g + 3] + t.w;
+        }
+    __syncthreads();  // what follows lies over the halves
+    store(sums);
   }
   AC4K_LTL(3, wall_clock64());
 }
@@ -773,13 +845,14 @@ static int allow_dynamic_lds(Kernel *kern, std::atomic<uint32_t> &done_mask, int
 }
 
 // LDS stages per tile shape: enough k-steps in flight to cover the memory latency
-constexpr int tile_stages(int mi, int nj) { return mi * nj >= 16 ? 3 : mi * nj >= 8 ? 4 : mi * nj >= 4 ? 6 : 8; }
+constexpr int tile_k_waves(int mi, int nj) { return mi * nj > 8 ? 1 : 2; }
+constexpr int tile_stages(int mi, int nj) { return mi * nj >= 16 ? 3 : mi * nj > 8 ? 4 : mi * nj == 8 ? 5 : mi * nj >= 4 ? 6 : 8; }
 
 template <int D_DT, int BIAS_DT, int MI, int NJ>
 static int launch_tile_p(const LinearArgs &a, const SplitK &sk, hipStream_t st) {
-  constexpr int PS = tile_stages(MI, NJ);
+  constexpr int PS = tile_stages(MI, NJ), KW = tile_k_waves(MI, NJ);
   const bool early = a.K % P_BK != 0;
-  auto *kern = early ? linear_nvfp4_tile256p_kernel<D_DT, BIAS_DT, MI, NJ, PS, true> : linear_nvfp4_tile256p_kernel<D_DT, BIAS_DT, MI, NJ, PS, false>;
+  auto *kern = early ? linear_nvfp4_tile256p_kernel<D_DT, BIAS_DT, MI, NJ, PS, KW, true> : linear_nvfp4_tile256p_kernel<D_DT, BIAS_DT, MI, NJ, PS, KW, false>;
   using PL = PLayout<64 * MI, 64 * NJ, PS>;
   static std::atomic<uint32_t> lds_ok[2];
   if (int rc = allow_dynamic_lds(kern, lds_ok[early], PL::LDS_BYTES)) return rc;
@@ -857,24 +930,22 @@ static int64_t tile_scratch_bytes(int64_t M, int64_t N, int64_t K) {
 // rounds of 256 workgroups, stages per range times the time of a 128-k stage of that tile, a prologue and epilogue per round
 // and for more than one range the partial sums and the second launch.  A stage takes `stage` as long as up to three fifths of the
 // CUs have work and grows with their share from there to stage + 0.4 power, as the clock comes down.  Fitted to 1000 random shapes of
-// M = 129 to 12000, N = 256 to 28672, K = 256 to 14336 with every tile and up to 32 ranges that fit the scratch (750 of them; the others
-// alike), and checked on 431 more: on average 0.3 % slower than the fastest of these plans, and on six of the 431 by 2 to 5 % slower than
-// the plan of tile_scratch_bytes, which on average is 3 % slower than the fastest and at most 36 %.  (Fitted to 50 shapes before: 0.5 %,
-// and 19 slower by 2 to 11 %, short K and few tiles above all: 285 x 504 x 1280 12.3 us, 11.0 with five ranges; 437 x 3968 x 6720 42.0
-// and 38.6.)  The sweeps held up to four rounds of
-// workgroups and 32 ranges, and so does the plan.
+// M = 129 to 12000, N = 256 to 28672, K = 256 to 14336 with every tile and up to 32 ranges that fit the scratch, and checked on 431 more: on
+// average 0.2 and 0.3 % slower than the fastest of these plans, 22 of the 431 by 2 to 10 % (few tiles in many ranges).  (The costs of the
+// loops before, with what pairs of waves now multiply together decoded by each of them: 0.8 %, 60 by 2 to 12 %.)  The sweeps held up to
+// four rounds of workgroups and 32 ranges, and so does the plan.
 // The tiles of 192 rows are what fills a round where 128 or 256 rows leave CUs idle (us, best of the other tiles / with
-// them): 4096 x 5120 x 5120 197.5 / 180.9, 7000 x 5120 x 5120 328.4 / 284.6, 6000 x 4096 x 4096 171.5 / 157.6, 300 x 14336 x 4096 50.9 / 45.3.
+// them, loops before these): 4096 x 5120 x 5120 197.5 / 180.9, 7000 x 5120 x 5120 328.4 / 284.6, 6000 x 4096 x 4096 171.5 / 157.6, 300 x 14336 x 4096 50.9 / 45.3.
 struct TileCost {
   int mi, nj;
   double stage, power, fixed;
 };
-constexpr TileCost TILE_COSTS[] = {{4, 4, 2.05, 2.015, 9.02},    {3, 4, 1.674, 1.595, 8.74}, {4, 2, 1.319, 0.798, 7.434}, {2, 4, 1.294, 0.908, 7.6},
-                                   {3, 2, 1.104, 0.584, 7.455}, {2, 2, 0.88, 0.257, 7.583}, {2, 1, 0.593, 0.139, 6.231}};
+constexpr TileCost TILE_COSTS[] = {{4, 4, 2.108, 2.15, 10.693}, {3, 4, 1.658, 1.677, 8.526}, {4, 2, 1.299, 0.913, 7.309}, {2, 4, 1.275, 0.884, 7.907},
+                                   {3, 2, 1.053, 0.532, 7.527}, {2, 2, 0.781, 0.281, 7.892}, {2, 1, 0.519, 0.14, 4.738}};
 static TilePlan tile_plan(int64_t M, int64_t N, int64_t K, int64_t scratch) {
   TilePlan best{};
   if (forced_tile_plan(M, N, K, best) && best.partial_bytes <= scratch) return best;
-  constexpr double ROUND_US = 3.29, SPLIT_US = 2.98, PARTIAL_BYTES_PER_US = 10.3e6;  // (8 bytes of a sum: written and read)
+  constexpr double ROUND_US = 4.77, SPLIT_US = 2.83, PARTIAL_BYTES_PER_US = 7.81e6;  // (8 bytes of a sum: written and read)
   const int stages = (int)ceil_div(K, P_BK);
   const int64_t sums_bytes = M * N * 4;
   const SplitCosts s = split_costs(M, N, stages, PARTIAL_BYTES_PER_US, SPLIT_US, scratch / sums_bytes < 32 ? (int)(scratch / sums_bytes) : 32);
@@ -969,7 +1040,7 @@ struct KWLayout {
   static constexpr int STAGE_BYTES = OFF_SFA + 4 * BM * 4;
   static constexpr int PS = (160 * 1024) / STAGE_BYTES < 8 ? (160 * 1024) / STAGE_BYTES : 8;  // ring slots
   static constexpr int LDS_BYTES = PS * STAGE_BYTES;
-  static constexpr int NROW = (BM + BN) / 8 / 4;          // 8-row transfers per wave per stage
+  static constexpr int NRW = BN / 8 / 4, NRA = BM / 8 / 4, NROW = NRW + NRA;  // 8-row transfers per wave per stage
   static constexpr int NSCW = BN / 64, NSCA = BM / 64;    // scale transfers per stage (1 KB each)
   static constexpr int NPIECES = NROW + 1;                // every wave issues the same count
   static constexpr int PPW = MI * NJ / 4;                 // 32 x 32 output blocks a wave finishes
@@ -986,12 +1057,11 @@ __global__ __launch_bounds__(256, 1) void linear_nvfp4_ksplit_kernel(LinearArgs 
   AC4K_LTL(0, wall_clock64());
   const int tid = threadIdx.x, lane = tid & 63, half = lane >> 5, r32 = lane & 31;
   const int swave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int64_t tiles_n = ceil_div(a.N, BN);
-  const int64_t tm = blockIdx.x / tiles_n, tn = blockIdx.x % tiles_n;
-  const int64_t m0 = tm * BM, n0 = tn * BN;
+  const uint32_t tiles_n = (uint32_t)ceil_div(a.N, BN), row_of_tiles = (uint32_t)__builtin_amdgcn_readfirstlane((int)(blockIdx.x / tiles_n));
+  const int64_t m0 = (int64_t)row_of_tiles * BM, n0 = (int64_t)(blockIdx.x - row_of_tiles * tiles_n) * BN;
   const int nst_all = (int)ceil_div(a.K, KW_BK);
-  const int s0 = (int)((int64_t)nst_all * blockIdx.y / sk.splits);
-  const int nst = (int)((int64_t)nst_all * (blockIdx.y + 1) / sk.splits) - s0;  // >= 1: splits <= stages
+  const StageRange range = stage_range(nst_all, blockIdx.y, sk.splits);
+  const int s0 = range.first, nst = range.count;  // >= 1: splits <= stages
   const StageWalk<TAIL> walk{s0, (int)(a.K >> 6)};
   const int64_t kb = a.K >> 1;
   // workgroup b starts at stage b % nst of its range and wraps around, so that the workgroups of a
@@ -1005,36 +1075,33 @@ __global__ __launch_bounds__(256, 1) void linear_nvfp4_ksplit_kernel(LinearArgs 
 
   // --- this wave's transfers of a stage
   const uint32_t lds_base = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) char *)kwlds;
-  // rows: transfer t = swave * NROW + q moves rows 8 t .. 8 t + 7 of the stage (weight rows first), lane l
-  // the piece of row l / 8 that belongs at position l % 8
+  // rows: a transfer moves eight rows of the stage, lane l the piece of row l / 8 that belongs at position l % 8; every wave as many of
+  // the weights (the first NRW) as of the activation
   // On a weight image (a.prepacked) a stage is two blocks of the row's 128-row band, 64 bytes of the row in
   // each, pieces at p ^ ((row >> 1) & 3), and the four chunk planes of scale dwords sit behind the blocks' data.
   const int64_t img_band_bytes = (a.K / W_BLOCK_K) * (int64_t)W_BLOCK_BYTES;
   uint32_t offR[L::NROW], ldsR[L::NROW];
-  const uint8_t *srcR[L::NROW];
-  int strR[L::NROW];  // bytes per step of the walk along k
 #pragma unroll
   for (int q = 0; q < L::NROW; ++q) {
-    const int t = swave * L::NROW + q;
-    const bool isW = t < BN / 8;
-    const int loc = (isW ? t : t - BN / 8) * 8 + (lane >> 3);
+    const bool isW = q < L::NRW;
+    const int t = isW ? swave * L::NRW + q : swave * L::NRA + q - L::NRW;
+    const int loc = t * 8 + (lane >> 3);
     const int pp = (lane & 7) ^ (loc & 7);  // the piece of the stage row that belongs at this lane's position
     if (isW && a.prepacked) {
       const int64_t wrow = n0 + loc;  // rows past N exist in the image (zeros)
       const int64_t band = wrow / W_BLOCK_ROWS, within = wrow % W_BLOCK_ROWS;
       offR[q] = (uint32_t)(band * img_band_bytes + (pp >> 2) * W_BLOCK_BYTES + within * 64 + (((pp & 3) ^ ((within >> 1) & 3)) * 16));
-      strR[q] = walk.step(W_BLOCK_BYTES / 2);
-      srcR[q] = uniform_ptr(a.B + walk.start(strR[q]));
     } else {
       const int64_t rows = isW ? a.N : a.M, first = isW ? n0 : m0;
       const int64_t row = first + loc < rows ? loc : rows - 1 - first;  // rows past the matrix read its last row
       offR[q] = (uint32_t)(row * kb + pp * 16);
-      strR[q] = walk.step(KW_ROW / 4);
-      srcR[q] = uniform_ptr((isW ? a.B + n0 * kb : a.A + m0 * kb) + walk.start(strR[q]));
     }
-    strR[q] = __builtin_amdgcn_readfirstlane(strR[q]);
-    ldsR[q] = (uint32_t)__builtin_amdgcn_readfirstlane(t * 1024);
+    ldsR[q] = (uint32_t)__builtin_amdgcn_readfirstlane((isW ? L::OFF_W : L::OFF_A) + t * 1024);
   }
+  // bytes per step of the walk along k
+  const int strideW = __builtin_amdgcn_readfirstlane(walk.step(a.prepacked ? W_BLOCK_BYTES / 2 : KW_ROW / 4)), strideA = walk.step(KW_ROW / 4);
+  const uint8_t *srcW = uniform_ptr((a.prepacked ? a.B : a.B + n0 * kb) + walk.start(strideW));
+  const uint8_t *srcA = uniform_ptr(a.A + m0 * kb + walk.start(strideA));
   // scales: one transfer is 256 dwords of the [chunk][row] picture, a lane the four dwords of rows
   // 4 g .. 4 g + 3 of one chunk (16 bytes of the scale tensor).  Transfers 0 .. NSCW - 1 are the weights',
   // the others the activation's; a wave past the last transfer repeats the last one.
@@ -1067,144 +1134,83 @@ __global__ __launch_bounds__(256, 1) void linear_nvfp4_ksplit_kernel(LinearArgs 
   // the loop keeps issuing, so that it stays free of branches and its wait counts stay fixed: those transfers
   // read the last stage again (cache hits) into slots nobody reads any more.
   // (`st` counts from the start of the range; a weight image has K % 128 == 0, so its stages start at whole blocks)
-  auto issue_piece = [&](uint32_t base, int st, int q) {
-    if (q < L::NROW)
-      dma16(srcR[q] + walk.offset(st, strR[q]), offR[q], base, ldsR[q]);
-    else
-      dma16(srcS + walk.offset(st, strideS), offS, base, ldsS);
+  struct Src {
+    const uint8_t *w, *a, *s;
   };
-  // the transfers of a stage are issued in four parts, one per 16-k sub-step
-  auto issue_part = [&](uint32_t base, int st, int part) {
-#pragma unroll
-    for (int q = 0; q < NP; ++q)
-      if (q * 4 / NP == part) issue_piece(base, st, q);
+  auto src_at = [&](int st) { return Src{srcW + walk.offset(st, strideW), srcA + walk.offset(st, strideA), srcS + walk.offset(st, strideS)}; };
+  auto issue_piece = [&](uint32_t base, const Src &p, int q) {
+    if (q < L::NROW) dma16(q < L::NRW ? p.w : p.a, offR[q], base, ldsR[q]);
+    else dma16(p.s, offS, base, ldsS);
   };
 
   // --- this wave's fragments of a stage: chunk swave; lane (r32, half) holds elements [32 half, 32 half + 32)
   // of the chunk of one row per fragment (16 packed bytes) and the two block scales that go with them
-  struct Frags {
-    uint4 x[MI], w[NJ];
-    uint32_t xs[MI], ws[NJ];
-    float wfac;
-  };
+  TileWave<MI, NJ> w;
+  w.clear();
   const int piece = swave * 2 + half;
   const int f_off = r32 * KW_ROW + ((piece ^ (r32 & 7)) * 16);  // rows 32 apart share the swizzle term
   const int ws_off = L::OFF_SFW + (swave * BN + r32) * 4 + half * 2;
   const int xs_off = L::OFF_SFA + (swave * BM + r32) * 4 + half * 2;
-  auto load_frags = [&](int slot, int step) {
-    const char *st = kwlds + slot * L::STAGE_BYTES;
-    Frags f;
-    f.wfac = walk.weight_factor(stage_of(step), swave);
-#pragma unroll
-    for (int j = 0; j < NJ; ++j) {
-      f.w[j] = *reinterpret_cast<const uint4 *>(st + L::OFF_W + f_off + j * 32 * KW_ROW);
-      f.ws[j] = *reinterpret_cast<const uint16_t *>(st + ws_off + j * 128);
-    }
-#pragma unroll
-    for (int i = 0; i < MI; ++i) {
-      f.x[i] = *reinterpret_cast<const uint4 *>(st + L::OFF_A + f_off + i * 32 * KW_ROW);
-      f.xs[i] = *reinterpret_cast<const uint16_t *>(st + xs_off + i * 128);
-    }
-    return f;
+  constexpr int NF = MI + NJ, NM = MI * NJ;
+  auto load_item = [&](uint32_t stage_off, int set, int r) {  // as in the tile kernel
+    const char *st = kwlds + stage_off;
+    const int f = r % NF;
+    if (r < NF) w.packed[set][f] = *reinterpret_cast<const uint4 *>(st + (f < MI ? L::OFF_A + f * 32 * KW_ROW : L::OFF_W + (f - MI) * 32 * KW_ROW) + f_off);
+    else w.sf[set][f] = *reinterpret_cast<const uint16_t *>(st + (f < MI ? xs_off + f * 128 : ws_off + (f - MI) * 128));
   };
-
-  f32x16 acc[MI][NJ];
-#pragma unroll
-  for (int i = 0; i < MI; ++i)
-#pragma unroll
-    for (int j = 0; j < NJ; ++j)
-#pragma unroll
-      for (int e = 0; e < 16; ++e) acc[i][j][e] = 0.0f;
-
-  DecFrags<MI, NJ> D[2];
-  auto decode = [&](DecFrags<MI, NJ> &d, const Frags &f, auto S) {
-    constexpr int s = decltype(S)::value;
-#pragma unroll
-    for (int j = 0; j < NJ; ++j)
-      d.b[j] = decode_dword<(s >= 2)>(dword_of<s>(f.w[j]), __builtin_amdgcn_cvt_scalef32_pk_f16_fp8(f.ws[j], f.wfac, false));
-#pragma unroll
-    for (int i = 0; i < MI; ++i)
-      d.a[i] = decode_dword<(s >= 2)>(dword_of<s>(f.x[i]), __builtin_amdgcn_cvt_scalef32_pk_f16_fp8(f.xs[i], 1.0f, false));
-  };
-  auto mfma_all = [&](const DecFrags<MI, NJ> &d) {
-#pragma unroll
-    for (int i = 0; i < MI; ++i)
-#pragma unroll
-      for (int jj = 0; jj < NJ; ++jj) {
-        const int j = (i & 1) ? NJ - 1 - jj : jj;  // neighbours share an operand
-        acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(d.b[j], d.a[i], acc[i][j], 0, 0, 0);  // D^T block
-      }
-  };
-  auto interleave = [&]() {  // the decode of the next sub-step rides in the shadow of the MFMAs
-    constexpr int NMFMA = MI * NJ, NVALU = 8 * (MI + NJ) + (MI + NJ);
-    constexpr int PER = (NVALU + NMFMA - 1) / NMFMA;
-#pragma unroll
-    for (int g = 0; g < NMFMA; ++g) {
-      __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-      __builtin_amdgcn_sched_group_barrier(0x002, PER, 0);
-    }
-    __builtin_amdgcn_sched_barrier(0);
-  };
-  using I0 = std::integral_constant<int, 0>;
-  using I1 = std::integral_constant<int, 1>;
-  using I2 = std::integral_constant<int, 2>;
-  using I3 = std::integral_constant<int, 3>;
 
   // prologue: the first PS stages in flight, stage 0 landed and its fragments in registers (every wave's,
   // before slot 0 is refilled), then stage 1 landed
 #pragma unroll
   for (int d = 0; d < PS; ++d) {
+    const Src p = src_at(stage_of(d));
 #pragma unroll
-    for (int q = 0; q < NP; ++q) issue_piece(lds_base + d * L::STAGE_BYTES, stage_of(d), q);
+    for (int q = 0; q < NP; ++q) issue_piece(lds_base + d * L::STAGE_BYTES, p, q);
   }
   wait_vmcnt<(PS - 1) * NP>();
   __syncthreads();
-  Frags F0 = load_frags(0, 0), F1;
-  decode(D[0], F0, I0{});
+  float wfac = walk.weight_factor(stage_of(0), swave);  // of the stage whose fragments were read last
+#pragma unroll
+  for (int r = 0; r < 2 * NF; ++r) load_item(0, 0, r);
+#pragma unroll
+  for (int e = 0; e < 4 * NF; ++e) w.decode_item(0, 0, 0, e, wfac);
   wait_vmcnt<(PS - 2) * NP>();
   asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
   __syncthreads();
 
-  int slot_cur = 0, slot_next = 1;
+  uint32_t st_cur = 0, st_nxt = L::STAGE_BYTES;  // LDS offsets of the stages at hand and next
 #ifdef AC4K_LINEAR_TIMELINE
   const uint64_t tl_c0 = __builtin_readcyclecounter();
 #endif
   AC4K_LTL(1, wall_clock64());
-  // one stage: `cur` holds its fragments, `nxt` receives those of the next one (two named sets that swap
-  // roles, so that no register is copied between stages)
-  auto stage_step = [&](const Frags &cur, Frags &nxt, int s) {
+  // one stage: set `cur` holds its fragments, the other receives those of the next one
+  auto stage_step = [&](int s, int cur) {
     // The slot of this stage is free (every wave had its fragments in registers before the previous
     // barrier): stage s + PS goes there.
-    const int st_new = stage_of(s + PS);
-    const uint32_t base_new = lds_base + slot_cur * L::STAGE_BYTES;
+    const uint32_t base_new = lds_base + st_cur;
+    const Src src = src_at(stage_of(s + PS));
+    wfac = walk.weight_factor(stage_of(s + 1), swave);
     // fragments of the next stage (it landed before the previous barrier) travel from LDS while this
     // one is decoded and multiplied (past the range: a stage nobody uses)
-    nxt = load_frags(slot_next, s + 1);
-    decode(D[1], cur, I1{});
-    issue_part(base_new, st_new, 0);
-    mfma_all(D[0]);
-    interleave();
-    decode(D[0], cur, I2{});
-    issue_part(base_new, st_new, 1);
-    mfma_all(D[1]);
-    interleave();
-    decode(D[1], cur, I3{});
-    issue_part(base_new, st_new, 2);
-    mfma_all(D[0]);
-    interleave();
-    decode(D[0], nxt, I0{});
-    issue_part(base_new, st_new, 3);
-    mfma_all(D[1]);
-    interleave();
+#pragma unroll
+    for (int sub = 0; sub < 4; ++sub)
+      w.substep(sub & 1, sub < 3 ? cur : 1 - cur, (sub + 1) & 3, [&](int m) {
+        if (sub < 3) deal<2 * NF, 3 * NM>(sub * NM + m, [&](int r) { load_item(st_nxt, 1 - cur, r); });
+        deal<NP, 4 * NM>(sub * NM + m, [&](int q) { issue_piece(base_new, src, q); });
+      }, wfac);
     wait_vmcnt<(PS - 2) * NP>();                        // own transfers of stage s + 2 have landed
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // and the fragments of stage s + 1 are in registers
     __syncthreads();
-    slot_cur = slot_next;
-    slot_next = slot_next + 1 == PS ? 0 : slot_next + 1;
+    st_cur = st_nxt;
+    st_nxt = st_nxt + L::STAGE_BYTES == (uint32_t)L::LDS_BYTES ? 0 : st_nxt + L::STAGE_BYTES;
   };
-  for (int s = 0; s < nst; s += 2) {
-    stage_step(F0, F1, s);
-    if (s + 1 < nst) stage_step(F1, F0, s + 1);
+  {
+    int s = 0;
+    do {  // (nst >= 1)
+      stage_step(s, 0);
+      if (s + 1 < nst) stage_step(s + 1, 1);
+      s += 2;
+    } while (s < nst);
   }
   AC4K_LTL(2, wall_clock64());
 #ifdef AC4K_LINEAR_TIMELINE
@@ -1216,6 +1222,7 @@ __global__ __launch_bounds__(256, 1) void linear_nvfp4_ksplit_kernel(LinearArgs 
   // --- the four k parts meet: wave d finishes blocks p = d * PPW + q (i = p / NJ, j = p % NJ).
   // acc[i][j]: lane l, element e <-> m = 32 i + (l & 31), n = 32 j + (e >> 2) * 8 + (l >> 5) * 4 + (e & 3)
   constexpr int PPW = L::PPW;
+  const auto &acc = w.acc;
   float4 *xch = reinterpret_cast<float4 *>(kwlds);
   auto xch_at = [&](int d, int src, int q, int g) { return xch + ((((d * 4 + src) * PPW + q) * 4 + g) * 64 + lane); };
 #pragma unroll

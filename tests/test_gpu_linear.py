@@ -628,3 +628,33 @@ def test_operands_aligned_to_eight_bytes(m, n, k):
     for a, b in ((shifted(aq), bq), (aq, shifted(bq))):
         out = ops().linear(*a, *b, out=torch.empty((m, n), dtype=torch.float32, device="cuda"))
         torch.testing.assert_close(out.cpu(), ref, atol=1e-5, rtol=1e-4)
+
+
+# K ranges of one stage up to two more than the ring of a tile holds: shorter than the ring (fetched and waited for as a whole), as
+# long, an odd and an even number of steps; and, where the two waves of a pair take a half of every stage, sums that only both hold
+@pytest.mark.parametrize("mi,nj", sorted({p[:2] for p in TILE_PLANS}))
+def test_ranges_about_as_long_as_the_stage_ring(mi, nj, linear_tuning):
+    linear_tuning(mi, nj, 1)
+    for stages in range(1, 11):
+        check_tight(64 * mi + 37, 64 * nj + 130, 128 * stages, seed=stages)
+    linear_tuning(mi, nj, 3)  # ranges of three and four stages
+    check_tight(64 * mi + 37, 64 * nj + 130, 1280, seed=1)
+
+
+# scale tensors on four bytes: the tile kernel fetches 16 bytes of them at a time
+@pytest.mark.parametrize("mi,nj", sorted({p[:2] for p in TILE_PLANS}))
+@pytest.mark.parametrize("at", [4, 8, 12])
+def test_scales_aligned_to_four_bytes(mi, nj, at, linear_tuning):
+    def shifted(q):
+        buf = torch.empty(q[1].numel() + 16, dtype=torch.uint8, device="cuda")
+        sf = buf[at:at + q[1].numel()].view(q[1].shape)
+        sf.copy_(q[1].view(torch.uint8))
+        assert sf.data_ptr() % 16 == at
+        return q[0], sf.view(torch.float8_e4m3fn), q[2]
+
+    linear_tuning(mi, nj, 1)
+    for k in (640, 704):
+        m, n = 64 * mi + 37, 64 * nj + 130
+        aq, bq = gpu_quant(make_input((m, k), seed=m)), gpu_quant(make_input((n, k), seed=n, std=0.02))
+        ref = ops().linear(*aq, *bq)
+        assert torch.equal(ops().linear(*shifted(aq), *shifted(bq)), ref), k
