@@ -1377,7 +1377,7 @@ struct SkinnyArgs {
   float *partial;      // [splitK][M][N]
   int64_t M, N, K, Np;
   int ks_len, split_k;
-  int prepacked = 0;  // B is a weight image (LDS-ring kernel only), B_sf unused
+  int prepacked = 0;  // B is a weight image (LDS-ring kernel, 16-row workgroups), B_sf unused
 };
 
 constexpr int SK_ROWS = 128;   // weight rows per workgroup
@@ -2085,20 +2085,26 @@ __global__ __launch_bounds__(ST_THREADS, 1) void linear_nvfp4_stream64_kernel(Sk
 // 16 x 4096 x 14336, weights from HBM, 17.8 -> 11.4 us (64 rows, K split in four, and the second launch before), M = 1 15.8 -> 10.4; 16 x 4096 x 4096 10.2 -> 5.1; 1 x 20000 x 2880 23.4 -> 11.2; 32 x 1024 x 1024
 // 7.6 -> 3.2.  Three steps ahead and two workgroups on a CU: two more cost 0.7 us at 16 x 4096 x 14336 in registers, sixteen waves 2.5 us at
 // 1 x 14336 x 4096, four waves 3 us at 16 x 4096 x 14336; loads past the caches lose where the activation is read again.
+// On a weight image a wave's step is one kilobyte of a block and its scales lie behind it: 16 x 4096 x 14336 10.1 us (plain 11.2), 16 x 14336 x 4096
+// 10.9 (12.5), 8 x 20480 x 8192 23.4 (26.8); the ring kernel, which took all of M <= 32 there, 18.1, 16.1 and 38.7.
 // ===========================================================================
 constexpr int R16_DEPTH = 3;
 
-// MT: tiles of 16 activation rows.  TAIL: K is no multiple of 128.
-template <int D_DT, int BIAS_DT, int MT, bool TAIL>
+// MT: tiles of 16 activation rows.  TAIL: K is no multiple of 128.  PRE: B is a weight image, whose blocks hold a step of 128 rows each.
+template <int D_DT, int BIAS_DT, int MT, bool TAIL, bool PRE>
 __global__ __launch_bounds__(64 * R16_WAVES, 2) void linear_nvfp4_rows16_kernel(SkinnyArgs a) {
+  static_assert(!(PRE && TAIL), "an image has whole steps");
   __shared__ float4 part[R16_WAVES][MT][64];
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), r = lane & 15, g = lane >> 4;
   const int64_t n0 = (int64_t)blockIdx.x * R16_ROWS, kb = a.K >> 1;
   const int nst = (int)ceil_div(a.K, R16_STEP);
   const int cnt = (nst - wave + R16_WAVES - 1) / R16_WAVES;  // steps of this wave; none where K is short
   const int wr = n0 + r < a.N ? r : (int)(a.N - 1 - n0);  // rows past N read the last row; their outputs are never stored
-  const uint8_t *const w_src = uniform_ptr(a.B + n0 * kb), *const ws_src = uniform_ptr(reinterpret_cast<const uint8_t *>(a.B_sf) + n0 * 4);
-  const uint32_t w_row = (uint32_t)(wr * kb), ws_row = (uint32_t)(wr * 4);
+  const uint8_t *const w_src = uniform_ptr(PRE ? a.B + n0 / W_BLOCK_ROWS * nst * W_BLOCK_BYTES : a.B + n0 * kb);
+  const uint8_t *const ws_src = uniform_ptr(PRE ? nullptr : reinterpret_cast<const uint8_t *>(a.B_sf) + n0 * 4);
+  const int in_block = (int)(n0 % W_BLOCK_ROWS) + r;  // PRE: rows past N exist (zeros)
+  const uint32_t w_row = PRE ? in_block * (W_BLOCK_K / 2) + ((g ^ ((in_block >> 1) & 3)) * 16) : (uint32_t)(wr * kb);
+  const uint32_t ws_row = PRE ? W_BLOCK_DATA + (g >> 1) * (W_BLOCK_ROWS * 4) + in_block * 4 + (g & 1) * 2 : (uint32_t)(wr * 4);
   uint32_t x_row[MT], xs_row[MT];
 #pragma unroll
   for (int i = 0; i < MT; ++i) {
@@ -2113,8 +2119,13 @@ __global__ __launch_bounds__(64 * R16_WAVES, 2) void linear_nvfp4_rows16_kernel(
     const int s = wave + t * R16_WAVES;
     const uint32_t gg = TAIL && s == nst - 1 ? g & 1 : g;
     const int64_t at = (int64_t)s * (R16_STEP / 2);
-    st.w = *reinterpret_cast<const uint4 *>(w_src + at + (w_row + gg * 16));
-    st.ws = *reinterpret_cast<const uint16_t *>(ws_src + (int64_t)(2 * s) * a.Np * 4 + ((gg >> 1) * (uint32_t)a.Np * 4 + ws_row + (gg & 1) * 2));
+    if constexpr (PRE) {
+      st.w = *reinterpret_cast<const uint4 *>(w_src + (int64_t)s * W_BLOCK_BYTES + w_row);
+      st.ws = *reinterpret_cast<const uint16_t *>(w_src + (int64_t)s * W_BLOCK_BYTES + ws_row);
+    } else {
+      st.w = *reinterpret_cast<const uint4 *>(w_src + at + (w_row + gg * 16));
+      st.ws = *reinterpret_cast<const uint16_t *>(ws_src + (int64_t)(2 * s) * a.Np * 4 + ((gg >> 1) * (uint32_t)a.Np * 4 + ws_row + (gg & 1) * 2));
+    }
 #pragma unroll
     for (int i = 0; i < MT; ++i) {
       st.x[i] = *reinterpret_cast<const uint4 *>(a.Aq + at + (x_row[i] + gg * 16));
@@ -2329,8 +2340,9 @@ static int launch_skinny(const SkinnyArgs &a, const SkinnyPlan &p, hipStream_t s
                                 a.bias, a.M, a.N, a.K, a.Mp, a.Np}, D_DT, BIAS_DT, st);
   if (p.rows16) {
     const bool tail = a.K % R16_STEP != 0;
-    auto *kern = a.M <= 16 ? tail ? linear_nvfp4_rows16_kernel<D_DT, BIAS_DT, 1, true> : linear_nvfp4_rows16_kernel<D_DT, BIAS_DT, 1, false>
-                           : tail ? linear_nvfp4_rows16_kernel<D_DT, BIAS_DT, 2, true> : linear_nvfp4_rows16_kernel<D_DT, BIAS_DT, 2, false>;
+    auto *kern = a.M <= 16 ? tail ? linear_nvfp4_rows16_kernel<D_DT, BIAS_DT, 1, true, false> : linear_nvfp4_rows16_kernel<D_DT, BIAS_DT, 1, false, false>
+                           : tail ? linear_nvfp4_rows16_kernel<D_DT, BIAS_DT, 2, true, false> : linear_nvfp4_rows16_kernel<D_DT, BIAS_DT, 2, false, false>;
+    if (a.prepacked) kern = a.M <= 16 ? linear_nvfp4_rows16_kernel<D_DT, BIAS_DT, 1, false, true> : linear_nvfp4_rows16_kernel<D_DT, BIAS_DT, 2, false, true>;
     hipLaunchKernelGGL(kern, dim3((unsigned)ceil_div(a.N, R16_ROWS)), dim3(64 * R16_WAVES), 0, st, a);
     return 0;
   }
@@ -2766,7 +2778,7 @@ static int64_t weight_image_bytes(int64_t N, int64_t K) {
   return ceil_div(N, W_BLOCK_ROWS) * (K / W_BLOCK_K) * W_BLOCK_BYTES;
 }
 
-// How a linear on a weight image runs: the LDS-ring kernel for decode-sized M (K >= 256), the K-split-waves
+// How a linear on a weight image runs: the LDS-ring kernel or 16-row workgroups for decode-sized M (K >= 256), the K-split-waves
 // kernel for 32 < M <= 128, the tile kernel otherwise, split along K when the workspace entry point of the plain
 // layout would split too.
 struct PrepackedPlan {
@@ -2776,6 +2788,22 @@ struct PrepackedPlan {
   TilePlan tp;
   int64_t partial_bytes;
 };
+// 16-row workgroups on an image, where a step of a wave's rows is one run of a kilobyte, against its ring kernel, by these estimates (us,
+// weights from HBM, fitted to 160 shapes of N = 256 to 28672, K = 256 to 16384 and M = 1 to 32).  Ring / 16 rows as measured:
+// M = 1, 4096 x 4096 10.5 / 4.3, 28672 x 8192 32.3 / 28.1; M = 8, 28672 x 8192 32.5 / 31.2; M = 16, 4096 x 14336 18.1 / 10.1, 14336 x 4096 16.1 / 10.9,
+// 28672 x 8192 33.0 / 35.0, 27264 x 256 5.3 / 4.7; M = 20, 12288 x 12288 39.5 / 30.6, 27264 x 256 5.4 / 6.9, 28672 x 4096 21.0 / 24.1; M = 32,
+// 4096 x 14336 17.8 / 14.8, 2688 x 14208 14.8 / 11.8, 14336 x 14336 33.5 / 47.6, 256 x 14336 10.4 / 12.4.
+static bool rows16_faster_image(int64_t M, int64_t N, int64_t K, const SkinnyPlan &p) {
+  const double m = (double)M, cus = (double)decode_cu_count(), million = 1e-6 * (double)N * (double)K;
+  const double steps = (double)ceil_div(ceil_div(K, R16_STEP), R16_WAVES), wgs = (double)ceil_div(N, R16_ROWS) / (2.0 * cus);
+  const double last = wgs > 1.0 && wgs < 2.0 ? sqrt(2.0 / wgs) : 1.0;  // a second round that is not full
+  const double rows16 = M <= 16 ? fmax(0.35 * wgs + (0.10 + 0.0022 * m) * million, (0.37 + 0.003 * m) * steps)
+                                : fmax(last * (wgs + (0.126 + 0.0016 * m) * million), (0.5 + 0.006 * m) * steps);
+  const double rounds = ceil((double)(p.groups * p.split_k) / cus), stages = (double)ceil_div(ceil_div(K, ST_BK), p.split_k);
+  const double ring = 4.2 + 0.03 * m + 0.8 * stages + 0.3 * fmin(stages, 8.0);
+  return 2.5 + rows16 < rounds * ring + (p.split_k > 1 ? 4.0 : 0.0);
+}
+
 static bool prepacked_plan(int64_t M, int64_t N, int64_t K, PrepackedPlan &p) {
   const int64_t bytes = weight_image_bytes(N, K);
   if (M < 1 || bytes == 0 || bytes >= (1ll << 32) || (K >> 1) * 256 >= (1ll << 31) || N >= (1ll << 27)) return false;
@@ -2783,8 +2811,9 @@ static bool prepacked_plan(int64_t M, int64_t N, int64_t K, PrepackedPlan &p) {
   p.mid = !p.ring && ksplit_shape(M, N, K);
   if (p.ring) {
     plan_lds_ring(M, N, K, p.sp);
-    p.sp.rows16 = p.sp.fused = p.sp.lds_x = false;
-    p.partial_bytes = p.sp.partial_bytes;
+    p.sp.rows16 = !forced_decode_kernel() && rows16_faster_image(M, N, K, p.sp);
+    p.sp.fused = p.sp.lds_x = false;
+    p.partial_bytes = p.sp.rows16 ? 0 : p.sp.partial_bytes;
   } else if (p.mid) {
     p.kp = ksplit_plan(M, N, K, true);
     p.partial_bytes = p.kp.partial_bytes;

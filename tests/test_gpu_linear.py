@@ -658,3 +658,23 @@ def test_scales_aligned_to_four_bytes(mi, nj, at, linear_tuning):
         aq, bq = gpu_quant(make_input((m, k), seed=m)), gpu_quant(make_input((n, k), seed=n, std=0.02))
         ref = ops().linear(*aq, *bq)
         assert torch.equal(ops().linear(*shifted(aq), *shifted(bq)), ref), k
+
+
+# 16 weight rows per workgroup on a weight image: bands that end early, one and two tiles of activation rows, waves with no step and
+# every remainder of the steps, the last band of several; the same sums as on the plain layout
+@pytest.mark.parametrize("m", [1, 15, 16, 17, 32])
+@pytest.mark.parametrize("n,k", [(1, 256), (16, 384), (130, 1024), (129, 1152), (4, 2944), (1000, 3072), (300, 4224)])
+def test_sixteen_row_workgroups_on_an_image(m, n, k):
+    import ctypes
+    from ac4k_kernel_amd import _lib
+    lib = _lib.load()
+    assert lib.ac4k_linear_nvfp4_prepacked_workspace_bytes(m, n, k) == 0
+    check_tight(m, n, k, seed=m + k, image=True)
+    aq, bq = gpu_quant(make_input((m, k), seed=m)), gpu_quant(make_input((n, k), seed=n, std=0.02))
+    image = ops().prepack_weight(bq[0], bq[1])
+    for dt in (torch.bfloat16, torch.float16, torch.float32):
+        bias = make_input((1, n), seed=3).to(dt).cuda()
+        out = ops().linear_prepacked(*aq, image, bq[2], bias=bias, out=torch.empty((m, n), dtype=dt, device="cuda"))
+        torch.testing.assert_close(out.cpu(), T.linear_nvfp4(*cpu(aq), *cpu(bq), bias=bias.cpu(), out_dtype=dt), atol=ATOL, rtol=RTOL)
+        if lib.ac4k_debug_linear_decode_kernel(m, n, k, ctypes.byref(ctypes.c_int())) == 4:
+            assert torch.equal(ops().linear(*aq, *bq, bias=bias, out=torch.empty((m, n), dtype=dt, device="cuda")), out)
