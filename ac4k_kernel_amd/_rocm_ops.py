@@ -40,12 +40,13 @@ def _check_tensor(t, dtype, name: str, suffix: str = "") -> None:
 
 
 _raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+_current_device = getattr(torch._C, "_cuda_getDevice", torch.cuda.current_device)  # operands on a GPU: torch is initialised
 
 
 def _stream() -> int:
     """hipStream_t of torch's current stream on the current device."""
     if _raw_stream is not None:
-        return _raw_stream(torch.cuda.current_device())
+        return _raw_stream(_current_device())
     return torch.cuda.current_stream().cuda_stream
 
 
@@ -60,6 +61,10 @@ def _quant_geometry(inp: torch.Tensor, cross_dim: int, reduce_dim: int):
     _check(0 <= cross_dim < inp.dim(), "cross_dim must be less than in.dim()")
     _check(0 <= reduce_dim < inp.dim(), "reduce_dim must be less than in.dim()")
     _check(cross_dim != reduce_dim, "cross_dim and reduce_dim must be different")
+    if inp.dim() == 2:
+        shape, stride = inp.shape, inp.stride()
+        _check(shape[0] > 0 and shape[1] > 0, "in must not be empty")
+        return [], (1, 1, shape[cross_dim], shape[reduce_dim], 0, 0, stride[cross_dim], stride[reduce_dim])
     shape, stride = list(inp.shape), list(inp.stride())
     lead = [i for i in range(inp.dim()) if i not in (cross_dim, reduce_dim)]
     lead_shape = [shape[i] for i in lead]
@@ -106,6 +111,22 @@ def quantize_nvfp4_with_global_scale(out, sf, global_scale, inp, cross_dim: int,
            "out must have shape [.., cross, align_up(reduce, 64) / 2]")
     _check_tensor(sf, torch.float8_e4m3fn, "sf")
     _check(list(sf.shape) == lead_shape + [_align_up(K, 64) // 64, _align_up(R, 16), 4], "meet invalid sf shape")
+    _quantize_nvfp4_bf16(out, sf, global_scale, inp, geom, swizzle, max_scale)
+
+
+def quantize_nvfp4_new(inp, cross_dim: int, reduce_dim: int, swizzle: bool, max_scale: float):
+    """The same into tensors made here, which need no checks: (out, sf, global_scale)."""
+    lead_shape, geom = _quant_geometry(inp, cross_dim, reduce_dim)
+    R, Kp = geom[2], (geom[3] + 63) // 64 * 64
+    dev = inp.device
+    out = torch.empty([*lead_shape, R, Kp // 2], dtype=torch.uint8, device=dev)
+    sf = torch.empty([*lead_shape, Kp // 64, (R + 15) // 16 * 16, 4], dtype=torch.float8_e4m3fn, device=dev)
+    global_scale = torch.empty((), dtype=torch.float32, device=dev)
+    _quantize_nvfp4_bf16(out, sf, global_scale, inp, geom, swizzle, max_scale)
+    return out, sf, global_scale
+
+
+def _quantize_nvfp4_bf16(out, sf, global_scale, inp, geom, swizzle, max_scale) -> None:
     _lib.check(_L.ac4k_quantize_nvfp4_bf16(out.data_ptr(), sf.data_ptr(), global_scale.data_ptr(), inp.data_ptr(),
                                            *geom, int(bool(swizzle)), float(max_scale), _stream()))
 
@@ -133,6 +154,14 @@ def quantize_int8(out, sf, inp, scale_max, cross_dim: int, reduce_dim: int) -> N
 
 
 def _check_linear_operand(x, x_sf, x_gs, rows, name):
+    # one pass over the attributes of a well-formed operand; what is wrong with another one is found out below
+    if isinstance(x, torch.Tensor) and isinstance(x_sf, torch.Tensor) and isinstance(x_gs, torch.Tensor) and x.dim() == 2:
+        K = x.size(1) * 2
+        if (x.dtype is torch.uint8 and x.is_cuda and x.is_contiguous()
+                and x_sf.dtype is torch.float8_e4m3fn and x_sf.is_cuda and x_sf.is_contiguous()
+                and x_sf.shape == ((K + 63) // 64, (rows + 15) // 16 * 16, 4)
+                and x_gs.dtype is torch.float32 and x_gs.is_cuda and x_gs.dim() == 0):
+            return K
     _check(x.dim() == 2, "{} must be a 2d matrix", name)
     _check_tensor(x, torch.uint8, name)
     K = x.size(1) * 2
@@ -155,32 +184,43 @@ def _bias_args(bias, N):
     return bias.data_ptr(), _DTYPE_TAG[bias.dtype]
 
 
+def _check_output(D):
+    if isinstance(D, torch.Tensor) and D.dim() == 2 and D.is_cuda and D.is_contiguous():
+        tag = _DTYPE_TAG.get(D.dtype)
+        if tag is not None:
+            return D.size(0), D.size(1), tag
+    _check(isinstance(D, torch.Tensor) and D.dim() == 2, "d must be a 2d matrix")
+    _check(D.dtype in _DTYPE_TAG, "d must be bfloat16, half or float")
+    _check(False, "d must be contiguous")
+
+
 def linear_nvfp4(D, A, A_sf, A_global_scale, B, B_sf, B_global_scale, bias=None) -> None:
     """Checks of linear_nvfp4.cu:759-805.  Shapes for which the library asks for scratch (too few output
     tiles for the GPU, long K) get a workspace tensor and the split-K kernels; everything else goes to
     the reference-shaped entry point, which allocates nothing and picks its kernel by shape."""
-    _check(isinstance(D, torch.Tensor) and D.dim() == 2, "d must be a 2d matrix")
-    _check(D.dtype in _DTYPE_TAG, "d must be bfloat16, half or float")
-    _check(D.is_cuda and D.is_contiguous(), "d must be contiguous")
-    M, N = D.shape
-    _check(A.dim() == 2 and A.size(0) == M, "A size(0) must be {}", M)
+    M, N, tag = _check_output(D)
+    if A.dim() != 2 or A.size(0) != M:
+        _check(False, "A size(0) must be {}", M)
     K = _check_linear_operand(A, A_sf, A_global_scale, M, "a")
-    _check(K % 16 == 0, "A size(1)*2 must be multiple of 16 but see {}", K)
-    _check(B.dim() == 2 and B.size(1) == A.size(1), "B size(1) must equal A size(1)")
-    _check(B.size(0) == N, "B size(0) must be {}", N)
+    if K % 16 != 0:
+        _check(False, "A size(1)*2 must be multiple of 16 but see {}", K)
+    if B.dim() != 2 or B.size(1) * 2 != K:
+        _check(False, "B size(1) must equal A size(1)")
+    if B.size(0) != N:
+        _check(False, "B size(0) must be {}", N)
     _check_linear_operand(B, B_sf, B_global_scale, N, "b")
-    bias_ptr, bias_tag = _bias_args(bias, N)
+    bias_ptr, bias_tag = (None, 0) if bias is None else _bias_args(bias, N)
     if M == 0 or N == 0:
         return
     nbytes = _L.ac4k_linear_nvfp4_scratch_bytes(M, N, K)
     if nbytes > 0:
-        ws = torch.empty((nbytes,), dtype=torch.uint8, device=D.device)
-        _lib.check(_L.ac4k_linear_nvfp4_workspace(D.data_ptr(), _DTYPE_TAG[D.dtype], A.data_ptr(), A_sf.data_ptr(),
+        ws = D.new_empty((nbytes,), dtype=torch.uint8)
+        _lib.check(_L.ac4k_linear_nvfp4_workspace(D.data_ptr(), tag, A.data_ptr(), A_sf.data_ptr(),
                                                   A_global_scale.data_ptr(), B.data_ptr(), B_sf.data_ptr(),
                                                   B_global_scale.data_ptr(), bias_ptr, bias_tag, M, N, K,
                                                   ws.data_ptr(), nbytes, _stream()))
         return
-    _lib.check(_L.ac4k_linear_nvfp4(D.data_ptr(), _DTYPE_TAG[D.dtype], A.data_ptr(), A_sf.data_ptr(),
+    _lib.check(_L.ac4k_linear_nvfp4(D.data_ptr(), tag, A.data_ptr(), A_sf.data_ptr(),
                                     A_global_scale.data_ptr(), B.data_ptr(), B_sf.data_ptr(),
                                     B_global_scale.data_ptr(), bias_ptr, bias_tag, M, N, K, _stream()))
 
@@ -203,10 +243,7 @@ def prepack_weight_nvfp4(B, B_sf) -> torch.Tensor:
 
 def linear_nvfp4_prepacked(D, A, A_sf, A_global_scale, W_image, B_global_scale, bias=None) -> None:
     """linear_nvfp4 on a weight image made by prepack_weight_nvfp4 (N = D.size(1), K = 2 * A.size(1))."""
-    _check(isinstance(D, torch.Tensor) and D.dim() == 2, "d must be a 2d matrix")
-    _check(D.dtype in _DTYPE_TAG, "d must be bfloat16, half or float")
-    _check(D.is_cuda and D.is_contiguous(), "d must be contiguous")
-    M, N = D.shape
+    M, N, tag = _check_output(D)
     _check(A.dim() == 2 and A.size(0) == M, "A size(0) must be {}", M)
     K = _check_linear_operand(A, A_sf, A_global_scale, M, "a")
     _check_tensor(W_image, torch.uint8, "w_image")
@@ -218,8 +255,8 @@ def linear_nvfp4_prepacked(D, A, A_sf, A_global_scale, W_image, B_global_scale, 
     if M == 0:
         return
     nbytes = _L.ac4k_linear_nvfp4_prepacked_workspace_bytes(M, N, K)
-    ws = torch.empty((nbytes,), dtype=torch.uint8, device=D.device) if nbytes > 0 else None
-    _lib.check(_L.ac4k_linear_nvfp4_prepacked(D.data_ptr(), _DTYPE_TAG[D.dtype], A.data_ptr(), A_sf.data_ptr(),
+    ws = D.new_empty((nbytes,), dtype=torch.uint8) if nbytes > 0 else None
+    _lib.check(_L.ac4k_linear_nvfp4_prepacked(D.data_ptr(), tag, A.data_ptr(), A_sf.data_ptr(),
                                               A_global_scale.data_ptr(), W_image.data_ptr(),
                                               B_global_scale.data_ptr(), bias_ptr, bias_tag, M, N, K,
                                               None if ws is None else ws.data_ptr(), nbytes, _stream()))
@@ -228,15 +265,8 @@ def linear_nvfp4_prepacked(D, A, A_sf, A_global_scale, W_image, B_global_scale, 
 def linear_nvfp4_fused(D, X, X_q, X_sf, X_global_scale, B, B_sf, B_global_scale, bias=None) -> None:
     """quantize(X, 0, 1) + linear_nvfp4 for a bf16 activation X [M, K], 1 <= M <= 32;
     X_q / X_sf / X_global_scale receive the quantized activation."""
-    _check(isinstance(D, torch.Tensor) and D.dim() == 2, "d must be a 2d matrix")
-    _check(D.dtype in _DTYPE_TAG, "d must be bfloat16, half or float")
-    _check(D.is_cuda and D.is_contiguous(), "d must be contiguous")
-    M, N = D.shape
-    _check_tensor(X, torch.bfloat16, "x")
-    _check(X.dim() == 2 and X.size(0) == M, "x must be [{}, K]", M)
-    _check(1 <= M <= 32, "the fused linear takes 1 <= M <= 32")
-    K = X.size(1)
-    _check(K % 64 == 0, "K must be a multiple of 64")
+    M, N, tag = _check_output(D)
+    K = _check_fused_activation(X, M)
     _check_tensor(X_q, torch.uint8, "x_q")
     _check(list(X_q.shape) == [M, K // 2], "x_q must be [M, K/2]")
     _check_linear_operand(X_q, X_sf, X_global_scale, M, "x")
@@ -248,11 +278,42 @@ def linear_nvfp4_fused(D, X, X_q, X_sf, X_global_scale, B, B_sf, B_global_scale,
         linear_nvfp4(D, X_q, X_sf, X_global_scale, B, B_sf, B_global_scale, bias)
         return
     nbytes = _L.ac4k_linear_nvfp4_workspace_bytes(M, N, K)  # 0: one K range per tile, no scratch
-    ws = torch.empty((nbytes,), dtype=torch.uint8, device=D.device) if nbytes > 0 else None
-    _lib.check(_L.ac4k_linear_nvfp4_fused_bf16(D.data_ptr(), _DTYPE_TAG[D.dtype], X.data_ptr(), X_q.data_ptr(),
+    ws = D.new_empty((nbytes,), dtype=torch.uint8) if nbytes > 0 else None
+    _lib.check(_L.ac4k_linear_nvfp4_fused_bf16(D.data_ptr(), tag, X.data_ptr(), X_q.data_ptr(),
                                                X_sf.data_ptr(), X_global_scale.data_ptr(), B.data_ptr(),
                                                B_sf.data_ptr(), B_global_scale.data_ptr(), bias_ptr, bias_tag,
                                                M, N, K, None if ws is None else ws.data_ptr(), nbytes, _stream()))
+
+
+def _check_fused_activation(X, M):
+    _check_tensor(X, torch.bfloat16, "x")
+    _check(X.dim() == 2 and X.size(0) == M, "x must be [{}, K]", M)
+    _check(1 <= M <= 32, "the fused linear takes 1 <= M <= 32")
+    K = X.size(1)
+    _check(K % 64 == 0, "K must be a multiple of 64")
+    return K
+
+
+def linear_nvfp4_fused_scratch(D, X, B, B_sf, B_global_scale, bias=None) -> bool:
+    """linear_nvfp4_fused for a caller who does not ask for the quantized activation: it and the workspace are one allocation.
+    False, with nothing done, for a K that runs as the composition."""
+    M, N, tag = _check_output(D)
+    K = _check_fused_activation(X, M)
+    if K == 0 or K % 256 != 0:
+        return False
+    _check(B.dim() == 2 and B.size(0) == N and B.size(1) == K // 2, "weight must be [N, K/2]")
+    _check_linear_operand(B, B_sf, B_global_scale, N, "b")
+    bias_ptr, bias_tag = (None, 0) if bias is None else _bias_args(bias, N)
+    nbytes = _L.ac4k_linear_nvfp4_workspace_bytes(M, N, K)  # 0: one K range per tile, no scratch
+    q_bytes, sf_bytes = _align_up(M * K // 2, 256), K // 64 * _align_up(M, 16) * 4  # (a multiple of 256: K % 256 == 0)
+    ws_bytes = _align_up(nbytes, 256)
+    ws = D.new_empty((ws_bytes + q_bytes + sf_bytes + 4,), dtype=torch.uint8)
+    at = ws.data_ptr()
+    q = at + ws_bytes
+    _lib.check(_L.ac4k_linear_nvfp4_fused_bf16(D.data_ptr(), tag, X.data_ptr(), q, q + q_bytes, q + q_bytes + sf_bytes, B.data_ptr(),
+                                               B_sf.data_ptr(), B_global_scale.data_ptr(), bias_ptr, bias_tag,
+                                               M, N, K, at if nbytes > 0 else None, nbytes, _stream()))
+    return True
 
 
 def _check_attention_operand(x, x_sf, x_gs, B, H, rows, width, name):
@@ -339,9 +400,12 @@ def mha_int8_x_fp8_fwd(o, q, q_sf, q_quantize_block_size: int, k, k_sf, k_quanti
                                           v_sf.data_ptr(), B, H, Nq, Nkv, Dqk, Dv, float(sm_scale), _stream()))
 
 
-def _attention(entry, workspace_bytes, o, q, k, v, scale: float, sm_scale: float) -> bool:
+def _attention(entry, workspace_bytes, o, q, k, v, scale: float, sm_scale: float, bnhd: bool) -> bool:
     try:
-        (B, H, Nq, Dqk), (k_B, k_H, Nkv, k_D), (v_B, v_H, v_N, Dv), (o_B, o_H, o_N, o_D) = q.shape, k.shape, v.shape, o.shape
+        if bnhd:
+            (B, Nq, H, Dqk), (k_B, Nkv, k_H, k_D), (v_B, v_N, v_H, Dv), (o_B, o_N, o_H, o_D) = q.shape, k.shape, v.shape, o.shape
+        else:
+            (B, H, Nq, Dqk), (k_B, k_H, Nkv, k_D), (v_B, v_H, v_N, Dv), (o_B, o_H, o_N, o_D) = q.shape, k.shape, v.shape, o.shape
     except ValueError:  # not 4D
         return False
     dev, bf16 = q.get_device(), torch.bfloat16  # -1 on the CPU
@@ -349,28 +413,31 @@ def _attention(entry, workspace_bytes, o, q, k, v, scale: float, sm_scale: float
             and dev >= 0 and dev == k.get_device() == v.get_device() == o.get_device()
             and q.dtype is bf16 and k.dtype is bf16 and v.dtype is bf16 and o.dtype is bf16):
         return False
-    (q_b, q_h, q_n, q_d), (k_b, k_h, k_n, k_d), (v_b, v_h, v_n, v_d) = q.stride(), k.stride(), v.stride()
+    if bnhd:
+        (q_b, q_n, q_h, q_d), (k_b, k_n, k_h, k_d), (v_b, v_n, v_h, v_d), (o_b, o_n, o_h, o_d) = q.stride(), k.stride(), v.stride(), o.stride()
+    else:
+        (q_b, q_h, q_n, q_d), (k_b, k_h, k_n, k_d), (v_b, v_h, v_n, v_d), (o_b, o_h, o_n, o_d) = q.stride(), k.stride(), v.stride(), o.stride()
     if q_d != 1 or k_d != 1 or v_d != 1:
         return False
     nbytes = workspace_bytes(B, H, Nq, Nkv, Dqk, Dv)
     if nbytes < 0:
         return False
-    ws = torch.empty((nbytes,), dtype=torch.uint8, device=q.device)
-    _lib.check(entry(o.data_ptr(), *o.stride(), q.data_ptr(), q_b, q_h, q_n, k.data_ptr(), k_b, k_h, k_n, v.data_ptr(), v_b, v_h, v_n,
+    ws = q.new_empty((nbytes,), dtype=torch.uint8)
+    _lib.check(entry(o.data_ptr(), o_b, o_h, o_n, o_d, q.data_ptr(), q_b, q_h, q_n, k.data_ptr(), k_b, k_h, k_n, v.data_ptr(), v_b, v_h, v_n,
                      B, H, Nq, Nkv, Dqk, Dv, scale, sm_scale, ws.data_ptr(), nbytes, _stream()))
     return True
 
 
-def attention_int8_x_fp8(o, q, k, v, v_scale_max: float, sm_scale: float) -> bool:
+def attention_int8_x_fp8(o, q, k, v, v_scale_max: float, sm_scale: float, bnhd: bool = False) -> bool:
     """The whole `_int8_x_fp8_attention` (python/ac4k_kernel/ops/attention.py:137-190) behind one C call on bf16 q, k, v
-    viewed as [B,H,N,D] (any batch, head and token strides).  False, with nothing done, for operands this call does not
+    of [B,H,N,D], or of [B,N,H,D] with `bnhd` (any batch, head and token strides).  False, with nothing done, for operands this call does not
     take - odd shapes, other dtypes and the ones an operator-by-operator call rejects with its own message."""
-    return _attention(_L.ac4k_attention_int8_x_fp8_bf16, _L.ac4k_attention_int8_x_fp8_workspace_bytes, o, q, k, v, v_scale_max, sm_scale)
+    return _attention(_L.ac4k_attention_int8_x_fp8_bf16, _L.ac4k_attention_int8_x_fp8_workspace_bytes, o, q, k, v, v_scale_max, sm_scale, bnhd)
 
 
-def attention_nvfp4(o, q, k, v, sm_scale: float) -> bool:
+def attention_nvfp4(o, q, k, v, sm_scale: float, bnhd: bool = False) -> bool:
     """The same for `_nvfp4_attention` (python/ac4k_kernel/ops/attention.py:100-133) on dense q, k, v."""
-    return _attention(_L.ac4k_attention_nvfp4_bf16, _L.ac4k_attention_nvfp4_workspace_bytes, o, q, k, v, 2688.0, sm_scale)
+    return _attention(_L.ac4k_attention_nvfp4_bf16, _L.ac4k_attention_nvfp4_workspace_bytes, o, q, k, v, 2688.0, sm_scale, bnhd)
 
 
 def quantize_int8_token_block(y, scale, x_bhnd, block: int) -> None:

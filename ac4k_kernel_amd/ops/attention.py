@@ -45,12 +45,11 @@ def _int8_x_fp8_attention(q, k, v, layout, Q_QUANTIZE_BLOCK_SIZE=64, K_QUANTIZE_
     if out is None:
         out_shape = (B, Nq, H, Dv) if layout == "BNHD" else (B, H, Nq, Dv)
         out = torch.empty(out_shape, dtype=torch.bfloat16, device=q.device)
-    bhnd = (lambda t: t.permute(0, 2, 1, 3)) if layout == "BNHD" else (lambda t: t)
-    o_bhnd = bhnd(out)  # the kernel writes through the strides
     # the operator takes dense V only; everything else goes operator by operator
     if (Q_QUANTIZE_BLOCK_SIZE, K_QUANTIZE_BLOCK_SIZE) == (64, 128) and v.is_contiguous() and _rocm_ops.attention_int8_x_fp8(
-            o_bhnd, bhnd(q), bhnd(k), bhnd(v), 2.25, 1 / math.sqrt(Dqk)):
+            out, q, k, v, 2.25, 1 / math.sqrt(Dqk), layout == "BNHD"):
         return out
+    o_bhnd = out.permute(0, 2, 1, 3) if layout == "BNHD" else out  # the kernel writes through the strides
     n_dim = 1 if layout == "BNHD" else 2
     k = k - k.mean(dim=n_dim, keepdim=True)
     q_int8, q_sf = _int8_quantize(q, layout, n_dim, BLOCK_SIZE=Q_QUANTIZE_BLOCK_SIZE)
@@ -72,12 +71,11 @@ def _nvfp4_attention(q, k, v, layout, out=None):
     if out is None:
         out_shape = (B, Nq, H, Dv) if layout == "BNHD" else (B, H, Nq, Dv)
         out = torch.empty(out_shape, dtype=torch.bfloat16, device=q.device)
-    bhnd = (lambda t: t.permute(0, 2, 1, 3)) if layout == "BNHD" else (lambda t: t)
-    o_bhnd = bhnd(out)  # the kernel writes through the strides
     # the quantizers take dense tensors only; everything else goes operator by operator
     if q.is_contiguous() and k.is_contiguous() and v.is_contiguous() and _rocm_ops.attention_nvfp4(
-            o_bhnd, bhnd(q), bhnd(k), bhnd(v), 1 / math.sqrt(Dqk)):
+            out, q, k, v, 1 / math.sqrt(Dqk), layout == "BNHD"):
         return out
+    o_bhnd = out.permute(0, 2, 1, 3) if layout == "BNHD" else out  # the kernel writes through the strides
     n_dim = 1 if layout == "BNHD" else 2
     q_fp4, q_sf, q_alpha = quantize(q, n_dim, 3)
     k_fp4, k_sf, k_alpha = quantize(k, n_dim, 3)

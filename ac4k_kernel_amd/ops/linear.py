@@ -17,8 +17,7 @@ class Ac4kLinearOp(torch.nn.Module):
         if (bias is not None) and (bias.ndim == 1):
             bias = bias.reshape(1, -1)
         if out is None:
-            m, n = x.shape[0], weight.shape[0]
-            out = torch.empty((m, n), dtype=torch.bfloat16, device=x.device)
+            out = torch.empty((x.size(0), weight.size(0)), dtype=torch.bfloat16, device=x.device)
         linear_nvfp4(out, x, x_scale, x_global_scale, weight, weight_scale, weight_global_scale, bias)
         return out
 
@@ -47,6 +46,8 @@ def fused_linear(x, weight, weight_scale, weight_global_scale, bias=None, out=No
         bias = bias.reshape(1, -1)
     if out is None:
         out = torch.empty((m, n), dtype=torch.bfloat16, device=dev)
+    if not return_quantized and _rocm_ops.linear_nvfp4_fused_scratch(out, x, weight, weight_scale, weight_global_scale, bias):
+        return out
     x_q = torch.empty((m, k // 2), dtype=torch.uint8, device=dev)
     x_sf = torch.empty((k // 64, align_up(m, 16), 4), dtype=torch.float8_e4m3fn, device=dev)
     x_gs = torch.empty((), dtype=torch.float32, device=dev)
@@ -67,6 +68,6 @@ def linear_prepacked(x, x_scale, x_global_scale, weight_image, weight_global_sca
             if bias is None:
                 raise RuntimeError("linear_prepacked needs out, n or bias to know N")
             n = bias.shape[-1]
-        out = torch.empty((x.shape[0], n), dtype=torch.bfloat16, device=x.device)
+        out = torch.empty((x.size(0), n), dtype=torch.bfloat16, device=x.device)
     _rocm_ops.linear_nvfp4_prepacked(out, x, x_scale, x_global_scale, weight_image, weight_global_scale, bias)
     return out

@@ -94,6 +94,8 @@ class Ac4kQuantizeOp(torch.nn.Module):
 
         if max_scale is None:
             max_scale = 448.0 * 6.0  # FLOAT8_E4M3_MAX * FLOAT4_E2M1_MAX
+        if output is None and sf is None:
+            return _rocm_ops.quantize_nvfp4_new(input, cross_dim, reduce_dim, swizzle, float(max_scale))
         # out [.., cross, align_up(reduce, 64) / 2] u8, sf [.., align_up(reduce, 64) / 64, align_up(cross, 16), 4]
         Kp = align_up(K, 64)
         if output is None:

@@ -678,3 +678,17 @@ def test_sixteen_row_workgroups_on_an_image(m, n, k):
         torch.testing.assert_close(out.cpu(), T.linear_nvfp4(*cpu(aq), *cpu(bq), bias=bias.cpu(), out_dtype=dt), atol=ATOL, rtol=RTOL)
         if lib.ac4k_debug_linear_decode_kernel(m, n, k, ctypes.byref(ctypes.c_int())) == 4:
             assert torch.equal(ops().linear(*aq, *bq, bias=bias, out=torch.empty((m, n), dtype=dt, device="cuda")), out)
+
+
+@pytest.mark.parametrize("M,N,K", [(1, 16, 256), (1, 300, 512), (17, 64, 768), (32, 512, 4096), (16, 48, 64), (5, 48, 320), (3, 4100, 14336)])
+def test_fused_without_the_quantized_activation(M, N, K):
+    """A caller who does not ask for the quantized activation: it, its scales and the workspace share one allocation."""
+    g = torch.Generator(device="cuda").manual_seed(M * 1000 + N)
+    x = torch.randn((M, K), generator=g, device="cuda").to(torch.bfloat16)
+    wq = ops().quantize(torch.randn((N, K), generator=g, device="cuda").to(torch.bfloat16), 0, 1)
+    bias = torch.randn((N,), generator=g, device="cuda")
+    for dtype in (torch.bfloat16, torch.float32):
+        outs = [torch.full((M, N), float("nan"), dtype=dtype, device="cuda") for _ in range(2)]
+        ops().fused_linear(x, *wq, bias=bias, out=outs[0])
+        ops().fused_linear(x, *wq, bias=bias, out=outs[1], return_quantized=True)
+        assert torch.equal(outs[0], outs[1])
