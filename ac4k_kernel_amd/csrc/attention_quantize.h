@@ -18,6 +18,8 @@ struct AttnQuantArgs {
   float v_smax;
   // filled by attn_quant_plan
   int nsplit, span;
+  int waves;    // of a workgroup of the statistics
+  int classes;  // 0, or: the tiles take the statistics themselves, a span as so many interleaved sums
   float inv_nkv;
   // filled by attn_quant_layout: the operands of ac4k_mha_int8_x_fp8_fwd and the partial results, all in the workspace
   int Dp, Dvp, nqb, nkb, nvb;

@@ -6,6 +6,7 @@
 //                                   result per span (no atomics, so a call gives the same bits every time)
 //   2. attn_quantize_int8_fp8_kernel  every workgroup adds up the partials of its own channels (a few KB from L2) and
 //                                   quantizes one tile of V, K or Q
+// and as one for short heads, whose tiles take the statistics themselves (aq_own_faster).
 // Both are bound by HBM: 2 (K + V) bytes read in the first, 2 (Q + K + V) read and half of that written in the second.
 // MI355X, quantizers alone: B 1, N 16384, H 40, D 128 (BNHD) 350 -> 208 us = 84 (4.0 TB/s) + 124 (6.1 TB/s); a whole
 // attention of 777 queries on 257 keys, B 2, H 12, D 64: 64 -> 21 us, three launches instead of nine.  The operands are those
@@ -153,11 +154,77 @@ __device__ __forceinline__ void aq_join_spans(const uint32_t *part, int D, int n
   __syncthreads();
 }
 
+// The statistics of a short head by its tiles themselves, with no launch in front.  The sums of K are taken in the order of
+// aq_column_stats, so they have its bits: a span is a.classes interleaved sums there (its waves, times the tokens that a wave reads at
+// once), and `part` holds those of all spans.  Bound by the waits for the loads.
+// PAIRS sums of a lane at a time, ROWS tokens of each in flight.
+template <int PAIRS, int ROWS>
+__device__ __forceinline__ void aq_own_partial_sums(const AttnQuantArgs &a, int b, int head, float *part) {
+  const int tid = threadIdx.x, ls = aq_lane_shift(a.D), c = tid & ((1 << ls) - 1), slots = 256 >> ls, pairs = a.nsplit * a.classes;
+  if (c * 8 >= a.D) return;
+  const int c0 = aq_channel(c, a.D), step = a.classes;
+  const uint16_t *src = a.k.p + b * a.k.s_b + head * a.k.s_h + c0;
+  for (int p = tid >> ls; p < pairs; p += PAIRS * slots) {
+    int n[PAIRS], end[PAIRS];
+    float s[PAIRS][8] = {};
+#pragma unroll
+    for (int q = 0; q < PAIRS; ++q) {
+      const int split = (p + q * slots) / step, beg = split * a.span, last = beg + a.span < a.Nkv ? beg + a.span : a.Nkv;
+      n[q] = beg + p + q * slots - split * step;
+      end[q] = p + q * slots < pairs ? last : 0;
+    }
+    for (int i = 0; i < a.span; i += ROWS * step) {
+      uint4 v[PAIRS][ROWS];
+#pragma unroll
+      for (int q = 0; q < PAIRS; ++q)
+#pragma unroll
+        for (int u = 0; u < ROWS; ++u) {
+          v[q][u] = make_uint4(0, 0, 0, 0);
+          const int k = n[q] + i + u * step;
+          if (k < end[q]) v[q][u] = aq_load(src + (int64_t)k * a.k.s_n);
+        }
+#pragma unroll
+      for (int q = 0; q < PAIRS; ++q)
+#pragma unroll
+        for (int u = 0; u < ROWS; ++u) {
+          const uint32_t w[4] = {v[q][u].x, v[q][u].y, v[q][u].z, v[q][u].w};
+#pragma unroll
+          for (int e = 0; e < 4; ++e) {
+            s[q][2 * e] += bf16_lo(w[e]);
+            s[q][2 * e + 1] += bf16_hi(w[e]);
+          }
+        }
+    }
+#pragma unroll
+    for (int q = 0; q < PAIRS; ++q)
+      if (p + q * slots < pairs)
+#pragma unroll
+        for (int e = 0; e < 8; ++e) part[(p + q * slots) * a.D + c0 + e] = s[q][e];
+  }
+}
+__device__ __forceinline__ void aq_own_sums(const AttnQuantArgs &a, int b, int head, float *part, uint32_t *channel) {
+  if (a.classes == 1) aq_own_partial_sums<1, 8>(a, b, head, part);
+  else aq_own_partial_sums<2, 4>(a, b, head, part);
+  __syncthreads();
+  const int tid = threadIdx.x;
+  if (tid < a.D) {
+    float all = 0.0f;
+    for (int split = 0; split < a.nsplit; ++split) {
+      float sum = 0.0f;
+#pragma unroll 8
+      for (int k = 0; k < a.classes; ++k) sum += part[(split * a.classes + k) * a.D + tid];
+      all += sum;
+    }
+    channel[tid] = __float_as_uint(all);
+  }
+  __syncthreads();
+}
+
 // `BLOCK` tokens of one head to int8 with one scale; MEAN: minus the token mean of their channel, both rounded to
 // bf16 as the subtraction of two bf16 tensors rounds them.
-template <int BLOCK, bool MEAN>
+template <int BLOCK, bool MEAN, bool OWN>
 __device__ __forceinline__ void aq_int8_tile(const AttnQuantArgs &a, const AttnOperand &t, int N, int nb, int8_t *y,
-                                             float *scale, int b, int head, int blk, uint32_t *wmax, uint32_t *channel) {
+                                             float *scale, int b, int head, int blk, uint32_t *wmax, uint32_t *channel, float *part) {
   const int tid = threadIdx.x;
   const int ls = aq_lane_shift(a.D), c = tid & ((1 << ls) - 1), r0 = tid >> ls, rstep = 256 >> ls;
   constexpr int NV = BLOCK / 16;  // vectors per thread with 16 lanes per row (half of them with eight)
@@ -174,7 +241,8 @@ __device__ __forceinline__ void aq_int8_tile(const AttnQuantArgs &a, const AttnO
     if (live && r < rows) v[j] = aq_load_stream(src + r * t.s_n);
   }
   if (MEAN) {
-    aq_join_spans(reinterpret_cast<const uint32_t *>(a.ksum + bh * a.Dp), a.D, a.nsplit, (int64_t)a.B * a.H * a.Dp, channel,
+    if constexpr (OWN) aq_own_sums(a, b, head, part, channel);
+    else aq_join_spans(reinterpret_cast<const uint32_t *>(a.ksum + bh * a.Dp), a.D, a.nsplit, (int64_t)a.B * a.H * a.Dp, channel,
                   [](uint32_t sum, uint32_t x) { return __float_as_uint(__uint_as_float(sum) + __uint_as_float(x)); });
     float mean[8];
 #pragma unroll
@@ -215,7 +283,8 @@ __device__ __forceinline__ void aq_int8_tile(const AttnQuantArgs &a, const AttnO
 
 // 64 kv positions per wave, all channels of one head, to e4m3 along kv (the cross-major layout of the quantizers: a lane
 // holds eight channels of 16 stored positions)
-__device__ __forceinline__ void aq_fp8_tile(const AttnQuantArgs &a, int b, int head, int blk, uint32_t *channel) {
+template <bool OWN>
+__device__ __forceinline__ void aq_fp8_tile(const AttnQuantArgs &a, int b, int head, int blk, uint32_t *channel, uint32_t *part) {
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, kb = lane & 3, rg = lane >> 2;
   const int64_t bh = (int64_t)b * a.H + head;
   const int k0 = (blk * 4 + wave) * 64 + kb * 16;
@@ -223,13 +292,39 @@ __device__ __forceinline__ void aq_fp8_tile(const AttnQuantArgs &a, int b, int h
   const int c0 = aq_channel(live ? rg : 0, a.Dv);
   const uint16_t *src = a.v.p + b * a.v.s_b + head * a.v.s_h + c0;
   uint4 v[16];
+  u16x2 top[4] = {};
+  auto load = [&](int k1) {
 #pragma unroll
-  for (int i = 0; i < 16; ++i) {
-    const int k = k0 + ((i & 3) >> 1) * 8 + (i >> 2) * 2 + (i & 1);  // the 16-group swizzle
-    v[i] = make_uint4(0, 0, 0, 0);
-    if (live && k < a.Nkv) v[i] = aq_load(src + (int64_t)k * a.v.s_n);
-  }
-  aq_join_spans(a.vmax + bh * a.Dvp, a.Dv, a.nsplit, (int64_t)a.B * a.H * a.Dvp, channel, [](uint32_t m, uint32_t x) { return umax32(m, x); });
+    for (int i = 0; i < 16; ++i) {
+      const int k = k1 + ((i & 3) >> 1) * 8 + (i >> 2) * 2 + (i & 1);  // the 16-group swizzle
+      v[i] = make_uint4(0, 0, 0, 0);
+      if (live && k < a.Nkv) v[i] = aq_load(src + (int64_t)k * a.v.s_n);
+    }
+    if constexpr (OWN) {
+#pragma unroll
+      for (int i = 0; i < 16; ++i) {
+        const uint32_t w[4] = {v[i].x, v[i].y, v[i].z, v[i].w};
+#pragma unroll
+        for (int j = 0; j < 4; ++j) top[j] = __builtin_elementwise_max(top[j], __builtin_bit_cast(u16x2, w[j] & 0x7fff7fffu));
+      }
+    }
+  };
+  if constexpr (OWN)
+    for (int other = 0; other < a.nvb; ++other)
+      if (other != blk) load((other * 4 + wave) * 64 + kb * 16);
+  load(k0);
+  if constexpr (OWN) {  // maxima of the whole head: over the four lanes of a channel, then over the waves
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+#pragma unroll
+      for (int x = 1; x < 4; x *= 2)
+        top[j] = __builtin_elementwise_max(top[j], __builtin_bit_cast(u16x2, __shfl_xor((int)__builtin_bit_cast(uint32_t, top[j]), x)));
+      if (live && kb == 0) part[wave * 128 + c0 + 2 * j] = top[j].x, part[wave * 128 + c0 + 2 * j + 1] = top[j].y;
+    }
+    __syncthreads();
+    if (tid < a.Dv) channel[tid] = umax32(umax32(part[tid], part[128 + tid]), umax32(part[256 + tid], part[384 + tid]));
+    __syncthreads();
+  } else aq_join_spans(a.vmax + bh * a.Dvp, a.Dv, a.nsplit, (int64_t)a.B * a.H * a.Dvp, channel, [](uint32_t m, uint32_t x) { return umax32(m, x); });
   uint32_t mx[8];
 #pragma unroll
   for (int e = 0; e < 8; ++e) mx[e] = channel[c0 + e];
@@ -259,23 +354,25 @@ __device__ __forceinline__ void aq_fp8_tile(const AttnQuantArgs &a, int b, int h
   }
 }
 
+template <bool OWN>
 __global__ __launch_bounds__(256) void attn_quantize_int8_fp8_kernel(AttnQuantArgs a) {
   __shared__ uint32_t wmax[4], channel[128];
+  extern __shared__ __attribute__((aligned(16))) float aq_part[];  // OWN: aq_own_bytes
   uint32_t idx = blockIdx.x;
   const uint32_t BH = a.B * a.H;
   int b, head, blk;
   const uint32_t nv = BH * a.nvb, nk = BH * a.nkb;
   if (idx < nv) {
     aq_tile(a.v, a.H, a.nvb, idx, b, head, blk);
-    aq_fp8_tile(a, b, head, blk, channel);
+    aq_fp8_tile<OWN>(a, b, head, blk, channel, reinterpret_cast<uint32_t *>(aq_part));
   } else if (idx < nv + nk) {
     idx -= nv;
     aq_tile(a.k, a.H, a.nkb, idx, b, head, blk);
-    aq_int8_tile<AQ_K_BLOCK, true>(a, a.k, a.Nkv, a.nkb, a.k8, a.k_sf, b, head, blk, wmax, channel);
+    aq_int8_tile<AQ_K_BLOCK, true, OWN>(a, a.k, a.Nkv, a.nkb, a.k8, a.k_sf, b, head, blk, wmax, channel, aq_part);
   } else {
     idx -= nv + nk;
     aq_tile(a.q, a.H, a.nqb, idx, b, head, blk);
-    aq_int8_tile<AQ_Q_BLOCK, false>(a, a.q, a.Nq, a.nqb, a.q8, a.q_sf, b, head, blk, wmax, channel);
+    aq_int8_tile<AQ_Q_BLOCK, false, OWN>(a, a.q, a.Nq, a.nqb, a.q8, a.q_sf, b, head, blk, wmax, channel, aq_part);
   }
 }
 
@@ -396,12 +493,53 @@ static int64_t aq_spans(int64_t groups, int64_t Nkv) {
   return n < ceil_div(Nkv, AQ_MIN_SPAN) ? n : ceil_div(Nkv, AQ_MIN_SPAN);
 }
 static int aq_heads_per_wave(int D) { return D > 64 ? 4 : 8; }  // where the rows of neighbouring heads are adjacent
+static bool aq_heads_adjacent(const AttnQuantArgs &a, const AttnOperand &t) { return t.s_h < t.s_n && a.H > 1; }
+
+// workgroups of the statistics of one operand
+static int64_t aq_stat_units(const AttnQuantArgs &a, const AttnOperand &t, int D) {
+  return (int64_t)a.nsplit * a.B * ceil_div(a.H, aq_heads_adjacent(a, t) ? aq_heads_per_wave(D) : 1);
+}
+// LDS of a tile that takes the statistics itself: the sums of K, or the maxima of V of four waves
+static int aq_own_bytes(const AttnQuantArgs &a, int classes) {
+  const int sums = a.nsplit * classes * a.D * 4;
+  return sums > 2048 ? sums : 2048;
+}
+
+// Whether the tiles of short heads take the statistics themselves (the operands have the same bits either way).  That takes a launch
+// and its 4 us away and adds, in every tile of K, `rounds` waits for eight loads a lane and the joining of the sums; heads of more than
+// 512 keys would be read by too many tiles.  Whole calls of 777 queries, us, two launches -> one: BNHD 4 heads of 32 keys, D = 64, 13.7 -> 10.5, 2 x 12
+// of 257 21.0 -> 19.1, 2 x 40 of 128, D = 128, 31.3 -> 28.3; BHND 12 heads of 512, D = 64, 22.4 -> 19.5, 2 x 40 of 77 25.9 -> 21.6.  Behind the line: BNHD
+// 4 heads of 257, D = 128 (five rounds) 19.1 -> 19.0, of 400 20.5 -> 22.1; BHND 2 x 12 heads of 700, D = 64, 29.8 -> 31.9.
+// Grids of many heads pay for the registers of this kernel (112 against 91) in waves: 4096 heads of 49, D = 32, 81.6 -> 88.0, 3072 of 64,
+// D = 64, 71.9 -> 72.3; wide heads gain more than that: 3072 of 128, D = 128, 186 -> 164.
+static bool aq_own_faster(const AttnQuantArgs &a, int classes) {
+  const int slots = 256 >> (a.D > 64 ? 4 : 3);  // sums that a tile takes at a time
+  const int64_t rounds = ceil_div(a.nsplit * classes, slots) * ceil_div(ceil_div(a.span, classes), 8);
+  return a.Nkv <= 512 && rounds <= (classes == 1 ? 6 : 3) &&  // (so 48 KB of LDS at most)
+         (int64_t)a.B * a.H <= (a.D > 64 ? 4096 : 2048);
+}
 
 void attn_quant_plan(AttnQuantArgs &a) {
-  const int64_t groups = 2 * (int64_t)a.B * ceil_div(a.H, a.k.s_h < a.k.s_n && a.H > 1 ? aq_heads_per_wave(a.D) : 1);
+  const bool k_adjacent = aq_heads_adjacent(a, a.k);
+  const int64_t groups = 2 * (int64_t)a.B * ceil_div(a.H, k_adjacent ? aq_heads_per_wave(a.D) : 1);
   a.span = (int)ceil_div(a.Nkv, aq_spans(groups, a.Nkv));
   a.nsplit = (int)ceil_div(a.Nkv, a.span);
   a.inv_nkv = 1.0f / (float)a.Nkv;
+  // Sixteen waves a workgroup where a span lasts them for several rounds of loads: with about two workgroups per CU (more
+  // would be more spans) the loads in flight are what the pass lives on, 116 us with 4 waves, 95 with 8, 83 with 16 for
+  // K and V of 16384 x 40 x 128.  Short spans: eight (one round, 4.9 against 5.6 us at 257 x 12 x 64).
+  // More workgroups than the GPU holds at once, neighbouring tokens in a wave: no more waves than one round of loads needs, so
+  // that the sums of a wave meet fewer others and more workgroups are there (BHND, us with eight waves and now: 1024 x 8 windows
+  // of 49 tokens, D = 32, 80 and 17; 256 x 12 of 64, D = 64, 32 and 11; 128 x 16 of 100, D = 128, 23 and 18).
+  a.waves = a.span > 256 ? AQ_STAT_WAVES : 8;
+  if (a.span <= 256 && aq_stat_units(a, a.k, a.D) + aq_stat_units(a, a.v, a.Dv) > 1024 && !k_adjacent && !aq_heads_adjacent(a, a.v)) {
+    const int rows = AQ_STAT_LOADS * aq_heads_per_wave(a.D > a.Dv ? a.D : a.Dv);
+    for (a.waves = 1; a.waves * rows < a.span; a.waves *= 2) {}
+  }
+  // classes of one token each are one sum in the order of the tokens
+  int classes = a.waves * (k_adjacent ? 1 : aq_heads_per_wave(a.D));
+  if (classes >= a.span) classes = 1;
+  a.classes = aq_own_faster(a, classes) ? classes : 0;
 }
 
 int64_t attn_quant_layout(AttnQuantArgs &a, void *ws) {
@@ -425,26 +563,16 @@ int64_t attn_quant_layout(AttnQuantArgs &a, void *ws) {
 }
 
 void launch_attn_quant(const AttnQuantArgs &a, hipStream_t st) {
-  auto adjacent = [&](const AttnOperand &t) { return t.s_h < t.s_n && a.H > 1; };
-  auto units = [&](const AttnOperand &t, int D) {
-    return (int64_t)a.nsplit * a.B * ceil_div(a.H, adjacent(t) ? aq_heads_per_wave(D) : 1);
-  };
-  const int64_t uk = units(a.k, a.D), uv = units(a.v, a.Dv);
-  // Sixteen waves a workgroup where a span lasts them for several rounds of loads: with about two workgroups per CU (more
-  // would be more spans) the loads in flight are what the pass lives on, 116 us with 4 waves, 95 with 8, 83 with 16 for
-  // K and V of 16384 x 40 x 128.  Short spans: eight (one round, 4.9 against 5.6 us at 257 x 12 x 64).
-  // More workgroups than the GPU holds at once, neighbouring tokens in a wave: no more waves than one round of loads needs, so
-  // that the sums of a wave meet fewer others and more workgroups are there (BHND, us with eight waves and now: 1024 x 8 windows
-  // of 49 tokens, D = 32, 80 and 17; 256 x 12 of 64, D = 64, 32 and 11; 128 x 16 of 100, D = 128, 23 and 18).
-  int waves = a.span > 256 ? AQ_STAT_WAVES : 8;
-  if (a.span <= 256 && uk + uv > 1024 && !adjacent(a.k) && !adjacent(a.v)) {
-    const int rows = AQ_STAT_LOADS * aq_heads_per_wave(a.D > a.Dv ? a.D : a.Dv);
-    for (waves = 1; waves * rows < a.span; waves *= 2) {}
+  const dim3 tiles((unsigned)((int64_t)a.B * a.H * (a.nvb + a.nkb + a.nqb)));
+  if (a.classes > 0) {
+    hipLaunchKernelGGL(attn_quantize_int8_fp8_kernel<true>, tiles, dim3(256), aq_own_bytes(a, a.classes), st, a);
+    return;
   }
+  const int64_t uk = aq_stat_units(a, a.k, a.D), uv = aq_stat_units(a, a.v, a.Dv);
   // (less LDS, more workgroups; the LDS sized by the launch instead cost the kernel of long spans 0.1 us)
-  hipLaunchKernelGGL(waves <= 4 ? attn_column_stats_kernel<4> : attn_column_stats_kernel<AQ_STAT_WAVES>,
-                     dim3((unsigned)(uk > uv ? uk : uv), 2), dim3(64 * waves), 0, st, a);
-  hipLaunchKernelGGL(attn_quantize_int8_fp8_kernel, dim3((unsigned)((int64_t)a.B * a.H * (a.nvb + a.nkb + a.nqb))), dim3(256), 0, st, a);
+  hipLaunchKernelGGL(a.waves <= 4 ? attn_column_stats_kernel<4> : attn_column_stats_kernel<AQ_STAT_WAVES>,
+                     dim3((unsigned)(uk > uv ? uk : uv), 2), dim3(64 * a.waves), 0, st, a);
+  hipLaunchKernelGGL(attn_quantize_int8_fp8_kernel<false>, tiles, dim3(256), 0, st, a);
 }
 
 int64_t attn_nvfp4_layout(AttnNvfp4Args &a, void *ws) {

@@ -147,6 +147,26 @@ def test_whole_call_with_exact_means_is_bit_identical(B, Nq, Nkv, H, Dqk, Dv, la
     assert torch.equal(got, want) and torch.isfinite(got).all()
 
 
+# short heads, whose tiles take sums and maxima themselves: edges of spans, of tiles of K (128) and V (256) and of the rule (512 keys, heads)
+@pytest.mark.parametrize("B,Nkv,H,Dqk,Dv,layout", [(1, 1, 3, 64, 8, "BNHD"), (2, 32, 4, 128, 64, "BNHD"), (1, 33, 9, 8, 128, "BNHD"), (1, 128, 5, 100, 100, "BNHD"),
+                                                   (2, 129, 40, 64, 64, "BNHD"), (1, 255, 12, 40, 96, "BNHD"), (1, 257, 12, 64, 64, "BNHD"),
+                                                   (1, 511, 1, 128, 128, "BHND"), (1, 512, 4, 64, 72, "BHND"), (1, 513, 4, 64, 72, "BHND"),
+                                                   (2, 300, 40, 64, 64, "BHND"), (64, 49, 32, 32, 32, "BHND"), (64, 49, 33, 32, 32, "BNHD"),
+                                                   (128, 65, 32, 72, 128, "BHND")])
+def test_short_heads_take_their_own_statistics(B, Nkv, H, Dqk, Dv, layout, monkeypatch):
+    shape = lambda n, d: (B, n, H, d) if layout == "BNHD" else (B, H, n, d)  # noqa: E731
+    q, v = make_input(shape(21, Dqk), seed=1).cuda(), make_input(shape(Nkv, Dv), seed=3).cuda()
+    k = exact_mean_keys(shape(Nkv, Dqk), 1 if layout == "BNHD" else 2, 2)
+    for n in (0, Nkv - 1):  # the maximum in the first and in the last token
+        w = v.clone()
+        w.select(1 if layout == "BNHD" else 2, n).mul_(30.0)
+        got = ops().attention(q, k, w, layout=layout)
+        with monkeypatch.context() as m:
+            m.setattr(binding(), "attention_int8_x_fp8", lambda *a: False)
+            want = ops().attention(q, k, w, layout=layout)
+        assert torch.equal(got, want) and torch.isfinite(got).all()
+
+
 # numbers of token spans around those that are in flight together, and the most; more channels than lanes of a wave, and few
 @pytest.mark.parametrize("spans", [2, 7, 8, 9, 16, 17, 31, 32])
 @pytest.mark.parametrize("Dqk,Dv", [(128, 100), (8, 128)])
