@@ -929,23 +929,26 @@ static int64_t tile_scratch_bytes(int64_t M, int64_t N, int64_t K) {
 // Picks the tile and the K split by measured costs in microseconds on 256 CUs, with at most `scratch` bytes of partial sums:
 // rounds of 256 workgroups, stages per range times the time of a 128-k stage of that tile, a prologue and epilogue per round
 // and for more than one range the partial sums and the second launch.  A stage takes `stage` as long as up to three fifths of the
-// CUs have work and grows with their share from there to stage + 0.4 power, as the clock comes down.  Fitted to 1000 random shapes of
-// M = 129 to 12000, N = 256 to 28672, K = 256 to 14336 with every tile and up to 32 ranges that fit the scratch, and checked on 431 more: on
-// average 0.2 and 0.3 % slower than the fastest of these plans, 22 of the 431 by 2 to 10 % (few tiles in many ranges).  (The costs of the
-// loops before, with what pairs of waves now multiply together decoded by each of them: 0.8 %, 60 by 2 to 12 %.)  The sweeps held up to
-// four rounds of workgroups and 32 ranges, and so does the plan.
+// CUs have work and grows with their share from there to stage + 0.4 power, as the clock comes down.  A round beyond the first takes `round`.
+// Fitted to 1000 random shapes of
+// M = 129 to 12000, N = 256 to 28672, K = 256 to 14336 with every tile and up to 32 ranges that fit the scratch and to 200 of K up to 2048 and M up
+// to 75600, and checked on 431 and 130 more: on average 0.3 and 0.1 % slower than the fastest of these plans, 24 of the 431 by 2 to 10 % (few tiles in many
+// ranges).  (The costs of the loops before, with what pairs of waves now multiply together decoded by each of them: 0.8 %, 60 by 2 to
+// 12 %; one time of a round for all tiles took 256 x 128, whose rounds end with the exchange of halves, on many rows of short K: 56744 x 384 x 384
+// 33.1 us, 256 x 256 30.2.)  The sweeps held up to four rounds of workgroups and 32 ranges, and so does the plan.
 // The tiles of 192 rows are what fills a round where 128 or 256 rows leave CUs idle (us, best of the other tiles / with
 // them, loops before these): 4096 x 5120 x 5120 197.5 / 180.9, 7000 x 5120 x 5120 328.4 / 284.6, 6000 x 4096 x 4096 171.5 / 157.6, 300 x 14336 x 4096 50.9 / 45.3.
 struct TileCost {
   int mi, nj;
-  double stage, power, fixed;
+  double stage, power, fixed, round;
 };
-constexpr TileCost TILE_COSTS[] = {{4, 4, 2.108, 2.15, 10.693}, {3, 4, 1.658, 1.677, 8.526}, {4, 2, 1.299, 0.913, 7.309}, {2, 4, 1.275, 0.884, 7.907},
-                                   {3, 2, 1.053, 0.532, 7.527}, {2, 2, 0.781, 0.281, 7.892}, {2, 1, 0.519, 0.14, 4.738}};
+constexpr TileCost TILE_COSTS[] = {{4, 4, 2.209, 2.092, 8.603, 4.001}, {3, 4, 1.652, 1.604, 8.664, 5.286}, {4, 2, 1.328, 0.823, 7.567, 5.041},
+                                   {2, 4, 1.254, 0.952, 7.927, 4.367}, {3, 2, 1.062, 0.522, 7.758, 5.014}, {2, 2, 0.781, 0.281, 7.945, 4.549},
+                                   {2, 1, 0.519, 0.139, 5.454, 4.77}};
 static TilePlan tile_plan(int64_t M, int64_t N, int64_t K, int64_t scratch) {
   TilePlan best{};
   if (forced_tile_plan(M, N, K, best) && best.partial_bytes <= scratch) return best;
-  constexpr double ROUND_US = 4.77, SPLIT_US = 2.83, PARTIAL_BYTES_PER_US = 7.81e6;  // (8 bytes of a sum: written and read)
+  constexpr double SPLIT_US = 3.41, PARTIAL_BYTES_PER_US = 7.8e6;  // (8 bytes of a sum: written and read)
   const int stages = (int)ceil_div(K, P_BK);
   const int64_t sums_bytes = M * N * 4;
   const SplitCosts s = split_costs(M, N, stages, PARTIAL_BYTES_PER_US, SPLIT_US, scratch / sums_bytes < 32 ? (int)(scratch / sums_bytes) : 32);
@@ -960,8 +963,8 @@ static TilePlan tile_plan(int64_t M, int64_t N, int64_t K, int64_t scratch) {
       if (best.splits && least + s.sums_us[sp] >= best_t) break;  // nor will more ranges be faster
       const double len = s.len[sp];
       const int64_t full = tiles * sp / 256, tail = tiles * sp % 256;
-      double t = c.fixed - ROUND_US + (double)full * (len * (c.stage + 0.4 * c.power) + ROUND_US) + s.sums_us[sp];
-      if (tail) t += len * (c.stage + (tail > 153 ? ((double)tail / 256.0 - 0.6) * c.power : 0.0)) + ROUND_US;
+      double t = c.fixed - c.round + (double)full * (len * (c.stage + 0.4 * c.power) + c.round) + s.sums_us[sp];
+      if (tail) t += len * (c.stage + (tail > 153 ? ((double)tail / 256.0 - 0.6) * c.power : 0.0)) + c.round;
       if (best.splits == 0 || t < best_t) {
         best_t = t;
         best = TilePlan{c.mi, c.nj, sp, sp > 1 ? sp * sums_bytes : 0};
