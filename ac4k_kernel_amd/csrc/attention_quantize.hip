@@ -9,7 +9,7 @@
 // and as one for short heads, whose tiles take the statistics themselves (aq_own_faster).
 // Both are bound by HBM: 2 (K + V) bytes read in the first, 2 (Q + K + V) read and half of that written in the second.
 // MI355X, quantizers alone: B 1, N 16384, H 40, D 128 (BNHD) 350 -> 208 us = 84 (4.0 TB/s) + 124 (6.1 TB/s); a whole
-// attention of 777 queries on 257 keys, B 2, H 12, D 64: 64 -> 21 us, three launches instead of nine.  The operands are those
+// attention of 777 queries on 257 keys, B 2, H 12, D 64: 64 -> 21 us, three launches instead of nine, 19 with two.  The operands are those
 // of the separate calls bit for bit, except that a channel mean of K summed in another order may round to the other bf16.
 #include "attention_quantize.h"
 #include "quantize_nvfp4.h"
