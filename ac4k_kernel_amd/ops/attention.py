@@ -33,6 +33,11 @@ def _int8_quantize(x, layout, dim, type="token", BLOCK_SIZE=64, HDIM_ALIGN=16):
     return y, scale
 
 
+def _as_bhnd(layout, *operands):
+    """Views of [B,H,N,D]; operands of [B,N,H,D] with another number of dims are refused here (RuntimeError)."""
+    return tuple(t.permute(0, 2, 1, 3) for t in operands) if layout == "BNHD" else operands
+
+
 def _int8_x_fp8_attention(q, k, v, layout, Q_QUANTIZE_BLOCK_SIZE=64, K_QUANTIZE_BLOCK_SIZE=128, out=None):
     """INT8 (QK) x FP8 (PV) attention (python/ac4k_kernel/ops/attention.py:137-190)."""
     assert layout in ["BNHD", "BHND"], f"Unsupported layout: {layout}"
@@ -49,7 +54,7 @@ def _int8_x_fp8_attention(q, k, v, layout, Q_QUANTIZE_BLOCK_SIZE=64, K_QUANTIZE_
     if (Q_QUANTIZE_BLOCK_SIZE, K_QUANTIZE_BLOCK_SIZE) == (64, 128) and v.is_contiguous() and _rocm_ops.attention_int8_x_fp8(
             out, q, k, v, 2.25, 1 / math.sqrt(Dqk), layout == "BNHD"):
         return out
-    o_bhnd = out.permute(0, 2, 1, 3) if layout == "BNHD" else out  # the kernel writes through the strides
+    o_bhnd = _as_bhnd(layout, out, q, k, v)[0]  # the kernel writes through the strides
     n_dim = 1 if layout == "BNHD" else 2
     k = k - k.mean(dim=n_dim, keepdim=True)
     q_int8, q_sf = _int8_quantize(q, layout, n_dim, BLOCK_SIZE=Q_QUANTIZE_BLOCK_SIZE)
@@ -75,7 +80,7 @@ def _nvfp4_attention(q, k, v, layout, out=None):
     if q.is_contiguous() and k.is_contiguous() and v.is_contiguous() and _rocm_ops.attention_nvfp4(
             out, q, k, v, 1 / math.sqrt(Dqk), layout == "BNHD"):
         return out
-    o_bhnd = out.permute(0, 2, 1, 3) if layout == "BNHD" else out  # the kernel writes through the strides
+    o_bhnd = _as_bhnd(layout, out, q, k, v)[0]  # the kernel writes through the strides
     n_dim = 1 if layout == "BNHD" else 2
     q_fp4, q_sf, q_alpha = quantize(q, n_dim, 3)
     k_fp4, k_sf, k_alpha = quantize(k, n_dim, 3)

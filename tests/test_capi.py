@@ -231,6 +231,17 @@ def test_a_linear_asks_for_its_scratch_once(monkeypatch):
         assert (name, args[-2]) == (("ac4k_linear_nvfp4_workspace", size) if size else ("ac4k_linear_nvfp4", k))
 
 
+@pytest.mark.parametrize("precision", ["int8+fp8e4m3", "nvfp4"])
+@pytest.mark.parametrize("which", ["q", "k", "v", "out"])
+def test_attention_refuses_operands_that_are_not_4d(precision, which):
+    import torch
+    from ac4k_kernel_amd import ops
+    t = {name: torch.zeros((2, 64, 4, 64), dtype=torch.bfloat16) for name in ("q", "k", "v", "out")}
+    t[which] = t[which][0]
+    with pytest.raises(RuntimeError):
+        ops.attention(t["q"], t["k"], t["v"], out=t["out"], layout="BNHD", precision=precision)
+
+
 def decode_kernel(m, n, k):
     from ac4k_kernel_amd import _lib
     launches = ctypes.c_int(-1)
