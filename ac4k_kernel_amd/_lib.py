@@ -42,6 +42,7 @@ SIGNATURES = {
     "ac4k_prepack_weight_nvfp4_bytes": (_i64, [_i64, _i64]),
     "ac4k_prepack_weight_nvfp4": (_int, [_vp, _vp, _vp, _i64, _i64, _vp]),
     "ac4k_linear_nvfp4_prepacked_workspace_bytes": (_i64, [_i64, _i64, _i64]),
+    "ac4k_debug_linear_prepacked_decode_kernel": (_int, [_i64, _i64, _i64]),
     "ac4k_linear_nvfp4_prepacked": (_int, [_vp, _int, _vp, _vp, _vp, _vp, _vp, _vp, _int, _i64, _i64, _i64,
                                            _vp, _i64, _vp]),
     "ac4k_linear_nvfp4_fused_bf16": (_int, [_vp, _int, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _int,

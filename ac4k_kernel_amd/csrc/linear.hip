@@ -2853,6 +2853,12 @@ extern "C" __attribute__((visibility("default"))) int64_t ac4k_linear_nvfp4_prep
   return prepacked_plan(M, N, K, p) ? p.partial_bytes : 0;
 }
 
+extern "C" __attribute__((visibility("default"))) int ac4k_debug_linear_prepacked_decode_kernel(int64_t M, int64_t N, int64_t K) {
+  PrepackedPlan p;
+  if (!prepacked_plan(M, N, K, p) || !p.ring) return 0;
+  return p.sp.rows16 ? DECODE_ROWS16 : DECODE_LDS_RING;
+}
+
 extern "C" __attribute__((visibility("default"))) int ac4k_linear_nvfp4_prepacked(void *D, int d_dtype, const void *A, const void *A_sf, const float *A_gs,
                                                                                   const void *W_image, const float *B_gs, const void *bias,
                                                                                   int bias_dtype, int64_t M, int64_t N, int64_t K, void *workspace,

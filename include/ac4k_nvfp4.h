@@ -198,8 +198,9 @@ int ac4k_debug_linear_decode_kernel(int64_t M, int64_t N, int64_t K, int *fused_
  * the order the kernels fetch them, and the linear then reads the image instead of B and B_sf.
  * The arithmetic is untouched: same nibbles, same scale bytes, and for M > 32 the same order of accumulation, so the
  * output is bit-identical to the entry point of the plain layout that runs the same kernel
- * (ac4k_linear_nvfp4, or ac4k_linear_nvfp4_skinny for the shapes it splits along K).  For M <= 32 it is where the plain
- * layout streams through the 128-row LDS ring, too, and otherwise equal up to the order of the fp32 sums.
+ * (ac4k_linear_nvfp4, or ac4k_linear_nvfp4_skinny for the shapes it splits along K).  For M <= 32 each layout
+ * chooses its kernel by measured costs of its own, and the output is equal up to the order of the fp32 sums; bit-identical where both
+ * run the same kernel (ac4k_debug_linear_prepacked_decode_kernel and ac4k_debug_linear_decode_kernel both 2 or both 4).
  * Image: one block of 9216 bytes per (128 rows, 128 k), blocks of a 128-row band consecutive along
  * k, bands consecutive along n, N padded with zero rows to a whole band.  A block holds 128 rows x
  * 64 packed bytes, the 16-byte piece p of row r at position p ^ ((r >> 1) & 3) of its row, then the
@@ -209,8 +210,8 @@ int ac4k_debug_linear_decode_kernel(int64_t M, int64_t N, int64_t K, int *fused_
  * image (16-byte aligned).
  * ac4k_linear_nvfp4_prepacked: contract of ac4k_linear_nvfp4 with W_image in place of B and B_sf;
  * `workspace` as for ac4k_linear_nvfp4_skinny, of ac4k_linear_nvfp4_prepacked_workspace_bytes(M,N,K)
- * bytes (may be NULL when that is 0).  M <= 32 with K >= 256 streams the image through the LDS
- * ring, 32 < M <= 128 runs the K-split-waves kernel; everything else runs the tile kernel, split along K when there are too few tiles. */
+ * bytes (may be NULL when that is 0).  M <= 32 with K >= 256 streams the image through the 128-row LDS ring or runs 16 weight rows
+ * per workgroup, 32 < M <= 128 runs the K-split-waves kernel; everything else runs the tile kernel, split along K when there are too few tiles. */
 int64_t ac4k_prepack_weight_nvfp4_bytes(int64_t N, int64_t K);
 int ac4k_prepack_weight_nvfp4(void *image, const void *B, const void *B_sf, int64_t N, int64_t K,
                               ac4k_stream_t stream);
@@ -219,6 +220,10 @@ int ac4k_linear_nvfp4_prepacked(void *D, int d_dtype, const void *A, const void 
                                 const float *A_gs, const void *W_image, const float *B_gs,
                                 const void *bias, int bias_dtype, int64_t M, int64_t N, int64_t K,
                                 void *workspace, int64_t workspace_bytes, ac4k_stream_t stream);
+
+/* Testing aid: which decode-sized kernel a linear of this shape runs on a weight image, numbered as in ac4k_debug_linear_decode_kernel: 2, 4,
+ * or 0 for neither.  Runs nothing. */
+int ac4k_debug_linear_prepacked_decode_kernel(int64_t M, int64_t N, int64_t K);
 
 /* Fused decode-sized linear: quantize(X,0,1) followed by linear(...) in one call.  No single
  * reference function: it equals the composition the reference's tests make

@@ -668,6 +668,7 @@ def test_sixteen_row_workgroups_on_an_image(m, n, k):
     import ctypes
     from ac4k_kernel_amd import _lib
     lib = _lib.load()
+    assert lib.ac4k_debug_linear_prepacked_decode_kernel(m, n, k) == 4
     assert lib.ac4k_linear_nvfp4_prepacked_workspace_bytes(m, n, k) == 0
     check_tight(m, n, k, seed=m + k, image=True)
     aq, bq = gpu_quant(make_input((m, k), seed=m)), gpu_quant(make_input((n, k), seed=n, std=0.02))

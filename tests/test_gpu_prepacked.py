@@ -91,6 +91,20 @@ def test_lds_ring_kernel_bit_identical(m, n, k, linear_tuning):
     check_oracle(aq, wq, bias, d_img, torch.bfloat16)
 
 
+# decode-sized M as the library chooses, each layout by itself: the same bits where both run the same kernel (2: 128-row LDS ring, 4: 16
+# weight rows per workgroup), the values of the oracle in any case
+@pytest.mark.parametrize("m,n,k,plain,image", [(24, 28672, 1024, 2, 2), (32, 24700, 2176, 2, 2), (16, 4096, 1024, 4, 4), (32, 1000, 1152, 4, 4),
+                                               (16, 28672, 2048, 2, 4), (17, 28672, 512, 4, 2), (24, 14336, 3072, 3, 4)])
+def test_decode_kernels_of_both_layouts(m, n, k, plain, image):
+    from ac4k_kernel_amd import _lib
+    lib = _lib.load()
+    assert (lib.ac4k_debug_linear_decode_kernel(m, n, k, None), lib.ac4k_debug_linear_prepacked_decode_kernel(m, n, k)) == (plain, image)
+    aq, wq, bias, d_img, d_plain = both(m, n, k, seed=m, bias_dtype=torch.float32, o_dtype=torch.float32)
+    assert plain != image or torch.equal(d_img, d_plain)
+    check_oracle(aq, wq, bias, d_img, torch.float32)
+    check_oracle(aq, wq, bias, d_plain, torch.float32)
+
+
 # shapes whose plain layout runs another kernel (N < 128, or M <= 32 with K % 256 == 128): oracle only
 @pytest.mark.parametrize("m,n,k", [(40, 64, 256), (7, 33, 384), (32, 300, 128), (200, 5, 640)])
 @pytest.mark.parametrize("o", [torch.bfloat16, torch.float16, torch.float32])
