@@ -2796,15 +2796,18 @@ struct PrepackedPlan {
 // M = 1, 4096 x 4096 10.5 / 4.3, 28672 x 8192 32.3 / 28.1; M = 8, 28672 x 8192 32.5 / 31.2; M = 16, 4096 x 14336 18.1 / 10.1, 14336 x 4096 16.1 / 10.9,
 // 28672 x 8192 33.0 / 35.0, 27264 x 256 5.3 / 4.7; M = 20, 12288 x 12288 39.5 / 30.6, 27264 x 256 5.4 / 6.9, 28672 x 4096 21.0 / 24.1; M = 32,
 // 4096 x 14336 17.8 / 14.8, 2688 x 14208 14.8 / 11.8, 14336 x 14336 33.5 / 47.6, 256 x 14336 10.4 / 12.4.
+// Two tiles of activation rows (M > 16): two workgroups on a CU have their steps nearly one after the other (24 x 4096 x 8192 8.8 us, 4112 rows 13.3), and
+// the estimates have to differ by more than they err: of 423 shapes of M = 17 to 32 383 take 16 rows, four of these 3 to
+// 5 % slower than the ring (394 and 13 by 2 to 18 % without the two: 31 x 320 x 14080 10.7 / 12.7, 29 x 22656 x 512 6.7 / 7.7).
 static bool rows16_faster_image(int64_t M, int64_t N, int64_t K, const SkinnyPlan &p) {
   const double m = (double)M, cus = (double)decode_cu_count(), million = 1e-6 * (double)N * (double)K;
   const double steps = (double)ceil_div(ceil_div(K, R16_STEP), R16_WAVES), wgs = (double)ceil_div(N, R16_ROWS) / (2.0 * cus);
   const double last = wgs > 1.0 && wgs < 2.0 ? sqrt(2.0 / wgs) : 1.0;  // a second round that is not full
   const double rows16 = M <= 16 ? fmax(0.35 * wgs + (0.10 + 0.0022 * m) * million, (0.37 + 0.003 * m) * steps)
-                                : fmax(last * (wgs + (0.126 + 0.0016 * m) * million), (0.5 + 0.006 * m) * steps);
+                                : fmax(last * (wgs + (0.126 + 0.0016 * m) * million), (wgs > 0.5 ? 1.8 : 1.0) * (0.5 + 0.006 * m) * steps);
   const double rounds = ceil((double)(p.groups * p.split_k) / cus), stages = (double)ceil_div(ceil_div(K, ST_BK), p.split_k);
   const double ring = 4.2 + 0.03 * m + 0.8 * stages + 0.3 * fmin(stages, 8.0);
-  return 2.5 + rows16 < rounds * ring + (p.split_k > 1 ? 4.0 : 0.0);
+  return (M <= 16 ? 1.0 : 1.1) * (2.5 + rows16) < rounds * ring + (p.split_k > 1 ? 4.0 : 0.0);
 }
 
 static bool prepacked_plan(int64_t M, int64_t N, int64_t K, PrepackedPlan &p) {

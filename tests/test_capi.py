@@ -258,6 +258,17 @@ def test_sixteen_row_workgroups_stay_within_a_launch(m, k):
     assert decode_kernel(16, 2 ** 27 - 16, 256)[0] == 4  # the last that a launch carries
 
 
+def test_sixteen_row_workgroups_on_an_image_where_they_are_faster():
+    """M above 16, where the ring (2) was taken from shapes on which 16-row workgroups (4) are 4 to 18 % slower, and others that they are faster on."""
+    from ac4k_kernel_amd import _lib
+    f = _lib.load().ac4k_debug_linear_prepacked_decode_kernel
+    for shape in ((31, 320, 14080), (29, 22656, 512), (22, 384, 13568), (28, 384, 12672), (26, 888, 13312), (31, 19840, 512)):
+        assert f(*shape) == 2, shape
+    for shape in ((24, 4096, 8192), (24, 4112, 2048), (32, 4096, 14336), (20, 12288, 12288), (32, 128, 2048), (16, 4096, 14336), (1, 28672, 8192)):
+        assert f(*shape) == 4, shape
+    assert f(33, 4096, 4096) == 0 and f(16, 4096, 128) == 0
+
+
 def test_fused_calls_and_linears_sum_alike():
     """A fused call in one launch sums as the 16-row kernels do, so a linear of the same shape runs one of them: the two are equal bit
     for bit.  Shapes of one launch are among all of these sizes."""
