@@ -66,8 +66,8 @@ __device__ __forceinline__ void decode8(uint32_t w, f16x2 sp, f16x2 (&h)[4]) {
 // the tiles in bands of GROUP_M tile-rows, column by column inside a band: the workgroups resident
 // on one XCD at a time then cover a compact GROUP_M x (CUs / GROUP_M) patch and share its operand
 // panels through that L2.
-// (32 bits: a grid has fewer than 2^32 workgroups.  The quotients of 64 bits that were here, and of the K ranges below, took every workgroup
-// a third of a microsecond: 300 x 1024 x 256 5.23 -> 4.83 us, 2898 x 600 x 256 5.83 -> 5.46.)
+// (32 bits: a grid has fewer than 2^32 workgroups.  The quotients of 64 bits that were here, and of the range below where there is only one, took every
+// workgroup a third of a microsecond: 300 x 1024 x 256 5.23 -> 4.83 us, 2898 x 600 x 256 5.83 -> 5.46.)
 struct TileCoord {
   uint32_t m, n;
 };
@@ -242,8 +242,8 @@ __global__ __launch_bounds__(256) void linear_nvfp4_tile128_kernel(LinearArgs a)
 // Bound by instruction issue of a single wave per SIMD and, where the whole GPU is busy for long, by power.  Cycles per MFMA and wave, with
 // KW == 1, the decoding pinned between the MFMAs and the scales fetched a dword per lane / now: 256 x 256 41.2 / 35.2, 256 x 128 51 / 39,
 // 192 x 128 58 / 44, 128 x 128 70 / 51.  Back to back, us: 1024 x 4096 x 4096 38.3 / 32.8, 1001 x 5003 x 2880 35.7 / 33.6, 2048 x 4096 x 4096
-// 58.2 / 53.8, 2048 x 14336 x 4096 183.8 / 175.5, 75600 x 5120 x 5120 2776 / 2673 (the clock comes down by half of what the loop gains).  The
-// exchange costs half a microsecond a round: two stages of K lose by it what they gain (381 x 21120 x 256 11.6 / 12.0).
+// 58.2 / 53.8, 2048 x 14336 x 4096 183.8 / 175.5, 75600 x 5120 x 5120 2776 / 2673 (the clock comes down by half of what the loop gains).  256 x 128
+// and 128 x 256 tiles run KW == 2 on long ranges only (PAIR_STAGES), for the exchange.
 // Split-K: blockIdx.y selects a contiguous range of stages; with more than one range the
 // accumulators go to an fp32 partial buffer and a second kernel adds the ranges.
 // Requires K % 64 == 0, K >= 128 and 16-byte aligned operands.  EARLY: K % 128 == 64.  The stages start one
@@ -497,9 +497,10 @@ __device__ __forceinline__ void store_tile(const f32x16 (&acc)[MI][NJ], char *ld
   }
 }
 
-// MI = 32-row fragments per wave along M: 4 (BM = 256), 3 (BM = 192) or 2 (BM = 128);
-// NJ = 32-column fragments per wave along N: 4 (BN = 256), 2 (BN = 128) or 1 (BN = 64);
-// PS = LDS stages: PS - 1 k-steps are in flight ahead of the one being multiplied, which a small
+// MI = 32-row fragments that a wave stores along M: 4 (BM = 256), 3 (BM = 192) or 2 (BM = 128);
+// NJ = 32-column fragments that a wave stores along N: 4 (BN = 256), 2 (BN = 128) or 1 (BN = 64);
+// KW = waves that share the K of a stage; with two of them a wave multiplies twice as many fragments along one side (WI x WJ);
+// PS = LDS stages: PS - 1 k-steps (KW == 2: PS) are in flight ahead of the one being multiplied, which a small
 // tile needs because its k-step is much shorter than the memory latency.
 template <int D_DT, int BIAS_DT, int MI, int NJ, int PS, int KW, bool EARLY>
 __global__ __launch_bounds__(256, 1) void linear_nvfp4_tile256p_kernel(LinearArgs a, SplitK sk) {
@@ -845,12 +846,11 @@ static int allow_dynamic_lds(Kernel *kern, std::atomic<uint32_t> &done_mask, int
 }
 
 // LDS stages per tile shape: enough k-steps in flight to cover the memory latency
-constexpr int tile_k_waves(int mi, int nj) { return mi * nj > 8 ? 1 : 2; }
-constexpr int tile_stages(int mi, int nj) { return mi * nj >= 16 ? 3 : mi * nj > 8 ? 4 : mi * nj == 8 ? 5 : mi * nj >= 4 ? 6 : 8; }
+constexpr int tile_stages(int mi, int nj, int kw) { return mi * nj >= 16 ? 3 : mi * nj > 8 ? 4 : mi * nj == 8 ? 3 + kw : mi * nj >= 4 ? 6 : 8; }
 
-template <int D_DT, int BIAS_DT, int MI, int NJ>
-static int launch_tile_p(const LinearArgs &a, const SplitK &sk, hipStream_t st) {
-  constexpr int PS = tile_stages(MI, NJ), KW = tile_k_waves(MI, NJ);
+template <int D_DT, int BIAS_DT, int MI, int NJ, int KW>
+static int launch_tile_kw(const LinearArgs &a, const SplitK &sk, hipStream_t st) {
+  constexpr int PS = tile_stages(MI, NJ, KW);
   const bool early = a.K % P_BK != 0;
   auto *kern = early ? linear_nvfp4_tile256p_kernel<D_DT, BIAS_DT, MI, NJ, PS, KW, true> : linear_nvfp4_tile256p_kernel<D_DT, BIAS_DT, MI, NJ, PS, KW, false>;
   using PL = PLayout<64 * MI, 64 * NJ, PS>;
@@ -859,6 +859,19 @@ static int launch_tile_p(const LinearArgs &a, const SplitK &sk, hipStream_t st) 
   const int64_t ntiles = ceil_div(a.M, 64 * MI) * ceil_div(a.N, 64 * NJ);
   hipLaunchKernelGGL(kern, dim3((unsigned)ntiles, (unsigned)sk.splits), dim3(256), PL::LDS_BYTES, st, a, sk);
   return 0;
+}
+
+// 256 x 128 and 128 x 256 tiles multiply in pairs of waves from this length of a range on: the exchange of halves costs them 1.4 us a round, a
+// stage 0.08 less in pairs.  us, back to back, every wave by itself / pairs (and the loops before, which had no pairs): 8155 x 2056 x 256
+// 24.9 / 28.5 (27.3), x 512 31.7 / 36.7 (34.8), x 1024 47.4 / 50.0 (50.9), x 1792 74.3 / 74.4 (78.6), x 2304 88.9 / 87.7 (94.4); 473 x 11008 x 256
+// 9.3 / 10.4 (10.2), x 1792 23.6 / 23.9 (25.6), x 2304 28.6 / 28.2 (30.8).  The smaller tiles exchange half as much, and in
+// pairs they are faster than their loops before at any length.
+constexpr int PAIR_STAGES = 15;
+template <int D_DT, int BIAS_DT, int MI, int NJ>
+static int launch_tile_p(const LinearArgs &a, const SplitK &sk, hipStream_t st) {
+  if constexpr (MI * NJ == 8)
+    if (ceil_div(ceil_div(a.K, P_BK), sk.splits) < PAIR_STAGES) return launch_tile_kw<D_DT, BIAS_DT, MI, NJ, 1>(a, sk, st);
+  return launch_tile_kw<D_DT, BIAS_DT, MI, NJ, MI * NJ <= 8 ? 2 : 1>(a, sk, st);
 }
 
 // Tile shape and K split of the packed-LDS kernel for one problem.
@@ -934,8 +947,9 @@ static int64_t tile_scratch_bytes(int64_t M, int64_t N, int64_t K) {
 // M = 129 to 12000, N = 256 to 28672, K = 256 to 14336 with every tile and up to 32 ranges that fit the scratch and to 200 of K up to 2048 and M up
 // to 75600, and checked on 431 and 130 more: on average 0.3 and 0.1 % slower than the fastest of these plans, 24 of the 431 by 2 to 10 % (few tiles in many
 // ranges).  (The costs of the loops before, with what pairs of waves now multiply together decoded by each of them: 0.8 %, 60 by 2 to
-// 12 %; one time of a round for all tiles took 256 x 128, whose rounds end with the exchange of halves, on many rows of short K: 56744 x 384 x 384
-// 33.1 us, 256 x 256 30.2.)  The sweeps held up to four rounds of workgroups and 32 ranges, and so does the plan.
+// 12 %; one time of a round for all tiles took 256 x 128, whose rounds ended with the exchange of halves, on many rows of short K: 56744 x 384 x 384
+// 33.1 us, 256 x 256 30.2.  Fitted with the exchange in the short ranges of 256 x 128 and 128 x 256, too; taking its time out of
+// their costs chose them where the small tiles are faster than their estimate: 171 x 8409 x 192 7.0 -> 8.8.)  The sweeps held up to four rounds of workgroups and 32 ranges, and so does the plan.
 // The tiles of 192 rows are what fills a round where 128 or 256 rows leave CUs idle (us, best of the other tiles / with
 // them, loops before these): 4096 x 5120 x 5120 197.5 / 180.9, 7000 x 5120 x 5120 328.4 / 284.6, 6000 x 4096 x 4096 171.5 / 157.6, 300 x 14336 x 4096 50.9 / 45.3.
 struct TileCost {

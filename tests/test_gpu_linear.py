@@ -641,6 +641,17 @@ def test_ranges_about_as_long_as_the_stage_ring(mi, nj, linear_tuning):
     check_tight(64 * mi + 37, 64 * nj + 130, 1280, seed=1)
 
 
+# 256 x 128 and 128 x 256 tiles: every wave by itself up to ranges of 14 stages, pairs of waves from 15 on; the longest range of a launch decides for all
+@pytest.mark.parametrize("mi,nj", [(4, 2), (2, 4)])
+@pytest.mark.parametrize("splits,stages", [(1, (13, 14, 15, 16)), (2, (27, 28, 29, 30)), (3, (40, 43))])
+def test_ranges_about_as_long_as_pairs_of_waves_take(mi, nj, splits, stages, linear_tuning):
+    linear_tuning(mi, nj, splits)
+    for st in stages:
+        for k in (128 * st, 128 * st - 64):
+            check_tight(64 * mi + 37, 64 * nj + 130, k, seed=st)
+        check_tight(64 * mi + 101, 64 * nj + 1, 128 * st, seed=st, image=True)
+
+
 # scale tensors on four bytes: the tile kernel fetches 16 bytes of them at a time
 @pytest.mark.parametrize("mi,nj", sorted({p[:2] for p in TILE_PLANS}))
 @pytest.mark.parametrize("at", [4, 8, 12])
