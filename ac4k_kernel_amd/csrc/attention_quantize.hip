@@ -506,20 +506,26 @@ static int aq_own_bytes(const AttnQuantArgs &a, int classes) {
 }
 
 // Whether the tiles of short heads take the statistics themselves (the operands have the same bits either way).  That takes a launch
-// and its 4 us away and adds, in every tile of K, `rounds` waits for eight loads a lane and the joining of the sums; heads of more than
-// 512 keys would be read by too many tiles.  Whole calls of 777 queries, us, two launches -> one: BNHD 4 heads of 32 keys, D = 64, 13.7 -> 10.5, 2 x 12
+// and its 4 us away and adds, in every tile of K, waits for eight loads a lane and the joining of the sums; heads of more than
+// 512 keys would be read by too many tiles.  `rounds` is the score that the timings below were sorted by: the waits of one sum of a lane with eight
+// tokens in flight.  That is what one class runs; several run two sums of four tokens, and wait two times where it says three, three where it says five.
+// Sums of up to 24 KB in LDS stay in front of the line.  Whole calls of 777 queries, us, two launches -> one: BNHD 4 heads of 32 keys, D = 64, 13.7 -> 10.5, 2 x 12
 // of 257 21.0 -> 19.1, 2 x 40 of 128, D = 128, 31.3 -> 28.3; BHND 12 heads of 512, D = 64, 22.4 -> 19.5, 2 x 40 of 77 25.9 -> 21.6.  Behind the line: BNHD
-// 4 heads of 257, D = 128 (five rounds) 19.1 -> 19.0, of 400 20.5 -> 22.1; BHND 2 x 12 heads of 700, D = 64, 29.8 -> 31.9.
-// Grids of many heads pay for the registers of this kernel (112 against 91) in waves: 4096 heads of 49, D = 32, 81.6 -> 88.0, 3072 of 64,
-// D = 64, 71.9 -> 72.3; wide heads gain more than that: 3072 of 128, D = 128, 186 -> 164.
+// 4 heads of 257, D = 128 (a score of five) 19.1 -> 19.0, of 400 20.5 -> 22.1; BHND 2 x 12 heads of 700, D = 64, 29.8 -> 31.9.
+// Grids of many tiles pay for the registers of this kernel (112 against 91) in waves, heads of more than one tile for what the tiles read again:
+// `pays`, in us, fitted to 611 calls of 16 to 512 keys, 1 to 4096 heads and 20 to 16000 queries (3 us rms), against 3.25 that the launch takes, less
+// a margin of 1.5 for what the fit errs.  2048 heads of 264, D = 40, 239 -> 272, 768 of 318 109 -> 121, 512 of 338, D = 64, 73 -> 79, 512 of 34 with 5510
+// queries each, D = 32, 342 -> 355: of the 611 36 were 1 to 14 % slower, none of the 537 that are in front of this line.  Few large tiles
+// gain: 3072 of 128, D = 128, 186 -> 164.
 static bool aq_own_faster(const AttnQuantArgs &a, int classes) {
   const int slots = 256 >> (a.D > 64 ? 4 : 3);  // sums that a tile takes at a time
-  const int64_t rounds = ceil_div(a.nsplit * classes, slots) * ceil_div(ceil_div(a.span, classes), 8);
-  return a.Nkv <= 512 && rounds <= (classes == 1 ? 6 : 3) &&  // (so 48 KB of LDS at most)
-         (int64_t)a.B * a.H <= (a.D > 64 ? 4096 : 2048);
+  const int64_t rounds = ceil_div(a.nsplit * classes, slots) * ceil_div(ceil_div(a.span, classes), 8), heads = (int64_t)a.B * a.H;
+  const double keys_mb = 1e-6 * (double)(heads * a.Nkv * (a.D > 64 ? 256 : 128));  // K as the lanes read it
+  const double pays = (double)heads * (0.23e-3 * a.nqb + 1.9e-3 * a.nkb) + (0.25 * (a.nvb - 1) - 0.164) * keys_mb;
+  return a.Nkv <= 512 && rounds <= (classes == 1 ? 6 : 3) && heads <= (a.D > 64 ? 4096 : 2048) && pays < 1.75;
 }
 
-void attn_quant_plan(AttnQuantArgs &a) {
+void attn_quant_plan(AttnQuantArgs &a) {  // (after attn_quant_layout)
   const bool k_adjacent = aq_heads_adjacent(a, a.k);
   const int64_t groups = 2 * (int64_t)a.B * ceil_div(a.H, k_adjacent ? aq_heads_per_wave(a.D) : 1);
   a.span = (int)ceil_div(a.Nkv, aq_spans(groups, a.Nkv));
