@@ -51,6 +51,7 @@ SIGNATURES = {
     "ac4k_mha_int8_x_fp8_fwd": (_int, [_vp] + [_i64] * 4 + [_vp, _vp, _int, _vp, _vp, _int, _vp, _vp] + [_i64] * 6 + [_f32, _vp]),
     "ac4k_attention_int8_x_fp8_workspace_bytes": (_i64, [_i64] * 6),
     "ac4k_attention_int8_x_fp8_bf16": (_int, [_vp] + [_i64] * 4 + ([_vp] + [_i64] * 3) * 3 + [_i64] * 6 + [_f32, _f32, _vp, _i64, _vp]),
+    "ac4k_debug_attention_quantize_int8_x_fp8": (_i64, ([_vp] + [_i64] * 3) * 3 + [_i64] * 6 + [_f32, _vp, _i64, _int, _vp, _vp]),
     "ac4k_attention_nvfp4_workspace_bytes": (_i64, [_i64] * 6),
     "ac4k_attention_nvfp4_bf16": (_int, [_vp] + [_i64] * 4 + ([_vp] + [_i64] * 3) * 3 + [_i64] * 6 + [_f32, _f32, _vp, _i64, _vp]),
     "ac4k_quantize_int8_token_block_bf16": (_int, [_vp, _vp, _vp] + [_i64] * 7 + [_int, _vp]),

@@ -1238,6 +1238,34 @@ extern "C" __attribute__((visibility("default"))) int64_t ac4k_attention_int8_x_
   return attn_quant_layout(a, nullptr);
 }
 
+// checks and plan of the quantizers; rc != 0: the call is refused
+static int attention_int8_plan(AttnQuantArgs &a, const void *q, int64_t q_b, int64_t q_h, int64_t q_n, const void *k, int64_t k_b, int64_t k_h,
+                               int64_t k_n, const void *v, int64_t v_b, int64_t v_h, int64_t v_n, int64_t B, int64_t H, int64_t Nq, int64_t Nkv,
+                               int64_t Dqk, int64_t Dv, float v_scale_max, void *workspace, int64_t workspace_bytes) {
+  if (int rc = attention_int8_args(a, B, H, Nq, Nkv, Dqk, Dv)) return rc;
+  if (int rc = attention_operands(a, q, q_b, q_h, q_n, k, k_b, k_h, k_n, v, v_b, v_h, v_n, workspace)) return rc;
+  AC4K_REQUIRE(v_scale_max > 0.0f, "v_scale_max must be positive");
+  const int64_t need = attn_quant_layout(a, workspace);
+  AC4K_REQUIRE(workspace_bytes >= need, "workspace too small: %lld bytes, %lld needed", (long long)workspace_bytes, (long long)need);
+  a.v_smax = v_scale_max;
+  attn_quant_plan(a);
+  return 0;
+}
+
+extern "C" __attribute__((visibility("default"))) int64_t ac4k_debug_attention_quantize_int8_x_fp8(
+    const void *q, int64_t q_b_stride, int64_t q_h_stride, int64_t q_n_stride, const void *k, int64_t k_b_stride, int64_t k_h_stride,
+    int64_t k_n_stride, const void *v, int64_t v_b_stride, int64_t v_h_stride, int64_t v_n_stride, int64_t B, int64_t H, int64_t Nq,
+    int64_t Nkv, int64_t Dqk, int64_t Dv, float v_scale_max, void *workspace, int64_t workspace_bytes, int two_launches, int *launches,
+    ac4k_stream_t stream) {
+  AttnQuantArgs a;
+  if (attention_int8_plan(a, q, q_b_stride, q_h_stride, q_n_stride, k, k_b_stride, k_h_stride, k_n_stride, v, v_b_stride, v_h_stride,
+                          v_n_stride, B, H, Nq, Nkv, Dqk, Dv, v_scale_max, workspace, workspace_bytes)) return -1;
+  if (two_launches) a.classes = 0;
+  launch_attn_quant(a, (hipStream_t)stream);
+  if (launches) *launches = a.classes > 0 ? 1 : 2;
+  return check_launch("ac4k_debug_attention_quantize_int8_x_fp8") ? -1 : (char *)a.ksum - (char *)workspace;
+}
+
 extern "C" __attribute__((visibility("default"))) int ac4k_attention_int8_x_fp8_bf16(
     void *O, int64_t o_b_stride, int64_t o_h_stride, int64_t o_n_stride, int64_t o_d_stride, const void *q, int64_t q_b_stride,
     int64_t q_h_stride, int64_t q_n_stride, const void *k, int64_t k_b_stride, int64_t k_h_stride, int64_t k_n_stride,
@@ -1245,14 +1273,8 @@ extern "C" __attribute__((visibility("default"))) int ac4k_attention_int8_x_fp8_
     int64_t Dqk, int64_t Dv, float v_scale_max, float sm_scale, void *workspace, int64_t workspace_bytes, ac4k_stream_t stream) {
   AC4K_REQUIRE(O, "null pointer argument");
   AttnQuantArgs a;
-  if (int rc = attention_int8_args(a, B, H, Nq, Nkv, Dqk, Dv)) return rc;
-  if (int rc = attention_operands(a, q, q_b_stride, q_h_stride, q_n_stride, k, k_b_stride, k_h_stride, k_n_stride, v, v_b_stride,
-                                  v_h_stride, v_n_stride, workspace)) return rc;
-  AC4K_REQUIRE(v_scale_max > 0.0f, "v_scale_max must be positive");
-  const int64_t need = attn_quant_layout(a, workspace);
-  AC4K_REQUIRE(workspace_bytes >= need, "workspace too small: %lld bytes, %lld needed", (long long)workspace_bytes, (long long)need);
-  a.v_smax = v_scale_max;
-  attn_quant_plan(a);
+  if (int rc = attention_int8_plan(a, q, q_b_stride, q_h_stride, q_n_stride, k, k_b_stride, k_h_stride, k_n_stride, v, v_b_stride,
+                                   v_h_stride, v_n_stride, B, H, Nq, Nkv, Dqk, Dv, v_scale_max, workspace, workspace_bytes)) return rc;
   launch_attn_quant(a, (hipStream_t)stream);
   if (int rc = check_launch("ac4k_attention_int8_x_fp8_bf16")) return rc;
   return ac4k_mha_int8_x_fp8_fwd(O, o_b_stride, o_h_stride, o_n_stride, o_d_stride, a.q8, a.q_sf, AQ_Q_BLOCK, a.k8, a.k_sf, AQ_K_BLOCK,

@@ -293,6 +293,16 @@ int ac4k_attention_int8_x_fp8_bf16(void *O, int64_t o_b_stride, int64_t o_h_stri
                                    float v_scale_max, float sm_scale, void *workspace, int64_t workspace_bytes,
                                    ac4k_stream_t stream);
 
+/* Testing aid: the quantizers of ac4k_attention_int8_x_fp8_bf16 alone, as that call launches them, or with two_launches != 0 as two launches
+ * also for the short heads that it takes in one.  Returns the bytes at the front of the workspace that hold the quantized operands, -1 on an
+ * error; *launches: how many it ran. */
+int64_t ac4k_debug_attention_quantize_int8_x_fp8(const void *q, int64_t q_b_stride, int64_t q_h_stride, int64_t q_n_stride,
+                                                 const void *k, int64_t k_b_stride, int64_t k_h_stride, int64_t k_n_stride,
+                                                 const void *v, int64_t v_b_stride, int64_t v_h_stride, int64_t v_n_stride,
+                                                 int64_t B, int64_t H, int64_t Nq, int64_t Nkv, int64_t Dqk, int64_t Dv,
+                                                 float v_scale_max, void *workspace, int64_t workspace_bytes,
+                                                 int two_launches, int *launches, ac4k_stream_t stream);
+
 /* Replaces _nvfp4_attention (python/ac4k_kernel/ops/attention.py:100-133) as a whole, in the same manner: q, k and v dense;
  * max_scale is that of quantize (2688). */
 int64_t ac4k_attention_nvfp4_workspace_bytes(int64_t B, int64_t H, int64_t Nq, int64_t Nkv, int64_t Dqk, int64_t Dv);

@@ -167,6 +167,37 @@ def test_short_heads_take_their_own_statistics(B, Nkv, H, Dqk, Dv, layout, monke
         assert torch.equal(got, want) and torch.isfinite(got).all()
 
 
+# one launch or two, the operands have the same bits: the tiles sum K in the order of the launch that they replace.  Keys whose sums are rounded
+# (a mean far from zero, magnitudes over several binades), so that another order shows.  Waves of one class and of several, spans that end early, one span
+# and many, heads that are neighbours in memory and not; where the rule takes two launches by itself the shape is there to pin it
+@pytest.mark.parametrize("B,Nkv,H,Dqk,Dv,layout,launches", [
+    (1, 1, 3, 64, 8, "BNHD", 1), (2, 32, 4, 128, 64, "BNHD", 1), (1, 33, 9, 8, 128, "BNHD", 1), (1, 128, 5, 100, 100, "BNHD", 1),
+    (2, 129, 40, 64, 64, "BNHD", 1), (1, 255, 12, 40, 96, "BNHD", 1), (2, 257, 12, 64, 64, "BNHD", 1), (1, 511, 1, 128, 128, "BHND", 1),
+    (1, 512, 4, 64, 72, "BHND", 1), (1, 513, 4, 64, 72, "BHND", 2), (2, 300, 40, 64, 64, "BHND", 2), (2, 300, 12, 64, 64, "BHND", 1),
+    (64, 49, 32, 32, 32, "BHND", 2), (64, 49, 16, 32, 32, "BNHD", 1), (128, 65, 32, 72, 128, "BHND", 1)])
+def test_one_launch_or_two_give_the_same_operands(B, Nkv, H, Dqk, Dv, layout, launches):
+    import ctypes
+    from ac4k_kernel_amd import _lib
+    lib = _lib.load()
+    Nq = 70
+    shape = lambda n, d: (B, n, H, d) if layout == "BNHD" else (B, H, n, d)  # noqa: E731
+    q, k, v = make_input(shape(Nq, Dqk), seed=1), make_input(shape(Nkv, Dqk), seed=2), make_input(shape(Nkv, Dv), seed=3)
+    k = ((k.float() + 3.0) * torch.exp2(make_input(k.shape, seed=4).float().mul(3.0).round())).to(torch.bfloat16)
+    q, k, v = q.cuda(), k.cuda(), v.cuda()
+    bhn = lambda t: (t.stride(0), t.stride(2), t.stride(1)) if layout == "BNHD" else t.stride()[:3]  # noqa: E731
+    nbytes = lib.ac4k_attention_int8_x_fp8_workspace_bytes(B, H, Nq, Nkv, Dqk, Dv)
+    got = []
+    for two in (0, 1):
+        ws, ran = torch.zeros((nbytes,), dtype=torch.uint8, device="cuda"), ctypes.c_int(0)
+        size = lib.ac4k_debug_attention_quantize_int8_x_fp8(
+            q.data_ptr(), *bhn(q), k.data_ptr(), *bhn(k), v.data_ptr(), *bhn(v), B, H, Nq, Nkv, Dqk, Dv, 2.25, ws.data_ptr(), nbytes, two,
+            ctypes.byref(ran), torch.cuda.current_stream().cuda_stream)
+        assert 0 < size <= nbytes, _lib.load().ac4k_last_error()
+        assert ran.value == (2 if two else launches)
+        got.append(ws[:size])
+    assert torch.equal(*got) and got[0].any()
+
+
 # numbers of token spans around those that are in flight together, and the most; more channels than lanes of a wave, and few
 @pytest.mark.parametrize("spans", [2, 7, 8, 9, 16, 17, 31, 32])
 @pytest.mark.parametrize("Dqk,Dv", [(128, 100), (8, 128)])
