@@ -548,6 +548,20 @@ def run_traffic(ops):
     print(json.dumps({"traffic_run": "done"}))
 
 
+def compact(v, depth=0):
+    """The result line as stdout gets it, all of it goes to stderr: a captured tail of stdout keeps about 14 KB, and a line without its
+    beginning is no JSON.  Six significant digits to a number; the entries of single workloads without what their keys and other fields say (sizes,
+    the rate of a roofline and its peak, the time of all steps) and without what was not measured."""
+    if isinstance(v, float):
+        return float(f"{v:.6g}")
+    if isinstance(v, dict):
+        said = ("workload", "total_ms", "plain_layout_ms_before", "plain_layout_ms_after", "rotating_bytes", "input_from") if depth > 1 else ()
+        if depth > 2:
+            said += ("achieved", "peak", "unit", "TFLOP/s", "GB/s")
+        return {k: compact(x, depth + 1) for k, x in v.items() if k not in said and not (depth > 1 and x is None)}
+    return [compact(x, depth + 1) for x in v] if isinstance(v, (list, tuple)) else v
+
+
 def run_quantize_timeline(ops, reps=20):
     """Phase boundaries of the single-launch nvfp4 quantizer from clock stamps inside the kernel
     (needs the library built by `python ac4k_kernel_amd/build.py --timeline`, loaded through
@@ -826,7 +840,8 @@ def main():
         summary.append("ref shapes: " + "  ".join(f"{n_} {v['TFLOP/s']:.0f}TF/{v['roofline']['frac']:.2f}"
                                                   for n_, v in line["ref_shapes"].items()))
     line["host"] = dict(HOST)
-    print(json.dumps(line), flush=True)
+    log("[bench] all of it: " + json.dumps(line))
+    print(json.dumps(compact(line)), flush=True)
     log("[bench] ---- summary (time, throughput, fraction of the roofline) ----")
     for ln in summary:
         log("[bench] " + ln)

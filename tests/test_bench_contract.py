@@ -26,6 +26,17 @@ def test_algorithmic_bytes():
     assert bench.MFMA_PEAK_TFLOPS == 2500.0 and bench.HBM_PEAK_GBS == 8000.0
 
 
+def test_result_line_is_short_and_keeps_what_is_asked_for():
+    import bench
+    roof = {"bound": "mfma", "achieved": 1438.9839614840855, "peak": 2500.0, "unit": "TFLOP/s", "frac": 0.5755935845936342, "traffic": None}
+    line = {"metric": "m", "value": 1438.9839614840855, "n_gpus": 1, "vs_baseline": None, "parity": True, "roofline": roof, "config": {"model": "x", "seq": None},
+            "shapes": {"a": {"workload": "a", "ms": 0.7640888690948486, "total_ms": 15.28, "roofline": roof, "image": None}}}
+    got = bench.compact(line)
+    assert got["value"] == 1438.98 and got["vs_baseline"] is None and got["n_gpus"] == 1 and got["parity"] is True
+    assert set(got["roofline"]) == set(roof) and got["config"] == line["config"]
+    assert got["shapes"] == {"a": {"ms": 0.764089, "roofline": {"bound": "mfma", "frac": 0.575594}}}
+
+
 def test_more_than_one_gpu_is_refused():
     r = subprocess.run([sys.executable, os.path.join(ROOT, "bench.py"), "--gpus", "2"], capture_output=True, text=True)
     assert r.returncode != 0
