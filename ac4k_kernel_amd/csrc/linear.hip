@@ -950,7 +950,9 @@ static int64_t tile_scratch_bytes(int64_t M, int64_t N, int64_t K) {
 // 12 %; one time of a round for all tiles took 256 x 128, whose rounds ended with the exchange of halves, on many rows of short K: 56744 x 384 x 384
 // 33.1 us, 256 x 256 30.2.)  The fit had the exchange in the short ranges of 256 x 128 and 128 x 256, too, which run without it: its time is taken out of the
 // rounds beyond the first (74018 x 320 x 384 43.5 -> 36.7, 300 shapes of more than one round 0.2 % less time on average, 10 of them 1 to 2.5 % more and 32
-// 1 to 7 % less; out of the first round, too, they were chosen where the small tiles are faster than their estimate: 171 x 8409 x 192 7.0 -> 8.8).  The sweeps held up to four rounds of workgroups and 32 ranges, and so does the plan.
+// 1 to 7 % less; out of the first round, too, they were chosen where the small tiles are faster than their estimate: 171 x 8409 x 192 7.0 -> 8.8).
+// It had no K of one stage; a round of 256 x 256 takes longer there: 71074 x 256 x 128 20.8 -> 17.0 us, and 260 shapes of K = 128 to 256 and more than
+// one round 2.3 % less time on average, one of them 2 % more.  The sweeps held up to four rounds of workgroups and 32 ranges, and so does the plan.
 // The tiles of 192 rows are what fills a round where 128 or 256 rows leave CUs idle (us, best of the other tiles / with
 // them, loops before these): 4096 x 5120 x 5120 197.5 / 180.9, 7000 x 5120 x 5120 328.4 / 284.6, 6000 x 4096 x 4096 171.5 / 157.6, 300 x 14336 x 4096 50.9 / 45.3.
 struct TileCost {
@@ -978,7 +980,9 @@ static TilePlan tile_plan(int64_t M, int64_t N, int64_t K, int64_t scratch) {
       if (best.splits && least + s.sums_us[sp] >= best_t) break;  // nor will more ranges be faster
       const double len = s.len[sp];
       const int64_t full = tiles * sp / 256, tail = tiles * sp % 256;
-      const double round = c.round - (c.mi * c.nj == 8 && len < PAIR_STAGES ? 1.4 - 0.08 * len : 0.0);  // no exchange
+      double round = c.round;
+      if (c.mi * c.nj == 8 && len < PAIR_STAGES) round -= 1.4 - 0.08 * len;  // no exchange
+      if (c.mi * c.nj == 16 && len < 2.0) round += 1.5;                      // one stage is over before the stores of the round in front
       double t = c.fixed - round + (double)full * (len * (c.stage + 0.4 * c.power) + round) + s.sums_us[sp];
       if (tail) t += len * (c.stage + (tail > 153 ? ((double)tail / 256.0 - 0.6) * c.power : 0.0)) + round;
       if (best.splits == 0 || t < best_t) {
